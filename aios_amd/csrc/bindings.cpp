@@ -745,8 +745,9 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       "attn_prefill",
       [](uintptr_t q, uintptr_t k, uintptr_t v, int slot, int start, int T, int H, int Hkv, int hd, int max_ctx,
          float scale, uintptr_t out, int ldo, uintptr_t st, uintptr_t block_table, int kv_fp8, float k_scale,
-         float v_scale) {
+         float v_scale, uintptr_t ws, size_t ws_bytes) {
         AttnPrefillArgs a;
+        a.ws = (float*)ws; a.ws_bytes = ws_bytes;
         a.kv_fp8 = kv_fp8; a.kv_scale_k = k_scale; a.kv_scale_v = v_scale;
         a.block_table = (const int*)block_table;
         a.q = (const float*)q; a.k_cache = (const bf16_t*)k; a.v_cache = (const bf16_t*)v;
@@ -757,7 +758,8 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       py::arg("q"), py::arg("k"), py::arg("v"), py::arg("slot"), py::arg("start"), py::arg("T"), py::arg("H"),
       py::arg("Hkv"), py::arg("hd"), py::arg("max_ctx"), py::arg("scale"), py::arg("out"), py::arg("ldo"),
       py::arg("st"), py::arg("block_table") = 0, py::arg("kv_fp8") = 0, py::arg("k_scale") = 1.f,
-      py::arg("v_scale") = 1.f);
+      py::arg("v_scale") = 1.f, py::arg("ws") = 0, py::arg("ws_bytes") = 0);
+  m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
   m.def("attn_prefill_supports", &attn_prefill_supports);
 
   // ------------------------------------------------------------------ layered decoders' row operations

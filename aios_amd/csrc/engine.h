@@ -358,6 +358,8 @@ class Engine {
   bool gm_ok_ = false;    // every layer's weights / head shape supported
   float *gm_x_ = nullptr, *gm_qkv_ = nullptr, *gm_q_ = nullptr, *gm_part_ = nullptr;
   bf16_t *gm_a16_ = nullptr, *gm_ff16_ = nullptr, *gm_attn16_ = nullptr;
+  float* gm_attn_ws_ = nullptr;  // partial results of attention launches split over the keys
+  size_t gm_attn_ws_bytes_ = 0;
   int *gm_tokens_ = nullptr, *gm_pos_ = nullptr, *gm_slot_ = nullptr;
   // chunks of <= 64 rows: the residual GEMMs' bf16(x * g_next) + per-tile sums (split RMSNorm)
   bf16_t* gm_xn16_ = nullptr;

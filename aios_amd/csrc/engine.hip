@@ -660,6 +660,8 @@ void Engine::finalize() {
       gm_ff16_ = (bf16_t*)dmalloc((size_t)G * cfg_.d_ff * 2);
       gm_attn16_ = (bf16_t*)dmalloc((size_t)G * qd * 2);
       ws += (size_t)G * (d + cfg_.d_ff + qd) * 2;
+      gm_attn_ws_bytes_ = attn_prefill_ws_bytes(hd);
+      gm_attn_ws_ = fbuf(gm_attn_ws_bytes_ / 4);
       gm_tokens_ = ibuf(G);
       gm_pos_ = ibuf(G);
       gm_slot_ = ibuf(G);
@@ -1314,6 +1316,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
       at.n_heads = H; at.n_kv_heads = Hkv; at.head_dim = hd; at.max_ctx = cfg_.max_ctx;
       at.scale = 1.f / std::sqrt((float)hd);
       at.out = gm_attn16_; at.ldo = qd;
+      at.ws = gm_attn_ws_; at.ws_bytes = gm_attn_ws_bytes_;
       launch_attn_prefill(at, stream_);
       // O projection (+ residual)
       std::memset(&g, 0, sizeof(g));

@@ -19,6 +19,12 @@
 // Online softmax per row in the log2 domain; fully masked rows cannot occur (key 0 <= pos).
 // Output: bf16 [T][n_heads * hd] (the O-projection GEMM's A operand).
 //
+// Splits over the keys: a launch of few (query block, KV head) workgroups -- a further turn of a
+// conversation, 300 new tokens behind 6000 cached ones: 80 workgroups for 256 CUs, each 98 tiles long --
+// cuts every workgroup's tiles into a.ns runs.  Each run leaves its unnormalised O (fp32), row max and
+// row sum in the workspace and attn_prefill_combine adds them up (fp32, in the order of the runs): 160 us
+// -> 62 us for both launches there (32 / 8 heads of 128, fp8 cache).
+//
 // VALU diet (rocprofv3 PMC at 2048 tokens: ~12 VALU instructions per MFMA, 129 TF/s): bf16 packing
 // in hardware (v_cvt_pk_bf16_f32, not a software RNE with a NaN test), raw v_exp_f32 (ocml's
 // exp2f adds range scaling), and the O rescale skipped when no row max of the wave moved.
@@ -41,6 +47,16 @@ __device__ __forceinline__ float raw_exp2(float x) { return __builtin_amdgcn_exp
 constexpr int FP_KT = 64;  // keys per tile
 
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+
+// the tiles of run z of the ns runs over the keys that query block [t0, t0 + BQ) sees
+struct FpRun {
+  int kt0, kt1;
+};
+__device__ __forceinline__ FpRun fp_run(int start, int T, int t0, int BQ, int ns, int z) {
+  const int ntiles = (start + min(T, t0 + BQ) - 1) / FP_KT + 1;  // to the block's highest query position
+  const int per = (ntiles + ns - 1) / ns;
+  return {min(z * per, ntiles), min((z + 1) * per, ntiles)};
+}
 
 // F8: the pool holds fp8 e4m3 codes (EngineConfig::kv_fp8): the tile loads move half the bytes and
 // staging converts the codes to bf16 (exact; v_cvt_scalef32_pk_bf16_fp8 at scale 1 -- its scale
@@ -120,8 +136,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   constexpr int ES = F8 ? 1 : 2;  // bytes per cached element
   const uint8_t* kc = (const uint8_t*)a.k_cache + (size_t)kvh * KV_BLOCK * HD * ES;
   const uint8_t* vc = (const uint8_t*)a.v_cache + (size_t)kvh * KV_BLOCK * HD * ES;
-  const int last_pos = start + min(T, t0 + BQ) - 1;  // highest query position of the block
-  const int ntiles = last_pos / FP_KT + 1;
+  // this run's tiles [kt0, kt1) of the block's (a.ns == 1: all of them)
+  const FpRun run = fp_run(start, T, t0, BQ, a.ns, blockIdx.z);
+  const int kt0 = run.kt0, kt1 = run.kt1;
+  if (kt0 >= kt1) return;  // (uniform; the combine counts the runs the same way)
+  const int klim = min(qpos, kt1 * FP_KT - 1);  // keys this lane sees in this run
+  // ... and the least of them over the wave's rows: a tile that ends there needs no mask
+  const int klim_w = min(start + min(T - 1, t0 + __builtin_amdgcn_readfirstlane(wave) * 32 / G), kt1 * FP_KT - 1);
 
   // tile loader: 64 keys x HD dims of K and of V, 16 B per piece, into register buffer r (2 of
   // them: tile kt + 2 is requested while tile kt is computed, so two tiles of math cover the
@@ -132,7 +153,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   struct Regs {
     PT k[PPT], v[PPT];
   };
-  const int nt_last = ntiles - 1;
+  const int nt_last = kt1 - 1;
   auto load = [&](Regs& r, int kt) {
     kt = min(kt, nt_last);  // (clamped: the pipeline's tail requests are re-reads, never unmapped blocks)
     const size_t tbase = (size_t)kv_block(a.block_table, maxb, a.slot, kt * FP_KT) * blk_stride +
@@ -190,18 +211,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     // ---- causal mask + online softmax for this lane's row (32 of the 64 keys; partner lane^32)
     const int kbase = kt * FP_KT;
-    const bool full = kbase + FP_KT - 1 <= qpos;
+    if (kbase + FP_KT - 1 > klim_w) {  // (wave-uniform)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (kbase + t * 32 + (r & 3) + 8 * (r >> 2) + 4 * half > klim) st[t][r] = -INFINITY;
+    }
     float mx = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = kbase + t * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
-        if (!full && key > qpos) st[t][r] = -INFINITY;
-        mx = fmaxf(mx, st[t][r]);
-      }
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[t][r]);
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m_run, mx);  // finite: key 0 of tile 0 is always visible
+    const float mx_run = fmaxf(m_run, mx);
+    // -inf only where a run has shown this row no key yet (never with one run: key 0 is visible): p = 0 then
+    const float mn = a.ns > 1 && mx_run == -INFINITY ? 0.f : mx_run;
     const float alpha = raw_exp2(m_run - mn);  // exp2(-inf) = 0 on the first tile
     float ps = 0.f;
     uint32_t pb[2][8];  // P^T as packed bf16 pairs, accumulator order
@@ -222,7 +247,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
     }
-    m_run = mn;
+    m_run = mx_run;
     // ---- O^T += V^T P^T over 4 k-steps of 16 keys: step s uses accumulator half t = s/2,
     //      registers 8*(s%2) .. +7, i.e. keys rho = 16s + 4*half + {0..3} and 16s + 8 + 4*half + {0..3}
 #pragma unroll
@@ -257,11 +282,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   bf16_t* L0 = fp_smem;
   bf16_t* L1 = fp_smem + TILE_ELEMS;
   Regs A, B;
-  load(A, 0);
-  load(B, 1);
+  load(A, kt0);
+  load(B, kt0 + 1);
   stage(A, L0);
   __syncthreads();
-  for (int kt = 0; kt < ntiles; kt += 2) {
+  for (int kt = kt0; kt < kt1; kt += 2) {
     load(A, kt + 2);
     math(L0, kt);
     stage(B, L1);
@@ -271,7 +296,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     stage(A, L0);
     __syncthreads();
   }
-  // ---- normalise and store bf16: O^T[dim][row], dim = 32 i + (r&3) + 8 (r>>2) + 4 half
+  // ---- O^T[dim][row], dim = 32 i + (r&3) + 8 (r>>2) + 4 half
+  if (a.ns > 1) {  // this run's part: O, row max and row sum in fp32
+    if (qvalid) {
+      const size_t pr = ((size_t)blockIdx.z * T + tq) * a.n_heads + h;
+      float* op = a.ws + pr * HD;
+#pragma unroll
+      for (int i = 0; i < OT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4)
+          *(float4*)(op + i * 32 + 8 * (r >> 2) + 4 * half) = make_float4(o[i][r], o[i][r + 1], o[i][r + 2], o[i][r + 3]);
+      if (half == 0) *(float2*)(a.ws + (size_t)a.ns * T * a.n_heads * HD + pr * 2) = make_float2(m_run, l_run);
+    }
+    return;
+  }
+  // ---- normalise and store bf16
   if (qvalid) {
     const float inv = (F8 ? a.kv_scale_v : 1.f) / l_run;
     bf16_t* op = a.out + (size_t)tq * a.ldo + (size_t)h * HD;
@@ -286,16 +325,65 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 }
 
+// One wave per (token, head): its runs' O added up by their row maxima, normalised, stored as bf16.
+// Bound by the partials' bytes (300 tokens, 32 heads of 128, 6 runs: 30 MB, most of them still cached).
+template <int HD>
+__global__ void __launch_bounds__(256) attn_prefill_combine(AttnPrefillArgs a, int BQ, float vscale) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int rows = a.T * a.n_heads;
+  if (row >= rows) return;
+  const int t = row / a.n_heads, h = row - t * a.n_heads;
+  const FpRun r0 = fp_run(a.start, a.T, t - t % BQ, BQ, a.ns, 0);
+  const int ntiles = (a.start + min(a.T, t - t % BQ + BQ) - 1) / FP_KT + 1;
+  const int n = (ntiles + r0.kt1 - 1) / r0.kt1;  // runs that hold tiles (r0.kt1: tiles of a run)
+  const float* ml = a.ws + (size_t)a.ns * rows * HD;
+  float M = -INFINITY;
+  for (int z = 0; z < n; ++z) M = fmaxf(M, ml[((size_t)z * rows + row) * 2]);
+  constexpr int V = HD / 64;
+  float L = 0.f, acc[V] = {};
+#pragma unroll 4
+  for (int z = 0; z < n; ++z) {
+    const size_t pr = (size_t)z * rows + row;
+    const float2 p = *(const float2*)(ml + pr * 2);
+    const float w = raw_exp2(p.x - M);
+    L += w * p.y;
+    const float* op = a.ws + pr * HD + lane * V;
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc[j] += w * op[j];
+  }
+  const float inv = vscale / L;
+  bf16_t* out = a.out + (size_t)t * a.ldo + (size_t)h * HD + lane * V;
+  if constexpr (V == 2) *(uint32_t*)out = pk_bf16(acc[0] * inv, acc[1] * inv);
+  else *out = f32_to_bf16(acc[0] * inv);
+}
+
 bool attn_prefill_supports(int n_heads, int n_kv_heads, int head_dim) {
   if (n_kv_heads <= 0 || n_heads % n_kv_heads) return false;
   const int G = n_heads / n_kv_heads;
   return (head_dim == 64 || head_dim == 128) && (G == 1 || G == 2 || G == 4 || G == 8);
 }
 
+// Workgroups that a launch split over the keys has at most: two per CU (the two LDS tile buffers), and
+// one more wave of them would only lengthen the tail.
+constexpr int FP_WG = 512;
+// Tiles of a run at the least: below, the partials' traffic and the second launch cost what the run saves.
+constexpr int FP_RUN = 8;
+
+static int prefill_runs(const AttnPrefillArgs& a, int BQ) {
+  const int wg = (a.T + BQ - 1) / BQ * a.n_kv_heads, ntiles = (a.start + a.T - 1) / FP_KT + 1;
+  const int ns = std::min(std::min(FP_WG, 2 * device_cu_count()) / wg, ntiles / FP_RUN);
+  const size_t need = (size_t)ns * a.T * a.n_heads * (a.head_dim + 2) * sizeof(float);
+  return ns > 1 && a.ws && need <= a.ws_bytes ? ns : 1;
+}
+
+// FP_WG workgroups of 128 rows each, O and (max, sum) in fp32
+size_t attn_prefill_ws_bytes(int head_dim) { return (size_t)FP_WG * 128 * (head_dim + 2) * sizeof(float); }
+
 template <int HD, bool F8>
-static void prefill_hd(const AttnPrefillArgs& a, int G, hipStream_t st) {
+static void prefill_hd(AttnPrefillArgs a, int G, hipStream_t st) {
   const int BQ = 128 / G;
-  dim3 grid((a.T + BQ - 1) / BQ, a.n_kv_heads);
+  a.ns = prefill_runs(a, BQ);
+  dim3 grid((a.T + BQ - 1) / BQ, a.n_kv_heads, a.ns);
   const size_t lds = (size_t)2 * FP_KT * ((HD + 8) + (HD + 32)) * sizeof(bf16_t);  // two K|V tile buffers
   switch (G) {
     case 1: hipLaunchKernelGGL((attn_prefill_kernel<HD, 1, F8>), grid, dim3(256), lds, st, a); break;
@@ -304,6 +392,9 @@ static void prefill_hd(const AttnPrefillArgs& a, int G, hipStream_t st) {
     case 8: hipLaunchKernelGGL((attn_prefill_kernel<HD, 8, F8>), grid, dim3(256), lds, st, a); break;
     default: throw std::runtime_error("attn_prefill: unsupported GQA group size");
   }
+  if (a.ns > 1)
+    hipLaunchKernelGGL((attn_prefill_combine<HD>), dim3((a.T * a.n_heads + 3) / 4), dim3(256), 0, st, a, BQ,
+                       F8 ? a.kv_scale_v : 1.f);
 }
 
 void launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t st) {

@@ -138,7 +138,11 @@ struct AttnPrefillArgs {
   int ldo;
   int kv_fp8 = 0;          // fp8 e4m3 pool: value = code * kv_scale_{k,v}
   float kv_scale_k = 1.f, kv_scale_v = 1.f;
+  float* ws = nullptr;     // workspace of launches split over the keys; null: none is split
+  size_t ws_bytes = 0;
+  int ns = 1;              // runs over the keys (the launcher's choice)
 };
+size_t attn_prefill_ws_bytes(int head_dim);  // enough for every launch that is split
 void launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t st);
 bool attn_prefill_supports(int n_heads, int n_kv_heads, int head_dim);  // keys per workgroup the launcher picks
 

@@ -805,6 +805,48 @@ def test_attention_prefill_causal(E, H, Hkv, hd, start, T, shuffle):
     assert err < 3e-2, err
 
 
+@pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (16, 8, 128)])
+@pytest.mark.parametrize("start,T", [(1023, 1), (960, 64), (1100, 37), (3777, 300), (961, 129), (4000, 31)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_attention_prefill_split_over_keys(E, H, Hkv, hd, start, T, fp8):
+    """a few new tokens behind many cached ones: the keys in runs, added up by the second launch -- against
+    float64, and no further from it than the launch in one run (a quarter more: other roundings of P)"""
+    max_ctx, slot, slots, G = 4224, 1, 2, H // Hkv
+    g = torch.Generator().manual_seed(start + T)
+    kc, vc = torch.randn(slots, Hkv, max_ctx, hd, generator=g) * 0.5, torch.randn(slots, Hkv, max_ctx, hd, generator=g)
+    sk, sv = (0.03, 0.04) if fp8 else (1.0, 1.0)
+    if fp8:
+        (kc, kd), (vc, vd) = fp8_codes(kc, sk), fp8_codes(vc, sv)
+    else:
+        kc, vc = kc.to(torch.bfloat16), vc.to(torch.bfloat16)
+        kd, vd = kc.float(), vc.float()
+    kp, bt = paged_cache(kc, True, seed=5)
+    vp, _ = paged_cache(vc, True, seed=5)
+    kp, vp, bt = kp.cuda(), vp.cuda(), bt.cuda()
+    q = torch.randn(T, H, hd, generator=g).cuda()
+    n = E.attn_prefill_ws_bytes(hd)
+    ws = torch.full((n // 4,), float("nan"), device="cuda")
+    scale, got = 1 / math.sqrt(hd), []
+    for w in (0, ws.data_ptr()):
+        out = torch.zeros(T, H * hd, dtype=torch.bfloat16, device="cuda")
+        E.attn_prefill(q.data_ptr(), kp.data_ptr(), vp.data_ptr(), slot, start, T, H, Hkv, hd, max_ctx, scale, out.data_ptr(),
+                       H * hd, stream(), bt.data_ptr(), kv_fp8=int(fp8), k_scale=sk, v_scale=sv, ws=w, ws_bytes=n if w else 0)
+        torch.cuda.synchronize()
+        got.append(out.double())
+    assert bool(torch.isfinite(ws).any())  # (the second launch was a split one)
+    L, f = start + T, scale * 1.4426950408889634 * sk
+    k, v = kd[slot, :, :L].cuda().double(), vd[slot, :, :L].cuda().double()
+    qq = (q * f).to(torch.bfloat16).double() / (1.4426950408889634 * sk)  # (rounded where the kernel rounds it)
+    ref = torch.empty(T, H, hd, dtype=torch.float64, device="cuda")
+    dead = torch.arange(L, device="cuda")[None, :] > torch.arange(start, L, device="cuda")[:, None]
+    for h in range(H):
+        s = (qq[:, h] @ k[h // G].T.contiguous()).masked_fill(dead, float("-inf"))
+        ref[:, h] = torch.softmax(s, -1) @ v[h // G]
+    one, split = ((y - ref.reshape(T, -1)).norm() / ref.norm() for y in got)
+    # 2^-9 on P and on the output, either of them rounded once
+    assert split < 2 ** -8 and split < 1.25 * one, (float(one), float(split))
+
+
 # ---- skinny (M <= 64) batched-decode GEMM: weights streamed into MFMA operands ---------------------
 @pytest.mark.parametrize("t", QTS)
 @pytest.mark.parametrize("M", [2, 16, 33, 64])
