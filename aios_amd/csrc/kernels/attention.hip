@@ -1,19 +1,10 @@
-// Split-K flash-decode GQA attention over the bf16 KV cache (decode shape),
+// Split-K flash-decode GQA attention over the paged KV cache (decode shape),
 // with the log-sum-exp combine fused in (last-arriving workgroup per (row, kv-head)).
 //
-// grid = (roles, 1, B), 512 threads (8 waves); every workgroup picks its role from seq_len (see
-// attn_decode_kernel).  The context is cut into 128-key passes (16 keys per wave); every
-// workgroup owns two passes at a time with ALL of their K and V loads issued up front (buffers A
-// and B), so up to 256 keys cost one memory round trip: P = ceil(passes / 2) workgroups per
-// (row, head set), capped by the grid (workgroups then loop, the next pass's loads issued while
-// the current one is scored).  At a 153-key context this is one workgroup per query head with
-// no combine; at 4k keys up to 32 workgroups per KV head.  (Round 1 walked up to three 64-key
-// passes serially in one 4-wave workgroup: 7.8 us per layer at 153 keys.)
-//
-// Inside a pass every lane loads 16 B = 8 dims of a key (LPK = hd/8 lanes per key).  Each WAVE
-// keeps its own online-softmax state (m, l, o) for the G = H/Hkv query heads of the group --
-// scores are reduced over the LPK lanes of a key with DPP (no LDS), and no workgroup barrier is
-// needed until the eight waves merge their states in LDS at the end.
+// grid = (roles, 1, B), 512 threads (8 waves).  The context is cut into 32-key tiles, dealt over the
+// waves of the P workgroups of a (row, KV head); a wave keeps its own online-softmax state for the KV head's
+// query heads (attn_core in attn_decode.h).  Short contexts of small batches: a workgroup per query head, without a
+// combine (attn_short).
 //
 // Combine: with more than one active workgroup each writes its partial (o, m, l) with
 // write-through (sc1, agent scope) stores, drains them (s_waitcnt vmcnt(0)), and after a
@@ -25,25 +16,24 @@
 
 namespace aios {
 
+// (head_dim 64: two workgroups to a CU, 128 registers; 128: the tiles in flight take the register file)
 template <int HD, int G, bool F8>
-__global__ void __launch_bounds__(512) attn_decode_kernel(AttnDecodeArgs a, AttnSplit sp_) {
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 4 : 2))) attn_decode_kernel(AttnDecodeArgs a, AttnSplit s) {
   kernarg_warm<sizeof(AttnDecodeArgs) + sizeof(AttnSplit)>();
-  attn_role<HD, G, F8>(a, sp_, blockIdx.x);
+  attn_role<HD, G, F8>(a, s, blockIdx.x);
 }
 
 template <int HD, bool F8>
 static void launch_hd(const AttnDecodeArgs& a, int G, hipStream_t st) {
   AttnSplit sp;
-  const int nwg = attn_plan(a, G, sp);
-  sp.xcd = attn_env_int("AIOS_ATTN_XCD", 1);  // XCD-aware short-mode roles (0: the plain mapping)
-  sp.n_attn = nwg;
-  dim3 grid(nwg, 1, a.B);
+  const dim3 grid(attn_plan(a, G, sp), 1, a.B), block(512);
+  constexpr int lds = at_lds_bytes<HD>();
   switch (G) {
-    case 1: hipLaunchKernelGGL((attn_decode_kernel<HD, 1, F8>), grid, dim3(512), 0, st, a, sp); break;
-    case 2: hipLaunchKernelGGL((attn_decode_kernel<HD, 2, F8>), grid, dim3(512), 0, st, a, sp); break;
-    case 4: hipLaunchKernelGGL((attn_decode_kernel<HD, 4, F8>), grid, dim3(512), 0, st, a, sp); break;
-    case 5: hipLaunchKernelGGL((attn_decode_kernel<HD, 5, F8>), grid, dim3(512), 0, st, a, sp); break;
-    case 8: hipLaunchKernelGGL((attn_decode_kernel<HD, 8, F8>), grid, dim3(512), 0, st, a, sp); break;
+    case 1: hipLaunchKernelGGL((attn_decode_kernel<HD, 1, F8>), grid, block, lds, st, a, sp); break;
+    case 2: hipLaunchKernelGGL((attn_decode_kernel<HD, 2, F8>), grid, block, lds, st, a, sp); break;
+    case 4: hipLaunchKernelGGL((attn_decode_kernel<HD, 4, F8>), grid, block, lds, st, a, sp); break;
+    case 5: hipLaunchKernelGGL((attn_decode_kernel<HD, 5, F8>), grid, block, lds, st, a, sp); break;
+    case 8: hipLaunchKernelGGL((attn_decode_kernel<HD, 8, F8>), grid, block, lds, st, a, sp); break;
     default: throw std::runtime_error("attn_decode: unsupported GQA group size " + std::to_string(G));
   }
 }

@@ -14,6 +14,9 @@
 
 namespace aios {
 
+// the value of x's leading bf16
+__device__ __forceinline__ float bf16_part(float x) { return __uint_as_float(pk_bf16(x, 0.f) << 16); }
+
 __device__ __forceinline__ void st_wt(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -34,9 +37,9 @@ __device__ __forceinline__ float group_sum(float v) {
   if constexpr (N == 16) v += dpp<0x140>(v);  // row_mirror: lane i <-> 15-i within 16
   return v;
 }
-// op(v[lane], v[lane ^ OFF]) for OFF = 8, 16, 32 without the LDS crossbar: DPP row rotate for 8;
-// for 16 / 32 the gfx950 v_permlane16/32_swap of v with itself returns the lower and the upper
-// row of every pair in r[0] / r[1] on all lanes, so op(r[0], r[1]) needs no lane select
+// op(v[lane], v[lane ^ OFF]) for OFF = 8, 16, 32 without the LDS crossbar: DPP row rotate for 8; the gfx950
+// v_permlane16/32_swap of v with itself returns the lower and the upper row of every pair in r[0] / r[1]
+// on all lanes, so op(r[0], r[1]) needs no lane select
 template <int OFF, typename Op>
 __device__ __forceinline__ float xlane_op(float v, Op op) {
   if constexpr (OFF == 8) {
@@ -65,6 +68,12 @@ __device__ __forceinline__ float keys_sum(float v) {
   return xlane_op<32>(v, OpAdd{});
 }
 
+// max / sum over the four 16-lane quarters of a wave (lanes of equal column)
+template <typename Op>
+__device__ __forceinline__ float quarters(float v, Op op) {
+  return xlane_op<32>(xlane_op<16>(v, op), op);
+}
+
 constexpr float kLog2e = 1.4426950408889634f;
 // masked-key score / empty-state max: finite, so exp2(kNeg - m) underflows to 0 and
 // exp2(kNeg - kNeg) = 1 without -inf compares on the hot path
@@ -73,9 +82,17 @@ constexpr float kNeg = -1e30f;
 // adds a range-scaling compare + 2 selects per call
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-__device__ __forceinline__ uint4 ld_nt16(const bf16_t* p) {
-  const gu32x4 v = __builtin_nontemporal_load((const gu32x4*)p);
-  return make_uint4(v[0], v[1], v[2], v[3]);
+typedef short av4i16 __attribute__((ext_vector_type(4)));
+typedef short av8i16 __attribute__((ext_vector_type(8)));
+
+// fp8 KV (OCP e4m3): 8 codes -> 8 bf16 (exact)
+__device__ __forceinline__ gu32x4 fp8x8_bf16x8(uint32_t w0, uint32_t w1) {
+  gu32x4 o;
+  o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, false));
+  o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, true));
+  o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, false));
+  o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, true));
+  return o;
 }
 
 __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
@@ -83,10 +100,6 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
 }
 
 typedef unsigned int gu32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint2 ld_nt8(const uint8_t* p) {
-  const gu32x2 v = __builtin_nontemporal_load((const gu32x2*)p);
-  return make_uint2(v[0], v[1]);
-}
 // fp8 KV (OCP e4m3): 2 codes (bytes 2*hi, 2*hi+1 of w) -> a bf16 pair (one v_cvt_scalef32_pk_bf16_fp8)
 template <bool HI>
 __device__ __forceinline__ uint32_t fp8x2_bf16x2(uint32_t w) {
@@ -98,249 +111,282 @@ __device__ __forceinline__ gf32x2 fp8x2_f32x2(uint32_t w) {
   return __builtin_amdgcn_cvt_pk_f32_fp8((int)w, HI);
 }
 
-// One workgroup's share: heads [h0, h0 + G) of KV head kvh, keys of the passes sp, sp + P, ...
-// (P active workgroups per (row, head set); counters indexed by `ci`).  `ppw` = passes per
-// workgroup the split aims for (1: more workgroups, each one 128-key pass; 2: both buffers).
+constexpr int AT_NW = 8;    // waves per workgroup
+// descriptor of n raw bytes at p (both uniform over the wave)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const uint8_t* p, int n) {
+  const uint64_t u = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), (short)0, n, 0x00020000);
+}
+constexpr int AT_TK = 32;   // keys per tile: one wave's unit of work
+// LDS row (bytes) of a wave's V tile: rows 32 B apart mod 256, so the 8 rows x 32 B that half a wave's
+// transposed read takes fall on distinct banks
+template <int HD>
+constexpr int at_vrow() { return HD * 2 + 32; }
+template <int HD>
+constexpr int at_lds_bytes() { return AT_NW * AT_TK * at_vrow<HD>(); }
+
+// One workgroup's share: the G query heads of KV head kvh over the 32-key tiles of P workgroups x 8 waves,
+// dealt wave by wave (tile t to wave t mod 8 P: 32 keys is also the granularity of the balance).
 //
-// VALU diet (the kernel is VALU-bound per CU once its loads are in flight): q . k runs on
-// v_dot2_f32_bf16 against q pre-rounded to bf16 pairs (4 instructions per 8 dims and head, as the
-// MFMA prefill path rounds q), P . V on packed v_pk_fma_f32 with the probabilities in fp32.
-// F8: the pool holds fp8 e4m3 codes (EngineConfig::kv_fp8): K converted to bf16 pairs for the same
-// v_dot2 (the layer's K scale folded into q), V to fp32 pairs for the P.V FMAs (its V scale applied to
-// the output).  At head_dim 128 a lane takes 16 dims (16 bytes: the bf16 path's load width -- with 8
-// dims per lane the fp8 kernel issued as many load instructions for half the bytes and measured only
-// 3 % faster than bf16 at 32k keys, latency- not byte-bound); head_dim 64 keeps 8 dims (8 bytes).
-#ifndef AIOS_ATTN_RESCALE_SKIP
-#define AIOS_ATTN_RESCALE_SKIP 1
-#endif
+// Per tile, on the matrix cores:
+//   S^T[key][c] = K Q^T   (16x16x32, K rows from global memory to the A operand's registers as they are).  Column
+//                         c holds head c mod GP (GP = 4 or 8 >= G): every head's scores, and with them its
+//                         probabilities in fp32, stand in 16 / GP columns.
+//   O^T[dim][c] += V^T P^T   Each of a head's columns multiplies another bf16 part of the same probability (p's
+//                         leading 8 bits, the next 8, the last 8): the three products' sum has p in all its
+//                         24 bits, at no matrix instruction more for GP = 4 (two passes for GP = 8).  P^T comes
+//                         from the S^T registers, its k order with it; V goes through a wave's own LDS tile
+//                         (row-major in, ds_read_b64_tr_b16 out: no barrier, a wave's LDS operations are in order).
+// The arithmetic of a tile is then ~100 VALU instructions a wave where dots and P.V on the VALU took ~900:
+// at 16000 fp8 keys a workgroup spent 10 us on 512 keys, against 3 us for its bytes.  Loads: two tiles per wave
+// in flight (registers), so 512 keys of a workgroup cost one memory round trip.
+// q is rounded to bf16 (scaled; fp8: by the layer's K scale too, V's scale on the output); scores, max, sum and
+// O in fp32.
 template <int HD, int G, bool F8 = false>
-__device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int kvh, int h0, int ci, int P_max,
-                                          int ppw, bool nt = false) {
-  constexpr int DPL = (F8 && HD == 128) ? 16 : 8;  // dims per lane
-  using KVT = typename std::conditional<F8 && DPL == 8, uint2, uint4>::type;
-  constexpr int ES = F8 ? 1 : 2;  // bytes per cached element
-  constexpr int NP = DPL / 2;     // bf16 / fp32 pairs per lane
-  constexpr int NW = 8;                // waves per workgroup
-  constexpr int LPK = HD / DPL;        // lanes per key
-  constexpr int KPS = 64 / LPK;        // keys per wave-instruction
-  constexpr int CH = 128;              // keys per workgroup pass
-  constexpr int KPW = CH / NW;         // keys per wave per pass
-  constexpr int STEPS = KPW / KPS;     // loads per lane per pass (each of K and V)
-  constexpr int NT = NW * 64;
-  __shared__ float s_o[NW][G][HD];
+__device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int kvh, int P_max) {
+  constexpr int GP = G <= 4 ? 4 : 8;
+  constexpr int NR = GP == 4 ? 1 : 2;       // passes over P's bf16 parts
+  constexpr int ES = F8 ? 1 : 2;            // bytes per cached element
+  constexpr int EL = 16 / ES;               // elements per 16-B load
+  constexpr int KL = HD / (4 * EL);         // K loads per lane and 16 keys
+  constexpr int VL = AT_TK * HD / EL / 64;  // V loads per lane and tile
+  constexpr int VPR = HD / EL;              // 16-B pieces of a V row
+  constexpr int DT = HD / 16;               // O^T tiles
+  constexpr int VROW = at_vrow<HD>();
+  constexpr int NW = AT_NW, NT = NW * 64;
+  extern __shared__ __attribute__((aligned(16))) uint8_t at_smem[];
+  float (*s_o)[G][HD] = (float (*)[G][HD])at_smem;  // (the merge; after the V tiles)
+  static_assert(sizeof(float) * NW * G * HD <= at_lds_bytes<HD>(), "merge buffer");
   __shared__ float s_m[NW][G], s_l[NW][G];
   __shared__ int s_last;
 
-  const int b = blockIdx.z;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int ksub = lane / LPK, dsl = lane % LPK;
-  // probe stamps (a.ts, null in production: one scalar compare per site): 0 entry, 1 seq_len known,
-  // 2 first pass computed (its K/V landed), 3 waves merged, 4 partial published + ticket, 5 (m, l)
-  // weights ready (last arriver), 6 done
-  // (probe builds only, -DAIOS_ATTN_PROBES=1 / AIOS_BUILD_PROBES=1: a branch per stamp site in the
-  // pass loop costs production launches, as the GEMVs' probe branches did)
+  const int b = blockIdx.z, h0 = kvh * G, ci = h0;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int col = lane & 15, q4 = lane >> 4;
+  // probe stamps (a.ts; probe builds only, -DAIOS_ATTN_PROBES=1): 0 entry, 1 seq_len known, 2 first tile
+  // computed (its K/V landed), 3 waves merged, 4 partial published + ticket, 5 (m, l) weights ready (last
+  // arriver), 6 done
   auto stamp = [&](int k) __attribute__((always_inline)) {
     if (AIOS_ATTN_PROBES && a.ts && threadIdx.x == 0)
       a.ts[((size_t)blockIdx.z * gridDim.x + blockIdx.x) * 8 + k] = __builtin_amdgcn_s_memrealtime();
   };
   stamp(0);
-  static_assert(CH == KV_BLOCK, "one decode pass = one paged KV block");
-  const int slot = a.slot ? a.slot[b] : b;
-  // paged KV: pass c reads physical block bt[c]; a row-indexed table (bt_rows) is looked up
-  // without waiting for slot[b], so its load overlaps the seq_len / slot loads
+  // q first: everything after waits for older loads only, and the tiles below are the youngest
+  constexpr int KS = HD / 32;
+  float4 qr[KS][2];
+  {
+    const float* qp = a.q + ((size_t)b * a.n_heads + h0 + min(col & (GP - 1), G - 1)) * HD;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      // bf16: element 32 s + 8 q4; fp8: a 16-element K piece serves two steps
+      const float* x = qp + (F8 ? 64 * (s >> 1) + 16 * q4 + 8 * (s & 1) : 32 * s + 8 * q4);
+      qr[s][0] = *(const float4*)x;
+      qr[s][1] = *(const float4*)(x + 4);
+    }
+  }
+  // the row's numbers through the scalar cache (uniform addresses; written by earlier launches), requested together
+  using cint = const __attribute__((address_space(4))) int*;
+  // paged KV: tile t lies in block bt[t / 4]
+  static_assert(KV_BLOCK == 4 * AT_TK, "four tiles per paged KV block");
   const int maxb = a.max_ctx / KV_BLOCK;
-  const int* btr = a.block_table ? a.block_table + (size_t)(a.bt_rows ? b : slot) * maxb : nullptr;
   const size_t blk_stride = (size_t)a.n_kv_heads * KV_BLOCK * HD;
-  const int koff = wave * KPW + ksub;  // this lane's key within a pass (+ s * KPS)
-  const uint8_t* kc = (const uint8_t*)a.k_cache + ((size_t)kvh * KV_BLOCK * HD + (size_t)koff * HD + dsl * DPL) * ES;
-  const uint8_t* vc = (const uint8_t*)a.v_cache + ((size_t)kvh * KV_BLOCK * HD + (size_t)koff * HD + dsl * DPL) * ES;
-  const int cmax = maxb - 1;           // last chunk with valid memory
-
-  const int len = a.seq_len[b];
-  const int nchunk = (len + CH - 1) / CH;
-  const int P = max(1, min((nchunk + ppw - 1) / ppw, P_max));
-  if (sp >= P) return;  // uniform: this workgroup has no chunk, issues no K/V traffic
+  const int len = ((cint)a.seq_len)[b];
+  const int slot = ((cint)(a.slot ? a.slot : a.seq_len))[b];  // (no slots: row b; the value read is not used)
+  const int row = a.slot ? slot : b;
+  const bool paged = a.block_table != nullptr;
+  const cint btr = (cint)(a.block_table + (size_t)(a.bt_rows ? b : row) * maxb);
+  const int ntile = (len + AT_TK - 1) / AT_TK;
+  // tiles go to the P workgroups in turn, and in a workgroup to its waves.  From 9 tiles up as many workgroups as have
+  // 4 tiles: what a CU alone can draw from memory (~40 B/ns) bounds a short launch more than the combine does
+  const int P = ntile <= NW ? 1 : max(1, min((ntile + 3) / 4, P_max));
+  if (sp >= P) return;  // uniform: this workgroup has no tile, issues no K/V traffic
   stamp(1);
 
-  // two passes in flight per workgroup: buffers A and B (static, so they stay in VGPRs)
-  KVT kA[STEPS], vA[STEPS], kB[STEPS], vB[STEPS];
-  const bool tail = a.kv_tail != 0;
-  auto ld = [&](const uint8_t* p) __attribute__((always_inline)) { return *(const KVT*)p; };
-  auto ld_nt = [&](const uint8_t* p) __attribute__((always_inline)) {
-    if constexpr (F8 && DPL == 8) return ld_nt8(p);
-    else return ld_nt16((const bf16_t*)p);
+  struct Tile {
+    gu32x4 k[2][KL], v[VL];
+    size_t base;  // of the tile in its pool, bytes
+    int bytes;    // of its live keys
   };
-  auto issue = [&](KVT (&kr)[STEPS], KVT (&vr)[STEPS], int chunk) __attribute__((always_inline)) {
-    const int c = min(chunk, cmax);  // clamped: always a mapped block
-    const size_t base = (size_t)(btr ? btr[c] : slot * maxb + c) * blk_stride * ES;  // (bytes)
-    if (tail && (chunk + 1) * CH > len) {
-      // the context's last, partly filled block: only the lanes of live keys load (a 153-key context
-      // fetched 2 x 64 KB for 25 keys of its second block); dead keys hold zeros (scores masked, V x 0)
-      const int k0 = chunk * CH + koff;
+  Tile tA, tB;
+  // this lane's 16-B pieces: K of key (16 j + col): elements 4 EL i + EL q4 ..; V piece lane + 64 i, row-major
+  const uint32_t koff = (uint32_t)(col * HD + q4 * EL) * ES, voff = (uint32_t)lane * 16;
+  const size_t hoff = (size_t)kvh * KV_BLOCK * HD * ES;
+  // A tile is a buffer of its live keys' bytes: dead keys of the last tile, and all keys past it, read as zeros without
+  // a memory access.  So every path issues the same loads, and the wait for one tile's leaves the next one's in
+  // flight (a skipped issue made it wait for both); P = 0 meets no stale V either.
+  auto block_of = [&](int tile) __attribute__((always_inline)) { return paged ? btr[min(tile >> 2, maxb - 1)] : 0; };
+  auto place = [&](Tile& t, int tile, int blk) __attribute__((always_inline)) {
+    const int live = min(max(len - tile * AT_TK, 0), AT_TK);
+    t.bytes = __builtin_amdgcn_readfirstlane(live * HD * ES);
+    t.base = hoff + (live ? (size_t)(paged ? blk : row * maxb + (tile >> 2)) * blk_stride + (size_t)(tile & 3) * AT_TK * HD : 0) * ES;
+  };
+  // (streaming loads, aux 2: every K/V line is read once per launch)
+  auto issue_k = [&](Tile& t) __attribute__((always_inline)) {
+    const auto r = uniform_rsrc((const uint8_t*)a.k_cache + t.base, t.bytes);
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s) {
-        kr[s] = KVT{};
-        vr[s] = KVT{};
-        if (k0 + s * KPS < len) {
-          kr[s] = ld(kc + base + (size_t)s * KPS * HD * ES);
-          vr[s] = ld(vc + base + (size_t)s * KPS * HD * ES);
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < KL; ++i)
+        t.k[j][i] = __builtin_amdgcn_raw_buffer_load_b128(r, koff + (16 * j * HD + 4 * EL * i) * ES, 0, 2);
+  };
+  auto issue_v = [&](Tile& t) __attribute__((always_inline)) {
+    const auto r = uniform_rsrc((const uint8_t*)a.v_cache + t.base, t.bytes);
+#pragma unroll
+    for (int i = 0; i < VL; ++i) t.v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 1024 * i, 0, 2);
+  };
+  const int step = P * NW, t0 = sp + P * wave;
+  place(tA, t0, block_of(t0));
+  issue_k(tA);
+  issue_v(tA);
+  place(tB, t0 + step, block_of(t0 + step));
+  issue_k(tB);
+
+  // Q^T (B operand): lane (col, q4) holds head col mod GP's elements of the K pieces' order
+  gbf16x8 qf[KS];
+  {
+    const float qs = a.scale * kLog2e * (F8 ? a.kv_scale_k : 1.f);  // scores in the log2 domain: exp2 below
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const float4 x0 = qr[s][0], x1 = qr[s][1];
+      const uint4 u = make_uint4(pk_bf16(x0.x * qs, x0.y * qs), pk_bf16(x0.z * qs, x0.w * qs),
+                                 pk_bf16(x1.x * qs, x1.y * qs), pk_bf16(x1.z * qs, x1.w * qs));
+      __builtin_memcpy(&qf[s], &u, 16);
+    }
+  }
+  float m = kNeg, l = 0.f;  // column's running max; this lane's part of its sum
+  gf32x4 o[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i) o[i] = gf32x4{0.f, 0.f, 0.f, 0.f};
+  uint8_t* vt = at_smem + wave * (AT_TK * VROW);
+  // which part of P this lane's column multiplies (GP = 8: two passes, the leading and middle parts first)
+  const int term0 = GP == 4 ? col >> 2 : col >> 3;
+  const uint32_t sel0 = term0 == 0 ? ~0u : 0u, sel1 = term0 == 1 ? ~0u : 0u, sel2 = term0 == 2 ? ~0u : 0u;
+
+  // (after_s: what to issue once the K registers are free)
+  auto math = [&](Tile& t, int tile, auto after_s) __attribute__((always_inline)) {
+    const bool part = (tile + 1) * AT_TK > len;  // the context's last, partly filled tile
+    const int live = len - tile * AT_TK;
+    // ---- S^T: keys 16 j + 4 q4 + e of column col
+    gf32x4 st[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      st[j] = gf32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        gu32x4 w;
+        if constexpr (F8) w = fp8x8_bf16x8(t.k[j][s >> 1][2 * (s & 1)], t.k[j][s >> 1][2 * (s & 1) + 1]);
+        else w = t.k[j][s];
+        st[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8, w), qf[s], st[j], 0, 0, 0);
+      }
+    }
+    after_s();
+    // ---- online softmax of the tile's 32 keys per column
+    if (part) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (16 * j + 4 * q4 + e >= live) st[j][e] = kNeg;
+    }
+    float mx = st[0][0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) mx = fmaxf(mx, st[i >> 2][i & 3]);
+    const float mn = fmaxf(m, quarters(mx, OpMax{}));
+    // O is rescaled only when some column's max grew (wave-uniform)
+    if (__builtin_amdgcn_ballot_w64(mn > m)) {
+      const float alpha = fast_exp2(m - mn);
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[i][e] *= alpha;
+      m = mn;
+    }
+    float p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      p[i] = fast_exp2(st[i >> 2][i & 3] - m);
+      l += p[i];
+    }
+    // ---- P^T's bf16 parts: this column's term0 (NR passes: term0, term0 + 2)
+    gbf16x8 pf[NR];
+    {
+      float r0[8], r1[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float hi = bf16_part(p[i]);
+        const float rm = p[i] - hi;          // (exact)
+        const float lo = rm - bf16_part(rm);  // (exact: 8 bits left)
+        const uint32_t pu = __float_as_uint(p[i]), mu = __float_as_uint(rm), lu = __float_as_uint(lo);
+        if constexpr (GP == 4) {
+          r0[i] = __uint_as_float((pu & sel0) | (mu & sel1) | (lu & sel2));
+        } else {
+          r0[i] = __uint_as_float((pu & sel0) | (mu & sel1));
+          r1[i] = __uint_as_float(lu & sel0);
         }
       }
-    } else if (nt) {  // streaming (nt) policy: K/V lines read once per launch (long mode)
+      uint4 u = make_uint4(pk_bf16(r0[0], r0[1]), pk_bf16(r0[2], r0[3]), pk_bf16(r0[4], r0[5]), pk_bf16(r0[6], r0[7]));
+      __builtin_memcpy(&pf[0], &u, 16);
+      if constexpr (NR == 2) {
+        u = make_uint4(pk_bf16(r1[0], r1[1]), pk_bf16(r1[2], r1[3]), pk_bf16(r1[4], r1[5]), pk_bf16(r1[6], r1[7]));
+        __builtin_memcpy(&pf[1], &u, 16);
+      }
+    }
+    // ---- V to the wave's LDS tile, row-major
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s) kr[s] = ld_nt(kc + base + (size_t)s * KPS * HD * ES);
+    for (int i = 0; i < VL; ++i) {
+      const int p = lane + 64 * i, key = p / VPR, c = p % VPR;
+      if constexpr (F8) {
+        *(gu32x4*)(vt + key * VROW + c * 32) = fp8x8_bf16x8(t.v[i][0], t.v[i][1]);
+        *(gu32x4*)(vt + key * VROW + c * 32 + 16) = fp8x8_bf16x8(t.v[i][2], t.v[i][3]);
+      } else {
+        *(gu32x4*)(vt + key * VROW + c * 16) = t.v[i];
+      }
+    }
+    // ---- O^T += V^T P^T: k slots of quarter q4 are keys 4 q4 .. + 3 and 16 + 4 q4 .. + 3 (P^T's registers)
+    const uint8_t* va = vt + (4 * q4 + (col >> 2)) * VROW + (col & 3) * 8;
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s) vr[s] = ld_nt(vc + base + (size_t)s * KPS * HD * ES);
-    } else {
+    for (int i = 0; i < DT; ++i) {
+      using tp = __attribute__((address_space(3))) av4i16*;
+      const av4i16 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tp)(va + 32 * i));
+      const av4i16 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tp)(va + 16 * VROW + 32 * i));
+      const av8i16 xv = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+      const gbf16x8 vf = __builtin_bit_cast(gbf16x8, xv);
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s) kr[s] = ld(kc + base + (size_t)s * KPS * HD * ES);
-#pragma unroll
-      for (int s = 0; s < STEPS; ++s) vr[s] = ld(vc + base + (size_t)s * KPS * HD * ES);
+      for (int r = 0; r < NR; ++r) o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[r], o[i], 0, 0, 0);
     }
   };
-  issue(kA, vA, sp);
-  if (sp + P < nchunk) issue(kB, vB, sp + P);
-  const float qs = a.scale * kLog2e * (F8 ? a.kv_scale_k : 1.f);  // scores in the log2 domain: exp2 below
-  const float vs = F8 ? a.kv_scale_v : 1.f;                         // (fp8: V's scale, on the output)
-  uint32_t q2[G][NP];                 // q * scale as bf16 pairs
+  // a wave's registers hold one and a half tiles in flight: the next tile's V is requested when this one's K is used
+  for (int t = t0; t < ntile; t += 2 * step) {
+    math(tA, t, [&]() __attribute__((always_inline)) { issue_v(tB); });
+    if (t == t0) stamp(2);
+    place(tA, t + 2 * step, block_of(t + 2 * step));
+    issue_k(tA);
+    if (t + step >= ntile) break;
+    math(tB, t + step, [&]() __attribute__((always_inline)) { issue_v(tA); });
+    place(tB, t + 3 * step, block_of(t + 3 * step));
+    issue_k(tB);
+  }
+  // ---- a head's columns summed (row rotates within 16 lanes), then the 8 waves merged in LDS
+  l = quarters(l, OpAdd{});
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const float* qp = a.q + ((size_t)b * a.n_heads + h0 + g) * HD + dsl * DPL;
+  for (int i = 0; i < DT; ++i)
 #pragma unroll
-    for (int j = 0; j < DPL / 4; ++j) {
-      const float4 q0 = *(const float4*)(qp + 4 * j);
-      q2[g][2 * j] = pk_bf16(q0.x * qs, q0.y * qs);
-      q2[g][2 * j + 1] = pk_bf16(q0.z * qs, q0.w * qs);
+    for (int e = 0; e < 4; ++e) {
+      o[i][e] += dpp<0x128>(o[i][e]);                                // row_ror:8
+      if constexpr (GP == 4) o[i][e] += dpp<0x124>(o[i][e]);         // row_ror:4
+    }
+  __syncthreads();  // every wave is done with its V tile: the LDS is the merge's
+  if (col < G) {
+#pragma unroll
+    for (int i = 0; i < DT; ++i) *(float4*)&s_o[wave][col][16 * i + 4 * q4] = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
+    if (q4 == 0) {
+      s_m[wave][col] = m;
+      s_l[wave][col] = l;
     }
   }
-  float m[G], l[G];
-  gf32x2 o[G][NP];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = kNeg;
-    l[g] = 0.f;
-#pragma unroll
-    for (int i = 0; i < NP; ++i) o[g][i] = gf32x2{0.f, 0.f};
-  }
-  auto pass = [&](const KVT (&kr)[STEPS], const KVT (&vr)[STEPS], int c) __attribute__((always_inline)) {
-    // ---- scores of this lane's STEPS keys for the G heads (reduced over the key's LPK lanes)
-    float sc[STEPS][G];
-#pragma unroll
-    for (int s = 0; s < STEPS; ++s) {
-      const bool valid = c * CH + koff + s * KPS < len;
-      uint32_t kb[NP];
-      if constexpr (F8 && DPL == 16) {
-        const uint32_t w4[4] = {kr[s].x, kr[s].y, kr[s].z, kr[s].w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) { kb[2 * i] = fp8x2_bf16x2<false>(w4[i]); kb[2 * i + 1] = fp8x2_bf16x2<true>(w4[i]); }
-      } else if constexpr (F8) {
-        kb[0] = fp8x2_bf16x2<false>(kr[s].x); kb[1] = fp8x2_bf16x2<true>(kr[s].x);
-        kb[2] = fp8x2_bf16x2<false>(kr[s].y); kb[3] = fp8x2_bf16x2<true>(kr[s].y);
-      } else {
-        kb[0] = kr[s].x; kb[1] = kr[s].y; kb[2] = kr[s].z; kb[3] = kr[s].w;
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        float d = dot2_bf16(kb[0], q2[g][0], 0.f);
-#pragma unroll
-        for (int i = 1; i < NP; ++i) d = dot2_bf16(kb[i], q2[g][i], d);
-        d = group_sum<LPK>(d);
-        sc[s][g] = valid ? d : kNeg;
-      }
-    }
-    // ---- online softmax over this lane's keys (round 6: per key group -- the LPK lanes of a key share
-    // its score, so (m, l) are uniform over them; the cross-key-group max / sum, two 3-stage lane
-    // reductions per head and pass, move to the end of the pass loop: the fp8 long mode's passes are
-    // bound by their own VALU chain, profiles/long_context_r6.txt)
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      float mx = sc[0][g];
-#pragma unroll
-      for (int s = 1; s < STEPS; ++s) mx = fmaxf(mx, sc[s][g]);
-      const float mn = fmaxf(m[g], mx);
-      float ps = 0.f;
-#pragma unroll
-      for (int s = 0; s < STEPS; ++s) {
-        const float p = fast_exp2(sc[s][g] - mn);
-        sc[s][g] = p;
-        ps += p;
-      }
-      // rescale only when some lane's max grew (a wave-uniform branch: past the first passes of a long
-      // context the running max rarely moves, and the NP packed multiplies + exp2 per head were per pass)
-      if (AIOS_ATTN_RESCALE_SKIP == 0 || __builtin_amdgcn_ballot_w64(mn > m[g])) {
-        const float alpha = fast_exp2(m[g] - mn);
-        l[g] *= alpha;
-#pragma unroll
-        for (int i = 0; i < NP; ++i) o[g][i] *= alpha;
-      }
-      l[g] += ps;
-      m[g] = mn;
-    }
-    // ---- P.V (lane-local over its keys; merged across key groups and waves at the end)
-#pragma unroll
-    for (int s = 0; s < STEPS; ++s) {
-      gf32x2 vf[NP];
-      if constexpr (F8 && DPL == 16) {
-        const uint32_t w4[4] = {vr[s].x, vr[s].y, vr[s].z, vr[s].w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) { vf[2 * i] = fp8x2_f32x2<false>(w4[i]); vf[2 * i + 1] = fp8x2_f32x2<true>(w4[i]); }
-      } else if constexpr (F8) {
-        vf[0] = fp8x2_f32x2<false>(vr[s].x); vf[1] = fp8x2_f32x2<true>(vr[s].x);
-        vf[2] = fp8x2_f32x2<false>(vr[s].y); vf[3] = fp8x2_f32x2<true>(vr[s].y);
-      } else {
-        const uint32_t w[4] = {vr[s].x, vr[s].y, vr[s].z, vr[s].w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vf[i] = gf32x2{__uint_as_float(w[i] << 16), __uint_as_float(w[i] & 0xffff0000u)};
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const gf32x2 pp = gf32x2{sc[s][g], sc[s][g]};
-#pragma unroll
-        for (int i = 0; i < NP; ++i) o[g][i] = __builtin_elementwise_fma(pp, vf[i], o[g][i]);
-      }
-    }
-  };
-  for (int c = sp; c < nchunk; c += 2 * P) {
-    pass(kA, vA, c);
-    if (c == sp) stamp(2);
-    if (c + 2 * P < nchunk) issue(kA, vA, c + 2 * P);
-    if (c + P < nchunk) {
-      pass(kB, vB, c + P);
-      if (c + 3 * P < nchunk) issue(kB, vB, c + 3 * P);
-    }
-  }
-  // ---- merge the key groups of a wave (shuffles: their (m, l, o) rescaled to the wave's max), then the 8
-  // waves in LDS (one barrier)
-  float of[G][DPL];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const float M = keys_max<LPK>(m[g]);
-    const float w = fast_exp2(m[g] - M);
-    l[g] = keys_sum<LPK>(l[g] * w);
-    m[g] = M;
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      of[g][2 * i] = keys_sum<LPK>(o[g][i].x * w);
-      of[g][2 * i + 1] = keys_sum<LPK>(o[g][i].y * w);
-    }
-  }
-  if (ksub == 0) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      float4* dst = (float4*)&s_o[wave][g][dsl * DPL];
-#pragma unroll
-      for (int j = 0; j < DPL / 4; ++j) dst[j] = make_float4(of[g][4 * j], of[g][4 * j + 1], of[g][4 * j + 2], of[g][4 * j + 3]);
-    }
-  }
-  if (lane < G) {
-    // m/l are wave-uniform after keys_max/keys_sum; lane g publishes head g
-    float mv = m[0], lv = l[0];
-#pragma unroll
-    for (int g = 1; g < G; ++g)
-      if (lane == g) { mv = m[g]; lv = l[g]; }
-    s_m[wave][lane] = mv;
-    s_l[wave][lane] = lv;
-  }
+  const float vs = F8 ? a.kv_scale_v : 1.f;
   __syncthreads();
   stamp(3);
   const int nact = P;  // workgroups that arrive
@@ -491,57 +537,209 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   stamp(6);
 }
 
-// Up to ATTN_SPLIT_LEN keys the G query heads of a KV head are split over G workgroups (one head
-// each; the K/V re-reads hit L2): 4x less dot / softmax / P.V work per workgroup on the latency-
-// bound short contexts of agent turns.  Beyond that one workgroup set per (KV head, head set of
-// GL <= 4 query heads) computes its heads (the KV stream, not the arithmetic, dominates; GL = 4
-// keeps G = 8 groups in registers).  The grid is flat (one x-slot per role of the larger mode)
-// and each workgroup derives its role from seq_len, so a hipGraph-captured launch sized for
-// max_ctx carries no idle head-split grid (round-2 probe: 384 idle 512-thread workgroups cost
-// 4 us at a 256-key context).
-constexpr int ATTN_SPLIT_LEN = 512;
-template <int G>
-struct AttnGL { static constexpr int value = (G % 4 == 0) ? 4 : G; };
+// Contexts up to ATTN_SPLIT_LEN keys of a launch that leaves CUs idle: a workgroup per QUERY head walks all (<= 4)
+// 128-key passes, without a combine.  Its G workgroups per KV head read the same K and V (from L2 after the first,
+// see the roles below), so a launch this short is one memory round trip of 64 KB on each of n_heads CUs and little
+// else; attn_core's one workgroup per KV head then waits for a longer chain: 130 keys, 32 / 8 heads of 128: 5.2 us
+// here, 7.5 us there (4.0 and 4.9 us for 32 / 4 heads of 64); 500 keys of three rows: equal.
+// VALU: q . k on v_dot2_f32_bf16 (q rounded to bf16 pairs), P . V in fp32.  Every lane loads 16 B (fp8 at head_dim 64:
+// 8 B) of a key; two passes in flight.
+template <int HD, bool F8 = false>
+__device__ __forceinline__ void attn_short(const AttnDecodeArgs& a, int kvh, int h) {
+  constexpr int DPL = (F8 && HD == 128) ? 16 : 8;  // dims per lane
+  using KVT = typename std::conditional<F8 && DPL == 8, uint2, uint4>::type;
+  constexpr int ES = F8 ? 1 : 2;  // bytes per cached element
+  constexpr int NP = DPL / 2;     // bf16 / fp32 pairs per lane
+  constexpr int NW = AT_NW;
+  constexpr int LPK = HD / DPL;        // lanes per key
+  constexpr int KPS = 64 / LPK;        // keys per wave-instruction
+  constexpr int CH = 128;              // keys per pass
+  constexpr int KPW = CH / NW;         // keys per wave per pass
+  constexpr int STEPS = KPW / KPS;     // loads per lane per pass (each of K and V)
+  extern __shared__ __attribute__((aligned(16))) uint8_t at_smem[];
+  float (*s_o)[HD] = (float (*)[HD])at_smem;
+  __shared__ float s_m[NW], s_l[NW];
 
+  const int b = blockIdx.z;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int ksub = lane / LPK, dsl = lane % LPK;
+  static_assert(CH == KV_BLOCK, "one pass = one paged KV block");
+  const int slot = a.slot ? a.slot[b] : b;
+  const int maxb = a.max_ctx / KV_BLOCK;
+  const int* btr = a.block_table ? a.block_table + (size_t)(a.bt_rows ? b : slot) * maxb : nullptr;
+  const size_t blk_stride = (size_t)a.n_kv_heads * KV_BLOCK * HD;
+  const int koff = wave * KPW + ksub;  // this lane's key within a pass (+ s * KPS)
+  const uint8_t* kc = (const uint8_t*)a.k_cache + ((size_t)kvh * KV_BLOCK * HD + (size_t)koff * HD + dsl * DPL) * ES;
+  const uint8_t* vc = (const uint8_t*)a.v_cache + ((size_t)kvh * KV_BLOCK * HD + (size_t)koff * HD + dsl * DPL) * ES;
+  const int len = a.seq_len[b];
+  const int nchunk = (len + CH - 1) / CH;
+
+  KVT kA[STEPS], vA[STEPS], kB[STEPS], vB[STEPS];
+  auto ld = [&](const uint8_t* p) __attribute__((always_inline)) { return *(const KVT*)p; };
+  auto issue = [&](KVT (&kr)[STEPS], KVT (&vr)[STEPS], int c) __attribute__((always_inline)) {
+    const size_t base = (size_t)(btr ? btr[c] : slot * maxb + c) * blk_stride * ES;  // (bytes)
+    if ((c + 1) * CH > len) {
+      // the context's last, partly filled block: only the lanes of live keys load (a 153-key context
+      // fetched 2 x 64 KB for 25 keys of its second block); dead keys hold zeros (scores masked, V x 0)
+      const int k0 = c * CH + koff;
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) {
+        kr[s] = KVT{};
+        vr[s] = KVT{};
+        if (k0 + s * KPS < len) {
+          kr[s] = ld(kc + base + (size_t)s * KPS * HD * ES);
+          vr[s] = ld(vc + base + (size_t)s * KPS * HD * ES);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) kr[s] = ld(kc + base + (size_t)s * KPS * HD * ES);
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) vr[s] = ld(vc + base + (size_t)s * KPS * HD * ES);
+    }
+  };
+  issue(kA, vA, 0);
+  if (1 < nchunk) issue(kB, vB, 1);
+  const float qs = a.scale * kLog2e * (F8 ? a.kv_scale_k : 1.f);  // scores in the log2 domain: exp2 below
+  uint32_t q2[NP];                 // q * scale as bf16 pairs
+  {
+    const float* qp = a.q + ((size_t)b * a.n_heads + h) * HD + dsl * DPL;
+#pragma unroll
+    for (int j = 0; j < DPL / 4; ++j) {
+      const float4 q0 = *(const float4*)(qp + 4 * j);
+      q2[2 * j] = pk_bf16(q0.x * qs, q0.y * qs);
+      q2[2 * j + 1] = pk_bf16(q0.z * qs, q0.w * qs);
+    }
+  }
+  float m = kNeg, l = 0.f;  // per key group: the LPK lanes of a key share its score
+  gf32x2 o[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) o[i] = gf32x2{0.f, 0.f};
+  auto pass = [&](const KVT (&kr)[STEPS], const KVT (&vr)[STEPS], int c) __attribute__((always_inline)) {
+    float sc[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const bool valid = c * CH + koff + s * KPS < len;
+      uint32_t kb[NP];
+      if constexpr (F8 && DPL == 16) {
+        const uint32_t w4[4] = {kr[s].x, kr[s].y, kr[s].z, kr[s].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { kb[2 * i] = fp8x2_bf16x2<false>(w4[i]); kb[2 * i + 1] = fp8x2_bf16x2<true>(w4[i]); }
+      } else if constexpr (F8) {
+        kb[0] = fp8x2_bf16x2<false>(kr[s].x); kb[1] = fp8x2_bf16x2<true>(kr[s].x);
+        kb[2] = fp8x2_bf16x2<false>(kr[s].y); kb[3] = fp8x2_bf16x2<true>(kr[s].y);
+      } else {
+        kb[0] = kr[s].x; kb[1] = kr[s].y; kb[2] = kr[s].z; kb[3] = kr[s].w;
+      }
+      float d = dot2_bf16(kb[0], q2[0], 0.f);
+#pragma unroll
+      for (int i = 1; i < NP; ++i) d = dot2_bf16(kb[i], q2[i], d);
+      d = group_sum<LPK>(d);
+      sc[s] = valid ? d : kNeg;
+    }
+    float mx = sc[0];
+#pragma unroll
+    for (int s = 1; s < STEPS; ++s) mx = fmaxf(mx, sc[s]);
+    const float mn = fmaxf(m, mx);
+    float ps = 0.f;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      sc[s] = fast_exp2(sc[s] - mn);
+      ps += sc[s];
+    }
+    if (__builtin_amdgcn_ballot_w64(mn > m)) {  // (wave-uniform: some lane's max grew)
+      const float alpha = fast_exp2(m - mn);
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < NP; ++i) o[i] *= alpha;
+    }
+    l += ps;
+    m = mn;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      gf32x2 vf[NP];
+      if constexpr (F8 && DPL == 16) {
+        const uint32_t w4[4] = {vr[s].x, vr[s].y, vr[s].z, vr[s].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { vf[2 * i] = fp8x2_f32x2<false>(w4[i]); vf[2 * i + 1] = fp8x2_f32x2<true>(w4[i]); }
+      } else if constexpr (F8) {
+        vf[0] = fp8x2_f32x2<false>(vr[s].x); vf[1] = fp8x2_f32x2<true>(vr[s].x);
+        vf[2] = fp8x2_f32x2<false>(vr[s].y); vf[3] = fp8x2_f32x2<true>(vr[s].y);
+      } else {
+        const uint32_t w[4] = {vr[s].x, vr[s].y, vr[s].z, vr[s].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vf[i] = gf32x2{__uint_as_float(w[i] << 16), __uint_as_float(w[i] & 0xffff0000u)};
+      }
+      const gf32x2 pp = gf32x2{sc[s], sc[s]};
+#pragma unroll
+      for (int i = 0; i < NP; ++i) o[i] = __builtin_elementwise_fma(pp, vf[i], o[i]);
+    }
+  };
+  for (int c = 0; c < nchunk; c += 2) {
+    pass(kA, vA, c);
+    if (c + 2 < nchunk) issue(kA, vA, c + 2);
+    if (c + 1 < nchunk) {
+      pass(kB, vB, c + 1);
+      if (c + 3 < nchunk) issue(kB, vB, c + 3);
+    }
+  }
+  // ---- merge the key groups of a wave (their (m, l, o) rescaled to the wave's max), then the 8 waves in LDS
+  const float M = keys_max<LPK>(m), w = fast_exp2(m - M);
+  l = keys_sum<LPK>(l * w);
+  float of[DPL];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    of[2 * i] = keys_sum<LPK>(o[i].x * w);
+    of[2 * i + 1] = keys_sum<LPK>(o[i].y * w);
+  }
+  if (ksub == 0) {
+    float4* dst = (float4*)&s_o[wave][dsl * DPL];
+#pragma unroll
+    for (int j = 0; j < DPL / 4; ++j) dst[j] = make_float4(of[4 * j], of[4 * j + 1], of[4 * j + 2], of[4 * j + 3]);
+  }
+  if (lane == 0) {
+    s_m[wave] = M;
+    s_l[wave] = l;
+  }
+  __syncthreads();
+  const int d = threadIdx.x;
+  if (d >= HD) return;
+  float W = s_m[0];
+#pragma unroll
+  for (int v = 1; v < NW; ++v) W = fmaxf(W, s_m[v]);
+  float L = 0.f, acc = 0.f;
+#pragma unroll
+  for (int v = 0; v < NW; ++v) {
+    const float sw = fast_exp2(s_m[v] - W);
+    L += sw * s_l[v];
+    acc += sw * s_o[v][d];
+  }
+  if (F8) acc *= a.kv_scale_v;
+  const size_t oi = ((size_t)b * a.n_heads + h) * HD + d;
+  if (a.out16) a.out16[oi] = f32_to_bf16(acc / L);
+  else if (a.out_wt) st_wt(a.out + oi, acc / L);
+  else a.out[oi] = acc / L;
+}
+
+// The grid is flat (one x-slot per role of the larger form) and each workgroup derives its role from seq_len, so a
+// launch captured for max_ctx serves every context; workgroups without keys return at once.
+constexpr int ATTN_SPLIT_LEN = 512;
 struct AttnSplit {
-  int p_long;   // workgroups per (row, head set) in the long mode
-  int p_short;  // workgroups per (row, head) in the short mode
-  int ppw;      // passes per workgroup the split aims for
-  int n_attn;   // attention workgroups of the flat grid
-  int xcd;      // short mode: the G query heads of a KV head on one XCD (attention.hip)
+  int p;    // workgroups per (row, KV head) of attn_core
 };
 
-
-// workgroup wg's role in the flat grid (see attn_decode_kernel, attention.hip); returns with the
-// whole workgroup (every early exit inside is workgroup-uniform)
 template <int HD, int G, bool F8 = false>
-__device__ __forceinline__ void attn_role(const AttnDecodeArgs& a, const AttnSplit& sp_, int wg) {
-  const int len = a.seq_len[blockIdx.z];
-  if (G > 1 && len <= a.short_len) {
-    // XCD-aware roles: workgroups are dealt round-robin over the 8 XCDs (blockIdx % 8), so
-    // workgroup wg takes query head (wg % 8) * (H / 8) + (wg / 8) / P -- the G query heads of a KV
-    // head then run on one XCD and read its K/V from that XCD's L2 after the first miss (the plain
-    // mapping put them on G different XCDs: G MALL/HBM reads of every K/V line)
-    int h, sp;
-    if ((a.n_heads & 7) == 0 && sp_.xcd) {
-      if (wg >= a.n_heads * sp_.p_short) return;
-      const int j = wg >> 3;
-      h = (wg & 7) * (a.n_heads >> 3) + j / sp_.p_short;
-      sp = j % sp_.p_short;
-    } else {
-      h = wg / sp_.p_short;
-      sp = wg % sp_.p_short;
-    }
-    if (h >= a.n_heads) return;
-    attn_core<HD, 1, F8>(a, sp, h / G, h, h, sp_.p_short, sp_.ppw);
+__device__ __forceinline__ void attn_role(const AttnDecodeArgs& a, const AttnSplit& s, int wg) {
+  if (G > 1 && a.seq_len[blockIdx.z] <= a.short_len) {
+    // workgroups are dealt round-robin over the 8 XCDs (blockIdx % 8), so workgroup wg takes query head
+    // (wg % 8) * (H / 8) + wg / 8: the G query heads of a KV head then run on one XCD and read its K/V from that
+    // XCD's L2 after the first miss (the plain mapping put them on G different XCDs)
+    if (wg >= a.n_heads) return;
+    const int h = (a.n_heads & 7) == 0 ? (wg & 7) * (a.n_heads >> 3) + (wg >> 3) : wg;
+    attn_short<HD, F8>(a, h / G, h);
   } else {
-    constexpr int GL = AttnGL<G>::value;
-    const int hsi = wg / sp_.p_long, sp = wg % sp_.p_long;
-    if (hsi >= a.n_kv_heads * (G / GL)) return;
-    const int kvh = hsi / (G / GL), h0 = kvh * G + (hsi % (G / GL)) * GL;
-    // long mode: every K/V line is read by exactly one workgroup -> streaming loads (round 4,
-    // same box: --prompt 4000 546.9 -> 567.0 tok/s, 16000 467.6 -> 487.3)
-    attn_core<HD, GL, F8>(a, sp, kvh, h0, h0, sp_.p_long, sp_.ppw, a.kv_nt != 0);
+    if (wg >= a.n_kv_heads * s.p) return;
+    attn_core<HD, G, F8>(a, wg % s.p, wg / s.p, s.p);
   }
 }
 
@@ -551,37 +749,31 @@ inline int attn_env_int(const char* k, int dflt) {
 }
 
 int attn_decode_split(int max_ctx, int B, int n_kv_heads);
-// the launcher's defaults filled in (split, combine, K/V load policy, short-mode length)
+// the launcher's defaults filled in (split, combine)
 inline AttnDecodeArgs attn_resolve(const AttnDecodeArgs& a) {
   AttnDecodeArgs b = a;
   if (b.split <= 0) b.split = attn_decode_split(a.max_ctx, a.B, a.n_kv_heads);
   if (b.combine_trips == 0) b.combine_trips = attn_env_int("AIOS_ATTN_COMBINE", 1);
-  if (b.kv_nt < 0) b.kv_nt = attn_env_int("AIOS_ATTN_NT", 1);
-  if (b.kv_tail < 0) b.kv_tail = attn_env_int("AIOS_ATTN_TAIL", 1);
-  // Batched decode fills the chip with (row, KV head) workgroups on its own: from
-  // AIOS_ATTN_GROUPED_MIN such workgroups up, every context length takes the grouped mode (one
-  // K/V read for the G query heads of a KV head) instead of the per-query-head split that buys
-  // batch-1 latency with G x the K/V reads and workgroups
+  // The short form as long as its workgroups (a row's query heads) are resident at once, two to a CU at head_dim 64
+  // and one at 128 (registers); beyond, attn_core's (a row's KV heads): 12 rows of 450 keys, 32 / 8 heads of 128:
+  // 14.6 us short, 11.5 us core; 16 rows, 32 / 4 heads of 64: 7.5 and 8.1 us.  AIOS_ATTN_GROUPED_MIN=n: attn_core
+  // from n such workgroups up.
   if (b.short_len < 0) {
-    const int grouped_min = attn_env_int("AIOS_ATTN_GROUPED_MIN", 128);
-    b.short_len = (grouped_min > 0 && a.B * a.n_kv_heads >= grouped_min) ? 0 : ATTN_SPLIT_LEN;
+    const int grouped_min = attn_env_int("AIOS_ATTN_GROUPED_MIN", 0);
+    const bool core = grouped_min > 0 ? a.B * a.n_kv_heads >= grouped_min
+                                      : a.B * a.n_heads > device_cu_count() * (a.head_dim == 64 ? 2 : 1);
+    b.short_len = core ? 0 : ATTN_SPLIT_LEN;
   }
   return b;
 }
 
-// the launch shape for AttnDecodeArgs a (split already resolved): fills the split and returns the
-// flat workgroup count (one x-slot per role of the larger mode)
+// the launch shape for AttnDecodeArgs a (split already resolved): fills the split and returns the flat
+// workgroup count (one x-slot per role of the larger form)
 inline int attn_plan(const AttnDecodeArgs& a, int G, AttnSplit& sp) {
-  const int nch = std::max(1, a.max_ctx / 128);  // 128-key passes
-  sp.p_long = std::max(1, std::min(nch, a.split / ATTN_CHUNK));
-  // short mode: one workgroup per query head walks all (<= 4) passes -- the probe's best at
-  // <= 256 keys (a combine costs more than the second pass it would spread)
-  sp.p_short = std::max(1, std::min(4, attn_env_int("AIOS_ATTN_SHORT_P", 1)));
-  sp.ppw = std::max(1, std::min(2, attn_env_int("AIOS_ATTN_PPW", 1)));
-  if (sp.p_long > a.n_chunks || sp.p_long > 64 || sp.p_short > a.n_chunks)
+  const int nch = std::max(1, a.max_ctx / 128);
+  sp.p = std::max(1, std::min(nch, a.split / ATTN_CHUNK));
+  if (sp.p > a.n_chunks || sp.p > 64)
     throw std::runtime_error("attn_decode: more splits than partial buffers / 64");
-  const int GL = (G % 4 == 0) ? 4 : G;
-  sp.n_attn = std::max(a.n_kv_heads * (G / GL) * sp.p_long, G > 1 && a.short_len != 0 ? a.n_heads * sp.p_short : 0);
-  return std::max(a.n_kv_heads * (G / GL) * sp.p_long, G > 1 && a.short_len != 0 ? a.n_heads * sp.p_short : 0);
+  return std::max(a.n_kv_heads * sp.p, G > 1 && a.short_len != 0 ? a.n_heads : 0);
 }
 }  // namespace aios

@@ -109,11 +109,9 @@ struct AttnDecodeArgs {
   float* ml;               // [B][n_heads][n_chunks][2]
   float* out;              // [B][n_heads*hd]
   bf16_t* out16 = nullptr; // if set: the output as bf16 instead (the batched-decode GEMM's A operand)
-  int short_len = -1;      // contexts up to this many keys split by query head (-1: launcher decides)
+  int short_len = -1;      // contexts up to this many keys: a workgroup per query head (-1: launcher decides)
   int* counters;           // [B][n_kv_heads] arrival tickets, zero-initialised, self re-arming
   unsigned long long* ts = nullptr;  // probes: [grid][8] s_memrealtime phase stamps (tools/attn_probe.py --stamps)
-  int kv_nt = -1;          // long mode: K/V loads with the streaming (nt) policy (-1: AIOS_ATTN_NT, default 1)
-  int kv_tail = -1;        // last partial block: loads only for live keys (-1: AIOS_ATTN_TAIL, default 1)
   int combine_trips = 0;   // split-K combine: 0 = launcher (AIOS_ATTN_COMBINE, default one round trip), 2 = two
   int out_wt = 0;          // fp32 out with write-through (agent-scope) stores
   int kv_fp8 = 0;          // fp8 e4m3 pool: value = code * kv_scale_{k,v}

@@ -538,6 +538,52 @@ def test_attention_decode_fp8_kv(E, hd, H, Hkv, lens, max_ctx, grouped, monkeypa
         assert torch.allclose(out[b].cpu(), ref, atol=5e-4, rtol=5e-3), (b, (out[b].cpu() - ref).abs().max())
 
 
+@pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (16, 8, 128), (40, 8, 128), (64, 8, 128), (6, 3, 64)])
+@pytest.mark.parametrize("lens", [(1, 32, 33, 255), (256, 257, 288, 513), (31, 512, 1025, 4001), (2048, 2049), (4096,)])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("grouped", ["", "1"])  # "1": no form of its own for short contexts
+def test_attention_decode_tiles(E, H, Hkv, hd, lens, fp8, grouped, monkeypatch):
+    """edges of the 32-key tiles, of the waves' and workgroups' shares and of the short form, NaN in every dead key:
+    probabilities and sums in 32 bits (about 2^-22 each over at most 4096 terms; P in 16 bits would be 2^-9 off)"""
+    if grouped:
+        monkeypatch.setenv("AIOS_ATTN_GROUPED_MIN", grouped)
+    B, G, max_ctx = len(lens), H // Hkv, 4096
+    g = torch.Generator().manual_seed(sum(lens))
+    kc, vc = torch.randn(B, Hkv, max_ctx, hd, generator=g) * 0.5, torch.randn(B, Hkv, max_ctx, hd, generator=g)
+    sk, sv = (0.03, 0.04) if fp8 else (1.0, 1.0)
+    if fp8:
+        (kc, kd), (vc, vd) = fp8_codes(kc, sk), fp8_codes(vc, sv)
+    else:
+        kc, vc = kc.to(torch.bfloat16), vc.to(torch.bfloat16)
+        kd, vd = kc.float(), vc.float()
+    for b, n in enumerate(lens):
+        for c in (kc, vc):
+            c[b, :, n:] = 0x7f if fp8 else float("nan")  # (e4m3's NaN)
+    kp, bt = paged_cache(kc, True, seed=5)
+    vp, _ = paged_cache(vc, True, seed=5)
+    kp, vp, bt = kp.cuda(), vp.cuda(), bt.cuda()
+    q = torch.randn(B, H, hd, generator=g).cuda()
+    seq = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    slot = torch.arange(B, dtype=torch.int32, device="cuda")
+    nch, scale = max_ctx // E.ATTN_CHUNK, 1 / math.sqrt(hd)
+    opart, ml = torch.empty(B, H, nch, hd, device="cuda"), torch.empty(B, H, nch, 2, device="cuda")
+    f = scale * 1.4426950408889634 * sk
+    qq = (q * f).to(torch.bfloat16).double() / (1.4426950408889634 * sk)  # (rounded where the kernel rounds it)
+    for bt_rows in (0, 1):
+        out, cnt = torch.empty(B, H * hd, device="cuda"), torch.zeros(B, H, dtype=torch.int32, device="cuda")
+        E.attn_decode(q.data_ptr(), kp.data_ptr(), vp.data_ptr(), seq.data_ptr(), slot.data_ptr(), B, H, Hkv, hd, max_ctx, nch,
+                      scale, opart.data_ptr(), ml.data_ptr(), out.data_ptr(), cnt.data_ptr(), stream(), 0, bt.data_ptr(), bt_rows,
+                      kv_fp8=int(fp8), k_scale=sk, v_scale=sv)
+        torch.cuda.synchronize()
+        assert int(cnt.abs().sum()) == 0
+        for b, n in enumerate(lens):
+            k, v = kd[b, :, :n].cuda().double(), vd[b, :, :n].cuda().double()
+            p = torch.softmax((qq[b].view(Hkv, G, 1, hd) * k[:, None]).sum(-1), -1)
+            ref = (p[..., None] * v[:, None]).sum(2).reshape(-1)
+            err = float((out[b].double() - ref).norm() / ref.norm())
+            assert err < 2e-5, (b, n, err)
+
+
 @pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64)])
 @pytest.mark.parametrize("start,T", [(0, 37), (70, 130), (0, 300)])
 def test_attention_prefill_fp8_kv(E, H, Hkv, hd, start, T):
