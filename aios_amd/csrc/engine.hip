@@ -747,7 +747,7 @@ void Engine::finalize() {
 
 // Measured prefill-GEMM plans (kernels/gemm_pf.hip): every distinct projection launch of this model
 // -- QKV stack, O, gate/up (SwiGLU), down, per weight-format signature -- timed over its candidate
-// tiles / K splits at M = 64 .. gm_rows_ (powers of two), the fastest kept per M bucket in the
+// tiles / K splits at M = 64 .. gm_rows_ (gemm_pf_bucket), the fastest kept per M bucket in the
 // process-wide plan cache (one tuning per shape per process; ~0.3 s for Mistral-7B).  Activations
 // are random bf16 (a zero fill clocks the chip differently).  AIOS_GEMM_PF_TUNE=0: model plans only.
 void Engine::tune_prefill_gemm() {
@@ -765,7 +765,7 @@ void Engine::tune_prefill_gemm() {
   launch_f32_to_bf16(tmp, gm_attn16_, (size_t)G * qd, stream_);
   launch_f32_to_bf16(tmp, gm_ff16_, (size_t)G * ff, stream_);
   std::set<std::string> seen;
-  for (int M = 64; M <= G; M *= 2) {
+  for (int M = 64; M <= G; M = gemm_pf_bucket(M + 1)) {
     for (const LayerW& L : layers_) {
       auto tune = [&](GemmQArgs& g, const char* what) {
         std::string sig = std::string(what) + ":" + std::to_string(M);

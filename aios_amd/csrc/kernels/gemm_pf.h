@@ -153,14 +153,29 @@ struct PfDma {
   }
 };
 
-// 8 codes (bytes of w0 then w1) -> bf16x8 fragment of sc * q - of
+// 8 codes -> bf16x8 fragment of sc * q - of: bytes of w0 then w1 (masked to M each, shifted left by SH bits as they lie).
+// A masked code in a 16-bit half is, read as an fp16 denormal, code * 2^-24 exactly, and v_fma_mix_f32 takes it as it is:
+// two codes per mask instead of one v_cvt_f32_ubyteN each, with the scale's exponent raised to match -- the same
+// fused multiply-add, bit for bit.  (Per four codes 9 instructions instead of 11.5; the decode shares the vector
+// issue with the matrix instructions, and at up to 160 rows it is what bounds the tile.)
+template <uint32_t M, int SH = 0>
 __device__ __forceinline__ gbf16x8 pf_dq8(uint32_t w0, uint32_t w1, float sc, float of) {
-  asm volatile("" : "+v"(w0), "+v"(w1));  // one v_cvt_f32_ubyteN per byte
+  constexpr uint32_t MM = (M << SH) * 0x10001u;
+  const float s = sc * (float)(1 << (24 - SH));
+  auto two = [&](uint32_t x, float& a, float& b) __attribute__((always_inline)) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const h2 h = __builtin_bit_cast(h2, x & MM);
+    a = fmaf((float)h[0], s, -of);
+    b = fmaf((float)h[1], s, -of);
+  };
+  float q[8];
+  two(w0, q[0], q[2]);
+  two(w0 >> 8, q[1], q[3]);
+  two(w1, q[4], q[6]);
+  two(w1 >> 8, q[5], q[7]);
   uint32_t p[4];
-  p[0] = pk_bf16(fmaf(sc, (float)(w0 & 0xff), -of), fmaf(sc, (float)((w0 >> 8) & 0xff), -of));
-  p[1] = pk_bf16(fmaf(sc, (float)((w0 >> 16) & 0xff), -of), fmaf(sc, (float)(w0 >> 24), -of));
-  p[2] = pk_bf16(fmaf(sc, (float)(w1 & 0xff), -of), fmaf(sc, (float)((w1 >> 8) & 0xff), -of));
-  p[3] = pk_bf16(fmaf(sc, (float)((w1 >> 16) & 0xff), -of), fmaf(sc, (float)(w1 >> 24), -of));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) p[i] = pk_bf16(q[2 * i], q[2 * i + 1]);
   gbf16x8 r;
   __builtin_memcpy(&r, p, 16);
   return r;
@@ -204,12 +219,12 @@ __device__ __forceinline__ gbf16x8 pf_bdec(const PfBRaw& r, int q, int kt, int d
   } else if constexpr (QT == QT_Q8_0) {  // (pf8 body) fragment S = the K-step's 32-block S: cw / b1.xy
     const uint32_t w0 = (S == 0 ? r.cw.x : r.b1.x) ^ 0x80808080u, w1 = (S == 0 ? r.cw.y : r.b1.y) ^ 0x80808080u;
     const float d = h2f((uint16_t)(r.scw >> (16 * S)));
-    f = pf_dq8(w0, w1, d, 128.f * d);
+    f = pf_dq8<0xff>(w0, w1, d, 128.f * d);
   } else if constexpr (QT == QT_Q4_0) {  // block S: weights 8q.. = low nibbles (q < 2) / high (q >= 2)
     const int sh = 4 * (q >> 1);
-    const uint32_t w0 = ((S == 0 ? r.cw.x : r.b1.x) >> sh) & 0x0f0f0f0fu, w1 = ((S == 0 ? r.cw.y : r.b1.y) >> sh) & 0x0f0f0f0fu;
+    const uint32_t w0 = (S == 0 ? r.cw.x : r.b1.x) >> sh, w1 = (S == 0 ? r.cw.y : r.b1.y) >> sh;
     const float d = h2f((uint16_t)(r.scw >> (16 * S)));
-    f = pf_dq8(w0, w1, d, 8.f * d);
+    f = pf_dq8<0xf>(w0, w1, d, 8.f * d);
   } else if constexpr (QT == QT_Q6_K) {
     const float d = h2f((uint16_t)(r.dw >> (16 * dpar)));
     const float ds = d * (float)(int8_t)((r.scw >> (16 * (q >> 1) + 8 * S)) & 0xff);
@@ -217,20 +232,22 @@ __device__ __forceinline__ gbf16x8 pf_bdec(const PfBRaw& r, int q, int kt, int d
     const int j0 = 2 * (q & 1);  // code words j0, j0 + 1 of the chunk
     const uint32_t c0 = S == 0 ? (r.cw.x & 0x0f0f0f0fu) : ((r.cw.x >> 4) & 0x0f0f0f0fu);
     const uint32_t c1 = S == 0 ? (r.cw.y & 0x0f0f0f0fu) : ((r.cw.y >> 4) & 0x0f0f0f0fu);
-    f = pf_dq8(c0 | (((hv >> (2 * j0)) & 0x03030303u) << 4), c1 | (((hv >> (2 * j0 + 2)) & 0x03030303u) << 4), ds,
-               32.f * ds);
+    f = pf_dq8<0x3f>(c0 | (((hv >> (2 * j0)) & 0x03030303u) << 4), c1 | (((hv >> (2 * j0 + 2)) & 0x03030303u) << 4), ds,
+                     32.f * ds);
   } else {  // Q4_K
     const float d = h2f((uint16_t)(r.mt.x & 0xffff)), dmin = h2f((uint16_t)(r.mt.x >> 16));
     const uint32_t fl = kq_field(r.mt.y, r.mt.z, r.mt.w, kt & 3);
     const float ds = d * (float)((fl >> (6 * S)) & 63), dm = dmin * (float)((fl >> (12 + 6 * S)) & 63);
-    uint32_t c0 = S == 0 ? (r.cw.x & 0x0f0f0f0fu) : ((r.cw.x >> 4) & 0x0f0f0f0fu);
-    uint32_t c1 = S == 0 ? (r.cw.y & 0x0f0f0f0fu) : ((r.cw.y >> 4) & 0x0f0f0f0fu);
     if constexpr (QT == QT_Q5_K) {  // (pf8 body) qh bytes 8q.. in hb: bit 2g + S
+      uint32_t c0 = S == 0 ? (r.cw.x & 0x0f0f0f0fu) : ((r.cw.x >> 4) & 0x0f0f0f0fu);
+      uint32_t c1 = S == 0 ? (r.cw.y & 0x0f0f0f0fu) : ((r.cw.y >> 4) & 0x0f0f0f0fu);
       const int sh = 2 * (kt & 3) + S;
       c0 |= ((r.hb.x >> sh) & 0x01010101u) << 4;
       c1 |= ((r.hb.y >> sh) & 0x01010101u) << 4;
+      f = pf_dq8<0x1f>(c0, c1, ds, dm);
+    } else {
+      f = pf_dq8<0xf, 4 * S>(r.cw.x, r.cw.y, ds, dm);
     }
-    f = pf_dq8(c0, c1, ds, dm);
   }
   return f;
 }
@@ -422,13 +439,11 @@ __device__ __forceinline__ gbf16x8 pf_bdec32(const PfBRaw32& r, int h, int kt, i
     const uint32_t w0 = (S == 0 ? r.c0.x : (S == 1 ? r.c1.x : (S == 2 ? r.b1.x : r.b1.z))) ^ 0x80808080u;
     const uint32_t w1 = (S == 0 ? r.c0.y : (S == 1 ? r.c1.y : (S == 2 ? r.b1.y : r.b1.w))) ^ 0x80808080u;
     const float d = h2f((uint16_t)(r.scw >> (16 * (S >> 1))));
-    f = pf_dq8(w0, w1, d, 128.f * d);
+    f = pf_dq8<0xff>(w0, w1, d, 128.f * d);
   } else if constexpr (QT == QT_Q4_0) {  // block S >> 1: low nibbles = weights 0..15, high = 16..31
     const uint2 cw = (S >> 1) ? r.c1 : r.c0;
-    const uint32_t w0 = (S & 1) ? ((cw.x >> 4) & 0x0f0f0f0fu) : (cw.x & 0x0f0f0f0fu);
-    const uint32_t w1 = (S & 1) ? ((cw.y >> 4) & 0x0f0f0f0fu) : (cw.y & 0x0f0f0f0fu);
     const float d = h2f((uint16_t)(r.scw >> (16 * (S >> 1))));
-    f = pf_dq8(w0, w1, d, 8.f * d);
+    f = pf_dq8<0xf, 4 * (S & 1)>(cw.x, cw.y, d, 8.f * d);
   } else {
     const uint2 cw = (S & 1) ? r.c1 : r.c0;
     const uint32_t w0 = (S < 2) ? (cw.x & 0x0f0f0f0fu) : ((cw.x >> 4) & 0x0f0f0f0fu);
@@ -440,8 +455,8 @@ __device__ __forceinline__ gbf16x8 pf_bdec32(const PfBRaw32& r, int h, int kt, i
       const float d = h2f((uint16_t)(r.dw >> (16 * dpar)));
       const float ds = d * (float)(int8_t)((r.scw >> (8 * idx)) & 0xff);
       const int j0 = 2 * h;  // code words 2h, 2h + 1 of the chunk
-      f = pf_dq8(w0 | (((hv >> (2 * j0)) & 0x03030303u) << 4), w1 | (((hv >> (2 * j0 + 2)) & 0x03030303u) << 4), ds,
-                 32.f * ds);
+      f = pf_dq8<0x3f>(w0 | (((hv >> (2 * j0)) & 0x03030303u) << 4), w1 | (((hv >> (2 * j0 + 2)) & 0x03030303u) << 4), ds,
+                       32.f * ds);
     } else {  // Q4_K / Q5_K: sub-block 2g (S < 2) or 2g + 1
       const float d = h2f((uint16_t)(r.mt.x & 0xffff)), dmin = h2f((uint16_t)(r.mt.x >> 16));
       const uint32_t fl = kq_field(r.mt.y, r.mt.z, r.mt.w, kt & 3);
@@ -450,9 +465,9 @@ __device__ __forceinline__ gbf16x8 pf_bdec32(const PfBRaw32& r, int h, int kt, i
       if constexpr (QT == QT_Q5_K) {  // + bit (2g + hi) of the weights' qh bytes as bit 4
         const int sh = 2 * (kt & 3) + sb;
         const uint32_t h0 = (S & 1) ? r.b1.z : r.b1.x, h1 = (S & 1) ? r.b1.w : r.b1.y;
-        f = pf_dq8(w0 | (((h0 >> sh) & 0x01010101u) << 4), w1 | (((h1 >> sh) & 0x01010101u) << 4), ds, dm);
+        f = pf_dq8<0x1f>(w0 | (((h0 >> sh) & 0x01010101u) << 4), w1 | (((h1 >> sh) & 0x01010101u) << 4), ds, dm);
       } else {
-        f = pf_dq8(w0, w1, ds, dm);
+        f = pf_dq8<0xf, S < 2 ? 0 : 4>(cw.x, cw.y, ds, dm);
       }
     }
   }
@@ -614,8 +629,11 @@ struct Pf4Layout {
   static constexpr int SLOT = (A_BYTES + NW * WB + 255) / 256 * 256;
   // ring depth: as many slots as 160 KB of LDS holds, up to AIOS_PF4_NS (deeper rings keep more K-steps of
   // DMA in flight for the one workgroup per CU; the counted waits are (NS - 1) / (NS - 2) x PW)
-  static constexpr int NS_FIT = (160 * 1024) / SLOT;
-  static constexpr int NS = NS_FIT < AIOS_PF4_NS ? NS_FIT : AIOS_PF4_NS;
+  template <int KG>
+  static constexpr int slots() {
+    return (160 * 1024) / (KG * SLOT) < AIOS_PF4_NS ? (160 * 1024) / (KG * SLOT) : AIOS_PF4_NS;
+  }
+  static constexpr int NS = slots<1>();
   static constexpr int NA = BM / (8 * NW), NCODE = CODE / 1024, NMETA = META / 1024, NHB = HB / 1024,
                        NSC = SC / 256, ND = DW / 256;
   static constexpr int PW = NA + NCODE + NMETA + NHB + NSC + ND;  // DMA instructions per wave per slot
@@ -677,15 +695,15 @@ struct Pf4Dma {
         return;
       }
       if constexpr (i < L::NA) {
-        pf_glds16((const uint8_t*)a.A + kt * 128 + off[i], dst + (NW * i + wv) * 1024);
+        pf_glds16((const uint8_t*)a.A + kt * 128, off[i], dst + (NW * i + wv) * 1024);
       } else if constexpr (i < L::NA + L::NCODE) {
-        pf_glds16(w.p0 + (L::BF ? kt * 128 : (L::L8 ? kt * 64 : kt * 32)) + off[i], wb + (i - L::NA) * 1024);
+        pf_glds16(w.p0 + (L::BF ? kt * 128 : (L::L8 ? kt * 64 : kt * 32)), off[i], wb + (i - L::NA) * 1024);
       } else if constexpr (i < L::NA + L::NCODE + L::NMETA) {
-        pf_glds16(w.p1 + (L::Q6 ? kt * 16 : (kt >> 2) * 16) + off[i], wb + L::OFF_META);
+        pf_glds16(w.p1 + (L::Q6 ? kt * 16 : (kt >> 2) * 16), off[i], wb + L::OFF_META);
       } else if constexpr (i < L::NA + L::NCODE + L::NMETA + L::NHB) {
-        pf_glds16(w.p2 + (kt >> 2) * 32 + off[i], wb + L::OFF_HB);
+        pf_glds16(w.p2 + (kt >> 2) * 32, off[i], wb + L::OFF_HB);
       } else if constexpr (i < L::NA + L::NCODE + L::NMETA + L::NHB + L::NSC) {
-        pf_glds4((L::Q6 ? w.p2 : w.p1) + kt * 4 + off[i], wb + L::OFF_SC);
+        pf_glds4((L::Q6 ? w.p2 : w.p1) + kt * 4, off[i], wb + L::OFF_SC);
       } else {
         pf_glds4(w.p3 + (((off[i] + (uint32_t)(kt >> 2)) >> 1) << 2), wb + L::OFF_DW);
       }
@@ -725,13 +743,25 @@ __device__ __forceinline__ void pf4_braw(const uint8_t* wbase, int cl, int h, Pf
   }
 }
 
-template <int QT, int BM, int WC, int EPI, int PROBE = 0>
+// KG = 2 (tiles below 256 rows): two groups of four waves, each with half of the slice's K-steps and slots of its
+// own, their accumulators added through LDS at the end.  One wave per SIMD runs a K-step's LDS reads, decode,
+// matrix instructions and DMA issue one after the other (64 x 128 tiles: 1900 cycles a step, of which 256 are
+// matrix instructions); the second wave fills its gaps.  Both groups have the same number of steps (pf4_kg).
+// Gate/up of 28672 x 4096 Q4_K: 64 rows 47 -> 35 us, 130 rows (one 160-row tile) 78 -> 57 us.
+template <int QT, int BM, int WC, int EPI, int PROBE = 0, int KG = 1>
 __device__ __forceinline__ void pf4_body(const GemmQArgs& a, int m0, int n0, int seg, int kt0, int kt1, int S) {
   using L = Pf4Layout<QT, BM, WC>;
-  constexpr int MT = BM / 32, CT = WC / 32, NS = L::NS, PW = L::PW;
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
+  constexpr int MT = BM / 32, CT = WC / 32, NS = L::template slots<KG>(), PW = L::PW;
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem0[];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wv = KG == 1 ? wave : wave & 3, grp = KG == 1 ? 0 : wave >> 2;
+  uint8_t* pf_smem = pf_smem0 + (KG == 1 ? 0 : grp * (NS * L::SLOT));
+  if constexpr (KG == 2) {
+    const int mid = (kt0 + kt1) >> 1;
+    if (grp) kt0 = mid;
+    else kt1 = mid;
+  }
   QWeight w;
   w.qtype = QT;
   w.rows = seg == 0 ? a.seg[0].rows : (seg == 1 ? a.seg[1].rows : a.seg[2].rows);
@@ -859,32 +889,54 @@ __device__ __forceinline__ void pf4_body(const GemmQArgs& a, int m0, int n0, int
   pf_vmcnt<0>();  // no LDS-DMA may land after this workgroup's LDS is released
 
   // epilogue -- C/D map of the 32x32 accumulator: col = lane & 31, row = (e & 3) + 8 (e >> 2) + 4 h
-#pragma unroll
-  for (int c = 0; c < CT; ++c) {
-    const int n = n0 + wv * WC + 32 * c + r32;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = m0 + 32 * i + (e & 3) + 8 * (e >> 2) + 4 * h;
-        const float v = acc[i][c][e];
-        if constexpr (EPI == GEPI_SWIGLU_BF16) {
-          const float up = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
-          if (m < a.M && !(r32 & 1)) a.C16[(size_t)m * a.ldc + (n >> 1)] = f32_to_bf16(glu_act(v, a.act) * up);
-        } else if constexpr (EPI == GEPI_STORE16) {
-          if (m < a.M) a.C16[(size_t)m * a.ldc + n] = f32_to_bf16(store16_val(a, n, v));
-        } else if constexpr (EPI == GEPI_QKV) {
-          pf_qkv_out(a, m, n, v, !(r32 & 1));
-        } else if (m < a.M) {
-          float* cp = a.C + (size_t)m * a.ldc + n;
-          if (S > 1) unsafeAtomicAdd(cp, v);
-          else if constexpr (EPI == GEPI_ACCUM) *cp += v;
-          else *cp = v;
-        }
-      }
+  auto out = [&](int m, int n, float v) __attribute__((always_inline)) {
+    if constexpr (EPI == GEPI_SWIGLU_BF16) {
+      const float up = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
+      if (m < a.M && !(r32 & 1)) a.C16[(size_t)m * a.ldc + (n >> 1)] = f32_to_bf16(glu_act(v, a.act) * up);
+    } else if constexpr (EPI == GEPI_STORE16) {
+      if (m < a.M) a.C16[(size_t)m * a.ldc + n] = f32_to_bf16(store16_val(a, n, v));
+    } else if constexpr (EPI == GEPI_QKV) {
+      pf_qkv_out(a, m, n, v, !(r32 & 1));
+    } else if (m < a.M) {
+      float* cp = a.C + (size_t)m * a.ldc + n;
+      if (S > 1) unsafeAtomicAdd(cp, v);
+      else if constexpr (EPI == GEPI_ACCUM) *cp += v;
+      else *cp = v;
     }
+  };
+  if constexpr (KG == 2) {
+    // group g keeps the accumulators' elements 8 g .. 8 g + 7 (16 rows of every 32) and takes the other group's from
+    // LDS; (group 0's) + (group 1's) in either
+    static_assert(CT == 1, "32 columns per wave");
+    float* xb = (float*)pf_smem0;
+    __syncthreads();  // every wave's LDS reads and DMAs are done
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xb[((wave * MT + i) * 8 + e) * 64 + lane] = grp ? acc[i][0][e] : acc[i][0][8 + e];
+    __syncthreads();
+    const int n = n0 + wv * WC + r32;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = (grp ? acc[i][0][8 + e] : acc[i][0][e]) + xb[(((wave ^ 4) * MT + i) * 8 + e) * 64 + lane];
+        out(m0 + 32 * i + 16 * grp + (e & 3) + 8 * (e >> 2) + 4 * h, n, v);
+      }
+    return;
   }
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) out(m0 + 32 * i + (e & 3) + 8 * (e >> 2) + 4 * h, n0 + wv * WC + 32 * c + r32, acc[i][c][e]);
 }
+
+// K groups of a pf4 workgroup: two below 256 rows (at 256 one group's slots and accumulators take the CU).  Slices
+// lie on even K-steps then (the launcher keeps such tiles to K % 128 == 0).
+template <int BM>
+constexpr int pf4_kg() { return BM < 256 ? 2 : 1; }
 
 // ==== pf8: 8 waves (two per SIMD) x 32 columns, 16x16x32 MFMA ======================================
 // The 8-wave 16x16x32 body ran the compute-only probe at 1.33 PF per busy CU against 1.16 for pf4's
@@ -1122,32 +1174,33 @@ struct PfcDma {
 
   __device__ __forceinline__ void A(const GemmQArgs& a, int kt, uint32_t dst, int wv) const {
 #pragma unroll
-    for (int i = 0; i < L::NA; ++i) pf_glds16((const uint8_t*)a.A + kt * 128 + offA[i], dst + (NW * i + wv) * 1024);
+    for (int i = 0; i < L::NA; ++i) pf_glds16((const uint8_t*)a.A + kt * 128, offA[i], dst + (NW * i + wv) * 1024);
   }
   // the A pieces i with i % NP == P
   template <int P, int NP>
   __device__ __forceinline__ void A_part(const GemmQArgs& a, int kt, uint32_t dst, int wv) const {
 #pragma unroll
     for (int i = 0; i < L::NA; ++i)
-      if (i % NP == P) pf_glds16((const uint8_t*)a.A + kt * 128 + offA[i], dst + (NW * i + wv) * 1024);
+      if (i % NP == P) pf_glds16((const uint8_t*)a.A + kt * 128, offA[i], dst + (NW * i + wv) * 1024);
   }
   // code piece pc of half block hsrc into the wave's half-block buffer at dst
   __device__ __forceinline__ void code(const QWeight& w, int hsrc, int pc, uint32_t dst) const {
     // (a register select: offC[pc] with a runtime pc puts the array in scratch, and the scratch
     // load's vmcnt(0) drained every in-flight DMA)
-    pf_glds16(w.p0 + hsrc * 64 + (pc ? offC[1] : offC[0]), dst + pc * 1024);
+    pf_glds16(w.p0 + hsrc * 64, pc ? offC[1] : offC[0], dst + pc * 1024);
   }
   // record piece pr (rows 8 pr .. 8 pr + 7) of block bsrc; lanes 0..31
   __device__ __forceinline__ void rec(const QWeight& w, int bsrc, int pr, uint32_t nbk, uint32_t dst) const {
-    if ((threadIdx.x & 63) < 32) pf_glds4((L::Q6 ? w.p2 : w.p1) + bsrc * 16 + offR + pr * 128 * nbk, dst + pr * 128);
+    pf_glds_part<32, 4>((L::Q6 ? w.p2 : w.p1) + bsrc * 16 + (size_t)(pr * 128 * nbk), offR, dst + pr * 128);
   }
   // Q6_K high-bit piece pc (rows 16 pc ..) of half block hsrc; lanes 0..31
   __device__ __forceinline__ void hi(const QWeight& w, int hsrc, int pc, uint32_t nbk, uint32_t dst) const {
-    if ((threadIdx.x & 63) < 32) pf_glds16(w.p1 + hsrc * 32 + offH + pc * 1024 * nbk, dst + pc * 512);
+    pf_glds_part<32, 16>(w.p1 + hsrc * 32 + (size_t)(pc * 1024 * nbk), offH, dst + pc * 512);
   }
   // Q6_K d piece pr (rows 8 pr ..) of block bsrc: the dword holding each row's f16 d; lanes 0..7
   __device__ __forceinline__ void dq(const QWeight& w, int bsrc, int pr, uint32_t nbk, uint32_t dst) const {
-    if ((threadIdx.x & 63) < 8) pf_glds4(w.p3 + (((offD + pr * 8 * nbk + (uint32_t)bsrc) * 2u) & ~3u), dst + pr * 32);
+    const uint32_t to = __builtin_amdgcn_readfirstlane(dst + pr * 32);
+    if ((threadIdx.x & 63) < 8) pf_glds4(w.p3 + (((offD + pr * 8 * nbk + (uint32_t)bsrc) * 2u) & ~3u), to);
   }
 };
 
@@ -1190,7 +1243,8 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
   // G(s): phase-split -- A pieces in the first phases (longest lead), then code (+ high bits), then
   // records (+ d); PH_ALL = every phase (prologue)
   constexpr int PH_ALL = -1;
-  auto group = [&](int s, auto phc) __attribute__((always_inline)) {
+  // (j: s mod 4, the place in a 256-block, as the slice starts on a block)
+  auto group = [&](int s, int j, auto phc) __attribute__((always_inline)) {
     constexpr int ph = decltype(phc)::value;
     // A piece i in phase i % NG (all before the decode wait at phase NG)
     if constexpr (ph == PH_ALL) {
@@ -1199,10 +1253,11 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
       dma.template A_part<(ph < 0 ? 0 : ph), NG>(a, min(kt0 + s + NSA, klast),
                                                  lds0 + (uint32_t)(((s + 3 * NSA) % NSA) * L::A_BYTES), wv);
     }
-    const int H = (kt0 >> 1) + ((s + 4) >> 1), B = (kt0 >> 2) + ((s + 6) >> 2), pr = (s + 6) & 3;
+    const int H = (kt0 >> 1) + ((s + 4) >> 1), B = (kt0 >> 2) + ((s + 6) >> 2);
+    const int pr = (j + 6) & 3;
     if constexpr (ph == PH_ALL || ph == NPH - 2 || (NPH == 2 && ph == 0)) {
-      dma.code(w, min(H, hlast), s & 1, cb + (uint32_t)(H & 1) * CBS);
-      if constexpr (L::Q6) dma.hi(w, min(H, hlast), s & 1, nbk, hb + (uint32_t)(H & 1) * HBS);
+      dma.code(w, min(H, hlast), j & 1, cb + (uint32_t)(H & 1) * CBS);
+      if constexpr (L::Q6) dma.hi(w, min(H, hlast), j & 1, nbk, hb + (uint32_t)(H & 1) * HBS);
     }
     if constexpr (ph == PH_ALL || ph == NPH - 1) {
       dma.rec(w, min(B, blast), pr, nbk, rb + (uint32_t)(B & 1) * RBS);
@@ -1226,15 +1281,15 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
       dma.rec(w, B0, pr, nbk, rb + (uint32_t)(B0 & 1) * RBS);
       if constexpr (L::Q6) dma.dq(w, B0, pr, nbk, db + (uint32_t)(B0 & 1) * DBS);
     }
-    group(-2, std::integral_constant<int, PH_ALL>{});
+    group(-2, 2, std::integral_constant<int, PH_ALL>{});
   }
 
   gbf16x8 bf[2][2], fa[GR], fb[GR];
   PfBRaw raw[2];
   int rkt = kt0;
   // raw bytes of (absolute) K-step kt for this lane's two columns
-  auto read_raw = [&](int kt) __attribute__((always_inline)) {
-    const int H = kt >> 1, j = kt & 1, B = kt >> 2;
+  auto read_raw = [&](int kt, int place) __attribute__((always_inline)) {
+    const int H = kt >> 1, j = place & 1, B = kt >> 2;
     const uint8_t* cbp = pf_smem + L::OFF_CB + (H & 1) * CBS + wv * L::CB_W;
     const uint8_t* rbp = pf_smem + L::OFF_RB + (B & 1) * RBS + wv * L::RB_W;
 #pragma unroll
@@ -1244,7 +1299,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
       r.cw = *(const uint2*)(cbp + row * 64 + (((2 * j + (q >> 1)) ^ ((row >> 2) & 3)) << 4) + 8 * (q & 1));
       if constexpr (L::Q6) {
         r.hb = *(const uint2*)(pf_smem + L::OFF_HB + (H & 1) * HBS + wv * L::HB_W + row * 32 + (2 * j + (q >> 1)) * 8);
-        r.scw = *(const uint32_t*)(rbp + row * 16 + 4 * (kt & 3));
+        r.scw = *(const uint32_t*)(rbp + row * 16 + 4 * place);
         r.dw = *(const uint32_t*)(pf_smem + L::OFF_D + (B & 1) * DBS + wv * L::D_W + row * 4);
       } else {
         r.mt = *(const uint4*)(rbp + row * 16);
@@ -1252,13 +1307,13 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
     }
     rkt = kt;
   };
-  auto dec = [&](auto sc) __attribute__((always_inline)) {
+  auto dec = [&](auto sc, int place) __attribute__((always_inline)) {
     constexpr int S2 = decltype(sc)::value;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int cl = 16 * c + r16;
       const int dpar = L::Q6 ? (int)(((uint32_t)(wcol0 + cl) * nbk + (uint32_t)(rkt >> 2)) & 1u) : 0;
-      bf[c][S2] = pf_bdec<QT, S2>(raw[c], q, rkt, dpar);
+      bf[c][S2] = pf_bdec<QT, S2>(raw[c], q, place, dpar);
       asm volatile("" : "+v"(bf[c][S2]));  // keep the decode in this phase (else sunk past the barrier)
     }
   };
@@ -1281,14 +1336,21 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
     }
   };
   if constexpr (!(PROBE & 1)) pf_vmcnt<PW>();  // the prologue group landed (G(-2) in flight)
-  read_raw(kt0);
-  dec(std::integral_constant<int, 0>{});
+  read_raw(kt0, 0);
+  dec(std::integral_constant<int, 0>{}, 0);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   pf_barrier();
   ldA(pf_smem, fa, 0);
 
+  // four K-steps (a block) per turn of the loop: what a step takes from its place in the block -- record fields, DMA
+  // pieces, buffer halves -- is then fixed in the code.  At 256 rows two: four spill registers, and the reloads'
+  // waits drain the DMA (460 -> 537 us for 2048 x 28672 x 4096; two steps 448 us).  Vector instructions of a step and
+  // wave besides the matrix ones: 167 before, 124 at 256 rows, 108 at 128 (28672 x 4096, 256 rows: 77.8 -> 73.6 us).
+  constexpr int UN = BM == 256 ? 2 : 4;
   int cur = 0;
-  for (int s = 0; s < nk; ++s) {
+  for (int su = 0; su < nk; su += UN) static_for<UN>([&](auto jc) __attribute__((always_inline)) {
+    constexpr int J = decltype(jc)::value;
+    const int s = su + J, place = UN == 4 ? J : (su & 2) + J;
     const uint8_t* slot = pf_smem + cur * L::A_BYTES;
     const int nxt = cur == NSA - 1 ? 0 : cur + 1;
     static_for<NPH>([&](auto pc) {
@@ -1297,16 +1359,16 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
       auto& cf = (p % 2 == 0) ? fa : fb;
       auto& nf = (p % 2 == 0) ? fb : fa;
       if constexpr (p + 1 < NPH) ldA(slot, nf, p + 1);
-      if constexpr (p == 0) dec(std::integral_constant<int, 1>{});
+      if constexpr (p == 0) dec(std::integral_constant<int, 1>{}, place);
       if constexpr (p == NG) {
         // G(s-2) landed -- step s+1's codes / records and this wave's A pieces of it -- with only
         // G(s-1)'s first-phase pieces younger
         if constexpr (!(PROBE & 1)) pf_vmcnt<PRE_WAIT>();
-        read_raw(kt0 + s + 1);  // (past the last step: stale buffers, unused)
-        dec(std::integral_constant<int, 0>{});
+        read_raw(kt0 + s + 1, (place + 1) & 3);  // (past the last step: stale buffers, unused)
+        dec(std::integral_constant<int, 0>{}, (place + 1) & 3);
       }
       // G(s-1): its slot / buffers were released by B(s) (past the end: clamped re-loads, unused)
-      if constexpr (!(PROBE & 4)) group(s - 1, pc);
+      if constexpr (!(PROBE & 4)) group(s - 1, (place + 3) & 3, pc);
       if constexpr (p + 1 < NPH) {
         mfma_range(cf, p, 0, 2 * GR);
       } else {
@@ -1323,7 +1385,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
       for (int i = 0; i < GR; ++i) fa[i] = fb[i];
     }
     cur = nxt;
-  }
+  });
   pf_vmcnt<0>();  // no LDS-DMA may land after this workgroup's LDS is released
 
 #pragma unroll
@@ -1676,15 +1738,16 @@ __device__ __forceinline__ void pf_stream_k(const GemmQArgs& a, int BN, int ipw,
 }
 
 template <int QT0, int QT1, int BM, int WC, int EPI>
-__global__ void __launch_bounds__(256) gemm_pf4sk_kernel(GemmQArgs a, int ipw) {
-  pf_stream_k<QT0, QT1, BM, EPI, 1>(a, 4 * WC, ipw, [&](int m0, int n0, int seg, int kt0, int kt1, int S) {
+__global__ void __launch_bounds__(256 * pf4_kg<BM>()) gemm_pf4sk_kernel(GemmQArgs a, int ipw) {
+  constexpr int KG = pf4_kg<BM>();
+  pf_stream_k<QT0, QT1, BM, EPI, KG>(a, 4 * WC, ipw, [&](int m0, int n0, int seg, int kt0, int kt1, int S) {
     if constexpr (QT0 != QT1) {
       if (seg == a.nseg - 1) {
-        pf4_body<QT1, BM, WC, EPI>(a, m0, n0, seg, kt0, kt1, S);
+        pf4_body<QT1, BM, WC, EPI, 0, KG>(a, m0, n0, seg, kt0, kt1, S);
         return;
       }
     }
-    pf4_body<QT0, BM, WC, EPI>(a, m0, n0, seg, kt0, kt1, S);
+    pf4_body<QT0, BM, WC, EPI, 0, KG>(a, m0, n0, seg, kt0, kt1, S);
   });
 }
 
@@ -1775,8 +1838,8 @@ void pf8_launch(const GemmQArgs& a, int S, hipStream_t st) {
 }
 
 template <int QT0, int QT1, int BM, int WC, int EPI, int PROBE = 0>
-__global__ void __launch_bounds__(256) gemm_pf4_kernel(GemmQArgs a) {
-  constexpr int BN = 4 * WC;
+__global__ void __launch_bounds__(256 * pf4_kg<BM>()) gemm_pf4_kernel(GemmQArgs a) {
+  constexpr int BN = 4 * WC, KG = pf4_kg<BM>();
   const int nN = a.N / BN, nM = (a.M + BM - 1) / BM, total = nN * nM;
   const int L = xcd_remap(blockIdx.x, total);
   const int tn = L % nN, tm = L / nN;
@@ -1784,15 +1847,15 @@ __global__ void __launch_bounds__(256) gemm_pf4_kernel(GemmQArgs a) {
   int seg = 0;
   if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
   if (a.nseg > 2 && n0 >= a.seg_n0[2]) seg = 2;
-  const int S = gridDim.y, nk_all = a.K / 64;
-  const int kt0 = (int)((long)blockIdx.y * nk_all / S), kt1 = (int)((long)(blockIdx.y + 1) * nk_all / S);
+  const int S = gridDim.y, nk_all = a.K / (64 * KG);
+  const int kt0 = KG * (int)((long)blockIdx.y * nk_all / S), kt1 = KG * (int)((long)(blockIdx.y + 1) * nk_all / S);
   if constexpr (QT0 != QT1) {
     if (seg == a.nseg - 1) {
-      pf4_body<QT1, BM, WC, EPI, PROBE>(a, m0, n0, seg, kt0, kt1, S);
+      pf4_body<QT1, BM, WC, EPI, PROBE, KG>(a, m0, n0, seg, kt0, kt1, S);
       return;
     }
   }
-  pf4_body<QT0, BM, WC, EPI, PROBE>(a, m0, n0, seg, kt0, kt1, S);
+  pf4_body<QT0, BM, WC, EPI, PROBE, KG>(a, m0, n0, seg, kt0, kt1, S);
 }
 
 // pf4's tail split (256 x 4 WC tiles): as gemm_pf8t_kernel, the last R tiles as two 128-row halves
@@ -1825,24 +1888,29 @@ __global__ void __launch_bounds__(256) gemm_pf4t_kernel(GemmQArgs a, int F) {
   else pf4_body<QT0, 128, WC, EPI>(a, m0, n0, seg, 0, kt1, 1);
 }
 
+template <int QT, int BM, int WC>
+constexpr int pf4_lds_one() {
+  using L = Pf4Layout<QT, BM, WC>;
+  constexpr int KG = pf4_kg<BM>(), ring = KG * L::template slots<KG>() * L::SLOT, sum = KG == 2 ? BM * 4 * WC * 4 : 0;
+  return ring > sum ? ring : sum;  // (the sum over the groups exchanges half of each)
+}
 template <int QT0, int QT1, int BM, int WC>
 constexpr int pf4_lds_bytes() {
-  using L0 = Pf4Layout<QT0, BM, WC>;
-  using L1 = Pf4Layout<QT1, BM, WC>;
-  return L0::NS * L0::SLOT > L1::NS * L1::SLOT ? L0::NS * L0::SLOT : L1::NS * L1::SLOT;
+  return pf4_lds_one<QT0, BM, WC>() > pf4_lds_one<QT1, BM, WC>() ? pf4_lds_one<QT0, BM, WC>() : pf4_lds_one<QT1, BM, WC>();
 }
 
 template <int QT0, int QT1, int BM, int WC>
 void pf4_launch(const GemmQArgs& a, int S, hipStream_t st) {
   constexpr int lds = pf4_lds_bytes<QT0, QT1, BM, WC>();
   static_assert(lds <= 160 * 1024, "LDS");
+  constexpr int KG = pf4_kg<BM>(), NT = 256 * KG;
   if (S < 0) {  // stream-K (STORE / ACCUM only)
     int grid = 0;
-    const int ipw = pf_sk_ipw(a, BM, 4 * WC, 1, grid);
+    const int ipw = pf_sk_ipw(a, BM, 4 * WC, KG, grid);
     if (a.epi == GEPI_STORE)
-      hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_STORE>), dim3(grid), dim3(256), lds, st, a, ipw);
+      hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_STORE>), dim3(grid), dim3(NT), lds, st, a, ipw);
     else
-      hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_ACCUM>), dim3(grid), dim3(256), lds, st, a, ipw);
+      hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_ACCUM>), dim3(grid), dim3(NT), lds, st, a, ipw);
     return;
   }
   if constexpr (BM == 256) {
@@ -1860,7 +1928,7 @@ void pf4_launch(const GemmQArgs& a, int S, hipStream_t st) {
       return;
     }
   }
-  const dim3 grid((a.N / (4 * WC)) * ((a.M + BM - 1) / BM), S), block(256);
+  const dim3 grid((a.N / (4 * WC)) * ((a.M + BM - 1) / BM), S), block(NT);
   switch (a.epi) {
     case GEPI_STORE: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_STORE>), grid, block, lds, st, a); break;
     case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_ACCUM>), grid, block, lds, st, a); break;
@@ -1941,7 +2009,7 @@ bool pf_launch_fmt(const GemmQArgs& a, int BM, int BN, int S, hipStream_t st) {
     pf4_launch<QT0, QT1, bm, 32>(a, S, st); \
     return true;                            \
   }
-  PF_GO8(256) PF_GO8(128) PF_GO8(64) PF_GO4(256) PF_GO4(128) PF_GO4(64)
+  PF_GO8(256) PF_GO8(128) PF_GO8(64) PF_GO4(256) PF_GO4(160) PF_GO4(128) PF_GO4(96) PF_GO4(64)
 #undef PF_GO8
 #undef PF_GO4
   return false;

@@ -62,8 +62,11 @@ static double pf_model(const GemmQArgs& a, int bm, int bn, int S, bool bf) {
   return t;
 }
 
-static bool pf_tile_ok(const GemmQArgs& a, int bn) {
+// the tiles there are (gemm_pf.h pf_launch_fmt), largest first
+static const struct { int bm, bn; } PF_TILES[] = {{256, 256}, {256, 128}, {160, 128}, {128, 256}, {128, 128}, {96, 128}, {64, 256}, {64, 128}};
+static bool pf_tile_ok(const GemmQArgs& a, int bm, int bn) {
   if (a.N % bn) return false;
+  if (bn == 128 && bm < 256 && a.K % 128) return false;  // (two K groups of equal length)
   for (int s = 0; s < a.nseg; ++s)
     if (a.seg_n0[s] % bn || a.seg[s].rows % bn) return false;
   return true;
@@ -72,14 +75,16 @@ static bool pf_tile_ok(const GemmQArgs& a, int bn) {
 // Measured plans: one per (shape, formats, epilogue, M bucket), filled by gemm_pf_autotune (the
 // engine tunes its projection shapes at finalize); the model below is the fallback.
 using PfKey = std::tuple<int, int, int, int, int, int, int, int, int, int>;
-static int pf_bucket(int M) {
-  int b = 64;
-  while (b < M && b < 2048) b <<= 1;
-  return M > 2048 ? (M + 2047) / 2048 * 2048 : b;
+// (Two or three to a doubling, where tiles of 32 rows more or less change the plan: 130 rows ran the plan of 256, whose
+// gate/up took 83 us where one 160-row tile takes 58.)
+int gemm_pf_bucket(int M) {
+  for (int b : {64, 96, 128, 160, 192, 256, 320, 384, 512, 640, 768, 1024, 1280, 1536, 2048})
+    if (M <= b) return b;
+  return (M + 2047) / 2048 * 2048;
 }
 static PfKey pf_key(const GemmQArgs& a) {
   // (+ the CU budget: a CU-masked co-resident engine plans for its own CUs)
-  return PfKey(a.N, a.K, pf_bucket(a.M), a.epi, a.seg[0].qtype, a.seg[a.nseg - 1].qtype, a.nseg,
+  return PfKey(a.N, a.K, gemm_pf_bucket(a.M), a.epi, a.seg[0].qtype, a.seg[a.nseg - 1].qtype, a.nseg,
                a.nseg > 1 ? a.seg_n0[1] : 0, a.nseg > 2 ? a.seg_n0[2] : 0, device_cu_count());
 }
 static std::mutex pf_mu;
@@ -104,7 +109,7 @@ static bool pf_no_split(const GemmQArgs& a) {
 // (every stream-K segment then spans >= 2 steps / 256-blocks); AIOS_GEMM_PF_SK=0 keeps it out of plans
 static bool pf_sk_ok(const GemmQArgs& a, int bm, int bn, bool bf) {
   if (pf_no_split(a) || !pf_env("AIOS_GEMM_PF_SK", 1)) return false;
-  const int units = bn == 256 && !bf ? a.K / 256 : a.K / 64;
+  const int units = bn == 256 && !bf ? a.K / 256 : (bn == 128 && bm < 256 ? a.K / 128 : a.K / 64);
   const double tiles = (double)((a.M + bm - 1) / bm) * (a.N / bn);
   return units % 2 == 0 && units >= 4 && tiles < 2.0 * device_cu_count();
 }
@@ -113,19 +118,21 @@ static bool pf_sk_ok(const GemmQArgs& a, int bm, int bn, bool bf) {
 static std::vector<PfPlan> pf_candidates(const GemmQArgs& a, bool bf) {
   std::vector<PfPlan> out;
   const int nk = a.K / 64;
-  for (int bm : {256, 128, 64})
-    for (int bn : {256, 128}) {
-      if (!pf_tile_ok(a, bn)) continue;
-      for (int S : {1, 2, 3, 4, 6, 8, 12, 16, -1}) {
-        if (a.ksplit > 0 && S != a.ksplit) continue;
-        if (S < 0 && !pf_sk_ok(a, bm, bn, bf)) continue;
-        if (S > 1 && (pf_no_split(a) || nk / S < 2)) continue;
-        if (!bf && bn == 256 && (a.K / 256) / S < 1) continue;
-        PfPlan p;
-        p.bm = bm; p.bn = bn; p.s = S;
-        out.push_back(p);
-      }
+  for (const auto& t : PF_TILES) {
+    if (!pf_tile_ok(a, t.bm, t.bn)) continue;
+    for (int S : {1, 2, 3, 4, 6, 8, 12, 16, -1}) {
+      if (a.ksplit > 0 && S != a.ksplit) continue;
+      if (S < 0 && !pf_sk_ok(a, t.bm, t.bn, bf)) continue;
+      if (S > 1 && (pf_no_split(a) || nk / S < 2)) continue;
+      if (!bf && t.bn == 256 && (a.K / 256) / S < 1) continue;
+      // (not timed: slices that make over three rounds of workgroups)
+      const double wgs = (double)((a.M + t.bm - 1) / t.bm) * (a.N / t.bn) * S;
+      if (S > 1 && a.ksplit <= 0 && wgs > 3.0 * device_cu_count()) continue;
+      PfPlan p;
+      p.bm = t.bm; p.bn = t.bn; p.s = S;
+      out.push_back(p);
     }
+  }
   return out;
 }
 
@@ -157,21 +164,20 @@ static PfPlan pf_model_plan(const GemmQArgs& a, bool bf, bool s1_only) {
   int fbm = 0, fbn = 0;
   if (tile) std::sscanf(tile, "%dx%d", &fbm, &fbn);
   const int nk = a.K / 64;
-  for (int bm : {256, 128, 64}) {
-    for (int bn : {256, 128}) {
-      if (fbm && (bm != fbm || bn != fbn)) continue;
-      if (!pf_tile_ok(a, bn)) continue;
-      for (int S : {1, 2, 3, 4, 6, 8, 12, 16, -1}) {
-        if (a.ksplit > 0 && S != a.ksplit) continue;
-        if (a.ksplit <= 0 && split != 0 && S != split) continue;  // (AIOS_GEMM_PF_SPLIT=-1: stream-K)
-        if (S < 0 && (s1_only || !pf_sk_ok(a, bm, bn, bf))) continue;
-        if (S > 1 && (s1_only || pf_no_split(a) || nk / S < 2)) continue;
-        if (!bf && bn == 256 && (a.K / 256) / S < 1) continue;  // pf8c slices whole 256-blocks
-        const double t = pf_model(a, bm, bn, S, bf);
-        if (t < bt) {
-          bt = t;
-          best.bm = bm; best.bn = bn; best.s = S;
-        }
+  for (const auto& tile_ : PF_TILES) {
+    const int bm = tile_.bm, bn = tile_.bn;
+    if (fbm && (bm != fbm || bn != fbn)) continue;
+    if (!pf_tile_ok(a, bm, bn)) continue;
+    for (int S : {1, 2, 3, 4, 6, 8, 12, 16, -1}) {
+      if (a.ksplit > 0 && S != a.ksplit) continue;
+      if (a.ksplit <= 0 && split != 0 && S != split) continue;  // (AIOS_GEMM_PF_SPLIT=-1: stream-K)
+      if (S < 0 && (s1_only || !pf_sk_ok(a, bm, bn, bf))) continue;
+      if (S > 1 && (s1_only || pf_no_split(a) || nk / S < 2)) continue;
+      if (!bf && bn == 256 && (a.K / 256) / S < 1) continue;  // pf8c slices whole 256-blocks
+      const double t = pf_model(a, bm, bn, S, bf);
+      if (t < bt) {
+        bt = t;
+        best.bm = bm; best.bn = bn; best.s = S;
       }
     }
   }

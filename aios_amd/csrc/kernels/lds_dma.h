@@ -38,4 +38,39 @@ __device__ __forceinline__ void pf_glds4(const void* src, uint32_t lds) {
                : "memory");
 }
 
+// ... from a uniform base and a 32-bit byte offset per lane: no 64-bit addition per lane and request
+__device__ __forceinline__ void pf_glds16(const void* base, uint32_t off, uint32_t lds) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(off), "s"(base), "s"(lds)
+               : "memory");
+}
+__device__ __forceinline__ void pf_glds4(const void* base, uint32_t off, uint32_t lds) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(off), "s"(base), "s"(lds)
+               : "memory");
+}
+
+// ... both uniform operands through v_readfirstlane, for a request inside a branch that not all lanes take (the compiler
+// puts uniform values into vector registers there); s_nop: a scalar register written by the vector unit is read as
+// an address five cycles later at the earliest
+template <int LANES, int BYTES>
+__device__ __forceinline__ void pf_glds_part(const void* base, uint32_t off, uint32_t lds) {
+  const uint64_t b = (uint64_t)base;
+  const uint64_t u = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
+  const uint32_t to = __builtin_amdgcn_readfirstlane(lds);
+  if ((threadIdx.x & 63) < LANES) {
+    uint32_t keep;
+    if constexpr (BYTES == 16)
+      asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                   : "=&s"(keep) : "v"(off), "s"(u), "s"(to) : "memory");
+    else
+      asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
+                   : "=&s"(keep) : "v"(off), "s"(u), "s"(to) : "memory");
+  }
+}
+
 }  // namespace aios

@@ -922,7 +922,7 @@ void LayeredDecoder::tune() {
   HIP_CHECK(hipMalloc(&tmp, (size_t)step_rows_ * dp_ * 4));
   fill_random_f32(tmp, (size_t)step_rows_ * dp_, 0x7u, 0.f, 1.f, e_.stream_);
   launch_f32_to_bf16(tmp, h16_, (size_t)step_rows_ * dp_, e_.stream_);
-  for (int M = 64; M <= step_rows_; M *= 2) {
+  for (int M = 64; M <= step_rows_; M = gemm_pf_bucket(M + 1)) {
     auto go = [&](const bf16_t* A, int lda, const bf16_t* wt, int N, int K, int epi, float* C, int ldc, bf16_t* C16, int act) {
       GemmQArgs g;
       std::memset(&g, 0, sizeof(g));

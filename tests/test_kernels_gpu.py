@@ -1315,6 +1315,45 @@ def test_gemm_pf_stream_k(E, monkeypatch, fmt, N, K, tile, epi):
     assert per_row < 1e-2, per_row
 
 
+@pytest.mark.parametrize("tile", ["64x128", "96x128", "128x128", "160x128"])
+@pytest.mark.parametrize("fmt", list(PF_SEGS))
+@pytest.mark.parametrize("M,K,S", [(33, 256, 1), (96, 256, 2), (97, 1280, 1), (160, 1280, 3), (161, 512, 1), (300, 1280, -1)])
+def test_gemm_pf_two_k_groups(E, monkeypatch, tile, fmt, M, K, S):
+    """128-column tiles below 256 rows: two groups of waves on half of the K-steps each, down to one step per group,
+    slices on even K-steps, rows just at and past a tile's edge"""
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    if S < 0:
+        monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", "-1")
+    mats, W = pf_mats(E, fmt, K)
+    N = W.shape[0]
+    want = [int(v) for v in tile.split("x")] + [S]
+    if list(E.gemm_pf_plan(mats, M, E.GEPI_ACCUM, max(S, 0))) != want:
+        pytest.skip("no such plan for this shape")
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M))
+    A = x.to(torch.bfloat16).cuda()
+    for epi, base in ((E.GEPI_STORE, 0.0), (E.GEPI_ACCUM, 1.0)):
+        C = torch.full((M, N), 1.0, device="cuda")
+        E.gemm_q(A.data_ptr(), K, mats, M, C.data_ptr(), 0, N, epi, stream(), max(S, 0))
+        torch.cuda.synchronize()
+        ref, got = x.double() @ W.double().T, C.cpu().double() - base
+        per_row = ((got - ref).norm(dim=1) / ref.norm(dim=1)).max().item()
+        assert per_row < 1e-2, per_row
+
+
+def test_gemm_pf_odd_k_steps(E):
+    """bf16, K an odd number of 64s: a tile without K groups, also where only 128-column ones divide N"""
+    for N in (384, 512):
+        m, W = qmat(E, GGMLType.BF16, N, 192, seed=5, std=0.05)
+        x = torch.randn(100, 192, generator=torch.Generator().manual_seed(N))
+        A, C = x.to(torch.bfloat16).cuda(), torch.zeros(100, N, device="cuda")
+        bm, bn, _ = E.gemm_pf_plan([m], 100, E.GEPI_STORE, 0)
+        assert bm == 256 or bn == 256
+        E.gemm_q(A.data_ptr(), 192, [m], 100, C.data_ptr(), 0, N, E.GEPI_STORE, stream(), 0)
+        torch.cuda.synchronize()
+        ref = x.double() @ W.double().T
+        assert float((C.cpu().double() - ref).norm() / ref.norm()) < 6e-3
+
+
 @pytest.mark.parametrize("tile", ["256x256", "128x256", "64x128"])
 @pytest.mark.parametrize("M", [40, 300])
 def test_gemm_pf_swiglu(E, monkeypatch, tile, M):

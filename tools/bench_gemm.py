@@ -79,7 +79,7 @@ def main():
                 C = torch.zeros(M, N, device="cuda")
                 C16 = torch.zeros(M, N // 2, device="cuda", dtype=torch.bfloat16)
                 plan = E.gemm_pf_plan([m], M, E.GEPI_ACCUM, 0)
-                for tile in ("256x256", "128x256", "64x256", "256x128", "128x128", "64x128"):
+                for tile in ("256x256", "128x256", "64x256", "256x128", "160x128", "128x128", "96x128", "64x128"):
                     os.environ["AIOS_GEMM_PF_TILE"] = tile
                     for S in ((1,) if epi == "swiglu" else (1, 2, 4, 8)):
                         if epi == "swiglu":
