@@ -14,8 +14,9 @@
 
 namespace aios {
 
-// the value of x's leading bf16
-__device__ __forceinline__ float bf16_part(float x) { return __uint_as_float(pk_bf16(x, 0.f) << 16); }
+// the two values of a bf16 pair
+__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
 __device__ __forceinline__ void st_wt(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -117,6 +118,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const uint8_t* p,
   const uint64_t u = (uint64_t)p;
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
   return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), (short)0, n, 0x00020000);
+}
+// the lane's number, computed here and now (the asm has no inputs to be hoisted with)
+__device__ __forceinline__ int lane_again() {
+  int z = 0;
+  asm volatile("" : "+s"(z));
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
 }
 constexpr int AT_TK = 32;   // keys per tile: one wave's unit of work
 // LDS row (bytes) of a wave's V tile: rows 32 B apart mod 256, so the 8 rows x 32 B that half a wave's
@@ -312,26 +319,19 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
     // ---- P^T's bf16 parts: this column's term0 (NR passes: term0, term0 + 2)
     gbf16x8 pf[NR];
     {
-      float r0[8], r1[8];
+      uint32_t w[NR][4];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float hi = bf16_part(p[i]);
-        const float rm = p[i] - hi;          // (exact)
-        const float lo = rm - bf16_part(rm);  // (exact: 8 bits left)
-        const uint32_t pu = __float_as_uint(p[i]), mu = __float_as_uint(rm), lu = __float_as_uint(lo);
-        if constexpr (GP == 4) {
-          r0[i] = __uint_as_float((pu & sel0) | (mu & sel1) | (lu & sel2));
-        } else {
-          r0[i] = __uint_as_float((pu & sel0) | (mu & sel1));
-          r1[i] = __uint_as_float(lu & sel0);
-        }
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t hi = pk_bf16(p[2 * i], p[2 * i + 1]);
+        const float r0 = p[2 * i] - bf16_lo(hi), r1 = p[2 * i + 1] - bf16_hi(hi);  // (exact)
+        const uint32_t mid = pk_bf16(r0, r1);
+        const uint32_t lo = pk_bf16(r0 - bf16_lo(mid), r1 - bf16_hi(mid));          // (exact: 8 bits left)
+        w[0][i] = (hi & sel0) | (mid & sel1);
+        if constexpr (GP == 4) w[0][i] |= lo & sel2;
+        else w[1][i] = lo & sel0;
       }
-      uint4 u = make_uint4(pk_bf16(r0[0], r0[1]), pk_bf16(r0[2], r0[3]), pk_bf16(r0[4], r0[5]), pk_bf16(r0[6], r0[7]));
-      __builtin_memcpy(&pf[0], &u, 16);
-      if constexpr (NR == 2) {
-        u = make_uint4(pk_bf16(r1[0], r1[1]), pk_bf16(r1[2], r1[3]), pk_bf16(r1[4], r1[5]), pk_bf16(r1[6], r1[7]));
-        __builtin_memcpy(&pf[1], &u, 16);
-      }
+#pragma unroll
+      for (int r = 0; r < NR; ++r) __builtin_memcpy(&pf[r], w[r], 16);
     }
     // ---- V to the wave's LDS tile, row-major
 #pragma unroll
@@ -378,19 +378,22 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
       if constexpr (GP == 4) o[i][e] += dpp<0x124>(o[i][e]);         // row_ror:4
     }
   __syncthreads();  // every wave is done with its V tile: the LDS is the merge's
-  if (col < G) {
+  // (the thread's number read again, opaque to the compiler: kept through the loop it costs registers that spill)
+  const int tid = wave * 64 + lane_again();
+  const int mlane = tid & 63, mc = tid & 15, mq = mlane >> 4;
+  if (mc < G) {
 #pragma unroll
-    for (int i = 0; i < DT; ++i) *(float4*)&s_o[wave][col][16 * i + 4 * q4] = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
-    if (q4 == 0) {
-      s_m[wave][col] = m;
-      s_l[wave][col] = l;
+    for (int i = 0; i < DT; ++i) *(float4*)&s_o[wave][mc][16 * i + 4 * mq] = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
+    if (mq == 0) {
+      s_m[wave][mc] = m;
+      s_l[wave][mc] = l;
     }
   }
   const float vs = F8 ? a.kv_scale_v : 1.f;
   __syncthreads();
   stamp(3);
   const int nact = P;  // workgroups that arrive
-  for (int idx = threadIdx.x; idx < G * HD; idx += NT) {
+  for (int idx = tid; idx < G * HD; idx += NT) {
     const int g = idx / HD, d = idx - g * HD;
     float M = s_m[0][g];
 #pragma unroll
@@ -424,7 +427,7 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains its sc1 stores
   __syncthreads();
   int* cnt = a.counters + (size_t)b * a.n_heads + ci;
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     const int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s_last = (t == nact - 1);
   }
@@ -447,14 +450,14 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   // sweep and folds them after the weights are ready -- same order of sums as the two-trip path
   auto one_trip = [&](auto ob) __attribute__((always_inline)) {
     constexpr int OB = decltype(ob)::value;
-    const int idx = threadIdx.x;
+    const int idx = tid;
     const bool act = idx < G * HD;
     const int g = act ? idx / HD : 0, d = act ? idx - g * HD : 0;
     const float* op = a.o_part + ((size_t)b * a.n_heads + h0 + g) * a.n_chunks * HD + d;
     float ov[OB];
 #pragma unroll
     for (int j = 0; j < OB; ++j) ov[j] = ld_wt(op + (size_t)min(j, nact - 1) * HD);  // clamped: in bounds
-    for (int i = threadIdx.x; i < G * nact; i += NT) {
+    for (int i = tid; i < G * nact; i += NT) {
       const int gg = i / nact, p = i - gg * nact;
       const float* mlp = a.ml + (((size_t)b * a.n_heads + h0 + gg) * a.n_chunks + p) * 2;
       s_pm[gg][p] = ld_wt(mlp);
@@ -462,8 +465,8 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
     }
     __syncthreads();
     if (wave < G) {
-      const float mv = lane < nact ? s_pm[wave][lane] : kNeg;
-      const float lv = lane < nact ? s_pl[wave][lane] : 0.f;
+      const float mv = mlane < nact ? s_pm[wave][mlane] : kNeg;
+      const float lv = mlane < nact ? s_pl[wave][mlane] : 0.f;
       float M = mv;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
@@ -471,7 +474,7 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
       float L = e * lv;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
-      if (lane < nact) s_pm[wave][lane] = e / L;
+      if (mlane < nact) s_pm[wave][mlane] = e / L;
     }
     __syncthreads();
     stamp(5);
@@ -490,11 +493,11 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
     if (nact <= 8) one_trip(std::integral_constant<int, 8>{});
     else if (nact <= 16) one_trip(std::integral_constant<int, 16>{});
     else one_trip(std::integral_constant<int, 32>{});
-    if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
+    if (tid == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
     stamp(6);
     return;
   }
-  for (int i = threadIdx.x; i < G * nact; i += NT) {
+  for (int i = tid; i < G * nact; i += NT) {
     const int g = i / nact, p = i - g * nact;
     const float* mlp = a.ml + (((size_t)b * a.n_heads + h0 + g) * a.n_chunks + p) * 2;
     s_pm[g][p] = ld_wt(mlp);
@@ -503,8 +506,8 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   __syncthreads();
   if (wave < G) {
     const int g = wave;
-    const float mv = lane < nact ? s_pm[g][lane] : kNeg;
-    const float lv = lane < nact ? s_pl[g][lane] : 0.f;
+    const float mv = mlane < nact ? s_pm[g][mlane] : kNeg;
+    const float lv = mlane < nact ? s_pl[g][mlane] : 0.f;
     float M = mv;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
@@ -512,11 +515,11 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
     float L = e * lv;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
-    if (lane < nact) s_pm[g][lane] = e / L;
+    if (mlane < nact) s_pm[g][mlane] = e / L;
   }
   __syncthreads();
   stamp(5);
-  for (int idx = threadIdx.x; idx < G * HD; idx += NT) {
+  for (int idx = tid; idx < G * HD; idx += NT) {
     const int g = idx / HD, d = idx - g * HD;
     const int h = h0 + g;
     const float* op = a.o_part + ((size_t)b * a.n_heads + h) * a.n_chunks * HD + d;
@@ -533,7 +536,7 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
     else if (a.out_wt) st_wt(a.out + ((size_t)b * a.n_heads + h) * HD + d, acc);
       else a.out[((size_t)b * a.n_heads + h) * HD + d] = acc;
   }
-  if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
+  if (tid == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
   stamp(6);
 }
 
