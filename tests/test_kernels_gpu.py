@@ -1036,6 +1036,37 @@ def test_gemm_ring_swiglu(E, M):
     assert torch.allclose(out.float().cpu(), ref, atol=2e-2, rtol=2e-2), (out.float().cpu() - ref).abs().max()
 
 
+@pytest.mark.parametrize("M", [2, 7, 16, 17, 32])
+@pytest.mark.parametrize("N,K,ksplit", [(128, 64, 0), (384, 2112, 0), (256, 1088, 3), (128, 4160, 16)])
+@pytest.mark.parametrize("epi", ["store", "accum", "store16", "swiglu"])
+def test_gemm_ring_bf16(E, M, N, K, ksplit, epi):
+    """bf16 weights through the ring, slots of 64 k: one slot, odd counts of them, slices of unequal length, the
+    deepest split.  The products are exact: float64 differs by the fp32 sums (K 2^-24) and a
+    16-bit result's rounding (half a unit of 8 bits: up to 2^-8 of the value)."""
+    g = torch.Generator().manual_seed(K + M)
+    W = (torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16)
+    m = E.QMatrix(int(GGMLType.BF16), N, K, W.view(torch.int16).numpy())
+    A = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    y, Ad = A.double() @ W.double().T, A.cuda()
+    tol = K * 2.0 ** -24 + (2.0 ** -8 if epi in ("store16", "swiglu") else 0.0)
+    for _ in range(2):  # the second launch re-uses the re-armed tickets
+        if epi == "swiglu":
+            out = torch.zeros(M, N // 2, dtype=torch.bfloat16, device="cuda")
+            E.gemm_q(Ad.data_ptr(), K, [m], M, 0, out.data_ptr(), N // 2, E.GEPI_SWIGLU_BF16, stream(), ksplit)
+            ref = torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2]
+        elif epi == "store16":
+            out, ref = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda"), y
+            E.gemm_q(Ad.data_ptr(), K, [m], M, 0, out.data_ptr(), N, E.GEPI_STORE16, stream(), ksplit)
+        else:
+            out = torch.full((M, N), 3.0, device="cuda")
+            ref = y + (3.0 if epi == "accum" else 0.0)
+            E.gemm_q(Ad.data_ptr(), K, [m], M, out.data_ptr(), 0, N, E.GEPI_ACCUM if epi == "accum" else E.GEPI_STORE,
+                     stream(), ksplit)
+        torch.cuda.synchronize()
+        got = out.cpu().double()
+        assert ((got - ref).norm(dim=1) / ref.norm(dim=1)).max() < tol
+
+
 # ---- the LDS-DMA engine serving B = 2..4 rows from one weight stream (small-batch decode) --------
 @pytest.mark.parametrize("t", [GGMLType.Q4_K, GGMLType.Q6_K, GGMLType.Q5_K, GGMLType.Q8_0])
 @pytest.mark.parametrize("K", [4096, 14336])
