@@ -711,9 +711,9 @@ void Engine::finalize() {
         const int parts = gemm_skinny_ntile(p);
         if (nrm_fuse_ && parts > 0 && parts % 4 == 0 && parts <= 64 && d % 128 == 0) {
           const int Gs = std::min(G, 64);
-          gm_nparts_ = parts;
+          gm_nparts_ = d / 16;
           gm_xn16_ = (bf16_t*)dmalloc((size_t)Gs * d * 2);
-          gm_npart_ = fbuf((size_t)Gs * parts);
+          gm_npart_ = fbuf((size_t)Gs * gm_nparts_);
           ws += (size_t)Gs * d * 2;
         }
       }
@@ -728,7 +728,7 @@ void Engine::finalize() {
         if (nrm_fuse_ && Bm <= 64 && parts > 0 && parts % 4 == 0 && parts <= 64 && d % 128 == 0) {
           nrm_parts_ = parts;
           dec_xn16_ = (bf16_t*)dmalloc((size_t)Bm * d * 2);
-          nrm_part_ = fbuf((size_t)Bm * parts);
+          nrm_part_ = fbuf((size_t)Bm * (d / 16));
           ws += (size_t)Bm * d * 2;
         }
         // TP: the all-reduce after O / down writes the next GEMM's split-norm operand itself
@@ -913,12 +913,12 @@ void Engine::layer_decode_gemm(int l, int B) {
   bf16_t* vc = kv_layer(v_cache_, l);
   // consumer side of the split RMSNorm: A = bf16(x * g) from the previous residual GEMM
   auto nrm_in = [&](GemmQArgs& g) {
-    g.A = dec_xn16_; g.nrm_in = nrm_part_; g.nrm_parts = nrm_parts_; g.nrm_eps = cfg_.norm_eps;
+    g.A = dec_xn16_; g.nrm_in = nrm_part_; g.nrm_parts = d / 16; g.nrm_eps = cfg_.norm_eps;
   };
   // producer side: residual add + bf16(x_new * g_next) + per-tile sums of squares
   auto nrm_out = [&](GemmQArgs& g, const float* g_next) {
     g.epi = GEPI_ACCUM_NORM; g.nrm_g = g_next; g.nrm_out16 = dec_xn16_; g.nrm_part = nrm_part_;
-    g.nrm_parts = nrm_parts_;
+    g.nrm_parts = d / 16;
   };
   // TP: the same contract, produced by the fused all-reduce (C1 / C2) into tpn_part_
   auto tpn_in = [&](GemmQArgs& g) {
@@ -999,7 +999,7 @@ void Engine::layer_decode_gemm(int l, int B) {
   if (fn) nrm_out(g, g_next);
   nrm_lm_ = (fn || tpn) && l + 1 == cfg_.n_layers;
   lm_nrm_in_ = tpn ? tpn_part_ : nrm_part_;
-  lm_nrm_parts_ = tpn ? tpn_parts_ : nrm_parts_;
+  lm_nrm_parts_ = tpn ? tpn_parts_ : d / 16;
   gemm(g);
   if (tp) tp_reduce(attn_, g_next);
 }
@@ -1250,7 +1250,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
   static const bool short_fuse = !(std::getenv("AIOS_PREFILL_SHORT_FUSE") && std::atoi(std::getenv("AIOS_PREFILL_SHORT_FUSE")) == 0);
   for (int r0 = 0; r0 < T; r0 += gm_rows_) {
     const int n = std::min(gm_rows_, T - r0);
-    // (the fused epilogues are the ring GEMM's: chunks of <= 32 rows; longer chunks take the prefill
+    // (the fused epilogues are the batched-decode GEMMs': chunks of <= 32 rows; longer chunks take the prefill
     // GEMM, kernels/gemm_pf.hip, with the plain epilogues)
     const bool sh = short_fuse && !tp && n <= 32;
     const bool fnp = sh && gm_nparts_ > 0;

@@ -184,7 +184,7 @@ static PfPlan pf_model_plan(const GemmQArgs& a, bool bf, bool s1_only) {
   return best;
 }
 
-// Serves M >= AIOS_GEMM_PF_MIN_M (default 33: the ring GEMM keeps 5..32) for Q4_K / Q5_K / Q6_K / mixed
+// Serves M >= AIOS_GEMM_PF_MIN_M (default 33: gemm_wk.hip keeps 2..32) for Q4_K / Q5_K / Q6_K / mixed
 // Q4_K|Q6_K, Q5_K|Q6_K / Q4_0 / Q8_0 / bf16 weight stacks with the STORE / ACCUM / SWIGLU epilogues; false -> the caller's
 // fallback (formats and fused epilogues this kernel does not do).
 static bool pf_eligible(const GemmQArgs& a);

@@ -19,10 +19,7 @@
 // the MP x 256 bf16 X rows of those k (skinny's xsw swizzle).  Steps are lock-stepped with raw
 // s_barrier (in-flight LDS-DMA survives it) exactly as in the batch-1 engine.
 //
-// bf16 weights: a slot is 64 k of the tile's rows, 128 B a row like the codes of a quantised superblock, and the 16-byte
-// units are the MFMA operands as they are.  (The register-streamed skinny GEMM meets at a barrier every 128 k and has
-// 64 KB a CU in flight: the 16-row step of a 2.6 GB model took 2151 us with it and takes 1999 with the ring; 9 rows of
-// TinyLlama, 8 steps, 10806 -> 10092.)
+// Serves what gemm_wk.hip leaves: long K in Q6_K up to 16 rows, and K or a workspace that its slices do not fit.
 #include "skinny_epi.h"
 
 namespace aios {
@@ -30,7 +27,6 @@ namespace aios {
 constexpr int RG_RB = 8;  // MFMA waves: 128-row tiles
 constexpr int RG_NL = 2;  // loader waves
 constexpr int RG_SMAX = 8;  // K slices at most (the engine sizes its split-K slabs for 8: gemm_skinny_ws_bytes)
-constexpr int RG_SMAX_BF = 16;  // bf16: narrow outputs (2048 columns: 16 tiles) fill the chip with 16; slabs as they allow
 constexpr int RG_THREADS = (RG_RB + RG_NL) * 64;
 
 // XR (M <= 8): the workgroup's X slice (8 rows x <= 4096 k, bf16, row stride + 16 B against bank
@@ -45,24 +41,23 @@ constexpr int RG_XR_BYTES = (RG_XR_ROWS * (RG_XR_KMAX + 8) * 2 + 255) / 256 * 25
 
 template <int QT, int MT, bool XR = false>
 struct RgLayout {
-  static constexpr bool Q6 = QT == QT_Q6_K, BF = QT == QT_BF16;
+  static constexpr bool Q6 = QT == QT_Q6_K;
   static constexpr int MP = 16 * MT;
-  static constexpr int KB = BF ? 64 : 256;          // k of a slot
   static constexpr int CODES = 128 * 128;           // 8 chunks x 16 B per row
   static constexpr int HI = Q6 ? 128 * 64 : 0;      // Q6_K: 8 B of high bits per chunk
-  static constexpr int META = BF ? 0 : 128 * 16;    // Q4_K: scale/min record; Q6_K: 8 int8 scale pairs
+  static constexpr int META = 128 * 16;             // Q4_K: scale/min record; Q6_K: 8 int8 scale pairs
   static constexpr int DQ = Q6 ? 512 : 0;           // Q6_K: the aligned dword holding the row's f16 d
-  static constexpr int XB = XR ? 0 : MP * KB * 2;   // X rows, bf16 (XR: resident, not in the slot)
+  static constexpr int XB = XR ? 0 : MP * 256 * 2;  // X rows, bf16 (XR: resident, not in the slot)
   static constexpr int OFF_HI = CODES, OFF_META = OFF_HI + HI, OFF_D = OFF_META + META, OFF_X = OFF_D + DQ;
   static constexpr int SLOT = (OFF_X + XB + 255) / 256 * 256;
   // DMA instructions per slot: 1 KB each, Q6_K d as 4-byte pieces (256 B per instruction: a narrow
   // LDS-DMA lands lane i at base + 4 i whatever its width -- measured, a 2-byte one zero-fills)
-  static constexpr int NI_CODES = 16, NI_HI = HI / 1024, NI_META = META / 1024, NI_D = Q6 ? 2 : 0, NI_X = XB / 1024;
+  static constexpr int NI_CODES = 16, NI_HI = HI / 1024, NI_META = 2, NI_D = Q6 ? 2 : 0, NI_X = XB / 1024;
   static constexpr int TI = NI_CODES + NI_HI + NI_META + NI_D + NI_X;
   static constexpr int PL = (TI + RG_NL - 1) / RG_NL;  // per loader (exact: the vmcnt immediates)
   // (one slot below what fits: a smaller chip-wide prologue burst lands the first slot sooner, as
   // measured for the batch-1 engine, profiles/decode_mistral_rocprof_r4_final.txt)
-  static constexpr int RFIT = std::min(BF ? 8 : 6, (150 * 1024 - (XR ? RG_XR_BYTES : 0)) / SLOT);
+  static constexpr int RFIT = std::min(6, (150 * 1024 - (XR ? RG_XR_BYTES : 0)) / SLOT);
   static constexpr int R = RFIT >= 4 ? RFIT - RG_RSUB : RFIT;
   static_assert(R >= 3 && (R - 2) * PL <= 63, "ring depth / vmcnt immediate");
 };
@@ -114,14 +109,9 @@ __device__ __forceinline__ void rg_dma_slot(const GemmQArgs& a, const QWeight& w
       width = 4;
     } else {  // X: dest unit u = (m, ud) holds k units ud ^ h(m) of row m (rows past M re-read row M-1)
       j -= L::NI_D;
-      if constexpr (L::BF) {  // rows of 128 B, unit ud of row m holds k unit ud ^ (m >> 1 & 7)
-        const int u = 64 * j + lane, m = u >> 3, ud = u & 7;
-        src = (const uint8_t*)(a.A + (size_t)min(m, a.M - 1) * a.lda + sb * 64 + 8 * (ud ^ ((m >> 1) & 7)));
-      } else {
-        const int u = 64 * j + lane, m = u >> 5, ud = u & 31;
-        const int mm = min(m, a.M - 1);
-        src = (const uint8_t*)(a.A + (size_t)mm * a.lda + sb * 256 + 8 * (ud ^ rg_xh(m)));
-      }
+      const int u = 64 * j + lane, m = u >> 5, ud = u & 31;
+      const int mm = min(m, a.M - 1);
+      src = (const uint8_t*)(a.A + (size_t)mm * a.lda + sb * 256 + 8 * (ud ^ rg_xh(m)));
       region = L::OFF_X + j * 1024;
     }
     auto* ldst = (__attribute__((address_space(3))) void*)(dst + region);
@@ -154,22 +144,6 @@ __device__ __forceinline__ void rg_compute_slot(const uint8_t* slot, int sb, int
   const int rr = lane & 15, q = lane >> 4;
   const int r = 16 * wave + rr;  // tile row
   const bf16_t* xs = (const bf16_t*)(slot + L::OFF_X);
-  if constexpr (L::BF) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const uint4 w = *(const uint4*)(slot + r * 128 + (((4 * u + q) ^ (r & 7)) << 4));
-      gbf16x8 wf, xf;
-      __builtin_memcpy(&wf, &w, 16);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int m = 16 * mt + rr;
-        const uint4 xv = *(const uint4*)(slot + L::OFF_X + m * 128 + (((4 * u + q) ^ ((m >> 1) & 7)) << 4));
-        __builtin_memcpy(&xf, &xv, 16);
-        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc[mt], 0, 0, 0);
-      }
-    }
-    return;
-  } else
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int cc = q + 4 * u;  // chunk within the superblock
@@ -240,7 +214,7 @@ __device__ __forceinline__ void rg_body(const GemmQArgs& a, int S, int rg, int s
   w.p2 = s == 0 ? a.seg[0].p2 : (s == 1 ? a.seg[1].p2 : a.seg[2].p2);
   w.p3 = s == 0 ? a.seg[0].p3 : (s == 1 ? a.seg[1].p3 : a.seg[2].p3);
   const int row0 = n0 - (s == 0 ? a.seg_n0[0] : (s == 1 ? a.seg_n0[1] : a.seg_n0[2]));
-  const int nbk = a.K / L::KB;
+  const int nbk = a.K >> 8;
   const int sb0 = (int)((long)sp * nbk / S), sb1 = (int)((long)(sp + 1) * nbk / S);
   const int T = sb1 - sb0;  // ring steps (>= 1: S <= nbk)
   uint8_t* ring = rg_smem + (XR ? RG_XR_BYTES : 0);
@@ -316,24 +290,9 @@ __global__ void __launch_bounds__(RG_THREADS) gemm_ring_kernel(GemmQArgs a, int 
   __shared__ float inv_s[MP];
   const bool nrm = a.nrm_in != nullptr;
   if (nrm) {
-    // all of a row's (<= 64, multiple-of-4) partial sums requested at once: a dependent load per
-    // part held wave 0 -- a loader wave -- ~3 us before its first weight request
-    for (int m = threadIdx.x; m < MP; m += RG_THREADS) {
-      float t = 0.f;
-      if (m < a.M) {
-        const float4* p = (const float4*)(a.nrm_in + (size_t)m * a.nrm_parts);
-        const int n4 = a.nrm_parts >> 2;
-#pragma unroll
-        for (int h = 0; h < 16; h += 8) {
-          float4 v[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = h + j < n4 ? p[h + j] : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) t += (v[j].x + v[j].y) + (v[j].z + v[j].w);
-        }
-      }
-      inv_s[m] = rsqrtf(t / (float)a.K + a.nrm_eps);
-    }
+    NrmRows<MP, RG_THREADS / 64> nr;
+    nr.load(a, threadIdx.x >> 6, threadIdx.x & 63);
+    nr.done(a, threadIdx.x >> 6, threadIdx.x & 63, inv_s);
     // ordered before the epilogue by the ring's barriers
   }
   float* is = nrm ? inv_s : nullptr;
@@ -354,13 +313,11 @@ static int rg_env(const char* name, int dflt) {
 template <int QT0, int QT1, int MT, bool XR>
 static bool rg_launch(const GemmQArgs& a, hipStream_t st) {
   const int ntile = a.N / 128;
-  constexpr bool BF = QT0 == QT_BF16;
-  const int nbk = a.K / RgLayout<QT0, MT, XR>::KB;
+  const int nbk = a.K / 256;
   const int cus = device_cu_count();
   // one dispatch round: tiles x slices <= CUs (one 640-thread workgroup per CU, LDS-bound)
   int S = a.ksplit > 0 ? a.ksplit : std::max(1, cus / ntile);
-  S = std::max(1, std::min({S, nbk, BF ? RG_SMAX_BF : RG_SMAX}));
-  if (BF && a.ws) S = std::max(1, std::min(S, (int)(a.ws_bytes / ((size_t)16 * MT * a.N * 4))));
+  S = std::max(1, std::min({S, nbk, RG_SMAX}));
   if (S > 1 && (!a.ws || !a.cnt || a.cnt_len < ntile || a.ws_bytes < (size_t)S * 16 * MT * a.N * 4)) S = 1;
   if (XR && ((nbk + S - 1) / S) * 256 > RG_XR_KMAX) return false;  // the resident slice must fit
   const size_t lds = (size_t)(XR ? RG_XR_BYTES : 0) +
@@ -373,12 +330,6 @@ static bool rg_launch(const GemmQArgs& a, hipStream_t st) {
     case GEPI_QKV: RG_GO(GEPI_QKV); break;
     case GEPI_ACCUM: RG_GO(GEPI_ACCUM); break;
     case GEPI_ACCUM_NORM: RG_GO(GEPI_ACCUM_NORM); break;
-    case GEPI_STORE16:
-      if constexpr (BF) RG_GO(GEPI_STORE16);
-      break;
-    case GEPI_STORE_GLU:
-      if constexpr (BF) RG_GO(GEPI_STORE_GLU);
-      break;
     default: RG_GO(GEPI_SWIGLU_BF16); break;
   }
 #undef RG_GO
@@ -386,36 +337,31 @@ static bool rg_launch(const GemmQArgs& a, hipStream_t st) {
 }
 
 // AIOS_GEMM_RING: 1 (default) = the ring GEMM serves the batched-decode shapes it supports
-// (M 5..32, Q4_K / Q6_K / mixed Q4_K|Q6_K / bf16, 128-row tiles, K % 256 == 0, bf16 K % 64 == 0); 0 = skinny only
+// (M 5..32, Q4_K / Q6_K / mixed Q4_K|Q6_K, 128-row tiles, K % 256 == 0); 0 = skinny only
 bool launch_gemm_ring(const GemmQArgs& a, hipStream_t st) {
   static const int on = rg_env("AIOS_GEMM_RING", 1);
   static const int min_m = rg_env("AIOS_GEMM_RING_MIN_M", 2);
-  const int qt0 = a.seg[0].qtype, qt1 = a.seg[a.nseg - 1].qtype;
-  const bool bf = qt0 == QT_BF16;
-  if ((a.epi == GEPI_STORE16 || a.epi == GEPI_STORE_GLU) && !bf) return false;
-  if (!on || a.M < min_m || a.M > 32 || a.N % 128 || a.K % (bf ? 64 : 256) || a.lda % 8) return false;
-  if (bf && ((uintptr_t)a.A & 15)) return false;  // (16-byte requests)
-  if (a.nrm_in && (a.nrm_parts <= 0 || a.nrm_parts > 64 || a.nrm_parts % 4)) return false;
+  if (a.epi == GEPI_STORE16 || a.epi == GEPI_STORE_GLU) return false;
+  if (!on || a.M < min_m || a.M > 32 || a.N % 128 || a.K % 256 || a.lda % 8) return false;
+  if (a.nrm_in && (a.nrm_parts <= 0 || a.nrm_parts % 4)) return false;
   if (a.epi == GEPI_SWIGLU_BF16 && a.ldc % 2) return false;
-  if (a.epi == GEPI_STORE_GLU && (a.glu_n0 % 4 || a.ldc16 % 2)) return false;
   if (a.epi != GEPI_SWIGLU_BF16 && a.ldc % 4) return false;
   for (int s = 0; s < a.nseg; ++s)
     if (a.seg_n0[s] % 128 || a.seg[s].rows % 128) return false;
-  // the split-RMSNorm producer's per-tile partials follow the skinny kernel's 128-row tiles too
-  if (a.epi == GEPI_ACCUM_NORM && (!a.nrm_g || !a.nrm_out16 || !a.nrm_part || a.N / 128 != a.nrm_parts)) return false;
+  if (a.epi == GEPI_ACCUM_NORM && (!a.nrm_g || !a.nrm_out16 || !a.nrm_part || a.N / 16 != a.nrm_parts)) return false;
+  const int qt0 = a.seg[0].qtype, qt1 = a.seg[a.nseg - 1].qtype;
   for (int s = 0; s + 1 < a.nseg; ++s)
     if (a.seg[s].qtype != qt0) return false;
+#ifdef AIOS_BF16_ONLY
+  return false;
+#else
   auto go = [&](auto mt, auto xr) {
     constexpr int MT = decltype(mt)::value;
     constexpr bool XR = decltype(xr)::value;
-    if constexpr (!XR)
-      if (bf && qt1 == QT_BF16) return rg_launch<QT_BF16, QT_BF16, MT, false>(a, st);
-#ifndef AIOS_BF16_ONLY
     if (qt0 == QT_Q4_K && qt1 == QT_Q4_K) return rg_launch<QT_Q4_K, QT_Q4_K, MT, XR>(a, st);
     if (qt0 == QT_Q6_K && qt1 == QT_Q6_K) return rg_launch<QT_Q6_K, QT_Q6_K, MT, XR>(a, st);
     if (qt0 == QT_Q4_K && qt1 == QT_Q6_K && (a.epi == GEPI_QKV || a.epi == GEPI_STORE))
       return rg_launch<QT_Q4_K, QT_Q6_K, MT, XR>(a, st);
-#endif
     return false;
   };
   // AIOS_RING_XR (default 1): M <= 8 with the X slice resident in LDS (falls back when it does not fit)
@@ -423,6 +369,7 @@ bool launch_gemm_ring(const GemmQArgs& a, hipStream_t st) {
   if (a.M <= RG_XR_ROWS && xr_on && go(std::integral_constant<int, 1>{}, std::true_type{})) return true;
   if (a.M <= 16) return go(std::integral_constant<int, 1>{}, std::false_type{});
   return go(std::integral_constant<int, 2>{}, std::false_type{});
+#endif
 }
 
 }  // namespace aios

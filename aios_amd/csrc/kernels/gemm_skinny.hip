@@ -193,39 +193,19 @@ __device__ __forceinline__ void sk_body(const GemmQArgs& a, int S) {
     }
   };
 
-  // ---- fused RMSNorm (consumer): the producer's per-tile sums of squares, nG <= 16 lanes per row
-  // (power of two >= parts / 4, one float4 each), loaded before everything else and reduced in a
-  // fixed order once the first X chunk has landed -> inv_s[m]
-  constexpr int NR = (MP * 16 + NT - 1) / NT;
+  // ---- fused RMSNorm (consumer): the producer's sums of squares, loaded before everything else and added up once the
+  // first X chunk has landed -> inv_s[m]
   __shared__ float inv_s[MP];
   const bool nrm = a.nrm_in != nullptr;
-  int nlg = 0;
-  gf32x4 nv[NR];
-  if (nrm) {
-    const int p4 = a.nrm_parts >> 2;
-    while ((1 << nlg) < p4) ++nlg;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int u = tid + NT * r, m = u >> nlg, j = u & ((1 << nlg) - 1);
-      nv[r] = gf32x4{0.f, 0.f, 0.f, 0.f};
-      if (m < a.M && j < p4) nv[r] = *(const gf32x4*)(a.nrm_in + (size_t)m * a.nrm_parts + 4 * j);
-    }
-  }
+  NrmRows<MP, NT / 64> nr;
+  if (nrm) nr.load(a, wave, lane);
   // prologue: X chunk c0 first (oldest loads), then the weight ring, then X chunk c0+1
   x_load(c0);
 #pragma unroll
   for (int u = 0; u < SK_NL; ++u) w_load(tb + u, ring[u], !MB || (u & 1) == 0);
   stamp(1);
   x_store(0, c0);
-  if (nrm) {
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int u = tid + NT * r, m = u >> nlg;
-      float s = (nv[r][0] + nv[r][1]) + (nv[r][2] + nv[r][3]);
-      for (int o = 1; o < (1 << nlg); o <<= 1) s += __shfl_xor(s, o, 64);
-      if ((u & ((1 << nlg) - 1)) == 0 && m < MP) inv_s[m] = rsqrtf(s / (float)a.K + a.nrm_eps);
-    }
-  }
+  if (nrm) nr.done(a, wave, lane, inv_s);
   x_load(min(c0 + 1, c1 - 1));
   __syncthreads();
   stamp(2);
@@ -263,7 +243,7 @@ __global__ void __launch_bounds__(RB * 64) gemm_skinny_kernel(GemmQArgs a, int S
   sk_body<QT0, RB, MT, EPI>(a, S);
 }
 
-int gemm_skinny_cnt_len(int N) { return N / 64 + 1; }
+int gemm_skinny_cnt_len(int N) { return N / 16 + 1; }
 
 static int sk_env(const char* name, int dflt) {
   const char* e = std::getenv(name);
@@ -324,8 +304,8 @@ static bool sk_fits(const GemmQArgs& a) {
   if ((a.epi == GEPI_STORE16 || a.epi == GEPI_STORE_GLU) && a.seg[0].qtype != QT_BF16) return false;
   if (a.epi == GEPI_STORE_GLU && (a.glu_n0 % 4 || a.ldc16 % 2)) return false;
   if ((a.epi != GEPI_SWIGLU_BF16 && a.ldc % 4) || a.lda % 8) return false;
-  if (a.nrm_in && (a.nrm_parts % 4 || a.nrm_parts > 64)) return false;
-  if (a.epi == GEPI_ACCUM_NORM && (!a.nrm_g || !a.nrm_out16 || !a.nrm_part || a.N / (16 * sk_rb(a)) != a.nrm_parts))
+  if (a.nrm_in && (a.nrm_parts % 4 || a.nrm_parts <= 0)) return false;
+  if (a.epi == GEPI_ACCUM_NORM && (!a.nrm_g || !a.nrm_out16 || !a.nrm_part || a.N / 16 != a.nrm_parts))
     return false;
   switch (a.seg[0].qtype) {
     case QT_Q4_K: case QT_Q5_K: case QT_Q6_K: case QT_Q4_0: case QT_Q8_0: case QT_F16: case QT_BF16: return true;

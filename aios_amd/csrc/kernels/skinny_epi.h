@@ -11,6 +11,102 @@ namespace aios {
 
 constexpr int SK_SB = 8;  // slices summed per batch of loads in the last arriver
 
+// One lane's 4 outputs of row m, columns n .. n + 3 (v), through the epilogue; inv_s: the fused RMSNorm's row scales or
+// null; res: the residual if the caller has read it.  Returns the sum of squares of the new residual row slice (GEPI_ACCUM_NORM), else 0.
+template <int EPI>
+__device__ __forceinline__ float sk_finish(const GemmQArgs& a, const float* inv_s, int m, int n, gf32x4 v,
+                                           const float4* res = nullptr) {
+  if (m >= a.M) return 0.f;
+  if (inv_s) v *= inv_s[m];
+  if constexpr (EPI == GEPI_SWIGLU_BF16) {
+    const uint32_t pk = pk_bf16(glu_act(v[0], a.act) * v[1], glu_act(v[2], a.act) * v[3]);
+    *(uint32_t*)(a.C16 + (size_t)m * a.ldc + (n >> 1)) = pk;
+  } else if constexpr (EPI == GEPI_STORE16) {
+    if (a.bias16 || a.unary)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = store16_val(a, n + j, v[j]);
+    *(uint2*)(a.C16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]));
+  } else if constexpr (EPI == GEPI_STORE_GLU) {
+    if (n < a.glu_n0)  // (a multiple of 4: the lane's 4 columns are on one side)
+      *(float4*)(a.C + (size_t)m * a.ldc + n) = make_float4(v[0], v[1], v[2], v[3]);
+    else
+      *(uint32_t*)(a.C16 + (size_t)m * a.ldc16 + ((n - a.glu_n0) >> 1)) =
+          pk_bf16(glu_act(v[0], a.act) * v[1], glu_act(v[2], a.act) * v[3]);
+  } else if constexpr (EPI == GEPI_QKV) {
+    // the lane's 4 consecutive columns are two RoPE pairs (2i, 2i + 1)
+    const int hd = a.head_dim, pos = a.pos[m], slot = a.slot ? a.slot[m] : 0;
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+      const int c = a.col0 + n + j;
+      float v0 = v[j], v1 = v[j + 1];
+      const int part = c < a.q_dim ? 0 : (c < a.q_dim + a.kv_dim ? 1 : 2);
+      const int r = c - (part == 0 ? 0 : (part == 1 ? a.q_dim : a.q_dim + a.kv_dim));
+      const int head = r / hd, lr = r - head * hd;
+      if (part < 2) {
+        const float2 t = a.rope_cs[(size_t)pos * (hd >> 1) + (lr >> 1)];
+        const float o0 = v0 * t.x - v1 * t.y, o1 = v0 * t.y + v1 * t.x;
+        v0 = o0;
+        v1 = o1;
+      }
+      if (part == 0) {
+        *(float2*)(a.q_out + (size_t)m * a.q_dim + c) = make_float2(v0, v1);
+      } else {
+        bf16_t* cache = part == 1 ? a.k_cache : a.v_cache;
+        const size_t base = kv_offset(a.block_table, a.max_ctx / KV_BLOCK, slot, a.n_kv_heads, head, pos, hd);
+        if (a.kv_fp8) kv_store_pair(cache, base + lr, base + lr + 1, v0, v1, 1, part == 1 ? a.kv_inv_k : a.kv_inv_v);
+        else *(uint32_t*)(cache + base + lr) = pk_bf16(v0, v1);
+      }
+    }
+  } else {
+    float4* c = (float4*)(a.C + (size_t)m * a.ldc + n);
+    if constexpr (EPI == GEPI_ACCUM_NORM) {
+      if (a.bias16) v += *(const gf32x4*)(a.bias16 + n);
+      const float4 o = res ? *res : *c;
+      const float4 x = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
+      *c = x;
+      const float4 g = *(const float4*)(a.nrm_g + n);
+      *(uint2*)(a.nrm_out16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(x.x * g.x, x.y * g.y),
+                                                                    pk_bf16(x.z * g.z, x.w * g.w));
+      return (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w);
+    } else if constexpr (EPI == GEPI_ACCUM) {
+      const float4 o = res ? *res : *c;
+      *c = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
+    } else {
+      *c = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  }
+  return 0.f;
+}
+
+// The fused RMSNorm's consumer: inv_s[m] of MP rows from the producer's sums of squares (nrm_parts per row, a multiple
+// of 4), a wave per row, added up in a fixed order.  load() requests, done() writes inv_s (ordered by the caller).
+template <int MP, int NW>
+struct NrmRows {
+  static constexpr int R = (MP + NW - 1) / NW;
+  gf32x4 v[R];
+  __device__ __forceinline__ void load(const GemmQArgs& a, int wave, int lane) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int m = wave + NW * r;
+      v[r] = gf32x4{0.f, 0.f, 0.f, 0.f};
+      if (m < a.M && 4 * lane < a.nrm_parts) v[r] = *(const gf32x4*)(a.nrm_in + (size_t)m * a.nrm_parts + 4 * lane);
+    }
+  }
+  __device__ __forceinline__ void done(const GemmQArgs& a, int wave, int lane, float* inv_s) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int m = wave + NW * r;
+      if (m >= MP) continue;
+      for (int j = 256 + 4 * lane; j < a.nrm_parts; j += 256)
+        if (m < a.M) v[r] += *(const gf32x4*)(a.nrm_in + (size_t)m * a.nrm_parts + j);
+      float s = (v[r][0] + v[r][1]) + (v[r][2] + v[r][3]);
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
+      if (lane == 0) inv_s[m] = rsqrtf(s / (float)a.K + a.nrm_eps);
+    }
+  }
+};
+
 // Returns false for a split-K workgroup that was not its tile's last arriver (nothing written).
 // red: >= RB * 16 * MT floats of workgroup-shared scratch (free after the main loop);
 // last_flag: a __shared__ int of the caller.  NTB: threads of the workgroup, which ALL call this
@@ -25,68 +121,13 @@ __device__ __forceinline__ bool sk_epilogue(const GemmQArgs& a, gf32x4 (&acc)[MT
   const int rr = lane & 15, q = lane >> 4;
   // ---- epilogue.  lane holds D[n = 4q + j][m = 16 mt + rr], j = 0..3
   const int nl = 16 * wave + 4 * q;  // tile-local first row of this lane's 4 outputs
-  // returns the sum of squares of the new residual row slice (GEPI_ACCUM_NORM), else 0
   auto finish = [&](int m, int n, gf32x4 v) __attribute__((always_inline)) -> float {
-    if (m >= a.M) return 0.f;
-    if (nrm) v *= inv_s[m];
-    if constexpr (EPI == GEPI_SWIGLU_BF16) {
-      const uint32_t pk = pk_bf16(glu_act(v[0], a.act) * v[1], glu_act(v[2], a.act) * v[3]);
-      *(uint32_t*)(a.C16 + (size_t)m * a.ldc + (n >> 1)) = pk;
-    } else if constexpr (EPI == GEPI_STORE16) {
-      if (a.bias16 || a.unary)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = store16_val(a, n + j, v[j]);
-      *(uint2*)(a.C16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]));
-    } else if constexpr (EPI == GEPI_STORE_GLU) {
-      if (n < a.glu_n0)  // (a multiple of 4: the lane's 4 columns are on one side)
-        *(float4*)(a.C + (size_t)m * a.ldc + n) = make_float4(v[0], v[1], v[2], v[3]);
-      else
-        *(uint32_t*)(a.C16 + (size_t)m * a.ldc16 + ((n - a.glu_n0) >> 1)) =
-            pk_bf16(glu_act(v[0], a.act) * v[1], glu_act(v[2], a.act) * v[3]);
-    } else if constexpr (EPI == GEPI_QKV) {
-      // the lane's 4 consecutive columns are two RoPE pairs (2i, 2i + 1)
-      const int hd = a.head_dim, pos = a.pos[m], slot = a.slot ? a.slot[m] : 0;
-#pragma unroll
-      for (int j = 0; j < 4; j += 2) {
-        const int c = a.col0 + n + j;
-        float v0 = v[j], v1 = v[j + 1];
-        const int part = c < a.q_dim ? 0 : (c < a.q_dim + a.kv_dim ? 1 : 2);
-        const int r = c - (part == 0 ? 0 : (part == 1 ? a.q_dim : a.q_dim + a.kv_dim));
-        const int head = r / hd, lr = r - head * hd;
-        if (part < 2) {
-          const float2 t = a.rope_cs[(size_t)pos * (hd >> 1) + (lr >> 1)];
-          const float o0 = v0 * t.x - v1 * t.y, o1 = v0 * t.y + v1 * t.x;
-          v0 = o0;
-          v1 = o1;
-        }
-        if (part == 0) {
-          *(float2*)(a.q_out + (size_t)m * a.q_dim + c) = make_float2(v0, v1);
-        } else {
-          bf16_t* cache = part == 1 ? a.k_cache : a.v_cache;
-          const size_t base = kv_offset(a.block_table, a.max_ctx / KV_BLOCK, slot, a.n_kv_heads, head, pos, hd);
-          if (a.kv_fp8) kv_store_pair(cache, base + lr, base + lr + 1, v0, v1, 1, part == 1 ? a.kv_inv_k : a.kv_inv_v);
-          else *(uint32_t*)(cache + base + lr) = pk_bf16(v0, v1);
-        }
-      }
-    } else {
-      float4* c = (float4*)(a.C + (size_t)m * a.ldc + n);
-      if constexpr (EPI == GEPI_ACCUM_NORM) {
-        if (a.bias16) v += *(const gf32x4*)(a.bias16 + n);
-        const float4 o = *c;
-        const float4 x = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
-        *c = x;
-        const float4 g = *(const float4*)(a.nrm_g + n);
-        *(uint2*)(a.nrm_out16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(x.x * g.x, x.y * g.y),
-                                                                      pk_bf16(x.z * g.z, x.w * g.w));
-        return (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w);
-      } else if constexpr (EPI == GEPI_ACCUM) {
-        const float4 o = *c;
-        *c = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
-      } else {
-        *c = make_float4(v[0], v[1], v[2], v[3]);
-      }
-    }
-    return 0.f;
+    return sk_finish<EPI>(a, nrm ? inv_s : nullptr, m, n, v);
+  };
+  // a tile's sum of squares stands in the first of its ROWS / 16 parts, zeros in the others
+  auto put_part = [&](int m, float s) __attribute__((always_inline)) {
+    float* p = a.nrm_part + (size_t)m * a.nrm_parts + rg * RB;
+    for (int j = 0; j < RB; ++j) p[j] = j ? 0.f : s;
   };
   if (S == 1) {
     float ss[MT];
@@ -106,7 +147,7 @@ __device__ __forceinline__ bool sk_epilogue(const GemmQArgs& a, gf32x4 (&acc)[MT
       if (tid < a.M) {
         float s = red[tid];
         for (int w = 1; w < RB; ++w) s += red[w * MP + tid];
-        a.nrm_part[(size_t)tid * a.nrm_parts + rg] = s;
+        put_part(tid, s);
       }
     }
     return true;
@@ -153,7 +194,7 @@ __device__ __forceinline__ bool sk_epilogue(const GemmQArgs& a, gf32x4 (&acc)[MT
       // a row's ROWS / 4 units sit on consecutive lanes of one wave
 #pragma unroll
       for (int o = 1; o < ROWS / 4; o <<= 1) s += __shfl_xor(s, o, 64);
-      if (n4 == 0 && m < a.M) a.nrm_part[(size_t)m * a.nrm_parts + rg] = s;
+      if (n4 == 0 && m < a.M) put_part(m, s);
     }
   }
   return true;

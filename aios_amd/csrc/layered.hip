@@ -867,9 +867,9 @@ void LayeredDecoder::finalize() {
       p.M = 64; p.N = dp_; p.K = dims_[0].kout; p.nseg = 1; p.seg[0] = mat(w_[owner_[0]].out, dp_, dims_[0].kout);
       const int parts = gemm_skinny_ntile(p);
       if (parts > 0 && parts % 4 == 0 && parts <= 64) {
-        nparts_ = parts;
+        nparts_ = dp_ / 16;
         xn16_ = balloc((size_t)64 * dp_);
-        npart_ = falloc((size_t)64 * parts);
+        npart_ = falloc((size_t)64 * nparts_);
       }
     }
   }

@@ -240,8 +240,8 @@ struct GemmQArgs {
   float kv_inv_k, kv_inv_v;
   // RMSNorm split across two skinny GEMMs (batched decode: no normalisation launch).
   //  producer (GEPI_ACCUM_NORM = residual add): also writes bf16(x_new * nrm_g) to nrm_out16
-  //    [M][ldc] and, per output tile t, sum_n x_new[m][n]^2 to nrm_part[m * nrm_parts + t]
-  //    (nrm_parts = gemm_skinny_ntile(producer args); fixed-order reductions, no atomics)
+  //    [M][ldc] and, per 16 columns t, sum_n x_new[m][n]^2 to nrm_part[m * nrm_parts + t]
+  //    (nrm_parts = N / 16; wider tiles: their sum in the first part and zeros in the others; fixed order)
   //  consumer (any epilogue, nrm_in set): A is that bf16(x * g); output row m is scaled by
   //    rsqrt(sum_t nrm_in[m * nrm_parts + t] / K + nrm_eps) before the epilogue
   const float* nrm_g;

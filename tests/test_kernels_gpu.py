@@ -1036,31 +1036,49 @@ def test_gemm_ring_swiglu(E, M):
     assert torch.allclose(out.float().cpu(), ref, atol=2e-2, rtol=2e-2), (out.float().cpu() - ref).abs().max()
 
 
-@pytest.mark.parametrize("M", [2, 7, 16, 17, 32])
-@pytest.mark.parametrize("N,K,ksplit", [(128, 64, 0), (384, 2112, 0), (256, 1088, 3), (128, 4160, 16)])
+# ---- K over the waves (gemm_wk.hip): the same rows, Q4_K / Q6_K / mixed / bf16 -----------------------------------
+@pytest.mark.parametrize("M", [2, 15, 16, 17, 32])
+@pytest.mark.parametrize("segs,K,ksplit", [
+    ([("Q4_K", 64)], 256, 0), ([("Q4_K", 4288)], 2304, 0), ([("Q6_K", 192)], 4352, 0), ([("Q4_K", 128)], 14336, 0),
+    ([("Q6_K", 128)], 2560, 3), ([("Q4_K", 256), ("Q4_K", 64), ("Q6_K", 64)], 4096, 0),
+    ([("Q4_K", 3968), ("Q4_K", 192), ("Q6_K", 192)], 4352, 2),
+    ([("BF16", 64)], 64, 0), ([("BF16", 4288)], 2112, 0), ([("BF16", 128)], 8256, 0), ([("BF16", 192)], 1088, 8)])
 @pytest.mark.parametrize("epi", ["store", "accum", "store16", "swiglu"])
-def test_gemm_ring_bf16(E, M, N, K, ksplit, epi):
-    """bf16 weights through the ring, slots of 64 k: one slot, odd counts of them, slices of unequal length, the
-    deepest split.  The products are exact: float64 differs by the fp32 sums (K 2^-24) and a
-    16-bit result's rounding (half a unit of 8 bits: up to 2^-8 of the value)."""
+def test_gemm_wk(E, M, segs, K, ksplit, epi):
+    """waves with no k, uneven slices and tile ranges, ranges per format, K split over workgroups.  The kernel's weights
+    are bf16, and so are the reference's; products are exact, so float64 differs by the fp32 sums (K 2^-24), by a
+    16-bit result's rounding (up to 2^-8) and, quantised, by weights at a rounding boundary (scale arithmetic in fp32:
+    one in ~2^14 off by 2^-8, so 2^-13 in all is ample)"""
+    bf, mixed = segs[0][0] == "BF16", len(segs) > 1
+    if (epi == "store16" and not bf) or (mixed and epi != "store"):
+        pytest.skip("not a form of this format")
     g = torch.Generator().manual_seed(K + M)
-    W = (torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16)
-    m = E.QMatrix(int(GGMLType.BF16), N, K, W.view(torch.int16).numpy())
-    A = torch.randn(M, K, generator=g).to(torch.bfloat16)
-    y, Ad = A.double() @ W.double().T, A.cuda()
-    tol = K * 2.0 ** -24 + (2.0 ** -8 if epi in ("store16", "swiglu") else 0.0)
+    mats, W = [], []
+    for i, (t, n) in enumerate(segs):
+        if bf:
+            w = (torch.randn(n, K, generator=g) * 0.05).to(torch.bfloat16)
+            mats.append(E.QMatrix(int(GGMLType.BF16), n, K, w.view(torch.int16).numpy()))
+        else:
+            m, w = qmat(E, GGMLType[t], n, K, seed=70 + i, std=0.05)
+            mats.append(m)
+        W.append(w.to(torch.bfloat16).double())
+    W = torch.cat(W)
+    N, lda = W.shape[0], K + 8
+    A = torch.randn(M, lda, generator=g).to(torch.bfloat16)
+    y, Ad = A[:, :K].double() @ W.T, A.cuda()
+    tol = K * 2.0 ** -24 + (2.0 ** -8 if epi in ("store16", "swiglu") else 0.0) + (0.0 if bf else 2.0 ** -13)
     for _ in range(2):  # the second launch re-uses the re-armed tickets
         if epi == "swiglu":
             out = torch.zeros(M, N // 2, dtype=torch.bfloat16, device="cuda")
-            E.gemm_q(Ad.data_ptr(), K, [m], M, 0, out.data_ptr(), N // 2, E.GEPI_SWIGLU_BF16, stream(), ksplit)
+            E.gemm_q(Ad.data_ptr(), lda, mats, M, 0, out.data_ptr(), N // 2, E.GEPI_SWIGLU_BF16, stream(), ksplit)
             ref = torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2]
         elif epi == "store16":
             out, ref = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda"), y
-            E.gemm_q(Ad.data_ptr(), K, [m], M, 0, out.data_ptr(), N, E.GEPI_STORE16, stream(), ksplit)
+            E.gemm_q(Ad.data_ptr(), lda, mats, M, 0, out.data_ptr(), N, E.GEPI_STORE16, stream(), ksplit)
         else:
             out = torch.full((M, N), 3.0, device="cuda")
             ref = y + (3.0 if epi == "accum" else 0.0)
-            E.gemm_q(Ad.data_ptr(), K, [m], M, out.data_ptr(), 0, N, E.GEPI_ACCUM if epi == "accum" else E.GEPI_STORE,
+            E.gemm_q(Ad.data_ptr(), lda, mats, M, out.data_ptr(), 0, N, E.GEPI_ACCUM if epi == "accum" else E.GEPI_STORE,
                      stream(), ksplit)
         torch.cuda.synchronize()
         got = out.cpu().double()

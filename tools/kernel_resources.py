@@ -32,6 +32,7 @@ HOT = [
     "aios::attn_decode_kernel<*",
     "aios::gemm_skinny_kernel<*",
     "aios::gemm_ring_kernel<*",
+    "aios::gemm_wk_kernel<*",
     "aios::sample_kernel*",
     "aios::get_rows_step_kernel*",
     "aios::latent_prep_kernel*",
