@@ -374,7 +374,8 @@ class Engine {
   // RMSNorm / mixed-QKV / split-K work, tools/gpu_minb_ab.sh: B=3 GEMV 956 vs GEMM 1065 tok/s, B=2 829 vs 712)
   // round 3: the LDS-DMA GEMV engine serves B = 2..4 from one weight stream (gemv_lds.h):
   // B = 2 / 3 / 4 1.82 / 2.29 / 2.45 ms vs the skinny GEMM's 3.25 / 2.83 / 2.84 (profiles/lds_batched_r3.txt)
-  int dec_gemm_min_b_ = 5;
+  int dec_gemm_min_b_ = 5;  // (where default_gemm_min_b() has no better number)
+  int default_gemm_min_b() const;
   bf16_t *dec_a16_ = nullptr, *dec_ff16_ = nullptr;
   // split-K slabs + arrival tickets of the skinny GEMM (shared by every decode GEMM of a step)
   float* gk_ws_ = nullptr;

@@ -668,6 +668,7 @@ void Engine::finalize() {
       if (const char* e = std::getenv("AIOS_DECODE_GEMM_MIN_B")) {
         dec_gemm_min_b_ = std::atoi(e);
       } else {
+        dec_gemm_min_b_ = default_gemm_min_b();
         // B rows go through the B-row LDS-DMA engine only if EVERY projection's LDS plan fits at that
         // B; where one does not (e.g. a 28672-wide down projection at B = 4: 115 KB of staged x), the
         // row-pair fallback is 2-3x slower than the skinny GEMM, so that B takes the GEMM path
@@ -895,6 +896,25 @@ void Engine::gemm(GemmQArgs& g) {
 // MFMA GEMM (weights dequantised once per step into MFMA operands, split-K reduced in-launch),
 // with explicit RMSNorm -> bf16 and RoPE/KV-write launches in place of the GEMV prologue /
 // epilogue fusions.  SwiGLU runs in the gate/up GEMM's epilogue (bf16 out for the down GEMM).
+// Rows from which the GEMMs win (us a step, 8 steps behind ~300 keys, GEMV / GEMM):
+//   TinyLlama Q4_K (25 MB a layer)   2 rows  912 / 798    3 rows 1044 / 801    4 rows 1101 / 796
+//   Mistral-7B Q4_K (123 MB)         2 rows 1761 / 2024   3 rows 1969 / 2025   4 rows 2231 / 2014
+//   Qwen3-8B Q4_K (108 MB)           2 rows 2130 / 2337   3 rows 2389 / 2348   4 rows 2685 / 2364
+//   TinyLlama bf16                   2 rows  852 / 1006   3 rows  919 / 1012   4 rows  976 / 1007
+// The int8 GEMV's dot work grows with the rows, the GEMM's does not: it wins from 4, and from 2 where the layers are
+// so small that launches bound a step.  Only where K-shared waves serve every projection (Q4_K / Q6_K) and the GEMV
+// would take int8 activations; across ranks as before.
+int Engine::default_gemm_min_b() const {
+  if (!cfg_.act_q8 || cfg_.tp_size > 1) return dec_gemm_min_b_;
+  size_t bytes = 0;
+  for (const auto& L : layers_)
+    for (const QMat* m : {&L.wq, &L.wk, &L.wv, &L.wo, &L.wgu, &L.wdown}) {
+      if (m->w.qtype != QT_Q4_K && m->w.qtype != QT_Q6_K) return dec_gemm_min_b_;
+      bytes += (size_t)m->w.rows * m->w.cols / 256 * (m->w.qtype == QT_Q4_K ? 144 : 210);
+    }
+  return std::min(dec_gemm_min_b_, bytes <= layers_.size() * ((size_t)64 << 20) ? 2 : 4);
+}
+
 bool Engine::nrm_on(int B) const { return nrm_parts_ > 0 && dec_xn16_ && cfg_.tp_size == 1 && B <= 64; }
 // AIOS_TP_NORM_FUSE=0 restores the separate RMSNorm launches after C1 / C2 (A/B and tests)
 bool Engine::tpn_on(int B) const {
