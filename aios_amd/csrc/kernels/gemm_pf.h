@@ -1327,6 +1327,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
     }
   };
   auto mfma_range = [&](const gbf16x8(&f)[GR], int p, int k0, int k1) __attribute__((always_inline)) {
+    if constexpr (BM < 256) __builtin_amdgcn_s_setprio(1);
     const int sp = p / NG, g = p % NG;
 #pragma unroll
     for (int k = 0; k < 2 * GR; ++k) {
@@ -1334,6 +1335,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
       const int c = k / GR, i = k % GR;
       acc[g * GR + i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i], bf[c][sp], acc[g * GR + i][c], 0, 0, 0);
     }
+    if constexpr (BM < 256) __builtin_amdgcn_s_setprio(0);
   };
   if constexpr (!(PROBE & 1)) pf_vmcnt<PW>();  // the prologue group landed (G(-2) in flight)
   read_raw(kt0, 0);
@@ -1342,6 +1344,12 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
   pf_barrier();
   ldA(pf_smem, fa, 0);
 
+  // The decode beside the MFMAs: at 256 rows its instructions are dealt out among the phase's MFMAs (in a run of their
+  // own, 40 to 60 of them, they left the matrix pipe idle whenever both waves of a SIMD were in it: 2048 x 4096 x 14336
+  // 337 -> 316 us, 2048 x 28672 x 4096 430 -> 420, 711 x 24576 x 4096 185 -> 179); below, where a phase has fewer
+  // MFMAs, the wave in them takes the issue port first (300 x 28672 x 4096 139 -> 129, 711 x 4096 x 4096 51.3 -> 47.8;
+  // at 256 rows priority gave half of what dealing gives, and both together nothing;
+  // without a decode, bf16, priority lost 2 %, and so it did in pf4's tiles).
   // four K-steps (a block) per turn of the loop: what a step takes from its place in the block -- record fields, DMA
   // pieces, buffer halves -- is then fixed in the code.  At 256 rows two: four spill registers, and the reloads'
   // waits drain the DMA (460 -> 537 us for 2048 x 28672 x 4096; two steps 448 us).  Vector instructions of a step and
@@ -1371,6 +1379,13 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
       if constexpr (!(PROBE & 4)) group(s - 1, (place + 3) & 3, pc);
       if constexpr (p + 1 < NPH) {
         mfma_range(cf, p, 0, 2 * GR);
+        if constexpr (BM == 256 && (p == 0 || p == NG)) {
+#pragma unroll
+          for (int i = 0; i < 2 * GR; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);               // a matrix instruction,
+            __builtin_amdgcn_sched_group_barrier(0x2, L::Q6 ? 5 : 3, 0);   // a few of the decode
+          }
+        }
       } else {
         mfma_range(cf, p, 0, GR);
         __builtin_amdgcn_sched_barrier(0);
