@@ -1673,19 +1673,23 @@ __global__ void __launch_bounds__(512) gemm_pf8_kernel(GemmQArgs a) {
 // that cost 4.  Here the first T - R tiles run as usual and each of the last R runs as TWO 128-row
 // workgroups (the BM = 128 body on its half), dispatched last: the final round puts half-size work
 // on every CU.  K-quant stacks, S = 1 (plans with split-K fill the chip their own way).
-template <int QT0, int QT1, int EPI>
+// PARTS = 4, where the last round fills at most a quarter (4 R <= CUs): four 64-row workgroups, so that still one
+// per CU is left for it (24576 x 4096 at 711 rows, 288 tiles: no split 215 us, halves 181, quarters 167).
+template <int QT0, int QT1, int EPI, int PARTS>
 __global__ void __launch_bounds__(512) gemm_pf8t_kernel(GemmQArgs a, int F) {
+  constexpr int BT = 256 / PARTS;
   const int nN = a.N / 256;
-  int L, half = -1;
+  int L, part = -1;
   if ((int)blockIdx.x < F) {
     L = xcd_remap(blockIdx.x, F);
   } else {
     const int j = xcd_remap(blockIdx.x - F, gridDim.x - F);
-    L = F + (j >> 1);
-    half = j & 1;
+    L = F + j / PARTS;
+    part = j % PARTS;
   }
   const int tn = L % nN, tm = L / nN;
-  const int m0 = tm * 256 + (half > 0 ? 128 : 0), n0 = tn * 256;
+  const int m0 = tm * 256 + (part > 0 ? part * BT : 0), n0 = tn * 256;
+  if (m0 >= a.M) return;
   int seg = 0;
   if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
   if (a.nseg > 2 && n0 >= a.seg_n0[2]) seg = 2;
@@ -1693,23 +1697,23 @@ __global__ void __launch_bounds__(512) gemm_pf8t_kernel(GemmQArgs a, int F) {
   if constexpr (pf8_generic<QT0, QT1>()) {
     if constexpr (QT0 != QT1) {
       if (seg == a.nseg - 1) {
-        if (half < 0) pf8_body<QT1, 256, EPI>(a, m0, n0, seg, 0, kt1, 1);
-        else pf8_body<QT1, 128, EPI>(a, m0, n0, seg, 0, kt1, 1);
+        if (part < 0) pf8_body<QT1, 256, EPI>(a, m0, n0, seg, 0, kt1, 1);
+        else pf8_body<QT1, BT, EPI>(a, m0, n0, seg, 0, kt1, 1);
         return;
       }
     }
-    if (half < 0) pf8_body<QT0, 256, EPI>(a, m0, n0, seg, 0, kt1, 1);
-    else pf8_body<QT0, 128, EPI>(a, m0, n0, seg, 0, kt1, 1);
+    if (part < 0) pf8_body<QT0, 256, EPI>(a, m0, n0, seg, 0, kt1, 1);
+    else pf8_body<QT0, BT, EPI>(a, m0, n0, seg, 0, kt1, 1);
   } else {
     if constexpr (QT0 != QT1) {
       if (seg == a.nseg - 1) {
-        if (half < 0) pf8c_body<QT1, 256, EPI>(a, m0, n0, seg, 0, kt1, 1);
-        else pf8c_body<QT1, 128, EPI>(a, m0, n0, seg, 0, kt1, 1);
+        if (part < 0) pf8c_body<QT1, 256, EPI>(a, m0, n0, seg, 0, kt1, 1);
+        else pf8c_body<QT1, BT, EPI>(a, m0, n0, seg, 0, kt1, 1);
         return;
       }
     }
-    if (half < 0) pf8c_body<QT0, 256, EPI>(a, m0, n0, seg, 0, kt1, 1);
-    else pf8c_body<QT0, 128, EPI>(a, m0, n0, seg, 0, kt1, 1);
+    if (part < 0) pf8c_body<QT0, 256, EPI>(a, m0, n0, seg, 0, kt1, 1);
+    else pf8c_body<QT0, BT, EPI>(a, m0, n0, seg, 0, kt1, 1);
   }
 }
 
@@ -1828,15 +1832,20 @@ void pf8_launch(const GemmQArgs& a, int S, hipStream_t st) {
   if constexpr (BM == 256 && QT0 != QT_BF16) {  // (K-quant stacks: the tail split)
     const int F = pf_tail_full(a, 256, S);
     if (F >= 0) {
-      constexpr int l128 = pf8_lds_bytes<QT0, QT1, 128>();
-      constexpr int ldst = lds > l128 ? lds : l128;
-      const int T = (a.N / 256) * ((a.M + 255) / 256);
-      const dim3 grid(F + 2 * (T - F)), block(512);
-      switch (a.epi) {
-        case GEPI_STORE: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_STORE>), grid, block, ldst, st, a, F); break;
-        case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_ACCUM>), grid, block, ldst, st, a, F); break;
-        default: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_SWIGLU_BF16>), grid, block, ldst, st, a, F); break;
-      }
+      constexpr int l128 = pf8_lds_bytes<QT0, QT1, 128>(), l64 = pf8_lds_bytes<QT0, QT1, 64>();
+      constexpr int ldst = std::max({lds, l128, l64});
+      const int T = (a.N / 256) * ((a.M + 255) / 256), R = T - F;
+      auto go = [&](auto parts) {
+        constexpr int P = decltype(parts)::value;
+        const dim3 grid(F + P * R), block(512);
+        switch (a.epi) {
+          case GEPI_STORE: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_STORE, P>), grid, block, ldst, st, a, F); break;
+          case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_ACCUM, P>), grid, block, ldst, st, a, F); break;
+          default: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_SWIGLU_BF16, P>), grid, block, ldst, st, a, F); break;
+        }
+      };
+      if (4 * R <= device_cu_count()) go(std::integral_constant<int, 4>{});
+      else go(std::integral_constant<int, 2>{});
       return;
     }
   }

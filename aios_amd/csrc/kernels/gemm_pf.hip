@@ -57,7 +57,7 @@ static double pf_model(const GemmQArgs& a, int bm, int bn, int S, bool bf) {
   double t = std::ceil(tiles * S / cus) * t_wg;
   const double R = std::fmod(tiles, cus);
   if (bm == 256 && S == 1 && (bn == 128 || !bf) && tiles > cus && R > 0 && 2 * R <= cus)  // tail split
-    t = (std::floor(tiles / cus) + 0.6) * t_wg;
+    t = (std::floor(tiles / cus) + (bn == 256 && 4 * R <= cus ? 0.4 : 0.6)) * t_wg;
   if (S > 1) t += (double)a.M * a.N * 4 * S / 1.2e12 + (a.epi == GEPI_STORE ? (double)a.M * a.N * 4 / 4e12 : 0.0);
   return t;
 }

@@ -1274,6 +1274,25 @@ def test_gemm_pf_tail_split(E, monkeypatch, epi, tile, N, fmt):
         assert rel < 6e-3, rel
 
 
+@pytest.mark.parametrize("fmt", [GGMLType.Q4_K, GGMLType.Q6_K, GGMLType.Q8_0])
+@pytest.mark.parametrize("N,M", [(24576, 711), (24576, 700), (16384, 1300), (16384, 1410)])
+def test_gemm_pf_tail_parts(E, monkeypatch, fmt, N, M):
+    """the last round in quarters (288 and 320 tiles, 32 / 64 left: the last quarter of seven rows, or past M) and in
+    halves (384, 128 left): bit-identical to the plain launch, which sums in the same order"""
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", "256x256")
+    K = 512
+    m, _ = qmat(E, fmt, N, K, seed=151, std=0.02)
+    A = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).cuda()
+    outs = []
+    for tail in ("1", "0"):
+        monkeypatch.setenv("AIOS_GEMM_PF_TAIL", tail)
+        C = torch.full((M, N), 0.25, device="cuda")
+        E.gemm_q(A.data_ptr(), K, [m], M, C.data_ptr(), 0, N, E.GEPI_ACCUM, stream(), 1)
+        torch.cuda.synchronize()
+        outs.append(C)
+    assert torch.isfinite(outs[0]).all() and float(outs[0].std()) > 0.1 and torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("segs,M", [([(GGMLType.Q4_K, 8192)], 2100),
                                     ([(GGMLType.Q4_K, 4096), (GGMLType.Q4_K, 1024), (GGMLType.Q6_K, 1024)], 2800)])
 @pytest.mark.parametrize("epi", ["store", "accum"])
