@@ -1072,6 +1072,7 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
            })
       .def_property_readonly("vocab_size", &JsonGrammar::vocab_size)
       .def_property_readonly("cache_size", &JsonGrammar::cache_size);
+  m.attr("GEMM_PF_PLANS_VERSION") = GEMM_PF_PLANS_VERSION;
   m.def("gemm_pf_export", &gemm_pf_export);
   m.def("gemm_pf_import", &gemm_pf_import, py::arg("plans"));
 #ifndef AIOS_BF16_ONLY

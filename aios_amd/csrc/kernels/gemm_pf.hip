@@ -114,22 +114,29 @@ static bool pf_sk_ok(const GemmQArgs& a, int bm, int bn, bool bf) {
   return units % 2 == 0 && units >= 4 && tiles < 2.0 * device_cu_count();
 }
 
+// whether the kernels take this tile and split for these args: candidates, modelled and stored plans alike (a stored one
+// may be another build's: pf_launch_fmt would run its tile with K cut as it does not cut it, or not at all)
+static bool pf_plan_ok(const GemmQArgs& a, const PfPlan& p, bool bf) {
+  bool tile = false;
+  for (const auto& t : PF_TILES) tile = tile || (t.bm == p.bm && t.bn == p.bn);
+  if (!tile || !pf_tile_ok(a, p.bm, p.bn)) return false;
+  if (p.s < 0) return pf_sk_ok(a, p.bm, p.bn, bf);
+  if (p.s == 0 || (p.s > 1 && (pf_no_split(a) || a.K / 64 / p.s < 2))) return false;
+  return bf || p.bn != 256 || a.K / 256 / p.s >= 1;  // (pf8c slices whole 256-blocks)
+}
+
 // every plan the launcher could run for these args (ksplit > 0 pins the split)
 static std::vector<PfPlan> pf_candidates(const GemmQArgs& a, bool bf) {
   std::vector<PfPlan> out;
-  const int nk = a.K / 64;
   for (const auto& t : PF_TILES) {
-    if (!pf_tile_ok(a, t.bm, t.bn)) continue;
     for (int S : {1, 2, 3, 4, 6, 8, 12, 16, -1}) {
       if (a.ksplit > 0 && S != a.ksplit) continue;
-      if (S < 0 && !pf_sk_ok(a, t.bm, t.bn, bf)) continue;
-      if (S > 1 && (pf_no_split(a) || nk / S < 2)) continue;
-      if (!bf && t.bn == 256 && (a.K / 256) / S < 1) continue;
+      PfPlan p;
+      p.bm = t.bm; p.bn = t.bn; p.s = S;
+      if (!pf_plan_ok(a, p, bf)) continue;
       // (not timed: slices that make over three rounds of workgroups)
       const double wgs = (double)((a.M + t.bm - 1) / t.bm) * (a.N / t.bn) * S;
       if (S > 1 && a.ksplit <= 0 && wgs > 3.0 * device_cu_count()) continue;
-      PfPlan p;
-      p.bm = t.bm; p.bn = t.bn; p.s = S;
       out.push_back(p);
     }
   }
@@ -140,15 +147,12 @@ static PfPlan pf_model_plan(const GemmQArgs& a, bool bf, bool s1_only);
 static PfPlan pf_plan(const GemmQArgs& a, bool bf) {
   if (!std::getenv("AIOS_GEMM_PF_TILE") && !std::getenv("AIOS_GEMM_PF_SPLIT") && a.ksplit <= 0) {
     std::lock_guard<std::mutex> g(pf_mu);
-    if (a.epi == GEPI_QKV || pf_deterministic()) {  // (the best plan without split partials)
-      GemmQArgs b = a;
-      if (a.epi == GEPI_QKV) b.epi = GEPI_STORE;
-      auto it = pf_tuned_s1().find(pf_key(b));
-      if (it != pf_tuned_s1().end()) return it->second;
-    } else {
-      auto it = pf_tuned().find(pf_key(a));
-      if (it != pf_tuned().end()) return it->second;
-    }
+    const bool s1 = a.epi == GEPI_QKV || pf_deterministic();  // (the best plan without split partials)
+    GemmQArgs b = a;
+    if (a.epi == GEPI_QKV) b.epi = GEPI_STORE;
+    const auto& plans = s1 ? pf_tuned_s1() : pf_tuned();
+    auto it = plans.find(pf_key(b));
+    if (it != plans.end() && pf_plan_ok(a, it->second, bf)) return it->second;
   }
   return pf_model_plan(a, bf, false);
 }
@@ -163,21 +167,19 @@ static PfPlan pf_model_plan(const GemmQArgs& a, bool bf, bool s1_only) {
   const int split = pf_env("AIOS_GEMM_PF_SPLIT", 0);
   int fbm = 0, fbn = 0;
   if (tile) std::sscanf(tile, "%dx%d", &fbm, &fbn);
-  const int nk = a.K / 64;
   for (const auto& tile_ : PF_TILES) {
     const int bm = tile_.bm, bn = tile_.bn;
     if (fbm && (bm != fbm || bn != fbn)) continue;
-    if (!pf_tile_ok(a, bm, bn)) continue;
     for (int S : {1, 2, 3, 4, 6, 8, 12, 16, -1}) {
       if (a.ksplit > 0 && S != a.ksplit) continue;
       if (a.ksplit <= 0 && split != 0 && S != split) continue;  // (AIOS_GEMM_PF_SPLIT=-1: stream-K)
-      if (S < 0 && (s1_only || !pf_sk_ok(a, bm, bn, bf))) continue;
-      if (S > 1 && (s1_only || pf_no_split(a) || nk / S < 2)) continue;
-      if (!bf && bn == 256 && (a.K / 256) / S < 1) continue;  // pf8c slices whole 256-blocks
+      PfPlan p;
+      p.bm = bm; p.bn = bn; p.s = S;
+      if ((S != 1 && s1_only) || !pf_plan_ok(a, p, bf)) continue;
       const double t = pf_model(a, bm, bn, S, bf);
       if (t < bt) {
         bt = t;
-        best.bm = bm; best.bn = bn; best.s = S;
+        best = p;
       }
     }
   }
@@ -244,20 +246,21 @@ static bool pf_eligible(const GemmQArgs& a) {
 
 // Time every candidate plan for these args (real buffers; outputs overwritten) and keep the fastest
 // for their M bucket.  Returns the number of candidates timed (0: not a prefill-GEMM launch, or a
-// key already planned in this process -- tuned by an earlier engine or imported, gemm_pf_import: a
-// second engine never changes the plans a first one runs).
+// key already planned in this process -- tuned by an earlier engine or imported, gemm_pf_import, and a plan that
+// the kernels take: a second engine never changes the plans a first one runs).
 //
-// Stable choice (ADVICE r5): a measured plan replaces the modelled one only when it is > 5 % faster,
+// Stable choice: a measured plan replaces the modelled one only when it is > 5 % faster,
 // so timing noise (a co-tenant, TP ranks sharing the GPU) does not pick a different tile / split in
 // each process; ties keep the earlier candidate (a fixed order).  TP ranks then take rank 0's plans
 // (tp.py broadcasts gemm_pf_export), and AIOS_GEMM_PF_PLANS persists them across processes.
 int gemm_pf_autotune(const GemmQArgs& a, hipStream_t st) {
   if (!pf_eligible(a)) return 0;
+  const bool bf = a.seg[0].qtype == QT_BF16;
   {
     std::lock_guard<std::mutex> g(pf_mu);
-    if (pf_tuned().count(pf_key(a))) return 0;
+    const auto it = pf_tuned().find(pf_key(a));
+    if (it != pf_tuned().end() && pf_plan_ok(a, it->second, bf)) return 0;
   }
-  const bool bf = a.seg[0].qtype == QT_BF16;
   const std::vector<PfPlan> cands = pf_candidates(a, bf);
   if (cands.empty()) return 0;
   const PfPlan mp = pf_model_plan(a, bf, false), mp1 = pf_model_plan(a, bf, true);

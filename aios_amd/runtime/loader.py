@@ -118,7 +118,8 @@ def finalize(eng):
     """Engine.finalize with the prefill-GEMM plans persisted when AIOS_GEMM_PF_PLANS names a file:
     plans saved by an earlier process are installed first (finalize then times only shapes it does
     not hold), and the process's plans are written back -- every process serving a model runs the
-    same tile / split plans (per-process tuning noise changed prefill numerics)."""
+    same tile / split plans (each process's own timing could pick others, and with them another order
+    of sums).  Plans timed on another version of the kernels are timed again."""
     import json
 
     m = native.require()
@@ -126,15 +127,19 @@ def finalize(eng):
     if path and os.path.exists(path):
         try:
             with open(path) as f:
-                m.gemm_pf_import([int(v) for v in json.load(f)])
-        except (OSError, ValueError, RuntimeError) as e:
+                held = json.load(f)
+            if isinstance(held, dict) and held.get("version") == m.GEMM_PF_PLANS_VERSION:
+                m.gemm_pf_import([int(v) for v in held["plans"]])
+            else:
+                log.info("prefill plan file %s is of other kernels: timing again", path)
+        except (OSError, ValueError, KeyError, TypeError, RuntimeError) as e:
             log.warning("ignoring prefill plan file %s: %s", path, e)
     eng.finalize()
     if path:
         tmp = f"{path}.{os.getpid()}.tmp"
         try:
             with open(tmp, "w") as f:
-                json.dump(list(m.gemm_pf_export()), f)
+                json.dump({"version": m.GEMM_PF_PLANS_VERSION, "plans": list(m.gemm_pf_export())}, f)
             os.replace(tmp, path)
         except OSError as e:
             log.warning("cannot persist prefill plans to %s: %s", path, e)

@@ -1422,6 +1422,35 @@ def test_gemm_pf_odd_k_steps(E):
         assert float((C.cpu().double() - ref).norm() / ref.norm()) < 6e-3
 
 
+def pf_plan_entry(E, N, K, M, epi, bm, bn, S, s1=0):
+    """one line of a plan list for a bf16 matrix: shape, row bucket, epilogue, formats, segments, CUs; tile, slices, map"""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return [N, K, M, epi, int(GGMLType.BF16), int(GGMLType.BF16), 1, 0, 0, cus, bm, bn, S, s1]
+
+
+@pytest.mark.parametrize("K,N,tile", [(192, 640, (64, 128, 1)), (192, 896, (128, 128, 1)), (320, 640, (96, 128, 2)),
+                                      (320, 384, (160, 128, 1)), (128, 384, (64, 256, 1)), (128, 640, (64, 128, 3)),
+                                      (192, 1152, (64, 128, -1)), (128, 896, (48, 128, 1)), (128, 1152, (64, 128, 0))])
+def test_gemm_pf_imported_plan_that_does_not_fit(E, K, N, tile):
+    """a stored plan is one of this build's tiles and cuts K as its kernel does, or the modelled one serves: two K groups
+    (K an odd number of 64s), a width that does not divide N, more slices than K-steps, stream-K of too few, no such tile"""
+    E.gemm_pf_import(pf_plan_entry(E, N, K, 128, E.GEPI_STORE, *tile) + pf_plan_entry(E, N, K, 128, E.GEPI_STORE, *tile, s1=1))
+    m, W = qmat(E, GGMLType.BF16, N, K, seed=5, std=0.05)
+    assert list(E.gemm_pf_plan([m], 100, E.GEPI_STORE, 0)) != list(tile)
+    x = torch.randn(100, K, generator=torch.Generator().manual_seed(N)).to(torch.bfloat16)
+    A, C = x.cuda(), torch.zeros(100, N, device="cuda")
+    E.gemm_q(A.data_ptr(), K, [m], 100, C.data_ptr(), 0, N, E.GEPI_STORE, stream(), 0)
+    torch.cuda.synchronize()
+    ref = x.double() @ W.to(torch.bfloat16).double().T
+    assert float((C.cpu().double() - ref).norm() / ref.norm()) < K * 2.0 ** -24
+
+
+def test_gemm_pf_imported_plan_that_fits(E):
+    m, W = qmat(E, GGMLType.BF16, 1408, 256, seed=5, std=0.05)
+    E.gemm_pf_import(pf_plan_entry(E, 1408, 256, 128, E.GEPI_STORE, 64, 128, 2))
+    assert list(E.gemm_pf_plan([m], 100, E.GEPI_STORE, 0)) == [64, 128, 2]
+
+
 @pytest.mark.parametrize("tile", ["256x256", "128x256", "64x128"])
 @pytest.mark.parametrize("M", [40, 300])
 def test_gemm_pf_swiglu(E, monkeypatch, tile, M):

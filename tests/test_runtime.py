@@ -416,3 +416,22 @@ def test_tier_context_follows_reference_size_heuristic(tmp_path):
     with open(f, "wb") as fh:
         fh.truncate(9 * 10**9)  # sparse: only the size is read
     assert tier_context(get_preset("mistral-7b").__class__(**{**get_preset("mistral-7b").__dict__}), str(f)) == 8192
+
+
+@pytest.mark.parametrize("held,installed", [({"version": 7, "plans": [1] * 14}, [1] * 14), ({"version": 6, "plans": [1] * 14}, None),
+                                            ([1] * 14, None), ({"version": 7}, None), ("{", None)])
+def test_prefill_plan_file_holds_its_kernels_version(tmp_path, monkeypatch, held, installed):
+    """plans of this build's kernels are installed; another version's, a list without one and a broken file are not, and
+    the file is written anew with the process's plans"""
+    from types import SimpleNamespace
+
+    from aios_amd.runtime import loader
+
+    got, path = [], tmp_path / "plans.json"
+    path.write_text(held if isinstance(held, str) else json.dumps(held))
+    m = SimpleNamespace(GEMM_PF_PLANS_VERSION=7, gemm_pf_import=got.append, gemm_pf_export=lambda: [2] * 14)
+    monkeypatch.setattr(loader.native, "require", lambda: m)
+    monkeypatch.setenv("AIOS_GEMM_PF_PLANS", str(path))
+    loader.finalize(SimpleNamespace(finalize=lambda: None))
+    assert got == ([installed] if installed else [])
+    assert json.loads(path.read_text()) == {"version": 7, "plans": [2] * 14}
