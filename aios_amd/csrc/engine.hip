@@ -668,11 +668,10 @@ void Engine::finalize() {
       if (const char* e = std::getenv("AIOS_DECODE_GEMM_MIN_B")) {
         dec_gemm_min_b_ = std::atoi(e);
       } else {
-        dec_gemm_min_b_ = default_gemm_min_b();
         // B rows go through the B-row LDS-DMA engine only if EVERY projection's LDS plan fits at that
         // B; where one does not (e.g. a 28672-wide down projection at B = 4: 115 KB of staged x), the
-        // row-pair fallback is 2-3x slower than the skinny GEMM, so that B takes the GEMM path
-        // (ADVICE r3).  Also bounds the short-prompt prefill rows that use the GEMV path.
+        // row-pair fallback is 2-3x slower than the skinny GEMM, so that B takes the GEMM path.
+        // Also bounds the short-prompt prefill rows that use the GEMV path.
         for (int b = 2; b < dec_gemm_min_b_ && b <= Bm; ++b) {
           bool ok = true;
           for (int l = 0; l < cfg_.n_layers && ok; ++l) {
@@ -692,6 +691,7 @@ void Engine::finalize() {
             gm_min_rows_ = std::min(gm_min_rows_, b);
           }
         }
+        dec_gemm_min_b_ = std::min(dec_gemm_min_b_, default_gemm_min_b());
       }
       // split-K slabs + tickets for every skinny-GEMM call: batched decode (M <= max_batch, the
       // lm_head included) AND prefill chunks of 16-64 tokens (no lm_head) -- sized for the batch

@@ -248,6 +248,28 @@ def test_short_prompt_prefill_matches_reference(model_files, monkeypatch, T, q8)
     assert (logits - rl).abs().max().item() < 2e-2 * max(rl.abs().max().item(), 1.0)
 
 
+@pytest.mark.parametrize("T", [2, 3, 4])
+def test_short_prompts_take_the_gemms_where_a_projection_has_no_gemv_plan(monkeypatch, T):
+    """d_ff 5632 (176 chunks of 32) has no LDS plan at 2 rows, so prompts of 2 to 4 tokens run the GEMMs: bit for bit the
+    logits of an engine told so, and not those of the int8-activation GEMVs"""
+    import dataclasses
+
+    from aios_amd.runtime.loader import random_engine
+
+    cfg = dataclasses.replace(get_preset("tinyllama-1.1b"), n_layers=2, vocab_size=2048)
+    prompt, out = [1] + list(range(7, 6 + T)), {}
+    for how, env in (("default", {}), ("gemm", {"AIOS_PREFILL_GEMM_MIN": "2"}),
+                     ("gemv", {"AIOS_PREFILL_GEMM_MIN": "5", "AIOS_DECODE_GEMM_MIN_B": "5"})):
+        with monkeypatch.context() as mp:
+            for k, v in env.items():
+                mp.setenv(k, v)
+            eng = random_engine(cfg, "Q4_K_M", seed=3, max_ctx=256)
+            out[how] = np.asarray(eng.prefill(0, prompt, 0, True))
+            del eng
+    assert np.isfinite(out["default"]).all()
+    assert np.array_equal(out["default"], out["gemm"]) and not np.array_equal(out["default"], out["gemv"])
+
+
 @pytest.mark.parametrize("recipe", ["Q4_K_M", "mistral_shape"])
 @pytest.mark.parametrize("fuse", ["0", "1"])
 def test_short_chunk_prefill_fusions_match_reference(model_files, monkeypatch, recipe, fuse):
