@@ -18,6 +18,12 @@ namespace aios {
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
+// ... each halved: one from the exponent, down to 0 (values below 2^-125 lose it, beside a largest of 1)
+__device__ __forceinline__ uint32_t bf16x2_half(uint32_t w) {
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, w), u16x2{0x80, 0x80}));
+}
+
 __device__ __forceinline__ void st_wt(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -142,7 +148,10 @@ constexpr int at_lds_bytes() { return AT_NW * AT_TK * at_vrow<HD>(); }
 //                         probabilities in fp32, stand in 16 / GP columns.
 //   O^T[dim][c] += V^T P^T   Each of a head's columns multiplies another bf16 part of the same probability (p's
 //                         leading 8 bits, the next 8, the last 8): the three products' sum has p in all its
-//                         24 bits, at no matrix instruction more for GP = 4 (two passes for GP = 8).  P^T comes
+//                         24 bits, at no matrix instruction more for GP = 4 (two passes for GP = 8: half of the
+//                         leading part in each, the middle and the last one beside it).  A leading part stands alone
+//                         in its columns' sums, so an infinite value's product is what its probability makes it;
+//                         the other parts can be 0 and their sums, 0 x Inf, are left out then.  P^T comes
 //                         from the S^T registers, its k order with it; V goes through a wave's own LDS tile
 //                         (row-major in, ds_read_b64_tr_b16 out: no barrier, a wave's LDS operations are in order).
 // The arithmetic of a tile is then ~100 VALU instructions a wave where dots and P.V on the VALU took ~900:
@@ -266,7 +275,7 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
 #pragma unroll
   for (int i = 0; i < DT; ++i) o[i] = gf32x4{0.f, 0.f, 0.f, 0.f};
   uint8_t* vt = at_smem + wave * (AT_TK * VROW);
-  // which part of P this lane's column multiplies (GP = 8: two passes, the leading and middle parts first)
+  // which part of P this lane's column multiplies (GP = 8: 0 the leading one, 1 the middle and then the last one)
   const int term0 = GP == 4 ? col >> 2 : col >> 3;
   const uint32_t sel0 = term0 == 0 ? ~0u : 0u, sel1 = term0 == 1 ? ~0u : 0u, sel2 = term0 == 2 ? ~0u : 0u;
 
@@ -316,19 +325,20 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
       p[i] = fast_exp2(st[i >> 2][i & 3] - m);
       l += p[i];
     }
-    // ---- P^T's bf16 parts: this column's term0 (NR passes: term0, term0 + 2)
+    // ---- P^T's bf16 parts
     gbf16x8 pf[NR];
     {
       uint32_t w[NR][4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const uint32_t hi = pk_bf16(p[2 * i], p[2 * i + 1]);
+        uint32_t hi = pk_bf16(p[2 * i], p[2 * i + 1]);
         const float r0 = p[2 * i] - bf16_lo(hi), r1 = p[2 * i + 1] - bf16_hi(hi);  // (exact)
         const uint32_t mid = pk_bf16(r0, r1);
         const uint32_t lo = pk_bf16(r0 - bf16_lo(mid), r1 - bf16_hi(mid));          // (exact: 8 bits left)
+        if constexpr (GP == 8) hi = bf16x2_half(hi);
         w[0][i] = (hi & sel0) | (mid & sel1);
         if constexpr (GP == 4) w[0][i] |= lo & sel2;
-        else w[1][i] = lo & sel0;
+        else w[1][i] = (hi & sel0) | (lo & sel1);
       }
 #pragma unroll
       for (int r = 0; r < NR; ++r) __builtin_memcpy(&pf[r], w[r], 16);
@@ -370,6 +380,17 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   }
   // ---- a head's columns summed (row rotates within 16 lanes), then the 8 waves merged in LDS
   l = quarters(l, OpAdd{});
+  gf32x4 z = gf32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) z[e] = fmaf(o[i][e], 0.f, z[e]);
+  if (__builtin_amdgcn_ballot_w64((z[0] + z[1]) + (z[2] + z[3]) != 0.f)) {  // some Inf or NaN: the leading part's columns have it
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[i][e] = term0 && !__builtin_isfinite(o[i][e]) ? 0.f : o[i][e];
+  }
 #pragma unroll
   for (int i = 0; i < DT; ++i)
 #pragma unroll

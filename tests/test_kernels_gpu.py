@@ -584,6 +584,45 @@ def test_attention_decode_tiles(E, H, Hkv, hd, lens, fp8, grouped, monkeypatch):
             assert err < 2e-5, (b, n, err)
 
 
+@pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (40, 8, 128), (64, 8, 128), (16, 8, 64)])
+@pytest.mark.parametrize("grouped", ["", "1"])  # "1": no form of its own for short contexts
+def test_attention_decode_infinite_values(E, H, Hkv, hd, grouped, monkeypatch):
+    """an infinite value in V gives an infinite output of its sign, two of unlike sign NaN, and the other dimensions'
+    stay as they are (the probabilities' parts that are zero must not meet it: 0 x Inf)"""
+    if grouped:
+        monkeypatch.setenv("AIOS_ATTN_GROUPED_MIN", grouped)
+    lens, max_ctx, G = (40, 300, 1100), 2048, H // Hkv
+    B, inf = len(lens), float("inf")
+    g = torch.Generator().manual_seed(8)
+    kc, vc = torch.randn(B, Hkv, max_ctx, hd, generator=g) * 0.5, torch.randn(B, Hkv, max_ctx, hd, generator=g)
+    for b, n in enumerate(lens):
+        vc[b, :, 5, 3] = inf
+        vc[b, :, n - 1, 7] = -inf
+        vc[b, :, 5, 11], vc[b, :, 20, 11] = inf, -inf
+    kc, vc = kc.to(torch.bfloat16), vc.to(torch.bfloat16)
+    kp, bt = paged_cache(kc, True, seed=5)
+    vp, _ = paged_cache(vc, True, seed=5)
+    kp, vp, bt = kp.cuda(), vp.cuda(), bt.cuda()
+    q = torch.randn(B, H, hd, generator=g).cuda()
+    seq, slot = torch.tensor(lens, dtype=torch.int32, device="cuda"), torch.arange(B, dtype=torch.int32, device="cuda")
+    nch, scale = max_ctx // E.ATTN_CHUNK, 1 / math.sqrt(hd)
+    opart, ml = torch.empty(B, H, nch, hd, device="cuda"), torch.empty(B, H, nch, 2, device="cuda")
+    out, cnt = torch.empty(B, H * hd, device="cuda"), torch.zeros(B, H, dtype=torch.int32, device="cuda")
+    E.attn_decode(q.data_ptr(), kp.data_ptr(), vp.data_ptr(), seq.data_ptr(), slot.data_ptr(), B, H, Hkv, hd, max_ctx, nch,
+                  scale, opart.data_ptr(), ml.data_ptr(), out.data_ptr(), cnt.data_ptr(), stream(), 0, bt.data_ptr(), 0)
+    torch.cuda.synchronize()
+    f = scale * 1.4426950408889634
+    qq = (q * f).to(torch.bfloat16).cpu().double() / 1.4426950408889634
+    for b, n in enumerate(lens):
+        k, v = kc[b, :, :n].double(), vc[b, :, :n].double()
+        p = torch.softmax((qq[b].view(Hkv, G, 1, hd) * k[:, None]).sum(-1), -1)
+        got, fin = out[b].cpu().double().view(H, hd), torch.ones(hd, dtype=torch.bool)
+        fin[[3, 7, 11]] = False
+        assert (got[:, 3] == inf).all() and (got[:, 7] == -inf).all() and got[:, 11].isnan().all(), n
+        ref = (p[..., None] * v[:, None, :, fin]).sum(2).reshape(H, -1)
+        assert float((got[:, fin] - ref).norm() / ref.norm()) < 2e-5
+
+
 @pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64)])
 @pytest.mark.parametrize("start,T", [(0, 37), (70, 130), (0, 300)])
 def test_attention_prefill_fp8_kv(E, H, Hkv, hd, start, T):
