@@ -38,18 +38,23 @@ __device__ __forceinline__ void pf_glds4(const void* src, uint32_t lds) {
                : "memory");
 }
 
-// ... from a uniform base and a 32-bit byte offset per lane: no 64-bit addition per lane and request
+// ... from a uniform base and a 32-bit byte offset per lane: no 64-bit addition per lane and request.  A scalar register
+// that the vector unit wrote (v_readlane, where the base comes back from a spilled lane) is an address five wait states
+// later at the earliest; the compiler guards its own loads, but not one inside an asm.  The scalar unit waits for it by
+// itself, so the base goes through s_mov, in the place of the s_nop that M0 needs (s_nop 2 cost 1 to 2 %).
 __device__ __forceinline__ void pf_glds16(const void* base, uint32_t off, uint32_t lds) {
   uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep)
+  uint64_t from;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_mov_b64 %1, %3\n\tglobal_load_lds_dwordx4 %2, %1\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep), "=&s"(from)
                : "v"(off), "s"(base), "s"(lds)
                : "memory");
 }
 __device__ __forceinline__ void pf_glds4(const void* base, uint32_t off, uint32_t lds) {
   uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep)
+  uint64_t from;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_mov_b64 %1, %3\n\tglobal_load_lds_dword %2, %1\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep), "=&s"(from)
                : "v"(off), "s"(base), "s"(lds)
                : "memory");
 }

@@ -1,6 +1,5 @@
-"""A clean build (no cached objects) of the gfx950 engine compiles and links -- the driver's build()
-reuses in-tree objects by mtime, so this is the check that the sources alone still build
-CPU only: hipcc cross-compiles for gfx950 without a GPU.  Several minutes (the
+"""A clean build (no cached objects) of the gfx950 engine compiles and links: in-tree objects are
+reused by mtime, so this is the check that the sources alone still build.  CPU only: hipcc cross-compiles for gfx950 without a GPU.  Several minutes (the
 GEMV translation units dominate); AIOS_SKIP_CLEAN_BUILD=1 skips it."""
 import os
 import shutil
@@ -21,3 +20,21 @@ def test_clean_build_compiles_and_links(tmp_path):
     # the extension exports the pybind11 module init and carries gfx950 code objects
     data = out.read_bytes()
     assert b"PyInit__engine" in data and b"gfx950" in data
+
+
+def test_lds_dma_waits_for_a_scalar_base():
+    """LDS-DMA inside asm: a load's scalar base is written by the scalar unit in the asm itself, or five wait states lie
+    before it, for the vector unit may have written it just before (restored from a spilled lane) and the compiler does not
+    look into an asm; one wait state or instruction lies between the write to M0 and the load"""
+    import re
+
+    text = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "aios_amd", "csrc", "kernels", "lds_dma.h")).read()
+    loads = [a.split("\\n\\t") for a in re.findall(r'asm volatile\("([^"]*global_load_lds[^"]*)"', text)]
+    assert len(loads) == 6
+    for a in loads:
+        at = next(i for i, t in enumerate(a) if t.startswith("global_load_lds"))
+        m0 = next(i for i, t in enumerate(a) if t.startswith("s_mov_b32 m0"))
+        assert m0 + 1 < at and all(t.startswith("s_") for t in a[:at]), a
+        base = a[at].split()[-1]
+        states = sum(int(t.split()[1]) + 1 if t.startswith("s_nop") else 1 for t in a[:at])
+        assert base == "off" or states >= 5 or any(t.startswith(f"s_mov_b64 {base},") for t in a[:at]), a
