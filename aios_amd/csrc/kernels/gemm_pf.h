@@ -1725,14 +1725,14 @@ inline int pf_tail_full(const GemmQArgs& a, int BN, int S) {
   return (T > C && R > 0 && 2 * R <= C) ? T - R : -1;
 }
 
-// Stream-K (round 6): a launch whose output tiles do not fill the chip -- the N = 4096-6144
+// Stream-K: a launch whose output tiles do not fill the chip -- the N = 4096-6144
 // projections of a 512-token chunk have 32-192 tiles for 256 CUs -- runs one workgroup per CU over an
 // equal share of the flattened (tile, K-step) iteration space instead of split-K's equal slices of
 // every tile: workgroup w takes iterations [w * ipw, (w + 1) * ipw), i.e. the tail of one tile and the
 // head of the next, and adds each partial tile into C with the split-K atomics (STORE targets zeroed
-// first).  KG: K-steps per unit (4 for the K-quant pf8c body, which slices on 256-blocks).  A workgroup
+// first).  KG: K-steps per unit (2 for tiles of two K groups).  A workgroup
 // that runs a second segment barriers first: the previous body's last LDS reads against its prologue DMA.
-template <int QT0, int QT1, int BM, int EPI, int KG, typename Body>
+template <int BM, int EPI, int KG, typename Body>
 __device__ __forceinline__ void pf_stream_k(const GemmQArgs& a, int BN, int ipw, Body body) {
   const int nN = a.N / BN, nM = (a.M + BM - 1) / BM;
   const int nk = a.K / (64 * KG);
@@ -1759,7 +1759,7 @@ __device__ __forceinline__ void pf_stream_k(const GemmQArgs& a, int BN, int ipw,
 template <int QT0, int QT1, int BM, int WC, int EPI>
 __global__ void __launch_bounds__(256 * pf4_kg<BM>()) gemm_pf4sk_kernel(GemmQArgs a, int ipw) {
   constexpr int KG = pf4_kg<BM>();
-  pf_stream_k<QT0, QT1, BM, EPI, KG>(a, 4 * WC, ipw, [&](int m0, int n0, int seg, int kt0, int kt1, int S) {
+  pf_stream_k<BM, EPI, KG>(a, 4 * WC, ipw, [&](int m0, int n0, int seg, int kt0, int kt1, int S) {
     if constexpr (QT0 != QT1) {
       if (seg == a.nseg - 1) {
         pf4_body<QT1, BM, WC, EPI, 0, KG>(a, m0, n0, seg, kt0, kt1, S);
@@ -1770,27 +1770,10 @@ __global__ void __launch_bounds__(256 * pf4_kg<BM>()) gemm_pf4sk_kernel(GemmQArg
   });
 }
 
-template <int QT0, int QT1, int BM, int EPI>
+template <int BM, int EPI>
 __global__ void __launch_bounds__(512) gemm_pf8sk_kernel(GemmQArgs a, int ipw) {
-  constexpr int KG = pf8_generic<QT0, QT1>() ? 1 : 4;
-  pf_stream_k<QT0, QT1, BM, EPI, KG>(a, 256, ipw, [&](int m0, int n0, int seg, int kt0, int kt1, int S) {
-    if constexpr (pf8_generic<QT0, QT1>()) {
-      if constexpr (QT0 != QT1) {
-        if (seg == a.nseg - 1) {
-          pf8_body<QT1, BM, EPI>(a, m0, n0, seg, kt0, kt1, S);
-          return;
-        }
-      }
-      pf8_body<QT0, BM, EPI>(a, m0, n0, seg, kt0, kt1, S);
-    } else {
-      if constexpr (QT0 != QT1) {
-        if (seg == a.nseg - 1) {
-          pf8c_body<QT1, BM, EPI>(a, m0, n0, seg, kt0, kt1, S);
-          return;
-        }
-      }
-      pf8c_body<QT0, BM, EPI>(a, m0, n0, seg, kt0, kt1, S);
-    }
+  pf_stream_k<BM, EPI, 1>(a, 256, ipw, [&](int m0, int n0, int seg, int kt0, int kt1, int S) {
+    pf8_body<QT_BF16, BM, EPI>(a, m0, n0, seg, kt0, kt1, S);
   });
 }
 
@@ -1820,14 +1803,16 @@ template <int QT0, int QT1, int BM>
 void pf8_launch(const GemmQArgs& a, int S, hipStream_t st) {
   constexpr int lds = pf8_lds_bytes<QT0, QT1, BM>();
   static_assert(lds <= 160 * 1024, "LDS");
-  if (S < 0) {  // stream-K (STORE / ACCUM only: partial tiles are atomic adds)
-    int grid = 0;
-    const int ipw = pf_sk_ipw(a, BM, 256, pf8_generic<QT0, QT1>() ? 1 : 4, grid);
-    if (a.epi == GEPI_STORE)
-      hipLaunchKernelGGL((gemm_pf8sk_kernel<QT0, QT1, BM, GEPI_STORE>), dim3(grid), dim3(512), lds, st, a, ipw);
-    else
-      hipLaunchKernelGGL((gemm_pf8sk_kernel<QT0, QT1, BM, GEPI_ACCUM>), dim3(grid), dim3(512), lds, st, a, ipw);
-    return;
+  if constexpr (QT0 == QT_BF16) {
+    if (S < 0) {  // stream-K (STORE / ACCUM only: partial tiles are atomic adds; other formats: pf_sk_ok)
+      int grid = 0;
+      const int ipw = pf_sk_ipw(a, BM, 256, 1, grid);
+      if (a.epi == GEPI_STORE)
+        hipLaunchKernelGGL((gemm_pf8sk_kernel<BM, GEPI_STORE>), dim3(grid), dim3(512), lds, st, a, ipw);
+      else
+        hipLaunchKernelGGL((gemm_pf8sk_kernel<BM, GEPI_ACCUM>), dim3(grid), dim3(512), lds, st, a, ipw);
+      return;
+    }
   }
   if constexpr (BM == 256 && QT0 != QT_BF16) {  // (K-quant stacks: the tail split)
     const int F = pf_tail_full(a, 256, S);

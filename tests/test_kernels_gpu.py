@@ -1394,8 +1394,8 @@ def test_gemm_pf_production_shapes_vs_unquantized(E, monkeypatch, fmt, N, K, spl
 def test_gemm_pf_stream_k(E, monkeypatch, fmt, N, K, tile, epi):
     """Stream-K (AIOS_GEMM_PF_SPLIT=-1): one workgroup per CU over an equal share of the (tile, K-step)
     iterations, partial tiles added atomically -- the 512-token shapes of Mistral's QKV stack, O and
-    Q6_K down, and a bf16 matrix, every body (pf4 128-column, pf8c 256-column K-quant, pf8 bf16),
-    against the unquantized fp64 product"""
+    Q6_K down, and a bf16 matrix, every body (pf4 128-column, pf8 bf16 256-column), against the unquantized
+    fp64 product; quantised 256-column tiles have no such form and are in no plan"""
     monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
     monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", "-1")
     segs = {"mixed6144": [(GGMLType.Q4_K, 4096), (GGMLType.Q4_K, 1024), (GGMLType.Q6_K, 1024)],
@@ -1407,8 +1407,10 @@ def test_gemm_pf_stream_k(E, monkeypatch, fmt, N, K, tile, epi):
         _pf_cache[key] = (list(mats), torch.cat(refs, 0))
     mats, W = _pf_cache[key]
     M = 512
-    if E.gemm_pf_plan(mats, M, E.GEPI_ACCUM, 0)[2] != -1:
-        pytest.skip("stream-K not eligible for this tile / shape")
+    planned = E.gemm_pf_plan(mats, M, E.GEPI_ACCUM, 0)[2] == -1
+    assert planned == (fmt == "bf16" or tile.endswith("x128"))
+    if not planned:
+        pytest.skip("no stream-K of this tile and format")
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(K + N))
     A = x.to(torch.bfloat16).cuda()
     C = torch.full((M, N), 0.5, device="cuda")
@@ -1469,7 +1471,8 @@ def pf_plan_entry(E, N, K, M, epi, bm, bn, S, s1=0):
 
 @pytest.mark.parametrize("K,N,tile", [(192, 640, (64, 128, 1)), (192, 896, (128, 128, 1)), (320, 640, (96, 128, 2)),
                                       (320, 384, (160, 128, 1)), (128, 384, (64, 256, 1)), (128, 640, (64, 128, 3)),
-                                      (192, 1152, (64, 128, -1)), (128, 896, (48, 128, 1)), (128, 1152, (64, 128, 0))])
+                                      (192, 1152, (64, 128, -1)),
+                                      (128, 896, (48, 128, 1)), (128, 1152, (64, 128, 0))])
 def test_gemm_pf_imported_plan_that_does_not_fit(E, K, N, tile):
     """a stored plan is one of this build's tiles and cuts K as its kernel does, or the modelled one serves: two K groups
     (K an odd number of 64s), a width that does not divide N, more slices than K-steps, stream-K of too few, no such tile"""
