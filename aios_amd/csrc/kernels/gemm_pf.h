@@ -1383,7 +1383,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
 #pragma unroll
           for (int i = 0; i < 2 * GR; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);               // a matrix instruction,
-            __builtin_amdgcn_sched_group_barrier(0x2, L::Q6 ? 5 : 3, 0);   // a few of the decode
+            __builtin_amdgcn_sched_group_barrier(0x2, L::Q6 ? 4 : 3, 0);   // a few of the decode (Q6_K 5: 8 to 20 B spilled)
           }
         }
       } else {
@@ -1826,7 +1826,9 @@ void pf8_launch(const GemmQArgs& a, int S, hipStream_t st) {
         switch (a.epi) {
           case GEPI_STORE: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_STORE, P>), grid, block, ldst, st, a, F); break;
           case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_ACCUM, P>), grid, block, ldst, st, a, F); break;
-          default: hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_SWIGLU_BF16, P>), grid, block, ldst, st, a, F); break;
+          default:  // (one segment, so one format)
+            if constexpr (QT0 == QT1) hipLaunchKernelGGL((gemm_pf8t_kernel<QT0, QT1, GEPI_SWIGLU_BF16, P>), grid, block, ldst, st, a, F);
+            break;
         }
       };
       if (4 * R <= device_cu_count()) go(std::integral_constant<int, 4>{});
@@ -1842,7 +1844,9 @@ void pf8_launch(const GemmQArgs& a, int S, hipStream_t st) {
     case GEPI_STORE16:
       if constexpr (QT0 == QT_BF16) hipLaunchKernelGGL((gemm_pf8_kernel<QT0, QT1, BM, GEPI_STORE16>), grid, block, lds, st, a);
       break;
-    default: hipLaunchKernelGGL((gemm_pf8_kernel<QT0, QT1, BM, GEPI_SWIGLU_BF16>), grid, block, lds, st, a); break;
+    default:  // (one segment, so one format)
+      if constexpr (QT0 == QT1) hipLaunchKernelGGL((gemm_pf8_kernel<QT0, QT1, BM, GEPI_SWIGLU_BF16>), grid, block, lds, st, a);
+      break;
   }
 }
 
@@ -1932,7 +1936,9 @@ void pf4_launch(const GemmQArgs& a, int S, hipStream_t st) {
       switch (a.epi) {
         case GEPI_STORE: hipLaunchKernelGGL((gemm_pf4t_kernel<QT0, QT1, WC, GEPI_STORE>), grid, block, ldst, st, a, F); break;
         case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pf4t_kernel<QT0, QT1, WC, GEPI_ACCUM>), grid, block, ldst, st, a, F); break;
-        default: hipLaunchKernelGGL((gemm_pf4t_kernel<QT0, QT1, WC, GEPI_SWIGLU_BF16>), grid, block, ldst, st, a, F); break;
+        default:  // (one segment, so one format)
+          if constexpr (QT0 == QT1) hipLaunchKernelGGL((gemm_pf4t_kernel<QT0, QT1, WC, GEPI_SWIGLU_BF16>), grid, block, ldst, st, a, F);
+          break;
       }
       return;
     }
@@ -1945,7 +1951,9 @@ void pf4_launch(const GemmQArgs& a, int S, hipStream_t st) {
     case GEPI_STORE16:
       if constexpr (QT0 == QT_BF16) hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_STORE16>), grid, block, lds, st, a);
       break;
-    default: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_SWIGLU_BF16>), grid, block, lds, st, a); break;
+    default:  // (one segment, so one format)
+      if constexpr (QT0 == QT1) hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_SWIGLU_BF16>), grid, block, lds, st, a);
+      break;
   }
 }
 

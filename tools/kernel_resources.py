@@ -21,8 +21,9 @@ import sys
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SO = os.path.join(ROOT, "aios_amd")
 
-# decode-path kernel templates that must never touch scratch (mangled-name globs over the
-# demangled text); the batch>1 row-pair GEMV variants are fallbacks and are reported, not enforced
+# kernel templates that must never touch scratch (mangled-name globs over the demangled text): the decode path's, and the
+# prefill GEMMs', whose reloads would drain the DMA; the batch>1 row-pair GEMV variants are fallbacks and are reported,
+# not enforced, and so are the 256-row prefill tiles with the RoPE / KV-cache epilogue (<..., 256, .., 3, 0>)
 HOT = [
     "aios::gemv_lds_b1<*, *, 1, *>*",
     "aios::gemv_lds16<*",
@@ -33,6 +34,14 @@ HOT = [
     "aios::gemm_skinny_kernel<*",
     "aios::gemm_ring_kernel<*",
     "aios::gemm_wk_kernel<*",
+    "aios::gemm_pf8_kernel<*, [012], 0>*",
+    "aios::gemm_pf8_kernel<*, *, 64, 3, 0>*",
+    "aios::gemm_pf8_kernel<*, *, 128, 3, 0>*",
+    "aios::gemm_pf8t_kernel<*",
+    "aios::gemm_pf8sk_kernel<*",
+    "aios::gemm_pf4_kernel<*, [012], 0>*",
+    "aios::gemm_pf4t_kernel<*",
+    "aios::gemm_pf4sk_kernel<*",
     "aios::sample_kernel*",
     "aios::get_rows_step_kernel*",
     "aios::latent_prep_kernel*",
