@@ -747,10 +747,10 @@ void Engine::finalize() {
 }
 
 // Measured prefill-GEMM plans (kernels/gemm_pf.hip): every distinct projection launch of this model
-// -- QKV stack, O, gate/up (SwiGLU), down, per weight-format signature -- timed over its candidate
-// tiles / K splits at M = 64 .. gm_rows_ (gemm_pf_bucket), the fastest kept per M bucket in the
-// process-wide plan cache (one tuning per shape per process; ~0.3 s for Mistral-7B).  Activations
-// are random bf16 (a zero fill clocks the chip differently).  AIOS_GEMM_PF_TUNE=0: model plans only.
+// -- QKV stack, O, gate/up (SwiGLU), down, per weight-format signature -- timed with its layers' weights in turn over
+// candidate tiles / K splits at M = 64 .. gm_rows_ (gemm_pf_bucket), the fastest kept per M bucket in the
+// process-wide plan cache (one tuning per shape per process; 0.7 s for Mistral-7B Q4_K_M, 0.3 s for TinyLlama Q4_K_M).
+// Activations are random bf16 (a zero fill clocks the chip differently).  AIOS_GEMM_PF_TUNE=0: model plans only.
 void Engine::tune_prefill_gemm() {
   if (!gm_ok_ || cfg_.n_layers == 0) return;
   if (const char* e = std::getenv("AIOS_GEMM_PF_TUNE"))
@@ -765,36 +765,31 @@ void Engine::tune_prefill_gemm() {
   launch_f32_to_bf16(tmp, gm_a16_, (size_t)G * d, stream_);
   launch_f32_to_bf16(tmp, gm_attn16_, (size_t)G * qd, stream_);
   launch_f32_to_bf16(tmp, gm_ff16_, (size_t)G * ff, stream_);
-  std::set<std::string> seen;
+  std::vector<GemmQArgs> launches;
   for (int M = 64; M <= G; M = gemm_pf_bucket(M + 1)) {
     for (const LayerW& L : layers_) {
-      auto tune = [&](GemmQArgs& g, const char* what) {
-        std::string sig = std::string(what) + ":" + std::to_string(M);
-        for (int s = 0; s < g.nseg; ++s) sig += "," + std::to_string(g.seg[s].qtype);
-        if (!seen.insert(sig).second) return;
-        gemm_pf_autotune(g, stream_);
-      };
       GemmQArgs g;
       std::memset(&g, 0, sizeof(g));
       g.A = gm_a16_; g.lda = d; g.M = M; g.K = d; g.nseg = 3;
       g.seg[0] = L.wq.w; g.seg[1] = L.wk.w; g.seg[2] = L.wv.w;
       g.seg_n0[0] = 0; g.seg_n0[1] = qd; g.seg_n0[2] = qd + kvd;
       g.N = ldqkv; g.C = gm_qkv_; g.ldc = ldqkv; g.epi = GEPI_STORE;
-      tune(g, "qkv");
+      launches.push_back(g);
       std::memset(&g, 0, sizeof(g));
       g.A = gm_attn16_; g.lda = qd; g.M = M; g.K = qd; g.nseg = 1; g.seg[0] = L.wo.w; g.N = d; g.ldc = d;
       if (tp) { g.C = gm_part_; g.epi = GEPI_STORE; } else { g.C = gm_x_; g.epi = GEPI_ACCUM; }
-      tune(g, "o");
+      launches.push_back(g);
       std::memset(&g, 0, sizeof(g));
       g.A = gm_a16_; g.lda = d; g.M = M; g.K = d; g.nseg = 1; g.seg[0] = L.wgu.w; g.N = 2 * ff;
       g.C16 = gm_ff16_; g.ldc = ff; g.epi = GEPI_SWIGLU_BF16;
-      tune(g, "gu");
+      launches.push_back(g);
       std::memset(&g, 0, sizeof(g));
       g.A = gm_ff16_; g.lda = ff; g.M = M; g.K = ff; g.nseg = 1; g.seg[0] = L.wdown.w; g.N = d; g.ldc = d;
       if (tp) { g.C = gm_part_; g.epi = GEPI_STORE; } else { g.C = gm_x_; g.epi = GEPI_ACCUM; }
-      tune(g, "down");
+      launches.push_back(g);
     }
   }
+  gemm_pf_autotune(launches, stream_);
   HIP_CHECK(hipStreamSynchronize(stream_));
   HIP_CHECK(hipFree(tmp));
 }

@@ -6,6 +6,7 @@
 #include <map>
 #include <stdexcept>
 #include <mutex>
+#include <set>
 #include <tuple>
 #include <vector>
 
@@ -246,60 +247,104 @@ static bool pf_eligible(const GemmQArgs& a) {
   return true;
 }
 
-// Time every candidate plan for these args (real buffers; outputs overwritten) and keep the fastest
-// for their M bucket.  Returns the number of candidates timed (0: not a prefill-GEMM launch, or a
-// key already planned in this process -- tuned by an earlier engine or imported, gemm_pf_import, and a plan that
-// the kernels take: a second engine never changes the plans a first one runs).
+// Time the candidate plans of the launches (real buffers; outputs overwritten) and keep the fastest per key.  Launches of
+// one key -- a projection, layer by layer -- are timed with their weights in turn, as a pass runs them: the same matrix
+// again and again lies in the caches (with it, the plans of 2048-wide bf16 layers changed from process to process, and a
+// pass of 1500 rows with them: 8.65 to 9.24 ms; so: 8.61 to 8.63).  Returns the number of plans timed.  A key already
+// planned in this process -- tuned by an earlier engine or imported, gemm_pf_import -- is left if the kernels take its
+// plan: a second engine never changes the plans a first one runs.
 //
-// Stable choice: a measured plan replaces the modelled one only when it is > 5 % faster,
-// so timing noise (a co-tenant, TP ranks sharing the GPU) does not pick a different tile / split in
-// each process; ties keep the earlier candidate (a fixed order).  TP ranks then take rank 0's plans
-// (tp.py broadcasts gemm_pf_export), and AIOS_GEMM_PF_PLANS persists them across processes.
-int gemm_pf_autotune(const GemmQArgs& a, hipStream_t st) {
-  if (!pf_eligible(a)) return 0;
-  const bool bf = a.seg[0].qtype == QT_BF16;
-  {
+// Every candidate that the model puts within twice its best (no plan within 3 % of the fastest lay beyond, for five models'
+// 420 keys) in two launches, then those within 12 % of the fastest in four, forwards and backwards; the modelled plan stays
+// where it is within 2 %, and ties keep the earlier candidate.  TP ranks then take rank 0's plans (tp.py broadcasts
+// gemm_pf_export), and AIOS_GEMM_PF_PLANS persists them across processes.
+int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
+  std::vector<std::pair<PfKey, std::vector<const GemmQArgs*>>> work;  // in the order of the launches
+  for (const GemmQArgs& a : launches) {
+    if (!pf_eligible(a)) continue;
+    const PfKey k = pf_key(a);
+    const auto at = std::find_if(work.begin(), work.end(), [&](const auto& w) { return w.first == k; });
+    if (at != work.end()) {
+      at->second.push_back(&a);
+      continue;
+    }
     std::lock_guard<std::mutex> g(pf_mu);
-    const auto it = pf_tuned().find(pf_key(a));
-    if (it != pf_tuned().end() && pf_plan_ok(a, it->second, bf)) return 0;
+    const auto it = pf_tuned().find(k);
+    if (it == pf_tuned().end() || !pf_plan_ok(a, it->second, a.seg[0].qtype == QT_BF16)) work.push_back({k, {&a}});
   }
-  const std::vector<PfPlan> cands = pf_candidates(a, bf);
-  if (cands.empty()) return 0;
-  const PfPlan mp = pf_model_plan(a, bf, false), mp1 = pf_model_plan(a, bf, true);
-  float tm = -1.f, tm1 = -1.f;  // the modelled plans' measured times
-  hipEvent_t e0, e1;
-  HIP_CHECK(hipEventCreate(&e0));
-  HIP_CHECK(hipEventCreate(&e1));
-  PfPlan best = cands[0], best1 = cands[0];
-  float bt = 1e30f, bt1 = 1e30f;
-  for (const PfPlan& p : cands) {
-    pf_run(a, p, st);  // warm (code object load, caches)
-    HIP_CHECK(hipEventRecord(e0, st));
-    for (int r = 0; r < 3; ++r) pf_run(a, p, st);
-    HIP_CHECK(hipEventRecord(e1, st));
-    HIP_CHECK(hipEventSynchronize(e1));
-    float ms = 0.f;
-    HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-    if (ms < bt) {
-      bt = ms;
-      best = p;
+  std::vector<hipEvent_t> ev;
+  std::set<std::tuple<int, int, int, int, int, int>> loaded;  // (kernels that have run)
+  size_t at = 0;                                              // (the next weights)
+  int timed = 0;
+  // us of a launch under each plan: one after the other without a gap, n launches each
+  auto time = [&](const std::vector<const GemmQArgs*>& v, const std::vector<PfPlan>& plans, int n) {
+    const GemmQArgs& a = *v[0];
+    auto run = [&](const PfPlan& p) { pf_run(*v[at++ % v.size()], p, st); };
+    for (const PfPlan& p : plans) {
+      const int form = p.s == 1 ? (a.N / p.bn) * ((a.M + p.bm - 1) / p.bm) > device_cu_count() : p.s < 0 ? 2 : 3;
+      if (loaded.insert({a.seg[0].qtype, a.seg[a.nseg - 1].qtype, a.epi, p.bm, p.bn, form}).second) run(p);
     }
-    if (p.s == 1 && ms < bt1) {  // (stream-K is not an S = 1 plan either)
-      bt1 = ms;
-      best1 = p;
+    while (ev.size() <= plans.size()) {
+      ev.push_back(nullptr);
+      HIP_CHECK(hipEventCreate(&ev.back()));
     }
-    auto same = [](const PfPlan& x, const PfPlan& y) { return x.bm == y.bm && x.bn == y.bn && x.s == y.s; };
-    if (same(p, mp)) tm = ms;
-    if (same(p, mp1)) tm1 = ms;
+    run(plans[0]);
+    HIP_CHECK(hipEventRecord(ev[0], st));
+    for (size_t i = 0; i < plans.size(); ++i) {
+      for (int r = 0; r < n; ++r) run(plans[i]);
+      HIP_CHECK(hipEventRecord(ev[i + 1], st));
+    }
+    HIP_CHECK(hipEventSynchronize(ev[plans.size()]));
+    std::vector<float> us(plans.size());
+    for (size_t i = 0; i < plans.size(); ++i) {
+      HIP_CHECK(hipEventElapsedTime(&us[i], ev[i], ev[i + 1]));
+      us[i] *= 1e3f / n;
+    }
+    return us;
+  };
+  auto same = [](const PfPlan& x, const PfPlan& y) { return x.bm == y.bm && x.bn == y.bn && x.s == y.s; };
+  for (const auto& w : work) {
+    const auto& v = w.second;
+    const GemmQArgs& a = *v[0];
+    const bool bf = a.seg[0].qtype == QT_BF16;
+    const PfPlan mp = pf_model_plan(a, bf, false), mp1 = pf_model_plan(a, bf, true);
+    auto model = [&](const PfPlan& p) { return pf_model(a, p.bm, p.bn, p.s, bf); };
+    std::vector<PfPlan> c;
+    for (const PfPlan& p : pf_candidates(a, bf))
+      if (!mp.bm || model(p) <= 2 * model(mp) || same(p, mp1)) c.push_back(p);
+    if (c.empty()) continue;
+    if (&w == &work[0]) time(v, {c[0]}, 100);  // (the clocks)
+    const std::vector<float> us = time(v, c, 2);
+    timed += (int)c.size();
+    // the fastest, or the fastest without split partials
+    auto pick = [&](bool s1) {
+      auto in = [&](size_t i) { return !s1 || c[i].s == 1; };
+      float least = 1e30f;
+      for (size_t i = 0; i < c.size(); ++i)
+        if (in(i)) least = std::min(least, us[i]);
+      std::vector<PfPlan> f;
+      for (size_t i = 0; i < c.size(); ++i)
+        if (in(i) && (us[i] <= 1.12f * least || same(c[i], s1 ? mp1 : mp))) f.push_back(c[i]);
+      if (f.size() < 2) return f.empty() ? PfPlan() : f[0];
+      const size_t n = f.size();
+      std::vector<PfPlan> both(f);
+      both.insert(both.end(), f.rbegin(), f.rend());
+      const std::vector<float> t = time(v, both, 4);
+      auto sum = [&](size_t i) { return t[i] + t[2 * n - 1 - i]; };
+      size_t best = 0;
+      for (size_t i = 1; i < n; ++i)
+        if (sum(i) < sum(best)) best = i;
+      for (size_t i = 0; i < n; ++i)
+        if (same(f[i], s1 ? mp1 : mp) && sum(i) <= 1.02f * sum(best)) return f[i];
+      return f[best];
+    };
+    const PfPlan best = pick(false), best1 = best.s == 1 ? best : pick(true);
+    std::lock_guard<std::mutex> g(pf_mu);
+    pf_tuned()[w.first] = best;
+    if (best1.bm) pf_tuned_s1()[w.first] = best1;
   }
-  HIP_CHECK(hipEventDestroy(e0));
-  HIP_CHECK(hipEventDestroy(e1));
-  if (tm > 0.f && bt > 0.95f * tm) best = mp;
-  if (tm1 > 0.f && bt1 > 0.95f * tm1) best1 = mp1;
-  std::lock_guard<std::mutex> g(pf_mu);
-  pf_tuned()[pf_key(a)] = best;
-  if (bt1 < 1e30f) pf_tuned_s1()[pf_key(a)] = best1;
-  return (int)cands.size();
+  for (hipEvent_t e : ev) HIP_CHECK(hipEventDestroy(e));
+  return timed;
 }
 
 // every tuned plan as flat ints: 10 key fields, bm, bn, s, map (0: best, 1: best without split-K)

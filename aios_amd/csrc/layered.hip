@@ -922,13 +922,14 @@ void LayeredDecoder::tune() {
   HIP_CHECK(hipMalloc(&tmp, (size_t)step_rows_ * dp_ * 4));
   fill_random_f32(tmp, (size_t)step_rows_ * dp_, 0x7u, 0.f, 1.f, e_.stream_);
   launch_f32_to_bf16(tmp, h16_, (size_t)step_rows_ * dp_, e_.stream_);
+  std::vector<GemmQArgs> launches;
   for (int M = 64; M <= step_rows_; M = gemm_pf_bucket(M + 1)) {
     auto go = [&](const bf16_t* A, int lda, const bf16_t* wt, int N, int K, int epi, float* C, int ldc, bf16_t* C16, int act) {
       GemmQArgs g;
       std::memset(&g, 0, sizeof(g));
       g.A = A; g.lda = lda; g.M = M; g.N = N; g.K = K; g.nseg = 1; g.seg[0] = mat(wt, N, K);
       g.C = C; g.C16 = C16; g.ldc = ldc; g.epi = epi; g.act = act;
-      gemm_pf_autotune(g, e_.stream_);
+      launches.push_back(g);
     };
     if (loopw_) go((const bf16_t*)xin_, 2 * dp_, loopw_, dp_, 2 * dp_, GEPI_STORE, y_, dp_, nullptr, 0);
     for (int i = 0; i < nl_; ++i) {
@@ -954,6 +955,7 @@ void LayeredDecoder::tune() {
       if (D.rp && M <= pf_max_ctx_) go(cfull_, D.rp, w.ukv, D.qn + D.gn, D.rp, GEPI_STORE16, nullptr, D.qn + D.gn, kv_, act);
     }
   }
+  gemm_pf_autotune(launches, e_.stream_);
   HIP_CHECK(hipMemsetAsync(h16_, 0, (size_t)step_rows_ * dp_ * 2, e_.stream_));
   HIP_CHECK(hipStreamSynchronize(e_.stream_));
   HIP_CHECK(hipFree(tmp));

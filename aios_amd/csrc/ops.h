@@ -263,9 +263,9 @@ bool launch_gemm_pf(const GemmQArgs& a, hipStream_t st);
 bool gemm_pf_serves(const GemmQArgs& a);  // launch_gemm_pf would take a (gemm_pf.hip)
 void gemm_pf_plan(const GemmQArgs& a, int& bm, int& bn, int& s);
 bool gemm_pf_probe(const GemmQArgs& a, int probe, hipStream_t st);  // timing anatomy (tools only)
-// time every prefill-GEMM plan for these args (buffers overwritten) and keep the fastest for their M
-// bucket; returns the number of plans timed
-int gemm_pf_autotune(const GemmQArgs& a, hipStream_t st);
+// time the prefill-GEMM plans of these launches (buffers overwritten; those of like shape are one, with each one's
+// weights in turn) and keep the fastest for their M bucket; returns the number of plans timed
+int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st);
 int gemm_pf_bucket(int M);  // the row count whose plan serves M rows: plans are tuned at M = 64, then bucket(M + 1), ..
 // of the kernels that plans were timed on: a plan file of another number is timed again (2: K groups in the 128-column
 // tiles below 256 rows, more row buckets)

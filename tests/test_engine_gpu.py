@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from aios_amd.gguf.quants import GGMLType
 from aios_amd.models.config import get_preset
 from aios_amd.models.reference import ReferenceModel
 from aios_amd.models.synthetic import write_synthetic_gguf
@@ -500,9 +501,35 @@ print(json.dumps(sorted(native.require().gemm_pf_export())))
 """
 
 
+def test_prefill_plans_cover_every_projection_and_row_bucket():
+    """finalize plans each projection (per pair of formats) for every bucket of rows up to the context, once, and each plan
+    is one that the launcher runs"""
+    import dataclasses
+
+    from aios_amd.runtime import native
+    from aios_amd.runtime.loader import random_engine
+
+    m = native.require()
+    cfg = dataclasses.replace(get_preset("tinyllama-1.1b"), n_layers=8, d_ff=2816, vocab_size=512)
+    eng = random_engine(cfg, "Q4_K_M", seed=3, max_ctx=1024, max_batch=1)
+    d, kv = cfg.d_model, cfg.n_kv_heads * cfg.head_dim
+    v = list(m.gemm_pf_export())
+    plans = [v[i:i + 14] for i in range(0, len(v), 14)]
+    q4, q6 = int(GGMLType.Q4_K), int(GGMLType.Q6_K)
+    buckets = {64, 96, 128, 160, 192, 256, 320, 384, 512, 640, 768, 1024}
+    want = {(d + 2 * kv, d, 3): {(q4, q4), (q4, q6)}, (d, d, 1): {(q4, q4)}, (2 * cfg.d_ff, d, 1): {(q4, q4)},
+            (d, cfg.d_ff, 1): {(q4, q4), (q6, q6)}}
+    for (N, K, nseg), formats in want.items():
+        for one_slice in (0, 1):
+            got = [p for p in plans if (p[0], p[1], p[6], p[13]) == (N, K, nseg, one_slice)]
+            assert {(p[2], p[4], p[5]) for p in got} >= {(b, *f) for b in buckets for f in formats}
+            assert all(p[10] and p[11] and (p[12] == 1 or not one_slice) for p in got)
+    assert np.isfinite(np.asarray(eng.prefill(0, list(range(3, 203)), 0, True))).all()
+
+
 @pytest.mark.parametrize("deterministic", [False, True])
 def test_prefill_plans_persist_across_processes(tmp_path, deterministic):
-    """ADVICE r5 (medium): with AIOS_GEMM_PF_PLANS naming a file, a second process installs the first's
+    """with AIOS_GEMM_PF_PLANS naming a file, a second process installs the first's
     tuned prefill-GEMM plans instead of timing its own (the same plan list in both).  Split-K / stream-K
     plans add partial tiles with fp32 atomics in arrival order, so their last bits may still differ:
     the logits agree to float rounding and on the argmax; AIOS_GEMM_PF_DETERMINISTIC=1 keeps those plans
