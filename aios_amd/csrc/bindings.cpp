@@ -105,6 +105,44 @@ struct PyQMatrix {
   }
 };
 
+// a launch of the stacked matrices with the shared workspace; `more`: fields of the fused RMSNorm and of the QKV epilogue
+GemmQArgs gemm_q_args(const std::vector<PyQMatrix*>& segs, int M, int epi, int ksplit, const py::dict& more) {
+  GemmQArgs a;
+  std::memset(&a, 0, sizeof(a));
+  if (segs.empty() || segs.size() > 3) throw std::runtime_error("gemm_q: 1..3 segments");
+  a.nseg = (int)segs.size();
+  int n0 = 0;
+  for (int s = 0; s < a.nseg; ++s) { a.seg[s] = segs[s]->w; a.seg_n0[s] = n0; n0 += segs[s]->w.rows; }
+  a.M = M; a.N = n0; a.K = segs[0]->w.cols; a.epi = epi; a.ksplit = ksplit;
+  for (const auto& kv : more) {
+    const std::string k = py::cast<std::string>(kv.first);
+    auto ptr = [&](auto& f) { f = reinterpret_cast<std::decay_t<decltype(f)>>(py::cast<uintptr_t>(kv.second)); };
+    auto num = [&](auto& f) { f = py::cast<std::decay_t<decltype(f)>>(kv.second); };
+    if (k == "nrm_g") ptr(a.nrm_g);
+    else if (k == "nrm_out16") ptr(a.nrm_out16);
+    else if (k == "nrm_part") ptr(a.nrm_part);
+    else if (k == "nrm_in") ptr(a.nrm_in);
+    else if (k == "nrm_parts") num(a.nrm_parts);
+    else if (k == "nrm_eps") num(a.nrm_eps);
+    else if (k == "head_dim") num(a.head_dim);
+    else if (k == "q_dim") num(a.q_dim);
+    else if (k == "kv_dim") num(a.kv_dim);
+    else if (k == "n_kv_heads") num(a.n_kv_heads);
+    else if (k == "max_ctx") num(a.max_ctx);
+    else if (k == "rope_cs") ptr(a.rope_cs);
+    else if (k == "pos") ptr(a.pos);
+    else if (k == "slot") ptr(a.slot);
+    else if (k == "block_table") ptr(a.block_table);
+    else if (k == "q_out") ptr(a.q_out);
+    else if (k == "k_cache") ptr(a.k_cache);
+    else if (k == "v_cache") ptr(a.v_cache);
+    else throw std::runtime_error("gemm_q: no field " + k);
+  }
+  GemmWs& g = gemm_ws(M, a.N);
+  a.ws = g.ws; a.ws_bytes = g.bytes; a.cnt = g.cnt; a.cnt_len = g.cnt_len;
+  return a;
+}
+
 }  // namespace
 
 #ifndef AIOS_MODULE
@@ -393,6 +431,7 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
            py::arg("rows"))
       .def_property_readonly("kv_blocks_total", &Engine::kv_blocks_total)
       .def_property_readonly("norm_fused_parts", &Engine::norm_fused_parts)
+      .def_property_readonly("decode_gemm_min_batch", &Engine::decode_gemm_min_batch)
       .def("capture_graphs", &Engine::capture_graphs, py::arg("max_b"), py::call_guard<py::gil_scoped_release>())
       .def_property_readonly("stream", &Engine::stream_handle)
       .def_property_readonly("k_cache_ptr", &Engine::kv_cache_k)
@@ -690,26 +729,28 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       "gemm_q",
       [](uintptr_t A, int lda, std::vector<PyQMatrix*> segs, int M, uintptr_t C, uintptr_t C16, int ldc, int epi,
          uintptr_t st, int ksplit, uintptr_t dbg_ts, int act, int glu_n0, int ldc16, uintptr_t bias16, int unary,
-         float pos, float neg, float scale) {
-        GemmQArgs a;
-        std::memset(&a, 0, sizeof(a));
-        if (segs.empty() || segs.size() > 3) throw std::runtime_error("gemm_q: 1..3 segments");
-        a.A = (const bf16_t*)A; a.lda = lda; a.nseg = (int)segs.size();
-        int n0 = 0;
-        for (int s = 0; s < a.nseg; ++s) { a.seg[s] = segs[s]->w; a.seg_n0[s] = n0; n0 += segs[s]->w.rows; }
-        a.M = M; a.N = n0; a.K = segs[0]->w.cols;
-        a.C = (float*)C; a.C16 = (bf16_t*)C16; a.ldc = ldc; a.epi = epi; a.ksplit = ksplit;
+         float pos, float neg, float scale, py::dict more) {
+        GemmQArgs a = gemm_q_args(segs, M, epi, ksplit, more);
+        a.A = (const bf16_t*)A; a.lda = lda;
+        a.C = (float*)C; a.C16 = (bf16_t*)C16; a.ldc = ldc;
         a.dbg_ts = (unsigned long long*)dbg_ts;
         a.act = act; a.glu_n0 = glu_n0; a.ldc16 = ldc16; a.bias16 = (const float*)bias16; a.unary = unary;
         a.act_n = ActNum{pos, neg, scale};
-        GemmWs& g = gemm_ws(M, a.N);
-        a.ws = g.ws; a.ws_bytes = g.bytes; a.cnt = g.cnt; a.cnt_len = g.cnt_len;
         launch_gemm_q(a, S(st));
       },
       py::arg("A"), py::arg("lda"), py::arg("segs"), py::arg("M"), py::arg("C"), py::arg("C16"), py::arg("ldc"),
       py::arg("epi"), py::arg("stream"), py::arg("ksplit") = 0, py::arg("dbg_ts") = 0, py::arg("act") = 0,
       py::arg("glu_n0") = 0, py::arg("ldc16") = 0, py::arg("bias16") = 0, py::arg("unary") = 0,
-      py::arg("pos") = 0.f, py::arg("neg") = 0.f, py::arg("scale") = 1.f);
+      py::arg("pos") = 0.f, py::arg("neg") = 0.f, py::arg("scale") = 1.f, py::arg("more") = py::dict());
+  // whether the K-shared GEMM of 2..32 rows takes such a launch
+  m.def(
+      "gemm_wk_serves",
+      [](std::vector<PyQMatrix*> segs, int M, int epi, int ksplit, py::dict more) {
+        GemmQArgs a = gemm_q_args(segs, M, epi, ksplit, more);
+        a.lda = a.K; a.ldc = a.N;
+        return gemm_wk_serves(a);
+      },
+      py::arg("segs"), py::arg("M"), py::arg("epi"), py::arg("ksplit") = 0, py::arg("more") = py::dict());
   m.def(
       "gemm_pf_plan",
       [](std::vector<PyQMatrix*> segs, int M, int epi, int ksplit) {
@@ -739,6 +780,8 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
   m.attr("GEPI_STORE") = (int)GEPI_STORE;
   m.attr("GEPI_ACCUM") = (int)GEPI_ACCUM;
   m.attr("GEPI_SWIGLU_BF16") = (int)GEPI_SWIGLU_BF16;
+  m.attr("GEPI_QKV") = (int)GEPI_QKV;
+  m.attr("GEPI_ACCUM_NORM") = (int)GEPI_ACCUM_NORM;
   m.attr("GEPI_STORE16") = (int)GEPI_STORE16;
   m.attr("GEPI_STORE_GLU") = (int)GEPI_STORE_GLU;
   m.def(

@@ -189,6 +189,7 @@ class Engine {
   void release_slot(int slot);         // drop every block reference of the slot
   int kv_blocks_free() const { return (int)free_blocks_.size(); }
   int kv_blocks_total() const { return kv_nblocks_; }
+  int decode_gemm_min_batch() const { return dec_gemm_min_b_; }  // rows from which decode takes the GEMMs
   int norm_fused_parts() const { return nrm_parts_; }  // 0: batched-decode RMSNorm not split into the GEMMs
   std::vector<int> block_table(int slot) const;
 

@@ -891,16 +891,17 @@ void Engine::gemm(GemmQArgs& g) {
 // MFMA GEMM (weights dequantised once per step into MFMA operands, split-K reduced in-launch),
 // with explicit RMSNorm -> bf16 and RoPE/KV-write launches in place of the GEMV prologue /
 // epilogue fusions.  SwiGLU runs in the gate/up GEMM's epilogue (bf16 out for the down GEMM).
-// Rows from which the GEMMs win (us a step, 8 steps behind ~300 keys, GEMV / GEMM):
+// Rows from which the GEMMs win (us a step, 8 steps behind ~300 keys, GEMVs forced / GEMMs):
 //   TinyLlama Q4_K (25 MB a layer)   2 rows  912 / 798    3 rows 1044 / 801    4 rows 1101 / 796
 //   Mistral-7B Q4_K (123 MB)         2 rows 1761 / 2024   3 rows 1969 / 2025   4 rows 2231 / 2014
 //   Qwen3-8B Q4_K (108 MB)           2 rows 2130 / 2337   3 rows 2389 / 2348   4 rows 2685 / 2364
 //   TinyLlama bf16                   2 rows  852 / 1006   3 rows  919 / 1012   4 rows  976 / 1007
 // The int8 GEMV's dot work grows with the rows, the GEMM's does not: it wins from 4, and from 2 where the layers are
-// so small that launches bound a step.  Only where K-shared waves serve every projection (Q4_K / Q6_K) and the GEMV
-// would take int8 activations; across ranks as before.
+// so small that launches bound a step (TinyLlama's d_ff has no GEMV plan at 2 rows either, so its GEMVs above are the
+// row-pair ones).  Only where K-shared waves serve every projection (Q4_K / Q6_K) and the GEMV would take int8
+// activations; across ranks as before.
 int Engine::default_gemm_min_b() const {
-  if (!cfg_.act_q8 || cfg_.tp_size > 1) return dec_gemm_min_b_;
+  if (!cfg_.act_q8 || cfg_.tp_size > 1 || !gemm_wk_on()) return dec_gemm_min_b_;
   size_t bytes = 0;
   for (const auto& L : layers_)
     for (const QMat* m : {&L.wq, &L.wk, &L.wv, &L.wo, &L.wgu, &L.wdown}) {

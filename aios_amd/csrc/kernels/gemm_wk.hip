@@ -308,60 +308,27 @@ __global__ void __launch_bounds__(WK_W * 64) __attribute__((amdgpu_waves_per_eu(
   wk_body<QT0, NS, MT, EPI, false>(a, p, rg, sp, t0, t0 + p.q0 + (rg < p.r0 ? 1 : 0), smem, inv_s, last_flag);
 }
 
-template <int QT0, int QT1, int NS, int MT>
-static bool wk_launch(const GemmQArgs& a, int S, hipStream_t st) {
-  const int nt = a.N / 16, cus = device_cu_count();
-  const int nt0 = QT0 != QT1 ? a.seg_n0[a.nseg - 1] / 16 : nt;
-  const int G = std::min(nt, std::max(1, cus / S));
-  int g0 = G;
-  if (QT0 != QT1) {  // groups in the share of the bytes (144 and 210 per 256 weights)
-    if (G < 2) return false;
-    g0 = std::max(1, std::min({G - 1, nt0, (int)((long)G * nt0 * 144 / ((long)nt0 * 144 + (long)(nt - nt0) * 210))}));
-    if (G - g0 > nt - nt0) g0 = G - (nt - nt0);
-  }
-  if (S > 1 && (!a.ws || !a.cnt || a.cnt_len < G || a.ws_bytes < (size_t)S * 16 * MT * a.N * 4)) return false;
-  const int nu = a.K / (QT0 == QT_BF16 ? 64 : 256), n1 = nt - nt0, g1 = std::max(G - g0, 1);
-  const WkPlan p = {S, G, g0, nt0, nt0 / g0, nt0 % g0, n1 / g1, n1 % g1, nu / S, nu % S, a.seg_n0[a.nseg - 1], a.seg[a.nseg - 1]};
-  const dim3 grid(G * S), block(WK_W * 64);
-#define WK_GO(E) hipLaunchKernelGGL((gemm_wk_kernel<QT0, QT1, NS, MT, E>), grid, block, 0, st, a, p)
-  if constexpr (QT0 != QT1) {
-    if (a.epi == GEPI_QKV) WK_GO(GEPI_QKV);
-    else WK_GO(GEPI_STORE);
-    return true;
-  } else {
-    switch (a.epi) {
-      case GEPI_STORE: WK_GO(GEPI_STORE); break;
-      case GEPI_QKV:  // (three segments' four planes and the cache's arguments: more scalars than there are)
-        if constexpr (QT0 == QT_Q6_K && NS * MT == 4) return false;
-        else WK_GO(GEPI_QKV);
-        break;
-      case GEPI_ACCUM: WK_GO(GEPI_ACCUM); break;
-      case GEPI_ACCUM_NORM: WK_GO(GEPI_ACCUM_NORM); break;
-      case GEPI_STORE16:
-        if constexpr (QT0 == QT_BF16) WK_GO(GEPI_STORE16);
-        break;
-      case GEPI_STORE_GLU:
-        if constexpr (QT0 == QT_BF16) WK_GO(GEPI_STORE_GLU);
-        break;
-      default: WK_GO(GEPI_SWIGLU_BF16); break;
-    }
-    return true;
-  }
-#undef WK_GO
-}
+// what a launch is given: K slices, stages of the longest wave (NS), 16-row groups (MT), workgroups that share the tiles
+struct WkRoute {
+  int S, ns, mt, G;
+};
 
-static int wk_env(const char* name, int dflt) {
-  const char* e = std::getenv(name);
-  return e ? std::atoi(e) : dflt;
+bool gemm_wk_on() {
+  const char* e = std::getenv("AIOS_GEMM_WK");  // (read per call: tests compare both)
+  return !e || std::atoi(e);
 }
 
 // AIOS_GEMM_WK: 1 (default) = this serves M = 2..32 of Q4_K / Q6_K / bf16 and the packed Q4_K | Q6_K QKV; 0 = the ring
 // (quantised) and skinny GEMMs
-bool launch_gemm_wk(const GemmQArgs& a, hipStream_t st) {
-  static const int on = wk_env("AIOS_GEMM_WK", 1);
-  if (!on || a.M < 2 || a.M > 32 || a.N % 16 || a.lda % 8) return false;
+static bool wk_route(const GemmQArgs& a, WkRoute& r) {
+  if (!gemm_wk_on() || a.M < 2 || a.M > 32 || a.N % 16 || a.lda % 8) return false;
   const int qt0 = a.seg[0].qtype, qt1 = a.seg[a.nseg - 1].qtype;
-  const bool bf = qt0 == QT_BF16;
+  const bool bf = qt0 == QT_BF16, mixed = qt0 == QT_Q4_K && qt1 == QT_Q6_K;
+#ifdef AIOS_BF16_ONLY
+  if (!bf) return false;
+#endif
+  if (!mixed && (qt0 != qt1 || (!bf && qt0 != QT_Q4_K && qt0 != QT_Q6_K))) return false;
+  if (mixed && a.epi != GEPI_QKV && a.epi != GEPI_STORE) return false;
   if ((a.epi == GEPI_STORE16 || a.epi == GEPI_STORE_GLU) && !bf) return false;
   if (a.K % (bf ? 64 : 256) || ((uintptr_t)a.A & 3)) return false;
   if (((size_t)(a.M - 1) * a.lda + a.K) * 2 >= 0xfffffff0u || (size_t)a.K * 32 >= 0x7fffffffu) return false;
@@ -375,37 +342,90 @@ bool launch_gemm_wk(const GemmQArgs& a, hipStream_t st) {
   // K's slices: as few as leave a wave at most NSM stages.  Two (X: 64 or 128 registers; a bf16 stage's weights take 32):
   // with four at 16 rows the longer prologue costs more than slabs save, 4096 x 14336 in two slices 16.3 us, in four 14.6,
   // 2048 x 5632 in one 8.7, in two 7.5; but a second slice that the registers do not ask for loses, 4096 x 4096 6.3 -> 8.5.
-  const int MT = a.M <= 16 ? 1 : 2, NSM = bf ? 2 / MT : 2, un = bf ? 64 : 256, nu = a.K / un, ups = 256 / un;
+  r.mt = a.M <= 16 ? 1 : 2;
+  const int NSM = bf ? 2 / r.mt : 2, un = bf ? 64 : 256, nu = a.K / un, ups = 256 / un;
   auto stages = [&](int S) {  // of the longest wave
     const int n = (nu + S - 1) / S;
     return ((n + WK_W - 1) / WK_W + ups - 1) / ups;
   };
-  int S = std::max(1, std::min(a.ksplit, nu));
-  while (stages(S) > NSM) ++S;
-  if (S > WK_SMAX) return false;
+  r.S = std::max(1, std::min(a.ksplit, nu));
+  while (stages(r.S) > NSM) ++r.S;
+  if (r.S > WK_SMAX) return false;
+  r.ns = stages(r.S);
   // Q6_K's long down projection: the ring's deeper stream still wins up to 16 rows, 4096 x 14336 in 18.5 - 19.2 us to
   // 19.0 - 19.5 here
-  if (qt0 == QT_Q6_K && S > 2 && MT == 1 && a.N % 128 == 0) return false;
-  const int ns = stages(S);
+  if (qt0 == QT_Q6_K && r.S > 2 && r.mt == 1 && a.N % 128 == 0) return false;
+  // (three segments' four planes and the cache's arguments: more scalars than there are)
+  if (a.epi == GEPI_QKV && qt0 == QT_Q6_K && r.ns * r.mt == 4) return false;
+  r.G = std::min(a.N / 16, std::max(1, device_cu_count() / r.S));
+  if (mixed && r.G < 2) return false;
+  return r.S == 1 || (a.ws && a.cnt && a.cnt_len >= r.G && a.ws_bytes >= (size_t)r.S * 16 * r.mt * a.N * 4);
+}
+
+bool gemm_wk_serves(const GemmQArgs& a) {
+  WkRoute r;
+  return wk_route(a, r);
+}
+
+template <int QT0, int QT1, int NS, int MT>
+static void wk_launch(const GemmQArgs& a, const WkRoute& r, hipStream_t st) {
+  const int nt = a.N / 16, S = r.S, G = r.G;
+  const int nt0 = QT0 != QT1 ? a.seg_n0[a.nseg - 1] / 16 : nt;
+  int g0 = G;
+  if (QT0 != QT1) {  // groups in the share of the bytes (144 and 210 per 256 weights)
+    g0 = std::max(1, std::min({G - 1, nt0, (int)((long)G * nt0 * 144 / ((long)nt0 * 144 + (long)(nt - nt0) * 210))}));
+    if (G - g0 > nt - nt0) g0 = G - (nt - nt0);
+  }
+  const int nu = a.K / (QT0 == QT_BF16 ? 64 : 256), n1 = nt - nt0, g1 = std::max(G - g0, 1);
+  const WkPlan p = {S, G, g0, nt0, nt0 / g0, nt0 % g0, n1 / g1, n1 % g1, nu / S, nu % S, a.seg_n0[a.nseg - 1], a.seg[a.nseg - 1]};
+  const dim3 grid(G * S), block(WK_W * 64);
+#define WK_GO(E) hipLaunchKernelGGL((gemm_wk_kernel<QT0, QT1, NS, MT, E>), grid, block, 0, st, a, p)
+  if constexpr (QT0 != QT1) {
+    if (a.epi == GEPI_QKV) WK_GO(GEPI_QKV);
+    else WK_GO(GEPI_STORE);
+  } else {
+    switch (a.epi) {
+      case GEPI_STORE: WK_GO(GEPI_STORE); break;
+      case GEPI_QKV:
+        if constexpr (QT0 != QT_Q6_K || NS * MT < 4) WK_GO(GEPI_QKV);  // (else: wk_route)
+        break;
+      case GEPI_ACCUM: WK_GO(GEPI_ACCUM); break;
+      case GEPI_ACCUM_NORM: WK_GO(GEPI_ACCUM_NORM); break;
+      case GEPI_STORE16:
+        if constexpr (QT0 == QT_BF16) WK_GO(GEPI_STORE16);
+        break;
+      case GEPI_STORE_GLU:
+        if constexpr (QT0 == QT_BF16) WK_GO(GEPI_STORE_GLU);
+        break;
+      default: WK_GO(GEPI_SWIGLU_BF16); break;
+    }
+  }
+#undef WK_GO
+}
+
+bool launch_gemm_wk(const GemmQArgs& a, hipStream_t st) {
+  WkRoute r;
+  if (!wk_route(a, r)) return false;
   auto go = [&](auto q0, auto q1) {
     constexpr int A = decltype(q0)::value, B = decltype(q1)::value;
-    if (MT == 1) {
-      if (ns <= 1) return wk_launch<A, B, 1, 1>(a, S, st);
-      return wk_launch<A, B, 2, 1>(a, S, st);
+    if (r.mt == 1) {
+      if (r.ns <= 1) wk_launch<A, B, 1, 1>(a, r, st);
+      else wk_launch<A, B, 2, 1>(a, r, st);
+    } else {
+      if (A == QT_BF16 || r.ns <= 1) wk_launch<A, B, 1, 2>(a, r, st);
+      else if constexpr (A != QT_BF16) wk_launch<A, B, 2, 2>(a, r, st);
     }
-    if (ns <= 1) return wk_launch<A, B, 1, 2>(a, S, st);
-    if constexpr (A != QT_BF16) return wk_launch<A, B, 2, 2>(a, S, st);
-    return false;
   };
 #define WK_T(Q) std::integral_constant<int, Q>{}
-  if (bf) return qt1 == QT_BF16 && go(WK_T(QT_BF16), WK_T(QT_BF16));
+  const int qt0 = a.seg[0].qtype, qt1 = a.seg[a.nseg - 1].qtype;
+  if (qt0 == QT_BF16) go(WK_T(QT_BF16), WK_T(QT_BF16));
 #ifndef AIOS_BF16_ONLY
-  if (qt0 == QT_Q4_K && qt1 == QT_Q4_K) return go(WK_T(QT_Q4_K), WK_T(QT_Q4_K));
-  if (qt0 == QT_Q6_K && qt1 == QT_Q6_K) return go(WK_T(QT_Q6_K), WK_T(QT_Q6_K));
-  if (qt0 == QT_Q4_K && qt1 == QT_Q6_K && (a.epi == GEPI_QKV || a.epi == GEPI_STORE)) return go(WK_T(QT_Q4_K), WK_T(QT_Q6_K));
+  else if (qt0 == QT_Q6_K) go(WK_T(QT_Q6_K), WK_T(QT_Q6_K));
+  else if (qt1 == QT_Q6_K) go(WK_T(QT_Q4_K), WK_T(QT_Q6_K));
+  else go(WK_T(QT_Q4_K), WK_T(QT_Q4_K));
 #endif
 #undef WK_T
-  return false;
+  return true;
 }
 
 }  // namespace aios

@@ -258,6 +258,10 @@ int gemm_skinny_cnt_len(int N);
 // output tiles of the skinny kernel for these args (0: not served by the skinny kernel)
 int gemm_skinny_ntile(const GemmQArgs& a);
 void launch_gemm_q(const GemmQArgs& a, hipStream_t st);
+// 2..32 rows with K shared by a workgroup's waves (kernels/gemm_wk.hip): whether it may (AIOS_GEMM_WK), and whether it
+// takes these args
+bool gemm_wk_on();
+bool gemm_wk_serves(const GemmQArgs& a);
 // the prefill GEMM (kernels/gemm_pf.hip): true if it took the launch; its tile / split plan for a shape
 bool launch_gemm_pf(const GemmQArgs& a, hipStream_t st);
 bool gemm_pf_serves(const GemmQArgs& a);  // launch_gemm_pf would take a (gemm_pf.hip)

@@ -116,7 +116,7 @@ def measure(preset: str, recipe: str, batch: int, prompt: int, steps: int, warmu
     dt = time.perf_counter() - t0
     hist = eng.decode_loop_history(batch, prompt + warmup + 1, steps)
     assert all(0 <= t < cfg.vocab_size for t in hist), "invalid token ids from decode loop"
-    info = dict(weight_gb=round(eng.weight_bytes / 1e9, 3), kv_gb=round(eng.kv_bytes / 1e9, 3),
+    info = dict(gemm_from=eng.decode_gemm_min_batch, weight_gb=round(eng.weight_bytes / 1e9, 3), kv_gb=round(eng.kv_bytes / 1e9, 3),
                 workspace_gb=round(eng.workspace_bytes / 1e9, 3))
     del eng
     return dt, info
@@ -426,6 +426,7 @@ def main():
     n = world
     total_tokens = n * args.batch * args.steps
     value = total_tokens / dt
+    gemm_from = info.pop("gemm_from")
     if rank == 0:
         headline = args.model == "mistral-7b" and args.recipe == "Q4_K_M"
         out = {
@@ -456,7 +457,7 @@ def main():
                 "activations": ("int8 per-32-block activations with fp32 scales in the quantised GEMVs "
                                 "(q8_1 as llama.cpp), fp32 residual stream, fp32 accumulate" if act_q8 else
                                 "fp32 activations in the GEMVs, fp32 accumulate") +
-                               "; int8 GEMV engine up to B = 4, bf16 MFMA operands for B >= 5; attention: " +
+                               f"; bf16 MFMA operands from B = {gemm_from}; attention: " +
                                ("fp8 e4m3 KV cache (per-layer scales)" if args.kv_dtype != "bf16" else "bf16 KV cache") +
                                ", bf16-rounded q, fp32 softmax",
                 "per_gpu_batch": args.batch,

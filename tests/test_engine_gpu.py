@@ -357,6 +357,34 @@ def test_batched_int8_gemv_engine_matches_single_rows(model_files, monkeypatch, 
         assert np.abs(single - batched[b]).max() < 2e-3 * max(np.abs(single).max(), 1.0)
 
 
+@pytest.mark.parametrize("B", [2, 3])
+def test_small_batches_stay_on_the_gemv_without_the_k_shared_gemm(monkeypatch, B):
+    """AIOS_GEMM_WK=0: the row count from which decode takes the GEMMs is the one measured for the GEMMs that are left -- bit
+    for bit the logits of an engine told 5; with the K-shared GEMM small models take it from 2 rows.  (d_ff 6144: every
+    projection has a GEMV plan.)"""
+    import dataclasses
+
+    from aios_amd.runtime.loader import random_engine
+
+    cfg, outs = dataclasses.replace(get_preset("tinyllama-1.1b"), n_layers=2, vocab_size=2048, d_ff=6144), {}
+    prompts = [list(range(5 + b, 15 + 2 * b)) for b in range(B)]
+    for how, env in (("off", {"AIOS_GEMM_WK": "0"}), ("off, gemv", {"AIOS_GEMM_WK": "0", "AIOS_DECODE_GEMM_MIN_B": "5"}),
+                     ("on", {}), ("on, gemm", {"AIOS_DECODE_GEMM_MIN_B": "2"})):
+        with monkeypatch.context() as mp:
+            for k, v in env.items():
+                mp.setenv(k, v)
+            eng = random_engine(cfg, "Q4_K_M", seed=3, max_ctx=256, max_batch=4)
+            for s, p in enumerate(prompts):
+                eng.prefill(s, p, 0, False)
+            eng.decode(list(range(B)), [7] * B, [len(p) for p in prompts])
+            assert eng.decode_gemm_min_batch == (5 if how.startswith("off") else 2)
+            outs[how] = np.asarray(eng.last_logits(B)).reshape(B, -1)
+            del eng
+    assert np.isfinite(outs["on"]).all()
+    assert np.array_equal(outs["off"], outs["off, gemv"]) and np.array_equal(outs["on"], outs["on, gemm"])
+    assert not np.array_equal(outs["on"], outs["off"])
+
+
 @pytest.mark.parametrize("recipe,rb,split", [("Q4_K_M", "0", "0"), ("Q4_K_M", "4", "1"),
                                              ("mistral_shape", "0", "1"), ("mistral_shape", "4", "0")])
 def test_batched_decode_split_rmsnorm_matches_explicit(model_files, monkeypatch, recipe, rb, split):
