@@ -240,8 +240,8 @@ static void launch_big(const GemmQArgs& a, hipStream_t st) {
 // operand registers; returns false when the shape / workspace does not fit it
 bool launch_gemm_skinny(const GemmQArgs& a, hipStream_t st);
 bool gemm_skinny_mixed_ok(const GemmQArgs& a);
-// M <= 32: Q4_K / Q6_K / bf16 with K shared by a workgroup's waves (gemm_wk.hip); Q4_K / Q6_K on the LDS-DMA ring
-// (gemm_ring.hip); false when they do not serve the shape
+// M <= 32: Q4_K / Q6_K / bf16 with K shared by a workgroup's waves (gemm_wk.hip); Q6_K on the LDS-DMA ring (gemm_ring.hip);
+// false when they do not serve the shape
 bool launch_gemm_wk(const GemmQArgs& a, hipStream_t st);
 bool launch_gemm_ring(const GemmQArgs& a, hipStream_t st);
 // M >= 33, Q4_K / Q6_K / mixed / bf16 stacks: the LDS-DMA prefill GEMM (gemm_pf.hip)

@@ -352,9 +352,12 @@ static bool wk_route(const GemmQArgs& a, WkRoute& r) {
   while (stages(r.S) > NSM) ++r.S;
   if (r.S > WK_SMAX) return false;
   r.ns = stages(r.S);
-  // Q6_K's long down projection: the ring's deeper stream still wins up to 16 rows, 4096 x 14336 in 18.5 - 19.2 us to
-  // 19.0 - 19.5 here
-  if (qt0 == QT_Q6_K && r.S > 2 && r.mt == 1 && a.N % 128 == 0) return false;
+  // Q6_K's long down projections up to 16 rows: the ring's deeper stream is the faster one where its 128-row tiles in
+  // eight slices cover three quarters of the CUs.  us here / ring, 4 and 16 rows (7 runs each, apart by 2 % at most):
+  //   4096 x 14336 19.3 / 18.3, 19.8 / 19.1    4096 x 12288 18.1 / 16.6, 18.4 / 17.4    5120 x 17408 28.2 / 26.2, 29.0 / 27.1
+  //   3584 x 18944 22.7 / 22.0, 23.4 / 23.1    8192 x 28672 59.1 / 55.1, 60.2 / 57.3    4096 x 11008 16.5 / 16.5, 17.0 / 16.9
+  //   2048 x 8704 11.5 / 12.4, 11.8 / 13.2
+  if (qt0 == QT_Q6_K && r.S > 2 && r.mt == 1 && a.N % 128 == 0 && a.N / 128 * 8 * 4 >= 3 * device_cu_count()) return false;
   // (three segments' four planes and the cache's arguments: more scalars than there are)
   if (a.epi == GEPI_QKV && qt0 == QT_Q6_K && r.ns * r.mt == 4) return false;
   r.G = std::min(a.N / 16, std::max(1, device_cu_count() / r.S));

@@ -937,7 +937,9 @@ def test_attention_prefill_split_over_keys(E, H, Hkv, hd, start, T, fp8):
 @pytest.mark.parametrize("M", [2, 16, 33, 64])
 @pytest.mark.parametrize("ksplit", [1, 3])
 @pytest.mark.parametrize("epi", ["store", "accum", "swiglu"])
-def test_gemm_skinny(E, t, M, ksplit, epi):
+@pytest.mark.parametrize("own", ["", "0"])  # "0": without the kernels that take up to 32 rows of some formats
+def test_gemm_skinny(E, t, M, ksplit, epi, own, monkeypatch):
+    small_gemms(monkeypatch, own, own)
     N, K = 256, 2048
     m, W = qmat(E, t, N, K, seed=31, std=0.05)
     A = torch.randn(M, K, device="cuda").to(torch.bfloat16)
@@ -960,7 +962,9 @@ def test_gemm_skinny(E, t, M, ksplit, epi):
 @pytest.mark.parametrize("t", [GGMLType.Q4_K, GGMLType.Q6_K])
 @pytest.mark.parametrize("M", [8, 40])
 @pytest.mark.parametrize("ksplit", [9, 16])
-def test_gemm_skinny_wide_split(E, t, M, ksplit):
+@pytest.mark.parametrize("own", ["", "0"])
+def test_gemm_skinny_wide_split(E, t, M, ksplit, own, monkeypatch):
+    small_gemms(monkeypatch, own, own)
     # K = 14336 over 9 / 16 slices: the last arriver sums the slabs in batches of 8 (fixed order)
     N, K = 256, 14336
     m, W = qmat(E, t, N, K, seed=61, std=0.01)
@@ -975,7 +979,9 @@ def test_gemm_skinny_wide_split(E, t, M, ksplit):
 
 
 @pytest.mark.parametrize("M", [4, 32])
-def test_gemm_skinny_mixed_segments_long_k(E, M):
+@pytest.mark.parametrize("own", ["", "0"])
+def test_gemm_skinny_mixed_segments_long_k(E, M, own, monkeypatch):
+    small_gemms(monkeypatch, own, own)
     # Q4_K_M-style QKV (Q4_K q/k + Q6_K v, one mixed-format launch) and a K = 14336 down projection with the
     # automatic split: every tile's last arriver reduces the slabs (tickets re-armed per launch)
     K = 4096
@@ -1035,16 +1041,25 @@ def test_gemm_error_vs_unquantized_product(E, t, M, ksplit):
     assert per_row < 1e-2, per_row
 
 
-# ---- the LDS-DMA ring GEMM (gemm_ring.hip): batched decode M = 5..32 on Q4_K / Q6_K / mixed stacks ----
+def small_gemms(monkeypatch, wk="", ring=""):
+    """which kernels may take 2..32 rows ("": as by default)"""
+    for name, v in (("AIOS_GEMM_WK", wk), ("AIOS_GEMM_RING", ring)):
+        if v:
+            monkeypatch.setenv(name, v)
+
+
+# ---- batched decode M = 5..32 on Q4_K / Q6_K / mixed stacks; the LDS-DMA ring GEMM (gemm_ring.hip) ----
 @pytest.mark.parametrize("M", [5, 8, 13, 16, 17, 24, 32])
 @pytest.mark.parametrize("segs,K", [([(GGMLType.Q4_K, 384)], 4096), ([(GGMLType.Q6_K, 256)], 14336),
                                     ([(GGMLType.Q4_K, 256), (GGMLType.Q4_K, 128), (GGMLType.Q6_K, 128)], 4096),
                                     ([(GGMLType.Q4_K, 128)], 1024)])
 @pytest.mark.parametrize("epi", ["store", "accum"])
-def test_gemm_ring_vs_unquantized(E, M, segs, K, epi):
+@pytest.mark.parametrize("wk", ["", "0"])  # "0": without the K-shared GEMM (Q6_K: the ring; the others: skinny)
+def test_gemm_ring_vs_unquantized(E, M, segs, K, epi, wk, monkeypatch):
     """Against the UNQUANTIZED fp32 product (exact dequantised weights x the fp32 activations): ring
     slots of one 256-k superblock, the automatic split-K (one dispatch round) reduced by the tile's
     last arriver, padded activation rows (M not a multiple of 16), the mixed-format QKV launch"""
+    small_gemms(monkeypatch, wk)
     mats, refs = zip(*[qmat(E, t, n, K, seed=80 + i, std=0.02) for i, (t, n) in enumerate(segs)])
     W = torch.cat(refs, 0)
     N = W.shape[0]
@@ -1063,9 +1078,11 @@ def test_gemm_ring_vs_unquantized(E, M, segs, K, epi):
 
 
 @pytest.mark.parametrize("M", [6, 16, 32])
-def test_gemm_ring_swiglu(E, M):
+@pytest.mark.parametrize("t,wk", [(GGMLType.Q4_K, ""), (GGMLType.Q4_K, "0"), (GGMLType.Q6_K, "0")])
+def test_gemm_ring_swiglu(E, M, t, wk, monkeypatch):
+    small_gemms(monkeypatch, wk)
     N, K = 512, 4096
-    m, W = qmat(E, GGMLType.Q4_K, N, K, seed=91, std=0.05)
+    m, W = qmat(E, t, N, K, seed=91, std=0.05)
     A = torch.randn(M, K, device="cuda").to(torch.bfloat16)
     out = torch.zeros(M, N // 2, dtype=torch.bfloat16, device="cuda")
     E.gemm_q(A.data_ptr(), K, [m], M, 0, out.data_ptr(), N // 2, E.GEPI_SWIGLU_BF16, stream())
@@ -1102,6 +1119,8 @@ def test_gemm_wk(E, M, segs, K, ksplit, epi):
             mats.append(m)
         W.append(w.to(torch.bfloat16).double())
     W = torch.cat(W)
+    assert E.gemm_wk_serves(mats, M, {"store": E.GEPI_STORE, "accum": E.GEPI_ACCUM, "store16": E.GEPI_STORE16,
+                                      "swiglu": E.GEPI_SWIGLU_BF16}[epi], ksplit)
     N, lda = W.shape[0], K + 8
     A = torch.randn(M, lda, generator=g).to(torch.bfloat16)
     y, Ad = A[:, :K].double() @ W.T, A.cuda()
@@ -1122,6 +1141,131 @@ def test_gemm_wk(E, M, segs, K, ksplit, epi):
         torch.cuda.synchronize()
         got = out.cpu().double()
         assert ((got - ref).norm(dim=1) / ref.norm(dim=1)).max() < tol
+
+
+SMALL = {"wk": ("", ""), "ring": ("0", ""), "skinny": ("0", "0")}
+
+
+def small_mat(E, t, rows, K, seed):
+    """(matrix, its values as the kernels multiply them: rounded to bf16)"""
+    if t == "BF16":
+        w = (torch.randn(rows, K, generator=torch.Generator().manual_seed(seed)) * 0.05).to(torch.bfloat16)
+        return E.QMatrix(int(GGMLType.BF16), rows, K, w.view(torch.int16).numpy()), w.double()
+    m, w = qmat(E, GGMLType[t], rows, K, seed=seed, std=0.05)
+    return m, w.to(torch.bfloat16).double()
+
+
+def sum_tol(t, K):
+    """fp32 sums of K exact products, and quantised weights at a rounding boundary (see test_gemm_wk)"""
+    return K * 2.0 ** -24 + (0.0 if t == "BF16" else 2.0 ** -13)
+
+
+def test_gemm_wk_leaves_q6k_down_to_the_ring(E):
+    """long K up to 16 rows where the ring's tiles in eight slices cover three quarters of the CUs; not below, and no other
+    format; the packed Q6_K QKV from 17 rows up has no form with a wave's two stages"""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    edge = -(-3 * cus // 32) * 128
+    K = 8448  # three slices
+    mats = {(t, n): E.QMatrix(int(GGMLType[t]), n, K, np.zeros(n * K // 256 * b, np.uint8))
+            for t, b in (("Q6_K", 210), ("Q4_K", 144)) for n in (edge - 128, edge)}
+    assert not E.gemm_wk_serves([mats["Q6_K", edge]], 16, E.GEPI_ACCUM)
+    assert E.gemm_wk_serves([mats["Q6_K", edge - 128]], 16, E.GEPI_ACCUM)
+    assert E.gemm_wk_serves([mats["Q6_K", edge]], 17, E.GEPI_ACCUM) and E.gemm_wk_serves([mats["Q4_K", edge]], 16, E.GEPI_ACCUM)
+    assert not E.gemm_wk_serves([mats["Q6_K", edge - 128]], 17, E.GEPI_QKV)
+    assert E.gemm_wk_serves([mats["Q4_K", edge]], 17, E.GEPI_QKV)
+
+
+@pytest.mark.parametrize("kernel,t", [("wk", "Q4_K"), ("wk", "Q6_K"), ("wk", "BF16"), ("ring", "Q6_K"), ("skinny", "Q4_K"),
+                                      ("skinny", "Q6_K"), ("skinny", "BF16")])
+@pytest.mark.parametrize("M", [2, 17, 32])
+@pytest.mark.parametrize("K1,K2", [(256, 512), (2304, 1024), (256, 8192)])
+def test_small_gemm_split_rmsnorm(E, kernel, t, M, K1, K2, monkeypatch):
+    """the residual GEMM's bf16(x g) and sums of squares per 16 columns (wider tiles: the first part holds the tile's), and
+    the next GEMM's rows scaled by them, up to 512 parts a row, against float64"""
+    small_gemms(monkeypatch, *SMALL[kernel])
+    g = torch.Generator().manual_seed(K2 + M)
+    (m1, W1), (m2, W2) = small_mat(E, t, K2, K1, 11), small_mat(E, t, 128, K2, 12)
+    A = torch.randn(M, K1, generator=g).to(torch.bfloat16)
+    res, gain = torch.randn(M, K2, generator=g), torch.rand(K2, generator=g) + 0.5
+    Ad, gd, C = A.cuda(), gain.cuda(), res.cuda()
+    x16, part = torch.zeros(M, K2, dtype=torch.bfloat16, device="cuda"), torch.full((M, K2 // 16), float("nan"), device="cuda")
+    more = dict(nrm_g=gd.data_ptr(), nrm_out16=x16.data_ptr(), nrm_part=part.data_ptr(), nrm_parts=K2 // 16)
+    assert E.gemm_wk_serves([m1], M, E.GEPI_ACCUM_NORM, more=more) == (kernel == "wk")
+    E.gemm_q(Ad.data_ptr(), K1, [m1], M, C.data_ptr(), 0, K2, E.GEPI_ACCUM_NORM, stream(), more=more)
+    torch.cuda.synchronize()
+    ref = res.double() + A.double() @ W1.T
+    assert ((C.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)).max() < sum_tol(t, K1) + 2.0 ** -23
+    assert torch.equal(x16, (C * gd).to(torch.bfloat16))
+    sq = C.cpu().double().pow(2).sum(1)
+    assert ((part.cpu().double().sum(1) - sq).abs() / sq).max() < 2.0 ** -20  # (at most 128 squares an fp32 sum)
+    y, more = torch.zeros(M, 128, device="cuda"), dict(nrm_in=part.data_ptr(), nrm_parts=K2 // 16, nrm_eps=1e-5)
+    assert E.gemm_wk_serves([m2], M, E.GEPI_STORE, more=more) == (kernel == "wk")
+    E.gemm_q(x16.data_ptr(), K2, [m2], M, y.data_ptr(), 0, 128, E.GEPI_STORE, stream(), more=more)
+    torch.cuda.synchronize()
+    ref = (x16.cpu().double() @ W2.T) * torch.rsqrt(sq / K2 + 1e-5)[:, None]
+    assert ((y.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)).max() < sum_tol(t, K2) + 2.0 ** -19
+
+
+@pytest.mark.parametrize("kernel,ts", [("wk", "Q4_K Q4_K Q4_K"), ("wk", "Q4_K Q4_K Q6_K"), ("wk", "Q6_K Q6_K Q6_K"),
+                                       ("wk", "BF16 BF16 BF16"), ("ring", "Q6_K Q6_K Q6_K"), ("skinny", "Q4_K Q4_K Q6_K")])
+@pytest.mark.parametrize("M", [2, 17, 32])
+@pytest.mark.parametrize("K", [512, 4096])
+def test_small_gemm_qkv(E, kernel, ts, M, K, monkeypatch):
+    """the packed QKV product through RoPE to q and the paged cache, fused RMSNorm in front, against float64"""
+    small_gemms(monkeypatch, *SMALL[kernel])
+    ts, H, Hkv, hd, slots, max_ctx = ts.split(), 4, 2, 64, 4, 256
+    rows = (H * hd, Hkv * hd, Hkv * hd)
+    mats, W = zip(*[small_mat(E, t, n, K, 21 + i) for i, (t, n) in enumerate(zip(ts, rows))])
+    served = kernel == "wk" and not (ts[0] == "Q6_K" and M > 16 and K > 2048)
+    g = torch.Generator().manual_seed(K + M)
+    A, part = torch.randn(M, K, generator=g).to(torch.bfloat16), torch.rand(M, K // 16, generator=g) * 32
+    pos = torch.arange(M) * 7 % 200 + torch.arange(M) // slots
+    slot = torch.arange(M) % slots
+    ang = torch.arange(max_ctx)[:, None].double() * 1e4 ** (-2.0 * torch.arange(hd // 2).double() / hd)
+    cs = torch.stack([ang.cos(), ang.sin()], -1).float()
+    kp, bt = paged_cache(torch.zeros(slots, Hkv, max_ctx, hd, dtype=torch.bfloat16), True, seed=3)
+    dev = [x.cuda() for x in (A, part, pos.int(), slot.int(), cs, kp, torch.zeros_like(kp), bt)]
+    Ad, pd, posd, slotd, csd, kd, vd, btd = dev
+    q = torch.zeros(M, rows[0], device="cuda")
+    more = dict(nrm_in=pd.data_ptr(), nrm_parts=K // 16, nrm_eps=1e-5, head_dim=hd, q_dim=rows[0], kv_dim=rows[1], n_kv_heads=Hkv,
+                max_ctx=max_ctx, rope_cs=csd.data_ptr(), pos=posd.data_ptr(), slot=slotd.data_ptr(), block_table=btd.data_ptr(),
+                q_out=q.data_ptr(), k_cache=kd.data_ptr(), v_cache=vd.data_ptr())
+    assert E.gemm_wk_serves(list(mats), M, E.GEPI_QKV, more=more) == served
+    E.gemm_q(Ad.data_ptr(), K, list(mats), M, 0, 0, sum(rows), E.GEPI_QKV, stream(), more=more)
+    torch.cuda.synchronize()
+    y = (A.double() @ torch.cat(W).T) * torch.rsqrt(part.double().sum(1) / K + 1e-5)[:, None]
+
+    def turn(x):
+        a, b, c, s = x[..., 0::2], x[..., 1::2], ang.cos()[pos][:, None], ang.sin()[pos][:, None]
+        return torch.stack([a * c - b * s, a * s + b * c], -1).reshape(x.shape)
+
+    yq, yk, yv = y.split(rows, 1)
+    ref = turn(yq.view(M, H, hd)).reshape(M, -1)
+    tol = max(sum_tol(t, K) for t in ts) + 2.0 ** -19
+    assert ((q.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)).max() < tol
+    for cache, ref in ((kd, turn(yk.view(M, Hkv, hd))), (vd, yv.view(M, Hkv, hd))):
+        got = unpaged(cache.cpu(), slots, max_ctx, bt)[slot, :, pos].double()
+        # (8 bits of significand: a value just above a power of two is rounded by up to 2^-8 of itself)
+        assert ((got - ref).flatten(1).norm(dim=1) / ref.flatten(1).norm(dim=1)).max() < tol + 2.0 ** -8
+
+
+@pytest.mark.parametrize("kernel", ["wk", "skinny"])
+@pytest.mark.parametrize("M", [2, 17, 32])
+@pytest.mark.parametrize("K", [64, 2112])
+def test_small_gemm_store_glu(E, kernel, M, K, monkeypatch):
+    """bf16: the first columns stored in fp32, the interleaved gate / up ones behind them through the GLU"""
+    small_gemms(monkeypatch, *SMALL[kernel])
+    n0, N = 64, 320
+    m, W = small_mat(E, "BF16", N, K, 31)
+    A = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    Ad, C, C16 = A.cuda(), torch.zeros(M, n0, device="cuda"), torch.zeros(M, (N - n0) // 2, dtype=torch.bfloat16, device="cuda")
+    assert E.gemm_wk_serves([m], M, E.GEPI_STORE_GLU, more={}) == (kernel == "wk")
+    E.gemm_q(Ad.data_ptr(), K, [m], M, C.data_ptr(), C16.data_ptr(), n0, E.GEPI_STORE_GLU, stream(), glu_n0=n0, ldc16=(N - n0) // 2)
+    torch.cuda.synchronize()
+    y = A.double() @ W.T
+    z = torch.nn.functional.silu(y[:, n0::2]) * y[:, n0 + 1::2]
+    assert ((C.cpu().double() - y[:, :n0]).norm(dim=1) / y[:, :n0].norm(dim=1)).max() < sum_tol("BF16", K)
+    assert ((C16.cpu().double() - z).norm(dim=1) / z.norm(dim=1)).max() < 2.0 ** -8
 
 
 # ---- the LDS-DMA engine serving B = 2..4 rows from one weight stream (small-batch decode) --------
