@@ -727,9 +727,9 @@ void Engine::finalize() {
         p.M = std::min(Bm, 64); p.N = d; p.K = d; p.nseg = 1; p.seg[0] = layers_[0].wo.w;
         const int parts = gemm_skinny_ntile(p);
         if (nrm_fuse_ && Bm <= 64 && parts > 0 && parts % 4 == 0 && parts <= 64 && d % 128 == 0) {
-          nrm_parts_ = parts;
+          nrm_parts_ = d / 16;
           dec_xn16_ = (bf16_t*)dmalloc((size_t)Bm * d * 2);
-          nrm_part_ = fbuf((size_t)Bm * (d / 16));
+          nrm_part_ = fbuf((size_t)Bm * nrm_parts_);
           ws += (size_t)Bm * d * 2;
         }
         // TP: the all-reduce after O / down writes the next GEMM's split-norm operand itself
@@ -929,12 +929,12 @@ void Engine::layer_decode_gemm(int l, int B) {
   bf16_t* vc = kv_layer(v_cache_, l);
   // consumer side of the split RMSNorm: A = bf16(x * g) from the previous residual GEMM
   auto nrm_in = [&](GemmQArgs& g) {
-    g.A = dec_xn16_; g.nrm_in = nrm_part_; g.nrm_parts = d / 16; g.nrm_eps = cfg_.norm_eps;
+    g.A = dec_xn16_; g.nrm_in = nrm_part_; g.nrm_parts = nrm_parts_; g.nrm_eps = cfg_.norm_eps;
   };
   // producer side: residual add + bf16(x_new * g_next) + per-tile sums of squares
   auto nrm_out = [&](GemmQArgs& g, const float* g_next) {
     g.epi = GEPI_ACCUM_NORM; g.nrm_g = g_next; g.nrm_out16 = dec_xn16_; g.nrm_part = nrm_part_;
-    g.nrm_parts = d / 16;
+    g.nrm_parts = nrm_parts_;
   };
   // TP: the same contract, produced by the fused all-reduce (C1 / C2) into tpn_part_
   auto tpn_in = [&](GemmQArgs& g) {
@@ -1015,7 +1015,7 @@ void Engine::layer_decode_gemm(int l, int B) {
   if (fn) nrm_out(g, g_next);
   nrm_lm_ = (fn || tpn) && l + 1 == cfg_.n_layers;
   lm_nrm_in_ = tpn ? tpn_part_ : nrm_part_;
-  lm_nrm_parts_ = tpn ? tpn_parts_ : d / 16;
+  lm_nrm_parts_ = tpn ? tpn_parts_ : nrm_parts_;
   gemm(g);
   if (tp) tp_reduce(attn_, g_next);
 }

@@ -387,11 +387,15 @@ def test_small_batches_stay_on_the_gemv_without_the_k_shared_gemm(monkeypatch, B
 
 @pytest.mark.parametrize("recipe,rb,split", [("Q4_K_M", "0", "0"), ("Q4_K_M", "4", "1"),
                                              ("mistral_shape", "0", "1"), ("mistral_shape", "4", "0")])
-def test_batched_decode_split_rmsnorm_matches_explicit(model_files, monkeypatch, recipe, rb, split):
-    """AIOS_GEMM_NORM_FUSE: the residual GEMMs (O, down) emit bf16(x * g_next) plus per-tile row
-    sums of squares and the next GEMM scales its rows by the inverse RMS -- the explicit
-    normalisation launches' result to bf16 rounding, with the reduction tiles over 4..16 parts
-    (AIOS_SKINNY_RB) on both the split-K last-arriver and the one-slice epilogue (AIOS_SKINNY_S)."""
+@pytest.mark.parametrize("wk,ring", [("1", "1"), ("0", "1"), ("0", "0")])
+def test_batched_decode_split_rmsnorm_matches_explicit(model_files, monkeypatch, recipe, rb, split, wk, ring):
+    """AIOS_GEMM_NORM_FUSE: the residual GEMMs (O, down) emit bf16(x * g_next) plus row sums of squares
+    per 16 columns and the next GEMM scales its rows by the inverse RMS -- the explicit
+    normalisation launches' result to bf16 rounding, by the K-shared GEMM, the ring (Q6_K) and the skinny one, the last
+    with tiles of 4 and 8 parts (AIOS_SKINNY_RB) on both the split-K last-arriver and the one-slice
+    epilogue (AIOS_SKINNY_S)."""
+    monkeypatch.setenv("AIOS_GEMM_WK", wk)
+    monkeypatch.setenv("AIOS_GEMM_RING", ring)
     monkeypatch.setenv("AIOS_DECODE_GEMM_MIN_B", "2")
     monkeypatch.setenv("AIOS_SKINNY_RB", rb)
     if split == "1":
@@ -403,7 +407,7 @@ def test_batched_decode_split_rmsnorm_matches_explicit(model_files, monkeypatch,
     for fuse in ("0", "1"):
         monkeypatch.setenv("AIOS_GEMM_NORM_FUSE", fuse)
         eng, cfg = _load(path, max_slots=4, max_batch=4, act_q8=False)
-        want_parts = cfg.d_model // (16 * (4 if rb == "4" else 8)) if fuse == "1" else 0
+        want_parts = cfg.d_model // 16 if fuse == "1" else 0
         assert eng.norm_fused_parts == want_parts
         firsts = [int(np.argmax(eng.prefill(s, p, 0, True))) for s, p in enumerate(prompts)]
         eng.decode_loop_prepare(list(range(B)), firsts, [len(p) for p in prompts])
