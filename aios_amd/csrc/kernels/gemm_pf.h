@@ -934,7 +934,7 @@ __device__ __forceinline__ void pf4_body(const GemmQArgs& a, int m0, int n0, int
 }
 
 // K groups of a pf4 workgroup: two below 256 rows (at 256 one group's slots and accumulators take the CU).  Slices
-// lie on even K-steps then (the launcher keeps such tiles to K % 128 == 0).
+// lie on even K-steps then, so a K of an odd number of steps (bf16 only) runs in one group (pf4_launch).
 template <int BM>
 constexpr int pf4_kg() { return BM < 256 ? 2 : 1; }
 
@@ -1850,9 +1850,9 @@ void pf8_launch(const GemmQArgs& a, int S, hipStream_t st) {
   }
 }
 
-template <int QT0, int QT1, int BM, int WC, int EPI, int PROBE = 0>
-__global__ void __launch_bounds__(256 * pf4_kg<BM>()) gemm_pf4_kernel(GemmQArgs a) {
-  constexpr int BN = 4 * WC, KG = pf4_kg<BM>();
+template <int QT0, int QT1, int BM, int WC, int EPI, int PROBE = 0, int KG = pf4_kg<BM>()>
+__global__ void __launch_bounds__(256 * KG) gemm_pf4_kernel(GemmQArgs a) {
+  constexpr int BN = 4 * WC;
   const int nN = a.N / BN, nM = (a.M + BM - 1) / BM, total = nN * nM;
   const int L = xcd_remap(blockIdx.x, total);
   const int tn = L % nN, tm = L / nN;
@@ -1901,30 +1901,35 @@ __global__ void __launch_bounds__(256) gemm_pf4t_kernel(GemmQArgs a, int F) {
   else pf4_body<QT0, 128, WC, EPI>(a, m0, n0, seg, 0, kt1, 1);
 }
 
-template <int QT, int BM, int WC>
+template <int QT, int BM, int WC, int KG>
 constexpr int pf4_lds_one() {
   using L = Pf4Layout<QT, BM, WC>;
-  constexpr int KG = pf4_kg<BM>(), ring = KG * L::template slots<KG>() * L::SLOT, sum = KG == 2 ? BM * 4 * WC * 4 : 0;
+  constexpr int ring = KG * L::template slots<KG>() * L::SLOT, sum = KG == 2 ? BM * 4 * WC * 4 : 0;
   return ring > sum ? ring : sum;  // (the sum over the groups exchanges half of each)
 }
-template <int QT0, int QT1, int BM, int WC>
+template <int QT0, int QT1, int BM, int WC, int KG = pf4_kg<BM>()>
 constexpr int pf4_lds_bytes() {
-  return pf4_lds_one<QT0, BM, WC>() > pf4_lds_one<QT1, BM, WC>() ? pf4_lds_one<QT0, BM, WC>() : pf4_lds_one<QT1, BM, WC>();
+  return std::max(pf4_lds_one<QT0, BM, WC, KG>(), pf4_lds_one<QT1, BM, WC, KG>());
 }
 
-template <int QT0, int QT1, int BM, int WC>
+template <int QT0, int QT1, int BM, int WC, int KG = pf4_kg<BM>()>
 void pf4_launch(const GemmQArgs& a, int S, hipStream_t st) {
-  constexpr int lds = pf4_lds_bytes<QT0, QT1, BM, WC>();
+  if constexpr (QT0 == QT_BF16 && KG == 2 && (BM == 64 || BM == 128)) {
+    if (a.K % 128) return pf4_launch<QT0, QT1, BM, WC, 1>(a, S, st);
+  }
+  constexpr int lds = pf4_lds_bytes<QT0, QT1, BM, WC, KG>();
   static_assert(lds <= 160 * 1024, "LDS");
-  constexpr int KG = pf4_kg<BM>(), NT = 256 * KG;
-  if (S < 0) {  // stream-K (STORE / ACCUM only)
-    int grid = 0;
-    const int ipw = pf_sk_ipw(a, BM, 4 * WC, KG, grid);
-    if (a.epi == GEPI_STORE)
-      hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_STORE>), dim3(grid), dim3(NT), lds, st, a, ipw);
-    else
-      hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_ACCUM>), dim3(grid), dim3(NT), lds, st, a, ipw);
-    return;
+  constexpr int NT = 256 * KG;
+  if constexpr (KG == pf4_kg<BM>()) {  // (an odd number of K-steps: no stream-K, pf_sk_ok)
+    if (S < 0) {  // stream-K (STORE / ACCUM only)
+      int grid = 0;
+      const int ipw = pf_sk_ipw(a, BM, 4 * WC, KG, grid);
+      if (a.epi == GEPI_STORE)
+        hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_STORE>), dim3(grid), dim3(NT), lds, st, a, ipw);
+      else
+        hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_ACCUM>), dim3(grid), dim3(NT), lds, st, a, ipw);
+      return;
+    }
   }
   if constexpr (BM == 256) {
     const int F = pf_tail_full(a, 4 * WC, S);
@@ -1945,14 +1950,14 @@ void pf4_launch(const GemmQArgs& a, int S, hipStream_t st) {
   }
   const dim3 grid((a.N / (4 * WC)) * ((a.M + BM - 1) / BM), S), block(NT);
   switch (a.epi) {
-    case GEPI_STORE: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_STORE>), grid, block, lds, st, a); break;
-    case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_ACCUM>), grid, block, lds, st, a); break;
-    case GEPI_QKV: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_QKV>), grid, block, lds, st, a); break;
+    case GEPI_STORE: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_STORE, 0, KG>), grid, block, lds, st, a); break;
+    case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_ACCUM, 0, KG>), grid, block, lds, st, a); break;
+    case GEPI_QKV: hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_QKV, 0, KG>), grid, block, lds, st, a); break;
     case GEPI_STORE16:
-      if constexpr (QT0 == QT_BF16) hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_STORE16>), grid, block, lds, st, a);
+      if constexpr (QT0 == QT_BF16) hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_STORE16, 0, KG>), grid, block, lds, st, a);
       break;
     default:  // (one segment, so one format)
-      if constexpr (QT0 == QT1) hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_SWIGLU_BF16>), grid, block, lds, st, a);
+      if constexpr (QT0 == QT1) hipLaunchKernelGGL((gemm_pf4_kernel<QT0, QT1, BM, WC, GEPI_SWIGLU_BF16, 0, KG>), grid, block, lds, st, a);
       break;
   }
 }

@@ -1593,18 +1593,34 @@ def test_gemm_pf_two_k_groups(E, monkeypatch, tile, fmt, M, K, S):
         assert per_row < 1e-2, per_row
 
 
-def test_gemm_pf_odd_k_steps(E):
-    """bf16, K an odd number of 64s: a tile without K groups, also where only 128-column ones divide N"""
-    for N in (384, 512):
-        m, W = qmat(E, GGMLType.BF16, N, 192, seed=5, std=0.05)
-        x = torch.randn(100, 192, generator=torch.Generator().manual_seed(N))
-        A, C = x.to(torch.bfloat16).cuda(), torch.zeros(100, N, device="cuda")
-        bm, bn, _ = E.gemm_pf_plan([m], 100, E.GEPI_STORE, 0)
-        assert bm == 256 or bn == 256
-        E.gemm_q(A.data_ptr(), 192, [m], 100, C.data_ptr(), 0, N, E.GEPI_STORE, stream(), 0)
+@pytest.mark.parametrize("tile", ["", "64x128", "128x128", "256x128", "64x256", "256x256"])
+@pytest.mark.parametrize("K,S", [(192, 1), (960, 1), (960, 2), (960, 3)])
+@pytest.mark.parametrize("epi", ["store", "accum", "store16"])
+def test_gemm_pf_odd_k_steps(E, monkeypatch, tile, K, S, epi):
+    """bf16, K an odd number of 64s: the small 128-column tiles in one K group (uneven slices too), those without K groups
+    and the one planned, also where only 128-column ones divide N; the planned one is no larger than the rows ask for"""
+    if tile:
+        monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    if S > 1 and (not tile or epi == "store16"):
+        pytest.skip("split by hand only")
+    e = {"store": E.GEPI_STORE, "accum": E.GEPI_ACCUM, "store16": E.GEPI_STORE16}[epi]
+    for N, M in ((384, 33), (512, 100), (384, 129)):
+        m, W = qmat(E, GGMLType.BF16, N, K, seed=5, std=0.05)
+        bm, bn, s = E.gemm_pf_plan([m], M, e, S if S > 1 else 0)
+        if tile and (not bm or (S > 1 and s != S)):
+            continue
+        if tile:
+            assert [bm, bn] == [int(v) for v in tile.split("x")]
+        else:
+            assert bm <= 128
+        x = torch.randn(M, K, generator=torch.Generator().manual_seed(N)).to(torch.bfloat16)
+        A, C = x.cuda(), torch.ones(M, N, device="cuda", dtype=torch.bfloat16 if epi == "store16" else torch.float32)
+        E.gemm_q(A.data_ptr(), K, [m], M, 0 if epi == "store16" else C.data_ptr(), C.data_ptr() if epi == "store16" else 0, N, e,
+                 stream(), S if S > 1 else 0)
         torch.cuda.synchronize()
-        ref = x.double() @ W.double().T
-        assert float((C.cpu().double() - ref).norm() / ref.norm()) < 6e-3
+        ref = x.double() @ W.to(torch.bfloat16).double().T + (1.0 if epi == "accum" else 0.0)
+        err = (C.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)
+        assert err.max() < K * 2.0 ** -24 + (2.0 ** -8 if epi == "store16" else 0.0)
 
 
 def pf_plan_entry(E, N, K, M, epi, bm, bn, S, s1=0):
@@ -1613,7 +1629,7 @@ def pf_plan_entry(E, N, K, M, epi, bm, bn, S, s1=0):
     return [N, K, M, epi, int(GGMLType.BF16), int(GGMLType.BF16), 1, 0, 0, cus, bm, bn, S, s1]
 
 
-@pytest.mark.parametrize("K,N,tile", [(192, 640, (64, 128, 1)), (192, 896, (128, 128, 1)), (320, 640, (96, 128, 2)),
+@pytest.mark.parametrize("K,N,tile", [(192, 640, (96, 128, 1)), (192, 896, (160, 128, 1)), (320, 640, (96, 128, 2)),
                                       (320, 384, (160, 128, 1)), (128, 384, (64, 256, 1)), (128, 640, (64, 128, 3)),
                                       (192, 1152, (64, 128, -1)),
                                       (128, 896, (48, 128, 1)), (128, 1152, (64, 128, 0))])

@@ -34,12 +34,12 @@ HOT = [
     "aios::gemm_skinny_kernel<*",
     "aios::gemm_ring_kernel<*",
     "aios::gemm_wk_kernel<*",
-    "aios::gemm_pf8_kernel<*, [012], 0>*",
+    "aios::gemm_pf8_kernel<*, [0125], 0>*",
     "aios::gemm_pf8_kernel<*, *, 64, 3, 0>*",
     "aios::gemm_pf8_kernel<*, *, 128, 3, 0>*",
     "aios::gemm_pf8t_kernel<*",
     "aios::gemm_pf8sk_kernel<*",
-    "aios::gemm_pf4_kernel<*, [012], 0>*",
+    "aios::gemm_pf4_kernel<*, [0125], 0, *>*",
     "aios::gemm_pf4t_kernel<*",
     "aios::gemm_pf4sk_kernel<*",
     "aios::sample_kernel*",
