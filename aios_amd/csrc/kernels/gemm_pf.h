@@ -743,11 +743,11 @@ __device__ __forceinline__ void pf4_braw(const uint8_t* wbase, int cl, int h, Pf
   }
 }
 
-// KG = 2 (tiles below 256 rows): two groups of four waves, each with half of the slice's K-steps and slots of its
+// KG = 2 (pf4_groups): two groups of four waves, each with half of the slice's K-steps and slots of its
 // own, their accumulators added through LDS at the end.  One wave per SIMD runs a K-step's LDS reads, decode,
 // matrix instructions and DMA issue one after the other (64 x 128 tiles: 1900 cycles a step, of which 256 are
-// matrix instructions); the second wave fills its gaps.  Both groups have the same number of steps (pf4_kg).
-// Gate/up of 28672 x 4096 Q4_K: 64 rows 47 -> 35 us, 130 rows (one 160-row tile) 78 -> 57 us.
+// matrix instructions); the second wave fills its gaps.  Both groups have the same number of steps.
+// Gate/up of 28672 x 4096 Q4_K, 64 rows: 47 -> 35 us.
 template <int QT, int BM, int WC, int EPI, int PROBE = 0, int KG = 1>
 __device__ __forceinline__ void pf4_body(const GemmQArgs& a, int m0, int n0, int seg, int kt0, int kt1, int S) {
   using L = Pf4Layout<QT, BM, WC>;
@@ -933,10 +933,25 @@ __device__ __forceinline__ void pf4_body(const GemmQArgs& a, int m0, int n0, int
       for (int e = 0; e < 16; ++e) out(m0 + 32 * i + (e & 3) + 8 * (e >> 2) + 4 * h, n0 + wv * WC + 32 * c + r32, acc[i][c][e]);
 }
 
-// K groups of a pf4 workgroup: two below 256 rows (at 256 one group's slots and accumulators take the CU).  Slices
-// lie on even K-steps then, so a K of an odd number of steps (bf16 only) runs in one group (pf4_launch).
-template <int BM>
-constexpr int pf4_kg() { return BM < 256 ? 2 : 1; }
+// K groups of a pf4 workgroup of this launch.  Two where the launch leaves a CU no second workgroup, which fills the gaps as
+// well as a second group and has no sums to exchange; and where a group has enough K-steps to pay for them.  One from 160
+// rows up: the slots and accumulators take the CU.  us in one / two groups, by workgroups on 256 CUs:
+//   28672 x 4096 Q4_K SwiGLU, 64 rows (224) 43 / 37, 130 rows in 64 (672) 86 / 94, in 160 (224) 58 / 61, 600 in 128 (1120) 186 / 215
+//   4096 x 4096 Q4_K, 100 rows in 64, one slice (64) 40 / 29, four (256) 18.0 / 17.1, eight of 8 steps (512) 20.7 / 24.8
+//   2048 x 2048 Q6_K, 40 rows in 64, eight slices of 4 steps (128) 9.6 / 10.4
+// The formats whose decode is longer (Q6_K 4096 x 11008, 100 rows in 128, eight slices (256) 33.0 / 34.4) take CUs to
+// spare.  bf16, which has no decode to hide, only 64 rows and those: 4096 x 4096, 64 rows, one slice (32) 37 / 31,
+// 100 rows in four (256) 18.4 / 19.7; 128 rows, one slice (32) 42 / 49.  Stream-K, a workgroup on every CU: Q4_K with 16
+// steps each (4096 x 14336 Q4_K, 100 rows in 64: 36.6 / 31.2; bf16, 200 rows of 2048 x 8704 22.6 / 33.3, Q6_K 30.0 / 39.2).
+// Slices of two groups lie on even K-steps (K % 128 == 0).
+inline int pf4_groups(const GemmQArgs& a, int bm, int S) {
+  const int qt = a.seg[0].qtype;
+  if (bm >= 160 || a.K % 128 || (qt == QT_BF16 && bm != 64)) return 1;
+  const int cus = device_cu_count(), steps = a.K / 64;
+  const long tiles = (long)(a.N / 128) * ((a.M + bm - 1) / bm);
+  if (S < 0) return qt == QT_Q4_K && a.K % 256 == 0 && tiles * steps >= 16L * cus ? 2 : 1;
+  return tiles * S <= (qt == QT_Q4_K ? cus : cus * 7 / 8) && steps / S >= 8 ? 2 : 1;
+}
 
 // ==== pf8: 8 waves (two per SIMD) x 32 columns, 16x16x32 MFMA ======================================
 // The 8-wave 16x16x32 body ran the compute-only probe at 1.33 PF per busy CU against 1.16 for pf4's
@@ -1756,9 +1771,8 @@ __device__ __forceinline__ void pf_stream_k(const GemmQArgs& a, int BN, int ipw,
   }
 }
 
-template <int QT0, int QT1, int BM, int WC, int EPI>
-__global__ void __launch_bounds__(256 * pf4_kg<BM>()) gemm_pf4sk_kernel(GemmQArgs a, int ipw) {
-  constexpr int KG = pf4_kg<BM>();
+template <int QT0, int QT1, int BM, int WC, int EPI, int KG>
+__global__ void __launch_bounds__(256 * KG) gemm_pf4sk_kernel(GemmQArgs a, int ipw) {
   pf_stream_k<BM, EPI, KG>(a, 4 * WC, ipw, [&](int m0, int n0, int seg, int kt0, int kt1, int S) {
     if constexpr (QT0 != QT1) {
       if (seg == a.nseg - 1) {
@@ -1850,7 +1864,7 @@ void pf8_launch(const GemmQArgs& a, int S, hipStream_t st) {
   }
 }
 
-template <int QT0, int QT1, int BM, int WC, int EPI, int PROBE = 0, int KG = pf4_kg<BM>()>
+template <int QT0, int QT1, int BM, int WC, int EPI, int PROBE = 0, int KG = 1>
 __global__ void __launch_bounds__(256 * KG) gemm_pf4_kernel(GemmQArgs a) {
   constexpr int BN = 4 * WC;
   const int nN = a.N / BN, nM = (a.M + BM - 1) / BM, total = nN * nM;
@@ -1907,34 +1921,31 @@ constexpr int pf4_lds_one() {
   constexpr int ring = KG * L::template slots<KG>() * L::SLOT, sum = KG == 2 ? BM * 4 * WC * 4 : 0;
   return ring > sum ? ring : sum;  // (the sum over the groups exchanges half of each)
 }
-template <int QT0, int QT1, int BM, int WC, int KG = pf4_kg<BM>()>
+template <int QT0, int QT1, int BM, int WC, int KG>
 constexpr int pf4_lds_bytes() {
   return std::max(pf4_lds_one<QT0, BM, WC, KG>(), pf4_lds_one<QT1, BM, WC, KG>());
 }
 
-template <int QT0, int QT1, int BM, int WC, int KG = pf4_kg<BM>()>
+template <int QT0, int QT1, int BM, int WC, int KG>
 void pf4_launch(const GemmQArgs& a, int S, hipStream_t st) {
-  if constexpr (QT0 == QT_BF16 && KG == 2 && (BM == 64 || BM == 128)) {
-    if (a.K % 128) return pf4_launch<QT0, QT1, BM, WC, 1>(a, S, st);
-  }
   constexpr int lds = pf4_lds_bytes<QT0, QT1, BM, WC, KG>();
   static_assert(lds <= 160 * 1024, "LDS");
   constexpr int NT = 256 * KG;
-  if constexpr (KG == pf4_kg<BM>()) {  // (an odd number of K-steps: no stream-K, pf_sk_ok)
+  if constexpr (KG == 1 || QT0 == QT_Q4_K) {  // (pf4_groups)
     if (S < 0) {  // stream-K (STORE / ACCUM only)
       int grid = 0;
       const int ipw = pf_sk_ipw(a, BM, 4 * WC, KG, grid);
       if (a.epi == GEPI_STORE)
-        hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_STORE>), dim3(grid), dim3(NT), lds, st, a, ipw);
+        hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_STORE, KG>), dim3(grid), dim3(NT), lds, st, a, ipw);
       else
-        hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_ACCUM>), dim3(grid), dim3(NT), lds, st, a, ipw);
+        hipLaunchKernelGGL((gemm_pf4sk_kernel<QT0, QT1, BM, WC, GEPI_ACCUM, KG>), dim3(grid), dim3(NT), lds, st, a, ipw);
       return;
     }
   }
   if constexpr (BM == 256) {
     const int F = pf_tail_full(a, 4 * WC, S);
     if (F >= 0) {
-      constexpr int l128 = pf4_lds_bytes<QT0, QT1, 128, WC>();
+      constexpr int l128 = pf4_lds_bytes<QT0, QT1, 128, WC, 1>();
       constexpr int ldst = lds > l128 ? lds : l128;
       const int T = (a.N / (4 * WC)) * ((a.M + 255) / 256);
       const dim3 grid(F + 2 * (T - F)), block(256);
@@ -2026,10 +2037,16 @@ bool pf_launch_fmt(const GemmQArgs& a, int BM, int BN, int S, hipStream_t st) {
     pf8_launch<QT0, QT1, bm>(a, S, st); \
     return true;                        \
   }
-#define PF_GO4(bm)                          \
-  if (BM == bm && BN == 128) {              \
-    pf4_launch<QT0, QT1, bm, 32>(a, S, st); \
-    return true;                            \
+#define PF_GO4(bm)                                                \
+  if (BM == bm && BN == 128) {                                    \
+    if constexpr (bm < 160 && (QT0 != QT_BF16 || bm == 64)) {     \
+      if (pf4_groups(a, bm, S) == 2) {                            \
+        pf4_launch<QT0, QT1, bm, 32, 2>(a, S, st);                \
+        return true;                                              \
+      }                                                           \
+    }                                                             \
+    pf4_launch<QT0, QT1, bm, 32, 1>(a, S, st);                    \
+    return true;                                                  \
   }
   PF_GO8(256) PF_GO8(128) PF_GO8(64) PF_GO4(256) PF_GO4(160) PF_GO4(128) PF_GO4(96) PF_GO4(64)
 #undef PF_GO8

@@ -65,11 +65,8 @@ static double pf_model(const GemmQArgs& a, int bm, int bn, int S, bool bf) {
 
 // the tiles there are (gemm_pf.h pf_launch_fmt), largest first
 static const struct { int bm, bn; } PF_TILES[] = {{256, 256}, {256, 128}, {160, 128}, {128, 256}, {128, 128}, {96, 128}, {64, 256}, {64, 128}};
-static bool pf_tile_ok(const GemmQArgs& a, int bm, int bn) {
+static bool pf_tile_ok(const GemmQArgs& a, int bn) {
   if (a.N % bn) return false;
-  // (two K groups of equal length; of an odd number of K-steps, 64 and 128 rows run in one: 640 x 960 bf16 at 40 rows
-  // 5.8 us, in the 256-row tile 10.7)
-  if (bn == 128 && bm < 256 && a.K % 128 && bm != 64 && bm != 128) return false;
   for (int s = 0; s < a.nseg; ++s)
     if (a.seg_n0[s] % bn || a.seg[s].rows % bn) return false;
   return true;
@@ -114,17 +111,17 @@ static bool pf_no_split(const GemmQArgs& a) {
 // 88 / 67 us, 4096 x 4096 Q4_K 63 / 42, 4096 x 14336 Q4_K 121 / 107, Q6_K 133 / 124
 static bool pf_sk_ok(const GemmQArgs& a, int bm, int bn, bool bf) {
   if (pf_no_split(a) || (bn == 256 && !bf) || !pf_env("AIOS_GEMM_PF_SK", 1)) return false;
-  const int units = bn == 128 && bm < 256 && a.K % 128 == 0 ? a.K / 128 : a.K / 64;  // (odd: no)
+  const int units = a.K / (64 * (bn == 128 ? pf4_groups(a, bm, -1) : 1));
   const double tiles = (double)((a.M + bm - 1) / bm) * (a.N / bn);
   return units % 2 == 0 && units >= 4 && tiles < 2.0 * device_cu_count();
 }
 
 // whether the kernels take this tile and split for these args: candidates, modelled and stored plans alike (a stored one
-// may be another build's: pf_launch_fmt would run its tile with K cut as it does not cut it, or not at all)
+// may be another build's: pf_launch_fmt would run a slice of no K-steps, or a tile that does not divide N, or nothing)
 static bool pf_plan_ok(const GemmQArgs& a, const PfPlan& p, bool bf) {
   bool tile = false;
   for (const auto& t : PF_TILES) tile = tile || (t.bm == p.bm && t.bn == p.bn);
-  if (!tile || !pf_tile_ok(a, p.bm, p.bn)) return false;
+  if (!tile || !pf_tile_ok(a, p.bn)) return false;
   if (p.s < 0) return pf_sk_ok(a, p.bm, p.bn, bf);
   if (p.s == 0 || (p.s > 1 && (pf_no_split(a) || a.K / 64 / p.s < 2))) return false;
   return bf || p.bn != 256 || a.K / 256 / p.s >= 1;  // (pf8c slices whole 256-blocks)

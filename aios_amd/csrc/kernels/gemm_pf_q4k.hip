@@ -27,7 +27,7 @@ bool gemm_pf_probe(const GemmQArgs& a, int probe, hipStream_t st) {
     }
   }
   if (probe >= 200) {
-    constexpr int lds4 = pf4_lds_bytes<QT_Q4_K, QT_Q4_K, 256, 64>();
+    constexpr int lds4 = pf4_lds_bytes<QT_Q4_K, QT_Q4_K, 256, 64, 1>();
     const dim3 g4((a.N / 256) * ((a.M + 255) / 256)), b4(256);
     switch (probe - 200) {
 #define P4_GO(P) case P: hipLaunchKernelGGL((gemm_pf4_kernel<QT_Q4_K, QT_Q4_K, 256, 64, GEPI_STORE, P>), g4, b4, lds4, st, a); return true;

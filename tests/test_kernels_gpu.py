@@ -1570,10 +1570,11 @@ def test_gemm_pf_stream_k(E, monkeypatch, fmt, N, K, tile, epi):
 
 @pytest.mark.parametrize("tile", ["64x128", "96x128", "128x128", "160x128"])
 @pytest.mark.parametrize("fmt", list(PF_SEGS))
-@pytest.mark.parametrize("M,K,S", [(33, 256, 1), (96, 256, 2), (97, 1280, 1), (160, 1280, 3), (161, 512, 1), (300, 1280, -1)])
+@pytest.mark.parametrize("M,K,S", [(33, 256, 1), (96, 256, 2), (97, 1280, 1), (160, 1280, 3), (161, 512, 1), (300, 1280, -1),
+                                   (33, 512, 1), (160, 1536, 3), (2048, 4096, -1)])
 def test_gemm_pf_two_k_groups(E, monkeypatch, tile, fmt, M, K, S):
-    """128-column tiles below 256 rows: two groups of waves on half of the K-steps each, down to one step per group,
-    slices on even K-steps, rows just at and past a tile's edge"""
+    """128-column tiles below 256 rows: two groups of waves on half of the K-steps each from 8 steps a slice (16 a
+    workgroup in stream-K), one below; slices on even K-steps, rows just at and past a tile's edge"""
     monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
     if S < 0:
         monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", "-1")
@@ -1593,7 +1594,7 @@ def test_gemm_pf_two_k_groups(E, monkeypatch, tile, fmt, M, K, S):
         assert per_row < 1e-2, per_row
 
 
-@pytest.mark.parametrize("tile", ["", "64x128", "128x128", "256x128", "64x256", "256x256"])
+@pytest.mark.parametrize("tile", ["", "64x128", "96x128", "128x128", "160x128", "256x128", "64x256", "256x256"])
 @pytest.mark.parametrize("K,S", [(192, 1), (960, 1), (960, 2), (960, 3)])
 @pytest.mark.parametrize("epi", ["store", "accum", "store16"])
 def test_gemm_pf_odd_k_steps(E, monkeypatch, tile, K, S, epi):
@@ -1612,7 +1613,7 @@ def test_gemm_pf_odd_k_steps(E, monkeypatch, tile, K, S, epi):
         if tile:
             assert [bm, bn] == [int(v) for v in tile.split("x")]
         else:
-            assert bm <= 128
+            assert bm <= 160
         x = torch.randn(M, K, generator=torch.Generator().manual_seed(N)).to(torch.bfloat16)
         A, C = x.cuda(), torch.ones(M, N, device="cuda", dtype=torch.bfloat16 if epi == "store16" else torch.float32)
         E.gemm_q(A.data_ptr(), K, [m], M, 0 if epi == "store16" else C.data_ptr(), C.data_ptr() if epi == "store16" else 0, N, e,
@@ -1629,13 +1630,12 @@ def pf_plan_entry(E, N, K, M, epi, bm, bn, S, s1=0):
     return [N, K, M, epi, int(GGMLType.BF16), int(GGMLType.BF16), 1, 0, 0, cus, bm, bn, S, s1]
 
 
-@pytest.mark.parametrize("K,N,tile", [(192, 640, (96, 128, 1)), (192, 896, (160, 128, 1)), (320, 640, (96, 128, 2)),
-                                      (320, 384, (160, 128, 1)), (128, 384, (64, 256, 1)), (128, 640, (64, 128, 3)),
-                                      (192, 1152, (64, 128, -1)),
-                                      (128, 896, (48, 128, 1)), (128, 1152, (64, 128, 0))])
+@pytest.mark.parametrize("K,N,tile", [(192, 640, (96, 128, 2)), (192, 896, (128, 256, 1)), (128, 384, (64, 256, 1)),
+                                      (128, 640, (64, 128, 3)), (192, 1152, (64, 128, -1)), (128, 896, (48, 128, 1)),
+                                      (128, 1152, (64, 128, 0))])
 def test_gemm_pf_imported_plan_that_does_not_fit(E, K, N, tile):
-    """a stored plan is one of this build's tiles and cuts K as its kernel does, or the modelled one serves: two K groups
-    (K an odd number of 64s), a width that does not divide N, more slices than K-steps, stream-K of too few, no such tile"""
+    """a stored plan is one of this build's tiles and divides N and K as its kernel does, or the modelled one serves: a width
+    that does not divide N, more slices than K-steps, stream-K of too few, no such tile, no slices"""
     E.gemm_pf_import(pf_plan_entry(E, N, K, 128, E.GEPI_STORE, *tile) + pf_plan_entry(E, N, K, 128, E.GEPI_STORE, *tile, s1=1))
     m, W = qmat(E, GGMLType.BF16, N, K, seed=5, std=0.05)
     assert list(E.gemm_pf_plan([m], 100, E.GEPI_STORE, 0)) != list(tile)
@@ -1648,9 +1648,17 @@ def test_gemm_pf_imported_plan_that_does_not_fit(E, K, N, tile):
 
 
 def test_gemm_pf_imported_plan_that_fits(E):
-    m, W = qmat(E, GGMLType.BF16, 1408, 256, seed=5, std=0.05)
-    E.gemm_pf_import(pf_plan_entry(E, 1408, 256, 128, E.GEPI_STORE, 64, 128, 2))
-    assert list(E.gemm_pf_plan([m], 100, E.GEPI_STORE, 0)) == [64, 128, 2]
+    """... and is run otherwise, whatever K groups its tile then has (K an odd number of 64s: one)"""
+    for N, K, tile in ((1408, 256, (64, 128, 2)), (1664, 192, (64, 128, 1)), (1664, 320, (128, 128, 1)), (1920, 192, (160, 128, 1))):
+        m, W = qmat(E, GGMLType.BF16, N, K, seed=5, std=0.05)
+        E.gemm_pf_import(pf_plan_entry(E, N, K, 128, E.GEPI_STORE, *tile))
+        assert list(E.gemm_pf_plan([m], 100, E.GEPI_STORE, 0)) == list(tile)
+        x = torch.randn(100, K, generator=torch.Generator().manual_seed(N)).to(torch.bfloat16)
+        A, C = x.cuda(), torch.zeros(100, N, device="cuda")
+        E.gemm_q(A.data_ptr(), K, [m], 100, C.data_ptr(), 0, N, E.GEPI_STORE, stream(), 0)
+        torch.cuda.synchronize()
+        ref = x.double() @ W.to(torch.bfloat16).double().T
+        assert float((C.cpu().double() - ref).norm() / ref.norm()) < K * 2.0 ** -24
 
 
 @pytest.mark.parametrize("tile", ["256x256", "128x256", "64x128"])
