@@ -358,6 +358,15 @@ static bool wk_route(const GemmQArgs& a, WkRoute& r) {
   //   3584 x 18944 22.7 / 22.0, 23.4 / 23.1    8192 x 28672 59.1 / 55.1, 60.2 / 57.3    4096 x 11008 16.5 / 16.5, 17.0 / 16.9
   //   2048 x 8704 11.5 / 12.4, 11.8 / 13.2
   if (qt0 == QT_Q6_K && r.S > 2 && r.mt == 1 && a.N % 128 == 0 && a.N / 128 * 8 * 4 >= 3 * device_cu_count()) return false;
+  // bf16, whose stream is all there is to it: the skinny GEMM is the faster one where a tile has little k for eight waves to
+  // share, where slabs cost (long K; two 16-row groups and a wide output), and where its tiles in eight slices are one
+  // round.  us here / skinny: 128256 x 512, 16 rows 45 / 37, 32000 x 64 9.8 / 5.4, 32000 x 512 13.3 / 15.9;
+  // 4096 x 14336 34 / 30, 2048 x 14336 18 / 24; 128256 x 4096, 32 rows 256 / 226, 16 rows 214 / 215, 32000 x 4096 equal;
+  // 4096 x 8192, 32 rows 25 / 22, 8192 x 8192 37 / 40
+  const int round = a.N / 128 * 8, cus = device_cu_count();
+  if (bf && (a.N > 125L * a.K || (a.K > 12288 && a.N >= 4096) ||
+             (r.mt == 2 && ((r.S >= 2 && a.N >= 65536) || (r.S >= 4 && 4 * round >= 3 * cus && round <= cus)))))
+    return false;
   // (three segments' four planes and the cache's arguments: more scalars than there are)
   if (a.epi == GEPI_QKV && qt0 == QT_Q6_K && r.ns * r.mt == 4) return false;
   r.G = std::min(a.N / 16, std::max(1, device_cu_count() / r.S));

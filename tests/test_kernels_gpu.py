@@ -1175,6 +1175,22 @@ def test_gemm_wk_leaves_q6k_down_to_the_ring(E):
     assert E.gemm_wk_serves([mats["Q4_K", edge]], 17, E.GEPI_QKV)
 
 
+def test_gemm_wk_leaves_some_bf16_to_skinny():
+    """wide outputs of little k, long K, and one round of skinny tiles where 17 rows ask for four slices: both sides of each"""
+    from aios_amd.runtime import native
+
+    E = native.require()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+
+    def serves(N, K, M):
+        return E.gemm_wk_serves([E.QMatrix(int(GGMLType.BF16), N, K, np.zeros(N * K, np.int16))], M, E.GEPI_ACCUM)
+
+    assert serves(8000, 64, 16) and not serves(8064, 64, 16)
+    assert serves(4096, 12288, 16) and not serves(4096, 12352, 16) and serves(2048, 12352, 16)
+    one = cus // 8 * 128  # (8 slices of these tiles: the CUs once)
+    assert serves(one, 8192, 16) and not serves(one, 8192, 17) and serves(2 * one, 8192, 17) and serves(one, 4096, 17)
+
+
 @pytest.mark.parametrize("kernel,t", [("wk", "Q4_K"), ("wk", "Q6_K"), ("wk", "BF16"), ("ring", "Q6_K"), ("skinny", "Q4_K"),
                                       ("skinny", "Q6_K"), ("skinny", "BF16")])
 @pytest.mark.parametrize("M", [2, 17, 32])
