@@ -23,11 +23,24 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(HD == 
   attn_role<HD, G, F8>(a, s, blockIdx.x);
 }
 
+// a workgroup or more per query head for every context (attn_lanes_only)
+template <int HD, bool F8>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) attn_lanes_kernel(AttnDecodeArgs a, AttnSplit s) {
+  kernarg_warm<sizeof(AttnDecodeArgs) + sizeof(AttnSplit)>();
+  attn_lanes<HD, F8, true>(a, blockIdx.x / s.p, blockIdx.x / s.p, blockIdx.x % s.p, s.p);
+}
+
 template <int HD, bool F8>
 static void launch_hd(const AttnDecodeArgs& a, int G, hipStream_t st) {
   AttnSplit sp;
   const dim3 grid(attn_plan(a, G, sp), 1, a.B), block(512);
   constexpr int lds = at_lds_bytes<HD>();
+  if constexpr (HD == 128) {
+    if (attn_lanes_only(a, G)) {
+      hipLaunchKernelGGL((attn_lanes_kernel<HD, F8>), dim3(a.n_heads * sp.p, 1, a.B), block, AT_NW * HD * 4, st, a, sp);
+      return;
+    }
+  }
   switch (G) {
     case 1: hipLaunchKernelGGL((attn_decode_kernel<HD, 1, F8>), grid, block, lds, st, a, sp); break;
     case 2: hipLaunchKernelGGL((attn_decode_kernel<HD, 2, F8>), grid, block, lds, st, a, sp); break;

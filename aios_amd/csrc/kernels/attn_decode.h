@@ -119,6 +119,7 @@ __device__ __forceinline__ gf32x2 fp8x2_f32x2(uint32_t w) {
 }
 
 constexpr int AT_NW = 8;    // waves per workgroup
+constexpr int ATTN_SPLIT_LEN = 512;  // keys of a short context
 // descriptor of n raw bytes at p (both uniform over the wave)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const uint8_t* p, int n) {
   const uint64_t u = (uint64_t)p;
@@ -138,6 +139,162 @@ template <int HD>
 constexpr int at_vrow() { return HD * 2 + 32; }
 template <int HD>
 constexpr int at_lds_bytes() { return AT_NW * AT_TK * at_vrow<HD>(); }
+
+// A workgroup's last part: the 8 waves' states of its G heads (s_o unnormalised, s_m, s_l; ordered before) merged, and the
+// output written (P == 1) or the partial published and, by the last of the P workgroups to arrive, all of them combined.
+template <int HD, int G, bool F8, typename Stamp>
+__device__ __forceinline__ void attn_meet(const AttnDecodeArgs& a, int h0, int sp, int nact, int tid, int wave, float (*s_o)[G][HD],
+                                          float (*s_m)[G], float (*s_l)[G], Stamp stamp) {
+  constexpr int NW = AT_NW, NT = NW * 64;
+  __shared__ int s_last;
+  const int b = blockIdx.z, mlane = tid & 63;
+  const float vs = F8 ? a.kv_scale_v : 1.f;
+  for (int idx = tid; idx < G * HD; idx += NT) {
+    const int g = idx / HD, d = idx - g * HD;
+    float M = s_m[0][g];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, s_m[w][g]);
+    float L = 0.f, acc = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float sw = fast_exp2(s_m[w][g] - M);
+      L += sw * s_l[w][g];
+      acc += sw * s_o[w][g][d];
+    }
+    const int h = h0 + g;
+    if (F8) acc *= vs;
+    if (nact == 1) {
+      if (a.out16) a.out16[((size_t)b * a.n_heads + h) * HD + d] = f32_to_bf16(acc / L);
+      else if (a.out_wt) st_wt(a.out + ((size_t)b * a.n_heads + h) * HD + d, acc / L);
+      else a.out[((size_t)b * a.n_heads + h) * HD + d] = acc / L;
+    } else {
+      st_wt(a.o_part + (((size_t)b * a.n_heads + h) * a.n_chunks + sp) * HD + d, acc);
+      if (d == 0) {
+        float* ml = a.ml + (((size_t)b * a.n_heads + h) * a.n_chunks + sp) * 2;
+        st_wt(ml, M);
+        st_wt(ml + 1, L);
+      }
+    }
+  }
+  if (nact == 1) {
+    stamp(6);
+    return;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains its sc1 stores
+  __syncthreads();
+  int* cnt = a.counters + (size_t)b * a.n_heads + h0;
+  if (tid == 0) {
+    const int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = (t == nact - 1);
+  }
+  __syncthreads();
+  stamp(4);
+  if (!s_last) return;
+  // ---- last arriver.  (1) one thread per (head, partial) loads that partial's (m, l);
+  //      (measured: one batch of (m, l) + o loads per output thread -- one round trip but 2x the
+  //      loads, the (m, l) ones redundant across a head's 128 threads -- was 1.3 us SLOWER at 1000
+  //      keys, 10.09 vs 8.73 us; hoisting the block-table loads above the seq_len test, or
+  //      issuing pass 0's K/V before seq_len is read, did not help either: 4.32-4.40 vs 4.18 us
+  //      at 153 keys, tools/attn_probe.py -- the short-context launch is the 1.7 us launch chain
+  //      plus one K/V round trip plus the merge, not the table lookups)
+  //      (2) wave g reduces head g's max M and total L and turns them into normalised weights
+  //      w_p = exp2(m_p - M) / L in LDS; (3) every output sums w_p * o_p with 16 loads in flight.
+  //      Two memory round trips for up to 64 partials (was one per 8 partials).
+  __shared__ float s_pm[G][64], s_pl[G][64];
+  // one memory round trip (round 4): when every output has one thread and the partials fit one
+  // register batch, each thread issues its output's nact partial loads TOGETHER with the (m, l)
+  // sweep and folds them after the weights are ready -- same order of sums as the two-trip path
+  auto one_trip = [&](auto ob) __attribute__((always_inline)) {
+    constexpr int OB = decltype(ob)::value;
+    const int idx = tid;
+    const bool act = idx < G * HD;
+    const int g = act ? idx / HD : 0, d = act ? idx - g * HD : 0;
+    const float* op = a.o_part + ((size_t)b * a.n_heads + h0 + g) * a.n_chunks * HD + d;
+    float ov[OB];
+#pragma unroll
+    for (int j = 0; j < OB; ++j) ov[j] = ld_wt(op + (size_t)min(j, nact - 1) * HD);  // clamped: in bounds
+    for (int i = tid; i < G * nact; i += NT) {
+      const int gg = i / nact, p = i - gg * nact;
+      const float* mlp = a.ml + (((size_t)b * a.n_heads + h0 + gg) * a.n_chunks + p) * 2;
+      s_pm[gg][p] = ld_wt(mlp);
+      s_pl[gg][p] = ld_wt(mlp + 1);
+    }
+    __syncthreads();
+    if (wave < G) {
+      const float mv = mlane < nact ? s_pm[wave][mlane] : kNeg;
+      const float lv = mlane < nact ? s_pl[wave][mlane] : 0.f;
+      float M = mv;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+      const float e = fast_exp2(mv - M);
+      float L = e * lv;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
+      if (mlane < nact) s_pm[wave][mlane] = e / L;
+    }
+    __syncthreads();
+    stamp(5);
+    if (act) {
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < OB; ++j)
+        if (j < nact) acc = fmaf(s_pm[g][j], ov[j], acc);
+      const int h = h0 + g;
+      if (a.out16) a.out16[((size_t)b * a.n_heads + h) * HD + d] = f32_to_bf16(acc);
+      else if (a.out_wt) st_wt(a.out + ((size_t)b * a.n_heads + h) * HD + d, acc);
+      else a.out[((size_t)b * a.n_heads + h) * HD + d] = acc;
+    }
+  };
+  if (G * HD <= NT && nact <= 32 && a.combine_trips != 2) {
+    if (nact <= 8) one_trip(std::integral_constant<int, 8>{});
+    else if (nact <= 16) one_trip(std::integral_constant<int, 16>{});
+    else one_trip(std::integral_constant<int, 32>{});
+    if (tid == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
+    stamp(6);
+    return;
+  }
+  for (int i = tid; i < G * nact; i += NT) {
+    const int g = i / nact, p = i - g * nact;
+    const float* mlp = a.ml + (((size_t)b * a.n_heads + h0 + g) * a.n_chunks + p) * 2;
+    s_pm[g][p] = ld_wt(mlp);
+    s_pl[g][p] = ld_wt(mlp + 1);
+  }
+  __syncthreads();
+  if (wave < G) {
+    const int g = wave;
+    const float mv = mlane < nact ? s_pm[g][mlane] : kNeg;
+    const float lv = mlane < nact ? s_pl[g][mlane] : 0.f;
+    float M = mv;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+    const float e = fast_exp2(mv - M);
+    float L = e * lv;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
+    if (mlane < nact) s_pm[g][mlane] = e / L;
+  }
+  __syncthreads();
+  stamp(5);
+  for (int idx = tid; idx < G * HD; idx += NT) {
+    const int g = idx / HD, d = idx - g * HD;
+    const int h = h0 + g;
+    const float* op = a.o_part + ((size_t)b * a.n_heads + h) * a.n_chunks * HD + d;
+    float acc = 0.f;
+    for (int c = 0; c < nact; c += 16) {
+      float ov[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) ov[j] = ld_wt(op + (size_t)min(c + j, nact - 1) * HD);
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (c + j < nact) acc = fmaf(s_pm[g][c + j], ov[j], acc);
+    }
+    if (a.out16) a.out16[((size_t)b * a.n_heads + h) * HD + d] = f32_to_bf16(acc);
+    else if (a.out_wt) st_wt(a.out + ((size_t)b * a.n_heads + h) * HD + d, acc);
+      else a.out[((size_t)b * a.n_heads + h) * HD + d] = acc;
+  }
+  if (tid == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
+  stamp(6);
+}
 
 // One workgroup's share: the G query heads of KV head kvh over the 32-key tiles of P workgroups x 8 waves,
 // dealt wave by wave (tile t to wave t mod 8 P: 32 keys is also the granularity of the balance).
@@ -170,14 +327,13 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   constexpr int VPR = HD / EL;              // 16-B pieces of a V row
   constexpr int DT = HD / 16;               // O^T tiles
   constexpr int VROW = at_vrow<HD>();
-  constexpr int NW = AT_NW, NT = NW * 64;
+  constexpr int NW = AT_NW;
   extern __shared__ __attribute__((aligned(16))) uint8_t at_smem[];
   float (*s_o)[G][HD] = (float (*)[G][HD])at_smem;  // (the merge; after the V tiles)
   static_assert(sizeof(float) * NW * G * HD <= at_lds_bytes<HD>(), "merge buffer");
   __shared__ float s_m[NW][G], s_l[NW][G];
-  __shared__ int s_last;
 
-  const int b = blockIdx.z, h0 = kvh * G, ci = h0;
+  const int b = blockIdx.z, h0 = kvh * G;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 15, q4 = lane >> 4;
   // probe stamps (a.ts; probe builds only, -DAIOS_ATTN_PROBES=1): 0 entry, 1 seq_len known, 2 first tile
@@ -410,166 +566,24 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
       s_l[wave][mc] = l;
     }
   }
-  const float vs = F8 ? a.kv_scale_v : 1.f;
   __syncthreads();
   stamp(3);
-  const int nact = P;  // workgroups that arrive
-  for (int idx = tid; idx < G * HD; idx += NT) {
-    const int g = idx / HD, d = idx - g * HD;
-    float M = s_m[0][g];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) M = fmaxf(M, s_m[w][g]);
-    float L = 0.f, acc = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float sw = fast_exp2(s_m[w][g] - M);
-      L += sw * s_l[w][g];
-      acc += sw * s_o[w][g][d];
-    }
-    const int h = h0 + g;
-    if (F8) acc *= vs;
-    if (nact == 1) {
-      if (a.out16) a.out16[((size_t)b * a.n_heads + h) * HD + d] = f32_to_bf16(acc / L);
-      else if (a.out_wt) st_wt(a.out + ((size_t)b * a.n_heads + h) * HD + d, acc / L);
-      else a.out[((size_t)b * a.n_heads + h) * HD + d] = acc / L;
-    } else {
-      st_wt(a.o_part + (((size_t)b * a.n_heads + h) * a.n_chunks + sp) * HD + d, acc);
-      if (d == 0) {
-        float* ml = a.ml + (((size_t)b * a.n_heads + h) * a.n_chunks + sp) * 2;
-        st_wt(ml, M);
-        st_wt(ml + 1, L);
-      }
-    }
-  }
-  if (nact == 1) {
-    stamp(6);
-    return;
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains its sc1 stores
-  __syncthreads();
-  int* cnt = a.counters + (size_t)b * a.n_heads + ci;
-  if (tid == 0) {
-    const int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = (t == nact - 1);
-  }
-  __syncthreads();
-  stamp(4);
-  if (!s_last) return;
-  // ---- last arriver.  (1) one thread per (head, partial) loads that partial's (m, l);
-  //      (measured: one batch of (m, l) + o loads per output thread -- one round trip but 2x the
-  //      loads, the (m, l) ones redundant across a head's 128 threads -- was 1.3 us SLOWER at 1000
-  //      keys, 10.09 vs 8.73 us; hoisting the block-table loads above the seq_len test, or
-  //      issuing pass 0's K/V before seq_len is read, did not help either: 4.32-4.40 vs 4.18 us
-  //      at 153 keys, tools/attn_probe.py -- the short-context launch is the 1.7 us launch chain
-  //      plus one K/V round trip plus the merge, not the table lookups)
-  //      (2) wave g reduces head g's max M and total L and turns them into normalised weights
-  //      w_p = exp2(m_p - M) / L in LDS; (3) every output sums w_p * o_p with 16 loads in flight.
-  //      Two memory round trips for up to 64 partials (was one per 8 partials).
-  __shared__ float s_pm[G][64], s_pl[G][64];
-  // one memory round trip (round 4): when every output has one thread and the partials fit one
-  // register batch, each thread issues its output's nact partial loads TOGETHER with the (m, l)
-  // sweep and folds them after the weights are ready -- same order of sums as the two-trip path
-  auto one_trip = [&](auto ob) __attribute__((always_inline)) {
-    constexpr int OB = decltype(ob)::value;
-    const int idx = tid;
-    const bool act = idx < G * HD;
-    const int g = act ? idx / HD : 0, d = act ? idx - g * HD : 0;
-    const float* op = a.o_part + ((size_t)b * a.n_heads + h0 + g) * a.n_chunks * HD + d;
-    float ov[OB];
-#pragma unroll
-    for (int j = 0; j < OB; ++j) ov[j] = ld_wt(op + (size_t)min(j, nact - 1) * HD);  // clamped: in bounds
-    for (int i = tid; i < G * nact; i += NT) {
-      const int gg = i / nact, p = i - gg * nact;
-      const float* mlp = a.ml + (((size_t)b * a.n_heads + h0 + gg) * a.n_chunks + p) * 2;
-      s_pm[gg][p] = ld_wt(mlp);
-      s_pl[gg][p] = ld_wt(mlp + 1);
-    }
-    __syncthreads();
-    if (wave < G) {
-      const float mv = mlane < nact ? s_pm[wave][mlane] : kNeg;
-      const float lv = mlane < nact ? s_pl[wave][mlane] : 0.f;
-      float M = mv;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
-      const float e = fast_exp2(mv - M);
-      float L = e * lv;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
-      if (mlane < nact) s_pm[wave][mlane] = e / L;
-    }
-    __syncthreads();
-    stamp(5);
-    if (act) {
-      float acc = 0.f;
-#pragma unroll
-      for (int j = 0; j < OB; ++j)
-        if (j < nact) acc = fmaf(s_pm[g][j], ov[j], acc);
-      const int h = h0 + g;
-      if (a.out16) a.out16[((size_t)b * a.n_heads + h) * HD + d] = f32_to_bf16(acc);
-      else if (a.out_wt) st_wt(a.out + ((size_t)b * a.n_heads + h) * HD + d, acc);
-      else a.out[((size_t)b * a.n_heads + h) * HD + d] = acc;
-    }
-  };
-  if (G * HD <= NT && nact <= 32 && a.combine_trips != 2) {
-    if (nact <= 8) one_trip(std::integral_constant<int, 8>{});
-    else if (nact <= 16) one_trip(std::integral_constant<int, 16>{});
-    else one_trip(std::integral_constant<int, 32>{});
-    if (tid == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
-    stamp(6);
-    return;
-  }
-  for (int i = tid; i < G * nact; i += NT) {
-    const int g = i / nact, p = i - g * nact;
-    const float* mlp = a.ml + (((size_t)b * a.n_heads + h0 + g) * a.n_chunks + p) * 2;
-    s_pm[g][p] = ld_wt(mlp);
-    s_pl[g][p] = ld_wt(mlp + 1);
-  }
-  __syncthreads();
-  if (wave < G) {
-    const int g = wave;
-    const float mv = mlane < nact ? s_pm[g][mlane] : kNeg;
-    const float lv = mlane < nact ? s_pl[g][mlane] : 0.f;
-    float M = mv;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
-    const float e = fast_exp2(mv - M);
-    float L = e * lv;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
-    if (mlane < nact) s_pm[g][mlane] = e / L;
-  }
-  __syncthreads();
-  stamp(5);
-  for (int idx = tid; idx < G * HD; idx += NT) {
-    const int g = idx / HD, d = idx - g * HD;
-    const int h = h0 + g;
-    const float* op = a.o_part + ((size_t)b * a.n_heads + h) * a.n_chunks * HD + d;
-    float acc = 0.f;
-    for (int c = 0; c < nact; c += 16) {
-      float ov[16];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) ov[j] = ld_wt(op + (size_t)min(c + j, nact - 1) * HD);
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        if (c + j < nact) acc = fmaf(s_pm[g][c + j], ov[j], acc);
-    }
-    if (a.out16) a.out16[((size_t)b * a.n_heads + h) * HD + d] = f32_to_bf16(acc);
-    else if (a.out_wt) st_wt(a.out + ((size_t)b * a.n_heads + h) * HD + d, acc);
-      else a.out[((size_t)b * a.n_heads + h) * HD + d] = acc;
-  }
-  if (tid == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
-  stamp(6);
+  attn_meet<HD, G, F8>(a, h0, sp, P, tid, wave, s_o, s_m, s_l, stamp);
 }
 
-// Contexts up to ATTN_SPLIT_LEN keys of a launch that leaves CUs idle: a workgroup per QUERY head walks all (<= 4)
-// 128-key passes, without a combine.  Its G workgroups per KV head read the same K and V (from L2 after the first,
-// see the roles below), so a launch this short is one memory round trip of 64 KB on each of n_heads CUs and little
-// else; attn_core's one workgroup per KV head then waits for a longer chain: 130 keys, 32 / 8 heads of 128: 5.2 us
+// A workgroup per QUERY head, P of them to a head's 128-key passes in turn.  Two uses.
+// Contexts up to ATTN_SPLIT_LEN keys of a launch that leaves CUs idle (P = 1): one workgroup walks all (<= 4) passes,
+// without a combine.  The G workgroups of a KV head read the same K and V (from L2 after the first, see the roles
+// below), so a launch this short is one memory round trip of 64 KB on each of n_heads CUs and little else; attn_core's
+// one workgroup per KV head then waits for a longer chain: 130 keys, 32 / 8 heads of 128: 5.2 us
 // here, 7.5 us there (4.0 and 4.9 us for 32 / 4 heads of 64); 500 keys of three rows: equal.
+// One head of 128 per KV head, every context (attn_lanes_only): attn_core's matrix columns are 4 heads wide, and of its
+// workgroups one fits a CU, of these two.
 // VALU: q . k on v_dot2_f32_bf16 (q rounded to bf16 pairs), P . V in fp32.  Every lane loads 16 B (fp8 at head_dim 64:
 // 8 B) of a key; two passes in flight.
-template <int HD, bool F8 = false>
-__device__ __forceinline__ void attn_short(const AttnDecodeArgs& a, int kvh, int h) {
+// (LONG: the second use; the first is P = 1)
+template <int HD, bool F8, bool LONG>
+__device__ __forceinline__ void attn_lanes(const AttnDecodeArgs& a, int kvh, int h, int sp, int P_max) {
   constexpr int DPL = (F8 && HD == 128) ? 16 : 8;  // dims per lane
   using KVT = typename std::conditional<F8 && DPL == 8, uint2, uint4>::type;
   constexpr int ES = F8 ? 1 : 2;  // bytes per cached element
@@ -581,8 +595,8 @@ __device__ __forceinline__ void attn_short(const AttnDecodeArgs& a, int kvh, int
   constexpr int KPW = CH / NW;         // keys per wave per pass
   constexpr int STEPS = KPW / KPS;     // loads per lane per pass (each of K and V)
   extern __shared__ __attribute__((aligned(16))) uint8_t at_smem[];
-  float (*s_o)[HD] = (float (*)[HD])at_smem;
-  __shared__ float s_m[NW], s_l[NW];
+  float (*s_o)[1][HD] = (float (*)[1][HD])at_smem;
+  __shared__ float s_m[NW][1], s_l[NW][1];
 
   const int b = blockIdx.z;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -597,9 +611,21 @@ __device__ __forceinline__ void attn_short(const AttnDecodeArgs& a, int kvh, int
   const uint8_t* vc = (const uint8_t*)a.v_cache + ((size_t)kvh * KV_BLOCK * HD + (size_t)koff * HD + dsl * DPL) * ES;
   const int len = a.seq_len[b];
   const int nchunk = (len + CH - 1) / CH;
+  const int P = !LONG || nchunk <= 2 ? 1 : min(nchunk, P_max);  // (two passes are in flight at once)
+  if (LONG && sp >= P) return;  // (uniform)
 
   KVT kA[STEPS], vA[STEPS], kB[STEPS], vB[STEPS];
-  auto ld = [&](const uint8_t* p) __attribute__((always_inline)) { return *(const KVT*)p; };
+  auto ld = [&](const uint8_t* p) __attribute__((always_inline)) {
+    if constexpr (LONG) {  // (read once per launch)
+      typedef uint32_t vec __attribute__((ext_vector_type(sizeof(KVT) / 4)));
+      const vec v = __builtin_nontemporal_load((const vec*)p);
+      KVT r;
+      __builtin_memcpy(&r, &v, sizeof(r));
+      return r;
+    } else {
+      return *(const KVT*)p;
+    }
+  };
   auto issue = [&](KVT (&kr)[STEPS], KVT (&vr)[STEPS], int c) __attribute__((always_inline)) {
     const size_t base = (size_t)(btr ? btr[c] : slot * maxb + c) * blk_stride * ES;  // (bytes)
     if ((c + 1) * CH > len) {
@@ -622,8 +648,8 @@ __device__ __forceinline__ void attn_short(const AttnDecodeArgs& a, int kvh, int
       for (int s = 0; s < STEPS; ++s) vr[s] = ld(vc + base + (size_t)s * KPS * HD * ES);
     }
   };
-  issue(kA, vA, 0);
-  if (1 < nchunk) issue(kB, vB, 1);
+  issue(kA, vA, sp);
+  if (sp + P < nchunk) issue(kB, vB, sp + P);
   const float qs = a.scale * kLog2e * (F8 ? a.kv_scale_k : 1.f);  // scores in the log2 domain: exp2 below
   uint32_t q2[NP];                 // q * scale as bf16 pairs
   {
@@ -699,12 +725,12 @@ __device__ __forceinline__ void attn_short(const AttnDecodeArgs& a, int kvh, int
       for (int i = 0; i < NP; ++i) o[i] = __builtin_elementwise_fma(pp, vf[i], o[i]);
     }
   };
-  for (int c = 0; c < nchunk; c += 2) {
+  for (int c = sp; c < nchunk; c += 2 * P) {
     pass(kA, vA, c);
-    if (c + 2 < nchunk) issue(kA, vA, c + 2);
-    if (c + 1 < nchunk) {
-      pass(kB, vB, c + 1);
-      if (c + 3 < nchunk) issue(kB, vB, c + 3);
+    if (c + 2 * P < nchunk) issue(kA, vA, c + 2 * P);
+    if (c + P < nchunk) {
+      pass(kB, vB, c + P);
+      if (c + 3 * P < nchunk) issue(kB, vB, c + 3 * P);
     }
   }
   // ---- merge the key groups of a wave (their (m, l, o) rescaled to the wave's max), then the 8 waves in LDS
@@ -717,26 +743,30 @@ __device__ __forceinline__ void attn_short(const AttnDecodeArgs& a, int kvh, int
     of[2 * i + 1] = keys_sum<LPK>(o[i].y * w);
   }
   if (ksub == 0) {
-    float4* dst = (float4*)&s_o[wave][dsl * DPL];
+    float4* dst = (float4*)&s_o[wave][0][dsl * DPL];
 #pragma unroll
     for (int j = 0; j < DPL / 4; ++j) dst[j] = make_float4(of[4 * j], of[4 * j + 1], of[4 * j + 2], of[4 * j + 3]);
   }
   if (lane == 0) {
-    s_m[wave] = M;
-    s_l[wave] = l;
+    s_m[wave][0] = M;
+    s_l[wave][0] = l;
   }
   __syncthreads();
+  if constexpr (LONG) {
+    attn_meet<HD, 1, F8>(a, h, sp, P, threadIdx.x, wave, s_o, s_m, s_l, [](int) {});
+    return;
+  }
   const int d = threadIdx.x;
   if (d >= HD) return;
-  float W = s_m[0];
+  float W = s_m[0][0];
 #pragma unroll
-  for (int v = 1; v < NW; ++v) W = fmaxf(W, s_m[v]);
+  for (int v = 1; v < NW; ++v) W = fmaxf(W, s_m[v][0]);
   float L = 0.f, acc = 0.f;
 #pragma unroll
   for (int v = 0; v < NW; ++v) {
-    const float sw = fast_exp2(s_m[v] - W);
-    L += sw * s_l[v];
-    acc += sw * s_o[v][d];
+    const float sw = fast_exp2(s_m[v][0] - W);
+    L += sw * s_l[v][0];
+    acc += sw * s_o[v][0][d];
   }
   if (F8) acc *= a.kv_scale_v;
   const size_t oi = ((size_t)b * a.n_heads + h) * HD + d;
@@ -747,21 +777,27 @@ __device__ __forceinline__ void attn_short(const AttnDecodeArgs& a, int kvh, int
 
 // The grid is flat (one x-slot per role of the larger form) and each workgroup derives its role from seq_len, so a
 // launch captured for max_ctx serves every context; workgroups without keys return at once.
-constexpr int ATTN_SPLIT_LEN = 512;
 struct AttnSplit {
-  int p;    // workgroups per (row, KV head) of attn_core
+  int p;           // workgroups per (row, KV head) of attn_core
+  int turn, most;  // where the grid has more x-slots: rows take other ones of them (row >> turn, at most `most`)
 };
 
 template <int HD, int G, bool F8 = false>
 __device__ __forceinline__ void attn_role(const AttnDecodeArgs& a, const AttnSplit& s, int wg) {
-  if (G > 1 && a.seq_len[blockIdx.z] <= a.short_len) {
+  if ((G > 1 || a.short_len > 0) && a.seq_len[blockIdx.z] <= a.short_len) {
     // workgroups are dealt round-robin over the 8 XCDs (blockIdx % 8), so workgroup wg takes query head
     // (wg % 8) * (H / 8) + wg / 8: the G query heads of a KV head then run on one XCD and read its K/V from that
     // XCD's L2 after the first miss (the plain mapping put them on G different XCDs)
     if (wg >= a.n_heads) return;
     const int h = (a.n_heads & 7) == 0 ? (wg & 7) * (a.n_heads >> 3) + (wg >> 3) : wg;
-    attn_short<HD, F8>(a, h / G, h);
+    attn_lanes<HD, F8, false>(a, h / G, h, 0, 1);
   } else {
+    // (the same slots in every row put two workgroups on some CUs and none on others: 16 rows of 1500 keys, 32 / 16 heads of
+    // 64 30 -> 21 us)
+    if (s.most) {
+      wg -= min((int)blockIdx.z >> s.turn, s.most) * (a.n_kv_heads * s.p);
+      if (wg < 0) wg += gridDim.x;
+    }
     if (wg >= a.n_kv_heads * s.p) return;
     attn_core<HD, G, F8>(a, wg % s.p, wg / s.p, s.p);
   }
@@ -780,15 +816,22 @@ inline AttnDecodeArgs attn_resolve(const AttnDecodeArgs& a) {
   if (b.combine_trips == 0) b.combine_trips = attn_env_int("AIOS_ATTN_COMBINE", 1);
   // The short form as long as its workgroups (a row's query heads) are resident at once, two to a CU at head_dim 64
   // and one at 128 (registers); beyond, attn_core's (a row's KV heads): 12 rows of 450 keys, 32 / 8 heads of 128:
-  // 14.6 us short, 11.5 us core; 16 rows, 32 / 4 heads of 64: 7.5 and 8.1 us.  AIOS_ATTN_GROUPED_MIN=n: attn_core
-  // from n such workgroups up.
+  // 14.6 us short, 11.5 us core; 16 rows, 32 / 4 heads of 64: 7.5 and 8.1 us.  One head of 64 per KV head, where
+  // either form has a workgroup a head: up to half of the CUs (8 rows of 400 keys, 16 heads 6.2 and 7.9 us, 16 rows of 500
+  // 9.8 and 8.9).  AIOS_ATTN_GROUPED_MIN=n: attn_core from n such workgroups up.
   if (b.short_len < 0) {
-    const int grouped_min = attn_env_int("AIOS_ATTN_GROUPED_MIN", 0);
-    const bool core = grouped_min > 0 ? a.B * a.n_kv_heads >= grouped_min
-                                      : a.B * a.n_heads > device_cu_count() * (a.head_dim == 64 ? 2 : 1);
-    b.short_len = core ? 0 : ATTN_SPLIT_LEN;
+    const int grouped_min = attn_env_int("AIOS_ATTN_GROUPED_MIN", 0), cus = device_cu_count(), wgs = a.B * a.n_heads;
+    const int most = a.head_dim != 64 ? cus : a.n_heads == a.n_kv_heads ? cus / 2 : 2 * cus;
+    b.short_len = (grouped_min > 0 ? a.B * a.n_kv_heads >= grouped_min : wgs > most) ? 0 : ATTN_SPLIT_LEN;
   }
   return b;
+}
+
+// Whether every context takes attn_lanes: one query head of 128 per KV head, bf16, or fp8 where the heads alone are more
+// than the CUs.  us, lanes / core, 32 heads: bf16 16 rows of 130 keys 9.5 / 13.1, of 600 27.7 / 30.9, one row of 600 8.6 / 9.5; fp8
+// 16 rows of 600 18.4 / 20.4, 4 of 4000 32 / 29.
+inline bool attn_lanes_only(const AttnDecodeArgs& a, int G) {
+  return G == 1 && a.head_dim == 128 && (!a.kv_fp8 || a.B * a.n_heads > device_cu_count());
 }
 
 // the launch shape for AttnDecodeArgs a (split already resolved): fills the split and returns the flat
@@ -798,6 +841,9 @@ inline int attn_plan(const AttnDecodeArgs& a, int G, AttnSplit& sp) {
   sp.p = std::max(1, std::min(nch, a.split / ATTN_CHUNK));
   if (sp.p > a.n_chunks || sp.p > 64)
     throw std::runtime_error("attn_decode: more splits than partial buffers / 64");
-  return std::max(a.n_kv_heads * sp.p, G > 1 && a.short_len != 0 ? a.n_heads : 0);
+  const int core = a.n_kv_heads * sp.p, slots = std::max(core, a.short_len != 0 ? a.n_heads : 0);
+  sp.most = slots / core - 1;
+  for (sp.turn = 0; sp.most && (2 << sp.turn) * (sp.most + 1) <= a.B;) ++sp.turn;
+  return slots;
 }
 }  // namespace aios

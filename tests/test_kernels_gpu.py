@@ -538,7 +538,8 @@ def test_attention_decode_fp8_kv(E, hd, H, Hkv, lens, max_ctx, grouped, monkeypa
         assert torch.allclose(out[b].cpu(), ref, atol=5e-4, rtol=5e-3), (b, (out[b].cpu() - ref).abs().max())
 
 
-@pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (16, 8, 128), (40, 8, 128), (64, 8, 128), (6, 3, 64)])
+@pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (16, 8, 128), (40, 8, 128), (64, 8, 128), (6, 3, 64),
+                                      (8, 8, 128), (96, 96, 128)])
 @pytest.mark.parametrize("lens", [(1, 32, 33, 255), (256, 257, 288, 513), (31, 512, 1025, 4001), (2048, 2049), (4096,)])
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("grouped", ["", "1"])  # "1": no form of its own for short contexts
@@ -582,6 +583,31 @@ def test_attention_decode_tiles(E, H, Hkv, hd, lens, fp8, grouped, monkeypatch):
             ref = (p[..., None] * v[:, None]).sum(2).reshape(-1)
             err = float((out[b].double() - ref).norm() / ref.norm())
             assert err < 2e-5, (b, n, err)
+
+
+def test_attention_decode_rows_in_turn(E):
+    """a grid with more slots than attn_core's workgroups (two heads of 64 per KV head, 11 and 16 rows): every row's KV heads
+    are taken once, whichever slots of the row they are, the others return"""
+    H, Hkv, hd, max_ctx, n = 32, 16, 64, 1024, 700
+    for B in (11, 16):
+        g = torch.Generator().manual_seed(B)
+        kc, vc = (torch.randn(B, Hkv, max_ctx, hd, generator=g).to(torch.bfloat16) for _ in range(2))
+        kp, vp = paged_cache(kc)[0].cuda(), paged_cache(vc)[0].cuda()
+        q = torch.randn(B, H, hd, generator=g).cuda()
+        seq = torch.tensor([n - b if b % 3 else 300 for b in range(B)], dtype=torch.int32, device="cuda")
+        slot, nch = torch.arange(B, dtype=torch.int32, device="cuda"), max_ctx // E.ATTN_CHUNK
+        opart, ml = torch.empty(B, H, nch, hd, device="cuda"), torch.empty(B, H, nch, 2, device="cuda")
+        out, cnt = torch.full((B, H * hd), float("nan"), device="cuda"), torch.zeros(B, H, dtype=torch.int32, device="cuda")
+        E.attn_decode(q.data_ptr(), kp.data_ptr(), vp.data_ptr(), seq.data_ptr(), slot.data_ptr(), B, H, Hkv, hd, max_ctx, nch, 0.125,
+                      opart.data_ptr(), ml.data_ptr(), out.data_ptr(), cnt.data_ptr(), stream())
+        torch.cuda.synchronize()
+        f = 0.125 * 1.4426950408889634
+        qq = (q * f).to(torch.bfloat16).double().cpu() / 1.4426950408889634
+        for b in range(B):
+            L = int(seq[b])
+            p = torch.softmax(qq[b].view(Hkv, 2, hd) @ kc[b, :, :L].double().transpose(1, 2), -1)
+            ref = (p @ vc[b, :, :L].double()).reshape(-1)
+            assert float((out[b].cpu().double() - ref).norm() / ref.norm()) < 2e-5, b
 
 
 @pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (40, 8, 128), (64, 8, 128), (16, 8, 64)])
