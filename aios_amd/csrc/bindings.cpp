@@ -37,7 +37,7 @@ struct GemmWs {
 };
 GemmWs& gemm_ws(int M, int N) {
   static GemmWs g;
-  const size_t need = gemm_skinny_ws_bytes(std::min(M, 64), N);
+  const size_t need = std::max(gemm_skinny_ws_bytes(std::min(M, 64), N), (size_t)64 << 20);  // (prefill plans of an engine: its widest product's)
   const int need_cnt = gemm_skinny_cnt_len(N);
   if (need > g.bytes) {
     HIP_CHECK(hipDeviceSynchronize());
@@ -761,6 +761,8 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
         int n0 = 0;
         for (int s = 0; s < a.nseg; ++s) { a.seg[s] = segs[s]->w; a.seg_n0[s] = n0; n0 += segs[s]->w.rows; }
         a.M = M; a.N = n0; a.K = segs[0]->w.cols; a.epi = epi; a.ksplit = ksplit;
+        const GemmWs& g = gemm_ws(M, n0);
+        a.ws = g.ws; a.ws_bytes = g.bytes; a.cnt = g.cnt; a.cnt_len = g.cnt_len;
         int bm = 0, bn = 0, sp = 0;
         gemm_pf_plan(a, bm, bn, sp);
         return py::make_tuple(bm, bn, sp);

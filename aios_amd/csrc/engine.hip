@@ -789,6 +789,9 @@ void Engine::tune_prefill_gemm() {
       launches.push_back(g);
     }
   }
+  for (GemmQArgs& g : launches) {
+    g.ws = gk_ws_; g.ws_bytes = gk_ws_bytes_; g.cnt = gk_cnt_; g.cnt_len = gk_cnt_len_;
+  }
   gemm_pf_autotune(launches, stream_);
   HIP_CHECK(hipStreamSynchronize(stream_));
   HIP_CHECK(hipFree(tmp));

@@ -25,6 +25,14 @@ extern template bool pf_launch_fmt<QT_Q4_0, QT_Q4_0>(const GemmQArgs&, int, int,
 extern template bool pf_launch_fmt<QT_Q8_0, QT_Q8_0>(const GemmQArgs&, int, int, int, hipStream_t);
 #endif
 
+#ifndef AIOS_BF16_ONLY
+bool pfk_serves(const GemmQArgs& a, int bm, int bn, int S);             // gemm_pfk.hip
+bool pfk_run(const GemmQArgs& a, int bm, int bn, int S, hipStream_t st);
+#else
+static bool pfk_serves(const GemmQArgs&, int, int, int) { return false; }
+static bool pfk_run(const GemmQArgs&, int, int, int, hipStream_t) { return false; }
+#endif
+
 static int pf_env(const char* name, int dflt) {
   const char* e = std::getenv(name);
   return e ? std::atoi(e) : dflt;
@@ -40,6 +48,13 @@ struct PfPlan {
 // its fp32 atomic traffic (and the zeroing of a STORE target).
 static double pf_model(const GemmQArgs& a, int bm, int bn, int S, bool bf) {
   const double cus = device_cu_count();
+  if (bn < 0) {  // K over the waves (gemm_pfk.h): us of a slot of 128 k, of a workgroup, of its rounds
+    const int MT = bm / 32, CT = -bn / 32;
+    const double tiles = (double)((a.M + bm - 1) / bm) * (a.N / -bn), q6 = a.seg[0].qtype == QT_Q6_K ? 1.3 : 1.0;
+    const double slot = std::max(0.08 + 0.032 * MT * CT + 0.07 * CT * q6, (bm * 256.0 + CT * 32 * 72 * q6) / 85e3);
+    const double wg = a.K / 128.0 / S * slot + 3.5 + 0.26 * MT * CT;
+    return (std::ceil(tiles * S / cus) * wg + (S > 1 ? 3.5 : 0.0) + 1.5) * 1e-6;
+  }
   const double tiles = (double)((a.M + bm - 1) / bm) * (a.N / bn);
   const double ksteps = (double)(a.K / 64) / S;
   // sustained MFMA fraction per tile shape (dequant VALU + LDS fragment reads beside the MFMAs)
@@ -63,8 +78,10 @@ static double pf_model(const GemmQArgs& a, int bm, int bn, int S, bool bf) {
   return t;
 }
 
-// the tiles there are (gemm_pf.h pf_launch_fmt), largest first
-static const struct { int bm, bn; } PF_TILES[] = {{256, 256}, {256, 128}, {160, 128}, {128, 256}, {128, 128}, {96, 128}, {64, 256}, {64, 128}};
+// the tiles there are, largest first: gemm_pf.h pf_launch_fmt, and with a minus before the columns gemm_pfk.hip (K over the waves)
+static const struct { int bm, bn; } PF_TILES[] = {{256, 256}, {256, 128}, {160, 128}, {128, 256}, {128, 128}, {96, 128}, {64, 256}, {64, 128},
+                                                  {160, -128}, {128, -128}, {96, -128}, {64, -128}, {160, -64}, {128, -64}, {96, -64}, {64, -64},
+                                                  {160, -32}, {128, -32}, {96, -32}, {64, -32}};
 static bool pf_tile_ok(const GemmQArgs& a, int bn) {
   if (a.N % bn) return false;
   for (int s = 0; s < a.nseg; ++s)
@@ -121,7 +138,8 @@ static bool pf_sk_ok(const GemmQArgs& a, int bm, int bn, bool bf) {
 static bool pf_plan_ok(const GemmQArgs& a, const PfPlan& p, bool bf) {
   bool tile = false;
   for (const auto& t : PF_TILES) tile = tile || (t.bm == p.bm && t.bn == p.bn);
-  if (!tile || !pf_tile_ok(a, p.bn)) return false;
+  if (!tile || !pf_tile_ok(a, std::abs(p.bn))) return false;
+  if (p.bn < 0) return pfk_serves(a, p.bm, -p.bn, p.s);
   if (p.s < 0) return pf_sk_ok(a, p.bm, p.bn, bf);
   if (p.s == 0 || (p.s > 1 && (pf_no_split(a) || a.K / 64 / p.s < 2))) return false;
   return bf || p.bn != 256 || a.K / 256 / p.s >= 1;  // (pf8c slices whole 256-blocks)
@@ -137,7 +155,7 @@ static std::vector<PfPlan> pf_candidates(const GemmQArgs& a, bool bf) {
       p.bm = t.bm; p.bn = t.bn; p.s = S;
       if (!pf_plan_ok(a, p, bf)) continue;
       // (not timed: slices that make over three rounds of workgroups)
-      const double wgs = (double)((a.M + t.bm - 1) / t.bm) * (a.N / t.bn) * S;
+      const double wgs = (double)((a.M + t.bm - 1) / t.bm) * (a.N / std::abs(t.bn)) * S;
       if (S > 1 && a.ksplit <= 0 && wgs > 3.0 * device_cu_count()) continue;
       out.push_back(p);
     }
@@ -171,7 +189,7 @@ static PfPlan pf_model_plan(const GemmQArgs& a, bool bf, bool s1_only) {
   if (tile) std::sscanf(tile, "%dx%d", &fbm, &fbn);
   for (const auto& tile_ : PF_TILES) {
     const int bm = tile_.bm, bn = tile_.bn;
-    if (fbm && (bm != fbm || bn != fbn)) continue;
+    if (fbm ? bm != fbm || bn != fbn : bn < 0) continue;  // (K over the waves: where timed, or pinned)
     for (int S : {1, 2, 3, 4, 6, 8, 12, 16, -1}) {
       if (a.ksplit > 0 && S != a.ksplit) continue;
       if (a.ksplit <= 0 && split != 0 && S != split) continue;  // (AIOS_GEMM_PF_SPLIT=-1: stream-K)
@@ -195,6 +213,7 @@ static bool pf_eligible(const GemmQArgs& a);
 static bool pf_run(const GemmQArgs& a, const PfPlan& p, hipStream_t st) {
   const int qt0 = a.seg[0].qtype, qt1 = a.seg[a.nseg - 1].qtype;
   if (p.s != 1 && a.epi == GEPI_QKV) return false;  // (plans keep S = 1 for it; a pinned split declines)
+  if (p.bn < 0) return pfk_run(a, p.bm, -p.bn, p.s, st);
   if (p.s != 1 && a.epi == GEPI_STORE)
     launch_zero_rows(a.C, a.ldc, a.M, a.N, st);  // (a kernel: the launch may be captured)
 #ifndef AIOS_BF16_ONLY
@@ -280,7 +299,7 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
     const GemmQArgs& a = *v[0];
     auto run = [&](const PfPlan& p) { pf_run(*v[at++ % v.size()], p, st); };
     for (const PfPlan& p : plans) {
-      const int form = p.s == 1 ? (a.N / p.bn) * ((a.M + p.bm - 1) / p.bm) > device_cu_count() : p.s < 0 ? 2 : 3;
+      const int form = p.bn < 0 ? 0 : p.s == 1 ? (a.N / p.bn) * ((a.M + p.bm - 1) / p.bm) > device_cu_count() : p.s < 0 ? 2 : 3;
       if (loaded.insert({a.seg[0].qtype, a.seg[a.nseg - 1].qtype, a.epi, p.bm, p.bn, form}).second) run(p);
     }
     while (ev.size() <= plans.size()) {
@@ -308,9 +327,18 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
     const bool bf = a.seg[0].qtype == QT_BF16;
     const PfPlan mp = pf_model_plan(a, bf, false), mp1 = pf_model_plan(a, bf, true);
     auto model = [&](const PfPlan& p) { return pf_model(a, p.bm, p.bn, p.s, bf); };
+    const std::vector<PfPlan> all = pf_candidates(a, bf);
+    double least = 1e30;
+    bool waves = false;
+    for (const PfPlan& p : all) {
+      least = std::min(least, model(p));
+      waves = waves || p.bn < 0;
+    }
     std::vector<PfPlan> c;
-    for (const PfPlan& p : pf_candidates(a, bf))
-      if (!mp.bm || model(p) <= 2 * model(mp) || same(p, mp1)) c.push_back(p);
+    for (const PfPlan& p : all) {
+      // (beside K over the waves no other tile below 256 columns was ever the fastest, three models' 240 keys)
+      if ((model(p) <= 2 * least && !(waves && p.bn == 128)) || same(p, mp) || same(p, mp1)) c.push_back(p);
+    }
     if (c.empty()) continue;
     if (&w == &work[0]) time(v, {c[0]}, 100);  // (the clocks)
     const std::vector<float> us = time(v, c, 2);
@@ -329,7 +357,8 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
       std::vector<PfPlan> both(f);
       both.insert(both.end(), f.rbegin(), f.rend());
       const std::vector<float> t = time(v, both, 4);
-      auto sum = [&](size_t i) { return t[i] + t[2 * n - 1 - i]; };
+      // (K over the waves by 4 % or not: 4096 x 4096 at 2048 rows, 3 % faster here, took 86 us of a pass where 128 x 256 tiles took 84)
+      auto sum = [&](size_t i) { return (t[i] + t[2 * n - 1 - i]) * (f[i].bn < 0 ? 1.04f : 1.f); };
       size_t best = 0;
       for (size_t i = 1; i < n; ++i)
         if (sum(i) < sum(best)) best = i;

@@ -1666,6 +1666,82 @@ def test_gemm_pf_odd_k_steps(E, monkeypatch, tile, K, S, epi):
         assert err.max() < K * 2.0 ** -24 + (2.0 ** -8 if epi == "store16" else 0.0)
 
 
+# ---- the prefill GEMM with K over the waves (gemm_pfk.h): BM x -BN tiles
+PFK_TILES = [f"{bm}x-{bn}" for bm in (64, 96, 128, 160) for bn in (32, 64, 128)]
+
+
+@pytest.mark.parametrize("tile", PFK_TILES)
+@pytest.mark.parametrize("fmt", ["q4k", "q6k", "mixed"])
+@pytest.mark.parametrize("K,S", [(256, 1), (1280, 1), (1280, 2), (1280, 4), (2048, 3)])
+def test_gemm_pfk(E, monkeypatch, tile, fmt, K, S):
+    """Every tile and format, one block of weights to several, slices of unlike length; rows at and past a tile's edge; a pitch
+    of its own for either matrix.  Bound: the weights' rounding to bf16, half an ulp evenly spread (2^-9 / sqrt 3), doubled."""
+    bm, bn = (int(v) for v in tile.split("x"))
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    mats, W = pf_mats(E, fmt, K)
+    N = W.shape[0]
+    for M, epi in ((33, "store"), (bm, "accum"), (bm + 1, "store"), (2 * bm - 3, "accum")):
+        e = E.GEPI_STORE if epi == "store" else E.GEPI_ACCUM
+        monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
+        if list(E.gemm_pf_plan(mats, M, e, 0)) != [bm, bn, S]:
+            assert tile == "160x-128" and fmt != "q4k"  # (LDS)
+            pytest.skip("no such tile")
+        x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+        A = torch.full((M, K + 8), float("nan"), dtype=torch.bfloat16)
+        A[:, :K] = x
+        A, C = A.cuda(), torch.full((M + 1, N + 4), 2.0, device="cuda")
+        for _ in range(2):  # (the tickets are armed again)
+            E.gemm_q(A.data_ptr(), K + 8, mats, M, C.data_ptr(), 0, N + 4, e, stream(), S if S > 1 else 0)
+        torch.cuda.synchronize()
+        ref = x.double() @ W.double().T
+        got = C[:M, :N].cpu().double()
+        got = got if epi == "store" else (got - 2) / 2
+        assert bool((C[:, N:] == 2).all()) and bool((C[M] == 2).all())
+        rel = float((got - ref).norm() / ref.norm())
+        assert rel < 2 * 2.0 ** -9 / 3 ** 0.5 + K * 2.0 ** -24, rel
+
+
+@pytest.mark.parametrize("tile", ["64x-32", "96x-64", "160x-128"])
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("S", [1, 3])
+def test_gemm_pfk_swiglu(E, monkeypatch, tile, act, S):
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
+    M, K = 161, 1024
+    mats, W = pf_mats(E, "q4k", K)
+    N = W.shape[0]
+    assert E.gemm_pf_plan(mats, M, E.GEPI_SWIGLU_BF16, 0)[1:] == (int(tile.split("x")[1]), S)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(act)).to(torch.bfloat16)
+    A, out = x.cuda(), torch.full((M, N // 2 + 2), 7.0, dtype=torch.bfloat16, device="cuda")
+    E.gemm_q(A.data_ptr(), K, mats, M, 0, out.data_ptr(), N // 2 + 2, E.GEPI_SWIGLU_BF16, stream(), 0, act=act)
+    torch.cuda.synchronize()
+    z = x.double() @ W.double().T
+    g = z[:, 0::2]
+    ref = (torch.nn.functional.gelu(g, approximate="tanh") if act else torch.nn.functional.silu(g)) * z[:, 1::2]
+    assert bool((out[:, N // 2:] == 7).all())
+    rel = float((out[:, :N // 2].cpu().double() - ref).norm() / ref.norm())
+    assert rel < 3 * 2 * 2.0 ** -9 / 3 ** 0.5, rel  # (the product of two rounded sums, rounded)
+
+
+def test_gemm_pfk_is_not_taken(E, monkeypatch):
+    """calls that its 16-byte stores or its workspace do not fit keep the other tiles: C off 16 bytes, a pitch off 4, more slices than
+    blocks; their results are the same products"""
+    K, M = 512, 70
+    mats, W = pf_mats(E, "q4k", K)
+    N = W.shape[0]
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    A, ref = x.cuda(), x.double() @ W.double().T
+    for off, ldc in ((1, N + 4), (0, N + 3), (0, N)):
+        buf = torch.zeros(M * ldc + 4, device="cuda")
+        E.gemm_q(A.data_ptr(), K, mats, M, buf[off:].data_ptr(), 0, ldc, E.GEPI_ACCUM, stream(), 0)
+        torch.cuda.synchronize()
+        got = buf[off:off + M * ldc].view(M, ldc)[:, :N].cpu().double()
+        assert float((got - ref).norm() / ref.norm()) < 2 * 2.0 ** -9 / 3 ** 0.5 + K * 2.0 ** -24
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", "64x-64")
+    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", "3")
+    assert E.gemm_pf_plan(mats, M, E.GEPI_STORE, 0)[0] == 0
+
+
 def pf_plan_entry(E, N, K, M, epi, bm, bn, S, s1=0):
     """one line of a plan list for a bf16 matrix: shape, row bucket, epilogue, formats, segments, CUs; tile, slices, map"""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
