@@ -62,6 +62,18 @@ __device__ __forceinline__ void pf_qkv_out(const GemmQArgs& a, int m, int n, flo
 }
 
 
+// Tile L of nM x nN: bands of 1024 rows, and down a band's row tiles before the next column tile.  An XCD works on 32 successive
+// tiles at a time, so 4 x 8 of 256 x 256: 12 panels of X and W go through its L2, where one row of tiles has 33.
+// us at 2048 rows, 256 x 256, along the rows -> so: 8192 x 4096 bf16 125 -> 116, Q6_K 140 -> 136, Q4_K 122 -> 120 (codes of 4.5 bits:
+// the panels of W are the small ones); 28672 x 4096 bf16 584 -> 570, Q4_K SwiGLU 491 -> 482
+template <int BM>
+__device__ __forceinline__ void pf_tile(int L, int nM, int nN, int& tm, int& tn) {
+  constexpr int GM = 1024 / BM;
+  const int band = L / (GM * nN), r = L - band * (GM * nN), g = min(GM, nM - band * GM);
+  tn = r / g;
+  tm = band * GM + r - tn * g;
+}
+
 // slot layout for one K-step: A, then the weight planes of BN columns
 template <int QT, int BM, int BN>
 struct PfLayout {
@@ -1648,7 +1660,8 @@ template <int QT0, int QT1, int BM, int EPI, int PROBE = 0>
 __global__ void __launch_bounds__(512) gemm_pf8_kernel(GemmQArgs a) {
   const int nN = a.N / 256, nM = (a.M + BM - 1) / BM, total = nN * nM;
   const int L = xcd_remap(blockIdx.x, total);
-  const int tn = L % nN, tm = L / nN;
+  int tm, tn;
+  pf_tile<BM>(L, nM, nN, tm, tn);
   const int m0 = tm * BM, n0 = tn * 256;
   int seg = 0;
   if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
@@ -1702,7 +1715,8 @@ __global__ void __launch_bounds__(512) gemm_pf8t_kernel(GemmQArgs a, int F) {
     L = F + j / PARTS;
     part = j % PARTS;
   }
-  const int tn = L % nN, tm = L / nN;
+  int tm, tn;
+  pf_tile<256>(L, (a.M + 255) / 256, nN, tm, tn);
   const int m0 = tm * 256 + (part > 0 ? part * BT : 0), n0 = tn * 256;
   if (m0 >= a.M) return;
   int seg = 0;
@@ -1758,7 +1772,8 @@ __device__ __forceinline__ void pf_stream_k(const GemmQArgs& a, int BN, int ipw,
   while (it < end) {
     const int L = (int)(it / nk), k0 = (int)(it - (long)L * nk);
     const int k1 = (int)(k0 + (end - it) < nk ? k0 + (end - it) : nk);
-    const int tn = L % nN, tm = L / nN;
+    int tm, tn;
+    pf_tile<BM>(L, nM, nN, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     int seg = 0;
     if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
@@ -1869,7 +1884,8 @@ __global__ void __launch_bounds__(256 * KG) gemm_pf4_kernel(GemmQArgs a) {
   constexpr int BN = 4 * WC;
   const int nN = a.N / BN, nM = (a.M + BM - 1) / BM, total = nN * nM;
   const int L = xcd_remap(blockIdx.x, total);
-  const int tn = L % nN, tm = L / nN;
+  int tm, tn;
+  pf_tile<BM>(L, nM, nN, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
   int seg = 0;
   if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
@@ -1898,7 +1914,8 @@ __global__ void __launch_bounds__(256) gemm_pf4t_kernel(GemmQArgs a, int F) {
     L = F + (j >> 1);
     half = j & 1;
   }
-  const int tn = L % nN, tm = L / nN;
+  int tm, tn;
+  pf_tile<256>(L, (a.M + 255) / 256, nN, tm, tn);
   const int m0 = tm * 256 + (half > 0 ? 128 : 0), n0 = tn * BN;
   int seg = 0;
   if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
@@ -1983,7 +2000,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_pf_kernel(GemmQArgs a) {
   constexpr int BN = NW * 32;
   const int nN = a.N / BN, nM = (a.M + BM - 1) / BM, total = nN * nM;
   const int L = xcd_remap(blockIdx.x, total);
-  const int tn = L % nN, tm = L / nN;
+  int tm, tn;
+  pf_tile<BM>(L, nM, nN, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
   int seg = 0;
   if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
