@@ -36,13 +36,10 @@ namespace aios {
 // GEPI_QKV (prefill chunks, non-NeoX RoPE, no QK-norm / bias, S = 1): the accumulator element
 // (m, n) of this lane goes to the attention inputs directly -- RoPE'd q fp32 to q_out[m][q_dim], RoPE'd
 // k and v as bf16 into the paged KV cache at (slot[m], pos[m]) -- the qkv_post launch and the fp32
-// QKV round trip folded into the epilogue.  The RoPE partner (column n ^ 1) is the lane ^ 1 in both
-// accumulator layouts (column = lane mod 16 / 32); every lane runs the DPP, the even one stores the pair.
-__device__ __forceinline__ void pf_qkv_out(const GemmQArgs& a, int m, int n, float v, bool even) {
-  const float w = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
-  if (!even || m >= a.M) return;
+// QKV round trip folded into the epilogue.  The RoPE partner (column n ^ 1) lies beside it in the 8-wave bodies; in the 4-wave
+// ones (column = lane mod 32) it is the lane ^ 1's: every lane runs the DPP, the even one stores the pair.
+__device__ __forceinline__ void pf_qkv_pair(const GemmQArgs& a, int m, int n, float v0, float v1) {  // columns n, n + 1
   const int hd = a.head_dim, pos = a.pos[m], slot = a.slot ? a.slot[m] : 0;
-  float v0 = v, v1 = w;
   const int part = n < a.q_dim ? 0 : (n < a.q_dim + a.kv_dim ? 1 : 2);
   const int r = n - (part == 0 ? 0 : (part == 1 ? a.q_dim : a.q_dim + a.kv_dim));
   const int head = r / hd, lr = r - head * hd;
@@ -60,7 +57,10 @@ __device__ __forceinline__ void pf_qkv_out(const GemmQArgs& a, int m, int n, flo
     *(uint32_t*)(cache + base + lr) = pk_bf16(v0, v1);
   }
 }
-
+__device__ __forceinline__ void pf_qkv_out(const GemmQArgs& a, int m, int n, float v, bool even) {
+  const float w = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
+  if (even && m < a.M) pf_qkv_pair(a, m, n, v, w);
+}
 
 // Tile L of nM x nN: bands of 1024 rows, and down a band's row tiles before the next column tile.  An XCD works on 32 successive
 // tiles at a time, so 4 x 8 of 256 x 256: 12 panels of X and W go through its L2, where one row of tiles has 33.
@@ -653,7 +653,17 @@ struct Pf4Layout {
   static_assert(NS >= 2 && (NS - 1) * PW <= 63, "pf4 ring depth / vmcnt immediate");
 };
 
-template <int QT, int BM, int WC, int NW = 4>
+// the column that position p of an 8-wave body's 32 holds (pf8_finish)
+template <int EPI>
+constexpr bool pf8_perm() {
+  return EPI == GEPI_SWIGLU_BF16 || EPI == GEPI_STORE16;
+}
+template <bool PERM>
+__device__ __forceinline__ int pf8_col(int p) {
+  return PERM ? 8 * ((p >> 2) & 3) + 4 * (p >> 4) + (p & 3) : p;
+}
+
+template <int QT, int BM, int WC, int NW = 4, bool PERM = false>  // PERM: pf8_col
 struct Pf4Dma {
   using L = Pf4Layout<QT, BM, WC, NW>;
   uint32_t off[L::PW];
@@ -672,23 +682,23 @@ struct Pf4Dma {
         const int p = 64 * (i - L::NA) + lane;
         if constexpr (L::BF) {
           const int col = p >> 3, c = (p & 7) ^ ((col >> 1) & 7);
-          o = ((uint32_t)(wcol0 + col) * (uint32_t)a.K + (uint32_t)(c * 8)) * 2u;
+          o = ((uint32_t)(wcol0 + pf8_col<PERM>(col)) * (uint32_t)a.K + (uint32_t)(c * 8)) * 2u;
         } else if constexpr (L::L8) {  // 4 x 16 B per column
           const int col = p >> 2, u = p & 3;
-          o = (uint32_t)(wcol0 + col) * nbk * 256u + (uint32_t)u * 16u;
+          o = (uint32_t)(wcol0 + pf8_col<PERM>(col)) * nbk * 256u + (uint32_t)u * 16u;
         } else {
           const int col = p >> 1, hh = p & 1;
-          o = (uint32_t)(wcol0 + col) * nbk * 128u + (uint32_t)hh * 16u;
+          o = (uint32_t)(wcol0 + pf8_col<PERM>(col)) * nbk * 128u + (uint32_t)hh * 16u;
         }
       } else if constexpr (i < L::NA + L::NCODE + L::NMETA) {
-        const uint32_t row = (uint32_t)(wcol0 + (lane & (WC - 1)));
+        const uint32_t row = (uint32_t)(wcol0 + pf8_col<PERM>(lane & (WC - 1)));
         o = L::Q6 ? row * nbk * 64u : row * nbk * 16u;
       } else if constexpr (i < L::NA + L::NCODE + L::NMETA + L::NHB) {  // Q5_K qh: 2 x 16 B per column
-        o = (uint32_t)(wcol0 + (lane >> 1)) * nbk * 32u + (uint32_t)(lane & 1) * 16u;
+        o = (uint32_t)(wcol0 + pf8_col<PERM>(lane >> 1)) * nbk * 32u + (uint32_t)(lane & 1) * 16u;
       } else if constexpr (i < L::NA + L::NCODE + L::NMETA + L::NHB + L::NSC) {
-        o = (uint32_t)(wcol0 + (lane & (WC - 1))) * nbk * 16u;  // (Q4_0 / Q8_0: K / 16 bytes of d per row)
+        o = (uint32_t)(wcol0 + pf8_col<PERM>(lane & (WC - 1))) * nbk * 16u;  // (Q4_0 / Q8_0: K / 16 bytes of d per row)
       } else {
-        o = (uint32_t)(wcol0 + (lane & (WC - 1))) * nbk;
+        o = (uint32_t)(wcol0 + pf8_col<PERM>(lane & (WC - 1))) * nbk;
       }
       off[i] = o;
     });
@@ -965,6 +975,127 @@ inline int pf4_groups(const GemmQArgs& a, int bm, int S) {
   return tiles * S <= (qt == QT_Q4_K ? cus : cus * 7 / 8) && steps / S >= 8 ? 2 : 1;
 }
 
+// ---- epilogue of the 8-wave bodies.  The weights are the matrix instruction's first operand, so a lane's four elements of an
+// accumulator are successive columns of one row.  A tile's outputs are then 16-byte (bf16: 8- and 16-byte) stores instead of a
+// store an element; and the residual of a batch of rows is requested before the batch in front of it is stored (a load behind
+// a store to what may be the same place waited for it, row by row).  With 256 x 256 tiles, us, one element at a time -> so:
+//   8192 x 1024 x 2048 rows: SwiGLU Q4_K 50 -> 40, bf16 out of bf16 48 -> 36, residual 73 -> 53 (Q4_K), fp32 43 -> 43 (67 MB);
+//   28672 x 4096 x 2048 rows SwiGLU Q4_K 482 -> 452; 128 x 256 tiles, 4096 x 4096 x 2048 rows, residual 90 -> 80
+// bf16 outputs: position p of a wave's 32 columns holds column pf8_col(p), so that the two accumulators of a row are eight
+// successive columns.
+// smem: a workgroup's LDS from its start; n0: the wave's first column
+template <int EPI, int MT>
+__device__ __forceinline__ void pf8_finish(const GemmQArgs& a, const gf32x4 (&acc)[MT][2], uint8_t* smem, int m0, int n0, int wv, int S) {
+  const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+  if constexpr (EPI == GEPI_SWIGLU_BF16) {
+    const bool vec = a.ldc % 4 == 0 && ((uintptr_t)a.C16 & 7) == 0;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = m0 + 16 * i + r16;
+      const float o0 = glu_act(acc[i][0][0], a.act) * acc[i][0][1], o1 = glu_act(acc[i][0][2], a.act) * acc[i][0][3];
+      const float o2 = glu_act(acc[i][1][0], a.act) * acc[i][1][1], o3 = glu_act(acc[i][1][2], a.act) * acc[i][1][3];
+      if (m >= a.M) continue;
+      bf16_t* p = a.C16 + (size_t)m * a.ldc + (n0 >> 1) + 4 * q;
+      const uint2 v = make_uint2(pk_bf16(o0, o1), pk_bf16(o2, o3));
+      if (vec) {
+        *(uint2*)p = v;
+      } else {
+        p[0] = (bf16_t)v.x; p[1] = (bf16_t)(v.x >> 16); p[2] = (bf16_t)v.y; p[3] = (bf16_t)(v.y >> 16);
+      }
+    }
+  } else if constexpr (EPI == GEPI_STORE16) {
+    const bool vec = a.ldc % 8 == 0 && ((uintptr_t)a.C16 & 15) == 0;
+    float b[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) b[e] = a.bias16 ? a.bias16[n0 + 8 * q + e] : 0.f;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = m0 + 16 * i + r16;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = acc[i][e >> 2][e & 3] + b[e];
+      if (a.unary) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = unary_act(v[e], a.unary - 1, a.act_n);
+      }
+      if (m >= a.M) continue;
+      bf16_t* p = a.C16 + (size_t)m * a.ldc + n0 + 8 * q;
+      const uint4 o = make_uint4(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]), pk_bf16(v[4], v[5]), pk_bf16(v[6], v[7]));
+      if (vec) {
+        *(uint4*)p = o;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[e] = (bf16_t)((&o.x)[e >> 1] >> (16 * (e & 1)));
+      }
+    }
+  } else if constexpr (EPI == GEPI_QKV) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = m0 + 16 * i + r16;
+      if (m >= a.M) continue;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) pf_qkv_pair(a, m, n0 + 16 * (e >> 2) + 4 * q + (e & 3), acc[i][e >> 2][e & 3], acc[i][e >> 2][(e & 3) + 1]);
+    }
+  } else if (S > 1) {
+    // K split: whole lines of 32 columns to an atomic instruction, turned through the wave's own LDS
+    constexpr int PITCH = 144;
+    __syncthreads();  // every wave's LDS reads and DMAs are done
+    uint8_t* own = smem + wv * (16 * PITCH);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) *(gf32x4*)(own + r16 * PITCH + 64 * c + 16 * q) = acc[i][c];
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = *(const float*)(own + (2 * j + (lane >> 5)) * PITCH + 4 * (lane & 31));
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int m = m0 + 16 * i + 2 * j + (lane >> 5);
+        if (m < a.M) unsafeAtomicAdd(a.C + (size_t)m * a.ldc + n0 + (lane & 31), v[j]);
+      }
+    }
+  } else if (a.ldc % 4 || ((uintptr_t)a.C & 15)) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int m = m0 + 16 * i + r16;
+        if (m >= a.M) continue;
+        float* p = a.C + (size_t)m * a.ldc + n0 + 16 * (e >> 2) + 4 * q + (e & 3);
+        *p = EPI == GEPI_ACCUM ? *p + acc[i][e >> 2][e & 3] : acc[i][e >> 2][e & 3];
+      }
+  } else {
+    constexpr int NB = MT < 4 ? MT : 4;  // row tiles of a batch
+    gf32x4 res[2][NB][2];
+    auto at = [&](int i, int c, bool in) __attribute__((always_inline)) {
+      const int m = m0 + 16 * i + r16;
+      return (gf32x4*)(a.C + (size_t)(in ? m : min(m, a.M - 1)) * a.ldc + n0 + 16 * c + 4 * q);
+    };
+    auto get = [&](int b) __attribute__((always_inline)) {
+      if constexpr (EPI == GEPI_ACCUM) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) res[b & 1][i][c] = *at(b * NB + i, c, false);
+      }
+    };
+    get(0);
+#pragma unroll
+    for (int b = 0; b < MT / NB; ++b) {
+      if (b + 1 < MT / NB) get(b + 1);
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        if (m0 + 16 * (b * NB + i) + r16 >= a.M) continue;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          if constexpr (EPI == GEPI_ACCUM) *at(b * NB + i, c, true) = res[b & 1][i][c] + acc[b * NB + i][c];
+          else *at(b * NB + i, c, true) = acc[b * NB + i][c];
+        }
+      }
+    }
+  }
+}
+
 // ==== pf8: 8 waves (two per SIMD) x 32 columns, 16x16x32 MFMA ======================================
 // The 8-wave 16x16x32 body ran the compute-only probe at 1.33 PF per busy CU against 1.16 for pf4's
 // one wave per SIMD (the SIMD's second wave covers the first's LDS latencies); this is that body
@@ -975,6 +1106,7 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
   constexpr int NW = 8, WC = 32;
   using L = Pf4Layout<QT, BM, WC, NW>;
   constexpr int MT = BM / 16, GR = MT < 8 ? MT : 8, NG = MT / GR, NPH = 2 * NG, NS = L::NS, PW = L::PW;
+  constexpr bool PERM = pf8_perm<EPI>();
   extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -998,7 +1130,7 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
     for (int c = 0; c < 2; ++c) acc[i][c] = gf32x4{0.f, 0.f, 0.f, 0.f};
 
   const int nk = kt1 - kt0, klast = kt1 - 1;
-  Pf4Dma<QT, BM, WC, NW> dma;
+  Pf4Dma<QT, BM, WC, NW, PERM> dma;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(pf_lds_addr(pf_smem));
   dma.init(a, wcol0, m0, wv);
 #pragma unroll
@@ -1042,7 +1174,7 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int cl = 16 * c + r16;
-      const int dpar = L::Q6 ? (int)(((uint32_t)(wcol0 + cl) * nbk + (uint32_t)(rkt >> 2)) & 1u) : 0;
+      const int dpar = L::Q6 ? (int)(((uint32_t)(wcol0 + pf8_col<PERM>(cl)) * nbk + (uint32_t)(rkt >> 2)) & 1u) : 0;
       bf[c][S2] = pf_bdec<QT, S2>(raw[c], q, rkt, dpar);
       asm volatile("" : "+v"(bf[c][S2]));  // keep the decode in this phase (else sunk past the barrier)
     }
@@ -1062,7 +1194,7 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
     for (int k = 0; k < 2 * GR; ++k) {
       if (k < k0 || k >= k1) continue;
       const int c = k / GR, i = k % GR;
-      acc[g * GR + i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i], bf[c][sp], acc[g * GR + i][c], 0, 0, 0);
+      acc[g * GR + i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[c][sp], f[i], acc[g * GR + i][c], 0, 0, 0);
     }
   };
   if constexpr (!(PROBE & 1)) {
@@ -1114,33 +1246,7 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
     cur = nxt;
   }
   pf_vmcnt<0>();  // no LDS-DMA may land after this workgroup's LDS is released
-
-  // epilogue -- C/D map of the 16x16 accumulator: col = lane & 15, row = 4 * (lane >> 4) + e
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int n = n0 + wv * WC + 16 * c + r16;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + 16 * i + 4 * q + e;
-        const float v = acc[i][c][e];
-        if constexpr (EPI == GEPI_SWIGLU_BF16) {
-          const float up = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
-          if (m < a.M && !(r16 & 1)) a.C16[(size_t)m * a.ldc + (n >> 1)] = f32_to_bf16(glu_act(v, a.act) * up);
-        } else if constexpr (EPI == GEPI_STORE16) {
-          if (m < a.M) a.C16[(size_t)m * a.ldc + n] = f32_to_bf16(store16_val(a, n, v));
-        } else if constexpr (EPI == GEPI_QKV) {
-          pf_qkv_out(a, m, n, v, !(r16 & 1));
-        } else if (m < a.M) {
-          float* cp = a.C + (size_t)m * a.ldc + n;
-          if (S > 1) unsafeAtomicAdd(cp, v);
-          else if constexpr (EPI == GEPI_ACCUM) *cp += v;
-          else *cp = v;
-        }
-      }
-    }
-  }
+  pf8_finish<EPI, MT>(a, acc, pf_smem, m0, n0 + wv * WC, wv, S);
 }
 
 // ==== pf8c: pf8 with the K-quant weight planes staged coalesced ==================================
@@ -1173,7 +1279,7 @@ struct PfcLayout {
   static constexpr int PRE = NA + 6 + (Q6 ? 6 : 0);    // prologue group: step 0's A, half block 0, block 0
 };
 
-template <int QT, int BM>
+template <int QT, int BM, bool PERM = false>  // PERM: pf8_col
 struct PfcDma {
   using L = PfcLayout<QT, BM>;
   static constexpr int NW = 8;
@@ -1191,13 +1297,16 @@ struct PfcDma {
 #pragma unroll
     for (int pc = 0; pc < 2; ++pc) {
       const int row = 16 * pc + (lane >> 2), u = (lane & 3) ^ ((row >> 2) & 3);
-      offC[pc] = (uint32_t)(wcol0 + row) * nbk * 128u + 16u * (uint32_t)u;
+      offC[pc] = (uint32_t)(wcol0 + pf8_col<PERM>(row)) * nbk * 128u + 16u * (uint32_t)u;
     }
     const int l32 = lane & 31;
-    offR = (uint32_t)(wcol0 + (l32 >> 2)) * nbk * 16u + 4u * (uint32_t)(l32 & 3);  // + 8 rows per piece
-    offH = (uint32_t)(wcol0 + (l32 >> 1)) * nbk * 64u + 16u * (uint32_t)(l32 & 1);  // + 16 rows per piece
-    offD = (uint32_t)(wcol0 + (lane & 7)) * nbk;                                      // + 8 rows per piece
+    offR = (uint32_t)(wcol0 + pf8_col<PERM>(l32 >> 2)) * nbk * 16u + 4u * (uint32_t)(l32 & 3);  // + r8(piece) rows
+    offH = (uint32_t)(wcol0 + pf8_col<PERM>(l32 >> 1)) * nbk * 64u + 16u * (uint32_t)(l32 & 1);  // + r16(piece) rows
+    offD = (uint32_t)(wcol0 + pf8_col<PERM>(lane & 7)) * nbk;                                      // + r8(piece) rows
   }
+  // columns of positions 8 pr and 16 pc
+  static __device__ __forceinline__ int r8(int pr) { return pf8_col<PERM>(8 * pr); }
+  static __device__ __forceinline__ int r16(int pc) { return pf8_col<PERM>(16 * pc); }
 
   __device__ __forceinline__ void A(const GemmQArgs& a, int kt, uint32_t dst, int wv) const {
 #pragma unroll
@@ -1218,16 +1327,16 @@ struct PfcDma {
   }
   // record piece pr (rows 8 pr .. 8 pr + 7) of block bsrc; lanes 0..31
   __device__ __forceinline__ void rec(const QWeight& w, int bsrc, int pr, uint32_t nbk, uint32_t dst) const {
-    pf_glds_part<32, 4>((L::Q6 ? w.p2 : w.p1) + bsrc * 16 + (size_t)(pr * 128 * nbk), offR, dst + pr * 128);
+    pf_glds_part<32, 4>((L::Q6 ? w.p2 : w.p1) + bsrc * 16 + (size_t)(r8(pr) * 16 * nbk), offR, dst + pr * 128);
   }
   // Q6_K high-bit piece pc (rows 16 pc ..) of half block hsrc; lanes 0..31
   __device__ __forceinline__ void hi(const QWeight& w, int hsrc, int pc, uint32_t nbk, uint32_t dst) const {
-    pf_glds_part<32, 16>(w.p1 + hsrc * 32 + (size_t)(pc * 1024 * nbk), offH, dst + pc * 512);
+    pf_glds_part<32, 16>(w.p1 + hsrc * 32 + (size_t)(r16(pc) * 64 * nbk), offH, dst + pc * 512);
   }
   // Q6_K d piece pr (rows 8 pr ..) of block bsrc: the dword holding each row's f16 d; lanes 0..7
   __device__ __forceinline__ void dq(const QWeight& w, int bsrc, int pr, uint32_t nbk, uint32_t dst) const {
     const uint32_t to = __builtin_amdgcn_readfirstlane(dst + pr * 32);
-    if ((threadIdx.x & 63) < 8) pf_glds4(w.p3 + (((offD + pr * 8 * nbk + (uint32_t)bsrc) * 2u) & ~3u), to);
+    if ((threadIdx.x & 63) < 8) pf_glds4(w.p3 + (((offD + r8(pr) * nbk + (uint32_t)bsrc) * 2u) & ~3u), to);
   }
 };
 
@@ -1237,6 +1346,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
   constexpr int NW = 8, WC = 32, NSA = L::NSA, PW = L::PW;
   // row tiles per phase: 4 at BM = 256 (8 phases; 8 ran out of registers once the DMA is spread)
   constexpr int MT = BM / 16, GR = MT >= 16 ? 4 : MT, NG = MT / GR, NPH = 2 * NG;
+  constexpr bool PERM = pf8_perm<EPI>();
   extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1261,7 +1371,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
 
   // kt0, kt1 are multiples of 4 (block-aligned slices)
   const int nk = kt1 - kt0, klast = kt1 - 1, hlast = (kt1 >> 1) - 1, blast = (kt1 >> 2) - 1;
-  PfcDma<QT, BM> dma;
+  PfcDma<QT, BM, PERM> dma;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(pf_lds_addr(pf_smem));
   dma.init(a, wcol0, m0, wv);
   constexpr uint32_t CBS = NW * L::CB_W, HBS = NW * L::HB_W, RBS = NW * L::RB_W, DBS = NW * L::D_W;
@@ -1339,7 +1449,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int cl = 16 * c + r16;
-      const int dpar = L::Q6 ? (int)(((uint32_t)(wcol0 + cl) * nbk + (uint32_t)(rkt >> 2)) & 1u) : 0;
+      const int dpar = L::Q6 ? (int)(((uint32_t)(wcol0 + pf8_col<PERM>(cl)) * nbk + (uint32_t)(rkt >> 2)) & 1u) : 0;
       bf[c][S2] = pf_bdec<QT, S2>(raw[c], q, place, dpar);
       asm volatile("" : "+v"(bf[c][S2]));  // keep the decode in this phase (else sunk past the barrier)
     }
@@ -1360,7 +1470,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
     for (int k = 0; k < 2 * GR; ++k) {
       if (k < k0 || k >= k1) continue;
       const int c = k / GR, i = k % GR;
-      acc[g * GR + i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i], bf[c][sp], acc[g * GR + i][c], 0, 0, 0);
+      acc[g * GR + i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[c][sp], f[i], acc[g * GR + i][c], 0, 0, 0);
     }
     if constexpr (BM < 256) __builtin_amdgcn_s_setprio(0);
   };
@@ -1429,32 +1539,7 @@ __device__ __forceinline__ void pf8c_body(const GemmQArgs& a, int m0, int n0, in
     cur = nxt;
   });
   pf_vmcnt<0>();  // no LDS-DMA may land after this workgroup's LDS is released
-
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int n = n0 + wv * WC + 16 * c + r16;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + 16 * i + 4 * q + e;
-        const float v = acc[i][c][e];
-        if constexpr (EPI == GEPI_SWIGLU_BF16) {
-          const float up = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
-          if (m < a.M && !(r16 & 1)) a.C16[(size_t)m * a.ldc + (n >> 1)] = f32_to_bf16(glu_act(v, a.act) * up);
-        } else if constexpr (EPI == GEPI_STORE16) {
-          if (m < a.M) a.C16[(size_t)m * a.ldc + n] = f32_to_bf16(store16_val(a, n, v));
-        } else if constexpr (EPI == GEPI_QKV) {
-          pf_qkv_out(a, m, n, v, !(r16 & 1));
-        } else if (m < a.M) {
-          float* cp = a.C + (size_t)m * a.ldc + n;
-          if (S > 1) unsafeAtomicAdd(cp, v);
-          else if constexpr (EPI == GEPI_ACCUM) *cp += v;
-          else *cp = v;
-        }
-      }
-    }
-  }
+  pf8_finish<EPI, MT>(a, acc, pf_smem, m0, n0 + wv * WC, wv, S);
 }
 
 // ==== pf8d: pf8c on v_mfma_f32_32x32x16_bf16 ======================================================

@@ -1666,6 +1666,36 @@ def test_gemm_pf_odd_k_steps(E, monkeypatch, tile, K, S, epi):
         assert err.max() < K * 2.0 ** -24 + (2.0 ** -8 if epi == "store16" else 0.0)
 
 
+@pytest.mark.parametrize("bm", [64, 128, 256])
+@pytest.mark.parametrize("fmt", ["Q4_K", "Q6_K", "Q5_K", "Q8_0", "BF16"])
+@pytest.mark.parametrize("epi", ["store", "accum", "split", "swiglu", "store16"])
+def test_gemm_pf8_outputs(E, monkeypatch, bm, fmt, epi):
+    """The 8-wave tiles' outputs: whole vectors, and a base and pitch that only single elements fit; ragged rows; nothing beside
+    them is written.  Bound: the weights' rounding to bf16, half an ulp evenly spread (2^-9 / sqrt 3), doubled; three such in a
+    rounded product of two sums."""
+    if epi == "store16" and fmt != "BF16":
+        pytest.skip("bf16 weights only")
+    K, N, M = 1024, 512, bm + 37
+    m, W = qmat(E, GGMLType[fmt], N, K, seed=7, std=0.05)
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", f"{bm}x256")
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(bm)).to(torch.bfloat16)
+    A, z = x.cuda(), x.double() @ W.double().T
+    half = epi in ("swiglu", "store16")
+    cols = N // 2 if epi == "swiglu" else N
+    ref = torch.nn.functional.silu(z[:, 0::2]) * z[:, 1::2] if epi == "swiglu" else z
+    e = {"store": E.GEPI_STORE, "accum": E.GEPI_ACCUM, "split": E.GEPI_ACCUM, "swiglu": E.GEPI_SWIGLU_BF16, "store16": E.GEPI_STORE16}[epi]
+    for off, ld in ((0, cols + 8), (1, cols + 8), (0, cols + 1)):
+        buf = torch.full(((M + 1) * ld + 8,), 2.0, device="cuda", dtype=torch.bfloat16 if half else torch.float32)
+        to = buf[off:].data_ptr()
+        E.gemm_q(A.data_ptr(), K, [m], M, 0 if half else to, to if half else 0, ld, e, stream(), 2 if epi == "split" else 1)
+        torch.cuda.synchronize()
+        out = buf[off:off + (M + 1) * ld].view(M + 1, ld).double().cpu()
+        assert bool((out[M] == 2).all()) and bool((out[:, cols:] == 2).all()) and bool((buf[:off] == 2).all())
+        got = out[:M, :cols] - (2.0 if epi in ("accum", "split") else 0.0)
+        rel = float((got - ref).norm() / ref.norm())
+        assert rel < (3 if half else 1) * 2 * 2.0 ** -9 / 3 ** 0.5 + K * 2.0 ** -24, (off, ld, rel)
+
+
 # ---- the prefill GEMM with K over the waves (gemm_pfk.h): BM x -BN tiles
 PFK_TILES = [f"{bm}x-{bn}" for bm in (64, 96, 128, 160) for bn in (32, 64, 128)]
 
