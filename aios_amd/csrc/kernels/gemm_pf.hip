@@ -25,6 +25,8 @@ extern template bool pf_launch_fmt<QT_Q4_0, QT_Q4_0>(const GemmQArgs&, int, int,
 extern template bool pf_launch_fmt<QT_Q8_0, QT_Q8_0>(const GemmQArgs&, int, int, int, hipStream_t);
 #endif
 
+bool pfkb_serves(const GemmQArgs& a, int bm, int bn, int S);            // gemm_pfk_bf16.hip
+bool pfkb_run(const GemmQArgs& a, int bm, int bn, int S, hipStream_t st);
 #ifndef AIOS_BF16_ONLY
 bool pfk_serves(const GemmQArgs& a, int bm, int bn, int S);             // gemm_pfk.hip
 bool pfk_run(const GemmQArgs& a, int bm, int bn, int S, hipStream_t st);
@@ -51,7 +53,7 @@ static double pf_model(const GemmQArgs& a, int bm, int bn, int S, bool bf) {
   if (bn < 0) {  // K over the waves (gemm_pfk.h): us of a slot of 128 k, of a workgroup, of its rounds
     const int MT = bm / 32, CT = -bn / 32;
     const double tiles = (double)((a.M + bm - 1) / bm) * (a.N / -bn), q6 = a.seg[0].qtype == QT_Q6_K ? 1.3 : 1.0;
-    const double slot = std::max(0.08 + 0.032 * MT * CT + 0.07 * CT * q6, (bm * 256.0 + CT * 32 * 72 * q6) / 85e3);
+    const double slot = std::max(0.08 + 0.032 * MT * CT + (bf ? 0.02 : 0.07) * CT * q6, (bm * 256.0 + CT * 32 * (bf ? 256 : 72) * q6) / 85e3);
     const double wg = a.K / 128.0 / S * slot + 3.5 + 0.26 * MT * CT;
     return (std::ceil(tiles * S / cus) * wg + (S > 1 ? 3.5 : 0.0) + 1.5) * 1e-6;
   }
@@ -139,7 +141,7 @@ static bool pf_plan_ok(const GemmQArgs& a, const PfPlan& p, bool bf) {
   bool tile = false;
   for (const auto& t : PF_TILES) tile = tile || (t.bm == p.bm && t.bn == p.bn);
   if (!tile || !pf_tile_ok(a, std::abs(p.bn))) return false;
-  if (p.bn < 0) return pfk_serves(a, p.bm, -p.bn, p.s);
+  if (p.bn < 0) return bf ? pfkb_serves(a, p.bm, -p.bn, p.s) : pfk_serves(a, p.bm, -p.bn, p.s);
   if (p.s < 0) return pf_sk_ok(a, p.bm, p.bn, bf);
   if (p.s == 0 || (p.s > 1 && (pf_no_split(a) || a.K / 64 / p.s < 2))) return false;
   return bf || p.bn != 256 || a.K / 256 / p.s >= 1;  // (pf8c slices whole 256-blocks)
@@ -213,7 +215,7 @@ static bool pf_eligible(const GemmQArgs& a);
 static bool pf_run(const GemmQArgs& a, const PfPlan& p, hipStream_t st) {
   const int qt0 = a.seg[0].qtype, qt1 = a.seg[a.nseg - 1].qtype;
   if (p.s != 1 && a.epi == GEPI_QKV) return false;  // (plans keep S = 1 for it; a pinned split declines)
-  if (p.bn < 0) return pfk_run(a, p.bm, -p.bn, p.s, st);
+  if (p.bn < 0) return qt0 == QT_BF16 ? pfkb_run(a, p.bm, -p.bn, p.s, st) : pfk_run(a, p.bm, -p.bn, p.s, st);
   if (p.s != 1 && a.epi == GEPI_STORE)
     launch_zero_rows(a.C, a.ldc, a.M, a.N, st);  // (a kernel: the launch may be captured)
 #ifndef AIOS_BF16_ONLY
@@ -336,8 +338,8 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
     }
     std::vector<PfPlan> c;
     for (const PfPlan& p : all) {
-      // (beside K over the waves no other tile below 256 columns was ever the fastest, three models' 240 keys)
-      if ((model(p) <= 2 * least && !(waves && p.bn == 128)) || same(p, mp) || same(p, mp1)) c.push_back(p);
+      // (quantised: beside K over the waves no other tile below 256 columns was ever the fastest, three models' 240 keys)
+      if ((model(p) <= 2 * least && !(waves && !bf && p.bn == 128)) || same(p, mp) || same(p, mp1)) c.push_back(p);
     }
     if (c.empty()) continue;
     if (&w == &work[0]) time(v, {c[0]}, 100);  // (the clocks)

@@ -23,6 +23,8 @@
 
 namespace aios {
 
+constexpr int PFK_LDS = 160 * 1024 - 64;  // dynamic LDS of these kernels at most: their last_flag lies beside it
+
 template <int QT, int MT, int CT, int NG>
 struct PfkLayout {
   static constexpr bool Q6 = QT == QT_Q6_K;
@@ -32,14 +34,14 @@ struct PfkLayout {
   // a W block (256 k): codes (128 B a column, units swizzled), high bits, records (Q6_K: int8 scales), dwords that hold d
   static constexpr int CODE = BN * 128, HB = Q6 ? BN * 64 : 0, REC = BN * 16, DW = Q6 ? (BN * 4 < 256 ? 256 : BN * 4) : 0;
   static constexpr int OFF_HB = CODE, OFF_REC = OFF_HB + HB, OFF_D = OFF_REC + REC, WB = OFF_D + DW;
-  static constexpr int NWB = (160 * 1024 - NSX * XS) / WB < 4 ? (160 * 1024 - NSX * XS) / WB : 4;
+  static constexpr int NWB = (PFK_LDS - NSX * XS) / WB < 4 ? (PFK_LDS - NSX * XS) / WB : 4;
   static constexpr int OFF_W = NSX * XS;
   static constexpr int NW = 4 * NG, NX = 2 * MT / NG;  // waves; DMA requests a wave, per X slot
   static constexpr int PC = 4 * CT, PR = 2 * CT;       // pieces of a W block: codes, records (high bits); a wave's (of few: some twice)
   static constexpr int NC = PC / NW, NR = PR > NW ? PR / NW : 1, NH = Q6 ? NR : 0, ND = Q6 ? 1 : 0, NWP = NC + NR + NH + ND;
   static constexpr int RED_BYTES = 2 * 4 * 32 * BN * 4;  // two row tiles of four partial sums
   static constexpr int TOTAL = OFF_W + NWB * WB > RED_BYTES ? OFF_W + NWB * WB : RED_BYTES;
-  static_assert(NWB < 2 || TOTAL <= 160 * 1024, "pfk LDS");
+  static_assert(NWB < 2 || TOTAL <= PFK_LDS, "pfk LDS");
 };
 
 // a 1-KB (256-B) request to LDS bytes lds ..
@@ -56,6 +58,115 @@ __device__ __forceinline__ void pfk_dma4(const void* base, uint32_t off, uint32_
                : "=&s"(from)
                : "v"(off), "s"(base), "s"(lds)
                : "memory", "m0");
+}
+
+// ---- end of a tile: the four partial sums of every output, the slices of K, the epilogue
+template <int MT, int CT, int NG, int EPI>
+__device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&acc)[MT][CT / NG], int m0, int n0, int sp, int S, int tile,
+                                          int ntile, int& last_flag) {
+  constexpr int BM = 32 * MT, BN = 32 * CT, NW = 4 * NG, CW = CT / NG;
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem0[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wv = wave & 3, cg = wave >> 2;
+  const int r32 = lane & 31, h = lane >> 5;
+  // ---- the four partial tiles meet, 32 rows at a time: [wave][row][columns], 16-B units swizzled by the row; a row tile is
+  // written while the one before it is added up
+  constexpr int QR = 8 * CT, RP = 64 * NW / QR, SRC = 32 * 32 * CT * 4;
+  auto unit = [&](int row, int q) __attribute__((always_inline)) {
+    return (uint32_t)(row * (32 * CT * 4) + ((q ^ (CT == 1 ? (row >> 1) & 7 : row & 15)) << 4));
+  };
+  const int q = tid % QR, n = n0 + 4 * q;
+  const auto ws = __builtin_amdgcn_make_buffer_rsrc((void*)a.ws, (short)0, 0x7fffffff, 0x00020000);
+  auto slab = [&](int k) __attribute__((always_inline)) {  // byte of slice k's partial sums of this tile
+    return (uint32_t)(k * ntile + tile) * (uint32_t)(BM * BN * 4);
+  };
+  auto finish = [&](int m, gf32x4 v) __attribute__((always_inline)) {
+    if constexpr (EPI == GEPI_SWIGLU_BF16) {
+      *(uint32_t*)(a.C16 + (size_t)m * a.ldc + (n >> 1)) =
+          (uint32_t)f32_to_bf16(glu_act(v[0], a.act) * v[1]) | ((uint32_t)f32_to_bf16(glu_act(v[2], a.act) * v[3]) << 16);
+    } else if constexpr (EPI == GEPI_STORE16) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = store16_val(a, n + e, v[e]);
+      *(uint2*)(a.C16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]));
+    } else {
+      float* cp = a.C + (size_t)m * a.ldc + n;
+      if constexpr (EPI == GEPI_ACCUM) v += *(const gf32x4*)cp;
+      *(gf32x4*)cp = v;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i <= MT; ++i) {
+    pf_barrier();
+    if (i < MT) {
+#pragma unroll
+      for (int c = 0; c < CW; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          *(gf32x4*)(pf_smem0 + (i & 1) * (4 * SRC) + wv * SRC + unit(r32, 8 * (cg * CW + c) + 2 * e + h)) =
+              gf32x4{acc[i][c][4 * e], acc[i][c][4 * e + 1], acc[i][c][4 * e + 2], acc[i][c][4 * e + 3]};
+    }
+    if (i > 0) {
+      const uint8_t* src = pf_smem0 + ((i - 1) & 1) * (4 * SRC);
+      gf32x4 v[32 / RP];
+#pragma unroll
+      for (int k = 0; k < 32 / RP; ++k) {
+        const uint32_t at = unit(tid / QR + RP * k, q);
+        v[k] = *(const gf32x4*)(src + at);
+#pragma unroll
+        for (int s = 1; s < 4; ++s) v[k] += *(const gf32x4*)(src + s * SRC + at);
+      }
+#pragma unroll
+      for (int k = 0; k < 32 / RP; ++k) {
+        const int row = 32 * (i - 1) + tid / QR + RP * k;
+        if (m0 + row >= a.M) continue;
+        if (S == 1) finish(m0 + row, v[k]);
+        else
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(gu32x4, v[k]), ws, slab(sp) + ((uint32_t)row * BN + 4 * q) * 4, 0, 16 /* sc1 */);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  if (S == 1) return;
+  // ---- K split over workgroups: the slabs are written through; a tile's last arriver adds them up, in the order of the slices
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains its slab stores
+  __syncthreads();
+  if (tid == 0) {
+    const int last = __hip_atomic_fetch_add(a.cnt + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
+    if (last) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __hip_atomic_store(a.cnt + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
+    }
+    last_flag = last;
+  }
+  __syncthreads();
+  if (!last_flag) return;
+  constexpr int NP = BM / RP, PB = NP < 8 ? NP : 8;  // rows of a lane; so many at a time
+#pragma unroll
+  for (int p0_ = 0; p0_ < NP; p0_ += PB) {
+    gf32x4 v[PB];
+#pragma unroll
+    for (int p = 0; p < PB; ++p) v[p] = gf32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < S; k0 += 4) {  // four slabs' loads in flight (past the last: read again, not added)
+      gf32x4 t[PB][4];
+#pragma unroll
+      for (int p = 0; p < PB; ++p) {
+        const int row = min(tid / QR + RP * min(p0_ + p, NP - 1), a.M - 1 - m0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t[p][k] = *(const gf32x4*)((const uint8_t*)a.ws + slab(min(k0 + k, S - 1)) + ((uint32_t)row * BN + 4 * q) * 4);
+      }
+#pragma unroll
+      for (int p = 0; p < PB; ++p)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (k0 + k < S) v[p] += t[p][k];
+    }
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+      const int row = tid / QR + RP * (p0_ + p);
+      if (p0_ + p < NP && m0 + row < a.M) finish(m0 + row, v[p]);
+    }
+  }
 }
 
 template <int QT, int MT, int CT, int NG, int EPI>
@@ -98,7 +209,6 @@ __device__ __forceinline__ void pfk_body(const GemmQArgs& a, int m0, int n0, int
   if constexpr (Q6) dcol = (uint32_t)(col0 + 64 * pd + (CT == 1 ? r32 : lane)) * nbk;
 
   const int t0 = 2 * b0, tlast = 2 * b1 - 1, blast = b1 - 1, nk = 2 * (b1 - b0);
-  const uint8_t* xb = (const uint8_t*)a.A - 1024;
   // request i of this wave's NX of slot t (absolute), of its NWP of block b
   auto req_x = [&](int i, int t, uint32_t dst) __attribute__((always_inline)) {
     pfk_dma1((const uint8_t*)a.A + (size_t)(uint32_t)min(t, tlast) * 256, xo[i], dst + (wave * NX + i) * 1024);
@@ -293,100 +403,7 @@ __device__ __forceinline__ void pfk_body(const GemmQArgs& a, int m0, int n0, int
   pf_vmcnt<0>();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
-  // ---- the four partial tiles meet, 32 rows at a time: [wave][row][columns], 16-B units swizzled by the row; a row tile is
-  // written while the one before it is added up
-  constexpr int QR = 8 * CT, RP = 64 * NW / QR, SRC = 32 * 32 * CT * 4;
-  auto unit = [&](int row, int q) __attribute__((always_inline)) {
-    return (uint32_t)(row * (32 * CT * 4) + ((q ^ (CT == 1 ? (row >> 1) & 7 : row & 15)) << 4));
-  };
-  const int q = tid % QR, n = n0 + 4 * q;
-  const auto ws = __builtin_amdgcn_make_buffer_rsrc((void*)a.ws, (short)0, 0x7fffffff, 0x00020000);
-  auto slab = [&](int k) __attribute__((always_inline)) {  // byte of slice k's partial sums of this tile
-    return (uint32_t)(k * ntile + tile) * (uint32_t)(L::BM * L::BN * 4);
-  };
-  auto finish = [&](int m, gf32x4 v) __attribute__((always_inline)) {
-    if constexpr (EPI == GEPI_SWIGLU_BF16) {
-      *(uint32_t*)(a.C16 + (size_t)m * a.ldc + (n >> 1)) =
-          (uint32_t)f32_to_bf16(glu_act(v[0], a.act) * v[1]) | ((uint32_t)f32_to_bf16(glu_act(v[2], a.act) * v[3]) << 16);
-    } else {
-      float* cp = a.C + (size_t)m * a.ldc + n;
-      if constexpr (EPI == GEPI_ACCUM) v += *(const gf32x4*)cp;
-      *(gf32x4*)cp = v;
-    }
-  };
-#pragma unroll
-  for (int i = 0; i <= MT; ++i) {
-    pf_barrier();
-    if (i < MT) {
-#pragma unroll
-      for (int c = 0; c < CW; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          *(gf32x4*)(pf_smem0 + (i & 1) * (4 * SRC) + wv * SRC + unit(r32, 8 * (cg * CW + c) + 2 * e + h)) =
-              gf32x4{acc[i][c][4 * e], acc[i][c][4 * e + 1], acc[i][c][4 * e + 2], acc[i][c][4 * e + 3]};
-    }
-    if (i > 0) {
-      const uint8_t* src = pf_smem0 + ((i - 1) & 1) * (4 * SRC);
-      gf32x4 v[32 / RP];
-#pragma unroll
-      for (int k = 0; k < 32 / RP; ++k) {
-        const uint32_t at = unit(tid / QR + RP * k, q);
-        v[k] = *(const gf32x4*)(src + at);
-#pragma unroll
-        for (int s = 1; s < 4; ++s) v[k] += *(const gf32x4*)(src + s * SRC + at);
-      }
-#pragma unroll
-      for (int k = 0; k < 32 / RP; ++k) {
-        const int row = 32 * (i - 1) + tid / QR + RP * k;
-        if (m0 + row >= a.M) continue;
-        if (S == 1) finish(m0 + row, v[k]);
-        else
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(gu32x4, v[k]), ws, slab(sp) + ((uint32_t)row * L::BN + 4 * q) * 4, 0, 16 /* sc1 */);
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  }
-  if (S == 1) return;
-  // ---- K split over workgroups: the slabs are written through; a tile's last arriver adds them up, in the order of the slices
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains its slab stores
-  __syncthreads();
-  if (tid == 0) {
-    const int last = __hip_atomic_fetch_add(a.cnt + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
-    if (last) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __hip_atomic_store(a.cnt + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
-    }
-    last_flag = last;
-  }
-  __syncthreads();
-  if (!last_flag) return;
-  constexpr int NP = L::BM / RP, PB = NP < 8 ? NP : 8;  // rows of a lane; so many at a time
-#pragma unroll
-  for (int p0_ = 0; p0_ < NP; p0_ += PB) {
-    gf32x4 v[PB];
-#pragma unroll
-    for (int p = 0; p < PB; ++p) v[p] = gf32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < S; k0 += 4) {  // four slabs' loads in flight (past the last: read again, not added)
-      gf32x4 t[PB][4];
-#pragma unroll
-      for (int p = 0; p < PB; ++p) {
-        const int row = min(tid / QR + RP * min(p0_ + p, NP - 1), a.M - 1 - m0);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) t[p][k] = *(const gf32x4*)((const uint8_t*)a.ws + slab(min(k0 + k, S - 1)) + ((uint32_t)row * L::BN + 4 * q) * 4);
-      }
-#pragma unroll
-      for (int p = 0; p < PB; ++p)
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (k0 + k < S) v[p] += t[p][k];
-    }
-#pragma unroll
-    for (int p = 0; p < PB; ++p) {
-      const int row = tid / QR + RP * (p0_ + p);
-      if (p0_ + p < NP && m0 + row < a.M) finish(m0 + row, v[p]);
-    }
-  }
+  pfk_close<MT, CT, NG, EPI>(a, acc, m0, n0, sp, S, tile, ntile, last_flag);
 }
 
 template <int QT0, int QT1, int MT, int CT, int NG, int EPI>

@@ -955,6 +955,9 @@ void LayeredDecoder::tune() {
       if (D.rp && M <= pf_max_ctx_) go(cfull_, D.rp, w.ukv, D.qn + D.gn, D.rp, GEPI_STORE16, nullptr, D.qn + D.gn, kv_, act);
     }
   }
+  for (GemmQArgs& g : launches) {
+    g.ws = e_.gk_ws_; g.ws_bytes = e_.gk_ws_bytes_; g.cnt = e_.gk_cnt_; g.cnt_len = e_.gk_cnt_len_;
+  }
   gemm_pf_autotune(launches, e_.stream_);
   HIP_CHECK(hipMemsetAsync(h16_, 0, (size_t)step_rows_ * dp_ * 2, e_.stream_));
   HIP_CHECK(hipStreamSynchronize(e_.stream_));

@@ -1731,6 +1731,37 @@ def test_gemm_pfk(E, monkeypatch, tile, fmt, K, S):
         assert rel < 2 * 2.0 ** -9 / 3 ** 0.5 + K * 2.0 ** -24, rel
 
 
+@pytest.mark.parametrize("tile", PFK_TILES)
+@pytest.mark.parametrize("K,S", [(128, 1), (640, 1), (640, 2), (1408, 3), (2048, 4)])
+@pytest.mark.parametrize("epi", ["store", "accum", "swiglu", "store16"])
+def test_gemm_pfk_bf16(E, monkeypatch, tile, K, S, epi):
+    """bf16 weights: one slot of 128 k to many, slices of unlike length, rows at and past a tile's edge, pitches of their own.  The
+    products are exact, so the bound is the sums' (K 2^-24), and of a bf16 result the rounding, half an ulp evenly spread, doubled."""
+    bm, bn = (int(v) for v in tile.split("x"))
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
+    N = 256
+    m, W = qmat(E, GGMLType.BF16, N, K, seed=5, std=0.05)
+    e = {"store": E.GEPI_STORE, "accum": E.GEPI_ACCUM, "swiglu": E.GEPI_SWIGLU_BF16, "store16": E.GEPI_STORE16}[epi]
+    half, cols = epi in ("swiglu", "store16"), N // 2 if epi == "swiglu" else N
+    for M in (33, bm, 2 * bm - 3):
+        assert list(E.gemm_pf_plan([m], M, e, 0)) == [bm, bn, S]
+        x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+        A = torch.full((M, K + 8), float("nan"), dtype=torch.bfloat16)
+        A[:, :K] = x
+        A, C = A.cuda(), torch.full((M + 1, cols + 4), 2.0, device="cuda", dtype=torch.bfloat16 if half else torch.float32)
+        for _ in range(2):  # (the tickets are armed again)
+            E.gemm_q(A.data_ptr(), K + 8, [m], M, 0 if half else C.data_ptr(), C.data_ptr() if half else 0, cols + 4, e, stream(), 0)
+        torch.cuda.synchronize()
+        z = x.double() @ W.double().T
+        ref = torch.nn.functional.silu(z[:, 0::2]) * z[:, 1::2] if epi == "swiglu" else z
+        got = C[:M, :cols].cpu().double()
+        got = (got - 2) / 2 if epi == "accum" else got
+        assert bool((C[:, cols:] == 2).all()) and bool((C[M] == 2).all())
+        rel = float((got - ref).norm() / ref.norm())
+        assert rel < K * 2.0 ** -24 + (2 * 2.0 ** -9 / 3 ** 0.5 if half else 2.0 ** -20), rel
+
+
 @pytest.mark.parametrize("tile", ["64x-32", "96x-64", "160x-128"])
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("S", [1, 3])

@@ -43,6 +43,7 @@ HOT = [
     "aios::gemm_pf4t_kernel<*",
     "aios::gemm_pf4sk_kernel<*",
     "aios::gemm_pfk_kernel<*",
+    "aios::gemm_pfkb_kernel<*",
     "aios::sample_kernel*",
     "aios::get_rows_step_kernel*",
     "aios::latent_prep_kernel*",
