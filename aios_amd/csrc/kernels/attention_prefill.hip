@@ -78,26 +78,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, half = lane >> 5;
-  // Causal balance: workgroup L (dispatch order, x fastest) and L + W/2 share a CU once the grid
-  // fills every CU twice (the second pass lands on the CUs in the same order), so the first half
-  // takes query blocks heaviest-first and the second half lightest-first: every CU gets blocks qb and
-  // nx-1-qb, nx + 1 key tiles in all.  (Before, both of a CU's workgroups had the same qb: at 2k
-  // tokens one CU did 64 tiles while the average was 33.)  Odd KV-head counts keep heaviest-first.
-  const int nx = gridDim.x, ny = gridDim.y;
-  int qb, kvh;
-  if ((ny & 1) == 0) {
-    const int L = blockIdx.y * nx + blockIdx.x, W2 = nx * ny / 2;
-    if (L < W2) {
-      qb = nx - 1 - L % nx;
-      kvh = L / nx;
-    } else {
-      qb = (L - W2) % nx;
-      kvh = ny / 2 + (L - W2) / nx;
-    }
-  } else {
-    qb = nx - 1 - blockIdx.x;
-    kvh = blockIdx.y;
-  }
+  // An XCD works on as few KV heads as there are for it, so their K and V stay in its L2: m XCDs share a list of hx heads' (query
+  // block, run) items, the longest first.  Causal balance: where the list fills its CUs twice at most, what comes after the
+  // first 32 m items (a CU's second workgroup) goes from the shortest up, so every CU gets about the same number of tiles.
+  // us, heads over all XCDs -> so: 1852 tokens behind 2048, 32 / 8 heads of 128 127 -> 112; 300 behind 6000, fp8, six runs 53 -> 49;
+  // 1500 tokens, 32 / 4 heads of 64 35 -> 27.
+  const int nx = (a.T + BQ - 1) / BQ, ny = a.n_kv_heads;
+  const int m = ny % 8 == 0 ? 1 : (8 % ny == 0 ? 8 / ny : 8), hx = ny % 8 == 0 ? ny / 8 : (8 % ny == 0 ? 1 : ny);
+  const int xcd = blockIdx.x & 7, W = hx * nx * a.ns, w = (blockIdx.x >> 3) * m + xcd % m;
+  if (w >= W) return;
+  const int item = w < 32 * m || W > 64 * m ? w : W - 1 - (w - 32 * m);
+  const int kvh = xcd / m * hx + item % hx, run_z = item / hx % a.ns, qb = nx - 1 - item / hx / a.ns;
   const int T = a.T, start = a.start;
   const int t0 = qb * BQ;
   // this lane's query row (column of S^T / O^T)
@@ -137,7 +128,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const uint8_t* kc = (const uint8_t*)a.k_cache + (size_t)kvh * KV_BLOCK * HD * ES;
   const uint8_t* vc = (const uint8_t*)a.v_cache + (size_t)kvh * KV_BLOCK * HD * ES;
   // this run's tiles [kt0, kt1) of the block's (a.ns == 1: all of them)
-  const FpRun run = fp_run(start, T, t0, BQ, a.ns, blockIdx.z);
+  const FpRun run = fp_run(start, T, t0, BQ, a.ns, run_z);
   const int kt0 = run.kt0, kt1 = run.kt1;
   if (kt0 >= kt1) return;  // (uniform; the combine counts the runs the same way)
   const int klim = min(qpos, kt1 * FP_KT - 1);  // keys this lane sees in this run
@@ -299,7 +290,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   // ---- O^T[dim][row], dim = 32 i + (r&3) + 8 (r>>2) + 4 half
   if (a.ns > 1) {  // this run's part: O, row max and row sum in fp32
     if (qvalid) {
-      const size_t pr = ((size_t)blockIdx.z * T + tq) * a.n_heads + h;
+      const size_t pr = ((size_t)run_z * T + tq) * a.n_heads + h;
       float* op = a.ws + pr * HD;
 #pragma unroll
       for (int i = 0; i < OT; ++i)
@@ -387,7 +378,9 @@ template <int HD, bool F8>
 static void prefill_hd(AttnPrefillArgs a, int G, hipStream_t st) {
   const int BQ = 128 / G;
   a.ns = prefill_runs(a, BQ);
-  dim3 grid((a.T + BQ - 1) / BQ, a.n_kv_heads, a.ns);
+  const int ny = a.n_kv_heads, m = ny % 8 == 0 ? 1 : (8 % ny == 0 ? 8 / ny : 8), hx = ny % 8 == 0 ? ny / 8 : (8 % ny == 0 ? 1 : ny);
+  const int W = hx * ((a.T + BQ - 1) / BQ) * a.ns;
+  const dim3 grid(8 * ((W + m - 1) / m));  // (the kernel's lists, one place in turn on each XCD)
   const size_t lds = (size_t)2 * FP_KT * ((HD + 8) + (HD + 32)) * sizeof(bf16_t);  // two K|V tile buffers
   switch (G) {
     case 1: hipLaunchKernelGGL((attn_prefill_kernel<HD, 1, F8>), grid, dim3(256), lds, st, a); break;
