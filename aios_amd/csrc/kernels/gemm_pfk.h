@@ -12,14 +12,15 @@
 // waves a SIMD meet at one barrier); beside the loop ~3 us to the first data and 5 us in which four partial tiles
 // meet.  Weights and X from memory, us, column-split tiles -> this:
 //   28672 x 4096 Q4_K SwiGLU, 64 / 130 / 300 rows  40 -> 29, 68 -> 46, 131 -> 91     6144 x 4096, 130 / 711 rows  40 -> 18, 78 -> 48
-//   4096 x 4096 Q4_K, 130 / 300 / 711 rows  22 -> 15, 37 -> 22, 53 -> 40             4096 x 14336 Q4_K, 130 / 300 rows  40 -> 31, 102 -> 51
-//   4096 x 14336 Q6_K, 130 rows  47 -> 39    2048 x 5632 Q4_K, 64 rows  37 -> 10     11264 x 2048 Q4_K SwiGLU, 64 rows  20 -> 11
+//   4096 x 4096 Q4_K, 130 / 300 / 700 rows  22 -> 15, 37 -> 20, 53 -> 33             4096 x 14336 Q4_K, 130 / 300 rows  40 -> 30, 102 -> 46
+//   4096 x 14336 Q6_K, 130 rows  47 -> 35    2048 x 5632 Q4_K, 64 rows  37 -> 10     11264 x 2048 Q4_K SwiGLU, 64 rows  20 -> 11
 // 256 x 256 tiles (gemm_pf.h) stay the faster ones for wide products from ~700 rows (28672 x 4096, 2048 rows: 444 / 533).
 //
 // Not better: one wave a SIMD (320 accumulators do not fit beside AGPRs; 128 rows 58 us); requests in one burst behind the barrier
 // (they hold each wave until the address unit has taken them: 48 to 49 us of 46); slices of a tile on different XCDs (4096 x 14336 33 of 31).
 #pragma once
 #include "gemm_pf.h"
+#include "skinny_epi.h"
 
 namespace aios {
 
@@ -80,20 +81,23 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
   auto slab = [&](int k) __attribute__((always_inline)) {  // byte of slice k's partial sums of this tile
     return (uint32_t)(k * ntile + tile) * (uint32_t)(BM * BN * 4);
   };
-  auto finish = [&](int m, gf32x4 v) __attribute__((always_inline)) {
-    if constexpr (EPI == GEPI_SWIGLU_BF16) {
-      *(uint32_t*)(a.C16 + (size_t)m * a.ldc + (n >> 1)) =
-          (uint32_t)f32_to_bf16(glu_act(v[0], a.act) * v[1]) | ((uint32_t)f32_to_bf16(glu_act(v[2], a.act) * v[3]) << 16);
-    } else if constexpr (EPI == GEPI_STORE16) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = store16_val(a, n + e, v[e]);
-      *(uint2*)(a.C16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]));
-    } else {
-      float* cp = a.C + (size_t)m * a.ldc + n;
-      if constexpr (EPI == GEPI_ACCUM) v += *(const gf32x4*)cp;
-      *(gf32x4*)cp = v;
-    }
+  // (the residual is requested ahead: a load behind a store to what may be the same place would wait for it, row by row.  us, so ->
+  // ahead: 4096 x 4096 Q4_K, 300 / 700 rows 22 -> 20, 40 -> 33; 4096 x 14336, 300 rows Q4_K 51 -> 46, Q6_K 63 -> 56; 130 rows Q6_K 39 -> 35)
+  auto residual = [&](int row) __attribute__((always_inline)) {
+    gf32x4 c = {};
+    if constexpr (EPI == GEPI_ACCUM) c = *(const gf32x4*)(a.C + (size_t)min(m0 + row, a.M - 1) * a.ldc + n);
+    return c;
   };
+  auto finish = [&](int row, gf32x4 v, gf32x4 res) __attribute__((always_inline)) {
+    sk_finish<EPI>(a, nullptr, m0 + row, n, v, (const float4*)&res);
+  };
+  gf32x4 res[MT][32 / RP];
+  if (S == 1) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int k = 0; k < 32 / RP; ++k) res[i][k] = residual(32 * i + tid / QR + RP * k);
+  }
 #pragma unroll
   for (int i = 0; i <= MT; ++i) {
     pf_barrier();
@@ -119,7 +123,7 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
       for (int k = 0; k < 32 / RP; ++k) {
         const int row = 32 * (i - 1) + tid / QR + RP * k;
         if (m0 + row >= a.M) continue;
-        if (S == 1) finish(m0 + row, v[k]);
+        if (S == 1) finish(row, v[k], res[i - 1][k]);
         else
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(gu32x4, v[k]), ws, slab(sp) + ((uint32_t)row * BN + 4 * q) * 4, 0, 16 /* sc1 */);
       }
@@ -144,16 +148,20 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
   constexpr int NP = BM / RP, PB = NP < 8 ? NP : 8;  // rows of a lane; so many at a time
 #pragma unroll
   for (int p0_ = 0; p0_ < NP; p0_ += PB) {
-    gf32x4 v[PB];
+    gf32x4 v[PB], c[PB];
 #pragma unroll
-    for (int p = 0; p < PB; ++p) v[p] = gf32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < S; k0 += 4) {  // four slabs' loads in flight (past the last: read again, not added)
+    for (int p = 0; p < PB; ++p) {
+      v[p] = gf32x4{0.f, 0.f, 0.f, 0.f};
+      c[p] = residual(tid / QR + RP * (p0_ + p));
+    }
+    for (int k0 = 0; k0 < S; k0 += 4) {  // four slabs' loads in flight
       gf32x4 t[PB][4];
 #pragma unroll
       for (int p = 0; p < PB; ++p) {
         const int row = min(tid / QR + RP * min(p0_ + p, NP - 1), a.M - 1 - m0);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) t[p][k] = *(const gf32x4*)((const uint8_t*)a.ws + slab(min(k0 + k, S - 1)) + ((uint32_t)row * BN + 4 * q) * 4);
+        for (int k = 0; k < 4; ++k)
+          if (k0 + k < S) t[p][k] = *(const gf32x4*)((const uint8_t*)a.ws + slab(k0 + k) + ((uint32_t)row * BN + 4 * q) * 4);
       }
 #pragma unroll
       for (int p = 0; p < PB; ++p)
@@ -164,7 +172,7 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
 #pragma unroll
     for (int p = 0; p < PB; ++p) {
       const int row = tid / QR + RP * (p0_ + p);
-      if (p0_ + p < NP && m0 + row < a.M) finish(m0 + row, v[p]);
+      if (p0_ + p < NP && m0 + row < a.M) finish(row, v[p], c[p]);
     }
   }
 }
