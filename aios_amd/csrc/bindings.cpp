@@ -752,6 +752,13 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       },
       py::arg("segs"), py::arg("M"), py::arg("epi"), py::arg("ksplit") = 0, py::arg("more") = py::dict());
   m.def(
+      "gemm_pf_fuses",
+      [](std::vector<PyQMatrix*> segs, int M, int epi, uintptr_t A, int lda, uintptr_t C, int ldc, const py::dict& more) {
+        GemmQArgs a = gemm_q_args(segs, M, epi, 0, more);
+        a.A = (const bf16_t*)A; a.lda = lda; a.C = (float*)C; a.ldc = ldc;
+        return gemm_pf_fuses(a);
+      });
+  m.def(
       "gemm_pf_plan",
       [](std::vector<PyQMatrix*> segs, int M, int epi, int ksplit) {
         GemmQArgs a;

@@ -714,9 +714,9 @@ void Engine::finalize() {
           const int Gs = std::min(G, 64);
           gm_nparts_ = d / 16;
           gm_xn16_ = (bf16_t*)dmalloc((size_t)Gs * d * 2);
-          gm_npart_ = fbuf((size_t)Gs * gm_nparts_);
           ws += (size_t)Gs * d * 2;
         }
+        gm_npart_ = fbuf(std::max((size_t)std::min(G, 64) * gm_nparts_, (size_t)G * (d / 64)));  // (... and of the longer ones)
       }
       if (Bm >= 2) {
         dec_a16_ = (bf16_t*)dmalloc((size_t)Bm * std::max(d, qd) * 2);
@@ -1273,34 +1273,50 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
     // GEMM, kernels/gemm_pf.hip, with the plain epilogues)
     const bool sh = short_fuse && !tp && n <= 32;
     const bool fnp = sh && gm_nparts_ > 0;
+    // longer chunks: the same fusions where both products of a norm, or the QKV product, run on tiles with K over the waves
+    const bool lf = nrm_fuse_ && !tp && n > 32 && d % 256 == 0;
+    auto fuses = [&](GemmQArgs q) {
+      q.ws = gk_ws_; q.ws_bytes = gk_ws_bytes_; q.cnt = gk_cnt_; q.cnt_len = gk_cnt_len_;
+      return gemm_pf_fuses(q);
+    };
     for (int i = 0; i < n; ++i) hp[i] = start_pos + r0 + i;
     HIP_CHECK(hipMemcpyAsync(gm_tokens_, tokens.data() + r0, n * 4, hipMemcpyHostToDevice, stream_));
     HIP_CHECK(hipMemcpyAsync(gm_pos_, hp.data(), n * 4, hipMemcpyHostToDevice, stream_));
     HIP_CHECK(hipMemcpyAsync(gm_slot_, hs.data(), n * 4, hipMemcpyHostToDevice, stream_));
     launch_get_rows(tok_embd_.w, gm_tokens_, n, gm_x_, d, 1.f, stream_);
+    bool down_normed = false;
     for (int l = 0; l < cfg_.n_layers; ++l) {
       const LayerW& L = layers_[l];
       bf16_t* kc = kv_layer(k_cache_, l);
       bf16_t* vc = kv_layer(v_cache_, l);
       // split-RMSNorm consumer / producer (as in layer_decode_gemm, on this chunk's rows)
+      // (longer chunks: parts of 64 columns, the operand in gm_a16_, which nothing else holds then)
       auto nrm_in = [&](GemmQArgs& g) {
-        g.A = gm_xn16_; g.nrm_in = gm_npart_; g.nrm_parts = gm_nparts_; g.nrm_eps = cfg_.norm_eps;
+        g.nrm_in = gm_npart_; g.nrm_eps = cfg_.norm_eps;
+        g.nrm_parts = fnp ? gm_nparts_ : d / 64;
+        if (fnp) g.A = gm_xn16_;
       };
       auto nrm_out = [&](GemmQArgs& g, const float* g_next) {
-        g.epi = GEPI_ACCUM_NORM; g.nrm_g = g_next; g.nrm_out16 = gm_xn16_; g.nrm_part = gm_npart_;
-        g.nrm_parts = gm_nparts_;
+        g.epi = GEPI_ACCUM_NORM; g.nrm_g = g_next; g.nrm_part = gm_npart_;
+        g.nrm_out16 = fnp ? gm_xn16_ : gm_a16_;
+        g.nrm_parts = fnp ? gm_nparts_ : d / 64;
       };
-      if (!(fnp && l > 0)) launch_rmsnorm_bf16(gm_x_, d, L.attn_norm, gm_a16_, d, n, d, cfg_.norm_eps, stream_);
-      GemmQArgs g;
-      std::memset(&g, 0, sizeof(g));
-      g.A = gm_a16_; g.lda = d; g.M = n; g.K = d;
-      if (fnp && l > 0) nrm_in(g);
-      g.nseg = 3;
-      g.seg[0] = L.wq.w; g.seg[1] = L.wk.w; g.seg[2] = L.wv.w;
-      g.seg_n0[0] = 0; g.seg_n0[1] = qd; g.seg_n0[2] = qd + kvd;
-      g.N = ldqkv; g.C = gm_qkv_; g.ldc = ldqkv; g.epi = GEPI_STORE;
-      // the RoPE / KV-cache epilogue: short chunks (ring / skinny GEMMs); the prefill GEMM's chunks
-      // (>= 33 rows) only with AIOS_PREFILL_QKV_EPI=1 -- it needs S = 1 plans, and at 2048 tokens
+      auto qkv_of = [&](const LayerW& w) {
+        GemmQArgs g;
+        std::memset(&g, 0, sizeof(g));
+        g.A = gm_a16_; g.lda = d; g.M = n; g.K = d;
+        g.nseg = 3;
+        g.seg[0] = w.wq.w; g.seg[1] = w.wk.w; g.seg[2] = w.wv.w;
+        g.seg_n0[0] = 0; g.seg_n0[1] = qd; g.seg_n0[2] = qd + kvd;
+        g.N = ldqkv; g.C = gm_qkv_; g.ldc = ldqkv; g.epi = GEPI_STORE;
+        return g;
+      };
+      const bool normed = (fnp && l > 0) || down_normed;  // the residual GEMM before left bf16(x g) and its rows' sums
+      if (!normed) launch_rmsnorm_bf16(gm_x_, d, L.attn_norm, gm_a16_, d, n, d, cfg_.norm_eps, stream_);
+      GemmQArgs g = qkv_of(L);
+      if (normed) nrm_in(g);
+      // the RoPE / KV-cache epilogue: short chunks (the decode GEMMs) and tiles with K over the waves; the prefill GEMM's others
+      // only with AIOS_PREFILL_QKV_EPI=1 -- they need S = 1 plans for it, and at 2048 tokens
       // the QKV GEMM then took 212.7 us against 115.7 (split-K) + 32 us of qkv_post (64 tokens:
       // 5.77 vs 4.6 ms per prompt), profiles/prefill_r5.txt
       const bool qepi_ok = !cfg_.qk_norm && !cfg_.rope_neox && !L.bqkv && rope_cs_ && !tp;
@@ -1313,7 +1329,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
         q.q_out = gm_q_; q.k_cache = kc; q.v_cache = vc;
         kv_write_args(q, l);
         static const int pf_qkv = [] { const char* e = std::getenv("AIOS_PREFILL_QKV_EPI"); return e ? std::atoi(e) : 0; }();
-        qepi = sh || (pf_qkv && gemm_pf_serves(q));
+        qepi = sh || (n > 32 && fuses(q)) || (pf_qkv && gemm_pf_serves(q));
         if (qepi) g = q;
       }
       gemm(g);
@@ -1341,20 +1357,31 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
       std::memset(&g, 0, sizeof(g));
       g.A = gm_attn16_; g.lda = qd; g.M = n; g.K = qd; g.nseg = 1; g.seg[0] = L.wo.w; g.N = d; g.ldc = d;
       if (tp) { g.C = gm_part_; g.epi = GEPI_STORE; } else { g.C = gm_x_; g.epi = GEPI_ACCUM; }
-      if (fnp) nrm_out(g, L.ffn_norm);
+      GemmQArgs gu;
+      std::memset(&gu, 0, sizeof(gu));
+      gu.A = gm_a16_; gu.lda = d; gu.M = n; gu.K = d; gu.nseg = 1; gu.seg[0] = L.wgu.w; gu.N = 2 * ff;
+      gu.C16 = gm_ff16_; gu.ldc = ff; gu.epi = GEPI_SWIGLU_BF16;
+      // this product with the norm of its output, where it and the next one, which reads that, both take their part
+      auto pair = [&](const GemmQArgs& out, const float* gain, GemmQArgs in) {
+        GemmQArgs o = out;
+        nrm_out(o, gain);
+        nrm_in(in);
+        return lf && fuses(o) && fuses(in);
+      };
+      const bool o_normed = fnp || pair(g, L.ffn_norm, gu);
+      if (o_normed) nrm_out(g, L.ffn_norm);
       gemm(g);
       if (tp) allreduce(gm_part_, (size_t)n * d, gm_x_);
       // FFN
-      if (!fnp) launch_rmsnorm_bf16(gm_x_, d, L.ffn_norm, gm_a16_, d, n, d, cfg_.norm_eps, stream_);
-      std::memset(&g, 0, sizeof(g));
-      g.A = gm_a16_; g.lda = d; g.M = n; g.K = d; g.nseg = 1; g.seg[0] = L.wgu.w; g.N = 2 * ff;
-      g.C16 = gm_ff16_; g.ldc = ff; g.epi = GEPI_SWIGLU_BF16;
-      if (fnp) nrm_in(g);
-      gemm(g);
+      if (!o_normed) launch_rmsnorm_bf16(gm_x_, d, L.ffn_norm, gm_a16_, d, n, d, cfg_.norm_eps, stream_);
+      if (o_normed) nrm_in(gu);
+      gemm(gu);
       std::memset(&g, 0, sizeof(g));
       g.A = gm_ff16_; g.lda = ff; g.M = n; g.K = ff; g.nseg = 1; g.seg[0] = L.wdown.w; g.N = d; g.ldc = d;
       if (tp) { g.C = gm_part_; g.epi = GEPI_STORE; } else { g.C = gm_x_; g.epi = GEPI_ACCUM; }
-      if (fnp && l + 1 < cfg_.n_layers) nrm_out(g, layers_[l + 1].attn_norm);  // (lm_head normalises its row)
+      // (the last layer: lm_head normalises its row)
+      down_normed = l + 1 < cfg_.n_layers && pair(g, layers_[l + 1].attn_norm, qkv_of(layers_[l + 1]));
+      if (down_normed || (fnp && l + 1 < cfg_.n_layers)) nrm_out(g, layers_[l + 1].attn_norm);
       gemm(g);
       if (tp) allreduce(gm_part_, (size_t)n * d, gm_x_);
     }

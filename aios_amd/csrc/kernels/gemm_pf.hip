@@ -142,6 +142,7 @@ static bool pf_plan_ok(const GemmQArgs& a, const PfPlan& p, bool bf) {
   for (const auto& t : PF_TILES) tile = tile || (t.bm == p.bm && t.bn == p.bn);
   if (!tile || !pf_tile_ok(a, std::abs(p.bn))) return false;
   if (p.bn < 0) return bf ? pfkb_serves(a, p.bm, -p.bn, p.s) : pfk_serves(a, p.bm, -p.bn, p.s);
+  if (a.nrm_in || a.epi == GEPI_ACCUM_NORM || (a.epi == GEPI_QKV && (a.kv_fp8 || p.s != 1))) return false;
   if (p.s < 0) return pf_sk_ok(a, p.bm, p.bn, bf);
   if (p.s == 0 || (p.s > 1 && (pf_no_split(a) || a.K / 64 / p.s < 2))) return false;
   return bf || p.bn != 256 || a.K / 256 / p.s >= 1;  // (pf8c slices whole 256-blocks)
@@ -169,12 +170,18 @@ static PfPlan pf_model_plan(const GemmQArgs& a, bool bf, bool s1_only);
 static PfPlan pf_plan(const GemmQArgs& a, bool bf) {
   if (!std::getenv("AIOS_GEMM_PF_TILE") && !std::getenv("AIOS_GEMM_PF_SPLIT") && a.ksplit <= 0) {
     std::lock_guard<std::mutex> g(pf_mu);
-    const bool s1 = a.epi == GEPI_QKV || pf_deterministic();  // (the best plan without split partials)
-    GemmQArgs b = a;
+    GemmQArgs b = a;  // (the plans of the plain epilogues)
     if (a.epi == GEPI_QKV) b.epi = GEPI_STORE;
-    const auto& plans = s1 ? pf_tuned_s1() : pf_tuned();
-    auto it = plans.find(pf_key(b));
-    if (it != plans.end() && pf_plan_ok(a, it->second, bf)) return it->second;
+    if (a.epi == GEPI_ACCUM_NORM) b.epi = GEPI_ACCUM;
+    const PfKey key = pf_key(b);
+    auto at = [&](const std::map<PfKey, PfPlan>& plans) {
+      const auto it = plans.find(key);
+      return it != plans.end() && pf_plan_ok(a, it->second, bf) ? it->second : PfPlan();
+    };
+    PfPlan p;
+    if (!pf_deterministic()) p = at(pf_tuned());
+    if (!p.bm && (pf_deterministic() || a.epi == GEPI_QKV)) p = at(pf_tuned_s1());  // (the best without split partials)
+    if (p.bm) return p;
   }
   return pf_model_plan(a, bf, false);
 }
@@ -214,7 +221,6 @@ static PfPlan pf_model_plan(const GemmQArgs& a, bool bf, bool s1_only) {
 static bool pf_eligible(const GemmQArgs& a);
 static bool pf_run(const GemmQArgs& a, const PfPlan& p, hipStream_t st) {
   const int qt0 = a.seg[0].qtype, qt1 = a.seg[a.nseg - 1].qtype;
-  if (p.s != 1 && a.epi == GEPI_QKV) return false;  // (plans keep S = 1 for it; a pinned split declines)
   if (p.bn < 0) return qt0 == QT_BF16 ? pfkb_run(a, p.bm, -p.bn, p.s, st) : pfk_run(a, p.bm, -p.bn, p.s, st);
   if (p.s != 1 && a.epi == GEPI_STORE)
     launch_zero_rows(a.C, a.ldc, a.M, a.N, st);  // (a kernel: the launch may be captured)
@@ -244,13 +250,13 @@ bool launch_gemm_pf(const GemmQArgs& a, hipStream_t st) {
 static bool pf_eligible(const GemmQArgs& a) {
   if (a.nseg < 1 || a.M < 1) return false;
   if (a.epi != GEPI_STORE && a.epi != GEPI_ACCUM && a.epi != GEPI_SWIGLU_BF16 && a.epi != GEPI_QKV &&
-      a.epi != GEPI_STORE16)
+      a.epi != GEPI_STORE16 && a.epi != GEPI_ACCUM_NORM)
     return false;
   if (a.epi == GEPI_STORE16 && (!a.C16 || a.seg[0].qtype != QT_BF16)) return false;
-  if (a.epi == GEPI_QKV && (a.kv_fp8 || a.col0 != 0 || !a.q_out || !a.k_cache || !a.v_cache || !a.pos || !a.rope_cs ||
+  if (a.epi == GEPI_QKV && (a.col0 != 0 || !a.q_out || !a.k_cache || !a.v_cache || !a.pos || !a.rope_cs ||
                             a.head_dim % 2 || a.N != a.q_dim + 2 * a.kv_dim))
     return false;
-  if (a.nrm_in || a.lda % 8 || ((uintptr_t)a.A & 15)) return false;
+  if (a.lda % 8 || ((uintptr_t)a.A & 15)) return false;
   const int qt0 = a.seg[0].qtype, qt1 = a.seg[a.nseg - 1].qtype;
   for (int s = 0; s + 1 < a.nseg; ++s)
     if (a.seg[s].qtype != qt0) return false;
@@ -263,6 +269,7 @@ static bool pf_eligible(const GemmQArgs& a) {
                   (qt0 == QT_Q8_0 && qt1 == QT_Q8_0);
   if (!bf && !kq) return false;
   if (a.epi == GEPI_SWIGLU_BF16 && (!a.C16 || a.nseg != 1)) return false;
+  if (a.epi == GEPI_ACCUM_NORM && a.nseg != 1) return false;
   if (a.epi != GEPI_SWIGLU_BF16 && a.epi != GEPI_QKV && a.epi != GEPI_STORE16 && !a.C) return false;
   return true;
 }
@@ -410,7 +417,13 @@ void gemm_pf_import(const std::vector<int>& v) {
 bool gemm_pf_serves(const GemmQArgs& a) {
   if (!pf_env("AIOS_GEMM_PF", 1) || a.M < pf_env("AIOS_GEMM_PF_MIN_M", 33) || !pf_eligible(a)) return false;
   const PfPlan p = pf_plan(a, a.seg[0].qtype == QT_BF16);
-  return p.bm != 0 && !(p.s != 1 && a.epi == GEPI_QKV);
+  return p.bm != 0;
+}
+
+// ... on tiles with K over the waves: those take GEPI_QKV with any plan, GEPI_ACCUM_NORM and nrm_in (a part per 64 columns)
+bool gemm_pf_fuses(const GemmQArgs& a) {
+  if (!pf_env("AIOS_GEMM_PF", 1) || a.M < pf_env("AIOS_GEMM_PF_MIN_M", 33) || !pf_eligible(a)) return false;
+  return pf_plan(a, a.seg[0].qtype == QT_BF16).bn < 0;
 }
 
 // the plan the launcher would pick (bindings / tools)

@@ -26,6 +26,47 @@ namespace aios {
 
 constexpr int PFK_LDS = 160 * 1024 - 64;  // dynamic LDS of these kernels at most: their last_flag lies beside it
 
+// The fused RMSNorm's consumer: the scales of the tile's rows from the producer's sums of squares (a part per 64 columns), eight
+// lanes a row, added up in a fixed order.  load() requests, done() adds up, put() writes them to LDS.
+template <int BM, int NW>
+struct PfkRows {
+  static constexpr int KI = (BM / NW + 7) / 8;  // rows of a lane's eighth
+  gf32x4 v[KI][2];
+  float inv[KI];
+  __device__ __forceinline__ const gf32x4* at(const GemmQArgs& a, int m0, int wave, int lane, int k, int j) const {
+    const int row = min(m0 + wave * (BM / NW) + 8 * k + (lane >> 3), a.M - 1);
+    return (const gf32x4*)(a.nrm_in + (size_t)row * a.nrm_parts + j);
+  }
+  __device__ __forceinline__ void load(const GemmQArgs& a, int m0, int wave, int lane) {
+#pragma unroll
+    for (int k = 0; k < KI; ++k)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        v[k][j] = gf32x4{0.f, 0.f, 0.f, 0.f};
+        const int p = 32 * j + 4 * (lane & 7);
+        if (p < a.nrm_parts) v[k][j] = *at(a, m0, wave, lane, k, p);
+      }
+  }
+  __device__ __forceinline__ void done(const GemmQArgs& a, int m0, int wave, int lane) {
+#pragma unroll
+    for (int k = 0; k < KI; ++k) {
+      gf32x4 t = v[k][0] + v[k][1];
+      for (int p = 64 + 4 * (lane & 7); p < a.nrm_parts; p += 32) t += *at(a, m0, wave, lane, k, p);
+      float s = (t[0] + t[1]) + (t[2] + t[3]);
+#pragma unroll
+      for (int o = 1; o < 8; o <<= 1) s += __shfl_xor(s, o, 64);
+      inv[k] = rsqrtf(s / (float)a.K + a.nrm_eps);
+    }
+  }
+  __device__ __forceinline__ void put(int wave, int lane, float* inv_s) const {
+#pragma unroll
+    for (int k = 0; k < KI; ++k) {
+      const int r = 8 * k + (lane >> 3);
+      if ((lane & 7) == 0 && r < BM / NW) inv_s[wave * (BM / NW) + r] = inv[k];
+    }
+  }
+};
+
 template <int QT, int MT, int CT, int NG>
 struct PfkLayout {
   static constexpr bool Q6 = QT == QT_Q6_K;
@@ -40,8 +81,10 @@ struct PfkLayout {
   static constexpr int NW = 4 * NG, NX = 2 * MT / NG;  // waves; DMA requests a wave, per X slot
   static constexpr int PC = 4 * CT, PR = 2 * CT;       // pieces of a W block: codes, records (high bits); a wave's (of few: some twice)
   static constexpr int NC = PC / NW, NR = PR > NW ? PR / NW : 1, NH = Q6 ? NR : 0, ND = Q6 ? 1 : 0, NWP = NC + NR + NH + ND;
-  static constexpr int RED_BYTES = 2 * 4 * 32 * BN * 4;  // two row tiles of four partial sums
-  static constexpr int TOTAL = OFF_W + NWB * WB > RED_BYTES ? OFF_W + NWB * WB : RED_BYTES;
+  static constexpr int RED_BYTES = 2 * 4 * 32 * BN * 4 + BM * 4;  // two row tiles of four partial sums, the rows' scales
+  // the rows' scales: behind the slots where there is room, else behind the partial sums once the loop is done
+  static constexpr bool KEEP = OFF_W + NWB * WB + BM * 4 > PFK_LDS;
+  static constexpr int USED = OFF_W + NWB * WB + (KEEP ? 0 : BM * 4), TOTAL = USED > RED_BYTES ? USED : RED_BYTES;
   static_assert(NWB < 2 || TOTAL <= PFK_LDS, "pfk LDS");
 };
 
@@ -61,15 +104,33 @@ __device__ __forceinline__ void pfk_dma4(const void* base, uint32_t off, uint32_
                : "memory", "m0");
 }
 
+// host: whether the epilogue's operands fit the stores of these kernels (bn: columns of a tile).  16-byte stores to C, 8-byte ones to C16 and
+// 4-byte ones of a gated product; a part of the split RMSNorm per 64 columns, on either side
+inline bool pfk_epi_ok(const GemmQArgs& a, int bn) {
+  auto off = [](const void* p, int n) { return ((uintptr_t)p & (n - 1)) != 0; };
+  if (a.nrm_in && (a.K % 256 || a.nrm_parts != a.K / 64 || off(a.nrm_in, 16))) return false;
+  switch (a.epi) {
+    case GEPI_STORE: case GEPI_ACCUM: return a.ldc % 4 == 0 && !off(a.C, 16);
+    case GEPI_ACCUM_NORM:
+      return a.ldc % 4 == 0 && !off(a.C, 16) && bn >= 64 && a.nrm_g && !off(a.nrm_g, 16) && a.nrm_out16 && !off(a.nrm_out16, 8) && a.nrm_part &&
+             a.nrm_parts == a.N / 64 && (!a.bias16 || !off(a.bias16, 16));
+    case GEPI_SWIGLU_BF16: return a.ldc % 2 == 0 && !off(a.C16, 4);
+    case GEPI_STORE16: return a.ldc % 4 == 0 && !off(a.C16, 8);
+    case GEPI_QKV: return !off(a.q_out, 8) && a.head_dim % 2 == 0 && a.q_dim % 2 == 0 && a.kv_dim % 2 == 0;
+    default: return false;
+  }
+}
+
 // ---- end of a tile: the four partial sums of every output, the slices of K, the epilogue
-template <int MT, int CT, int NG, int EPI>
+template <int MT, int CT, int NG, int EPI, bool KEEP, int TOTAL>
 __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&acc)[MT][CT / NG], int m0, int n0, int sp, int S, int tile,
-                                          int ntile, int& last_flag) {
+                                          int ntile, int& last_flag, const PfkRows<32 * MT, 4 * NG>& rows) {
   constexpr int BM = 32 * MT, BN = 32 * CT, NW = 4 * NG, CW = CT / NG;
   extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem0[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wv = wave & 3, cg = wave >> 2;
   const int r32 = lane & 31, h = lane >> 5;
+  float* inv_s = (float*)(pf_smem0 + (KEEP ? 2 * 4 * 32 * BN * 4 : TOTAL - BM * 4));
   // ---- the four partial tiles meet, 32 rows at a time: [wave][row][columns], 16-B units swizzled by the row; a row tile is
   // written while the one before it is added up
   constexpr int QR = 8 * CT, RP = 64 * NW / QR, SRC = 32 * 32 * CT * 4;
@@ -85,11 +146,17 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
   // ahead: 4096 x 4096 Q4_K, 300 / 700 rows 22 -> 20, 40 -> 33; 4096 x 14336, 300 rows Q4_K 51 -> 46, Q6_K 63 -> 56; 130 rows Q6_K 39 -> 35)
   auto residual = [&](int row) __attribute__((always_inline)) {
     gf32x4 c = {};
-    if constexpr (EPI == GEPI_ACCUM) c = *(const gf32x4*)(a.C + (size_t)min(m0 + row, a.M - 1) * a.ldc + n);
+    if constexpr (EPI == GEPI_ACCUM || EPI == GEPI_ACCUM_NORM) c = *(const gf32x4*)(a.C + (size_t)min(m0 + row, a.M - 1) * a.ldc + n);
     return c;
   };
   auto finish = [&](int row, gf32x4 v, gf32x4 res) __attribute__((always_inline)) {
-    sk_finish<EPI>(a, nullptr, m0 + row, n, v, (const float4*)&res);
+    if (a.nrm_in) v *= inv_s[row];
+    float ss = sk_finish<EPI>(a, nullptr, m0 + row, n, v, (const float4*)&res);
+    if constexpr (EPI == GEPI_ACCUM_NORM) {  // 64 columns of a row lie on 16 successive lanes
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o, 64);
+      if ((q & 15) == 0) a.nrm_part[(size_t)(m0 + row) * a.nrm_parts + (n >> 6)] = ss;
+    }
   };
   gf32x4 res[MT][32 / RP];
   if (S == 1) {
@@ -101,6 +168,7 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
 #pragma unroll
   for (int i = 0; i <= MT; ++i) {
     pf_barrier();
+    if (KEEP && i == 0 && a.nrm_in) rows.put(wave, lane, inv_s);
     if (i < MT) {
 #pragma unroll
       for (int c = 0; c < CW; ++c)
@@ -322,12 +390,18 @@ __device__ __forceinline__ void pfk_body(const GemmQArgs& a, int m0, int n0, int
 
   // ---- pipeline: X slots three deep, W blocks NWB deep; before the barrier B(t) a wave has waited for its own pieces of slot t
   // and read its last of slot t - 1, so behind it slot t is whole and the buffers of t - 1 are free
+  PfkRows<L::BM, NW> rows;
+  if (a.nrm_in) rows.load(a, m0, wave, lane);
   const uint32_t w0a = lds0 + L::OFF_W;
   issue_w(b0, w0a);
   issue_x(t0, lds0);
 #pragma unroll
   for (int p = 1; p < NWB - 1; ++p) issue_w(b0 + p, w0a + p * L::WB);
   issue_x(t0 + 1, lds0 + L::XS);
+  if (a.nrm_in) {
+    rows.done(a, m0, wave, lane);
+    if constexpr (!L::KEEP) rows.put(wave, lane, (float*)(pf_smem0 + L::TOTAL - L::BM * 4));
+  }
   pf_vmcnt<(NWB - 2) * NWP + NX>();
   pf_barrier();
 #pragma unroll
@@ -411,7 +485,7 @@ __device__ __forceinline__ void pfk_body(const GemmQArgs& a, int m0, int n0, int
   pf_vmcnt<0>();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
-  pfk_close<MT, CT, NG, EPI>(a, acc, m0, n0, sp, S, tile, ntile, last_flag);
+  pfk_close<MT, CT, NG, EPI, L::KEEP, L::TOTAL>(a, acc, m0, n0, sp, S, tile, ntile, last_flag, rows);
 }
 
 template <int QT0, int QT1, int MT, int CT, int NG, int EPI>
@@ -442,6 +516,10 @@ void pfk_launch(const GemmQArgs& a, int S, hipStream_t st) {
   switch (a.epi) {
     case GEPI_STORE: hipLaunchKernelGGL((gemm_pfk_kernel<QT0, QT1, MT, CT, NG, GEPI_STORE>), grid, block, lds, st, a); break;
     case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pfk_kernel<QT0, QT1, MT, CT, NG, GEPI_ACCUM>), grid, block, lds, st, a); break;
+    case GEPI_QKV: hipLaunchKernelGGL((gemm_pfk_kernel<QT0, QT1, MT, CT, NG, GEPI_QKV>), grid, block, lds, st, a); break;
+    case GEPI_ACCUM_NORM:
+      if constexpr (QT0 == QT1 && CT > 1) hipLaunchKernelGGL((gemm_pfk_kernel<QT0, QT1, MT, CT, NG, GEPI_ACCUM_NORM>), grid, block, lds, st, a);
+      break;
     default:
       if constexpr (QT0 == QT1) hipLaunchKernelGGL((gemm_pfk_kernel<QT0, QT1, MT, CT, NG, GEPI_SWIGLU_BF16>), grid, block, lds, st, a);
       break;

@@ -44,12 +44,12 @@ constexpr bool pfk_fits() {  // two blocks of weights beside the slots of X (160
   return PfkLayout<QT0, MT, CT, NG>::NWB >= 2 && PfkLayout<QT1, MT, CT, NG>::NWB >= 2;
 }
 
-// bm x bn tiles divide N and every segment (pf_plan_ok).  16-byte stores to C, 4-byte ones to C16; 32-bit offsets into X and the
+// bm x bn tiles divide N and every segment (pf_plan_ok).  32-bit offsets into X and the
 // planes; K slices: workspace for their slabs, a ticket per tile
 bool pfk_serves(const GemmQArgs& a, int bm, int bn, int S) {
-  if (a.epi != GEPI_STORE && a.epi != GEPI_ACCUM && a.epi != GEPI_SWIGLU_BF16) return false;
+  if (a.epi == GEPI_STORE16 || !pfk_epi_ok(a, bn)) return false;
   if (S < 1 || S > a.K / 256 || a.K % 256) return false;
-  if (a.epi == GEPI_SWIGLU_BF16 ? a.ldc % 2 || ((uintptr_t)a.C16 & 3) : a.ldc % 4 || ((uintptr_t)a.C & 15)) return false;
+  if ((a.epi == GEPI_SWIGLU_BF16 || a.epi == GEPI_ACCUM_NORM) && a.nseg != 1) return false;
   if ((size_t)a.M * a.lda * 2 >= 0xfffffff0u) return false;
   for (int s = 0; s < a.nseg; ++s)
     if ((size_t)a.seg[s].rows * a.K / 2 >= 0xfffffff0u) return false;

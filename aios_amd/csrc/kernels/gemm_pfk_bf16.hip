@@ -19,8 +19,8 @@ struct PfkbLayout {
   static constexpr int BM = 32 * MT, BN = 32 * CT, XS = BM * 256, SLOT = XS + BN * 256;
   static constexpr int NS = PFK_LDS / SLOT < 4 ? PFK_LDS / SLOT : 4;
   static constexpr int NW = 4 * NG, NX = BM / 4 / NW, NB = BN / 4 / NW, NR = NX + NB;  // waves; DMA requests a wave, per slot
-  static constexpr int RED_BYTES = 2 * 4 * 32 * BN * 4;
-  static constexpr int TOTAL = NS * SLOT > RED_BYTES ? NS * SLOT : RED_BYTES;
+  static constexpr int RED_BYTES = 2 * 4 * 32 * BN * 4 + BM * 4;
+  static constexpr int USED = NS * SLOT + BM * 4, TOTAL = USED > RED_BYTES ? USED : RED_BYTES;
   static_assert(NS >= 2 && TOTAL <= PFK_LDS && NX * 4 * NW == BM && NB * 4 * NW == BN, "pfkb slots");
 };
 
@@ -80,10 +80,16 @@ __global__ void __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(N
   constexpr int UB = NM > 2 ? 6 * NM / 10 : 1, UF = NM > 4 ? NM / 4 : 1;
   auto part = [](int n, int u, int from, int to) constexpr { return u <= from ? 0 : (u >= to ? n : n * (u - from) / (to - from)); };
   constexpr int PA = part(NR, 2 * NM, UB, UB + 2 * NM);  // of them, in step t
+  PfkRows<BM, L::NW> rows;
+  if (a.nrm_in) rows.load(a, m0, wave, lane);
 #pragma unroll
   for (int p = 0; p < NS; ++p)
 #pragma unroll
     for (int i = 0; i < (p < NS - 1 ? NR : PA); ++i) req(i, t0 + p, p * L::SLOT);
+  if (a.nrm_in) {
+    rows.done(a, m0, wave, lane);
+    rows.put(wave, lane, (float*)(pf_smem0 + L::TOTAL - BM * 4));
+  }
   pf_vmcnt<(NS - 2) * NR + PA>();
   pf_barrier();
 #pragma unroll
@@ -118,7 +124,7 @@ __global__ void __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(N
   }
   pf_vmcnt<0>();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  pfk_close<MT, CT, NG, EPI>(a, acc, m0, n0, sp, S, tile, ntile, last_flag);
+  pfk_close<MT, CT, NG, EPI, false, L::TOTAL>(a, acc, m0, n0, sp, S, tile, ntile, last_flag, rows);
 }
 
 // f(MT, CT, NG) of a tile, false if there is none: 64 to 160 rows; 32 columns (four waves), 64 or 128 (eight)
@@ -143,13 +149,10 @@ static bool pfkb_tile(int bm, int bn, F f) {
 #undef PFK_T
 }
 
-// bm x bn tiles divide N and every segment (pf_plan_ok).  Slots of 128 k; 16-byte stores to C, 8-byte ones to C16; 32-bit offsets into X
-// and W; K slices: workspace for their slabs, a ticket per tile
+// bm x bn tiles divide N and every segment (pf_plan_ok).  Slots of 128 k; 32-bit offsets into X and W; K slices: workspace for their slabs, a ticket per tile
 bool pfkb_serves(const GemmQArgs& a, int bm, int bn, int S) {
-  const bool half = a.epi == GEPI_SWIGLU_BF16 || a.epi == GEPI_STORE16;
-  if (!half && a.epi != GEPI_STORE && a.epi != GEPI_ACCUM) return false;
+  if (!pfk_epi_ok(a, bn)) return false;
   if (S < 1 || S > a.K / 128 || a.K % 128) return false;
-  if (half ? a.ldc % 4 || ((uintptr_t)a.C16 & 7) : a.ldc % 4 || ((uintptr_t)a.C & 15)) return false;
   if ((size_t)a.M * a.lda * 2 >= 0xfffffff0u) return false;
   for (int s = 0; s < a.nseg; ++s)
     if (a.seg[s].qtype != QT_BF16 || (size_t)a.seg[s].rows * a.K * 2 >= 0xfffffff0u || ((uintptr_t)a.seg[s].p0 & 15)) return false;
@@ -168,6 +171,10 @@ bool pfkb_run(const GemmQArgs& a, int bm, int bn, int S, hipStream_t st) {
     switch (a.epi) {
       case GEPI_STORE: hipLaunchKernelGGL((gemm_pfkb_kernel<MT, CT, NG, GEPI_STORE>), grid, block, lds, st, a); break;
       case GEPI_ACCUM: hipLaunchKernelGGL((gemm_pfkb_kernel<MT, CT, NG, GEPI_ACCUM>), grid, block, lds, st, a); break;
+      case GEPI_QKV: hipLaunchKernelGGL((gemm_pfkb_kernel<MT, CT, NG, GEPI_QKV>), grid, block, lds, st, a); break;
+      case GEPI_ACCUM_NORM:
+        if constexpr (CT > 1) hipLaunchKernelGGL((gemm_pfkb_kernel<MT, CT, NG, GEPI_ACCUM_NORM>), grid, block, lds, st, a);
+        break;
       case GEPI_STORE16: hipLaunchKernelGGL((gemm_pfkb_kernel<MT, CT, NG, GEPI_STORE16>), grid, block, lds, st, a); break;
       default: hipLaunchKernelGGL((gemm_pfkb_kernel<MT, CT, NG, GEPI_SWIGLU_BF16>), grid, block, lds, st, a); break;
     }

@@ -241,7 +241,8 @@ struct GemmQArgs {
   // RMSNorm split across two skinny GEMMs (batched decode: no normalisation launch).
   //  producer (GEPI_ACCUM_NORM = residual add): also writes bf16(x_new * nrm_g) to nrm_out16
   //    [M][ldc] and, per 16 columns t, sum_n x_new[m][n]^2 to nrm_part[m * nrm_parts + t]
-  //    (nrm_parts = N / 16; wider tiles: their sum in the first part and zeros in the others; fixed order)
+  //    (nrm_parts = N / 16; wider tiles: their sum in the first part and zeros in the others; fixed order.  Prefill GEMM,
+  //    gemm_pf_fuses: a part per 64 columns, nrm_parts = N / 64, on both sides)
   //  consumer (any epilogue, nrm_in set): A is that bf16(x * g); output row m is scaled by
   //    rsqrt(sum_t nrm_in[m * nrm_parts + t] / K + nrm_eps) before the epilogue
   const float* nrm_g;
@@ -264,6 +265,7 @@ bool gemm_wk_on();
 bool gemm_wk_serves(const GemmQArgs& a);
 // the prefill GEMM (kernels/gemm_pf.hip): true if it took the launch; its tile / split plan for a shape
 bool launch_gemm_pf(const GemmQArgs& a, hipStream_t st);
+bool gemm_pf_fuses(const GemmQArgs& a);  // whether the prefill GEMM would run these args, the decode GEMMs' fused epilogues among them, on tiles with K over the waves
 bool gemm_pf_serves(const GemmQArgs& a);  // launch_gemm_pf would take a (gemm_pf.hip)
 void gemm_pf_plan(const GemmQArgs& a, int& bm, int& bn, int& s);
 bool gemm_pf_probe(const GemmQArgs& a, int probe, hipStream_t st);  // timing anatomy (tools only)

@@ -419,6 +419,27 @@ def test_batched_decode_split_rmsnorm_matches_explicit(model_files, monkeypatch,
     assert np.abs(l0 - l1).max() < 1e-2 * max(np.abs(l0).max(), 1.0)
 
 
+@pytest.mark.parametrize("recipe,tile", [("mistral_shape", "64x-64"), ("mistral_shape", "96x-128"), ("BF16", "64x-64")])
+@pytest.mark.parametrize("kv", ["bf16", "fp8_e4m3"])
+def test_prefill_fused_norm_and_rope_match_explicit(model_files, monkeypatch, recipe, tile, kv):
+    """prompts above 32 tokens on tiles with K over the waves: RMSNorm split across the products, RoPE and the cache in the QKV product's
+    epilogue; against the explicit launches, to bf16 rounding (an fp8 code: a step of 1/16), a second portion behind the first"""
+    prompt = [1] + list(np.random.default_rng(2).integers(3, 500, 170))
+    outs = {}
+    for fuse in ("0", "1"):
+        monkeypatch.setenv("AIOS_GEMM_NORM_FUSE", fuse)
+        monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile if fuse == "1" else "64x128")
+        eng, cfg = _load(model_files[recipe], act_q8=False, kv_dtype=kv)
+        if kv != "bf16":
+            eng.set_kv_scales([1 / 32] * (2 * cfg.n_layers))
+        eng.prefill(0, prompt[:100], 0, False)
+        outs[fuse] = np.asarray(eng.prefill(0, prompt[100:], 100, True))
+        del eng
+    l0, l1 = outs["0"], outs["1"]
+    assert np.isfinite(l1).all() and not np.array_equal(l0, l1)
+    assert np.abs(l0 - l1).max() < (1e-2 if kv == "bf16" else 4e-2) * max(np.abs(l0).max(), 1.0)
+
+
 @pytest.mark.parametrize("recipe", ["Q4_K_M", "mistral_shape"])
 def test_batched_decode_mixed_format_qkv_launch(model_files, monkeypatch, recipe):
     """AIOS_SKINNY_MIXED: the Q4_K_M QKV stack (Q|K Q4_K, V Q6_K) as ONE skinny launch whose V

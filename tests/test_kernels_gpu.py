@@ -1784,6 +1784,82 @@ def test_gemm_pfk_swiglu(E, monkeypatch, tile, act, S):
     assert rel < 3 * 2 * 2.0 ** -9 / 3 ** 0.5, rel  # (the product of two rounded sums, rounded)
 
 
+@pytest.mark.parametrize("t,tile", [("Q4_K", "64x-64"), ("Q4_K", "160x-128"), ("Q6_K", "160x-64"), ("Q6_K", "96x-128"), ("BF16", "64x-64"),
+                                    ("BF16", "160x-128"), ("BF16", "128x-64")])
+@pytest.mark.parametrize("S", [1, 3])
+@pytest.mark.parametrize("M,K1,K2", [(33, 768, 256), (161, 1024, 2048), (300, 1024, 8192)])
+def test_gemm_pfk_split_rmsnorm(E, t, tile, S, M, K1, K2, monkeypatch):
+    """the residual's bf16(x g) and its sums of squares per 64 columns, and the next product's rows scaled by them, up to 128
+    parts a row, against float64"""
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
+    g = torch.Generator().manual_seed(K2 + M)
+    (m1, W1), (m2, W2) = small_mat(E, t, K2, K1, 11), small_mat(E, t, 128, K2, 12)
+    A = torch.randn(M, K1, generator=g).to(torch.bfloat16)
+    res, gain = torch.randn(M, K2, generator=g), torch.rand(K2, generator=g) + 0.5
+    Ad, gd, C = A.cuda(), gain.cuda(), res.cuda()
+    x16, part = torch.zeros(M, K2, dtype=torch.bfloat16, device="cuda"), torch.full((M, K2 // 64), float("nan"), device="cuda")
+    more = dict(nrm_g=gd.data_ptr(), nrm_out16=x16.data_ptr(), nrm_part=part.data_ptr(), nrm_parts=K2 // 64)
+    assert E.gemm_pf_fuses([m1], M, E.GEPI_ACCUM_NORM, Ad.data_ptr(), K1, C.data_ptr(), K2, more)
+    E.gemm_q(Ad.data_ptr(), K1, [m1], M, C.data_ptr(), 0, K2, E.GEPI_ACCUM_NORM, stream(), more=more)
+    torch.cuda.synchronize()
+    ref = res.double() + A.double() @ W1.T
+    assert ((C.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)).max() < sum_tol(t, K1) + 2.0 ** -23
+    assert torch.equal(x16, (C * gd).to(torch.bfloat16))
+    sq = C.cpu().double().pow(2).sum(1)
+    assert ((part.cpu().double().sum(1) - sq).abs() / sq).max() < 2.0 ** -20  # (64 squares an fp32 sum)
+    if K2 < 1024:
+        return  # (fewer blocks than slices)
+    y, more = torch.zeros(M, 128, device="cuda"), dict(nrm_in=part.data_ptr(), nrm_parts=K2 // 64, nrm_eps=1e-5)
+    assert E.gemm_pf_fuses([m2], M, E.GEPI_STORE, x16.data_ptr(), K2, y.data_ptr(), 128, more)
+    E.gemm_q(x16.data_ptr(), K2, [m2], M, y.data_ptr(), 0, 128, E.GEPI_STORE, stream(), more=more)
+    torch.cuda.synchronize()
+    ref = (x16.cpu().double() @ W2.T) * torch.rsqrt(sq / K2 + 1e-5)[:, None]
+    assert ((y.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)).max() < sum_tol(t, K2) + 2.0 ** -19
+
+
+@pytest.mark.parametrize("ts,tile", [("Q4_K Q4_K Q4_K", "64x-128"), ("Q4_K Q4_K Q6_K", "96x-64"), ("Q6_K Q6_K Q6_K", "160x-32"),
+                                     ("BF16 BF16 BF16", "128x-128"), ("BF16 BF16 BF16", "64x-32")])
+@pytest.mark.parametrize("S", [1, 2])
+@pytest.mark.parametrize("M,K", [(33, 512), (200, 2048)])
+def test_gemm_pfk_qkv(E, ts, tile, S, M, K, monkeypatch):
+    """the packed QKV product through RoPE to q and the paged cache, fused RMSNorm in front, against float64"""
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
+    ts, H, Hkv, hd, slots, max_ctx = ts.split(), 4, 2, 64, 4, 256
+    rows = (H * hd, Hkv * hd, Hkv * hd)
+    mats, W = zip(*[small_mat(E, t, n, K, 21 + i) for i, (t, n) in enumerate(zip(ts, rows))])
+    g = torch.Generator().manual_seed(K + M)
+    A, part = torch.randn(M, K, generator=g).to(torch.bfloat16), torch.rand(M, K // 64, generator=g) * 32
+    pos, slot = torch.arange(M) // slots * 3 + 1, torch.arange(M) % slots
+    ang = torch.arange(max_ctx)[:, None].double() * 1e4 ** (-2.0 * torch.arange(hd // 2).double() / hd)
+    cs = torch.stack([ang.cos(), ang.sin()], -1).float()
+    kp, bt = paged_cache(torch.zeros(slots, Hkv, max_ctx, hd, dtype=torch.bfloat16), True, seed=3)
+    dev = [x.cuda() for x in (A, part, pos.int(), slot.int(), cs, kp, torch.zeros_like(kp), bt)]
+    Ad, pd, posd, slotd, csd, kd, vd, btd = dev
+    q = torch.zeros(M, rows[0], device="cuda")
+    more = dict(nrm_in=pd.data_ptr(), nrm_parts=K // 64, nrm_eps=1e-5, head_dim=hd, q_dim=rows[0], kv_dim=rows[1], n_kv_heads=Hkv,
+                max_ctx=max_ctx, rope_cs=csd.data_ptr(), pos=posd.data_ptr(), slot=slotd.data_ptr(), block_table=btd.data_ptr(),
+                q_out=q.data_ptr(), k_cache=kd.data_ptr(), v_cache=vd.data_ptr())
+    assert E.gemm_pf_fuses(list(mats), M, E.GEPI_QKV, Ad.data_ptr(), K, 0, sum(rows), more)
+    E.gemm_q(Ad.data_ptr(), K, list(mats), M, 0, 0, sum(rows), E.GEPI_QKV, stream(), more=more)
+    torch.cuda.synchronize()
+    y = (A.double() @ torch.cat(W).T) * torch.rsqrt(part.double().sum(1) / K + 1e-5)[:, None]
+
+    def turn(x):
+        a, b, c, s = x[..., 0::2], x[..., 1::2], ang.cos()[pos][:, None], ang.sin()[pos][:, None]
+        return torch.stack([a * c - b * s, a * s + b * c], -1).reshape(x.shape)
+
+    yq, yk, yv = y.split(rows, 1)
+    ref = turn(yq.view(M, H, hd)).reshape(M, -1)
+    tol = max(sum_tol(t, K) for t in ts) + 2.0 ** -19
+    assert ((q.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)).max() < tol
+    for cache, ref in ((kd, turn(yk.view(M, Hkv, hd))), (vd, yv.view(M, Hkv, hd))):
+        got = unpaged(cache.cpu(), slots, max_ctx, bt)[slot, :, pos].double()
+        # (8 bits of significand: a value just above a power of two is rounded by up to 2^-8 of itself)
+        assert ((got - ref).flatten(1).norm(dim=1) / ref.flatten(1).norm(dim=1)).max() < tol + 2.0 ** -8
+
+
 def test_gemm_pfk_is_not_taken(E, monkeypatch):
     """calls that its 16-byte stores or its workspace do not fit keep the other tiles: C off 16 bytes, a pitch off 4, more slices than
     blocks; their results are the same products"""
