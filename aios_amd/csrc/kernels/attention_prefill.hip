@@ -83,12 +83,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   // first 32 m items (a CU's second workgroup) goes from the shortest up, so every CU gets about the same number of tiles.
   // us, heads over all XCDs -> so: 1852 tokens behind 2048, 32 / 8 heads of 128 127 -> 112; 300 behind 6000, fp8, six runs 53 -> 49;
   // 1500 tokens, 32 / 4 heads of 64 35 -> 27.
-  const int nx = (a.T + BQ - 1) / BQ, ny = a.n_kv_heads;
-  const int m = ny % 8 == 0 ? 1 : (8 % ny == 0 ? 8 / ny : 8), hx = ny % 8 == 0 ? ny / 8 : (8 % ny == 0 ? 1 : ny);
-  const int xcd = blockIdx.x & 7, W = hx * nx * a.ns, w = (blockIdx.x >> 3) * m + xcd % m;
+  const int nx = (a.T + BQ - 1) / BQ, m = 1 << a.lm;
+  const int xcd = blockIdx.x & 7, W = a.hx * nx * a.ns, w = ((blockIdx.x >> 3) << a.lm) + (xcd & (m - 1));
   if (w >= W) return;
-  const int item = w < 32 * m || W > 64 * m ? w : W - 1 - (w - 32 * m);
-  const int kvh = xcd / m * hx + item % hx, run_z = item / hx % a.ns, qb = nx - 1 - item / hx / a.ns;
+  int item = w < 32 * m || W > 64 * m ? w : W - 1 - (w - 32 * m);
+  int kvh = xcd >> a.lm, run_z = 0;
+  if (a.hx > 1) {  // (divisions only where there is something to divide: 0.3 us of a short prompt's 6)
+    kvh = kvh * a.hx + item % a.hx;
+    item /= a.hx;
+  }
+  if (a.ns > 1) {
+    run_z = item % a.ns;
+    item /= a.ns;
+  }
+  const int qb = nx - 1 - item;
   const int T = a.T, start = a.start;
   const int t0 = qb * BQ;
   // this lane's query row (column of S^T / O^T)
@@ -378,8 +386,11 @@ template <int HD, bool F8>
 static void prefill_hd(AttnPrefillArgs a, int G, hipStream_t st) {
   const int BQ = 128 / G;
   a.ns = prefill_runs(a, BQ);
-  const int ny = a.n_kv_heads, m = ny % 8 == 0 ? 1 : (8 % ny == 0 ? 8 / ny : 8), hx = ny % 8 == 0 ? ny / 8 : (8 % ny == 0 ? 1 : ny);
-  const int W = hx * ((a.T + BQ - 1) / BQ) * a.ns;
+  const int ny = a.n_kv_heads;
+  a.lm = ny % 8 == 0 ? 0 : (ny == 4 ? 1 : (ny == 2 ? 2 : 3));  // (neither a divisor nor a multiple of 8: all XCDs share all heads)
+  a.hx = ny % 8 == 0 ? ny / 8 : (8 % ny == 0 ? 1 : ny);
+  const int m = 1 << a.lm;
+  const int W = a.hx * ((a.T + BQ - 1) / BQ) * a.ns;
   const dim3 grid(8 * ((W + m - 1) / m));  // (the kernel's lists, one place in turn on each XCD)
   const size_t lds = (size_t)2 * FP_KT * ((HD + 8) + (HD + 32)) * sizeof(bf16_t);  // two K|V tile buffers
   switch (G) {

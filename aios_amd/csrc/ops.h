@@ -139,6 +139,7 @@ struct AttnPrefillArgs {
   float* ws = nullptr;     // workspace of launches split over the keys; null: none is split
   size_t ws_bytes = 0;
   int ns = 1;              // runs over the keys (the launcher's choice)
+  int lm = 0, hx = 1;      // 2^lm XCDs share the work of hx KV heads (the launcher's)
 };
 size_t attn_prefill_ws_bytes(int head_dim);  // enough for every launch that is split
 void launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t st);
