@@ -26,43 +26,37 @@ namespace aios {
 
 constexpr int PFK_LDS = 160 * 1024 - 64;  // dynamic LDS of these kernels at most: their last_flag lies beside it
 
-// The fused RMSNorm's consumer: the scales of the tile's rows from the producer's sums of squares (a part per 64 columns), eight
-// lanes a row, added up in a fixed order.  load() requests, done() adds up, put() writes them to LDS.
+// The fused RMSNorm's consumer: the scales of the tile's rows from the producer's sums of squares (at most 64 parts a row: one per 64
+// columns).  A wave has its rows' parts brought into its own share of an X slot that is not in use yet, so they travel with the first
+// requests (read into registers they were waited for together with all of those), and adds them up in a fixed order, eight lanes a row.
 template <int BM, int NW>
 struct PfkRows {
-  static constexpr int KI = (BM / NW + 7) / 8;  // rows of a lane's eighth
-  gf32x4 v[KI][2];
+  static constexpr int RW = BM / NW, NP = RW / 4, KI = (RW + 7) / 8;  // rows of a wave, its requests (4 rows each), rows of a lane's eighth
   float inv[KI];
-  __device__ __forceinline__ const gf32x4* at(const GemmQArgs& a, int m0, int wave, int lane, int k, int j) const {
-    const int row = min(m0 + wave * (BM / NW) + 8 * k + (lane >> 3), a.M - 1);
-    return (const gf32x4*)(a.nrm_in + (size_t)row * a.nrm_parts + j);
-  }
-  __device__ __forceinline__ void load(const GemmQArgs& a, int m0, int wave, int lane) {
-#pragma unroll
-    for (int k = 0; k < KI; ++k)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        v[k][j] = gf32x4{0.f, 0.f, 0.f, 0.f};
-        const int p = 32 * j + 4 * (lane & 7);
-        if (p < a.nrm_parts) v[k][j] = *at(a, m0, wave, lane, k, p);
-      }
-  }
-  __device__ __forceinline__ void done(const GemmQArgs& a, int m0, int wave, int lane) {
+  __device__ __forceinline__ void request(const GemmQArgs& a, int m0, int wave, int lane, uint32_t slot);
+  __device__ __forceinline__ void done(const GemmQArgs& a, int wave, int lane, const uint8_t* slot) {
+    const uint8_t* own = slot + wave * (RW * 256);
 #pragma unroll
     for (int k = 0; k < KI; ++k) {
-      gf32x4 t = v[k][0] + v[k][1];
-      for (int p = 64 + 4 * (lane & 7); p < a.nrm_parts; p += 32) t += *at(a, m0, wave, lane, k, p);
+      const int r = min(8 * k + (lane >> 3), RW - 1);
+      gf32x4 t = gf32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const gf32x4 u = *(const gf32x4*)(own + r * 256 + 128 * j + 16 * (lane & 7));
+        if (32 * j + 4 * (lane & 7) < a.nrm_parts) t += u;
+      }
       float s = (t[0] + t[1]) + (t[2] + t[3]);
 #pragma unroll
       for (int o = 1; o < 8; o <<= 1) s += __shfl_xor(s, o, 64);
       inv[k] = rsqrtf(s / (float)a.K + a.nrm_eps);
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the slot's own requests follow)
   }
   __device__ __forceinline__ void put(int wave, int lane, float* inv_s) const {
 #pragma unroll
     for (int k = 0; k < KI; ++k) {
       const int r = 8 * k + (lane >> 3);
-      if ((lane & 7) == 0 && r < BM / NW) inv_s[wave * (BM / NW) + r] = inv[k];
+      if ((lane & 7) == 0 && r < RW) inv_s[wave * RW + r] = inv[k];
     }
   }
 };
@@ -104,11 +98,20 @@ __device__ __forceinline__ void pfk_dma4(const void* base, uint32_t off, uint32_
                : "memory", "m0");
 }
 
+template <int BM, int NW>
+__device__ __forceinline__ void PfkRows<BM, NW>::request(const GemmQArgs& a, int m0, int wave, int lane, uint32_t slot) {
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int row = min(m0 + wave * RW + 4 * i + (lane >> 4), a.M - 1), u = 4 * (lane & 15) < a.nrm_parts ? lane & 15 : 0;
+    pfk_dma1(a.nrm_in, ((uint32_t)row * (uint32_t)a.nrm_parts + 4u * u) * 4u, slot + wave * (RW * 256) + i * 1024);
+  }
+}
+
 // host: whether the epilogue's operands fit the stores of these kernels (bn: columns of a tile).  16-byte stores to C, 8-byte ones to C16 and
 // 4-byte ones of a gated product; a part of the split RMSNorm per 64 columns, on either side
 inline bool pfk_epi_ok(const GemmQArgs& a, int bn) {
   auto off = [](const void* p, int n) { return ((uintptr_t)p & (n - 1)) != 0; };
-  if (a.nrm_in && (a.K % 256 || a.nrm_parts != a.K / 64 || off(a.nrm_in, 16))) return false;
+  if (a.nrm_in && (a.K % 256 || a.K > 4096 || a.nrm_parts != a.K / 64 || off(a.nrm_in, 16))) return false;
   switch (a.epi) {
     case GEPI_STORE: case GEPI_ACCUM: return a.ldc % 4 == 0 && !off(a.C, 16);
     case GEPI_ACCUM_NORM:
@@ -116,7 +119,8 @@ inline bool pfk_epi_ok(const GemmQArgs& a, int bn) {
              a.nrm_parts == a.N / 64 && (!a.bias16 || !off(a.bias16, 16));
     case GEPI_SWIGLU_BF16: return a.ldc % 2 == 0 && !off(a.C16, 4);
     case GEPI_STORE16: return a.ldc % 4 == 0 && !off(a.C16, 8);
-    case GEPI_QKV: return !off(a.q_out, 8) && a.head_dim % 2 == 0 && a.q_dim % 2 == 0 && a.kv_dim % 2 == 0;
+    case GEPI_QKV:  // (a lane's four columns in one head, its stores whole)
+      return !off(a.q_out, 16) && !off(a.k_cache, 8) && !off(a.v_cache, 8) && a.head_dim % 4 == 0 && a.q_dim % 4 == 0 && a.kv_dim % 4 == 0;
     default: return false;
   }
 }
@@ -142,33 +146,81 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
   auto slab = [&](int k) __attribute__((always_inline)) {  // byte of slice k's partial sums of this tile
     return (uint32_t)(k * ntile + tile) * (uint32_t)(BM * BN * 4);
   };
-  // (the residual is requested ahead: a load behind a store to what may be the same place would wait for it, row by row.  us, so ->
-  // ahead: 4096 x 4096 Q4_K, 300 / 700 rows 22 -> 20, 40 -> 33; 4096 x 14336, 300 rows Q4_K 51 -> 46, Q6_K 63 -> 56; 130 rows Q6_K 39 -> 35)
-  auto residual = [&](int row) __attribute__((always_inline)) {
-    gf32x4 c = {};
-    if constexpr (EPI == GEPI_ACCUM || EPI == GEPI_ACCUM_NORM) c = *(const gf32x4*)(a.C + (size_t)min(m0 + row, a.M - 1) * a.ldc + n);
-    return c;
+  // What an output needs besides its sum is requested ahead: a load behind a store to what may be the same place would wait for it, row by
+  // row.  us, residual so -> ahead: 4096 x 4096 Q4_K, 300 / 700 rows 22 -> 20, 40 -> 33; 4096 x 14336, 300 rows Q4_K 51 -> 46, Q6_K
+  // 63 -> 56; 130 rows Q6_K 39 -> 35.  6144 x 4096 to q and the cache, 130 rows in two slices 27 -> 25.
+  gf32x4 gain = {}, bias = {};
+  if constexpr (EPI == GEPI_ACCUM_NORM) {
+    gain = *(const gf32x4*)(a.nrm_g + n);
+    if (a.bias16) bias = *(const gf32x4*)(a.bias16 + n);
+  }
+  const int hd = EPI == GEPI_QKV ? a.head_dim : 4;
+  const int sect = EPI != GEPI_QKV || n < a.q_dim ? 0 : (n < a.q_dim + a.kv_dim ? 1 : 2);  // q, k, v
+  const int nr = sect == 0 ? n : n - (sect == 1 ? a.q_dim : a.q_dim + a.kv_dim), head = nr / hd, lr = nr - head * hd;
+  struct Ahead {
+    gf32x4 c;   // the residual | RoPE's (cos, sin) of the two pairs
+    size_t to;  // QKV: where the row's four elements go
   };
-  auto finish = [&](int row, gf32x4 v, gf32x4 res) __attribute__((always_inline)) {
+  auto ahead = [&](int row) __attribute__((always_inline)) {
+    Ahead h_;
+    h_.c = gf32x4{1.f, 0.f, 1.f, 0.f};
+    h_.to = 0;
+    const int m = min(m0 + row, a.M - 1);
+    if constexpr (EPI == GEPI_ACCUM || EPI == GEPI_ACCUM_NORM) {
+      h_.c = *(const gf32x4*)(a.C + (size_t)m * a.ldc + n);
+    } else if constexpr (EPI == GEPI_QKV) {
+      const int pos = a.pos[m], slot = a.slot ? a.slot[m] : 0;
+      if (sect < 2) {
+        const float2* cs = a.rope_cs + (size_t)pos * (hd >> 1) + (lr >> 1);
+        const float2 c0 = cs[0], c1 = cs[1];
+        h_.c = gf32x4{c0.x, c0.y, c1.x, c1.y};
+      }
+      h_.to = sect == 0 ? (size_t)m * a.q_dim + n : kv_offset(a.block_table, a.max_ctx / KV_BLOCK, slot, a.n_kv_heads, head, pos, hd) + lr;
+    }
+    return h_;
+  };
+  auto finish = [&](int row, gf32x4 v, const Ahead& h_) __attribute__((always_inline)) {
+    const int m = m0 + row;
     if (a.nrm_in) v *= inv_s[row];
-    float ss = sk_finish<EPI>(a, nullptr, m0 + row, n, v, (const float4*)&res);
-    if constexpr (EPI == GEPI_ACCUM_NORM) {  // 64 columns of a row lie on 16 successive lanes
+    if constexpr (EPI == GEPI_ACCUM_NORM) {
+      const gf32x4 x = h_.c + (v + bias);
+      *(gf32x4*)(a.C + (size_t)m * a.ldc + n) = x;
+      *(uint2*)(a.nrm_out16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(x[0] * gain[0], x[1] * gain[1]), pk_bf16(x[2] * gain[2], x[3] * gain[3]));
+      float ss = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
 #pragma unroll
-      for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o, 64);
-      if ((q & 15) == 0) a.nrm_part[(size_t)(m0 + row) * a.nrm_parts + (n >> 6)] = ss;
+      for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o, 64);  // 64 columns of a row lie on 16 successive lanes
+      if ((q & 15) == 0) a.nrm_part[(size_t)m * a.nrm_parts + (n >> 6)] = ss;
+    } else if constexpr (EPI == GEPI_QKV) {
+      const gf32x4 t = h_.c;
+      const float o0 = v[0] * t[0] - v[1] * t[1], o1 = v[0] * t[1] + v[1] * t[0];
+      const float o2 = v[2] * t[2] - v[3] * t[3], o3 = v[2] * t[3] + v[3] * t[2];
+      if (sect == 0) {
+        *(gf32x4*)(a.q_out + h_.to) = gf32x4{o0, o1, o2, o3};
+      } else {
+        bf16_t* cache = sect == 1 ? a.k_cache : a.v_cache;
+        const float inv = sect == 1 ? a.kv_inv_k : a.kv_inv_v;
+        if (a.kv_fp8) *(uint32_t*)((uint8_t*)cache + h_.to) = f32x2_to_fp8x2(o0 * inv, o1 * inv) | f32x2_to_fp8x2(o2 * inv, o3 * inv) << 16;
+        else *(uint2*)(cache + h_.to) = make_uint2(pk_bf16(o0, o1), pk_bf16(o2, o3));
+      }
+    } else {
+      sk_finish<EPI>(a, nullptr, m, n, v, (const float4*)&h_.c);
     }
   };
-  gf32x4 res[MT][32 / RP];
+  constexpr int AH = EPI == GEPI_QKV && RP < 32 ? 2 : MT;  // row tiles ahead (of 128 columns' QKV all do not fit beside the accumulators)
+  Ahead now[MT][32 / RP];
+  auto fetch = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 32 / RP; ++k) now[i][k] = ahead(32 * i + tid / QR + RP * k);
+  };
   if (S == 1) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int k = 0; k < 32 / RP; ++k) res[i][k] = residual(32 * i + tid / QR + RP * k);
+    for (int i = 0; i < AH; ++i) fetch(i);
   }
 #pragma unroll
   for (int i = 0; i <= MT; ++i) {
     pf_barrier();
     if (KEEP && i == 0 && a.nrm_in) rows.put(wave, lane, inv_s);
+    if (S == 1 && i > 0 && i - 1 + AH < MT) fetch(i - 1 + AH);
     if (i < MT) {
 #pragma unroll
       for (int c = 0; c < CW; ++c)
@@ -191,7 +243,7 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
       for (int k = 0; k < 32 / RP; ++k) {
         const int row = 32 * (i - 1) + tid / QR + RP * k;
         if (m0 + row >= a.M) continue;
-        if (S == 1) finish(row, v[k], res[i - 1][k]);
+        if (S == 1) finish(row, v[k], now[i - 1][k]);
         else
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(gu32x4, v[k]), ws, slab(sp) + ((uint32_t)row * BN + 4 * q) * 4, 0, 16 /* sc1 */);
       }
@@ -213,14 +265,15 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
   }
   __syncthreads();
   if (!last_flag) return;
-  constexpr int NP = BM / RP, PB = NP < 8 ? NP : 8;  // rows of a lane; so many at a time
+  constexpr int NP = BM / RP, PB = EPI == GEPI_QKV ? (NP < 4 ? NP : 4) : (NP < 8 ? NP : 8);  // rows of a lane; so many at a time
 #pragma unroll
   for (int p0_ = 0; p0_ < NP; p0_ += PB) {
-    gf32x4 v[PB], c[PB];
+    gf32x4 v[PB];
+    Ahead c[PB];
 #pragma unroll
     for (int p = 0; p < PB; ++p) {
       v[p] = gf32x4{0.f, 0.f, 0.f, 0.f};
-      c[p] = residual(tid / QR + RP * (p0_ + p));
+      c[p] = ahead(tid / QR + RP * (p0_ + p));
     }
     for (int k0 = 0; k0 < S; k0 += 4) {  // four slabs' loads in flight
       gf32x4 t[PB][4];
@@ -391,18 +444,18 @@ __device__ __forceinline__ void pfk_body(const GemmQArgs& a, int m0, int n0, int
   // ---- pipeline: X slots three deep, W blocks NWB deep; before the barrier B(t) a wave has waited for its own pieces of slot t
   // and read its last of slot t - 1, so behind it slot t is whole and the buffers of t - 1 are free
   PfkRows<L::BM, NW> rows;
-  if (a.nrm_in) rows.load(a, m0, wave, lane);
+  if (a.nrm_in) rows.request(a, m0, wave, lane, lds0 + 2 * L::XS);
   const uint32_t w0a = lds0 + L::OFF_W;
   issue_w(b0, w0a);
   issue_x(t0, lds0);
 #pragma unroll
   for (int p = 1; p < NWB - 1; ++p) issue_w(b0 + p, w0a + p * L::WB);
   issue_x(t0 + 1, lds0 + L::XS);
+  pf_vmcnt<(NWB - 2) * NWP + NX>();
   if (a.nrm_in) {
-    rows.done(a, m0, wave, lane);
+    rows.done(a, wave, lane, pf_smem0 + 2 * L::XS);
     if constexpr (!L::KEEP) rows.put(wave, lane, (float*)(pf_smem0 + L::TOTAL - L::BM * 4));
   }
-  pf_vmcnt<(NWB - 2) * NWP + NX>();
   pf_barrier();
 #pragma unroll
   for (int c = 0; c < CW; ++c) {

@@ -81,16 +81,18 @@ __global__ void __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(N
   auto part = [](int n, int u, int from, int to) constexpr { return u <= from ? 0 : (u >= to ? n : n * (u - from) / (to - from)); };
   constexpr int PA = part(NR, 2 * NM, UB, UB + 2 * NM);  // of them, in step t
   PfkRows<BM, L::NW> rows;
-  if (a.nrm_in) rows.load(a, m0, wave, lane);
+  if (a.nrm_in) rows.request(a, m0, wave, lane, lds0 + (NS - 1) * L::SLOT);
 #pragma unroll
-  for (int p = 0; p < NS; ++p)
+  for (int p = 0; p < NS - 1; ++p)
 #pragma unroll
-    for (int i = 0; i < (p < NS - 1 ? NR : PA); ++i) req(i, t0 + p, p * L::SLOT);
+    for (int i = 0; i < NR; ++i) req(i, t0 + p, p * L::SLOT);
+  pf_vmcnt<(NS - 2) * NR>();
   if (a.nrm_in) {
-    rows.done(a, m0, wave, lane);
+    rows.done(a, wave, lane, pf_smem0 + (NS - 1) * L::SLOT);
     rows.put(wave, lane, (float*)(pf_smem0 + L::TOTAL - BM * 4));
   }
-  pf_vmcnt<(NS - 2) * NR + PA>();
+#pragma unroll
+  for (int i = 0; i < PA; ++i) req(i, t0 + NS - 1, (NS - 1) * L::SLOT);
   pf_barrier();
 #pragma unroll
   for (int i = 0; i < MT + CW; ++i) rd(fa, wa, 0, 0, i);

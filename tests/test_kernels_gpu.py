@@ -1787,9 +1787,9 @@ def test_gemm_pfk_swiglu(E, monkeypatch, tile, act, S):
 @pytest.mark.parametrize("t,tile", [("Q4_K", "64x-64"), ("Q4_K", "160x-128"), ("Q6_K", "160x-64"), ("Q6_K", "96x-128"), ("BF16", "64x-64"),
                                     ("BF16", "160x-128"), ("BF16", "128x-64")])
 @pytest.mark.parametrize("S", [1, 3])
-@pytest.mark.parametrize("M,K1,K2", [(33, 768, 256), (161, 1024, 2048), (300, 1024, 8192)])
+@pytest.mark.parametrize("M,K1,K2", [(33, 768, 256), (161, 1024, 2048), (170, 1024, 4096), (40, 768, 8192)])
 def test_gemm_pfk_split_rmsnorm(E, t, tile, S, M, K1, K2, monkeypatch):
-    """the residual's bf16(x g) and its sums of squares per 64 columns, and the next product's rows scaled by them, up to 128
+    """the residual's bf16(x g) and its sums of squares per 64 columns, and the next product's rows scaled by them, up to 64
     parts a row, against float64"""
     monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
     monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
@@ -1808,10 +1808,11 @@ def test_gemm_pfk_split_rmsnorm(E, t, tile, S, M, K1, K2, monkeypatch):
     assert torch.equal(x16, (C * gd).to(torch.bfloat16))
     sq = C.cpu().double().pow(2).sum(1)
     assert ((part.cpu().double().sum(1) - sq).abs() / sq).max() < 2.0 ** -20  # (64 squares an fp32 sum)
-    if K2 < 1024:
-        return  # (fewer blocks than slices)
     y, more = torch.zeros(M, 128, device="cuda"), dict(nrm_in=part.data_ptr(), nrm_parts=K2 // 64, nrm_eps=1e-5)
-    assert E.gemm_pf_fuses([m2], M, E.GEPI_STORE, x16.data_ptr(), K2, y.data_ptr(), 128, more)
+    takes = K2 <= 4096 and (K2 >= 1024 or S == 1)  # (parts of a row; blocks for three slices)
+    assert E.gemm_pf_fuses([m2], M, E.GEPI_STORE, x16.data_ptr(), K2, y.data_ptr(), 128, more) == takes
+    if not takes:
+        return
     E.gemm_q(x16.data_ptr(), K2, [m2], M, y.data_ptr(), 0, 128, E.GEPI_STORE, stream(), more=more)
     torch.cuda.synchronize()
     ref = (x16.cpu().double() @ W2.T) * torch.rsqrt(sq / K2 + 1e-5)[:, None]
