@@ -760,7 +760,7 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       });
   m.def(
       "gemm_pf_plan",
-      [](std::vector<PyQMatrix*> segs, int M, int epi, int ksplit) {
+      [](std::vector<PyQMatrix*> segs, int M, int epi, int ksplit, uintptr_t out) {
         GemmQArgs a;
         std::memset(&a, 0, sizeof(a));
         if (segs.empty() || segs.size() > 3) throw std::runtime_error("gemm_pf_plan: 1..3 segments");
@@ -770,11 +770,12 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
         a.M = M; a.N = n0; a.K = segs[0]->w.cols; a.epi = epi; a.ksplit = ksplit;
         const GemmWs& g = gemm_ws(M, n0);
         a.ws = g.ws; a.ws_bytes = g.bytes; a.cnt = g.cnt; a.cnt_len = g.cnt_len;
+        a.C = (float*)out; a.C16 = (bf16_t*)out;  // (null: no tile that asks for an alignment of the outputs)
         int bm = 0, bn = 0, sp = 0;
         gemm_pf_plan(a, bm, bn, sp);
         return py::make_tuple(bm, bn, sp);
       },
-      py::arg("segs"), py::arg("M"), py::arg("epi"), py::arg("ksplit") = 0);
+      py::arg("segs"), py::arg("M"), py::arg("epi"), py::arg("ksplit") = 0, py::arg("out") = 0);
 #ifndef AIOS_BF16_ONLY
   m.def(
       "gemm_pf_probe",

@@ -113,14 +113,14 @@ inline bool pfk_epi_ok(const GemmQArgs& a, int bn) {
   auto off = [](const void* p, int n) { return ((uintptr_t)p & (n - 1)) != 0; };
   if (a.nrm_in && (a.K % 256 || a.K > 4096 || a.nrm_parts != a.K / 64 || off(a.nrm_in, 16))) return false;
   switch (a.epi) {
-    case GEPI_STORE: case GEPI_ACCUM: return a.ldc % 4 == 0 && !off(a.C, 16);
+    case GEPI_STORE: case GEPI_ACCUM: return a.C && a.ldc % 4 == 0 && !off(a.C, 16);
     case GEPI_ACCUM_NORM:
-      return a.ldc % 4 == 0 && !off(a.C, 16) && bn >= 64 && a.nrm_g && !off(a.nrm_g, 16) && a.nrm_out16 && !off(a.nrm_out16, 8) && a.nrm_part &&
+      return a.C && a.ldc % 4 == 0 && !off(a.C, 16) && bn >= 64 && a.nrm_g && !off(a.nrm_g, 16) && a.nrm_out16 && !off(a.nrm_out16, 8) && a.nrm_part &&
              a.nrm_parts == a.N / 64 && (!a.bias16 || !off(a.bias16, 16));
-    case GEPI_SWIGLU_BF16: return a.ldc % 2 == 0 && !off(a.C16, 4);
-    case GEPI_STORE16: return a.ldc % 4 == 0 && !off(a.C16, 8);
+    case GEPI_SWIGLU_BF16: return a.C16 && a.ldc % 2 == 0 && !off(a.C16, 4);
+    case GEPI_STORE16: return a.C16 && a.ldc % 4 == 0 && !off(a.C16, 8);
     case GEPI_QKV:  // (a lane's four columns in one head, its stores whole)
-      return !off(a.q_out, 16) && !off(a.k_cache, 8) && !off(a.v_cache, 8) && a.head_dim % 4 == 0 && a.q_dim % 4 == 0 && a.kv_dim % 4 == 0;
+      return a.q_out && a.k_cache && a.v_cache && !off(a.q_out, 16) && !off(a.k_cache, 8) && !off(a.v_cache, 8) && a.head_dim % 4 == 0 && a.q_dim % 4 == 0 && a.kv_dim % 4 == 0;
     default: return false;
   }
 }

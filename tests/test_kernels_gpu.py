@@ -1713,7 +1713,7 @@ def test_gemm_pfk(E, monkeypatch, tile, fmt, K, S):
     for M, epi in ((33, "store"), (bm, "accum"), (bm + 1, "store"), (2 * bm - 3, "accum")):
         e = E.GEPI_STORE if epi == "store" else E.GEPI_ACCUM
         monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
-        if list(E.gemm_pf_plan(mats, M, e, 0)) != [bm, bn, S]:
+        if list(E.gemm_pf_plan(mats, M, e, 0, out=256)) != [bm, bn, S]:
             assert tile == "160x-128" and fmt != "q4k"  # (LDS)
             pytest.skip("no such tile")
         x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
@@ -1745,7 +1745,7 @@ def test_gemm_pfk_bf16(E, monkeypatch, tile, K, S, epi):
     e = {"store": E.GEPI_STORE, "accum": E.GEPI_ACCUM, "swiglu": E.GEPI_SWIGLU_BF16, "store16": E.GEPI_STORE16}[epi]
     half, cols = epi in ("swiglu", "store16"), N // 2 if epi == "swiglu" else N
     for M in (33, bm, 2 * bm - 3):
-        assert list(E.gemm_pf_plan([m], M, e, 0)) == [bm, bn, S]
+        assert list(E.gemm_pf_plan([m], M, e, 0, out=256)) == [bm, bn, S]
         x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
         A = torch.full((M, K + 8), float("nan"), dtype=torch.bfloat16)
         A[:, :K] = x
@@ -1771,7 +1771,7 @@ def test_gemm_pfk_swiglu(E, monkeypatch, tile, act, S):
     M, K = 161, 1024
     mats, W = pf_mats(E, "q4k", K)
     N = W.shape[0]
-    assert E.gemm_pf_plan(mats, M, E.GEPI_SWIGLU_BF16, 0)[1:] == (int(tile.split("x")[1]), S)
+    assert E.gemm_pf_plan(mats, M, E.GEPI_SWIGLU_BF16, 0, out=256)[1:] == (int(tile.split("x")[1]), S)
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(act)).to(torch.bfloat16)
     A, out = x.cuda(), torch.full((M, N // 2 + 2), 7.0, dtype=torch.bfloat16, device="cuda")
     E.gemm_q(A.data_ptr(), K, mats, M, 0, out.data_ptr(), N // 2 + 2, E.GEPI_SWIGLU_BF16, stream(), 0, act=act)
