@@ -192,8 +192,9 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
       if ((q & 15) == 0) a.nrm_part[(size_t)m * a.nrm_parts + (n >> 6)] = ss;
     } else if constexpr (EPI == GEPI_QKV) {
       const gf32x4 t = h_.c;
-      const float o0 = v[0] * t[0] - v[1] * t[1], o1 = v[0] * t[1] + v[1] * t[0];
-      const float o2 = v[2] * t[2] - v[3] * t[3], o3 = v[2] * t[3] + v[3] * t[2];
+      if (sect < 2)  // (v's (1, 0) would turn an infinite value's partner into NaN)
+        v = gf32x4{v[0] * t[0] - v[1] * t[1], v[0] * t[1] + v[1] * t[0], v[2] * t[2] - v[3] * t[3], v[2] * t[3] + v[3] * t[2]};
+      const float o0 = v[0], o1 = v[1], o2 = v[2], o3 = v[3];
       if (sect == 0) {
         *(gf32x4*)(a.q_out + h_.to) = gf32x4{o0, o1, o2, o3};
       } else {

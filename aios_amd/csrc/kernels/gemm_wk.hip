@@ -54,17 +54,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t wk_rsrc(const void* p, uint32_
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, (int)n, 0x00020000);
 }
 
-// the residual that a lane's outputs are added to, requested before the tile's products (every wave: which of them adds
-// the tile up is not worth a branch here)
-template <int EPI>
-struct WkRes {
-  float4 c;
-  __device__ __forceinline__ void load(const GemmQArgs& a, int m, int n) {
-    if constexpr (EPI == GEPI_ACCUM || EPI == GEPI_ACCUM_NORM)
-      c = *(const float4*)(a.C + (size_t)min(m, a.M - 1) * a.ldc + n);
-  }
-};
-
 // X unit swizzle (16-B units of a 512-B row): 16 rows' reads of one unit fall on distinct banks
 __device__ __forceinline__ int wk_xh(int m) { return (m ^ (m << 1)) & 15; }
 
@@ -74,6 +63,7 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
                                         float* inv_s, int& last_flag) {
   constexpr bool BF = QT == QT_BF16, Q6 = QT == QT_Q6_K;
   constexpr int UK = BF ? 64 : 256;  // k of a unit (of K's split); a stage is 256
+  using Ahead = SkAhead<EPI, BF>;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rr = lane & 15, q = lane >> 4;
   const int S = p.S, ntile = a.N >> 4;
@@ -195,8 +185,8 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
     }
   };
   // one lane's outputs of tile t, rows 16 mt ..
-  auto finish = [&](int t, int mt, gf32x4 v, const WkRes<EPI>& res) __attribute__((always_inline)) {
-    float ss = sk_finish<EPI>(a, nrm ? inv_s : nullptr, 16 * mt + rr, 16 * t + 4 * q, v, &res.c);
+  auto finish = [&](int t, int mt, gf32x4 v, const Ahead& res) __attribute__((always_inline)) {
+    float ss = res.finish(a, nrm ? inv_s : nullptr, 16 * mt + rr, 16 * t + 4 * q, v);
     if constexpr (EPI == GEPI_ACCUM_NORM) {
       ss += __shfl_xor(ss, 16, 64);
       ss += __shfl_xor(ss, 32, 64);
@@ -205,7 +195,7 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
   };
   // the waves' parts of tile t (double-buffered in each wave's own LDS), one barrier, and wave (t MT + mt) mod 8 adds them
   // up; it has read them before it reaches the next barrier, which the next write to them follows
-  auto meet = [&](int t, const WkRes<EPI> (&res)[MT]) __attribute__((always_inline)) {
+  auto meet = [&](int t, const Ahead (&res)[MT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) *(gf32x4*)(own + ((t & 1) * MT + mt) * 1024 + 16 * lane) = acc[mt][0] + acc[mt][1];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -235,12 +225,29 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
 #pragma unroll
   for (int s = 0; s < NS; ++s) turn_x(x[s]);
   if (nrm) nr.done(a, wave, lane, inv_s);  // (read after the first tile's barrier)
+  // what the outputs need besides their sums is requested before the tile's products (by every wave: which of them adds the tile up
+  // is not worth a branch here).  Behind the sums it was one or two trips to memory at the end of a launch.
+  // bf16 weights, 8 steps of TinyLlama with 12 rows 8.60 -> 8.44 ms; beside a quantised format's decode it gave nothing (8 rows, TinyLlama
+  // 0.5 % faster, Mistral 0.9 % slower): there the residual only
+  int pos[MT], slot[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    pos[mt] = slot[mt] = 0;
+    if constexpr (EPI == GEPI_QKV && BF) {
+      const int m = min(16 * mt + rr, a.M - 1);
+      pos[mt] = a.pos[m];
+      if (a.slot) slot[mt] = a.slot[m];
+    }
+  }
+  auto ahead = [&](Ahead& res, int t, int mt) __attribute__((always_inline)) {
+    res.load(a, min(16 * mt + rr, a.M - 1), 16 * t + 4 * q, pos[mt], slot[mt]);
+  };
   for (int t = t0; t < t1; ++t) {
-    WkRes<EPI> res[MT];
+    Ahead res[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       acc[mt][0] = acc[mt][1] = gf32x4{0.f, 0.f, 0.f, 0.f};
-      res[mt].load(a, 16 * mt + rr, 16 * t + 4 * q);
+      ahead(res[mt], t, mt);
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -268,8 +275,8 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
   if (!last_flag) return;
   for (int i = wave; i < (t1 - t0) * MT; i += WK_W) {
     const int t = t0 + i / MT, mt = i % MT;
-    WkRes<EPI> res;
-    res.load(a, 16 * mt + rr, 16 * t + 4 * q);
+    Ahead res;
+    ahead(res, t, MT == 1 ? 0 : mt);
     gf32x4 v = gf32x4{0.f, 0.f, 0.f, 0.f};
     for (int k0 = 0; k0 < S; k0 += 4) {  // four slabs' loads in flight (past the last: read again, not added)
       gf32x4 part[4];
@@ -334,6 +341,7 @@ static bool wk_route(const GemmQArgs& a, WkRoute& r) {
   if (((size_t)(a.M - 1) * a.lda + a.K) * 2 >= 0xfffffff0u || (size_t)a.K * 32 >= 0x7fffffffu) return false;
   if (a.nrm_in && (a.nrm_parts <= 0 || a.nrm_parts % 4)) return false;
   if (a.epi == GEPI_SWIGLU_BF16 && a.ldc % 2) return false;
+  if (a.epi == GEPI_QKV && a.head_dim % 4) return false;  // (SkAhead)
   if (a.epi == GEPI_STORE_GLU && (a.glu_n0 % 4 || a.ldc16 % 2)) return false;
   if (a.epi != GEPI_SWIGLU_BF16 && a.ldc % 4) return false;
   if (a.epi == GEPI_ACCUM_NORM && (!a.nrm_g || !a.nrm_out16 || !a.nrm_part || a.N / 16 != a.nrm_parts)) return false;

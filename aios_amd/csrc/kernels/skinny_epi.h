@@ -78,6 +78,72 @@ __device__ __forceinline__ float sk_finish(const GemmQArgs& a, const float* inv_
   return 0.f;
 }
 
+// What a lane's outputs of row m, columns n .. n + 3 need besides their sum, requested by load() while the products run and used by
+// finish(): the residual, gain and bias (GEPI_ACCUM, GEPI_ACCUM_NORM), or RoPE's (cos, sin) of the two pairs and the place in q or the
+// cache (GEPI_QKV; head_dim a multiple of 4).  Other epilogues need nothing.  ALL false: the residual only.
+template <int EPI, bool ALL = true>
+struct SkAhead {
+  gf32x4 c, gain, bias;
+  size_t to;
+  __device__ __forceinline__ static int section(const GemmQArgs& a, int n) {  // q, k, v
+    return a.col0 + n < a.q_dim ? 0 : (a.col0 + n < a.q_dim + a.kv_dim ? 1 : 2);
+  }
+  // (m: a row there is; pos, slot: the row's)
+  __device__ __forceinline__ void load(const GemmQArgs& a, int m, int n, int pos, int slot) {
+    if constexpr (EPI == GEPI_ACCUM || EPI == GEPI_ACCUM_NORM) c = *(const gf32x4*)(a.C + (size_t)m * a.ldc + n);
+    if constexpr (ALL && EPI == GEPI_ACCUM_NORM) {
+      gain = *(const gf32x4*)(a.nrm_g + n);
+      if (a.bias16) bias = *(const gf32x4*)(a.bias16 + n);
+    }
+    if constexpr (ALL && EPI == GEPI_QKV) {
+      const int sect = section(a, n), hd = a.head_dim;
+      const int col = a.col0 + n, r = sect == 0 ? col : col - (sect == 1 ? a.q_dim : a.q_dim + a.kv_dim), head = r / hd, lr = r - head * hd;
+      c = gf32x4{1.f, 0.f, 1.f, 0.f};
+      if (sect < 2) {
+        const float2* cs = a.rope_cs + (size_t)pos * (hd >> 1) + (lr >> 1);
+        const float2 c0 = cs[0], c1 = cs[1];
+        c = gf32x4{c0.x, c0.y, c1.x, c1.y};
+      }
+      to = sect == 0 ? (size_t)m * a.q_dim + col : kv_offset(a.block_table, a.max_ctx / KV_BLOCK, slot, a.n_kv_heads, head, pos, hd) + lr;
+    }
+  }
+  // returns the sum of squares of the new residual (GEPI_ACCUM_NORM), else 0
+  __device__ __forceinline__ float finish(const GemmQArgs& a, const float* inv_s, int m, int n, gf32x4 v) const {
+    if (m >= a.M) return 0.f;
+    if constexpr (ALL && EPI == GEPI_ACCUM_NORM) {
+      if (inv_s) v *= inv_s[m];
+      if (a.bias16) v += bias;
+      const gf32x4 x = c + v;
+      *(gf32x4*)(a.C + (size_t)m * a.ldc + n) = x;
+      *(uint2*)(a.nrm_out16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(x[0] * gain[0], x[1] * gain[1]), pk_bf16(x[2] * gain[2], x[3] * gain[3]));
+      return (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
+    } else if constexpr (ALL && EPI == GEPI_QKV) {
+      if (inv_s) v *= inv_s[m];
+      const int sect = section(a, n);
+      if (sect < 2)  // (v's (1, 0) would turn an infinite value's partner into NaN)
+        v = gf32x4{v[0] * c[0] - v[1] * c[1], v[0] * c[1] + v[1] * c[0], v[2] * c[2] - v[3] * c[3], v[2] * c[3] + v[3] * c[2]};
+      if (sect == 0) {
+        float* q = a.q_out + to;  // (8-byte stores: q_out is not known to be aligned to more)
+        *(float2*)q = make_float2(v[0], v[1]);
+        *(float2*)(q + 2) = make_float2(v[2], v[3]);
+      } else {
+        bf16_t* cache = sect == 1 ? a.k_cache : a.v_cache;
+        const float inv = sect == 1 ? a.kv_inv_k : a.kv_inv_v;
+        if (a.kv_fp8) {
+          kv_store_pair(cache, to, to + 1, v[0], v[1], 1, inv);
+          kv_store_pair(cache, to + 2, to + 3, v[2], v[3], 1, inv);
+        } else {
+          *(uint32_t*)(cache + to) = pk_bf16(v[0], v[1]);
+          *(uint32_t*)(cache + to + 2) = pk_bf16(v[2], v[3]);
+        }
+      }
+      return 0.f;
+    } else {
+      return sk_finish<EPI>(a, inv_s, m, n, v, (const float4*)&c);
+    }
+  }
+};
+
 // The fused RMSNorm's consumer: inv_s[m] of MP rows from the producer's sums of squares (nrm_parts per row, a multiple
 // of 4), a wave per row, added up in a fixed order.  load() requests, done() writes inv_s (ordered by the caller).
 template <int MP, int NW>

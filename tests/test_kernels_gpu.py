@@ -1861,6 +1861,34 @@ def test_gemm_pfk_qkv(E, ts, tile, S, M, K, monkeypatch):
         assert ((got - ref).flatten(1).norm(dim=1) / ref.flatten(1).norm(dim=1)).max() < tol + 2.0 ** -8
 
 
+@pytest.mark.parametrize("kernel,M", [("pfk", 40), ("wk", 9)])
+def test_qkv_infinite_value_stays_alone(E, kernel, M, monkeypatch):
+    """V is not turned: an infinite sum does not reach its neighbour in the cache"""
+    if kernel == "pfk":
+        monkeypatch.setenv("AIOS_GEMM_PF_TILE", "64x-64")
+        monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", "1")
+    K, H, Hkv, hd, max_ctx = 256, 2, 1, 64, 256
+    rows = (H * hd, Hkv * hd, Hkv * hd)
+    Ws = [torch.ones(n, K) for n in rows]
+    Ws[2][4] = 3e38  # (row 4 of V: its sum overflows)
+    mats = [E.QMatrix(int(GGMLType.BF16), n, K, w.to(torch.bfloat16).view(torch.int16).numpy().reshape(-1)) for n, w in zip(rows, Ws)]
+    A = torch.ones(M, K, dtype=torch.bfloat16, device="cuda")
+    pos, slot = torch.arange(M, dtype=torch.int32, device="cuda"), torch.zeros(M, dtype=torch.int32, device="cuda")
+    cs = torch.ones(max_ctx, hd // 2, 2, device="cuda")
+    kd, vd = (torch.zeros(max_ctx // 128, Hkv, 128, hd, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    q = torch.zeros(M, rows[0], device="cuda")
+    more = dict(head_dim=hd, q_dim=rows[0], kv_dim=rows[1], n_kv_heads=Hkv, max_ctx=max_ctx, rope_cs=cs.data_ptr(), pos=pos.data_ptr(),
+                slot=slot.data_ptr(), q_out=q.data_ptr(), k_cache=kd.data_ptr(), v_cache=vd.data_ptr())
+    if kernel == "pfk":
+        assert E.gemm_pf_fuses(mats, M, E.GEPI_QKV, A.data_ptr(), K, 0, sum(rows), more)
+    else:
+        assert E.gemm_wk_serves(mats, M, E.GEPI_QKV, more=more)
+    E.gemm_q(A.data_ptr(), K, mats, M, 0, 0, sum(rows), E.GEPI_QKV, stream(), more=more)
+    torch.cuda.synchronize()
+    v = vd[0, 0, :M].float().cpu()
+    assert bool(torch.isinf(v[:, 4]).all()) and bool((v[:, [0, 1, 2, 3, 5, 6, 7]] == K).all())
+
+
 def test_gemm_pfk_is_not_taken(E, monkeypatch):
     """calls that its 16-byte stores or its workspace do not fit keep the other tiles: C off 16 bytes, a pitch off 4, more slices than
     blocks; their results are the same products"""
