@@ -1366,9 +1366,9 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
         GemmQArgs o = out;
         nrm_out(o, gain);
         nrm_in(in);
-        return lf && fuses(o) && fuses(in);
+        return fuses(o) && fuses(in);
       };
-      const bool o_normed = fnp || pair(g, L.ffn_norm, gu);
+      const bool o_normed = fnp || (lf && pair(g, L.ffn_norm, gu));
       if (o_normed) nrm_out(g, L.ffn_norm);
       gemm(g);
       if (tp) allreduce(gm_part_, (size_t)n * d, gm_x_);
@@ -1380,7 +1380,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
       g.A = gm_ff16_; g.lda = ff; g.M = n; g.K = ff; g.nseg = 1; g.seg[0] = L.wdown.w; g.N = d; g.ldc = d;
       if (tp) { g.C = gm_part_; g.epi = GEPI_STORE; } else { g.C = gm_x_; g.epi = GEPI_ACCUM; }
       // (the last layer: lm_head normalises its row)
-      down_normed = l + 1 < cfg_.n_layers && pair(g, layers_[l + 1].attn_norm, qkv_of(layers_[l + 1]));
+      down_normed = lf && l + 1 < cfg_.n_layers && pair(g, layers_[l + 1].attn_norm, qkv_of(layers_[l + 1]));
       if (down_normed || (fnp && l + 1 < cfg_.n_layers)) nrm_out(g, layers_[l + 1].attn_norm);
       gemm(g);
       if (tp) allreduce(gm_part_, (size_t)n * d, gm_x_);
