@@ -271,9 +271,66 @@ __global__ void __launch_bounds__(256) qkv_post_row_kernel(QkvPostArgs a) {
   }
 }
 
+// QK-norm or NeoX pairs, heads of 128, no bias (Qwen3), prompts: a workgroup per token row, a wave every fourth head and a lane the
+// pair it holds in each of them, so position, cache block, (cos, sin) and gains are read once a row and four heads' loads are in flight
+// (a wave per token and head read all of them in a chain: 711 rows of 32 + 2 x 8 heads, 32 MB, 17 us -> 10.8).  A few rows are the
+// other kernel's: there each head has a wave of its own.
+__global__ void __launch_bounds__(256) qkv_post_head_kernel(QkvPostArgs a) {
+  constexpr int HD = 128, HALF = 64, UNR = 4;
+  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int H = a.n_heads, Hkv = a.n_kv_heads, nh = H + 2 * Hkv;
+  const int pos = a.pos[t], slot = a.slot ? a.slot[t] : 0;
+  const size_t kvbase = (((size_t)kv_block(a.block_table, a.max_ctx / KV_BLOCK, slot, pos) * Hkv) * KV_BLOCK + (pos % KV_BLOCK)) * HD;
+  const float2 cs = a.rope_cs[(size_t)pos * HALF + lane];
+  const int ra = a.rope_neox ? lane : 2 * lane, rb = a.rope_neox ? lane + HALF : 2 * lane + 1;  // the pair of q and k; v's: 2 lane, 2 lane + 1
+  const float qa = a.q_norm ? a.q_norm[ra] : 1.f, qb = a.q_norm ? a.q_norm[rb] : 1.f;
+  const float ka = a.k_norm ? a.k_norm[ra] : 1.f, kb = a.k_norm ? a.k_norm[rb] : 1.f;
+  const float* src = a.qkv + (size_t)t * a.ldqkv;
+  for (int h0 = wave; h0 < nh; h0 += 4 * UNR) {
+    float x[UNR], y[UNR];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      const int h = min(h0 + 4 * u, nh - 1);
+      const bool v = h >= H + Hkv;
+      x[u] = src[h * HD + (v ? 2 * lane : ra)];
+      y[u] = src[h * HD + (v ? 2 * lane + 1 : rb)];
+    }
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      const int h = h0 + 4 * u;
+      if (h >= nh) break;
+      const int part = h < H ? 0 : (h < H + Hkv ? 1 : 2), head = part == 0 ? h : (part == 1 ? h - H : h - H - Hkv);
+      float v0 = x[u], v1 = y[u];
+      if (part < 2) {
+        if (part == 0 ? a.q_norm != nullptr : a.k_norm != nullptr) {
+          const float inv = rsqrtf(wave_sum(v0 * v0 + v1 * v1) / (float)HD + a.eps);
+          v0 *= inv * (part == 0 ? qa : ka);
+          v1 *= inv * (part == 0 ? qb : kb);
+        }
+        const float o0 = v0 * cs.x - v1 * cs.y, o1 = v0 * cs.y + v1 * cs.x;
+        v0 = o0;
+        v1 = o1;
+      }
+      const int ia = part == 2 ? 2 * lane : ra, ib = part == 2 ? 2 * lane + 1 : rb;
+      if (part == 0) {
+        float* q = a.q_out + ((size_t)t * H + head) * HD;
+        q[ia] = v0;
+        q[ib] = v1;
+      } else {
+        const size_t base = kvbase + (size_t)head * KV_BLOCK * HD;
+        kv_store_pair(part == 1 ? a.k_cache : a.v_cache, base + ia, base + ib, v0, v1, a.kv_fp8, part == 1 ? a.kv_inv_k : a.kv_inv_v);
+      }
+    }
+  }
+}
+
 void launch_qkv_post(const QkvPostArgs& a, hipStream_t st) {
   if (!a.rope_neox && !a.q_norm && !a.k_norm && !a.bias && a.rope_cs && a.head_dim % 2 == 0) {
     hipLaunchKernelGGL(qkv_post_row_kernel, dim3(a.T), dim3(256), 0, st, a);
+    return;
+  }
+  if (a.T > 32 && a.head_dim == 128 && a.rope_cs && !a.bias) {
+    hipLaunchKernelGGL(qkv_post_head_kernel, dim3(a.T), dim3(256), 0, st, a);
     return;
   }
   const int items = a.T * (a.n_heads + 2 * a.n_kv_heads);

@@ -704,6 +704,36 @@ def test_rmsnorm(E, n, y_off):
 
 
 @pytest.mark.parametrize("neox", [0, 1])
+@pytest.mark.parametrize("norm", ["", "q", "qk"])
+@pytest.mark.parametrize("T,H,Hkv", [(33, 8, 2), (70, 32, 8), (40, 5, 1)])
+def test_qkv_post_rows_match_one_by_one(E, neox, norm, T, H, Hkv):
+    """more than 32 rows of 128-wide heads with QK-norm or NeoX pairs (a workgroup a row) against the same rows in calls of one; sums of 128
+    squares in another order: 2^-22 of a value, a bf16 step at a rounding boundary"""
+    if not neox and not norm:
+        pytest.skip("the plain kernel's")
+    hd, max_ctx, slots = 128, 256, 2
+    qkv = torch.randn(T, (H + 2 * Hkv) * hd + 4, device="cuda")
+    qn, kn = (torch.rand(hd, device="cuda") + 0.5 for _ in range(2))
+    pos = (torch.arange(T, dtype=torch.int32) * 3 % 200 + torch.arange(T, dtype=torch.int32) // 67).cuda()
+    slot = (torch.arange(T, dtype=torch.int32) % slots).cuda()
+    ang = torch.arange(max_ctx)[:, None].double() * 1e6 ** (-2.0 * torch.arange(hd // 2).double() / hd)
+    cs = torch.stack([ang.cos(), ang.sin()], -1).float().cuda()
+    kp, bt = paged_cache(torch.zeros(slots, Hkv, max_ctx, hd, dtype=torch.bfloat16), True, seed=3)
+    bt = bt.cuda()
+    outs = []
+    for rows in (T, 1):
+        q, k, v = torch.zeros(T, H * hd, device="cuda"), kp.cuda(), torch.zeros_like(kp).cuda()
+        for r in range(0, T, rows):
+            E.qkv_post(qkv[r:].data_ptr(), qkv.shape[1], rows, H, Hkv, hd, qn.data_ptr() if "q" in norm else 0, kn.data_ptr() if "k" in norm else 0,
+                       1e-6, neox, 1e6, pos[r:].data_ptr(), slot[r:].data_ptr(), q[r:].data_ptr(), k.data_ptr(), v.data_ptr(), max_ctx, stream(),
+                       bt.data_ptr(), cs.data_ptr())
+        torch.cuda.synchronize()
+        outs.append((q.double(), k.double(), v.double()))
+    for i, (x, y) in enumerate(zip(*outs)):
+        assert float(y.abs().max()) > 1 and float((x - y).norm() / y.norm()) < (2.0 ** -22 if i == 0 else 2.0 ** -12 if i == 1 else 1e-30)
+
+
+@pytest.mark.parametrize("neox", [0, 1])
 def test_qkv_post_qknorm(E, neox):
     T, H, Hkv, hd, max_ctx = 4, 4, 2, 128, 128
     qkv = torch.randn(T, (H + 2 * Hkv) * hd, device="cuda")
