@@ -341,7 +341,7 @@ static bool wk_route(const GemmQArgs& a, WkRoute& r) {
   if (((size_t)(a.M - 1) * a.lda + a.K) * 2 >= 0xfffffff0u || (size_t)a.K * 32 >= 0x7fffffffu) return false;
   if (a.nrm_in && (a.nrm_parts <= 0 || a.nrm_parts % 4)) return false;
   if (a.epi == GEPI_SWIGLU_BF16 && a.ldc % 2) return false;
-  if (a.epi == GEPI_QKV && a.head_dim % 4) return false;  // (SkAhead)
+  if (a.epi == GEPI_QKV && bf && a.head_dim % 4) return false;  // (SkAhead: a lane's four columns in one head; quantised formats go by pairs)
   if (a.epi == GEPI_STORE_GLU && (a.glu_n0 % 4 || a.ldc16 % 2)) return false;
   if (a.epi != GEPI_SWIGLU_BF16 && a.ldc % 4) return false;
   if (a.epi == GEPI_ACCUM_NORM && (!a.nrm_g || !a.nrm_out16 || !a.nrm_part || a.N / 16 != a.nrm_parts)) return false;

@@ -1216,6 +1216,32 @@ def sum_tol(t, K):
     return K * 2.0 ** -24 + (0.0 if t == "BF16" else 2.0 ** -13)
 
 
+@pytest.mark.parametrize("t", ["Q4_K", "Q6_K", "BF16"])
+def test_gemm_wk_qkv_heads_of_pairs(E, t, monkeypatch):
+    """heads of a size that is no multiple of 4: quantised formats turn and store pairs and are served, bf16 leaves them to the skinny
+    GEMM; the same q and cache from either, to the error that each may have against float64 and, in the cache, a bf16 step of a value"""
+    K, M, H, hd, max_ctx = 512, 9, 32, 6, 256
+    n = H * hd
+    mats = [small_mat(E, t, n, K, 41 + i)[0] for i in range(3)]
+    g = torch.Generator().manual_seed(4)
+    A = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    cs = torch.randn(max_ctx, hd // 2, 2, generator=g).cuda()
+    pos = (torch.arange(M, dtype=torch.int32) * 5).cuda()
+    outs = []
+    for wk in ("1", "0"):
+        monkeypatch.setenv("AIOS_GEMM_WK", wk)
+        q = torch.zeros(M, n, device="cuda")
+        kd, vd = (torch.zeros(max_ctx // 128, H, 128, hd, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        more = dict(head_dim=hd, q_dim=n, kv_dim=n, n_kv_heads=H, max_ctx=max_ctx, rope_cs=cs.data_ptr(), pos=pos.data_ptr(),
+                    q_out=q.data_ptr(), k_cache=kd.data_ptr(), v_cache=vd.data_ptr())
+        assert E.gemm_wk_serves(mats, M, E.GEPI_QKV, more=more) == (wk == "1" and t != "BF16")
+        E.gemm_q(A.data_ptr(), K, mats, M, 0, 0, 3 * n, E.GEPI_QKV, stream(), more=more)
+        torch.cuda.synchronize()
+        outs.append((q.double(), kd.double(), vd.double()))
+    for x, y, step in zip(*outs, (0.0, 2.0 ** -8, 2.0 ** -8)):
+        assert float(y.abs().max()) > 0.1 and float((x - y).norm() / y.norm()) < 2 * sum_tol(t, K) + step
+
+
 def test_gemm_wk_leaves_q6k_down_to_the_ring(E):
     """long K up to 16 rows where the ring's tiles in eight slices cover three quarters of the CUs; not below, and no other
     format; the packed Q6_K QKV from 17 rows up has no form with a wave's two stages"""
