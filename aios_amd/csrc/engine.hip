@@ -1269,8 +1269,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
   static const bool short_fuse = !(std::getenv("AIOS_PREFILL_SHORT_FUSE") && std::atoi(std::getenv("AIOS_PREFILL_SHORT_FUSE")) == 0);
   for (int r0 = 0; r0 < T; r0 += gm_rows_) {
     const int n = std::min(gm_rows_, T - r0);
-    // (the fused epilogues are the batched-decode GEMMs': chunks of <= 32 rows; longer chunks take the prefill
-    // GEMM, kernels/gemm_pf.hip, with the plain epilogues)
+    // chunks of <= 32 rows: the batched-decode GEMMs and their fused epilogues
     const bool sh = short_fuse && !tp && n <= 32;
     const bool fnp = sh && gm_nparts_ > 0;
     // longer chunks: the same fusions where both products of a norm, or the QKV product, run on tiles with K over the waves

@@ -423,7 +423,17 @@ bool gemm_pf_serves(const GemmQArgs& a) {
 // ... on tiles with K over the waves: those take GEPI_QKV with any plan, GEPI_ACCUM_NORM and nrm_in (a part per 64 columns)
 bool gemm_pf_fuses(const GemmQArgs& a) {
   if (!pf_env("AIOS_GEMM_PF", 1) || a.M < pf_env("AIOS_GEMM_PF_MIN_M", 33) || !pf_eligible(a)) return false;
-  return pf_plan(a, a.seg[0].qtype == QT_BF16).bn < 0;
+  const bool bf = a.seg[0].qtype == QT_BF16;
+  const PfPlan p = pf_plan(a, bf);
+  if (p.bn >= 0) return false;
+  // (... and would run the plain product on: a split plan of other tiles falls back to the best unsplit one, which may be of these
+  // tiles, but was timed as the slower)
+  GemmQArgs b = a;
+  b.nrm_in = nullptr;
+  if (a.epi == GEPI_ACCUM_NORM) b.epi = GEPI_ACCUM;
+  if (a.epi == GEPI_QKV) { b.epi = GEPI_STORE; b.C = a.q_out; b.ldc = a.N; }
+  const PfPlan q = pf_plan(b, bf);
+  return p.bm == q.bm && p.bn == q.bn && p.s == q.s;
 }
 
 // the plan the launcher would pick (bindings / tools)

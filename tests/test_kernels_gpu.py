@@ -1964,6 +1964,27 @@ def test_gemm_pfk_is_not_taken(E, monkeypatch):
     assert E.gemm_pf_plan(mats, M, E.GEPI_STORE, 0)[0] == 0
 
 
+def test_gemm_pf_fuses_where_the_plain_product_runs_so(E):
+    """RoPE and the cache go into the QKV product only where its plain form's plan is a tile with K over the waves.  A split plan of other
+    tiles is faster than the best unsplit one, whatever tiles that has, and its product stays plain."""
+    K, M, H, Hkv, hd, max_ctx = 1152, 100, 4, 2, 64, 256
+    rows = (H * hd, Hkv * hd, Hkv * hd)
+    N, cus = sum(rows), torch.cuda.get_device_properties(0).multi_processor_count
+    mats = [small_mat(E, "BF16", n, K, 51 + i)[0] for i, n in enumerate(rows)]
+    A = torch.zeros(M, K, dtype=torch.bfloat16, device="cuda")
+    pos = torch.arange(M, dtype=torch.int32, device="cuda")
+    cs, q = torch.zeros(max_ctx, hd // 2, 2, device="cuda"), torch.zeros(M, rows[0], device="cuda")
+    kd, vd = (torch.zeros(max_ctx // 128, Hkv, 128, hd, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    more = dict(head_dim=hd, q_dim=rows[0], kv_dim=rows[1], n_kv_heads=Hkv, max_ctx=max_ctx, rope_cs=cs.data_ptr(), pos=pos.data_ptr(),
+                q_out=q.data_ptr(), k_cache=kd.data_ptr(), v_cache=vd.data_ptr())
+    bf = int(GGMLType.BF16)
+    for best, one, fuses in (((64, 128, 2), (64, -64, 1), False), ((64, -64, 2), (128, 128, 1), True), ((64, -64, 1), (64, -64, 1), True),
+                             ((64, 128, 1), (64, 128, 1), False)):
+        key = [N, K, 128, E.GEPI_STORE, bf, bf, 3, rows[0], rows[0] + rows[1], cus]
+        E.gemm_pf_import(key + list(best) + [0] + key + list(one) + [1])
+        assert E.gemm_pf_fuses(mats, M, E.GEPI_QKV, A.data_ptr(), K, 0, N, more) == fuses, (best, one)
+
+
 def pf_plan_entry(E, N, K, M, epi, bm, bn, S, s1=0):
     """one line of a plan list for a bf16 matrix: shape, row bucket, epilogue, formats, segments, CUs; tile, slices, map"""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
