@@ -1,6 +1,8 @@
 // Host side of the prefill GEMM (gemm_pf.h): which launches it serves and the tile / split-K plan.
 #include <algorithm>
+#include <climits>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <map>
@@ -111,9 +113,9 @@ static std::map<PfKey, PfPlan>& pf_tuned() {
   static std::map<PfKey, PfPlan> m;
   return m;
 }
-// the best plan without split-K per key (GEPI_QKV launches: the RoPE / KV-cache epilogue cannot
-// take split partials; they use the STORE shape's tuned S = 1 plan -- tuning them for real would
-// write the KV cache)
+// the best plan without split-K per key: GEPI_QKV launches whose STORE shape has a split plan of other tiles than those with K over the waves
+// (their RoPE / KV-cache epilogue takes no split partials; tuning it for real would write the KV cache), launches with less workspace than
+// the best plan's slabs take, and AIOS_GEMM_PF_DETERMINISTIC
 static std::map<PfKey, PfPlan>& pf_tuned_s1() {
   static std::map<PfKey, PfPlan> m;
   return m;
@@ -148,6 +150,14 @@ static bool pf_plan_ok(const GemmQArgs& a, const PfPlan& p, bool bf) {
   return bf || p.bn != 256 || a.K / 256 / p.s >= 1;  // (pf8c slices whole 256-blocks)
 }
 
+// ... with all the workspace it may ask for
+static bool pf_plan_fits(GemmQArgs a, const PfPlan& p, bool bf) {
+  float none;
+  int tickets;
+  a.ws = &none; a.ws_bytes = SIZE_MAX; a.cnt = &tickets; a.cnt_len = INT_MAX;
+  return pf_plan_ok(a, p, bf);
+}
+
 // every plan the launcher could run for these args (ksplit > 0 pins the split)
 static std::vector<PfPlan> pf_candidates(const GemmQArgs& a, bool bf) {
   std::vector<PfPlan> out;
@@ -180,7 +190,7 @@ static PfPlan pf_plan(const GemmQArgs& a, bool bf) {
     };
     PfPlan p;
     if (!pf_deterministic()) p = at(pf_tuned());
-    if (!p.bm && (pf_deterministic() || a.epi == GEPI_QKV)) p = at(pf_tuned_s1());  // (the best without split partials)
+    if (!p.bm) p = at(pf_tuned_s1());  // (the best without split partials or slabs)
     if (p.bm) return p;
   }
   return pf_model_plan(a, bf, false);
@@ -279,7 +289,8 @@ static bool pf_eligible(const GemmQArgs& a) {
 // again and again lies in the caches (with it, the plans of 2048-wide bf16 layers changed from process to process, and a
 // pass of 1500 rows with them: 8.65 to 9.24 ms; so: 8.61 to 8.63).  Returns the number of plans timed.  A key already
 // planned in this process -- tuned by an earlier engine or imported, gemm_pf_import -- is left if the kernels take its
-// plan: a second engine never changes the plans a first one runs.
+// plan, given the workspace: a second engine never changes the plans a first one runs (one whose workspace, its widest product's, is too
+// small for a plan's slabs runs the best plan without).
 //
 // Every candidate that the model puts within twice its best (no plan within 3 % of the fastest lay beyond, for five models'
 // 420 keys) in two launches, then those within 12 % of the fastest in four, forwards and backwards; the modelled plan stays
@@ -297,7 +308,7 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
     }
     std::lock_guard<std::mutex> g(pf_mu);
     const auto it = pf_tuned().find(k);
-    if (it == pf_tuned().end() || !pf_plan_ok(a, it->second, a.seg[0].qtype == QT_BF16)) work.push_back({k, {&a}});
+    if (it == pf_tuned().end() || !pf_plan_fits(a, it->second, a.seg[0].qtype == QT_BF16)) work.push_back({k, {&a}});
   }
   std::vector<hipEvent_t> ev;
   std::set<std::tuple<int, int, int, int, int, int>> loaded;  // (kernels that have run)

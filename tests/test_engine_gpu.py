@@ -580,6 +580,40 @@ def test_prefill_plans_cover_every_projection_and_row_bucket():
     assert np.isfinite(np.asarray(eng.prefill(0, list(range(3, 203)), 0, True))).all()
 
 
+def test_prefill_plans_of_a_first_engine_stay(monkeypatch):
+    """A plan with K sliced over workgroups asks for a workspace, and an engine's is its widest product's (here: cut by AIOS_SKINNY_SMAX).
+    A second engine without room for a plan of the first leaves it and runs the best plan that needs none; a plan that the
+    kernels do not take at all is timed again."""
+    import dataclasses
+
+    from aios_amd.runtime import native
+    from aios_amd.runtime.loader import random_engine
+
+    m = native.require()
+    cfg = dataclasses.replace(get_preset("test-mistral-shape"), n_layers=2, d_model=1280, vocab_size=512)
+    prompt = [1] + [int(t) for t in np.random.default_rng(5).integers(3, 512, 249)]
+    a = random_engine(cfg, "Q4_K_M", seed=3, max_ctx=512, max_batch=2)
+    q4, cus = int(GGMLType.Q4_K), torch.cuda.get_device_properties(0).multi_processor_count
+
+    def entry(rows, bm, bn, S):  # the output projection's: four slices of 256 rows are 5 MB
+        return [1280, 1024, rows, m.GEPI_ACCUM, q4, q4, 1, 0, 0, cus, bm, bn, S, 0]
+
+    def plans():
+        v = list(m.gemm_pf_export())
+        return [v[i:i + 14] for i in range(0, len(v), 14)]
+
+    sliced, none = entry(256, 64, -64, 4), entry(320, 48, 128, 1)
+    assert {tuple(p[:3]) for p in plans()} >= {(1280, 1024, 256), (1280, 1024, 320)}
+    m.gemm_pf_import(sliced + none)
+    la = np.asarray(a.prefill(0, prompt, 0, True))
+    monkeypatch.setenv("AIOS_SKINNY_SMAX", "1")
+    b = random_engine(cfg, "Q4_K_M", seed=3, max_ctx=512, max_batch=2)
+    lb = np.asarray(b.prefill(0, prompt, 0, True))
+    assert sliced in plans() and none not in plans()
+    # (bf16 activations: another order of sums moves one in some hundreds by 2^-8 of itself, a layer; two layers)
+    assert np.isfinite(la).all() and np.abs(la - lb).max() < 1e-2 * np.abs(la).max()
+
+
 @pytest.mark.parametrize("deterministic", [False, True])
 def test_prefill_plans_persist_across_processes(tmp_path, deterministic):
     """with AIOS_GEMM_PF_PLANS naming a file, a second process installs the first's
