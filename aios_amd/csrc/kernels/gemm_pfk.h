@@ -116,13 +116,42 @@ inline bool pfk_epi_ok(const GemmQArgs& a, int bn) {
     case GEPI_STORE: case GEPI_ACCUM: return a.C && a.ldc % 4 == 0 && !off(a.C, 16);
     case GEPI_ACCUM_NORM:
       return a.C && a.ldc % 4 == 0 && !off(a.C, 16) && bn >= 64 && a.nrm_g && !off(a.nrm_g, 16) && a.nrm_out16 && !off(a.nrm_out16, 8) && a.nrm_part &&
-             a.nrm_parts == a.N / 64 && (!a.bias16 || !off(a.bias16, 16));
+             a.nrm_parts == a.N / 64 && !a.bias16;
     case GEPI_SWIGLU_BF16: return a.C16 && a.ldc % 2 == 0 && !off(a.C16, 4);
     case GEPI_STORE16: return a.C16 && a.ldc % 4 == 0 && !off(a.C16, 8);
     case GEPI_QKV:  // (a lane's four columns in one head, its stores whole)
       return a.q_out && a.k_cache && a.v_cache && !off(a.q_out, 16) && !off(a.k_cache, 8) && !off(a.v_cache, 8) && a.head_dim % 4 == 0 && a.q_dim % 4 == 0 && a.kv_dim % 4 == 0;
     default: return false;
   }
+}
+
+// host: f(MT, CT, NG) of a tile, false if there is none: 64 to 160 rows; 32 columns (four waves), 64 or 128 (eight)
+template <typename F>
+inline bool pfk_tile(int bm, int bn, F f) {
+#define PFK_T(N) std::integral_constant<int, N> {}
+  auto cols = [&](auto mt) {
+    switch (bn) {
+      case 32: return f(mt, PFK_T(1), PFK_T(1));
+      case 64: return f(mt, PFK_T(2), PFK_T(2));
+      case 128: return f(mt, PFK_T(4), PFK_T(2));
+      default: return false;
+    }
+  };
+  switch (bm) {
+    case 64: return cols(PFK_T(2));
+    case 96: return cols(PFK_T(3));
+    case 128: return cols(PFK_T(4));
+    case 160: return cols(PFK_T(5));
+    default: return false;
+  }
+#undef PFK_T
+}
+
+// host: whether S slices of K have the workspace for their slabs and a ticket per tile
+inline bool pfk_slabs_ok(const GemmQArgs& a, int bm, int bn, int S) {
+  if (S == 1) return true;
+  const size_t tiles = (size_t)(a.N / bn) * ((a.M + bm - 1) / bm), by = (size_t)S * tiles * bm * bn * 4;
+  return a.ws && a.cnt && tiles <= (size_t)a.cnt_len && by <= a.ws_bytes && by < 0x7fffffff;
 }
 
 // ---- end of a tile: the four partial sums of every output, the slices of K, the epilogue
@@ -149,11 +178,8 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
   // What an output needs besides its sum is requested ahead: a load behind a store to what may be the same place would wait for it, row by
   // row.  us, residual so -> ahead: 4096 x 4096 Q4_K, 300 / 700 rows 22 -> 20, 40 -> 33; 4096 x 14336, 300 rows Q4_K 51 -> 46, Q6_K
   // 63 -> 56; 130 rows Q6_K 39 -> 35.  6144 x 4096 to q and the cache, 130 rows in two slices 27 -> 25.
-  gf32x4 gain = {}, bias = {};
-  if constexpr (EPI == GEPI_ACCUM_NORM) {
-    gain = *(const gf32x4*)(a.nrm_g + n);
-    if (a.bias16) bias = *(const gf32x4*)(a.bias16 + n);
-  }
+  gf32x4 gain = {};
+  if constexpr (EPI == GEPI_ACCUM_NORM) gain = *(const gf32x4*)(a.nrm_g + n);
   const int hd = EPI == GEPI_QKV ? a.head_dim : 4;
   const int sect = EPI != GEPI_QKV || n < a.q_dim ? 0 : (n < a.q_dim + a.kv_dim ? 1 : 2);  // q, k, v
   const int nr = sect == 0 ? n : n - (sect == 1 ? a.q_dim : a.q_dim + a.kv_dim), head = nr / hd, lr = nr - head * hd;
@@ -183,7 +209,7 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
     const int m = m0 + row;
     if (a.nrm_in) v *= inv_s[row];
     if constexpr (EPI == GEPI_ACCUM_NORM) {
-      const gf32x4 x = h_.c + (v + bias);
+      const gf32x4 x = h_.c + v;
       *(gf32x4*)(a.C + (size_t)m * a.ldc + n) = x;
       *(uint2*)(a.nrm_out16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(x[0] * gain[0], x[1] * gain[1]), pk_bf16(x[2] * gain[2], x[3] * gain[3]));
       float ss = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);

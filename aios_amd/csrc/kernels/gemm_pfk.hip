@@ -3,28 +3,6 @@
 
 namespace aios {
 
-// f(MT, CT, NG) of a tile, false if there is none: 64 to 160 rows; 32 columns (four waves), 64 or 128 (eight)
-template <typename F>
-static bool pfk_tile(int bm, int bn, F f) {
-#define PFK_T(N) std::integral_constant<int, N> {}
-  auto cols = [&](auto mt) {
-    switch (bn) {
-      case 32: return f(mt, PFK_T(1), PFK_T(1));
-      case 64: return f(mt, PFK_T(2), PFK_T(2));
-      case 128: return f(mt, PFK_T(4), PFK_T(2));
-      default: return false;
-    }
-  };
-  switch (bm) {
-    case 64: return cols(PFK_T(2));
-    case 96: return cols(PFK_T(3));
-    case 128: return cols(PFK_T(4));
-    case 160: return cols(PFK_T(5));
-    default: return false;
-  }
-#undef PFK_T
-}
-
 // g(QT0, QT1) of the weights' formats, false for others
 template <typename G>
 static bool pfk_fmt(const GemmQArgs& a, G g) {
@@ -44,8 +22,7 @@ constexpr bool pfk_fits() {  // two blocks of weights beside the slots of X (160
   return PfkLayout<QT0, MT, CT, NG>::NWB >= 2 && PfkLayout<QT1, MT, CT, NG>::NWB >= 2;
 }
 
-// bm x bn tiles divide N and every segment (pf_plan_ok).  32-bit offsets into X and the
-// planes; K slices: workspace for their slabs, a ticket per tile
+// bm x bn tiles divide N and every segment (pf_plan_ok).  32-bit offsets into X and the planes
 bool pfk_serves(const GemmQArgs& a, int bm, int bn, int S) {
   if (a.epi == GEPI_STORE16 || !pfk_epi_ok(a, bn)) return false;
   if (S < 1 || S > a.K / 256 || a.K % 256) return false;
@@ -53,10 +30,7 @@ bool pfk_serves(const GemmQArgs& a, int bm, int bn, int S) {
   if ((size_t)a.M * a.lda * 2 >= 0xfffffff0u) return false;
   for (int s = 0; s < a.nseg; ++s)
     if ((size_t)a.seg[s].rows * a.K / 2 >= 0xfffffff0u) return false;
-  if (S > 1) {
-    const size_t tiles = (size_t)(a.N / bn) * ((a.M + bm - 1) / bm), by = (size_t)S * tiles * bm * bn * 4;
-    if (!a.ws || !a.cnt || tiles > (size_t)a.cnt_len || by > a.ws_bytes || by >= 0x7fffffff) return false;
-  }
+  if (!pfk_slabs_ok(a, bm, bn, S)) return false;
   return pfk_fmt(a, [&](auto q0, auto q1) {
     return pfk_tile(bm, bn, [&](auto mt, auto ct, auto ng) {
       return pfk_fits<decltype(q0)::value, decltype(q1)::value, decltype(mt)::value, decltype(ct)::value, decltype(ng)::value>();

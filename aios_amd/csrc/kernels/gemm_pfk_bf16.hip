@@ -129,44 +129,19 @@ __global__ void __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(N
   pfk_close<MT, CT, NG, EPI, false, L::TOTAL>(a, acc, m0, n0, sp, S, tile, ntile, last_flag, rows);
 }
 
-// f(MT, CT, NG) of a tile, false if there is none: 64 to 160 rows; 32 columns (four waves), 64 or 128 (eight)
-template <typename F>
-static bool pfkb_tile(int bm, int bn, F f) {
-#define PFK_T(N) std::integral_constant<int, N> {}
-  auto cols = [&](auto mt) {
-    switch (bn) {
-      case 32: return f(mt, PFK_T(1), PFK_T(1));
-      case 64: return f(mt, PFK_T(2), PFK_T(2));
-      case 128: return f(mt, PFK_T(4), PFK_T(2));
-      default: return false;
-    }
-  };
-  switch (bm) {
-    case 64: return cols(PFK_T(2));
-    case 96: return cols(PFK_T(3));
-    case 128: return cols(PFK_T(4));
-    case 160: return cols(PFK_T(5));
-    default: return false;
-  }
-#undef PFK_T
-}
-
-// bm x bn tiles divide N and every segment (pf_plan_ok).  Slots of 128 k; 32-bit offsets into X and W; K slices: workspace for their slabs, a ticket per tile
+// bm x bn tiles divide N and every segment (pf_plan_ok).  Slots of 128 k; 32-bit offsets into X and W
 bool pfkb_serves(const GemmQArgs& a, int bm, int bn, int S) {
   if (!pfk_epi_ok(a, bn)) return false;
   if (S < 1 || S > a.K / 128 || a.K % 128) return false;
   if ((size_t)a.M * a.lda * 2 >= 0xfffffff0u) return false;
   for (int s = 0; s < a.nseg; ++s)
     if (a.seg[s].qtype != QT_BF16 || (size_t)a.seg[s].rows * a.K * 2 >= 0xfffffff0u || ((uintptr_t)a.seg[s].p0 & 15)) return false;
-  if (S > 1) {
-    const size_t tiles = (size_t)(a.N / bn) * ((a.M + bm - 1) / bm), by = (size_t)S * tiles * bm * bn * 4;
-    if (!a.ws || !a.cnt || tiles > (size_t)a.cnt_len || by > a.ws_bytes || by >= 0x7fffffff) return false;
-  }
-  return pfkb_tile(bm, bn, [](auto, auto, auto) { return true; });
+  if (!pfk_slabs_ok(a, bm, bn, S)) return false;
+  return pfk_tile(bm, bn, [](auto, auto, auto) { return true; });
 }
 
 bool pfkb_run(const GemmQArgs& a, int bm, int bn, int S, hipStream_t st) {
-  return pfkb_tile(bm, bn, [&](auto mt, auto ct, auto ng) {
+  return pfk_tile(bm, bn, [&](auto mt, auto ct, auto ng) {
     constexpr int MT = decltype(mt)::value, CT = decltype(ct)::value, NG = decltype(ng)::value;
     constexpr int lds = PfkbLayout<MT, CT, NG>::TOTAL;
     const dim3 grid((a.N / bn) * ((a.M + bm - 1) / bm), S), block(256 * NG);
