@@ -946,6 +946,39 @@ def test_attention_prefill_causal(E, H, Hkv, hd, start, T, shuffle):
     assert err < 3e-2, err
 
 
+@pytest.mark.parametrize("H,Hkv,hd,start,T", [
+    (128, 16, 64, 0, 200), (128, 16, 64, 0, 400), (128, 16, 64, 0, 600), (32, 32, 128, 100, 300), (16, 16, 64, 2000, 20),
+    (24, 3, 64, 0, 300), (24, 3, 64, 0, 1500), (24, 3, 64, 0, 2800), (24, 3, 64, 3000, 40), (12, 6, 128, 60, 200), (5, 5, 128, 0, 300),
+    (40, 5, 128, 2500, 17), (16, 2, 64, 0, 2100), (16, 2, 64, 0, 4200), (2, 2, 64, 3900, 300), (8, 1, 64, 0, 4200), (4, 1, 128, 3000, 70),
+    (8, 4, 128, 0, 4200), (64, 8, 128, 0, 300), (64, 8, 128, 0, 700), (64, 8, 128, 0, 1100)])
+def test_attention_prefill_lists_of_heads(E, H, Hkv, hd, start, T):
+    """Every query block of every KV head is somebody's, whatever number of heads an XCD's list holds: more than eight, numbers that divide
+    nothing, one and two; lists within one round of the XCDs' CUs, two, and more; keys in one run and in several.  Against float64,
+    2^-9 on P and on the output."""
+    max_ctx, slot, G = 4224, 1, H // Hkv
+    g = torch.Generator().manual_seed(start + T + H)
+    kc, vc = ((torch.randn(2, Hkv, max_ctx, hd, generator=g) * w).to(torch.bfloat16) for w in (0.5, 1.0))
+    kp, bt = paged_cache(kc, True, seed=5)
+    vp, _ = paged_cache(vc, True, seed=5)
+    kp, vp, bt = kp.cuda(), vp.cuda(), bt.cuda()
+    q = torch.randn(T, H, hd, generator=g).cuda()
+    n = E.attn_prefill_ws_bytes(hd)
+    ws, scale = torch.full((n // 4,), float("nan"), device="cuda"), 1 / math.sqrt(hd)
+    out = torch.full((T, H * hd), float("nan"), dtype=torch.bfloat16, device="cuda")
+    E.attn_prefill(q.data_ptr(), kp.data_ptr(), vp.data_ptr(), slot, start, T, H, Hkv, hd, max_ctx, scale, out.data_ptr(),
+                   H * hd, stream(), bt.data_ptr(), ws=ws.data_ptr(), ws_bytes=n)
+    torch.cuda.synchronize()
+    L, f = start + T, scale * 1.4426950408889634
+    k, v = kc[slot, :, :L].cuda().double(), vc[slot, :, :L].cuda().double()
+    qq = (q * f).to(torch.bfloat16).double() / 1.4426950408889634
+    dead = torch.arange(L, device="cuda")[None, :] > torch.arange(start, L, device="cuda")[:, None]
+    got = out.view(T, H, hd).double()
+    for h in range(H):
+        s = (qq[:, h] @ k[h // G].T.contiguous()).masked_fill_(dead, float("-inf"))
+        ref = torch.softmax(s, -1) @ v[h // G]
+        assert float((got[:, h] - ref).norm() / ref.norm()) < 2 ** -8, h
+
+
 @pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (16, 8, 128)])
 @pytest.mark.parametrize("start,T", [(1023, 1), (960, 64), (1100, 37), (3777, 300), (961, 129), (4000, 31)])
 @pytest.mark.parametrize("fp8", [False, True])
