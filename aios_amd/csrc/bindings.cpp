@@ -4,6 +4,8 @@
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 
+#include <climits>
+#include <cstdint>
 #include <cstring>
 
 #include "comm.h"
@@ -114,6 +116,8 @@ GemmQArgs gemm_q_args(const std::vector<PyQMatrix*>& segs, int M, int epi, int k
   int n0 = 0;
   for (int s = 0; s < a.nseg; ++s) { a.seg[s] = segs[s]->w; a.seg_n0[s] = n0; n0 += segs[s]->w.rows; }
   a.M = M; a.N = n0; a.K = segs[0]->w.cols; a.epi = epi; a.ksplit = ksplit;
+  size_t most_ws = SIZE_MAX;
+  int most_cnt = INT_MAX;
   for (const auto& kv : more) {
     const std::string k = py::cast<std::string>(kv.first);
     auto ptr = [&](auto& f) { f = reinterpret_cast<std::decay_t<decltype(f)>>(py::cast<uintptr_t>(kv.second)); };
@@ -136,10 +140,15 @@ GemmQArgs gemm_q_args(const std::vector<PyQMatrix*>& segs, int M, int epi, int k
     else if (k == "q_out") ptr(a.q_out);
     else if (k == "k_cache") ptr(a.k_cache);
     else if (k == "v_cache") ptr(a.v_cache);
+    else if (k == "kv_fp8") num(a.kv_fp8);
+    else if (k == "kv_inv_k") num(a.kv_inv_k);
+    else if (k == "kv_inv_v") num(a.kv_inv_v);
+    else if (k == "ws_bytes") num(most_ws);    // (less of the workspace than there is)
+    else if (k == "cnt_len") num(most_cnt);
     else throw std::runtime_error("gemm_q: no field " + k);
   }
   GemmWs& g = gemm_ws(M, a.N);
-  a.ws = g.ws; a.ws_bytes = g.bytes; a.cnt = g.cnt; a.cnt_len = g.cnt_len;
+  a.ws = g.ws; a.ws_bytes = std::min(g.bytes, most_ws); a.cnt = g.cnt; a.cnt_len = std::min(g.cnt_len, most_cnt);
   return a;
 }
 

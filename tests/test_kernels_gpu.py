@@ -1978,23 +1978,31 @@ def test_qkv_infinite_value_stays_alone(E, kernel, M, monkeypatch):
     assert bool(torch.isinf(v[:, 4]).all()) and bool((v[:, [0, 1, 2, 3, 5, 6, 7]] == K).all())
 
 
-def test_gemm_pfk_is_not_taken(E, monkeypatch):
-    """calls that its 16-byte stores or its workspace do not fit keep the other tiles: C off 16 bytes, a pitch off 4, more slices than
-    blocks; their results are the same products"""
-    K, M = 512, 70
-    mats, W = pf_mats(E, "q4k", K)
-    N = W.shape[0]
+@pytest.mark.parametrize("t,most", [("Q4_K", 2), ("BF16", 4)])
+def test_gemm_pfk_is_not_taken(E, t, most):
+    """With a plan of tiles with K over the waves in place, the calls that their 16-byte stores or slabs do not fit keep the other tiles: C off
+    16 bytes, a pitch off 4, more slices than blocks of K, a byte or a ticket too few.  Their results are the same products."""
+    K, M, N = 512, 70, 704
+    m, W = small_mat(E, t, N, K, 61)
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
-    A, ref = x.cuda(), x.double() @ W.double().T
-    for off, ldc in ((1, N + 4), (0, N + 3), (0, N)):
-        buf = torch.zeros(M * ldc + 4, device="cuda")
-        E.gemm_q(A.data_ptr(), K, mats, M, buf[off:].data_ptr(), 0, ldc, E.GEPI_ACCUM, stream(), 0)
+    A, ref = x.cuda(), x.double() @ W.T
+    cus, buf = torch.cuda.get_device_properties(0).multi_processor_count, torch.empty(M * (N + 4) + 4, device="cuda")
+
+    def taken(S, off=0, ldc=N, **more):
+        E.gemm_pf_import([N, K, 96, E.GEPI_ACCUM, int(GGMLType[t]), int(GGMLType[t]), 1, 0, 0, cus, 64, -64, S, 0])
+        C = buf.zero_()[off:off + M * ldc]
+        E.gemm_q(A.data_ptr(), K, [m], M, C.data_ptr(), 0, ldc, E.GEPI_ACCUM, stream(), 0, more=more)
         torch.cuda.synchronize()
-        got = buf[off:off + M * ldc].view(M, ldc)[:, :N].cpu().double()
-        assert float((got - ref).norm() / ref.norm()) < 2 * 2.0 ** -9 / 3 ** 0.5 + K * 2.0 ** -24
-    monkeypatch.setenv("AIOS_GEMM_PF_TILE", "64x-64")
-    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", "3")
-    assert E.gemm_pf_plan(mats, M, E.GEPI_STORE, 0)[0] == 0
+        got = C.view(M, ldc)[:, :N].cpu().double()
+        assert float((got - ref).norm() / ref.norm()) < sum_tol(t, K)
+        return E.gemm_pf_fuses([m], M, E.GEPI_ACCUM, A.data_ptr(), K, C.data_ptr(), ldc, more)
+
+    assert taken(1) and not taken(1, off=1) and taken(1, off=4) and not taken(1, ldc=N + 3) and taken(1, ldc=N + 4)
+    assert taken(most) and not taken(most + 1)
+    tiles = 2 * N // 64  # (two row tiles)
+    by = 2 * tiles * 64 * 64 * 4
+    assert taken(2, ws_bytes=by, cnt_len=tiles) and not taken(2, ws_bytes=by - 1) and not taken(2, cnt_len=tiles - 1)
+    assert taken(1, ws_bytes=0, cnt_len=0)
 
 
 def test_gemm_pf_fuses_where_the_plain_product_runs_so(E):
