@@ -679,8 +679,10 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
   m.def("qkv_post",
         [](uintptr_t qkv, int ldqkv, int T, int H, int Hkv, int hd, uintptr_t q_norm, uintptr_t k_norm, float eps,
            int rope_neox, float rope_base, uintptr_t pos, uintptr_t slot, uintptr_t q_out, uintptr_t k_cache,
-           uintptr_t v_cache, int max_ctx, uintptr_t st, uintptr_t block_table, uintptr_t rope_cs) {
+           uintptr_t v_cache, int max_ctx, uintptr_t st, uintptr_t block_table, uintptr_t rope_cs, int kv_fp8, float kv_inv_k,
+           float kv_inv_v) {
           QkvPostArgs a;
+          a.kv_fp8 = kv_fp8; a.kv_inv_k = kv_inv_k; a.kv_inv_v = kv_inv_v;
           a.block_table = (const int*)block_table;
           a.qkv = (const float*)qkv; a.ldqkv = ldqkv; a.T = T; a.n_heads = H; a.n_kv_heads = Hkv; a.head_dim = hd;
           a.q_norm = (const float*)q_norm; a.k_norm = (const float*)k_norm; a.eps = eps; a.rope_neox = rope_neox;
@@ -691,7 +693,8 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
         py::arg("qkv"), py::arg("ldqkv"), py::arg("T"), py::arg("H"), py::arg("Hkv"), py::arg("hd"), py::arg("q_norm"),
         py::arg("k_norm"), py::arg("eps"), py::arg("rope_neox"), py::arg("rope_base"), py::arg("pos"), py::arg("slot"),
         py::arg("q_out"), py::arg("k_cache"), py::arg("v_cache"), py::arg("max_ctx"), py::arg("st"),
-        py::arg("block_table") = 0, py::arg("rope_cs") = 0);
+        py::arg("block_table") = 0, py::arg("rope_cs") = 0, py::arg("kv_fp8") = 0, py::arg("kv_inv_k") = 1.f,
+        py::arg("kv_inv_v") = 1.f);
   m.def("sample",
         [](uintptr_t logits, int ldl, int B, int V, uintptr_t temperature, uintptr_t top_k, uint64_t seed,
            uintptr_t tokens, uintptr_t pos, uintptr_t mask, uintptr_t st, uintptr_t top_p, uintptr_t ts) {

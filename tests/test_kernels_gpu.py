@@ -733,6 +733,27 @@ def test_qkv_post_rows_match_one_by_one(E, neox, norm, T, H, Hkv):
         assert float(y.abs().max()) > 1 and float((x - y).norm() / y.norm()) < (2.0 ** -22 if i == 0 else 2.0 ** -12 if i == 1 else 1e-30)
 
 
+@pytest.mark.parametrize("neox,norm", [(0, 1), (1, 0), (1, 1)])
+def test_qkv_post_rows_fp8(E, neox, norm):
+    """... and into an fp8 cache: the bf16 call's values at K's and V's own scales, to a code (those values are rounded to 8 bits first)"""
+    T, H, Hkv, hd, max_ctx, inv = 70, 8, 2, 128, 256, (150.0, 300.0)
+    g = torch.Generator().manual_seed(6)
+    qkv, qn, kn = (x.cuda() for x in (torch.randn(T, (H + 2 * Hkv) * hd, generator=g), torch.rand(hd, generator=g) + 0.5, torch.rand(hd, generator=g) + 0.5))
+    pos = (torch.arange(T, dtype=torch.int32) * 3).cuda()
+    cs = torch.nn.functional.normalize(torch.randn(max_ctx, hd // 2, 2, generator=g), dim=-1).cuda()
+    caches = []
+    for dt in (torch.bfloat16, torch.uint8):
+        q = torch.zeros(T, H * hd, device="cuda")
+        k, v = (torch.zeros(max_ctx // KVB, Hkv, KVB, hd, dtype=dt, device="cuda") for _ in range(2))
+        E.qkv_post(qkv.data_ptr(), qkv.shape[1], T, H, Hkv, hd, qn.data_ptr() * norm, kn.data_ptr() * norm, 1e-6, neox, 1e6, pos.data_ptr(), 0, q.data_ptr(),
+                   k.data_ptr(), v.data_ptr(), max_ctx, stream(), 0, cs.data_ptr(), kv_fp8=int(dt == torch.uint8), kv_inv_k=inv[0], kv_inv_v=inv[1])
+        torch.cuda.synchronize()
+        caches.append([unpaged(c.cpu(), 1, max_ctx)[0][:, pos.cpu().long()] for c in (k, v)])
+    for x, code, i in zip(*caches, inv):
+        off = (code.int() - fp8_codes(x, 1 / i)[0].int()).abs()
+        assert int(off.max()) <= 1 and float((off > 0).float().mean()) < 0.1 and int((code & 127).max()) == 0x7e
+
+
 @pytest.mark.parametrize("neox", [0, 1])
 def test_qkv_post_qknorm(E, neox):
     T, H, Hkv, hd, max_ctx = 4, 4, 2, 128, 128
@@ -1948,6 +1969,37 @@ def test_gemm_pfk_qkv(E, ts, tile, S, M, K, monkeypatch):
         got = unpaged(cache.cpu(), slots, max_ctx, bt)[slot, :, pos].double()
         # (8 bits of significand: a value just above a power of two is rounded by up to 2^-8 of itself)
         assert ((got - ref).flatten(1).norm(dim=1) / ref.flatten(1).norm(dim=1)).max() < tol + 2.0 ** -8
+
+
+@pytest.mark.parametrize("t,tile,S", [("Q4_K", "64x-128", 1), ("Q6_K", "96x-64", 2), ("BF16", "64x-32", 1), ("BF16", "128x-128", 2)])
+def test_gemm_pfk_qkv_fp8(E, t, tile, S, monkeypatch):
+    """the same into an fp8 cache, K and V at scales of their own: the codes of float64, or the next one where that lies within the sums'
+    error of a code's edge (one in some thousands; 2 % leaves room), and the saturated ones"""
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
+    K, M, H, Hkv, hd, max_ctx, inv = 512, 70, 4, 2, 64, 256, (48.0, 300.0)
+    rows = (H * hd, Hkv * hd, Hkv * hd)
+    mats, W = zip(*[small_mat(E, t, n, K, 81 + i) for i, n in enumerate(rows)])
+    g = torch.Generator().manual_seed(K + M)
+    A, pos = torch.randn(M, K, generator=g).to(torch.bfloat16), torch.arange(M) * 3 + 1
+    ang = torch.arange(max_ctx)[:, None].double() * 1e4 ** (-2.0 * torch.arange(hd // 2).double() / hd)
+    cs = torch.stack([ang.cos(), ang.sin()], -1).float().cuda()
+    Ad, posd, q = A.cuda(), pos.int().cuda(), torch.zeros(M, rows[0], device="cuda")
+    kd, vd = (torch.zeros(max_ctx // KVB, Hkv, KVB, hd, dtype=torch.uint8, device="cuda") for _ in range(2))
+    more = dict(head_dim=hd, q_dim=rows[0], kv_dim=rows[1], n_kv_heads=Hkv, max_ctx=max_ctx, rope_cs=cs.data_ptr(), pos=posd.data_ptr(),
+                q_out=q.data_ptr(), k_cache=kd.data_ptr(), v_cache=vd.data_ptr(), kv_fp8=1, kv_inv_k=inv[0], kv_inv_v=inv[1])
+    assert E.gemm_pf_fuses(list(mats), M, E.GEPI_QKV, Ad.data_ptr(), K, 0, sum(rows), more)
+    E.gemm_q(Ad.data_ptr(), K, list(mats), M, 0, 0, sum(rows), E.GEPI_QKV, stream(), more=more)
+    torch.cuda.synchronize()
+    _, yk, yv = (A.double() @ torch.cat(W).T).split(rows, 1)
+    a, b, c, s = yk.view(M, Hkv, hd)[..., 0::2], yk.view(M, Hkv, hd)[..., 1::2], ang.cos()[pos][:, None], ang.sin()[pos][:, None]
+    yk = torch.stack([a * c - b * s, a * s + b * c], -1).reshape(M, Hkv, hd)
+    for cache, y, k in ((kd, yk, inv[0]), (vd, yv.view(M, Hkv, hd), inv[1])):
+        want, _ = fp8_codes(y, 1 / k)
+        got = unpaged(cache.cpu(), 1, max_ctx)[0][:, pos].transpose(0, 1)
+        off = (got.int() - want.int()).abs()
+        assert int(off.max()) <= 1 and float((off > 0).float().mean()) < 0.02 and int((want & 127).max()) > 100
+    assert int((fp8_codes(yv, 1 / inv[1])[0] & 127).max()) == 0x7e  # (V reaches 448)
 
 
 @pytest.mark.parametrize("kernel,M", [("pfk", 40), ("wk", 9)])
