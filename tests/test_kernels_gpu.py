@@ -1872,6 +1872,36 @@ def test_gemm_pfk_bf16(E, monkeypatch, tile, K, S, epi):
         assert rel < K * 2.0 ** -24 + (2 * 2.0 ** -9 / 3 ** 0.5 if half else 2.0 ** -20), rel
 
 
+@pytest.mark.parametrize("tile", ["64x256", "128x256", "256x256", "64x-32", "96x-64", "160x-128"])
+@pytest.mark.parametrize("bias,act", [(1, ""), (0, "relu2"), (1, "relu2"), (1, "silu"), (0, "xielu")])
+def test_gemm_pf_store16_bias_and_activation(E, monkeypatch, tile, bias, act):
+    """bf16 weights and outputs, a bias and an activation of each column, in the tiles whose lanes hold columns of their own order.  Bound:
+    the products are exact, so the sums (K 2^-24), an exponential (2^-20) and the rounding of the result (half an ulp, evenly spread), doubled"""
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", "1")
+    K, N, M = 512, 512, 97
+    m, W = small_mat(E, "BF16", N, K, 7)
+    g = torch.Generator().manual_seed(N)
+    x, b = torch.randn(M, K, generator=g).to(torch.bfloat16), torch.randn(N, generator=g) * 2
+    A, bd, out = x.cuda(), b.cuda(), torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    bm, bn = (int(v) for v in tile.split("x"))
+    assert list(E.gemm_pf_plan([m], M, E.GEPI_STORE16, 0, out=out.data_ptr())) == [bm, bn, 1]
+    pos, neg, scale = 0.7, 0.4, 1.25
+    kw = dict(unary=1 + {"relu2": E.ACT_RELU2, "silu": E.ACT_SILU, "xielu": E.ACT_XIELU}[act], pos=pos, neg=neg, scale=scale) if act else {}
+    E.gemm_q(A.data_ptr(), K, [m], M, 0, out.data_ptr(), N + 8, E.GEPI_STORE16, stream(), 0, bias16=bd.data_ptr() if bias else 0, **kw)
+    torch.cuda.synchronize()
+    z = x.double() @ W.T + (b.double() if bias else 0.0)
+    if act == "relu2":
+        z = scale * torch.relu(z) ** 2
+    elif act == "silu":
+        z = scale * torch.nn.functional.silu(z)
+    elif act == "xielu":
+        lo = z.clamp(max=0)
+        z = scale * (0.5 * z + torch.where(z > 0, pos * z * z, neg * (lo.exp() - 1 - lo)))
+    assert bool((out[:, N:] == 7).all()) and bool((out[M] == 7).all())
+    assert float((out[:M, :N].cpu().double() - z).norm() / z.norm()) < K * 2.0 ** -24 + 2.0 ** -20 + 2 * 2.0 ** -9 / 3 ** 0.5
+
+
 @pytest.mark.parametrize("tile", ["64x-32", "96x-64", "160x-128"])
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("S", [1, 3])
