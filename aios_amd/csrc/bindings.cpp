@@ -440,6 +440,7 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
            py::arg("rows"))
       .def_property_readonly("kv_blocks_total", &Engine::kv_blocks_total)
       .def_property_readonly("norm_fused_parts", &Engine::norm_fused_parts)
+      .def_property_readonly("prefill_fused", &Engine::prefill_fused)
       .def_property_readonly("decode_gemm_min_batch", &Engine::decode_gemm_min_batch)
       .def("capture_graphs", &Engine::capture_graphs, py::arg("max_b"), py::call_guard<py::gil_scoped_release>())
       .def_property_readonly("stream", &Engine::stream_handle)

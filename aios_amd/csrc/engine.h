@@ -191,6 +191,8 @@ class Engine {
   int kv_blocks_total() const { return kv_nblocks_; }
   int decode_gemm_min_batch() const { return dec_gemm_min_b_; }  // rows from which decode takes the GEMMs
   int norm_fused_parts() const { return nrm_parts_; }  // 0: batched-decode RMSNorm not split into the GEMMs
+  // of the last prompt's portions above 32 rows: norms split over two products, QKV products that wrote q and the cache themselves
+  std::pair<int, int> prefill_fused() const { return prefill_fused_; }
   std::vector<int> block_table(int slot) const;
 
   int kv_block_tokens() const { return kvb_; }
@@ -391,6 +393,7 @@ class Engine {
   bf16_t* dec_xn16_ = nullptr;
   float* nrm_part_ = nullptr;
   int nrm_fuse_ = 1;
+  std::pair<int, int> prefill_fused_{0, 0};
   int nrm_parts_ = 0;  // tiles of the d_model-wide producer GEMM (0: fusion unavailable)
   bool nrm_on(int B) const;
   bool tpn_on(int B) const;  // batched TP decode: C1 / C2 fused with the next RMSNorm

@@ -1263,6 +1263,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
   const int qd = H * hd, kvd = Hkv * hd, ldqkv = qd + 2 * kvd, V = cfg_.vocab_size;
   const bool tp = cfg_.tp_size > 1;
   std::vector<int> hp(gm_rows_), hs(gm_rows_, slot);
+  prefill_fused_ = {0, 0};
   // short chunks (n <= max_batch, the batched-decode GEMMs' shapes): the decode step's fusions --
   // RoPE + KV write in the QKV GEMM's epilogue and the split RMSNorm (the residual GEMMs write
   // bf16(x * g_next) + per-tile sums, the next GEMM scales its rows) -- 3 launches per layer fewer
@@ -1331,6 +1332,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
         qepi = sh || (n > 32 && fuses(q)) || (pf_qkv && gemm_pf_serves(q));
         if (qepi) g = q;
       }
+      prefill_fused_.second += qepi && n > 32;
       gemm(g);
       if (!qepi) {
       QkvPostArgs p;
@@ -1368,6 +1370,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
         return fuses(o) && fuses(in);
       };
       const bool o_normed = fnp || (lf && pair(g, L.ffn_norm, gu));
+      prefill_fused_.first += o_normed && !fnp;
       if (o_normed) nrm_out(g, L.ffn_norm);
       gemm(g);
       if (tp) allreduce(gm_part_, (size_t)n * d, gm_x_);
@@ -1380,6 +1383,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
       if (tp) { g.C = gm_part_; g.epi = GEPI_STORE; } else { g.C = gm_x_; g.epi = GEPI_ACCUM; }
       // (the last layer: lm_head normalises its row)
       down_normed = lf && l + 1 < cfg_.n_layers && pair(g, layers_[l + 1].attn_norm, qkv_of(layers_[l + 1]));
+      prefill_fused_.first += down_normed;
       if (down_normed || (fnp && l + 1 < cfg_.n_layers)) nrm_out(g, layers_[l + 1].attn_norm);
       gemm(g);
       if (tp) allreduce(gm_part_, (size_t)n * d, gm_x_);

@@ -423,21 +423,25 @@ def test_batched_decode_split_rmsnorm_matches_explicit(model_files, monkeypatch,
 @pytest.mark.parametrize("kv", ["bf16", "fp8_e4m3"])
 def test_prefill_fused_norm_and_rope_match_explicit(model_files, monkeypatch, recipe, tile, kv):
     """prompts above 32 tokens on tiles with K over the waves: RMSNorm split across the products, RoPE and the cache in the QKV product's
-    epilogue; against the explicit launches, to bf16 rounding (an fp8 code: a step of 1/16), a second portion behind the first"""
+    epilogue; against the explicit launches (other tiles) and against the norm's alone (the same tiles), to bf16 rounding (an fp8 code: a
+    step of 1/16), a second portion behind the first"""
     prompt = [1] + list(np.random.default_rng(2).integers(3, 500, 170))
     outs = {}
-    for fuse in ("0", "1"):
+    for fuse, t in (("0", "64x128"), ("0", tile), ("1", tile)):
         monkeypatch.setenv("AIOS_GEMM_NORM_FUSE", fuse)
-        monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile if fuse == "1" else "64x128")
+        monkeypatch.setenv("AIOS_GEMM_PF_TILE", t)
         eng, cfg = _load(model_files[recipe], act_q8=False, kv_dtype=kv)
         if kv != "bf16":
-            eng.set_kv_scales([1 / 32] * (2 * cfg.n_layers))
+            eng.set_kv_scales([1 / 32, 1 / 48] * cfg.n_layers)
         eng.prefill(0, prompt[:100], 0, False)
-        outs[fuse] = np.asarray(eng.prefill(0, prompt[100:], 100, True))
+        outs[fuse, t] = np.asarray(eng.prefill(0, prompt[100:], 100, True))
+        assert eng.prefill_fused == (0 if fuse == "0" else 2 * cfg.n_layers - 1, 0 if t == "64x128" else cfg.n_layers)
         del eng
-    l0, l1 = outs["0"], outs["1"]
-    assert np.isfinite(l1).all() and not np.array_equal(l0, l1)
-    assert np.abs(l0 - l1).max() < (1e-2 if kv == "bf16" else 4e-2) * max(np.abs(l0).max(), 1.0)
+    l1 = outs.pop(("1", tile))
+    assert np.isfinite(l1).all()
+    for l0 in outs.values():
+        assert not np.array_equal(l0, l1)
+        assert np.abs(l0 - l1).max() < (1e-2 if kv == "bf16" else 4e-2) * max(np.abs(l0).max(), 1.0)
 
 
 @pytest.mark.parametrize("recipe", ["Q4_K_M", "mistral_shape"])
