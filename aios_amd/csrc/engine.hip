@@ -749,7 +749,7 @@ void Engine::finalize() {
 // Measured prefill-GEMM plans (kernels/gemm_pf.hip): every distinct projection launch of this model
 // -- QKV stack, O, gate/up (SwiGLU), down, per weight-format signature -- timed with its layers' weights in turn over
 // candidate tiles / K splits at M = 64 .. gm_rows_ (gemm_pf_bucket), the fastest kept per M bucket in the
-// process-wide plan cache (one tuning per shape per process; 0.7 s for Mistral-7B Q4_K_M, 0.3 s for TinyLlama Q4_K_M).
+// process-wide plan cache (one tuning per shape per process; 0.75 s for Mistral-7B Q4_K_M, 0.3 s for TinyLlama Q4_K_M).
 // Activations are random bf16 (a zero fill clocks the chip differently).  AIOS_GEMM_PF_TUNE=0: model plans only.
 void Engine::tune_prefill_gemm() {
   if (!gm_ok_ || cfg_.n_layers == 0) return;
@@ -1273,7 +1273,10 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
     // chunks of <= 32 rows: the batched-decode GEMMs and their fused epilogues
     const bool sh = short_fuse && !tp && n <= 32;
     const bool fnp = sh && gm_nparts_ > 0;
-    // longer chunks: the same fusions where both products of a norm, or the QKV product, run on tiles with K over the waves
+    // longer chunks: the same fusions where both products of a norm, or the QKV product, run on tiles with K over the waves.  They cost
+    // the products part of what the launches took: us, Mistral at 130 rows, plain -> fused, QKV 20.1 -> 25.4 (Q4_K), 23.9 -> 28.3 (mixed), O
+    // 16.6 -> 18.0, gate/up 44.1 -> 45.6, down 30.0 -> 31.5 and 38.7 -> 39.9, against two norms of 4.9 and RoPE's 6.8 a layer; the prompt
+    // 4.75 -> 4.46 ms, 300 rows 7.37 -> 7.18, 1500 25.0 -> 24.8 (profiles/prefill_fused_products.txt)
     const bool lf = nrm_fuse_ && !tp && n > 32 && d % 256 == 0;
     auto fuses = [&](GemmQArgs q) {
       q.ws = gk_ws_; q.ws_bytes = gk_ws_bytes_; q.cnt = gk_cnt_; q.cnt_len = gk_cnt_len_;
@@ -1318,7 +1321,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
       // the RoPE / KV-cache epilogue: short chunks (the decode GEMMs) and tiles with K over the waves; the prefill GEMM's others
       // only with AIOS_PREFILL_QKV_EPI=1 -- they need S = 1 plans for it, and at 2048 tokens
       // the QKV GEMM then took 212.7 us against 115.7 (split-K) + 32 us of qkv_post (64 tokens:
-      // 5.77 vs 4.6 ms per prompt), profiles/prefill_r5.txt
+      // 5.77 vs 4.6 ms per prompt), profiles/prefill_r5.txt; before those tiles' epilogue took pairs of a lane's own
       const bool qepi_ok = !cfg_.qk_norm && !cfg_.rope_neox && !L.bqkv && rope_cs_ && !tp;
       bool qepi = false;
       if (qepi_ok) {

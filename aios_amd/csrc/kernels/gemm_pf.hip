@@ -356,7 +356,8 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
     }
     std::vector<PfPlan> c;
     for (const PfPlan& p : all) {
-      // (quantised: beside K over the waves no other tile below 256 columns was ever the fastest, three models' 240 keys)
+      // (quantised: beside K over the waves another tile of 128 columns is the fastest for 2 of three models' 270 keys, by 2 %; Mistral's prompts of
+      // 700 to 1536 rows as fast without them, its load 0.93 -> 0.75 s: profiles/prefill_tiles.txt)
       if ((model(p) <= 2 * least && !(waves && !bf && p.bn == 128)) || same(p, mp) || same(p, mp1)) c.push_back(p);
     }
     if (c.empty()) continue;
@@ -377,7 +378,8 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
       std::vector<PfPlan> both(f);
       both.insert(both.end(), f.rbegin(), f.rend());
       const std::vector<float> t = time(v, both, 4);
-      // (K over the waves by 4 % or not: 4096 x 4096 at 2048 rows, 3 % faster here, took 86 us of a pass where 128 x 256 tiles took 84)
+      // (K over the waves by 4 % or not: 4096 x 4096 at 2048 rows, 3 % faster here, took 86 us of a pass where 128 x 256 tiles took 84.  The
+      // plain forms are timed: what the fused ones save, a norm's or RoPE's launch of 5 to 20 us, and cost, 1 to 5 us, is not in it)
       auto sum = [&](size_t i) { return (t[i] + t[2 * n - 1 - i]) * (f[i].bn < 0 ? 1.04f : 1.f); };
       size_t best = 0;
       for (size_t i = 1; i < n; ++i)

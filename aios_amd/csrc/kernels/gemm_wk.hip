@@ -227,8 +227,8 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
   if (nrm) nr.done(a, wave, lane, inv_s);  // (read after the first tile's barrier)
   // what the outputs need besides their sums is requested before the tile's products (by every wave: which of them adds the tile up
   // is not worth a branch here).  Behind the sums it was one or two trips to memory at the end of a launch.
-  // bf16 weights, 8 steps of TinyLlama with 12 rows 8.60 -> 8.44 ms; beside a quantised format's decode it gave nothing (8 rows, TinyLlama
-  // 0.5 % faster, Mistral 0.9 % slower): there the residual only
+  // bf16 weights, 8 steps of TinyLlama with 12 rows 8.57 -> 8.43 ms, with 6 8.03 -> 7.90 (with 3, and Seledra's 16, no more than the runs differ,
+  // 1 to 2 %); beside a quantised format's decode nothing that shows (8 rows of TinyLlama and Mistral within 1 %): there the residual only
   int pos[MT], slot[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {

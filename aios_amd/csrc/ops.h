@@ -266,7 +266,8 @@ bool gemm_wk_on();
 bool gemm_wk_serves(const GemmQArgs& a);
 // the prefill GEMM (kernels/gemm_pf.hip): true if it took the launch; its tile / split plan for a shape
 bool launch_gemm_pf(const GemmQArgs& a, hipStream_t st);
-bool gemm_pf_fuses(const GemmQArgs& a);  // whether the prefill GEMM would run these args, the decode GEMMs' fused epilogues among them, on tiles with K over the waves
+// whether the prefill GEMM would run these args, the decode GEMMs' fused epilogues among them, on the tile with K over the waves that the plain product runs on
+bool gemm_pf_fuses(const GemmQArgs& a);
 bool gemm_pf_serves(const GemmQArgs& a);  // launch_gemm_pf would take a (gemm_pf.hip)
 void gemm_pf_plan(const GemmQArgs& a, int& bm, int& bn, int& s);
 bool gemm_pf_probe(const GemmQArgs& a, int probe, hipStream_t st);  // timing anatomy (tools only)
