@@ -677,6 +677,11 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
   m.def("swiglu", [](uintptr_t gu, int ldg, uintptr_t out, int ldo, int rows, int n, uintptr_t st) {
     launch_swiglu_interleaved((const float*)gu, ldg, (float*)out, ldo, rows, n, S(st));
   });
+  m.def("qkv_post_by_rows", [](int T, int hd, uintptr_t rope_cs, uintptr_t bias) {
+    QkvPostArgs a;
+    a.T = T; a.head_dim = hd; a.rope_cs = (const float2*)rope_cs; a.bias = (const float*)bias;
+    return qkv_post_by_rows(a);
+  }, py::arg("T"), py::arg("hd"), py::arg("rope_cs"), py::arg("bias") = 0);
   m.def("qkv_post",
         [](uintptr_t qkv, int ldqkv, int T, int H, int Hkv, int hd, uintptr_t q_norm, uintptr_t k_norm, float eps,
            int rope_neox, float rope_base, uintptr_t pos, uintptr_t slot, uintptr_t q_out, uintptr_t k_cache,

@@ -273,8 +273,10 @@ __global__ void __launch_bounds__(256) qkv_post_row_kernel(QkvPostArgs a) {
 
 // QK-norm or NeoX pairs, heads of 128, no bias (Qwen3), prompts: a workgroup per token row, a wave every fourth head and a lane the
 // pair it holds in each of them, so position, cache block, (cos, sin) and gains are read once a row and four heads' loads are in flight
-// (a wave per token and head read all of them in a chain: 711 rows of 32 + 2 x 8 heads, 32 MB, 17 us -> 10.8).  A few rows are the
-// other kernel's: there each head has a wave of its own.
+// (a wave per token and head read all of them in a chain).  Below 320 rows the CUs are not full and a wave's turns through its heads are
+// the longer chain: those rows are the other kernel's, where each head has a wave of its own.  us, a wave a head / this:
+//   32 + 2 x 8 heads, 33 / 128 / 256 / 300 / 400 / 711 / 2048 rows  3.5 / 7.2, 4.8 / 7.8, 8.0 / 8.7, 8.7 / 9.0, 10.9 / 9.4, 16.5 / 10.8, 50 / 21
+//   40 + 2 x 8, 300 / 400 rows  9.7 / 10.5, 11.8 / 10.9     16 + 2 x 8, 256 / 300 rows  5.7 / 6.3, 7.2 / 6.7     8 + 2 x 2, 96 / 300 rows  3.3 / 3.3, 3.8 / 3.7
 __global__ void __launch_bounds__(256) qkv_post_head_kernel(QkvPostArgs a) {
   constexpr int HD = 128, HALF = 64, UNR = 4;
   const int t = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -324,12 +326,14 @@ __global__ void __launch_bounds__(256) qkv_post_head_kernel(QkvPostArgs a) {
   }
 }
 
+bool qkv_post_by_rows(const QkvPostArgs& a) { return a.T >= 320 && a.head_dim == 128 && a.rope_cs && !a.bias; }
+
 void launch_qkv_post(const QkvPostArgs& a, hipStream_t st) {
   if (!a.rope_neox && !a.q_norm && !a.k_norm && !a.bias && a.rope_cs && a.head_dim % 2 == 0) {
     hipLaunchKernelGGL(qkv_post_row_kernel, dim3(a.T), dim3(256), 0, st, a);
     return;
   }
-  if (a.T > 32 && a.head_dim == 128 && a.rope_cs && !a.bias) {
+  if (qkv_post_by_rows(a)) {
     hipLaunchKernelGGL(qkv_post_head_kernel, dim3(a.T), dim3(256), 0, st, a);
     return;
   }

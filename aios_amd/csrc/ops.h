@@ -91,6 +91,7 @@ struct QkvPostArgs {
   float kv_inv_k = 1.f, kv_inv_v = 1.f;
 };
 void launch_qkv_post(const QkvPostArgs& a, hipStream_t st);
+bool qkv_post_by_rows(const QkvPostArgs& a);  // whether such rows with QK-norm or NeoX pairs have a workgroup each
 
 // ---- attention ---------------------------------------------------------------------------------
 struct AttnDecodeArgs {

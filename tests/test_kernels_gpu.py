@@ -705,22 +705,24 @@ def test_rmsnorm(E, n, y_off):
 
 @pytest.mark.parametrize("neox", [0, 1])
 @pytest.mark.parametrize("norm", ["", "q", "qk"])
-@pytest.mark.parametrize("T,H,Hkv", [(33, 8, 2), (70, 32, 8), (40, 5, 1)])
+@pytest.mark.parametrize("T,H,Hkv", [(320, 8, 2), (357, 32, 8), (400, 5, 1)])
 def test_qkv_post_rows_match_one_by_one(E, neox, norm, T, H, Hkv):
-    """more than 32 rows of 128-wide heads with QK-norm or NeoX pairs (a workgroup a row) against the same rows in calls of one; sums of 128
+    """320 rows and more of 128-wide heads with QK-norm or NeoX pairs (a workgroup a row) against the same rows in calls of one; sums of 128
     squares in another order: 2^-22 of a value, a bf16 step at a rounding boundary"""
     if not neox and not norm:
         pytest.skip("the plain kernel's")
     hd, max_ctx, slots = 128, 256, 2
     qkv = torch.randn(T, (H + 2 * Hkv) * hd + 4, device="cuda")
     qn, kn = (torch.rand(hd, device="cuda") + 0.5 for _ in range(2))
-    pos = (torch.arange(T, dtype=torch.int32) * 3 % 200 + torch.arange(T, dtype=torch.int32) // 67).cuda()
-    slot = (torch.arange(T, dtype=torch.int32) % slots).cuda()
+    at = torch.randperm(slots * max_ctx, generator=torch.Generator().manual_seed(T))[:T].int()
+    pos, slot = (at // slots).cuda(), (at % slots).cuda()
     ang = torch.arange(max_ctx)[:, None].double() * 1e6 ** (-2.0 * torch.arange(hd // 2).double() / hd)
     cs = torch.stack([ang.cos(), ang.sin()], -1).float().cuda()
     kp, bt = paged_cache(torch.zeros(slots, Hkv, max_ctx, hd, dtype=torch.bfloat16), True, seed=3)
     bt = bt.cuda()
     outs = []
+    assert E.qkv_post_by_rows(T, hd, cs.data_ptr()) and not E.qkv_post_by_rows(319, hd, cs.data_ptr())
+    assert not any(E.qkv_post_by_rows(T, *x) for x in ((64, cs.data_ptr()), (hd, 0), (hd, cs.data_ptr(), qn.data_ptr())))
     for rows in (T, 1):
         q, k, v = torch.zeros(T, H * hd, device="cuda"), kp.cuda(), torch.zeros_like(kp).cuda()
         for r in range(0, T, rows):
@@ -736,10 +738,10 @@ def test_qkv_post_rows_match_one_by_one(E, neox, norm, T, H, Hkv):
 @pytest.mark.parametrize("neox,norm", [(0, 1), (1, 0), (1, 1)])
 def test_qkv_post_rows_fp8(E, neox, norm):
     """... and into an fp8 cache: the bf16 call's values at K's and V's own scales, to a code (those values are rounded to 8 bits first)"""
-    T, H, Hkv, hd, max_ctx, inv = 70, 8, 2, 128, 256, (150.0, 300.0)
+    T, H, Hkv, hd, max_ctx, inv = 330, 8, 2, 128, 512, (150.0, 300.0)
     g = torch.Generator().manual_seed(6)
     qkv, qn, kn = (x.cuda() for x in (torch.randn(T, (H + 2 * Hkv) * hd, generator=g), torch.rand(hd, generator=g) + 0.5, torch.rand(hd, generator=g) + 0.5))
-    pos = (torch.arange(T, dtype=torch.int32) * 3).cuda()
+    pos = torch.randperm(max_ctx, generator=g)[:T].int().cuda()
     cs = torch.nn.functional.normalize(torch.randn(max_ctx, hd // 2, 2, generator=g), dim=-1).cuda()
     caches = []
     for dt in (torch.bfloat16, torch.uint8):
