@@ -66,12 +66,36 @@ __device__ __forceinline__ void pf_qkv_out(const GemmQArgs& a, int m, int n, flo
 // tiles at a time, so 4 x 8 of 256 x 256: 12 panels of X and W go through its L2, where one row of tiles has 33.
 // us at 2048 rows, 256 x 256, along the rows -> so: 8192 x 4096 bf16 125 -> 116, Q6_K 140 -> 136, Q4_K 122 -> 120 (codes of 4.5 bits:
 // the panels of W are the small ones); 28672 x 4096 bf16 584 -> 570, Q4_K SwiGLU 491 -> 482
+// Along the rows where bands cost more than they save (pf_bands).  us in bands / along the rows:
+//  K slices, more than one band, quantised 256-column and all 256 x 128 tiles: 4096 x 4096 Q4_K in two slices of 256 x 256, 1300 / 1852 / 2048 /
+//   4096 rows 79.6 / 77.5, 102.7 / 98.3, 108.6 / 103.1, 203.7 / 195.5; 4096 x 14336, 2048 rows Q4_K 232.9 / 224.3, Q6_K 251.6 / 246.5; bf16
+//   4096 x 4096, 256 x 128, 2048 rows 121.5 / 112.8.  But one band and bf16: 4096 x 14336, 128 x 256, 1024 rows 122 / 148; 256 x 256, 1300
+//   rows 174 / 181; 8704 x 2048, 256 x 128, 300 rows 54 / 58
+//  stream-K, all bands a multiple of eight tiles high: there successive ranges of tiles lie on successive XCDs, so each XCD would have one row of
+//   tiles and all of W.  bf16: 8704 x 2048, 1024 rows 85 / 62; 4096 x 4096, 700 / 1024 rows 55 / 46, 62 / 58
 template <int BM>
-__device__ __forceinline__ void pf_tile(int L, int nM, int nN, int& tm, int& tn) {
+__device__ __forceinline__ void pf_tile(int L, int nM, int nN, int& tm, int& tn, bool bands = true) {
   constexpr int GM = 1024 / BM;
+  if (!bands) {
+    tm = L / nN;
+    tn = L - tm * nN;
+    return;
+  }
   const int band = L / (GM * nN), r = L - band * (GM * nN), g = min(GM, nM - band * GM);
   tn = r / g;
   tm = band * GM + r - tn * g;
+}
+
+// whether a launch of nM rows of BM x BN tiles of QT weights goes in bands (gridDim.y slices of K: a trip to memory, only where it counts)
+template <int QT, int BM, int BN>
+__device__ __forceinline__ bool pf_bands(int nM) {
+  if constexpr ((BM < 256 && BN < 256) || (BN == 256 && QT == QT_BF16)) return true;
+  return nM <= 1024 / BM || gridDim.y == 1;
+}
+// ... and stream-K
+template <int BM>
+__device__ __forceinline__ bool pf_sk_bands(int nM) {
+  return nM % 8 != 0 || min(1024 / BM, nM) % 8 != 0;
 }
 
 // slot layout for one K-step: A, then the weight planes of BN columns
@@ -1746,7 +1770,7 @@ __global__ void __launch_bounds__(512) gemm_pf8_kernel(GemmQArgs a) {
   const int nN = a.N / 256, nM = (a.M + BM - 1) / BM, total = nN * nM;
   const int L = xcd_remap(blockIdx.x, total);
   int tm, tn;
-  pf_tile<BM>(L, nM, nN, tm, tn);
+  pf_tile<BM>(L, nM, nN, tm, tn, pf_bands<QT0, BM, 256>(nM));
   const int m0 = tm * BM, n0 = tn * 256;
   int seg = 0;
   if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
@@ -1858,7 +1882,7 @@ __device__ __forceinline__ void pf_stream_k(const GemmQArgs& a, int BN, int ipw,
     const int L = (int)(it / nk), k0 = (int)(it - (long)L * nk);
     const int k1 = (int)(k0 + (end - it) < nk ? k0 + (end - it) : nk);
     int tm, tn;
-    pf_tile<BM>(L, nM, nN, tm, tn);
+    pf_tile<BM>(L, nM, nN, tm, tn, pf_sk_bands<BM>(nM));
     const int m0 = tm * BM, n0 = tn * BN;
     int seg = 0;
     if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;
@@ -1970,7 +1994,7 @@ __global__ void __launch_bounds__(256 * KG) gemm_pf4_kernel(GemmQArgs a) {
   const int nN = a.N / BN, nM = (a.M + BM - 1) / BM, total = nN * nM;
   const int L = xcd_remap(blockIdx.x, total);
   int tm, tn;
-  pf_tile<BM>(L, nM, nN, tm, tn);
+  pf_tile<BM>(L, nM, nN, tm, tn, pf_bands<QT0, BM, BN>(nM));
   const int m0 = tm * BM, n0 = tn * BN;
   int seg = 0;
   if (a.nseg > 1 && n0 >= a.seg_n0[1]) seg = 1;

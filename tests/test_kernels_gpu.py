@@ -1808,6 +1808,29 @@ def test_gemm_pf8_outputs(E, monkeypatch, bm, fmt, epi):
         assert rel < (3 if half else 1) * 2 * 2.0 ** -9 / 3 ** 0.5 + K * 2.0 ** -24, (off, ld, rel)
 
 
+@pytest.mark.parametrize("fmt,tile,S,M", [
+    ("Q4_K", "256x256", 2, 1300), ("Q6_K", "128x256", 2, 1025), ("Q5_K", "256x256", 3, 1024), ("Q8_0", "64x256", 2, 1100),
+    ("BF16", "256x128", 2, 1500), ("BF16", "256x256", 2, 1300), ("BF16", "128x256", 2, 1200), ("Q5_K", "128x128", 2, 1200),
+    ("BF16", "128x128", -1, 1024), ("BF16", "128x256", -1, 1000), ("BF16", "96x128", -1, 760), ("Q5_K", "64x128", -1, 512),
+    ("BF16", "128x128", -1, 1500), ("BF16", "256x256", -1, 2048), ("Q5_K", "160x128", -1, 1500)])
+def test_gemm_pf_tile_orders(E, monkeypatch, fmt, tile, S, M):
+    """Products with K split, and stream-K, below and above 1024 rows, with row tiles in eights and not: every tile is somebody's, in bands
+    or along the rows.  Bound: see sum_tol"""
+    monkeypatch.setenv("AIOS_GEMM_PF_TILE", tile)
+    monkeypatch.setenv("AIOS_GEMM_PF_SPLIT", str(S))
+    K, N = 1024, 768
+    m, W = small_mat(E, fmt, N, K, 17)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    A, C = x.cuda(), torch.full((M + 1, N), 2.0, device="cuda")
+    bm, bn = (int(v) for v in tile.split("x"))
+    assert list(E.gemm_pf_plan([m], M, E.GEPI_STORE, 0, out=C.data_ptr())) == [bm, bn, S]
+    E.gemm_q(A.data_ptr(), K, [m], M, C.data_ptr(), 0, N, E.GEPI_STORE, stream(), 0)
+    torch.cuda.synchronize()
+    ref = x.double() @ W.T
+    assert bool((C[M] == 2).all())
+    assert float(((C[:M].cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)).max()) < sum_tol(fmt, K)
+
+
 # ---- the prefill GEMM with K over the waves (gemm_pfk.h): BM x -BN tiles
 PFK_TILES = [f"{bm}x-{bn}" for bm in (64, 96, 128, 160) for bn in (32, 64, 128)]
 
