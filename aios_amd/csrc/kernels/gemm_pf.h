@@ -729,12 +729,13 @@ struct Pf4Dma {
   }
 
   // K-step kt into the slot at LDS byte address dst (wave-uniform).  PROBE 16: weight pieces read
-  // contiguous 1 KB (wrong data; coalescing probe), PROBE 32: no weight pieces (timing only)
-  template <int PROBE = 0>
+  // contiguous 1 KB (wrong data; coalescing probe), PROBE 32: no weight pieces (timing only).  PART 1: A's pieces, 2: the weights'
+  template <int PROBE = 0, int PART = 0>
   __device__ __forceinline__ void issue(const GemmQArgs& a, const QWeight& w, int kt, uint32_t dst, int wv) const {
     const uint32_t wb = dst + L::OFF_B + (uint32_t)wv * L::WB;
     static_for<L::PW>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
+      if constexpr (PART && (PART == 1) != (i < L::NA)) return;
       if constexpr ((PROBE & 32) && i >= L::NA) return;
       if constexpr ((PROBE & 16) && i >= L::NA) {
         pf_glds16(w.p0 + kt * 4096 + (i - L::NA) * 1024 + (threadIdx.x & 63) * 16 + wv * 65536, wb + (i - L::NA) * 256);
@@ -1129,7 +1130,7 @@ template <int QT, int BM, int EPI, int PROBE = 0>
 __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int seg, int kt0, int kt1, int S) {
   constexpr int NW = 8, WC = 32;
   using L = Pf4Layout<QT, BM, WC, NW>;
-  constexpr int MT = BM / 16, GR = MT < 8 ? MT : 8, NG = MT / GR, NPH = 2 * NG, NS = L::NS, PW = L::PW;
+  constexpr int MT = BM / 16, GR = MT < 8 ? MT : 8, NG = MT / GR, NPH = 2 * NG, NS = L::NS, NA = L::NA, NB = L::PW - NA;
   constexpr bool PERM = pf8_perm<EPI>();
   extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1157,8 +1158,23 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
   Pf4Dma<QT, BM, WC, NW, PERM> dma;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(pf_lds_addr(pf_smem));
   dma.init(a, wcol0, m0, wv);
+  auto get_a = [&](int t, int slot) __attribute__((always_inline)) {
+    dma.template issue<PROBE, 1>(a, w, min(kt0 + t, klast), lds0 + slot * L::SLOT, wv);
+  };
+  auto get_b = [&](int t, int slot) __attribute__((always_inline)) {
+    dma.template issue<PROBE, 2>(a, w, min(kt0 + t, klast), lds0 + slot * L::SLOT, wv);
+  };
+  // Each part of a slot is asked for again as soon as it has been read, and waited for where it is read: A has one step of lead, B two.  (With one request
+  // of a whole slot at the end of a step and one wait for it in the middle of the next, two slots left half a step: bf16 256 x 256,
+  // us, weights from memory, so -> now: 1500 x 8704 x 2048 rows x columns x k 61.5 -> 54.8, 2048 x 11264 x 2048 120 -> 105, 2048 x 8192 x 8192 221 -> 212.)
+  // Requests go B(0) B(1) A(0) B(2) A(1) .., B(t + NS + 1) in the middle of step t, when the wave has read B(t + 1), A(t + NS) at its end,
+  // when all waves have read A(t).  Waits: B(t + 1) at its read, A(t + 1) at the barrier in front of its first read.
+  get_b(0, 0);
 #pragma unroll
-  for (int p = 0; p < NS; ++p) dma.template issue<PROBE>(a, w, min(kt0 + p, klast), lds0 + p * L::SLOT, wv);
+  for (int p = 0; p < NS - 1; ++p) {
+    get_b(p + 1, p + 1);
+    get_a(p, p);
+  }
 
   gbf16x8 bf[2][2], fa[GR], fb[GR];
   PfBRaw raw[2];
@@ -1221,12 +1237,13 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
       acc[g * GR + i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[c][sp], f[i], acc[g * GR + i][c], 0, 0, 0);
     }
   };
-  if constexpr (!(PROBE & 1)) {
-    pf_vmcnt<(NS - 1) * PW>();
-  }
+  if constexpr (!(PROBE & 1)) pf_vmcnt<(NS - 1) * (NA + NB)>();
   read_raw(pf_smem, kt0);
   dec(std::integral_constant<int, 0>{});
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  get_b(NS, 0);
+  get_a(NS - 1, NS - 1);
+  if constexpr (!(PROBE & 1)) pf_vmcnt<(NS - 1) * (NA + NB)>();
   pf_barrier();
   ldA(pf_smem, fa, 0);
 
@@ -1242,24 +1259,28 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
       if constexpr (p + 1 < NPH) ldA(slot, nf, p + 1);
       if constexpr (p == 0) dec(std::integral_constant<int, 1>{});  // this step's fragment 1
       if constexpr (p == NG) {
-        // own pieces of step t+1 landed (NS - 2 younger steps in flight): its raw bytes, fragment 0
-        if constexpr (!(PROBE & 1)) {
-          pf_vmcnt<(NS - 2) * PW>();
-        }
+        // this wave's weights of step t+1 landed: its raw bytes, fragment 0
+        if constexpr (!(PROBE & 1)) pf_vmcnt<NS * NA + (NS - 1) * NB>();
         read_raw(pf_smem + nxt * L::SLOT, kt0 + t + 1);
         dec(std::integral_constant<int, 0>{});
       }
       if constexpr (p + 1 < NPH) {
         mfma_range(cf, p, 0, 2 * GR);
+        if constexpr (p == NG && !(PROBE & 4)) {
+          __builtin_amdgcn_sched_barrier(0);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          get_b(t + NS + 1, nxt);
+        }
       } else {
-        // last phase: half the MFMAs; B(t+1); the next step's first reads and DMA(t + NS) into slot t
-        // under the other half
+        // last phase: half the MFMAs; the barrier; the next step's first reads and A(t + NS) into slot t under the other half
         mfma_range(cf, p, 0, GR);
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if constexpr (p == NG && !(PROBE & 4)) get_b(t + NS + 1, nxt);
+        if constexpr (!(PROBE & 1)) pf_vmcnt<(NS - 1) * NB + (NS - 2) * NA>();
         if constexpr (!(PROBE & 8)) pf_barrier();
         ldA(pf_smem + nxt * L::SLOT, nf, 0);
-        if constexpr (!(PROBE & 4)) dma.template issue<PROBE>(a, w, min(kt0 + t + NS, klast), lds0 + cur * L::SLOT, wv);
+        if constexpr (!(PROBE & 4)) get_a(t + NS, cur);
         mfma_range(cf, p, GR, 2 * GR);
       }
     });
