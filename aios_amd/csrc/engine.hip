@@ -639,8 +639,10 @@ void Engine::finalize() {
   // and the head layout has a flash-attention instantiation
   {
     if (const char* e = std::getenv("AIOS_PREFILL_GEMM_MIN")) gm_min_rows_ = std::max(1, std::atoi(e));
-    // one chunk per prompt up to 2048 tokens: the M tile count, not the chunk count, fills the chip
-    gm_rows_ = std::min(cfg_.max_ctx, 2048);
+    // one chunk per prompt up to 4096 tokens: the M tile count, not the chunk count, fills the chip.  ms, in chunks of 2048 -> of 4096:
+    // Mistral-7B Q4_K_M 2500 tokens 39.7 -> 38.1, 3500 56.9 -> 51.0, 3900 60.3 -> 56.0, 9000 151 -> 143; Qwen3-8B 3900 61.1 -> 57.3 (down is one
+    // round of unsplit 256 x 256 tiles, 374 us, where two chunks are two launches of K halves that meet in atomics, 215 each)
+    gm_rows_ = std::min(cfg_.max_ctx, 4096);
     if (const char* e = std::getenv("AIOS_PREFILL_GEMM_ROWS")) gm_rows_ = std::max(64, std::atoi(e));
     bool ok = attn_prefill_supports(H, Hkv, hd) && d % 64 == 0 && cfg_.d_ff % 64 == 0 && qd % 64 == 0 && kvd % 64 == 0;
     for (const auto& L : layers_) {
@@ -749,7 +751,7 @@ void Engine::finalize() {
 // Measured prefill-GEMM plans (kernels/gemm_pf.hip): every distinct projection launch of this model
 // -- QKV stack, O, gate/up (SwiGLU), down, per weight-format signature -- timed with its layers' weights in turn over
 // candidate tiles / K splits at M = 64 .. gm_rows_ (gemm_pf_bucket), the fastest kept per M bucket in the
-// process-wide plan cache (one tuning per shape per process; 0.75 s for Mistral-7B Q4_K_M, 0.3 s for TinyLlama Q4_K_M).
+// process-wide plan cache (one tuning per shape per process; 1.0 s for Mistral-7B Q4_K_M at a context of 4096, 0.3 s for TinyLlama Q4_K_M).
 // Activations are random bf16 (a zero fill clocks the chip differently).  AIOS_GEMM_PF_TUNE=0: model plans only.
 void Engine::tune_prefill_gemm() {
   if (!gm_ok_ || cfg_.n_layers == 0) return;

@@ -99,7 +99,7 @@ using PfKey = std::tuple<int, int, int, int, int, int, int, int, int, int>;
 // (Two or three to a doubling, where tiles of 32 rows more or less change the plan: 130 rows ran the plan of 256, whose
 // gate/up took 83 us where one 160-row tile takes 58.)
 int gemm_pf_bucket(int M) {
-  for (int b : {64, 96, 128, 160, 192, 256, 320, 384, 512, 640, 768, 1024, 1280, 1536, 2048})
+  for (int b : {64, 96, 128, 160, 192, 256, 320, 384, 512, 640, 768, 1024, 1280, 1536, 2048, 2560, 3072})
     if (M <= b) return b;
   return (M + 2047) / 2048 * 2048;
 }
@@ -358,7 +358,8 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st) {
     for (const PfPlan& p : all) {
       // (quantised: beside K over the waves another tile of 128 columns is the fastest for 2 of three models' 270 keys, by 2 %; Mistral's prompts of
       // 700 to 1536 rows as fast without them, its load 0.93 -> 0.75 s: profiles/prefill_tiles.txt)
-      if ((model(p) <= 2 * least && !(waves && !bf && p.bn == 128)) || same(p, mp) || same(p, mp1)) c.push_back(p);
+      // (above 2048 rows the model's tiles stand closer together, and a launch takes up to a millisecond)
+      if ((model(p) <= (a.M > 2048 ? 1.6 : 2) * least && !(waves && !bf && p.bn == 128)) || same(p, mp) || same(p, mp1)) c.push_back(p);
     }
     if (c.empty()) continue;
     if (&w == &work[0]) time(v, {c[0]}, 100);  // (the clocks)

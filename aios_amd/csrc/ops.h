@@ -278,8 +278,8 @@ int gemm_pf_autotune(const std::vector<GemmQArgs>& launches, hipStream_t st);
 int gemm_pf_bucket(int M);  // the row count whose plan serves M rows: plans are tuned at M = 64, then bucket(M + 1), ..
 // of the kernels that plans were timed on: a plan file of another number is timed again (2: K groups in the 128-column
 // tiles below 256 rows, more row buckets; 3: tiles with K over the waves; 4: of bf16 too, other
-// epilogues)
-constexpr int GEMM_PF_PLANS_VERSION = 4;
+// epilogues; 5: bf16 256 x 256 faster, row counts above 2048)
+constexpr int GEMM_PF_PLANS_VERSION = 5;
 std::vector<int> gemm_pf_export();              // the process's tuned prefill plans (flat ints)
 void gemm_pf_import(const std::vector<int>& v);  // ... installed (TP: the leader's; persisted sets)
 

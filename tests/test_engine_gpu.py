@@ -9,6 +9,7 @@ from aios_amd.gguf.quants import GGMLType
 from aios_amd.models.config import get_preset
 from aios_amd.models.reference import ReferenceModel
 from aios_amd.models.synthetic import write_synthetic_gguf
+from aios_amd.runtime.loader import random_engine
 
 pytestmark = pytest.mark.gpu
 
@@ -207,6 +208,20 @@ def test_prefill_gemm_chunks_match_reference(model_files, recipe, monkeypatch):
     eng.prefill(1, prompt[:100], 0, False)
     logits2 = torch.from_numpy(np.asarray(eng.prefill(1, prompt[100:], 100, True)))
     assert (logits2 - rl).abs().max().item() < 2e-2 * scale
+
+
+@pytest.mark.parametrize("T", [2049, 2561, 4090])
+def test_prefill_of_more_than_2048_rows_in_one_portion(T, monkeypatch):
+    """the same logits as in portions of 2048 rows (other tiles' sums and rounded activations: the bound of the portions' tests above)"""
+    cfg = get_preset("test-mistral-shape")
+    prompt = [1] + list(np.random.default_rng(T).integers(3, cfg.vocab_size, T - 1))
+    out = []
+    for rows in ("", "2048"):
+        if rows:
+            monkeypatch.setenv("AIOS_PREFILL_GEMM_ROWS", rows)
+        eng = random_engine(cfg, "Q4_K_M", seed=0, max_ctx=4096, max_batch=1)
+        out.append(torch.from_numpy(np.asarray(eng.prefill(0, prompt, 0, True))))
+    assert (out[0] - out[1]).abs().max().item() < 2e-2 * max(out[1].abs().max().item(), 1.0)
 
 
 @pytest.mark.parametrize("recipe", ["Q4_K_M", "mistral_shape", "Q5_K_M", "Q4_0", "Q8_0"])
