@@ -377,9 +377,21 @@ static bool wk_route(const GemmQArgs& a, WkRoute& r) {
     return false;
   // (three segments' four planes and the cache's arguments: more scalars than there are)
   if (a.epi == GEPI_QKV && qt0 == QT_Q6_K && r.ns * r.mt == 4) return false;
-  r.G = std::min(a.N / 16, std::max(1, device_cu_count() / r.S));
+  // One slice more where that deals the tiles out more evenly: G ranges of whole tiles leave CUs idle while the longest range ends.  With a split
+  // that there is anyway, from a fifth less for the longest range up; us before / so, 16 and 30 rows: 2048 x 8704 bf16 (three slices of
+  // 85 ranges, 43 of them two tiles long) 14.9 / 13.2, 16.0 / 16.0 (eight already); Q6_K 11.7 / 10.7, 14.3 / 13.2, Q4_K 9.7 / 9.0, 12.0 / 11.2;
+  // 4096 x 12288 Q4_K 14.4 / 14.1, 17.2 / 16.7; 2048 x 5632 bf16, 30 rows 12.2 / 11.2; but 5120 x 17408 Q4_K, 8 % less 20.7 / 21.6.
+  // Two slices instead of one: bf16 where its tiles are for half of the CUs at most and a wave has two stages: 2048 x 4096 9.2 / 8.5, 1024 x 4096
+  // 9.0 / 7.6, 2048 x 3072 8.5 / 7.9; but 2048 x 2048, one stage, 6.2 / 7.0, and Q4_K, a third of the bytes, 2048 x 4096 6.2 / 7.0.
+  auto groups = [&](int S) { return std::min(a.N / 16, std::max(1, cus / S)); };
+  auto longest = [&](int S) { return (long)((a.N / 16 + groups(S) - 1) / groups(S)) * ((nu + S - 1) / S); };
+  auto room = [&](int S) { return a.ws && a.cnt && a.cnt_len >= groups(S) && a.ws_bytes >= (size_t)S * 16 * r.mt * a.N * 4; };
+  if (a.ksplit == 0 && r.S < WK_SMAX && r.S < nu && room(r.S + 1) &&
+      (r.S > 1 ? 5 * longest(r.S + 1) <= 4 * longest(r.S) : bf && r.ns == 2 && a.N / 16 <= cus / 2))
+    r.ns = stages(++r.S);
+  r.G = groups(r.S);
   if (mixed && r.G < 2) return false;
-  return r.S == 1 || (a.ws && a.cnt && a.cnt_len >= r.G && a.ws_bytes >= (size_t)r.S * 16 * r.mt * a.N * 4);
+  return r.S == 1 || room(r.S);
 }
 
 bool gemm_wk_serves(const GemmQArgs& a) {

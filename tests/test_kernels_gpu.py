@@ -1255,6 +1255,23 @@ def test_gemm_wk(E, M, segs, K, ksplit, epi):
         assert ((got - ref).norm(dim=1) / ref.norm(dim=1)).max() < tol
 
 
+@pytest.mark.parametrize("M", [2, 16, 17, 32])
+@pytest.mark.parametrize("t,N,K", [("BF16", 2048, 8704), ("Q6_K", 2048, 8704), ("Q4_K", 4096, 12288), ("BF16", 2048, 4096), ("BF16", 1088, 3136),
+                                   ("BF16", 2048, 2048)])
+def test_gemm_wk_slices_chosen_for_even_ranges(E, M, t, N, K):
+    """K in one slice more than the registers ask for, where that deals the tiles out more evenly (the last: not); tolerance: test_gemm_wk"""
+    m, W = small_mat(E, t, N, K, seed=K + N)
+    assert E.gemm_wk_serves([m], M, E.GEPI_ACCUM, 0)
+    A = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    y, Ad = A.double() @ W.T, A.cuda()
+    for _ in range(2):
+        out = torch.full((M, N), 3.0, device="cuda")
+        E.gemm_q(Ad.data_ptr(), K, [m], M, out.data_ptr(), 0, N, E.GEPI_ACCUM, stream(), 0)
+        torch.cuda.synchronize()
+        got = out.cpu().double() - 3.0
+        assert ((got - y).norm(dim=1) / y.norm(dim=1)).max() < sum_tol(t, K) + 3.0 * 2.0 ** -24 * math.sqrt(N) / float(y.norm(dim=1).min())
+
+
 SMALL = {"wk": ("", ""), "ring": ("0", ""), "skinny": ("0", "0")}
 
 
