@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK + D
         if (!full && (uint32_t)(krel + t * 32 + (r & 3) + 8 * (r >> 2)) > qspan) st[t][r] = -INFINITY;
         mx = fmaxf(mx, st[t][r]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = lane_xor32(mx, LaneMax{});
     const float mn = fmaxf(m_run, mx);
     const float ms = mn == -INFINITY ? 0.f : mn;  // (no visible key yet: a window that starts in a later tile)
     const float alpha = __builtin_amdgcn_exp2f(m_run - ms);
@@ -191,7 +191,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK + D
         pb[t][r >> 1] = hi;
         pl[t][r >> 1] = pk_bf16(p0 - __uint_as_float(hi << 16), p1 - __uint_as_float(hi & 0xffff0000u));
       }
-    ps += __shfl_xor(ps, 32, 64);
+    ps = lane_xor32(ps, LaneAdd{});
     l_run = l_run * alpha + ps;
     if (__any(mn != m_run)) {
 #pragma unroll

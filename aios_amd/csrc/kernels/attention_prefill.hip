@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[t][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = lane_xor32(mx, LaneMax{});
     const float mx_run = fmaxf(m_run, mx);
     // -inf only where a run has shown this row no key yet (never with one run: key 0 is visible): p = 0 then
     const float mn = a.ns > 1 && mx_run == -INFINITY ? 0.f : mx_run;
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         ps += p0 + p1;
         pb[t][r >> 1] = pk_bf16(p0, p1);
       }
-    ps += __shfl_xor(ps, 32, 64);
+    ps = lane_xor32(ps, LaneAdd{});
     l_run = l_run * alpha + ps;
     // the O rescale only when some row max of this wave moved (alpha == 1 on every lane otherwise)
     if (__any(mn != m_run)) {

@@ -31,48 +31,34 @@ __device__ __forceinline__ float ld_wt(const float* p) {
   return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
-}
 // sum over aligned groups of N lanes (N = 8 or 16), result in every lane of the group
 template <int N>
 __device__ __forceinline__ float group_sum(float v) {
-  v += dpp<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp<0x141>(v);  // row_half_mirror: lane i <-> 7-i within 8
-  if constexpr (N == 16) v += dpp<0x140>(v);  // row_mirror: lane i <-> 15-i within 16
+  v += lane_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += lane_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += lane_dpp<0x141>(v);  // row_half_mirror: lane i <-> 7-i within 8
+  if constexpr (N == 16) v += lane_dpp<0x140>(v);  // row_mirror: lane i <-> 15-i within 16
   return v;
 }
-// op(v[lane], v[lane ^ OFF]) for OFF = 8, 16, 32 without the LDS crossbar: DPP row rotate for 8; the gfx950
-// v_permlane16/32_swap of v with itself returns the lower and the upper row of every pair in r[0] / r[1]
-// on all lanes, so op(r[0], r[1]) needs no lane select
+// op(v[lane], v[lane ^ OFF]) for OFF = 8, 16, 32
 template <int OFF, typename Op>
 __device__ __forceinline__ float xlane_op(float v, Op op) {
-  if constexpr (OFF == 8) {
-    return op(v, dpp<0x128>(v));  // row_ror:8 within 16 lanes = lane ^ 8
-  } else if constexpr (OFF == 16) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  } else {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  }
+  if constexpr (OFF == 8) return op(v, lane_dpp<0x128>(v));  // row_ror:8 within 16 lanes = lane ^ 8
+  else if constexpr (OFF == 16) return lane_xor16(v, op);
+  else return lane_xor32(v, op);
 }
-struct OpMax { __device__ float operator()(float a, float b) const { return fmaxf(a, b); } };
-struct OpAdd { __device__ float operator()(float a, float b) const { return a + b; } };
 // max / sum over the lanes that share (lane % LPK), i.e. across the 64/LPK key groups of a wave
 template <int LPK>
 __device__ __forceinline__ float keys_max(float v) {
-  if constexpr (LPK <= 8) v = xlane_op<8>(v, OpMax{});
-  if constexpr (LPK <= 16) v = xlane_op<16>(v, OpMax{});
-  return xlane_op<32>(v, OpMax{});
+  if constexpr (LPK <= 8) v = xlane_op<8>(v, LaneMax{});
+  if constexpr (LPK <= 16) v = xlane_op<16>(v, LaneMax{});
+  return xlane_op<32>(v, LaneMax{});
 }
 template <int LPK>
 __device__ __forceinline__ float keys_sum(float v) {
-  if constexpr (LPK <= 8) v = xlane_op<8>(v, OpAdd{});
-  if constexpr (LPK <= 16) v = xlane_op<16>(v, OpAdd{});
-  return xlane_op<32>(v, OpAdd{});
+  if constexpr (LPK <= 8) v = xlane_op<8>(v, LaneAdd{});
+  if constexpr (LPK <= 16) v = xlane_op<16>(v, LaneAdd{});
+  return xlane_op<32>(v, LaneAdd{});
 }
 
 // max / sum over the four 16-lane quarters of a wave (lanes of equal column)
@@ -223,13 +209,9 @@ __device__ __forceinline__ void attn_meet(const AttnDecodeArgs& a, int h0, int s
     if (wave < G) {
       const float mv = mlane < nact ? s_pm[wave][mlane] : kNeg;
       const float lv = mlane < nact ? s_pl[wave][mlane] : 0.f;
-      float M = mv;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+      const float M = wave_max(mv);
       const float e = fast_exp2(mv - M);
-      float L = e * lv;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
+      const float L = lanes_sum<64>(e * lv);
       if (mlane < nact) s_pm[wave][mlane] = e / L;
     }
     __syncthreads();
@@ -264,13 +246,9 @@ __device__ __forceinline__ void attn_meet(const AttnDecodeArgs& a, int h0, int s
     const int g = wave;
     const float mv = mlane < nact ? s_pm[g][mlane] : kNeg;
     const float lv = mlane < nact ? s_pl[g][mlane] : 0.f;
-    float M = mv;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+    const float M = wave_max(mv);
     const float e = fast_exp2(mv - M);
-    float L = e * lv;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
+    const float L = lanes_sum<64>(e * lv);
     if (mlane < nact) s_pm[g][mlane] = e / L;
   }
   __syncthreads();
@@ -464,7 +442,7 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
     float mx = st[0][0];
 #pragma unroll
     for (int i = 1; i < 8; ++i) mx = fmaxf(mx, st[i >> 2][i & 3]);
-    const float mn = fmaxf(m, quarters(mx, OpMax{}));
+    const float mn = fmaxf(m, quarters(mx, LaneMax{}));
     // O is rescaled only when some column's max grew (wave-uniform)
     if (__builtin_amdgcn_ballot_w64(mn > m)) {
       const float alpha = fast_exp2(m - mn);
@@ -535,7 +513,7 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
     issue_k(tB);
   }
   // ---- a head's columns summed (row rotates within 16 lanes), then the 8 waves merged in LDS
-  l = quarters(l, OpAdd{});
+  l = quarters(l, LaneAdd{});
   gf32x4 z = gf32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < DT; ++i)
@@ -551,8 +529,8 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   for (int i = 0; i < DT; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      o[i][e] += dpp<0x128>(o[i][e]);                                // row_ror:8
-      if constexpr (GP == 4) o[i][e] += dpp<0x124>(o[i][e]);         // row_ror:4
+      o[i][e] += lane_dpp<0x128>(o[i][e]);                                // row_ror:8
+      if constexpr (GP == 4) o[i][e] += lane_dpp<0x124>(o[i][e]);         // row_ror:4
     }
   __syncthreads();  // every wave is done with its V tile: the LDS is the merge's
   // (the thread's number read again, opaque to the compiler: kept through the loop it costs registers that spill)

@@ -530,12 +530,9 @@ __global__ void __launch_bounds__(256) delta_step_kernel(LinScanArgs a) {
     qq = fmaf(sq[n], sq[n], qq);
     kq = fmaf(sk[n], sq[n], kq);
   }
-#pragma unroll
-  for (int d = 32; d; d >>= 1) {
-    kk += __shfl_xor(kk, d, 64);
-    qq += __shfl_xor(qq, d, 64);
-    kq += __shfl_xor(kq, d, 64);
-  }
+  kk = wave_sum(kk);
+  qq = wave_sum(qq);
+  kq = wave_sum(kq);
   if ((tid & 63) == 0) {
     dots[tid >> 6][0] = kk;
     dots[tid >> 6][1] = qq;

@@ -46,9 +46,7 @@ struct PfkRows {
         if (32 * j + 4 * (lane & 7) < a.nrm_parts) t += u;
       }
       float s = (t[0] + t[1]) + (t[2] + t[3]);
-#pragma unroll
-      for (int o = 1; o < 8; o <<= 1) s += __shfl_xor(s, o, 64);
-      inv[k] = rsqrtf(s / (float)a.K + a.nrm_eps);
+      inv[k] = rsqrtf(lanes_sum<8>(s) / (float)a.K + a.nrm_eps);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the slot's own requests follow)
   }
@@ -213,8 +211,7 @@ __device__ __forceinline__ void pfk_close(const GemmQArgs& a, const gf32x16 (&ac
       *(gf32x4*)(a.C + (size_t)m * a.ldc + n) = x;
       *(uint2*)(a.nrm_out16 + (size_t)m * a.ldc + n) = make_uint2(pk_bf16(x[0] * gain[0], x[1] * gain[1]), pk_bf16(x[2] * gain[2], x[3] * gain[3]));
       float ss = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o, 64);  // 64 columns of a row lie on 16 successive lanes
+      ss = lanes_sum<16>(ss);  // 64 columns of a row lie on 16 successive lanes
       if ((q & 15) == 0) a.nrm_part[(size_t)m * a.nrm_parts + (n >> 6)] = ss;
     } else if constexpr (EPI == GEPI_QKV) {
       const gf32x4 t = h_.c;

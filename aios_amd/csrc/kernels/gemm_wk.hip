@@ -188,8 +188,7 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
   auto finish = [&](int t, int mt, gf32x4 v, const Ahead& res) __attribute__((always_inline)) {
     float ss = res.finish(a, nrm ? inv_s : nullptr, 16 * mt + rr, 16 * t + 4 * q, v);
     if constexpr (EPI == GEPI_ACCUM_NORM) {
-      ss += __shfl_xor(ss, 16, 64);
-      ss += __shfl_xor(ss, 32, 64);
+      ss = lane_xor32(lane_xor16(ss, LaneAdd{}), LaneAdd{});
       if (q == 0 && 16 * mt + rr < a.M) a.nrm_part[(size_t)(16 * mt + rr) * a.nrm_parts + t] = ss;
     }
   };

@@ -30,36 +30,9 @@ struct CuPlan {
   int racc_n;  // LDS row accumulators: 2 x the most pairs any workgroup owns, rounded to 4
 };
 
-template <int CTRL>
-__device__ __forceinline__ float cu_dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-// sum over the 64 lanes, result in every lane: quad / half-row / row DPP, then permlane swaps
-__device__ __forceinline__ float cu_wave_sum(float v) {
-  v += cu_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += cu_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += cu_dpp<0x141>(v);  // row_half_mirror
-  v += cu_dpp<0x140>(v);  // row_mirror
-  {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  return v;
-}
-
-// sum over each 32-lane half (lanes 0-31 / 32-63), result in every lane of the half
-__device__ __forceinline__ float cu_half_sum(float v) {
-  v += cu_dpp<0xB1>(v);
-  v += cu_dpp<0x4E>(v);
-  v += cu_dpp<0x141>(v);
-  v += cu_dpp<0x140>(v);
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
+// sum over the 64 lanes, and over each 32-lane half (lanes 0-31 / 32-63); the result in every lane of them
+__device__ __forceinline__ float cu_wave_sum(float v) { return lanes_sum<64>(v); }
+__device__ __forceinline__ float cu_half_sum(float v) { return lanes_sum<32>(v); }
 
 // ---------------------------------------------------------------------------------------------
 // Q4_K chunk PAIRS with the activation operand in registers (batch-1 ring consumers).

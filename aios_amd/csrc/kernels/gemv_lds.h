@@ -263,19 +263,19 @@ __device__ __forceinline__ float lg_half_sum_rows(const float (&v)[B], int p) {
   float u;
   if constexpr (B == 2) {
     const float send = b0 ? v[0] : v[1], keep = b0 ? v[1] : v[0];
-    u = keep + cu_dpp<0xB1>(send);          // quad_perm [1,0,3,2]: lane ^ 1
-    u += cu_dpp<0x4E>(u);                   // lane ^ 2 (same row class)
+    u = keep + lane_dpp<0xB1>(send);          // quad_perm [1,0,3,2]: lane ^ 1
+    u += lane_dpp<0x4E>(u);                   // lane ^ 2 (same row class)
   } else {
     const float v3 = B == 4 ? v[B - 1] : 0.f;
     const float s0 = b0 ? v[0] : v[2], s1 = b0 ? v[1] : v3;
     const float k0 = b0 ? v[2] : v[0], k1 = b0 ? v3 : v[1];
-    const float u0 = k0 + cu_dpp<0xB1>(s0), u1 = k1 + cu_dpp<0xB1>(s1);
+    const float u0 = k0 + lane_dpp<0xB1>(s0), u1 = k1 + lane_dpp<0xB1>(s1);
     const bool b1 = (p >> 1) & 1;
     const float send = b1 ? u0 : u1, keep = b1 ? u1 : u0;
-    u = keep + cu_dpp<0x4E>(send);          // lane ^ 2
+    u = keep + lane_dpp<0x4E>(send);          // lane ^ 2
   }
-  u += cu_dpp<0x124>(u);                    // row_ror:4 within 16 lanes (keeps lane & 3)
-  u += cu_dpp<0x128>(u);                    // row_ror:8
+  u += lane_dpp<0x124>(u);                    // row_ror:4 within 16 lanes (keeps lane & 3)
+  u += lane_dpp<0x128>(u);                    // row_ror:8
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(u), __float_as_uint(u), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }

@@ -540,14 +540,15 @@ __device__ __forceinline__ void gemv_epilogue1(const GemvArgs& a, int grow, floa
 // sum of two per-lane values over the wave with 7 cross-lane steps instead of 12:
 // returns (row-0 total, row-1 total) in every lane
 __device__ __forceinline__ float2 wave_sum_pair(float a0, float a1) {
-  const int lane = threadIdx.x & 63;
-  float keep = (lane & 32) ? a1 : a0;
-  const float send = (lane & 32) ? a0 : a1;
-  keep += __shfl_xor(send, 32, 64);
-#pragma unroll
-  for (int o = 16; o > 0; o >>= 1) keep += __shfl_xor(keep, o, 64);
-  const float other = __shfl_xor(keep, 32, 64);
-  return (lane & 32) ? make_float2(other, keep) : make_float2(keep, other);
+  // a0's halves added up in the lower lanes, a1's in the upper ones
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a0), __float_as_uint(a1), false, false);
+  float s = lane_xor16(__uint_as_float(r[0]) + __uint_as_float(r[1]), LaneAdd{});
+  s += lane_dpp<0x128>(s);
+  s += lane_dpp<0x124>(s);
+  s += lane_dpp<0x4E>(s);
+  s += lane_dpp<0xB1>(s);
+  const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+  return make_float2(__uint_as_float(t[0]), __uint_as_float(t[1]));
 }
 
 // ---------------------------------------------------------------------------------------------

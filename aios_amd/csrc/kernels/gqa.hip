@@ -102,8 +102,7 @@ __global__ void __launch_bounds__(256) gqa_norm_prep_kernel(GqaArgs a, float qf,
       if (c < a.dv) v[i] = in[a.v_off + g * a.dv + c] + (a.vb ? a.vb[g * a.dv + c] : 0.f);
       ss = fmaf(v[i], v[i], ss);
     }
-#pragma unroll
-    for (int d = 32; d; d >>= 1) ss += __shfl_xor(ss, d, 64);
+    ss = wave_sum(ss);
     const float inv = a.v_norm ? 1.f / sqrtf(ss / (float)a.dv + a.eps) : 1.f, lam = a.lambda ? *a.lambda : 0.f;
     const size_t at = blk + (size_t)a.G * GQA_BLOCK * a.dkp + ((size_t)g * GQA_BLOCK + key) * a.dvp;
 #pragma unroll
@@ -141,8 +140,7 @@ __global__ void __launch_bounds__(256) gqa_norm_prep_kernel(GqaArgs a, float qf,
         ss = fmaf(u, u, ss);
       }
     }
-#pragma unroll
-    for (int d = 32; d; d >>= 1) ss += __shfl_xor(ss, d, 64);
+    ss = wave_sum(ss);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
     inv = 1.f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)n + a.eps);
@@ -325,8 +323,7 @@ gqa_attn_kernel(GqaArgs a) {
       p[i] = key <= mypos && key >= mylow ? v : -INFINITY;
       mx = fmaxf(mx, p[i]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = lane_xor32(lane_xor16(mx, LaneMax{}), LaneMax{});
     const float mn = fmaxf(m_run, mx), ms = mn == -INFINITY ? 0.f : mn;
     const float alpha = __builtin_amdgcn_exp2f(m_run - ms);
     float ps = 0.f;
@@ -369,8 +366,7 @@ gqa_attn_kernel(GqaArgs a) {
       step(kt + 4, B);
     }
   }
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = lane_xor32(lane_xor16(l_run, LaneAdd{}), LaneAdd{});
   // the four waves' sums of a row: [row][column] fp32 over the V slices
   float* so = (float*)gq_smem;
   constexpr int OS = SLICE / 2;  // floats per wave
@@ -418,13 +414,9 @@ __global__ void __launch_bounds__(256) gqa_combine_kernel(GqaArgs a) {
     m = v.x;
     l = v.y;
   }
-  float M = m;
-#pragma unroll
-  for (int d = 32; d; d >>= 1) M = fmaxf(M, __shfl_xor(M, d, 64));
+  const float M = wave_max(m);
   const float wt = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
-  float L = l * wt;
-#pragma unroll
-  for (int d = 32; d; d >>= 1) L += __shfl_xor(L, d, 64);
+  const float L = wave_sum(l * wt);
   const int cols = a.dvp >> 2, groups = 64 / cols, grp = lane / cols, c = 4 * (lane - grp * cols);
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int s0 = 0; s0 < a.nsplit; s0 += groups) {

@@ -88,8 +88,7 @@ __device__ __forceinline__ void lin_keep(const LinScanArgs& a, int k, int nkeep)
 
 // sum over the workgroup (red: 4 floats)
 __device__ __forceinline__ float lin_block_sum(float v, float* red) {
-#pragma unroll
-  for (int d = 32; d; d >>= 1) v += __shfl_xor(v, d, 64);
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();

@@ -631,8 +631,7 @@ __global__ void __launch_bounds__(256) lin_norm_kernel(LinScanArgs a, int parts,
       ss += v[i][e] * v[i][e];
     }
   if constexpr (LANES == 64) {
-#pragma unroll
-    for (int d = 32; d; d >>= 1) ss += __shfl_xor(ss, d, 64);
+    ss = wave_sum(ss);
   } else {
     ss = lin_block_sum(ss, red);
   }

@@ -166,8 +166,7 @@ struct NrmRows {
       for (int j = 256 + 4 * lane; j < a.nrm_parts; j += 256)
         if (m < a.M) v[r] += *(const gf32x4*)(a.nrm_in + (size_t)m * a.nrm_parts + j);
       float s = (v[r][0] + v[r][1]) + (v[r][2] + v[r][3]);
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
+      s = lanes_sum<64>(s);
       if (lane == 0) inv_s[m] = rsqrtf(s / (float)a.K + a.nrm_eps);
     }
   }
@@ -205,8 +204,7 @@ __device__ __forceinline__ bool sk_epilogue(const GemmQArgs& a, gf32x4 (&acc)[MT
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         float s = ss[mt];
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
+        s = lane_xor32(lane_xor16(s, LaneAdd{}), LaneAdd{});
         if (q == 0 && active) red[wave * MP + 16 * mt + rr] = s;
       }
       __syncthreads();
