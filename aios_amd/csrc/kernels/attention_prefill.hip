@@ -62,22 +62,26 @@ __device__ __forceinline__ FpRun fp_run(int start, int T, int t0, int BQ, int ns
 // staging converts the codes to bf16 (exact; v_cvt_scalef32_pk_bf16_fp8 at scale 1 -- its scale
 // operand is applied as a power of two, so the layer's K scale is folded into q and its V scale into
 // the output instead) -- the LDS tiles and the MFMA math are the bf16 kernel's
-template <int HD, int G, bool F8 = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_prefill_kernel(AttnPrefillArgs a) {
+// KG = 2 (prefill_groups): eight waves, of which the first four take the even tiles of the workgroup's 128 rows and the others the odd ones;
+// their sums meet in LDS at the end.
+template <int HD, int G, bool F8, int KG>
+__global__ void __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_prefill_kernel(AttnPrefillArgs a) {
+  constexpr int NT = 256 * KG;
   constexpr int BQ = 128 / G;          // query positions per workgroup
-  constexpr int KS = HD / 16;          // k-steps of the S MFMA
+  constexpr int QS = HD / 16;          // k-steps of the S MFMA
   constexpr int OT = HD / 32;          // O^T accumulator tiles (32 dims each)
   constexpr int KROW = HD + 8;         // padded LDS row (bf16) of the K tile
   // padded LDS row (bf16) of the row-major V tile: a 16-lane transposed read takes 4 rows x 4
   // 8-byte column chunks and its 32-lane half two such groups 16 dims apart; rows HD + 32 elements
   // apart put the 4 rows 16 banks apart (mod 64) and the two groups 8 banks apart: conflict-free
   constexpr int VROW = HD + 32;
-  // two LDS tile buffers (dynamic: 2 x 37 KB for HD 128), K then V in each
+  // two LDS buffers (dynamic) of KG tiles (37 KB for HD 128), K then V in each
   constexpr int TILE_ELEMS = FP_KT * (KROW + VROW);
   extern __shared__ __attribute__((aligned(16))) bf16_t fp_smem[];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, half = lane >> 5;
+  const int wr = __builtin_amdgcn_readfirstlane(wave & 3), kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave >> 2);
   // An XCD works on as few KV heads as there are for it, so their K and V stay in its L2: m XCDs share a list of hx heads' (query
   // block, run) items, the longest first.  Causal balance: where the list fills its CUs twice at most, what comes after the
   // first 32 m items (a CU's second workgroup) goes from the shortest up, so every CU gets about the same number of tiles.
@@ -86,7 +90,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int nx = (a.T + BQ - 1) / BQ, m = 1 << a.lm;
   const int xcd = blockIdx.x & 7, W = a.hx * nx * a.ns, w = ((blockIdx.x >> 3) << a.lm) + (xcd & (m - 1));
   if (w >= W) return;
-  int item = w < 32 * m || W > 64 * m ? w : W - 1 - (w - 32 * m);
+  int item = KG > 1 || w < 32 * m || W > 64 * m ? w : W - 1 - (w - 32 * m);  // (of eight waves one workgroup fits a CU)
   int kvh = xcd >> a.lm, run_z = 0;
   if (a.hx > 1) {  // (divisions only where there is something to divide: 0.3 us of a short prompt's 6)
     kvh = kvh * a.hx + item % a.hx;
@@ -100,20 +104,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int T = a.T, start = a.start;
   const int t0 = qb * BQ;
   // this lane's query row (column of S^T / O^T)
-  const int row = wave * 32 + l32;
+  const int row = wr * 32 + l32;
   const int tq = t0 + row / G, g = row % G;
   const bool qvalid = tq < T;
   const int tql = qvalid ? tq : T - 1;
   const int qpos = start + tql;  // absolute position: keys <= qpos are visible
   const int h = kvh * G + g;
 
-  // Q^T fragments (B operand): lane holds Q[row][16s + 8*half + 0..7] for s = 0..KS-1
-  bf16x8_t qf[KS];
+  // Q^T fragments (B operand): lane holds Q[row][16s + 8*half + 0..7] for s = 0..QS-1
+  bf16x8_t qf[QS];
   {
     const float* qp = a.q + ((size_t)tql * a.n_heads + h) * HD + 8 * half;
     const float sc = a.scale * 1.4426950408889634f * (F8 ? a.kv_scale_k : 1.f);
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
+    for (int s = 0; s < QS; ++s) {
       const float4 x0 = *(const float4*)(qp + 16 * s), x1 = *(const float4*)(qp + 16 * s + 4);
       const uint4 u = make_uint4(pk_bf16(x0.x * sc, x0.y * sc), pk_bf16(x0.z * sc, x0.w * sc),
                                  pk_bf16(x1.x * sc, x1.y * sc), pk_bf16(x1.z * sc, x1.w * sc));
@@ -141,36 +145,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   if (kt0 >= kt1) return;  // (uniform; the combine counts the runs the same way)
   const int klim = min(qpos, kt1 * FP_KT - 1);  // keys this lane sees in this run
   // ... and the least of them over the wave's rows: a tile that ends there needs no mask
-  const int klim_w = min(start + min(T - 1, t0 + __builtin_amdgcn_readfirstlane(wave) * 32 / G), kt1 * FP_KT - 1);
+  const int klim_w = min(start + min(T - 1, t0 + wr * 32 / G), kt1 * FP_KT - 1);
+  const int khi_w = start + min(T - 1, t0 + (wr * 32 + 31) / G);  // the most of them: tiles behind it are nothing to this wave
 
   // tile loader: 64 keys x HD dims of K and of V, 16 B per piece, into register buffer r (2 of
   // them: tile kt + 2 is requested while tile kt is computed, so two tiles of math cover the
   // memory latency); stage() writes one buffer to an LDS tile buffer
-  constexpr int PIECES = FP_KT * HD / 8;  // 16-B pieces per tensor per tile
-  constexpr int PPT = PIECES / 256;        // per thread
+  constexpr int PIECES = FP_KT * HD / 8;      // 16-B pieces per tensor per tile
+  constexpr int PPT = KG * PIECES / NT;       // per thread, of KG tiles
   using PT = typename std::conditional<F8, u32x2_t, u32x4_t>::type;  // one 8-element piece
   struct Regs {
     PT k[PPT], v[PPT];
   };
   const int nt_last = kt1 - 1;
-  auto load = [&](Regs& r, int kt) {
-    kt = min(kt, nt_last);  // (clamped: the pipeline's tail requests are re-reads, never unmapped blocks)
-    const size_t tbase = (size_t)kv_block(a.block_table, maxb, a.slot, kt * FP_KT) * blk_stride +
-                         (size_t)(kt & 1) * FP_KT * HD;
+  static_assert(PIECES % NT == 0, "a thread's pieces of a tile");
+  auto load = [&](Regs& r, int kt0_) {  // tiles kt0_ .. + KG - 1
     static_for<PPT>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      const int idx = tid + 256 * i, key = idx / (HD / 8), c = idx % (HD / 8);
+      constexpr int i = decltype(I)::value, t = i / (PIECES / NT);
+      const int kt = min(kt0_ + t, nt_last);  // (clamped: the pipeline's tail requests are re-reads, never unmapped blocks)
+      const size_t tbase = (size_t)kv_block(a.block_table, maxb, a.slot, kt * FP_KT) * blk_stride +
+                           (size_t)(kt & 1) * FP_KT * HD;
+      const int idx = tid + NT * (i % (PIECES / NT)), key = idx / (HD / 8), c = idx % (HD / 8);
       const size_t off = (tbase + (size_t)key * HD + c * 8) * ES;
       r.k[i] = *(const PT*)(kc + off);
       r.v[i] = *(const PT*)(vc + off);
     });
   };
-  auto stage = [&](const Regs& r, bf16_t* buf) {
-    bf16_t* sK = buf;
-    bf16_t* sV = buf + FP_KT * KROW;
+  auto stage = [&](const Regs& r, bf16_t* buf0) {
     static_for<PPT>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      const int idx = tid + 256 * i, key = idx / (HD / 8), c = idx % (HD / 8);
+      constexpr int i = decltype(I)::value, t = i / (PIECES / NT);
+      const int idx = tid + NT * (i % (PIECES / NT)), key = idx / (HD / 8), c = idx % (HD / 8);
+      bf16_t* sK = buf0 + t * TILE_ELEMS;
+      bf16_t* sV = sK + FP_KT * KROW;
       if constexpr (F8) {
         auto cv = [](u32x2_t w) {
           u32x4_t o;
@@ -188,9 +194,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       }
     });
   };
-  // one 64-key tile of math on LDS buffer buf (a tile past the last one -- the odd count's pad --
-  // is fully masked: p = 0, alpha = 1)
-  auto math = [&](const bf16_t* buf, int kt) {
+  // one 64-key tile of math on LDS buffer buf
+  auto math = [&](const bf16_t* buf0, int kt_) {
+    const bf16_t* buf = buf0 + kg * TILE_ELEMS;
+    const int kt = kt_ + kg;
+    if ((KG > 1 && kt >= kt1) || kt * FP_KT > khi_w) return;  // (uniform over the wave)
     const bf16_t* sK = buf;
     const bf16_t* sV = buf + FP_KT * KROW;
     // ---- S^T = K Q^T for the tile's two 32-key halves
@@ -201,7 +209,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int e = 0; e < 16; ++e) st[t][e] = 0.f;
       const bf16_t* kr = sK + (t * 32 + l32) * KROW + 8 * half;
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
+      for (int s = 0; s < QS; ++s) {
         const uint4 u = *(const uint4*)(kr + 16 * s);
         bf16x8_t kf;
         __builtin_memcpy(&kf, &u, 16);
@@ -224,8 +232,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[t][r]);
     mx = lane_xor32(mx, LaneMax{});
     const float mx_run = fmaxf(m_run, mx);
-    // -inf only where a run has shown this row no key yet (never with one run: key 0 is visible): p = 0 then
-    const float mn = a.ns > 1 && mx_run == -INFINITY ? 0.f : mx_run;
+    // -inf only where a run or key group has shown this row no key yet (never with one of each: key 0 is visible): p = 0 then
+    const float mn = (KG > 1 || a.ns > 1) && mx_run == -INFINITY ? 0.f : mx_run;
     const float alpha = raw_exp2(m_run - mn);  // exp2(-inf) = 0 on the first tile
     float ps = 0.f;
     uint32_t pb[2][8];  // P^T as packed bf16 pairs, accumulator order
@@ -276,24 +284,57 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   // 2k-token layer): two register buffers A / B and two LDS tile buffers L0 / L1, ONE barrier per
   // tile.  Iteration kt computes tile kt from L[kt & 1] while tile kt + 2 is requested into the
   // register buffer just staged, then stages tile kt + 1 into the other LDS buffer (last read two
-  // iterations ago, before the previous barrier) and barriers.  Branch-free: tiles run in pairs, an
-  // odd count computes one fully masked pad tile.
+  // iterations ago, before the previous barrier) and barriers.  (An odd count's last tile ends the loop: a fully masked one
+  // behind it was 1.5 us of a short prompt's launch: us, with it -> so, 23 tokens, 32 / 4 heads of 64 5.8 -> 4.6, 130 tokens, 32 / 8 of 128
+  // 9.8 -> 8.5, 711 22.7 -> 20.6)
   bf16_t* L0 = fp_smem;
-  bf16_t* L1 = fp_smem + TILE_ELEMS;
+  bf16_t* L1 = fp_smem + KG * TILE_ELEMS;
   Regs A, B;
   load(A, kt0);
-  load(B, kt0 + 1);
+  load(B, kt0 + KG);
   stage(A, L0);
   __syncthreads();
-  for (int kt = kt0; kt < kt1; kt += 2) {
-    load(A, kt + 2);
+  for (int kt = kt0;; kt += 2 * KG) {  // (the exits are uniform)
+    load(A, kt + 2 * KG);
     math(L0, kt);
+    if (kt + KG >= kt1) break;
     stage(B, L1);
     __syncthreads();
-    load(B, kt + 3);
-    math(L1, kt + 1);
+    load(B, kt + 3 * KG);
+    math(L1, kt + KG);
+    if (kt + 2 * KG >= kt1) break;
     stage(A, L0);
     __syncthreads();
+  }
+  if constexpr (KG > 1) {  // ---- the second group's sums to the first
+    static_assert(KG == 2, "two key groups");
+    float* xo = (float*)fp_smem + wr * (OT * 16 * 64);
+    float* xm = (float*)fp_smem + 4 * (OT * 16 * 64) + wr * 128;
+    __syncthreads();  // every wave is done with its tiles
+    if (kg) {
+#pragma unroll
+      for (int i = 0; i < OT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) *(float4*)(xo + ((i * 4 + (r >> 2)) * 64 + lane) * 4) = make_float4(o[i][r], o[i][r + 1], o[i][r + 2], o[i][r + 3]);
+      xm[lane] = m_run;
+      xm[64 + lane] = l_run;
+    }
+    __syncthreads();
+    if (kg) return;
+    const float m1 = xm[lane], M = fmaxf(m_run, m1), M0 = M == -INFINITY ? 0.f : M;
+    const float w0 = raw_exp2(m_run - M0), w1 = raw_exp2(m1 - M0);
+    l_run = l_run * w0 + xm[64 + lane] * w1;
+    m_run = M;
+#pragma unroll
+    for (int i = 0; i < OT; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; r += 4) {
+        const float4 x = *(const float4*)(xo + ((i * 4 + (r >> 2)) * 64 + lane) * 4);
+        o[i][r] = o[i][r] * w0 + x.x * w1;
+        o[i][r + 1] = o[i][r + 1] * w0 + x.y * w1;
+        o[i][r + 2] = o[i][r + 2] * w0 + x.z * w1;
+        o[i][r + 3] = o[i][r + 3] * w0 + x.w * w1;
+      }
   }
   // ---- O^T[dim][row], dim = 32 i + (r&3) + 8 (r>>2) + 4 half
   if (a.ns > 1) {  // this run's part: O, row max and row sum in fp32
@@ -371,38 +412,60 @@ constexpr int FP_RUN = 8;
 // by the long ones anyway, and two or three runs only pay the second launch (TinyLlama, 909 tokens behind 179 in two
 // runs: the whole prefill 0.9 % slower; Mistral, 300 behind 6000 in six: 15035 -> 11880 us).
 
-static int prefill_runs(const AttnPrefillArgs& a, int BQ) {
-  const int wg = (a.T + BQ - 1) / BQ * a.n_kv_heads, ntiles = (a.start + a.T - 1) / FP_KT + 1;
-  if (4 * wg > std::min(FP_WG, 2 * device_cu_count())) return 1;
-  const int ns = std::min(std::min(FP_WG, 2 * device_cu_count()) / wg, ntiles / FP_RUN);
+// KG: key groups of a workgroup; of eight waves one is resident on a CU, of four two
+static int prefill_runs(const AttnPrefillArgs& a, int BQ, int KG) {
+  const int wg = (a.T + BQ - 1) / BQ * a.n_kv_heads, ntiles = (a.start + a.T - 1) / FP_KT + 1, slots = std::min(FP_WG, 2 * device_cu_count());
+  if (4 * wg > slots) return 1;
+  const int ns = std::min(slots / (KG * wg), ntiles / FP_RUN);
   const size_t need = (size_t)ns * a.T * a.n_heads * (a.head_dim + 2) * sizeof(float);
   return ns > 1 && a.ws && need <= a.ws_bytes ? ns : 1;
+}
+
+// Key groups of a launch: two where its workgroups are two rounds of the CUs at most, so that a second workgroup for every CU is not there
+// all the time, and the longest has ten tiles, which pay for the meeting.  us in one / two groups: 32 / 8 heads of 128, 130 tokens 8.7 / 10.9,
+// 500 17.5 / 17.3, 711 22.4 / 21.6, 1024 29.8 / 26.7, 1500 43.0 / 37.3, 2048 56.8 / 55.6, 3000 91 / 111; 1000 behind 2000 71.5 / 59.8, fp8
+// behind 3000 94.7 / 77.9; fp8 in runs, behind 6000: 16 tokens 23.9 / 24.1, 100 35.6 / 29.6, 300 56.5 / 53.1 (three runs instead of six);
+// 32 / 4 heads of 64, 500 tokens 11.3 / 10.6, 1000 19.2 / 16.3, 2000 36.2 / 33.9.
+static int prefill_groups(const AttnPrefillArgs& a, int BQ) {
+  const int wg = (a.T + BQ - 1) / BQ * a.n_kv_heads, ntiles = (a.start + a.T - 1) / FP_KT + 1;
+  return ntiles >= 10 && wg <= 2 * device_cu_count() ? 2 : 1;
 }
 
 // FP_WG workgroups of 128 rows each, O and (max, sum) in fp32
 size_t attn_prefill_ws_bytes(int head_dim) { return (size_t)FP_WG * 128 * (head_dim + 2) * sizeof(float); }
 
-template <int HD, bool F8>
-static void prefill_hd(AttnPrefillArgs a, int G, hipStream_t st) {
-  const int BQ = 128 / G;
-  a.ns = prefill_runs(a, BQ);
+template <int HD, int G, bool F8, int KG>
+static void prefill_go(AttnPrefillArgs a, hipStream_t st) {
+  constexpr int BQ = 128 / G;
+  a.ns = prefill_runs(a, BQ, KG);
   const int ny = a.n_kv_heads;
   a.lm = ny % 8 == 0 ? 0 : (ny == 4 ? 1 : (ny == 2 ? 2 : 3));  // (neither a divisor nor a multiple of 8: all XCDs share all heads)
   a.hx = ny % 8 == 0 ? ny / 8 : (8 % ny == 0 ? 1 : ny);
   const int m = 1 << a.lm;
   const int W = a.hx * ((a.T + BQ - 1) / BQ) * a.ns;
   const dim3 grid(8 * ((W + m - 1) / m));  // (the kernel's lists, one place in turn on each XCD)
-  const size_t lds = (size_t)2 * FP_KT * ((HD + 8) + (HD + 32)) * sizeof(bf16_t);  // two K|V tile buffers
-  switch (G) {
-    case 1: hipLaunchKernelGGL((attn_prefill_kernel<HD, 1, F8>), grid, dim3(256), lds, st, a); break;
-    case 2: hipLaunchKernelGGL((attn_prefill_kernel<HD, 2, F8>), grid, dim3(256), lds, st, a); break;
-    case 4: hipLaunchKernelGGL((attn_prefill_kernel<HD, 4, F8>), grid, dim3(256), lds, st, a); break;
-    case 8: hipLaunchKernelGGL((attn_prefill_kernel<HD, 8, F8>), grid, dim3(256), lds, st, a); break;
-    default: throw std::runtime_error("attn_prefill: unsupported GQA group size");
-  }
+  const size_t lds = (size_t)2 * KG * FP_KT * ((HD + 8) + (HD + 32)) * sizeof(bf16_t);  // two buffers of KG K|V tiles
+  hipLaunchKernelGGL((attn_prefill_kernel<HD, G, F8, KG>), grid, dim3(256 * KG), lds, st, a);
   if (a.ns > 1)
     hipLaunchKernelGGL((attn_prefill_combine<HD>), dim3((a.T * a.n_heads + 3) / 4), dim3(256), 0, st, a, BQ,
                        F8 ? a.kv_scale_v : 1.f);
+}
+
+template <int HD, int G, bool F8>
+static void prefill_form(const AttnPrefillArgs& a, hipStream_t st) {
+  if (prefill_groups(a, 128 / G) == 2) prefill_go<HD, G, F8, 2>(a, st);
+  else prefill_go<HD, G, F8, 1>(a, st);
+}
+
+template <int HD, bool F8>
+static void prefill_hd(const AttnPrefillArgs& a, int G, hipStream_t st) {
+  switch (G) {
+    case 1: prefill_form<HD, 1, F8>(a, st); break;
+    case 2: prefill_form<HD, 2, F8>(a, st); break;
+    case 4: prefill_form<HD, 4, F8>(a, st); break;
+    case 8: prefill_form<HD, 8, F8>(a, st); break;
+    default: throw std::runtime_error("attn_prefill: unsupported GQA group size");
+  }
 }
 
 void launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t st) {

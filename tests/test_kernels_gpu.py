@@ -1002,6 +1002,14 @@ def test_attention_prefill_lists_of_heads(E, H, Hkv, hd, start, T):
         assert float((got[:, h] - ref).norm() / ref.norm()) < 2 ** -8, h
 
 
+@pytest.mark.parametrize("H,Hkv,hd,start,T", [
+    (32, 8, 128, 0, 576), (32, 8, 128, 0, 577), (8, 8, 64, 0, 640), (8, 1, 64, 0, 641), (2, 2, 128, 0, 705), (16, 8, 128, 570, 7), (4, 1, 128, 639, 1),
+    (32, 4, 64, 1000, 333), (32, 8, 128, 4000, 16)])
+def test_attention_prefill_key_groups(E, H, Hkv, hd, start, T):
+    """nine tiles (one key group) and ten, even and odd counts of a workgroup, rows that the second group has no key for; in runs too"""
+    test_attention_prefill_lists_of_heads(E, H, Hkv, hd, start, T)
+
+
 @pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (16, 8, 128)])
 @pytest.mark.parametrize("start,T", [(1023, 1), (960, 64), (1100, 37), (3777, 300), (961, 129), (4000, 31)])
 @pytest.mark.parametrize("fp8", [False, True])
