@@ -2,7 +2,7 @@
 //   C[M][N] = X[M][K] x W[N][K]^T,  W in the repacked Q6_K planes (qweight.h).
 //
 // It serves the Q6_K launches where it is the faster one, or where the K-shared GEMM has no form (gemm_wk.hip, wk_route):
-// long K up to 16 rows, the packed QKV from 17 rows up.  The weight stream is the batch-1 engine's (gemv_lds.h): per CU
+// 8448 to 10240 k up to 16 rows, the packed QKV from 17 rows up.  The weight stream is the batch-1 engine's (gemv_lds.h): per CU
 // one workgroup, two loader waves move every weight byte HBM -> LDS by buffer_load ... lds into a ring of R slots, R - 1
 // in flight, never waiting for compute; eight MFMA waves dequantise the slot in registers and multiply it with the X rows
 // staged in the same slot (dequant-to-bf16 + v_mfma_f32_16x16x32_bf16, the weight rows as the A operand).

@@ -8,15 +8,22 @@
 // 16 rows, so 256 CUs share any N evenly, and most shapes need no K split over workgroups, whose slabs and ticket cost
 // ~4 us of a launch.
 //
-// Bounds: a launch of few tiles, ~4 us of launch, first loads and output; a long one, the weight decode beside the
-// stream (Q4_K 2.5 VALU instructions a weight: gate/up with the decode left out took 16.2 us of 19.2).  Measured in us, the LDS ring
-// GEMM (gemm_ring.hip) -> this, 16 / 32 rows, weights from memory:
+// The weights of a stage are asked for in whole lines, eight lanes to a row's 128 bytes, and take the order of the matrix instruction's
+// lanes through the wave's own LDS.  Asked for in that order (16 lanes, 16 rows) each lane is an address of its own to the address unit,
+// and a launch was as long as those take.  us, so -> in whole lines, 16 rows (3 rows alike, 30 rows 0.9 to 2.9 less):
+//   bf16 8704 x 2048 12.1 -> 9.9   2048 x 8704 13.1 -> 11.8   8192 x 2048 10.3 -> 8.8   2048 x 2048 6.2 -> 5.3   11264 x 2048 12.8 -> 10.9
+//   Q4_K 4096 x 14336 15.0 -> 13.9   4096 x 4096 6.6 -> 6.3   6144 x 4096 8.7 -> 8.0   28672 x 4096 19.8 -> 19.2   Q6_K 32000 x 4096 30.0 -> 28.5
+// Bounds: a launch of few tiles, ~4 us of launch, first loads and output; bf16, the stream (11264 x 2048 4.2 TB/s of the launch); a long quantised
+// one, the decode beside the stream (28672 x 4096: the vector unit is issued to for 58 % of a launch, the waves wait for 36 %).
+// Measured in us, the LDS ring GEMM (gemm_ring.hip) -> this before it asked for whole lines, 16 / 32 rows, weights from memory:
 //   4096 x 4096 Q4_K 10.1 -> 6.3 / 12.1 -> 8.2     28672 x 4096 Q4_K 20.6 -> 18.0 / 26.1 -> 20.8
 //   6144 x 4096 Q4_K 11.4 -> 8.5 / 13.2 -> 10.7    4096 x 14336 Q4_K 15.5 -> 14.6 / 18.4 -> 17.1
 //   2048 x 2048 Q4_K 8.0 -> 4.5 / 10.0 -> 5.5      2048 x 5632 Q4_K 10.1 -> 7.5 / 12.6 -> 9.4
 //   2048 x 2048 bf16 10.4 -> 5.9 / 12.4 -> 7.0     11264 x 2048 bf16 13.4 -> 12.6 / 15.1 -> 14.0
 // Not better: X streamed with the weights instead of kept (4096 x 14336 in one slice 19.0), two tiles of weights in
-// flight (gate/up 20.1: longer code, and the decode is the bound), 16 waves (22), weights requested before X (O 7.4).
+// flight (gate/up 20.1: longer code, and the decode is the bound), 16 waves (22), weights requested before X (O 7.4), by LDS-DMA into a ring of
+// the wave's own (20.3), all of a tile's next requests before its decode (21.3: the waves stand before the address unit), the records of
+// scales in whole lines too (the same).
 #include "gemm_pf.h"
 #include "skinny_epi.h"
 
@@ -34,8 +41,8 @@ struct WkPlan {
   QWeight w_last;
 };
 
-// one stage: 256 k of a tile's 16 rows.  Lane (row rr, quarter q) holds the chunks 2q and 2q + 1 (k 64 q .. + 63),
-// bf16: the MFMA operands as they are
+// one stage: 256 k of a tile's 16 rows.  a: as loaded, row 8i + lane / 8 of 16 B; turned (turn_w), lane (row rr, quarter q) holds the
+// chunks 2q and 2q + 1 (k 64 q .. + 63), bf16: the MFMA operands as they are
 template <int QT>
 struct WkRaw {
   gu32x4 a[2], b;
@@ -56,6 +63,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t wk_rsrc(const void* p, uint32_
 
 // X unit swizzle (16-B units of a 512-B row): 16 rows' reads of one unit fall on distinct banks
 __device__ __forceinline__ int wk_xh(int m) { return (m ^ (m << 1)) & 15; }
+// ... for 128-B rows of weights (two rows to the banks)
+__device__ __forceinline__ int wk_wh(int r) { return (r & 6) | (r >> 3); }
 
 // LAST: the tiles lie in the last segment (p.w_last)
 template <int QT, int NS, int MT, int EPI, bool LAST>
@@ -125,16 +134,16 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
         const int uu = u0 + 4 * s + u;
         const auto r = wk_rsrc(p0 + row0 * rb, live && uu < u1 ? 16 * rb : 0);
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
-          w.a[2 * u + f] = __builtin_amdgcn_raw_buffer_load_b128(r, rr * rb + 16 * q, uu * 128 + 64 * f, 2);
+        for (int i = 0; i < 2; ++i)
+          w.a[2 * u + i] = __builtin_amdgcn_raw_buffer_load_b128(r, (8 * i + (lane >> 3)) * rb + 16 * (lane & 7), uu * 128, 2);
       }
     } else {
       const int uu = u0 + s;
       const bool on = live && uu < u1;
       const auto rc = wk_rsrc(p0 + row0 * nbk * 128, on ? 16 * nbk * 128 : 0);
-      const uint32_t vo = rr * nbk * 128 + 32 * q;
-      w.a[0] = __builtin_amdgcn_raw_buffer_load_b128(rc, vo, uu * 128, 2);
-      w.a[1] = __builtin_amdgcn_raw_buffer_load_b128(rc, vo + 16, uu * 128, 2);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        w.a[i] = __builtin_amdgcn_raw_buffer_load_b128(rc, (8 * i + (lane >> 3)) * nbk * 128 + 16 * (lane & 7), uu * 128, 2);
       if constexpr (Q6) {
         const auto rh = wk_rsrc(plane([](const QWeight& v) { return v.p1; }) + row0 * nbk * 64, on ? 16 * nbk * 64 : 0);
         const auto rs = wk_rsrc(plane([](const QWeight& v) { return v.p2; }) + row0 * nbk * 16, on ? 16 * nbk * 16 : 0);
@@ -146,6 +155,21 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
         const auto rm = wk_rsrc(plane([](const QWeight& v) { return v.p1; }) + row0 * nbk * 16, on ? 16 * nbk * 16 : 0);
         w.b = __builtin_amdgcn_raw_buffer_load_b128(rm, rr * nbk * 16, uu * 16, 0);
       }
+    }
+  };
+  // a stage from whole lines to the lanes' own rows, through the wave's own LDS (behind the partial sums)
+  uint8_t* const codes = own + 4096;
+  auto turn_w = [&](WkRaw<QT>& w) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < (BF ? 4 : 1); ++u) {
+      uint8_t* const to = codes + 2048 * (u & 1);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = 8 * i + (lane >> 3);
+        *(gu32x4*)(to + r * 128 + 16 * ((lane & 7) ^ wk_wh(r))) = w.a[2 * u + i];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) w.a[2 * u + i] = *(const gu32x4*)(to + rr * 128 + 16 * ((BF ? 4 * i + q : 2 * q + i) ^ wk_wh(rr)));
     }
   };
   gf32x4 acc[MT][2];
@@ -222,7 +246,9 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
   for (int s = 0; s < NS; ++s) load(w[s], s, t0);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int s = 0; s < NS; ++s) turn_x(x[s]);
+  for (int s = 0; s < NS; ++s) {
+    turn_x(x[s]);
+  }
   if (nrm) nr.done(a, wave, lane, inv_s);  // (read after the first tile's barrier)
   // what the outputs need besides their sums is requested before the tile's products (by every wave: which of them adds the tile up
   // is not worth a branch here).  Behind the sums it was one or two trips to memory at the end of a launch.
@@ -250,7 +276,10 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      if (s + 1 < NS || u0 + s * (256 / UK) < u1) compute(w[s], x[s]);
+      if (s + 1 < NS || u0 + s * (256 / UK) < u1) {
+        turn_w(w[s]);
+        compute(w[s], x[s]);
+      }
       load(w[s], s, t + 1);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -359,35 +388,37 @@ static bool wk_route(const GemmQArgs& a, WkRoute& r) {
   while (stages(r.S) > NSM) ++r.S;
   if (r.S > WK_SMAX) return false;
   r.ns = stages(r.S);
-  // Q6_K's long down projections up to 16 rows: the ring's deeper stream is the faster one where its 128-row tiles in
-  // eight slices cover three quarters of the CUs.  us here / ring, 4 and 16 rows (7 runs each, apart by 2 % at most):
-  //   4096 x 14336 19.3 / 18.3, 19.8 / 19.1    4096 x 12288 18.1 / 16.6, 18.4 / 17.4    5120 x 17408 28.2 / 26.2, 29.0 / 27.1
-  //   3584 x 18944 22.7 / 22.0, 23.4 / 23.1    8192 x 28672 59.1 / 55.1, 60.2 / 57.3    4096 x 11008 16.5 / 16.5, 17.0 / 16.9
-  //   2048 x 8704 11.5 / 12.4, 11.8 / 13.2
-  if (qt0 == QT_Q6_K && r.S > 2 && r.mt == 1 && a.N % 128 == 0 && a.N / 128 * 8 * 4 >= 3 * device_cu_count()) return false;
-  // bf16, whose stream is all there is to it: the skinny GEMM is the faster one where a tile has little k for eight waves to
-  // share, where slabs cost (long K; two 16-row groups and a wide output), and where its tiles in eight slices are one
-  // round.  us here / skinny: 128256 x 512, 16 rows 45 / 37, 32000 x 64 9.8 / 5.4, 32000 x 512 13.3 / 15.9;
-  // 4096 x 14336 34 / 30, 2048 x 14336 18 / 24; 128256 x 4096, 32 rows 256 / 226, 16 rows 214 / 215, 32000 x 4096 equal;
-  // 4096 x 8192, 32 rows 25 / 22, 8192 x 8192 37 / 40
-  const int round = a.N / 128 * 8, cus = device_cu_count();
-  if (bf && (a.N > 125L * a.K || (a.K > 12288 && a.N >= 4096) ||
-             (r.mt == 2 && ((r.S >= 2 && a.N >= 65536) || (r.S >= 4 && 4 * round >= 3 * cus && round <= cus)))))
-    return false;
+  // Q6_K in three slices of at most 13 blocks, up to 16 rows: the ring's deeper stream where its 128-row tiles in eight slices cover three
+  // quarters of the CUs.  us here / ring, 4 and 16 rows: 4096 x 9216 14.6 / 14.0, 14.8 / 15.0   4096 x 10240 15.1 / 14.8, 15.6 / 15.9
+  //   6144 x 8448 17.1 / 17.0, 17.5 / 18.0   4096 x 8448 13.5 / 13.7, 13.5 / 14.5; but 4096 x 11008 15.0 / 16.0, 15.7 / 16.8
+  //   4096 x 12288 15.8 / 16.7, 16.5 / 17.4   4096 x 14336 17.8 / 18.6, 18.3 / 19.2   8192 x 28672 50.5 / 54.9, 53.4 / 57.6
+  const int cus = device_cu_count(), round = a.N / 128 * 8;
+  if (qt0 == QT_Q6_K && r.S == 3 && nu <= 40 && r.mt == 1 && a.N % 128 == 0 && 4 * round >= 3 * cus) return false;
+  // bf16 where a tile has little k for eight waves to share: the skinny GEMM.  us here / skinny, 16 rows: 128256 x 512 44 / 33, 32000 x 64 9.7 / 5.5;
+  // but 32000 x 512 13.2 / 15.4, 128256 x 4096 170 / 224, 32 rows 188 / 233.  And, for bf16 results as they were, where slabs cost (long K
+  // and a wide output; two 16-row groups of one round of its tiles), though it is ahead no longer: 4096 x 14336 24 / 27, 4096 x 8192, 32 rows 19 / 20
+  if (bf && (a.N > 125L * a.K || (a.K > 12288 && a.N >= 4096) || (r.mt == 2 && r.S >= 4 && 4 * round >= 3 * cus && round <= cus))) return false;
   // (three segments' four planes and the cache's arguments: more scalars than there are)
   if (a.epi == GEPI_QKV && qt0 == QT_Q6_K && r.ns * r.mt == 4) return false;
-  // One slice more where that deals the tiles out more evenly: G ranges of whole tiles leave CUs idle while the longest range ends.  With a split
-  // that there is anyway, from a fifth less for the longest range up; us before / so, 16 and 30 rows: 2048 x 8704 bf16 (three slices of
-  // 85 ranges, 43 of them two tiles long) 14.9 / 13.2, 16.0 / 16.0 (eight already); Q6_K 11.7 / 10.7, 14.3 / 13.2, Q4_K 9.7 / 9.0, 12.0 / 11.2;
-  // 4096 x 12288 Q4_K 14.4 / 14.1, 17.2 / 16.7; 2048 x 5632 bf16, 30 rows 12.2 / 11.2; but 5120 x 17408 Q4_K, 8 % less 20.7 / 21.6.
-  // Two slices instead of one: bf16 where its tiles are for half of the CUs at most and a wave has two stages: 2048 x 4096 9.2 / 8.5, 1024 x 4096
-  // 9.0 / 7.6, 2048 x 3072 8.5 / 7.9; but 2048 x 2048, one stage, 6.2 / 7.0, and Q4_K, a third of the bytes, 2048 x 4096 6.2 / 7.0.
+  // One slice more where that deals the tiles out more evenly: G ranges of whole tiles leave CUs idle while the longer ranges end.  With a split
+  // that there is anyway, from a fifth less for the longest range up, if a quarter of the ranges are longer ones; us before / so, 16 and 30 rows:
+  // 2048 x 8704 (three slices of 85 ranges, 43 of them two tiles long) bf16 12.7 / 11.8, 13.0 / 12.9 (eight already), Q6_K 11.1 / 10.2, 13.6 / 12.5,
+  // Q4_K 9.2 / 8.8, 11.4 / 10.8; 2048 x 5632 bf16, 30 rows 10.6 / 9.9; but 4096 x 12288 (one of 85 ranges is longer) Q4_K 12.5 / 13.2, 14.9 / 15.9,
+  // Q6_K 16.5 / 17.2; 5120 x 17408 Q4_K, 8 % less 18.4 / 18.8.
+  // bf16, two slices instead of one where its tiles are for three eighths of the CUs at most and a wave has two stages: 1024 x 4096 7.2 / 6.5,
+  // 1280 x 4096 7.3 / 6.8, 1536 x 4096 7.4 / 7.1, 1024 x 3072 6.7 / 6.3; but 2048 x 4096 7.5 / 7.8, 2048 x 2048, one stage, 5.3 / 6.6, Q4_K 2048 x 4096
+  // 5.8 / 6.8.  Four instead of two, which leave a wave one stage of more tiles, up to 7168 k and where the longest range gets shorter: 2048 x 5632
+  // 9.6 / 8.7, 2048 x 6912 10.2 / 9.4, 1536 x 5632 9.0 / 8.3, 4096 x 5632 12.9 / 12.4, 3072 x 8192 15.4 / 13.1; but 2048 x 8192 10.8 / 13.1.
   auto groups = [&](int S) { return std::min(a.N / 16, std::max(1, cus / S)); };
   auto longest = [&](int S) { return (long)((a.N / 16 + groups(S) - 1) / groups(S)) * ((nu + S - 1) / S); };
   auto room = [&](int S) { return a.ws && a.cnt && a.cnt_len >= groups(S) && a.ws_bytes >= (size_t)S * 16 * r.mt * a.N * 4; };
+  auto shorter = [&](int S) { return 5 * longest(S) <= 4 * longest(r.S); };
   if (a.ksplit == 0 && r.S < WK_SMAX && r.S < nu && room(r.S + 1) &&
-      (r.S > 1 ? 5 * longest(r.S + 1) <= 4 * longest(r.S) : bf && r.ns == 2 && a.N / 16 <= cus / 2))
-    r.ns = stages(++r.S);
+      (r.S > 1 ? shorter(r.S + 1) && 4 * (a.N / 16 % groups(r.S)) >= groups(r.S) : bf && r.ns == 2 && 8 * (a.N / 16) <= 3 * cus))
+    ++r.S;
+  else if (a.ksplit == 0 && bf && r.mt == 1 && r.S == 2 && room(4) && (a.K <= 7168 || shorter(4)))
+    r.S = 4;
+  r.ns = stages(r.S);
   r.G = groups(r.S);
   if (mixed && r.G < 2) return false;
   return r.S == 1 || room(r.S);

@@ -1280,6 +1280,24 @@ def test_gemm_wk_slices_chosen_for_even_ranges(E, M, t, N, K):
         assert ((got - y).norm(dim=1) / y.norm(dim=1)).max() < sum_tol(t, K) + 3.0 * 2.0 ** -24 * math.sqrt(N) / float(y.norm(dim=1).min())
 
 
+@pytest.mark.parametrize("M", [3, 16, 17])
+@pytest.mark.parametrize("t,N,K", [("BF16", 1600, 5632), ("BF16", 2048, 7168), ("BF16", 3072, 8192), ("BF16", 2048, 8192), ("Q6_K", 3072, 10240),
+                                   ("Q6_K", 3072, 10496), ("Q6_K", 3072, 14336)])
+def test_gemm_wk_four_slices_and_long_q6k(E, M, t, N, K):
+    """both sides of the lines for four slices in place of two, and for Q6_K's long products (10240: the ring's up to 16 rows);
+    tolerance: test_gemm_wk"""
+    m, W = small_mat(E, t, N, K, seed=K + N)
+    assert t == "BF16" or E.gemm_wk_serves([m], M, E.GEPI_ACCUM, 0) == (K > 10240 or M > 16)
+    A = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    y, Ad = A.double() @ W.T, A.cuda()
+    for _ in range(2):
+        out = torch.full((M, N), 3.0, device="cuda")
+        E.gemm_q(Ad.data_ptr(), K, [m], M, out.data_ptr(), 0, N, E.GEPI_ACCUM, stream(), 0)
+        torch.cuda.synchronize()
+        got = out.cpu().double() - 3.0
+        assert ((got - y).norm(dim=1) / y.norm(dim=1)).max() < sum_tol(t, K) + 3.0 * 2.0 ** -24 * math.sqrt(N) / float(y.norm(dim=1).min())
+
+
 SMALL = {"wk": ("", ""), "ring": ("0", ""), "skinny": ("0", "0")}
 
 
