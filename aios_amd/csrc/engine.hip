@@ -900,19 +900,25 @@ void Engine::gemm(GemmQArgs& g) {
 //   TinyLlama Q4_K (25 MB a layer)   2 rows  912 / 798    3 rows 1044 / 801    4 rows 1101 / 796
 //   Mistral-7B Q4_K (123 MB)         2 rows 1761 / 2024   3 rows 1969 / 2025   4 rows 2231 / 2014
 //   Qwen3-8B Q4_K (108 MB)           2 rows 2130 / 2337   3 rows 2389 / 2348   4 rows 2685 / 2364
-//   TinyLlama bf16                   2 rows  852 / 1006   3 rows  919 / 1012   4 rows  976 / 1007
-// The int8 GEMV's dot work grows with the rows, the GEMM's does not: it wins from 4, and from 2 where the layers are
+//   TinyLlama bf16 (88 MB)           2 rows  869 / 911    3 rows  922 / 904    4 rows  971 / 909
+//   Mistral-7B bf16 (436 MB)         2 rows 2969 / 3058   3 rows 3271 / 3089   4 rows 3813 / 3096
+// The GEMV's dot work grows with the rows, the GEMM's does not.  Quantised weights: it wins from 4, and from 2 where the layers are
 // so small that launches bound a step (TinyLlama's d_ff has no GEMV plan at 2 rows either, so its GEMVs above are the
-// row-pair ones).  Only where K-shared waves serve every projection (Q4_K / Q6_K) and the GEMV would take int8
-// activations; across ranks as before.
+// row-pair ones); where the GEMV would take int8 activations.  bf16: from 3.  Only where K-shared waves serve every projection (all
+// Q4_K / Q6_K, or all bf16); across ranks as before.
 int Engine::default_gemm_min_b() const {
-  if (!cfg_.act_q8 || cfg_.tp_size > 1 || !gemm_wk_on()) return dec_gemm_min_b_;
-  size_t bytes = 0;
+  if (cfg_.tp_size > 1 || !gemm_wk_on()) return dec_gemm_min_b_;
+  size_t bytes = 0, n = 0, bf = 0, kq = 0;
   for (const auto& L : layers_)
     for (const QMat* m : {&L.wq, &L.wk, &L.wv, &L.wo, &L.wgu, &L.wdown}) {
-      if (m->w.qtype != QT_Q4_K && m->w.qtype != QT_Q6_K) return dec_gemm_min_b_;
+      ++n;
+      bf += m->w.qtype == QT_BF16;
+      if (m->w.qtype != QT_Q4_K && m->w.qtype != QT_Q6_K) continue;
+      ++kq;
       bytes += (size_t)m->w.rows * m->w.cols / 256 * (m->w.qtype == QT_Q4_K ? 144 : 210);
     }
+  if (bf == n) return std::min(dec_gemm_min_b_, 3);
+  if (!cfg_.act_q8 || kq != n) return dec_gemm_min_b_;
   return std::min(dec_gemm_min_b_, bytes <= layers_.size() * ((size_t)64 << 20) ? 2 : 4);
 }
 

@@ -400,6 +400,29 @@ def test_small_batches_stay_on_the_gemv_without_the_k_shared_gemm(monkeypatch, B
     assert not np.array_equal(outs["on"], outs["off"])
 
 
+@pytest.mark.parametrize("B", [2, 3, 4])
+def test_bf16_batches_take_the_gemms_from_three_rows(monkeypatch, B):
+    """bf16 weights: the GEMMs from 3 rows, the GEMVs at 2; both round what a projection reads to bf16, eight times in two layers"""
+    import dataclasses
+
+    from aios_amd.runtime.loader import random_engine
+
+    cfg, outs = dataclasses.replace(get_preset("tinyllama-1.1b"), n_layers=2, vocab_size=2048), {}
+    prompts = [list(range(5 + b, 15 + 2 * b)) for b in range(B)]
+    for min_b in (None, "5"):
+        with monkeypatch.context() as mp:
+            if min_b:
+                mp.setenv("AIOS_DECODE_GEMM_MIN_B", min_b)
+            eng = random_engine(cfg, "BF16", seed=3, max_ctx=256, max_batch=4)
+            for s, p in enumerate(prompts):
+                eng.prefill(s, p, 0, False)
+            eng.decode(list(range(B)), [7] * B, [len(p) for p in prompts])
+            assert eng.decode_gemm_min_batch == int(min_b or 3)
+            outs[min_b] = np.asarray(eng.last_logits(B)).reshape(B, -1)
+            del eng
+    assert np.linalg.norm(outs[None] - outs["5"]) < 8 * 2.0 ** -9 * np.linalg.norm(outs["5"])
+
+
 @pytest.mark.parametrize("recipe,rb,split", [("Q4_K_M", "0", "0"), ("Q4_K_M", "4", "1"),
                                              ("mistral_shape", "0", "1"), ("mistral_shape", "4", "0")])
 @pytest.mark.parametrize("wk,ring", [("1", "1"), ("0", "1"), ("0", "0")])
