@@ -278,7 +278,9 @@ __device__ __forceinline__ void attn_meet(const AttnDecodeArgs& a, int h0, int s
 // dealt wave by wave (tile t to wave t mod 8 P: 32 keys is also the granularity of the balance).
 //
 // Per tile, on the matrix cores:
-//   S^T[key][c] = K Q^T   (16x16x32, K rows from global memory to the A operand's registers as they are).  Column
+//   S^T[key][c] = K Q^T   (16x16x32; K comes in whole lines and takes the A operand's order through the wave's own LDS tile: asked
+//                         for in that order, 16 lanes at 16 keys, each lane is an address of its own to the address unit: 16000 fp8 keys
+//                         15.0 -> 13.4 us, 16 rows of 1000 bf16 ones 16.3 -> 15.0, 32 / 8 heads of 128).  Column
 //                         c holds head c mod GP (GP = 4 or 8 >= G): every head's scores, and with them its
 //                         probabilities in fp32, stand in 16 / GP columns.
 //   O^T[dim][c] += V^T P^T   Each of a head's columns multiplies another bf16 part of the same probability (p's
@@ -301,8 +303,10 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   constexpr int ES = F8 ? 1 : 2;            // bytes per cached element
   constexpr int EL = 16 / ES;               // elements per 16-B load
   constexpr int KL = HD / (4 * EL);         // K loads per lane and 16 keys
-  constexpr int VL = AT_TK * HD / EL / 64;  // V loads per lane and tile
-  constexpr int VPR = HD / EL;              // 16-B pieces of a V row
+  constexpr int VL = AT_TK * HD / EL / 64;  // K or V loads per lane and tile
+  constexpr int VPR = HD / EL;              // 16-B pieces of a row
+  constexpr int KROW = HD * ES + 16;        // LDS row of K as cached: 16 rows' reads of one piece on distinct banks
+  static_assert(KROW <= at_vrow<HD>());
   constexpr int DT = HD / 16;               // O^T tiles
   constexpr int VROW = at_vrow<HD>();
   constexpr int NW = AT_NW;
@@ -354,13 +358,12 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   stamp(1);
 
   struct Tile {
-    gu32x4 k[2][KL], v[VL];
+    gu32x4 k[VL], v[VL];
     size_t base;  // of the tile in its pool, bytes
     int bytes;    // of its live keys
   };
   Tile tA, tB;
-  // this lane's 16-B pieces: K of key (16 j + col): elements 4 EL i + EL q4 ..; V piece lane + 64 i, row-major
-  const uint32_t koff = (uint32_t)(col * HD + q4 * EL) * ES, voff = (uint32_t)lane * 16;
+  const uint32_t voff = (uint32_t)lane * 16;  // this lane's 16-B pieces: lane + 64 i, row-major
   const size_t hoff = (size_t)kvh * KV_BLOCK * HD * ES;
   // A tile is a buffer of its live keys' bytes: dead keys of the last tile, and all keys past it, read as zeros without
   // a memory access.  So every path issues the same loads, and the wait for one tile's leaves the next one's in
@@ -375,10 +378,7 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   auto issue_k = [&](Tile& t) __attribute__((always_inline)) {
     const auto r = uniform_rsrc((const uint8_t*)a.k_cache + t.base, t.bytes);
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < KL; ++i)
-        t.k[j][i] = __builtin_amdgcn_raw_buffer_load_b128(r, koff + (16 * j * HD + 4 * EL * i) * ES, 0, 2);
+    for (int i = 0; i < VL; ++i) t.k[i] = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 1024 * i, 0, 2);
   };
   auto issue_v = [&](Tile& t) __attribute__((always_inline)) {
     const auto r = uniform_rsrc((const uint8_t*)a.v_cache + t.base, t.bytes);
@@ -417,6 +417,17 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
   auto math = [&](Tile& t, int tile, auto after_s) __attribute__((always_inline)) {
     const bool part = (tile + 1) * AT_TK > len;  // the context's last, partly filled tile
     const int live = len - tile * AT_TK;
+    // ---- K through the wave's LDS tile: this lane's pieces of key 16 j + col are elements 4 EL i + EL q4 ..
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const int p = lane + 64 * i;
+      *(gu32x4*)(vt + p / VPR * KROW + p % VPR * 16) = t.k[i];
+    }
+    gu32x4 kw[2][KL];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < KL; ++i) kw[j][i] = *(const gu32x4*)(vt + (16 * j + col) * KROW + (4 * i + q4) * 16);
     // ---- S^T: keys 16 j + 4 q4 + e of column col
     gf32x4 st[2];
 #pragma unroll
@@ -425,8 +436,8 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         gu32x4 w;
-        if constexpr (F8) w = fp8x8_bf16x8(t.k[j][s >> 1][2 * (s & 1)], t.k[j][s >> 1][2 * (s & 1) + 1]);
-        else w = t.k[j][s];
+        if constexpr (F8) w = fp8x8_bf16x8(kw[j][s >> 1][2 * (s & 1)], kw[j][s >> 1][2 * (s & 1) + 1]);
+        else w = kw[j][s];
         st[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8, w), qf[s], st[j], 0, 0, 0);
       }
     }
@@ -501,7 +512,8 @@ __device__ __forceinline__ void attn_core(const AttnDecodeArgs& a, int sp, int k
       for (int r = 0; r < NR; ++r) o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[r], o[i], 0, 0, 0);
     }
   };
-  // a wave's registers hold one and a half tiles in flight: the next tile's V is requested when this one's K is used
+  // a wave's registers hold one and a half tiles in flight: the next tile's V is requested when this one's K is used (K of the tile after the next
+  // as soon as this one's lies in LDS: no faster, and at head_dim 64 the registers spill)
   for (int t = t0; t < ntile; t += 2 * step) {
     math(tA, t, [&]() __attribute__((always_inline)) { issue_v(tB); });
     if (t == t0) stamp(2);
