@@ -1001,11 +1001,12 @@ inline int pf4_groups(const GemmQArgs& a, int bm, int S) {
 }
 
 // ---- epilogue of the 8-wave bodies.  The weights are the matrix instruction's first operand, so a lane's four elements of an
-// accumulator are successive columns of one row.  A tile's outputs are then 16-byte (bf16: 8- and 16-byte) stores instead of a
-// store an element; and the residual of a batch of rows is requested before the batch in front of it is stored (a load behind
-// a store to what may be the same place waited for it, row by row).  With 256 x 256 tiles, us, one element at a time -> so:
-//   8192 x 1024 x 2048 rows: SwiGLU Q4_K 50 -> 40, bf16 out of bf16 48 -> 36, residual 73 -> 53 (Q4_K), fp32 43 -> 43 (67 MB);
-//   28672 x 4096 x 2048 rows SwiGLU Q4_K 482 -> 452; 128 x 256 tiles, 4096 x 4096 x 2048 rows, residual 90 -> 80
+// accumulator are successive columns of one row.  They go to memory in the rows' own order, 8 (SwiGLU 2, bf16 4) lanes to a row's piece, turned
+// through the wave's own LDS: a store of 16 lanes at 16 rows is 64 addresses to the address unit.  And the residual of a batch of rows is
+// requested before the batch in front of it is stored (a load behind a store to what may be the same place waited for it, row by row).
+// With 256 x 256 tiles, us, one element at a time -> 16 bytes a lane -> turned: 8192 x 1024 x 2048 rows: SwiGLU Q4_K 50 -> 43 -> 38,
+// bf16 out of bf16 48 -> 36 -> 34, residual 73 -> 53 -> 51 (Q4_K), fp32 43 -> 42 -> 39 (67 MB); 28672 x 4096 x 2048 rows SwiGLU Q4_K
+// 482 -> 452 one to 16 bytes, 480 -> 464 turned; 3900 tokens of Mistral 55.5 -> 55.3 ms, 711 of Qwen3 14.3 -> 14.2.
 // bf16 outputs: position p of a wave's 32 columns holds column pf8_col(p), so that the two accumulators of a row are eight
 // successive columns.
 // smem: a workgroup's LDS from its start; n0: the wave's first column
@@ -1013,29 +1014,44 @@ template <int EPI, int MT>
 __device__ __forceinline__ void pf8_finish(const GemmQArgs& a, const gf32x4 (&acc)[MT][2], uint8_t* smem, int m0, int n0, int wv, int S) {
   const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   if constexpr (EPI == GEPI_SWIGLU_BF16) {
-    const bool vec = a.ldc % 4 == 0 && ((uintptr_t)a.C16 & 7) == 0;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int m = m0 + 16 * i + r16;
+    auto glu = [&](int i) __attribute__((always_inline)) {
       const float o0 = glu_act(acc[i][0][0], a.act) * acc[i][0][1], o1 = glu_act(acc[i][0][2], a.act) * acc[i][0][3];
       const float o2 = glu_act(acc[i][1][0], a.act) * acc[i][1][1], o3 = glu_act(acc[i][1][2], a.act) * acc[i][1][3];
-      if (m >= a.M) continue;
-      bf16_t* p = a.C16 + (size_t)m * a.ldc + (n0 >> 1) + 4 * q;
-      const uint2 v = make_uint2(pk_bf16(o0, o1), pk_bf16(o2, o3));
-      if (vec) {
-        *(uint2*)p = v;
-      } else {
+      return make_uint2(pk_bf16(o0, o1), pk_bf16(o2, o3));
+    };
+    bf16_t* const out = a.C16 + (n0 >> 1);
+    if (a.ldc % 8 == 0 && ((uintptr_t)a.C16 & 15) == 0) {  // 32 rows of 16 outputs at a time
+      constexpr int PITCH = 48;
+      __syncthreads();
+      uint8_t* own = smem + wv * (32 * PITCH);
+#pragma unroll
+      for (int i = 0; i < MT; i += 2) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *(uint2*)(own + (16 * j + r16) * PITCH + 8 * q) = glu(i + j);
+        const gf32x4 v = *(const gf32x4*)(own + (lane >> 1) * PITCH + 16 * (lane & 1));
+        const int m = m0 + 16 * i + (lane >> 1);
+        if (m < a.M) *(gf32x4*)(out + (size_t)m * a.ldc + 8 * (lane & 1)) = v;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const int m = m0 + 16 * i + r16;
+        const uint2 v = glu(i);
+        if (m >= a.M) continue;
+        bf16_t* p = out + (size_t)m * a.ldc + 4 * q;
         p[0] = (bf16_t)v.x; p[1] = (bf16_t)(v.x >> 16); p[2] = (bf16_t)v.y; p[3] = (bf16_t)(v.y >> 16);
       }
     }
   } else if constexpr (EPI == GEPI_STORE16) {
     const bool vec = a.ldc % 8 == 0 && ((uintptr_t)a.C16 & 15) == 0;
+    constexpr int PITCH = 80;
+    if (vec) __syncthreads();
+    uint8_t* own = smem + wv * (16 * PITCH);
     float b[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) b[e] = a.bias16 ? a.bias16[n0 + 8 * q + e] : 0.f;
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      const int m = m0 + 16 * i + r16;
       float v[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = acc[i][e >> 2][e & 3] + b[e];
@@ -1043,12 +1059,14 @@ __device__ __forceinline__ void pf8_finish(const GemmQArgs& a, const gf32x4 (&ac
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = unary_act(v[e], a.unary - 1, a.act_n);
       }
-      if (m >= a.M) continue;
-      bf16_t* p = a.C16 + (size_t)m * a.ldc + n0 + 8 * q;
       const uint4 o = make_uint4(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]), pk_bf16(v[4], v[5]), pk_bf16(v[6], v[7]));
       if (vec) {
-        *(uint4*)p = o;
-      } else {
+        *(uint4*)(own + r16 * PITCH + 16 * q) = o;
+        const gf32x4 t = *(const gf32x4*)(own + (lane >> 2) * PITCH + 16 * (lane & 3));
+        const int m = m0 + 16 * i + (lane >> 2);
+        if (m < a.M) *(gf32x4*)(a.C16 + (size_t)m * a.ldc + n0 + 8 * (lane & 3)) = t;
+      } else if (m0 + 16 * i + r16 < a.M) {
+        bf16_t* p = a.C16 + (size_t)(m0 + 16 * i + r16) * a.ldc + n0 + 8 * q;
 #pragma unroll
         for (int e = 0; e < 8; ++e) p[e] = (bf16_t)((&o.x)[e >> 1] >> (16 * (e & 1)));
       }
@@ -1091,10 +1109,14 @@ __device__ __forceinline__ void pf8_finish(const GemmQArgs& a, const gf32x4 (&ac
       }
   } else {
     constexpr int NB = MT < 4 ? MT : 4;  // row tiles of a batch
+    constexpr int PITCH = 144;
+    __syncthreads();
+    uint8_t* own = smem + wv * (16 * PITCH);
+    const int r8 = lane >> 3, u = lane & 7;
     gf32x4 res[2][NB][2];
     auto at = [&](int i, int c, bool in) __attribute__((always_inline)) {
-      const int m = m0 + 16 * i + r16;
-      return (gf32x4*)(a.C + (size_t)(in ? m : min(m, a.M - 1)) * a.ldc + n0 + 16 * c + 4 * q);
+      const int m = m0 + 16 * i + 8 * c + r8;
+      return (gf32x4*)(a.C + (size_t)(in ? m : min(m, a.M - 1)) * a.ldc + n0 + 4 * u);
     };
     auto get = [&](int b) __attribute__((always_inline)) {
       if constexpr (EPI == GEPI_ACCUM) {
@@ -1110,11 +1132,14 @@ __device__ __forceinline__ void pf8_finish(const GemmQArgs& a, const gf32x4 (&ac
       if (b + 1 < MT / NB) get(b + 1);
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
-        if (m0 + 16 * (b * NB + i) + r16 >= a.M) continue;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) *(gf32x4*)(own + r16 * PITCH + 64 * c + 16 * q) = acc[b * NB + i][c];
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-          if constexpr (EPI == GEPI_ACCUM) *at(b * NB + i, c, true) = res[b & 1][i][c] + acc[b * NB + i][c];
-          else *at(b * NB + i, c, true) = acc[b * NB + i][c];
+          gf32x4 v = *(const gf32x4*)(own + (8 * c + r8) * PITCH + 16 * u);
+          if (m0 + 16 * (b * NB + i) + 8 * c + r8 >= a.M) continue;
+          if constexpr (EPI == GEPI_ACCUM) v = res[b & 1][i][c] + v;
+          *at(b * NB + i, c, true) = v;
         }
       }
     }
