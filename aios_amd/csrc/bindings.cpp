@@ -515,7 +515,6 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
         c.allgather_cols((float*)data, rows, slice, ld, S(st));
       }, py::arg("data"), py::arg("rows"), py::arg("slice"), py::arg("ld"), py::arg("stream") = 0)
       .def_property("two_shot_min", &XgmiComm::two_shot_min, &XgmiComm::set_two_shot_min)
-      .def_property("call_wg", &XgmiComm::call_wg, &XgmiComm::set_call_wg)
       .def_property("bf16_payload", &XgmiComm::bf16_payload, &XgmiComm::set_bf16_payload)
       .def("error", &XgmiComm::error)
       .def("reset_error", &XgmiComm::reset_error)
@@ -663,6 +662,7 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
     HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
     return n;
   }, py::arg("device") = 0);
+  m.def("ar_waiting_wg", &ar_waiting_wg, py::arg("ranks"), py::arg("cus"));
   m.def("device_pci_bus_id", [](int dev) {
     char buf[64] = {0};
     HIP_CHECK(hipDeviceGetPCIBusId(buf, (int)sizeof(buf), dev));

@@ -19,15 +19,15 @@
 //
 // Why not a ring: a ring pays 2(W-1) latency hops and is bound by one link.
 //
-// Protocol (per workgroup g; epoch e = this WG's call counter, identical on every rank because
+// Protocol (per chunk g; epoch e = the chunk's call counter, identical on every rank because
 // every rank issues the same sequence of collectives with the same sizes):
 //   1. copy my part of chunk g into my stage buffer half e & 1
 //   2. release fence (system scope), store e into flag[phase][g][my_rank] of every peer
 //   3. wait until my own flag[phase][g][p] >= e for every peer (bounded spin -> error flag)
 //   4. consume the peers' half e & 1 (two-shot: reduce, publish result, flag phase 2, wait, gather)
-// Buffer position j is always owned by workgroup j / AR_CHUNK in every kernel (each call moves
-// at most AR_MAX_WG * AR_CHUNK elements; larger messages are split into several calls), so the
-// per-workgroup epochs stay consistent across calls of different sizes and kinds.  Double
+// Buffer position j always belongs to chunk j / AR_CHUNK in every kernel, and a chunk to one workgroup of a call (each call
+// moves at most AR_MAX_WG * AR_CHUNK elements; larger messages are split into several calls; a workgroup takes its chunks
+// in ascending order), so the per-chunk epochs stay consistent across calls of different sizes, kinds and grids.  Double
 // buffering is safe: a rank reuses half e&1 at epoch e+2, which needs every peer's epoch-(e+1)
 // phase-1 flag, which a peer sets only after it finished all its reads of epoch e.
 // Flags / buffers are uncached device memory (hipDeviceMallocUncached), so remote stores and
@@ -44,9 +44,9 @@
 namespace aios {
 
 constexpr int AR_MAX_RANKS = 8;
-constexpr int AR_MAX_WG = 512;
+constexpr int AR_MAX_WG = 512;                        // chunks of a call, and its workgroups at most
 constexpr int AR_THREADS = 256;
-constexpr int AR_CHUNK = AR_THREADS * 4;              // elements per workgroup per call
+constexpr int AR_CHUNK = AR_THREADS * 4;              // elements of a chunk
 constexpr size_t AR_MAX_CALL = (size_t)AR_MAX_WG * AR_CHUNK;  // elements per kernel call
 // C1 / C2 fused into the batch-1 row GEMV epilogue (EPI_TP_RESID, gemv_q8.h): per GEMV
 // workgroup ("slot") a private double-buffered stage of up to TPF_CAP partial outputs behind the
@@ -57,7 +57,7 @@ constexpr int TPF_CAP = 1024;
 struct ArDevCtx {
   float* buf[AR_MAX_RANKS];         // rank r's shared region: stage f32 [2][cap] | result f32 [2][cap] | stage bf16 [2][cap]
   uint32_t* flags[AR_MAX_RANKS];    // rank r's flags: [2 phases][AR_MAX_WG][AR_MAX_RANKS]
-  uint32_t* epoch;                  // my per-WG epoch counters [AR_MAX_WG] (local)
+  uint32_t* epoch;                  // my per-chunk epoch counters [AR_MAX_WG] (local)
   uint32_t* error;                  // set to 1 when a wait timed out (device view of pinned host memory)
   int rank, world;
   size_t cap;                       // elements per half-buffer (<= AR_MAX_CALL)
@@ -96,12 +96,6 @@ class XgmiComm {
   int world() const { return h_.world; }
   size_t capacity() const { return h_.cap; }
   size_t two_shot_min() const { return two_shot_min_; }
-  // workgroups per collective launch (elements per call = wg * AR_CHUNK, larger messages split):
-  // AR_MAX_WG by default; ranks that SHARE one GPU (the single-GPU test setting) must fit all their
-  // spinning workgroups on it at once, so tp.create_comm lowers it to 1024 / ranks-per-GPU.  Every
-  // rank must use the same value (the per-workgroup epochs follow the call sequence).
-  int call_wg() const { return (int)(call_cap_ / AR_CHUNK); }
-  void set_call_wg(int wg);
   void set_two_shot_min(size_t n) { two_shot_min_ = n; }
   // the fused O / down epilogue (EPI_TP_RESID): device context for GemvArgs::tp (null when off:
   // world 1 or AIOS_TP_FUSE=0) and the engine-workgroup cap that lets every rank's grid be resident
@@ -114,6 +108,7 @@ class XgmiComm {
   void disable_fuse() { fuse_on_ = false; }
   bool uncached() const { return uncached_; }
   int fuse_grid() const { return fuse_grid_; }
+  // n ranks share this rank's GPU (1: none does): bounds fuse_grid and the collectives' workgroups (ar_waiting_wg)
   void set_ranks_per_gpu(int n);
   bool bf16_payload() const { return bf16_; }
   void set_bf16_payload(bool on) { bf16_ = on; }
@@ -136,13 +131,17 @@ class XgmiComm {
   int device_ = 0;
   bool connected_ = false;
   size_t two_shot_min_ = 64 * 1024;  // floats (256 KB)
-  size_t call_cap_ = AR_MAX_CALL;    // elements per launch (see set_call_wg)
+  int max_wg_ = AR_MAX_WG;           // workgroups per collective launch
   bool bf16_ = true;                 // bf16 staging for the two-shot (prefill) path
   bool fuse_on_ = true;              // AIOS_TP_FUSE (default 1)
   bool uncached_ = false;            // shared regions got uncached memory (required by the fused path)
   int fuse_grid_ = 0;
 };
 
-void launch_allreduce(const ArDevCtx* ctx, int world, float* data, size_t n, float* residual, hipStream_t st);
+// Workgroups that a collective launch has at most where `ranks` ranks share a GPU of `cus` CUs: all of them together stand on half of the
+// CUs.  They wait there for a rank whose own collective comes behind kernels that need a CU to themselves (prefill attention and the
+// 256-row prefill tiles hold 480 to 512 of a SIMD's 512 registers, decode attention 464): on every CU, as with two workgroups a
+// CU before, those kernels found none to run on and the wait ran out.
+int ar_waiting_wg(int ranks, int cus);
 
 }  // namespace aios

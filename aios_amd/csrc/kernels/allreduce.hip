@@ -28,10 +28,10 @@ __device__ __forceinline__ uint32_t flag_idx(int phase, int g, int r) {
   return ((uint32_t)phase * AR_MAX_WG + g) * AR_MAX_RANKS + r;
 }
 
-// this WG's epoch (one increment per call), broadcast through LDS
+// chunk g's epoch (one increment per call), broadcast through LDS
 __device__ __forceinline__ uint32_t next_epoch(const ArDevCtx* c, int g, uint32_t* s_e) {
   if (threadIdx.x == 0) {
-    const uint32_t e = c->epoch[g] + 1;  // only this WG touches epoch[g]
+    const uint32_t e = c->epoch[g] + 1;  // only the chunk's workgroup touches epoch[g]
     c->epoch[g] = e;
     *s_e = e;
   }
@@ -48,16 +48,18 @@ __device__ __forceinline__ void publish(const ArDevCtx* c, int phase, int g, uin
     __hip_atomic_store(c->flags[t] + flag_idx(phase, g, c->rank), e, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// wait for every peer's epoch-e flag of `phase` (bounded: an exit every wave reaches)
-__device__ __forceinline__ void wait_peers(const ArDevCtx* c, int phase, int g, uint32_t e) {
+// wait for every peer's epoch-e flag of `phase` (bounded: an exit every wave reaches).  late: this thread's peer has missed a wait of this
+// launch, whose result is lost; it is not waited for again, so a launch of many chunks ends after one bound as one of a single chunk does
+__device__ __forceinline__ void wait_peers(const ArDevCtx* c, int phase, int g, uint32_t e, bool& late) {
   const int t = threadIdx.x;
-  if (t < c->world && t != c->rank) {
+  if (t < c->world && t != c->rank && !late) {
     uint32_t* f = c->flags[c->rank] + flag_idx(phase, g, t);
     const uint64_t t0 = wall_clock64();
     while ((int)(__hip_atomic_load(f, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM) - e) < 0) {
       __builtin_amdgcn_s_sleep(2);
       if (wall_clock64() - t0 > AR_TIMEOUT_TICKS) {
         __hip_atomic_store(c->error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        late = true;
         break;
       }
     }
@@ -80,7 +82,7 @@ __device__ __forceinline__ void put(float* data, float* residual, size_t i, floa
 // this thread's 4 new residual values at column j * RNORM_COLS + 4 t.  The block's sum of squares is
 // reduced in a fixed order, so every TP rank (same residual bits) writes the same parts.  Every
 // thread of the workgroup calls it.
-static_assert(AR_CHUNK == RNORM_COLS, "one all-reduce workgroup = one norm column block");
+static_assert(AR_CHUNK == RNORM_COLS, "one all-reduce chunk = one norm column block");
 __device__ __forceinline__ void norm_block(const ResidNorm& nm, int m, int j, int ncb, int t, float4 r) {
   __shared__ float s_red[AR_THREADS / 64];
   const int col = j * RNORM_COLS + 4 * t;
@@ -120,13 +122,12 @@ __global__ __launch_bounds__(AR_THREADS) void add_norm_kernel(float* __restrict_
 // in rank order on every rank (own partial at its rank's position), so all ranks produce the
 // bit-identical result and their on-device samplers stay in lock step.  NORM (C1 / C2 of the
 // batched TP decode): residual required, n = rows * d with d % RNORM_COLS == 0, and the workgroup
-// also writes the split-RMSNorm outputs of its column block (no separate RMSNorm launch).
+// also writes the split-RMSNorm outputs of its chunk's column block (no separate RMSNorm launch).
 template <bool NORM>
-__global__ __launch_bounds__(AR_THREADS) void allreduce_oneshot(const ArDevCtx* __restrict__ c, float* __restrict__ data,
-                                                                 size_t n, float* __restrict__ residual, int d,
-                                                                 ResidNorm nm) {
+__device__ __forceinline__ void oneshot_chunk(const ArDevCtx* __restrict__ c, int g, float* __restrict__ data, size_t n,
+                                              float* __restrict__ residual, int d, const ResidNorm& nm, bool& late) {
   __shared__ uint32_t s_e;
-  const int g = blockIdx.x, t = threadIdx.x;
+  const int t = threadIdx.x;
   const int rank = c->rank, world = c->world;
   const uint32_t e = next_epoch(c, g, &s_e);
   const size_t half = (size_t)(e & 1u) * c->cap;
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_oneshot(const ArDevCtx* 
   if (full) *(float4*)(mine + i) = *(const float4*)(data + i);
   else for (size_t k = i; k < n; ++k) mine[k] = data[k];
   publish(c, 0, g, e);
-  wait_peers(c, 0, g, e);
+  wait_peers(c, 0, g, e, late);
   if (full) {
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_oneshot(const ArDevCtx* 
       float4 r = *(const float4*)(residual + i);
       r.x += acc.x; r.y += acc.y; r.z += acc.z; r.w += acc.w;
       *(float4*)(residual + i) = r;
-      const size_t e0 = (size_t)g * AR_CHUNK;  // the workgroup's first element: one row, one column block
+      const size_t e0 = (size_t)g * AR_CHUNK;  // the chunk's first element: one row, one column block
       norm_block(nm, (int)(e0 / d), (int)(e0 % d) / RNORM_COLS, d / RNORM_COLS, t, r);
       return;
     }
@@ -164,15 +165,24 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_oneshot(const ArDevCtx* 
   }
 }
 
+// a workgroup takes chunks blockIdx.x, + gridDim.x, .. of the call in turn, here and below (one each unless ranks share a GPU: ar_waiting_wg)
+template <bool NORM>
+__global__ __launch_bounds__(AR_THREADS) void allreduce_oneshot(const ArDevCtx* __restrict__ c, float* __restrict__ data,
+                                                                 size_t n, float* __restrict__ residual, int d,
+                                                                 ResidNorm nm) {
+  bool late = false;
+  for (int g = blockIdx.x; (size_t)g * AR_CHUNK < n; g += gridDim.x) oneshot_chunk<NORM>(c, g, data, n, residual, d, nm, late);
+}
+
 // ---- two-shot: reduce-scatter (each rank sums its 1/world sub-shard of the chunk, pulling the
 // peers' staged partials -- bf16 when BF16, halving the link bytes) then all-gather of the reduced
 // sub-shards.  Each element is reduced once, by its owner, so every rank gets identical bits.
 // The host launches it only for n % 4 == 0.
 template <bool BF16>
-__global__ __launch_bounds__(AR_THREADS) void allreduce_twoshot(const ArDevCtx* __restrict__ c, float* __restrict__ data,
-                                                                 size_t n, float* __restrict__ residual) {
+__device__ __forceinline__ void twoshot_chunk(const ArDevCtx* __restrict__ c, int g, float* __restrict__ data, size_t n,
+                                              float* __restrict__ residual, bool& late) {
   __shared__ uint32_t s_e;
-  const int g = blockIdx.x, t = threadIdx.x;
+  const int t = threadIdx.x;
   const int rank = c->rank, world = c->world;
   const uint32_t e = next_epoch(c, g, &s_e);
   const size_t half = (size_t)(e & 1u) * c->cap;
@@ -192,7 +202,7 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_twoshot(const ArDevCtx* 
     }
   }
   publish(c, 0, g, e);
-  wait_peers(c, 0, g, e);
+  wait_peers(c, 0, g, e, late);
   // 2. reduce-scatter: float4 groups [lo, hi) of the chunk belong to this rank
   const int nq = AR_CHUNK / 4;
   const int lo = rank * nq / world, hi = (rank + 1) * nq / world;
@@ -219,7 +229,7 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_twoshot(const ArDevCtx* 
     put(data, residual, i, acc);
   }
   publish(c, 1, g, e);
-  wait_peers(c, 1, g, e);
+  wait_peers(c, 1, g, e, late);
   // 3. all-gather the other ranks' reduced sub-shards
   for (int p = 0; p < world; ++p) {
     if (p == rank) continue;
@@ -231,13 +241,18 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_twoshot(const ArDevCtx* 
     }
   }
 }
+template <bool BF16>
+__global__ __launch_bounds__(AR_THREADS) void allreduce_twoshot(const ArDevCtx* __restrict__ c, float* __restrict__ data,
+                                                                 size_t n, float* __restrict__ residual) {
+  bool late = false;
+  for (int g = blockIdx.x; (size_t)g * AR_CHUNK < n; g += gridDim.x) twoshot_chunk<BF16>(c, g, data, n, residual, late);
+}
 
 // ---- column all-gather: position j = r*rows*slice + b*slice + col is owned by rank r
-__global__ __launch_bounds__(AR_THREADS) void allgather_cols_kernel(const ArDevCtx* __restrict__ c,
-                                                                    float* __restrict__ data, int rows, int slice,
-                                                                    int ld) {
+__device__ __forceinline__ void allgather_chunk(const ArDevCtx* __restrict__ c, int g, float* __restrict__ data, int rows, int slice, int ld,
+                                                bool& late) {
   __shared__ uint32_t s_e;
-  const int g = blockIdx.x, t = threadIdx.x;
+  const int t = threadIdx.x;
   const int rank = c->rank;
   const uint32_t e = next_epoch(c, g, &s_e);
   const size_t half = (size_t)(e & 1u) * c->cap;
@@ -252,7 +267,7 @@ __global__ __launch_bounds__(AR_THREADS) void allgather_cols_kernel(const ArDevC
     }
   }
   publish(c, 0, g, e);
-  wait_peers(c, 0, g, e);
+  wait_peers(c, 0, g, e, late);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const size_t j = (size_t)g * AR_CHUNK + k * AR_THREADS + t;
@@ -262,6 +277,13 @@ __global__ __launch_bounds__(AR_THREADS) void allgather_cols_kernel(const ArDevC
       data[(w / slice) * (size_t)ld + (size_t)r * slice + w % slice] = __builtin_nontemporal_load(c->buf[r] + half + j);
     }
   }
+}
+__global__ __launch_bounds__(AR_THREADS) void allgather_cols_kernel(const ArDevCtx* __restrict__ c,
+                                                                    float* __restrict__ data, int rows, int slice,
+                                                                    int ld) {
+  bool late = false;
+  const size_t total = (size_t)rows * slice * c->world;
+  for (int g = blockIdx.x; (size_t)g * AR_CHUNK < total; g += gridDim.x) allgather_chunk(c, g, data, rows, slice, ld, late);
 }
 
 void* alloc_shared(size_t bytes, bool* uncached = nullptr) {
@@ -277,17 +299,11 @@ void* alloc_shared(size_t bytes, bool* uncached = nullptr) {
   return p;
 }
 
-int grid_for(size_t n) { return (int)std::max<size_t>(1, (n + AR_CHUNK - 1) / AR_CHUNK); }
+int grid_for(size_t n, int max_wg) { return (int)std::min<size_t>(max_wg, std::max<size_t>(1, (n + AR_CHUNK - 1) / AR_CHUNK)); }
 
 }  // namespace
 
-void launch_allreduce(const ArDevCtx* ctx, int world, float* data, size_t n, float* residual, hipStream_t st) {
-  (void)world;
-  if (n == 0) return;
-  if (n > AR_MAX_CALL) throw std::runtime_error("launch_allreduce: call above AR_MAX_CALL elements");
-  hipLaunchKernelGGL((allreduce_oneshot<false>), dim3(grid_for(n)), dim3(AR_THREADS), 0, st, ctx, data, n, residual, 0,
-                     ResidNorm{});
-}
+int ar_waiting_wg(int ranks, int cus) { return ranks > 1 ? std::min(AR_MAX_WG, std::max(1, cus / (2 * ranks))) : AR_MAX_WG; }
 
 void launch_add_norm(float* residual, const float* data, int rows, int d, const ResidNorm& nm, hipStream_t st) {
   if (rows <= 0) return;
@@ -384,10 +400,7 @@ void XgmiComm::connect(const std::vector<std::string>& handles) {
 
 void XgmiComm::set_ranks_per_gpu(int n) {
   fuse_grid_ = n > 1 ? std::max(1, device_cu_count() / n) : 0;
-}
-
-void XgmiComm::set_call_wg(int wg) {
-  call_cap_ = (size_t)std::max(1, std::min(AR_MAX_WG, wg)) * AR_CHUNK;
+  max_wg_ = ar_waiting_wg(n, device_cu_count());
 }
 
 void XgmiComm::allreduce(float* data, size_t n, float* residual, hipStream_t st) {
@@ -396,17 +409,16 @@ void XgmiComm::allreduce(float* data, size_t n, float* residual, hipStream_t st)
     if (residual) launch_add(residual, data, n, st);
     return;
   }
-  for (size_t off = 0; off < n; off += call_cap_) {
-    const size_t m = std::min(call_cap_, n - off);
+  for (size_t off = 0; off < n; off += h_.cap) {
+    const size_t m = std::min(h_.cap, n - off);
     float* d = data + off;
     float* r = residual ? residual + off : nullptr;
+    const dim3 grid(grid_for(m, max_wg_)), block(AR_THREADS);
     if (m >= two_shot_min_ && m % 4 == 0) {
-      if (bf16_)
-        hipLaunchKernelGGL((allreduce_twoshot<true>), dim3(grid_for(m)), dim3(AR_THREADS), 0, st, d_, d, m, r);
-      else
-        hipLaunchKernelGGL((allreduce_twoshot<false>), dim3(grid_for(m)), dim3(AR_THREADS), 0, st, d_, d, m, r);
+      if (bf16_) hipLaunchKernelGGL((allreduce_twoshot<true>), grid, block, 0, st, d_, d, m, r);
+      else hipLaunchKernelGGL((allreduce_twoshot<false>), grid, block, 0, st, d_, d, m, r);
     } else {
-      launch_allreduce(d_, h_.world, d, m, r, st);
+      hipLaunchKernelGGL((allreduce_oneshot<false>), grid, block, 0, st, d_, d, m, r, 0, ResidNorm{});
     }
   }
 }
@@ -416,11 +428,11 @@ void XgmiComm::allreduce_norm(float* data, int rows, int d, float* residual, con
   const size_t n = (size_t)rows * d;
   if (h_.world == 1) {
     launch_add_norm(residual, data, rows, d, nm, st);
-  } else if (d % RNORM_COLS == 0 && n <= call_cap_ && n < two_shot_min_) {
+  } else if (d % RNORM_COLS == 0 && n <= h_.cap && n < two_shot_min_) {
     if (nm.parts < d / RNORM_COLS || nm.parts > 64 || nm.parts % 4)
       throw std::runtime_error("XgmiComm::allreduce_norm: parts must be resid_norm_parts(d)");
-    hipLaunchKernelGGL((allreduce_oneshot<true>), dim3(grid_for(n)), dim3(AR_THREADS), 0, st, d_, data, n, residual, d,
-                       nm);
+    hipLaunchKernelGGL((allreduce_oneshot<true>), dim3(grid_for(n, max_wg_)), dim3(AR_THREADS), 0, st, d_, data, n, residual,
+                       d, nm);
   } else {
     allreduce(data, n, residual, st);
     launch_add_norm(residual, nullptr, rows, d, nm, st);
@@ -430,12 +442,12 @@ void XgmiComm::allreduce_norm(float* data, int rows, int d, float* residual, con
 void XgmiComm::allgather_cols(float* data, int rows, int slice, int ld, hipStream_t st) {
   if (!connected_) throw std::runtime_error("XgmiComm: allgather before connect()");
   if (h_.world == 1 || rows <= 0) return;
-  if ((size_t)h_.world * slice > call_cap_) throw std::runtime_error("XgmiComm: all-gather slice above capacity");
-  const int rows_per = (int)std::max<size_t>(1, call_cap_ / ((size_t)h_.world * slice));
+  if ((size_t)h_.world * slice > h_.cap) throw std::runtime_error("XgmiComm: all-gather slice above capacity");
+  const int rows_per = (int)std::max<size_t>(1, h_.cap / ((size_t)h_.world * slice));
   for (int r0 = 0; r0 < rows; r0 += rows_per) {
     const int nr = std::min(rows_per, rows - r0);
     const size_t total = (size_t)h_.world * nr * slice;
-    hipLaunchKernelGGL(allgather_cols_kernel, dim3(grid_for(total)), dim3(AR_THREADS), 0, st, d_,
+    hipLaunchKernelGGL(allgather_cols_kernel, dim3(grid_for(total, max_wg_)), dim3(AR_THREADS), 0, st, d_,
                        data + (size_t)r0 * ld, nr, slice, ld);
   }
 }

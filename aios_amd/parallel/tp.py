@@ -264,9 +264,7 @@ def create_comm(rank: int, world: int, device: int, cap_floats: int, group=None,
         dist.all_gather_object(ids, device_identity(device), group=group)
     per_gpu = ranks_per_gpu(world, ids)
     comm = m.XgmiComm(rank, world, device, cap_floats)
-    if per_gpu > 1:  # every spinning workgroup of every rank must be resident on the shared GPU at once
-        comm.call_wg = max(1, min(512, 1024 // per_gpu))
-        # ... including the O / down GEMV engines whose epilogue runs the all-reduce (EPI_TP_RESID)
+    if per_gpu > 1:  # the workgroups that wait for a peer leave CUs to what the peer has yet to run
         comm.set_ranks_per_gpu(per_gpu)
     if world == 1:
         return comm

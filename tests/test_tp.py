@@ -189,6 +189,19 @@ def test_engine_config_vocab_parallel_rules():
     assert native.engine_config(tied, tp_size=2).vocab_parallel == 0
 
 
+def test_collectives_of_ranks_that_share_a_gpu_leave_half_of_its_cus():
+    """what waits for a peer must not stand on every CU: the peer's kernels may need one to themselves before its own collective"""
+    from aios_amd.runtime import native
+
+    E = native.load(build_if_missing=False)
+    if E is None:
+        pytest.skip("native engine not built")
+    assert E.ar_waiting_wg(1, 256) == 512
+    for ranks in range(2, 9):
+        for cus in (304, 256, 120, 16):
+            assert 1 <= E.ar_waiting_wg(ranks, cus) <= max(1, cus // 2 // ranks)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("world,gemm_prefill,prompt_len", [(2, 0, 21), (4, 0, 21), (8, 0, 21), (2, 1, 21),
                                                           (2, 1, 640), (2, 1, 9)])
