@@ -296,9 +296,13 @@ def create_comm(rank: int, world: int, device: int, cap_floats: int, group=None,
 
 
 def xgmi_handshake(comm, rank: int, world: int, device: int, allgather):
-    """The runtime daemon's TP setup (launch_tp / worker.py, over the setup channel): fused-epilogue
-    eligibility on every rank, the collectives' self-test (a failure is an error here: the daemon
-    reports the tier as failed and routes to the next one), then the fused-epilogue self-test."""
+    """The runtime daemon's TP setup (launch_tp / worker.py, over the setup channel): the ranks of each
+    GPU, fused-epilogue eligibility on every rank, the collectives' self-test (a failure is an error
+    here: the daemon reports the tier as failed and routes to the next one), then the fused-epilogue
+    self-test."""
+    per_gpu = ranks_per_gpu(world, allgather(device_identity(device)))
+    if per_gpu > 1:
+        comm.set_ranks_per_gpu(per_gpu)
     flags = allgather([bool(comm.fuse_eligible), bool(comm.uncached)])
     if not all(f[0] and f[1] for f in flags):
         comm.disable_fuse()

@@ -202,6 +202,26 @@ def test_collectives_of_ranks_that_share_a_gpu_leave_half_of_its_cus():
             assert 1 <= E.ar_waiting_wg(ranks, cus) <= max(1, cus // 2 // ranks)
 
 
+@pytest.mark.parametrize("ids,want", [(["n/0", "n/0"], 2), (["n/0", "n/1"], None), (["n/0", "n/1", "n/0", "n/1"], 2)])
+def test_daemon_ranks_that_share_a_gpu_say_so_to_their_comm(monkeypatch, ids, want):
+    """the daemon's setup bounds what waits for a peer as create_comm does (before any collective runs)"""
+    import aios_amd.parallel.tp as tp
+
+    calls = []
+
+    class Comm:
+        fuse_eligible = uncached = True
+
+        def __getattr__(self, name):
+            return lambda *a: calls.append((name, *a))
+
+    monkeypatch.setattr(tp, "device_identity", lambda d: ids[d])
+    monkeypatch.setattr(tp, "comm_self_test", lambda *a: calls.append(("self_test",)) or True)
+    monkeypatch.setattr(tp, "check_fused_comm", lambda *a: None)
+    tp.xgmi_handshake(Comm(), 0, len(ids), 0, lambda obj: list(ids) if isinstance(obj, str) else [obj] * len(ids))
+    assert calls == ([("set_ranks_per_gpu", want)] if want else []) + [("self_test",)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("world,gemm_prefill,prompt_len", [(2, 0, 21), (4, 0, 21), (8, 0, 21), (2, 1, 21),
                                                           (2, 1, 640), (2, 1, 9)])
