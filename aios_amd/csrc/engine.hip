@@ -1364,7 +1364,6 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
       at.scale = 1.f / std::sqrt((float)hd);
       at.out = gm_attn16_; at.ldo = qd;
       at.ws = gm_attn_ws_; at.ws_bytes = gm_attn_ws_bytes_;
-      at.one_group = cfg_.tp_size > 1;
       launch_attn_prefill(at, stream_);
       // O projection (+ residual)
       std::memset(&g, 0, sizeof(g));

@@ -428,7 +428,7 @@ static int prefill_runs(const AttnPrefillArgs& a, int BQ, int KG) {
 // 32 / 4 heads of 64, 500 tokens 11.3 / 10.6, 1000 19.2 / 16.3, 2000 36.2 / 33.9.
 static int prefill_groups(const AttnPrefillArgs& a, int BQ) {
   const int wg = (a.T + BQ - 1) / BQ * a.n_kv_heads, ntiles = (a.start + a.T - 1) / FP_KT + 1;
-  return !a.one_group && ntiles >= 10 && wg <= 2 * device_cu_count() ? 2 : 1;
+  return ntiles >= 10 && wg <= 2 * device_cu_count() ? 2 : 1;
 }
 
 // FP_WG workgroups of 128 rows each, O and (max, sum) in fp32

@@ -139,9 +139,6 @@ struct AttnPrefillArgs {
   float kv_scale_k = 1.f, kv_scale_v = 1.f;
   float* ws = nullptr;     // workspace of launches split over the keys; null: none is split
   size_t ws_bytes = 0;
-  // one group of waves a workgroup whatever its keys: tensor-parallel ranks.  Two groups take a CU's whole register file, so ranks that share a GPU
-  // waited for each other: one's all-reduce stands on every CU until the other's attention has run
-  int one_group = 0;
   int ns = 1;              // runs over the keys (the launcher's choice)
   int lm = 0, hx = 1;      // 2^lm XCDs share the work of hx KV heads (the launcher's)
 };
