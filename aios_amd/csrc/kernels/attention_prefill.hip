@@ -160,13 +160,16 @@ __global__ void __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2
   const int nt_last = kt1 - 1;
   static_assert(PIECES % NT == 0, "a thread's pieces of a tile");
   auto load = [&](Regs& r, int kt0_) {  // tiles kt0_ .. + KG - 1
+    size_t tbase[KG];  // (once a tile: once a piece was a scalar load and a wait for each)
+    static_for<KG>([&](auto I) {
+      constexpr int t = decltype(I)::value;
+      const int kt = min(kt0_ + t, nt_last);  // (clamped: the pipeline's tail requests are re-reads, never unmapped blocks)
+      tbase[t] = (size_t)kv_block(a.block_table, maxb, a.slot, kt * FP_KT) * blk_stride + (size_t)(kt & 1) * FP_KT * HD;
+    });
     static_for<PPT>([&](auto I) {
       constexpr int i = decltype(I)::value, t = i / (PIECES / NT);
-      const int kt = min(kt0_ + t, nt_last);  // (clamped: the pipeline's tail requests are re-reads, never unmapped blocks)
-      const size_t tbase = (size_t)kv_block(a.block_table, maxb, a.slot, kt * FP_KT) * blk_stride +
-                           (size_t)(kt & 1) * FP_KT * HD;
       const int idx = tid + NT * (i % (PIECES / NT)), key = idx / (HD / 8), c = idx % (HD / 8);
-      const size_t off = (tbase + (size_t)key * HD + c * 8) * ES;
+      const size_t off = (tbase[t] + (size_t)key * HD + c * 8) * ES;
       r.k[i] = *(const PT*)(kc + off);
       r.v[i] = *(const PT*)(vc + off);
     });
@@ -194,11 +197,12 @@ __global__ void __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2
       }
     });
   };
-  // one 64-key tile of math on LDS buffer buf
-  auto math = [&](const bf16_t* buf0, int kt_) {
+  // one 64-key tile of math on LDS buffer buf.  ALL: every wave of the workgroup sees keys of the tile, as it does of those up to the first row
+  auto math = [&](const bf16_t* buf0, int kt_, auto ALL) {
     const bf16_t* buf = buf0 + kg * TILE_ELEMS;
     const int kt = kt_ + kg;
-    if ((KG > 1 && kt >= kt1) || kt * FP_KT > khi_w) return;  // (uniform over the wave)
+    if constexpr (!decltype(ALL)::value)
+      if ((KG > 1 && kt >= kt1) || kt * FP_KT > khi_w) return;  // (uniform over the wave)
     const bf16_t* sK = buf;
     const bf16_t* sV = buf + FP_KT * KROW;
     // ---- S^T = K Q^T for the tile's two 32-key halves
@@ -280,13 +284,15 @@ __global__ void __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2
     }
   };
 
-  // Pipeline (round 5; was: one register buffer, stage + two barriers per tile, 130-150 us per
+  // Pipeline (with one register buffer, stage and two barriers per tile: 130-150 us per
   // 2k-token layer): two register buffers A / B and two LDS tile buffers L0 / L1, ONE barrier per
   // tile.  Iteration kt computes tile kt from L[kt & 1] while tile kt + 2 is requested into the
   // register buffer just staged, then stages tile kt + 1 into the other LDS buffer (last read two
-  // iterations ago, before the previous barrier) and barriers.  (An odd count's last tile ends the loop: a fully masked one
-  // behind it was 1.5 us of a short prompt's launch: us, with it -> so, 23 tokens, 32 / 4 heads of 64 5.8 -> 4.6, 130 tokens, 32 / 8 of 128
-  // 9.8 -> 8.5, 711 22.7 -> 20.6)
+  // iterations ago, before the previous barrier) and barriers.  Pairs without a branch, so that a tile's staging is dealt out over the one
+  // before; an odd one behind them by itself (a fully masked tile to make a pair of it was 1.5 us of a short prompt's launch).
+  // us, pairs with that tile / an exit behind every tile / so: 32 / 4 heads of 64, 23 tokens 6.0 / 4.9 / 4.8, 32 / 8 of 128, 130 tokens 10.1 / 9.2 / 9.1,
+  // 711 (two key groups below) 23.7 / 22.8 / 21.5, 3000 102 / 102 / 95, 16 / 8 of 128, 4096 tokens 100 / 109 / 99, 3840 behind 500 111 / 119 / 110,
+  // fp8, 16 / 16 of 128, 2304 behind 2000 104 / 116 / 103.  (Half of what the exits lost was the block table, looked up for every piece.)
   bf16_t* L0 = fp_smem;
   bf16_t* L1 = fp_smem + KG * TILE_ELEMS;
   Regs A, B;
@@ -294,17 +300,22 @@ __global__ void __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2
   load(B, kt0 + KG);
   stage(A, L0);
   __syncthreads();
-  for (int kt = kt0;; kt += 2 * KG) {  // (the exits are uniform)
+  int kt = kt0;
+  for (; kt + 2 * KG <= kt1; kt += 2 * KG) {
     load(A, kt + 2 * KG);
-    math(L0, kt);
-    if (kt + KG >= kt1) break;
+    math(L0, kt, std::true_type{});
     stage(B, L1);
     __syncthreads();
     load(B, kt + 3 * KG);
-    math(L1, kt + KG);
-    if (kt + 2 * KG >= kt1) break;
+    math(L1, kt + KG, std::true_type{});
     stage(A, L0);
     __syncthreads();
+  }
+  if (kt < kt1) math(L0, kt, std::false_type{});
+  if (KG > 1 && kt + KG < kt1) {
+    stage(B, L1);
+    __syncthreads();
+    math(L1, kt + KG, std::false_type{});
   }
   if constexpr (KG > 1) {  // ---- the second group's sums to the first
     static_assert(KG == 2, "two key groups");
