@@ -832,6 +832,16 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       py::arg("v_scale") = 1.f, py::arg("ws") = 0, py::arg("ws_bytes") = 0);
   m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
   m.def("attn_prefill_supports", &attn_prefill_supports);
+  // (key groups of a workgroup, runs over the keys) of a launch that has a workspace (host only)
+  m.def("attn_prefill_form", [](int H, int Hkv, int hd, int start, int T) {
+    AttnPrefillArgs a;
+    float ws = 0;
+    a.ws = &ws; a.ws_bytes = attn_prefill_ws_bytes(hd);
+    a.start = start; a.T = T; a.n_heads = H; a.n_kv_heads = Hkv; a.head_dim = hd;
+    std::pair<int, int> r;
+    attn_prefill_form(a, &r.first, &r.second);
+    return r;
+  }, py::arg("H"), py::arg("Hkv"), py::arg("hd"), py::arg("start"), py::arg("T"));
 
   // ------------------------------------------------------------------ layered decoders' row operations
   auto next_args = [](int kind, uintptr_t g, uintptr_t out, int ldo) {

@@ -432,14 +432,29 @@ static int prefill_runs(const AttnPrefillArgs& a, int BQ, int KG) {
   return ns > 1 && a.ws && need <= a.ws_bytes ? ns : 1;
 }
 
-// Key groups of a launch: two where its workgroups are two rounds of the CUs at most, so that a second workgroup for every CU is not there
-// all the time, and the longest has ten tiles, which pay for the meeting.  us in one / two groups: 32 / 8 heads of 128, 130 tokens 8.7 / 10.9,
-// 500 17.5 / 17.3, 711 22.4 / 21.6, 1024 29.8 / 26.7, 1500 43.0 / 37.3, 2048 56.8 / 55.6, 3000 91 / 111; 1000 behind 2000 71.5 / 59.8, fp8
-// behind 3000 94.7 / 77.9; fp8 in runs, behind 6000: 16 tokens 23.9 / 24.1, 100 35.6 / 29.6, 300 56.5 / 53.1 (three runs instead of six);
-// 32 / 4 heads of 64, 500 tokens 11.3 / 10.6, 1000 19.2 / 16.3, 2000 36.2 / 33.9.
+// Key groups of a launch with ten tiles or more.  A CU holds one workgroup of two groups or two of one, so two groups win where no CU has a second
+// workgroup, or a second one that is much shorter than the first, and lose where it is as long: then it is two rounds in a row.
+// us in one / two groups:
+// Workgroups for every CU at most: 32 / 8 heads of 128, 512 tokens 17.1 / 17.5 (eight tiles), 1024 28.1 / 26.3, behind 2000 73.3 / 61.4.
+// More: 1504 tokens 41.7 / 38.0, 16 / 8 of 128, 3520 82.4 / 74.0, 4096 97.7 / 91.6, fp8, 8 / 2 of 128, 4800 behind 2000 150 / 116; but the fuller the second round 1920
+// 52.0 / 54.2, 2048 of 32 / 4 of 64 33.1 / 34.0; with G = 8, whose workgroups have few tiles, 64 / 8 of 128, 1024 tokens 33.5 / 38.4; and behind a
+// prefix, which makes all of them long, 2048 behind 2000 120 / 127, 32 / 4 of 64 73.5 / 80.7.
+// In runs, which fill the CUs in either form, two groups halve the partials, but the runs of late rows are the longer ones: 32 / 8 of 128, 512 behind
+// 2000 44.3 / 41.4, 16 / 8 of 64, 512 behind 4000 35.0 / 27.2; but 4 / 1 of 128, 4096 tokens 44.9 / 50.5; and where their whole runs fill fewer
+// CUs, fp8, 16 / 8 of 128, 768 behind 4000 53.0 / 57.6 (96 workgroups in five runs, or in two of two groups).
 static int prefill_groups(const AttnPrefillArgs& a, int BQ) {
-  const int wg = (a.T + BQ - 1) / BQ * a.n_kv_heads, ntiles = (a.start + a.T - 1) / FP_KT + 1;
-  return ntiles >= 10 && wg <= 2 * device_cu_count() ? 2 : 1;
+  const int wg = (a.T + BQ - 1) / BQ * a.n_kv_heads, ntiles = (a.start + a.T - 1) / FP_KT + 1, cus = device_cu_count();
+  if (ntiles < 10) return 1;
+  const int runs = prefill_runs(a, BQ, 1);
+  if (runs > 1) return 2 * prefill_runs(a, BQ, 2) >= runs && 2L * a.T <= 3L * a.start && a.T <= 2048 ? 2 : 1;
+  if (wg <= cus) return 2;
+  return a.T >= 17 * FP_KT && 4L * (wg - cus) * (a.T + a.start) <= (a.T < 36 * FP_KT ? 3L : 4L) * cus * (a.T - a.start) ? 2 : 1;
+}
+
+void attn_prefill_form(const AttnPrefillArgs& a, int* groups, int* runs) {
+  const int BQ = 128 / (a.n_heads / a.n_kv_heads);
+  *groups = prefill_groups(a, BQ);
+  *runs = prefill_runs(a, BQ, *groups);
 }
 
 // FP_WG workgroups of 128 rows each, O and (max, sum) in fp32

@@ -144,7 +144,8 @@ struct AttnPrefillArgs {
 };
 size_t attn_prefill_ws_bytes(int head_dim);  // enough for every launch that is split
 void launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t st);
-bool attn_prefill_supports(int n_heads, int n_kv_heads, int head_dim);  // keys per workgroup the launcher picks
+bool attn_prefill_supports(int n_heads, int n_kv_heads, int head_dim);
+void attn_prefill_form(const AttnPrefillArgs& a, int* groups, int* runs);  // key groups of a workgroup and runs over the keys that a launch takes
 
 // ---- sampling ---------------------------------------------------------------------------------
 // per row b: token[b] = argmax(logits[b])   (temperature[b] > 0 -> Gumbel-max sample from

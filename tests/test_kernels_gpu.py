@@ -1010,6 +1010,15 @@ def test_attention_prefill_key_groups(E, H, Hkv, hd, start, T):
     test_attention_prefill_lists_of_heads(E, H, Hkv, hd, start, T)
 
 
+@pytest.mark.parametrize("H,Hkv,hd,start,T,form", [
+    (2, 2, 64, 0, 2100, (1, 4)), (8, 1, 128, 0, 1024, (1, 2)), (4, 1, 128, 700, 1100, (1, 3)), (4, 1, 128, 740, 1100, (2, 3)),
+    (32, 8, 128, 2000, 1184, (1, 1)), (16, 16, 128, 0, 2300, (2, 1)), (64, 8, 64, 0, 1000, (1, 1))])
+def test_attention_prefill_forms(E, H, Hkv, hd, start, T, form):
+    """one group of waves and two, in one run and in several"""
+    assert E.attn_prefill_form(H, Hkv, hd, start, T) == form
+    test_attention_prefill_lists_of_heads(E, H, Hkv, hd, start, T)
+
+
 @pytest.mark.parametrize("H,Hkv,hd", [(32, 8, 128), (32, 4, 64), (8, 8, 64), (16, 8, 128)])
 @pytest.mark.parametrize("start,T", [(1023, 1), (960, 64), (1100, 37), (3777, 300), (961, 129), (4000, 31)])
 @pytest.mark.parametrize("fp8", [False, True])
