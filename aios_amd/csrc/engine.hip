@@ -750,7 +750,7 @@ void Engine::finalize() {
 
 // Measured prefill-GEMM plans (kernels/gemm_pf.hip): every distinct projection launch of this model
 // -- QKV stack, O, gate/up (SwiGLU), down, per weight-format signature -- timed with its layers' weights in turn over
-// candidate tiles / K splits at M = 64 .. gm_rows_ (gemm_pf_bucket), the fastest kept per M bucket in the
+// candidate tiles / K splits at M = 64 .. the bucket of gm_rows_ (gemm_pf_bucket), the fastest kept per M bucket in the
 // process-wide plan cache (one tuning per shape per process; 1.0 s for Mistral-7B Q4_K_M at a context of 4096, 0.3 s for TinyLlama Q4_K_M).
 // Activations are random bf16 (a zero fill clocks the chip differently).  AIOS_GEMM_PF_TUNE=0: model plans only.
 void Engine::tune_prefill_gemm() {
@@ -758,36 +758,54 @@ void Engine::tune_prefill_gemm() {
   if (const char* e = std::getenv("AIOS_GEMM_PF_TUNE"))
     if (std::atoi(e) == 0) return;
   const int d = cfg_.d_model, hd = cfg_.head_dim, qd = cfg_.n_heads * hd, kvd = cfg_.n_kv_heads * hd;
-  const int ff = cfg_.d_ff, G = gm_rows_, ldqkv = qd + 2 * kvd;
+  const int ff = cfg_.d_ff, G = gemm_pf_bucket(gm_rows_), ldqkv = qd + 2 * kvd;
   const bool tp = cfg_.tp_size > 1;
+  // (the rows of a bucket can be more than the engine's: buffers of their own then)
+  struct Bufs {
+    std::vector<void*> p;
+    void* get(size_t bytes) {
+      void* q = nullptr;
+      HIP_CHECK(hipMalloc(&q, bytes));
+      p.push_back(q);
+      return q;
+    }
+    ~Bufs() {
+      for (void* q : p) (void)hipFree(q);
+    }
+  } bufs;
   const size_t n = (size_t)G * std::max({d, qd, ff});
-  float* tmp = nullptr;
-  HIP_CHECK(hipMalloc(&tmp, n * 4));
+  const bool own = G > gm_rows_;
+  float* tmp = (float*)bufs.get(n * 4);
+  bf16_t* a16 = own ? (bf16_t*)bufs.get((size_t)G * d * 2) : gm_a16_;
+  bf16_t* attn16 = own ? (bf16_t*)bufs.get((size_t)G * qd * 2) : gm_attn16_;
+  bf16_t* ff16 = own ? (bf16_t*)bufs.get((size_t)G * ff * 2) : gm_ff16_;
+  float* x = own ? (float*)bufs.get((size_t)G * d * 4) : tp ? gm_part_ : gm_x_;
+  float* qkv = own ? (float*)bufs.get((size_t)G * ldqkv * 4) : gm_qkv_;
   fill_random_f32(tmp, n, 0x7u, 0.f, 1.f, stream_);
-  launch_f32_to_bf16(tmp, gm_a16_, (size_t)G * d, stream_);
-  launch_f32_to_bf16(tmp, gm_attn16_, (size_t)G * qd, stream_);
-  launch_f32_to_bf16(tmp, gm_ff16_, (size_t)G * ff, stream_);
+  launch_f32_to_bf16(tmp, a16, (size_t)G * d, stream_);
+  launch_f32_to_bf16(tmp, attn16, (size_t)G * qd, stream_);
+  launch_f32_to_bf16(tmp, ff16, (size_t)G * ff, stream_);
   std::vector<GemmQArgs> launches;
   for (int M = 64; M <= G; M = gemm_pf_bucket(M + 1)) {
     for (const LayerW& L : layers_) {
       GemmQArgs g;
       std::memset(&g, 0, sizeof(g));
-      g.A = gm_a16_; g.lda = d; g.M = M; g.K = d; g.nseg = 3;
+      g.A = a16; g.lda = d; g.M = M; g.K = d; g.nseg = 3;
       g.seg[0] = L.wq.w; g.seg[1] = L.wk.w; g.seg[2] = L.wv.w;
       g.seg_n0[0] = 0; g.seg_n0[1] = qd; g.seg_n0[2] = qd + kvd;
-      g.N = ldqkv; g.C = gm_qkv_; g.ldc = ldqkv; g.epi = GEPI_STORE;
+      g.N = ldqkv; g.C = qkv; g.ldc = ldqkv; g.epi = GEPI_STORE;
       launches.push_back(g);
       std::memset(&g, 0, sizeof(g));
-      g.A = gm_attn16_; g.lda = qd; g.M = M; g.K = qd; g.nseg = 1; g.seg[0] = L.wo.w; g.N = d; g.ldc = d;
-      if (tp) { g.C = gm_part_; g.epi = GEPI_STORE; } else { g.C = gm_x_; g.epi = GEPI_ACCUM; }
+      g.A = attn16; g.lda = qd; g.M = M; g.K = qd; g.nseg = 1; g.seg[0] = L.wo.w; g.N = d; g.ldc = d;
+      g.C = x; g.epi = tp ? GEPI_STORE : GEPI_ACCUM;
       launches.push_back(g);
       std::memset(&g, 0, sizeof(g));
-      g.A = gm_a16_; g.lda = d; g.M = M; g.K = d; g.nseg = 1; g.seg[0] = L.wgu.w; g.N = 2 * ff;
-      g.C16 = gm_ff16_; g.ldc = ff; g.epi = GEPI_SWIGLU_BF16;
+      g.A = a16; g.lda = d; g.M = M; g.K = d; g.nseg = 1; g.seg[0] = L.wgu.w; g.N = 2 * ff;
+      g.C16 = ff16; g.ldc = ff; g.epi = GEPI_SWIGLU_BF16;
       launches.push_back(g);
       std::memset(&g, 0, sizeof(g));
-      g.A = gm_ff16_; g.lda = ff; g.M = M; g.K = ff; g.nseg = 1; g.seg[0] = L.wdown.w; g.N = d; g.ldc = d;
-      if (tp) { g.C = gm_part_; g.epi = GEPI_STORE; } else { g.C = gm_x_; g.epi = GEPI_ACCUM; }
+      g.A = ff16; g.lda = ff; g.M = M; g.K = ff; g.nseg = 1; g.seg[0] = L.wdown.w; g.N = d; g.ldc = d;
+      g.C = x; g.epi = tp ? GEPI_STORE : GEPI_ACCUM;
       launches.push_back(g);
     }
   }
@@ -796,7 +814,6 @@ void Engine::tune_prefill_gemm() {
   }
   gemm_pf_autotune(launches, stream_);
   HIP_CHECK(hipStreamSynchronize(stream_));
-  HIP_CHECK(hipFree(tmp));
 }
 
 // TP: sum the row-parallel partials in `p` over the ranks and add the total into `residual`

@@ -622,6 +622,24 @@ def test_prefill_plans_cover_every_projection_and_row_bucket():
     assert np.isfinite(np.asarray(eng.prefill(0, list(range(3, 203)), 0, True))).all()
 
 
+@pytest.mark.parametrize("ctx,bucket", [(400, 512), (2100, 2560), (3500, 4096)])
+def test_prefill_plans_of_a_context_between_two_buckets(ctx, bucket):
+    """the longest portions have a timed plan too where the context ends inside their bucket, and it is asked for by their row count"""
+    import dataclasses
+
+    from aios_amd.runtime import native
+    from aios_amd.runtime.loader import random_engine
+
+    m = native.require()
+    cfg = dataclasses.replace(get_preset("test-mistral-shape"), n_layers=1, d_model=768, d_ff=bucket + 256, vocab_size=512)
+    eng = random_engine(cfg, "Q4_K_M", seed=3, max_ctx=ctx, max_batch=1)
+    v = list(m.gemm_pf_export())
+    kn = {(p[0], p[1]) for p in (v[i:i + 14] for i in range(0, len(v), 14)) if p[2] == bucket}
+    assert {(cfg.d_model, cfg.d_ff), (2 * cfg.d_ff, cfg.d_model)} <= kn
+    prompt = [1] + [int(t) for t in np.random.default_rng(5).integers(3, 512, ctx - 9)]
+    assert np.isfinite(np.asarray(eng.prefill(0, prompt, 0, True))).all()
+
+
 def test_prefill_plans_of_a_first_engine_stay(monkeypatch):
     """A plan with K sliced over workgroups asks for a workspace, and an engine's is its widest product's (here: cut by AIOS_SKINNY_SMAX).
     A second engine without room for a plan of the first leaves it and runs the best plan that needs none; a plan that the
