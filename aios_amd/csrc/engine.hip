@@ -657,7 +657,7 @@ void Engine::finalize() {
       gm_x_ = fbuf((size_t)G * d);
       gm_qkv_ = fbuf((size_t)G * (qd + 2 * kvd));
       gm_q_ = fbuf((size_t)G * qd);
-      gm_part_ = fbuf((size_t)G * d);
+      if (cfg_.tp_size > 1) gm_part_ = fbuf((size_t)G * d);
       gm_a16_ = (bf16_t*)dmalloc((size_t)G * d * 2);
       gm_ff16_ = (bf16_t*)dmalloc((size_t)G * cfg_.d_ff * 2);
       gm_attn16_ = (bf16_t*)dmalloc((size_t)G * qd * 2);

@@ -224,6 +224,17 @@ def test_prefill_of_more_than_2048_rows_in_one_portion(T, monkeypatch):
     assert (out[0] - out[1]).abs().max().item() < 2e-2 * max(out[1].abs().max().item(), 1.0)
 
 
+def test_prefill_workspace_of_a_row(monkeypatch):
+    """a row of a portion costs what one rank's layer reads and writes, and no buffer that only ranks use"""
+    cfg, ws = get_preset("test-mistral-shape"), []
+    for rows in ("1024", "2048"):
+        monkeypatch.setenv("AIOS_PREFILL_GEMM_ROWS", rows)
+        ws.append(random_engine(cfg, "Q4_K_M", seed=0, max_ctx=2048, max_batch=1).workspace_bytes)
+    d, q, kv = cfg.d_model, cfg.n_heads * cfg.head_dim, cfg.n_kv_heads * cfg.head_dim
+    row = 4 * (d + (q + 2 * kv) + q) + 2 * (d + cfg.d_ff + q) + 4 * (d // 64) + 12
+    assert 0 <= ws[1] - ws[0] - 1024 * row < 1024 * 4 * d // 2
+
+
 @pytest.mark.parametrize("recipe", ["Q4_K_M", "mistral_shape", "Q5_K_M", "Q4_0", "Q8_0"])
 @pytest.mark.parametrize("tile", ["", "256x256", "128x256", "64x128"])
 def test_prefill_gemm_pf_chunks_match_reference(model_files, recipe, tile, monkeypatch):
