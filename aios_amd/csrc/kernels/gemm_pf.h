@@ -1032,14 +1032,19 @@ __device__ __forceinline__ void pf8_finish(const GemmQArgs& a, const gf32x4 (&ac
         const int m = m0 + 16 * i + (lane >> 1);
         if (m < a.M) *(gf32x4*)(out + (size_t)m * a.ldc + 8 * (lane & 1)) = v;
       }
-    } else {
+    } else {  // (rows that only 8 bytes divide, or 2)
+      const bool vec = a.ldc % 4 == 0 && ((uintptr_t)a.C16 & 7) == 0;
 #pragma unroll
       for (int i = 0; i < MT; ++i) {
         const int m = m0 + 16 * i + r16;
         const uint2 v = glu(i);
         if (m >= a.M) continue;
         bf16_t* p = out + (size_t)m * a.ldc + 4 * q;
-        p[0] = (bf16_t)v.x; p[1] = (bf16_t)(v.x >> 16); p[2] = (bf16_t)v.y; p[3] = (bf16_t)(v.y >> 16);
+        if (vec) {
+          *(uint2*)p = v;
+        } else {
+          p[0] = (bf16_t)v.x; p[1] = (bf16_t)(v.x >> 16); p[2] = (bf16_t)v.y; p[3] = (bf16_t)(v.y >> 16);
+        }
       }
     }
   } else if constexpr (EPI == GEPI_STORE16) {

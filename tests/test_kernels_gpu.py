@@ -1839,6 +1839,18 @@ def test_gemm_pf8_outputs(E, monkeypatch, bm, fmt, epi):
     rounded product of two sums."""
     if epi == "store16" and fmt != "BF16":
         pytest.skip("bf16 weights only")
+    cols = 256 if epi == "swiglu" else 512
+    pf8_outputs(E, monkeypatch, bm, fmt, epi, ((0, cols + 8), (1, cols + 8), (0, cols + 1)))
+
+
+@pytest.mark.parametrize("bm", [64, 256])
+@pytest.mark.parametrize("fmt", ["Q4_K", "BF16"])
+def test_gemm_pf8_swiglu_rows_of_8_bytes(E, monkeypatch, bm, fmt):
+    """... and a base and pitches that 8 bytes fit, or one of the two"""
+    pf8_outputs(E, monkeypatch, bm, fmt, "swiglu", ((0, 260), (4, 264), (4, 260), (2, 260)))
+
+
+def pf8_outputs(E, monkeypatch, bm, fmt, epi, places):
     K, N, M = 1024, 512, bm + 37
     m, W = qmat(E, GGMLType[fmt], N, K, seed=7, std=0.05)
     monkeypatch.setenv("AIOS_GEMM_PF_TILE", f"{bm}x256")
@@ -1848,7 +1860,7 @@ def test_gemm_pf8_outputs(E, monkeypatch, bm, fmt, epi):
     cols = N // 2 if epi == "swiglu" else N
     ref = torch.nn.functional.silu(z[:, 0::2]) * z[:, 1::2] if epi == "swiglu" else z
     e = {"store": E.GEPI_STORE, "accum": E.GEPI_ACCUM, "split": E.GEPI_ACCUM, "swiglu": E.GEPI_SWIGLU_BF16, "store16": E.GEPI_STORE16}[epi]
-    for off, ld in ((0, cols + 8), (1, cols + 8), (0, cols + 1)):
+    for off, ld in places:
         buf = torch.full(((M + 1) * ld + 8,), 2.0, device="cuda", dtype=torch.bfloat16 if half else torch.float32)
         to = buf[off:].data_ptr()
         E.gemm_q(A.data_ptr(), K, [m], M, 0 if half else to, to if half else 0, ld, e, stream(), 2 if epi == "split" else 1)
