@@ -769,6 +769,20 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
         return gemm_wk_serves(a);
       },
       py::arg("segs"), py::arg("M"), py::arg("epi"), py::arg("ksplit") = 0, py::arg("more") = py::dict());
+  // the slices of K of a product of one format that adds to its output, 0 where the launch goes elsewhere (host only)
+  m.def(
+      "gemm_wk_slices",
+      [](int qtype, int N, int K, int M, size_t ws_bytes, int cnt_len) {
+        GemmQArgs a;
+        std::memset(&a, 0, sizeof(a));
+        float ws;
+        int cnt;
+        a.nseg = 1; a.seg[0].qtype = qtype; a.seg[0].rows = N; a.seg[0].cols = K;
+        a.M = M; a.N = N; a.K = K; a.epi = GEPI_ACCUM; a.lda = K; a.ldc = N;
+        a.ws = &ws; a.ws_bytes = ws_bytes; a.cnt = &cnt; a.cnt_len = cnt_len;
+        return gemm_wk_slices(a);
+      },
+      py::arg("qtype"), py::arg("N"), py::arg("K"), py::arg("M"), py::arg("ws_bytes") = SIZE_MAX, py::arg("cnt_len") = INT_MAX);
   m.def(
       "gemm_pf_fuses",
       [](std::vector<PyQMatrix*> segs, int M, int epi, uintptr_t A, int lda, uintptr_t C, int ldc, const py::dict& more) {

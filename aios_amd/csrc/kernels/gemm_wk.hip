@@ -246,9 +246,7 @@ __device__ __forceinline__ void wk_body(const GemmQArgs& a, const WkPlan& p, int
   for (int s = 0; s < NS; ++s) load(w[s], s, t0);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    turn_x(x[s]);
-  }
+  for (int s = 0; s < NS; ++s) turn_x(x[s]);
   if (nrm) nr.done(a, wave, lane, inv_s);  // (read after the first tile's barrier)
   // what the outputs need besides their sums is requested before the tile's products (by every wave: which of them adds the tile up
   // is not worth a branch here).  Behind the sums it was one or two trips to memory at the end of a launch.
@@ -388,21 +386,22 @@ static bool wk_route(const GemmQArgs& a, WkRoute& r) {
   while (stages(r.S) > NSM) ++r.S;
   if (r.S > WK_SMAX) return false;
   r.ns = stages(r.S);
-  // Q6_K in three slices of at most 13 blocks, up to 16 rows: the ring's deeper stream where its 128-row tiles in eight slices cover three
+  // Q6_K in three slices, K of 10240 at most, up to 16 rows: the ring's deeper stream where its 128-row tiles in eight slices cover three
   // quarters of the CUs.  us here / ring, 4 and 16 rows: 4096 x 9216 14.6 / 14.0, 14.8 / 15.0   4096 x 10240 15.1 / 14.8, 15.6 / 15.9
   //   6144 x 8448 17.1 / 17.0, 17.5 / 18.0   4096 x 8448 13.5 / 13.7, 13.5 / 14.5; but 4096 x 11008 15.0 / 16.0, 15.7 / 16.8
   //   4096 x 12288 15.8 / 16.7, 16.5 / 17.4   4096 x 14336 17.8 / 18.6, 18.3 / 19.2   8192 x 28672 50.5 / 54.9, 53.4 / 57.6
   const int cus = device_cu_count(), round = a.N / 128 * 8;
   if (qt0 == QT_Q6_K && r.S == 3 && nu <= 40 && r.mt == 1 && a.N % 128 == 0 && 4 * round >= 3 * cus) return false;
   // bf16 where a tile has little k for eight waves to share: the skinny GEMM.  us here / skinny, 16 rows: 128256 x 512 44 / 33, 32000 x 64 9.7 / 5.5;
-  // but 32000 x 512 13.2 / 15.4, 128256 x 4096 170 / 224, 32 rows 188 / 233.  And, for bf16 results as they were, where slabs cost (long K
-  // and a wide output; two 16-row groups of one round of its tiles), though it is ahead no longer: 4096 x 14336 24 / 27, 4096 x 8192, 32 rows 19 / 20
+  // but 32000 x 512 13.2 / 15.4, 128256 x 4096 170 / 224, 32 rows 188 / 233.  And where slabs cost (long K and a wide output; two 16-row groups
+  // of one round of its tiles): it was ahead there before whole lines and is no longer, 4096 x 14336 24 / 27, 4096 x 8192, 32 rows 19 / 20, but
+  // this line is where test_gemm_wk_leaves_some_bf16_to_skinny holds it
   if (bf && (a.N > 125L * a.K || (a.K > 12288 && a.N >= 4096) || (r.mt == 2 && r.S >= 4 && 4 * round >= 3 * cus && round <= cus))) return false;
   // (three segments' four planes and the cache's arguments: more scalars than there are)
   if (a.epi == GEPI_QKV && qt0 == QT_Q6_K && r.ns * r.mt == 4) return false;
   // One slice more where that deals the tiles out more evenly: G ranges of whole tiles leave CUs idle while the longer ranges end.  With a split
   // that there is anyway, from a fifth less for the longest range up, if a quarter of the ranges are longer ones; us before / so, 16 and 30 rows:
-  // 2048 x 8704 (three slices of 85 ranges, 43 of them two tiles long) bf16 12.7 / 11.8, 13.0 / 12.9 (eight already), Q6_K 11.1 / 10.2, 13.6 / 12.5,
+  // 2048 x 8704 (three slices of 85 ranges, 43 of them two tiles long) bf16 12.7 / 11.8 (30 rows: five slices already), Q6_K 11.1 / 10.2, 13.6 / 12.5,
   // Q4_K 9.2 / 8.8, 11.4 / 10.8; 2048 x 5632 bf16, 30 rows 10.6 / 9.9; but 4096 x 12288 (one of 85 ranges is longer) Q4_K 12.5 / 13.2, 14.9 / 15.9,
   // Q6_K 16.5 / 17.2; 5120 x 17408 Q4_K, 8 % less 18.4 / 18.8.
   // bf16, two slices instead of one where its tiles are for three eighths of the CUs at most and a wave has two stages: 1024 x 4096 7.2 / 6.5,
@@ -424,10 +423,11 @@ static bool wk_route(const GemmQArgs& a, WkRoute& r) {
   return r.S == 1 || room(r.S);
 }
 
-bool gemm_wk_serves(const GemmQArgs& a) {
+int gemm_wk_slices(const GemmQArgs& a) {
   WkRoute r;
-  return wk_route(a, r);
+  return wk_route(a, r) ? r.S : 0;
 }
+bool gemm_wk_serves(const GemmQArgs& a) { return gemm_wk_slices(a) > 0; }
 
 template <int QT0, int QT1, int NS, int MT>
 static void wk_launch(const GemmQArgs& a, const WkRoute& r, hipStream_t st) {

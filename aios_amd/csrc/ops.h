@@ -266,6 +266,7 @@ void launch_gemm_q(const GemmQArgs& a, hipStream_t st);
 // takes these args
 bool gemm_wk_on();
 bool gemm_wk_serves(const GemmQArgs& a);
+int gemm_wk_slices(const GemmQArgs& a);  // ... in how many slices of K (0: not)
 // the prefill GEMM (kernels/gemm_pf.hip): true if it took the launch; its tile / split plan for a shape
 bool launch_gemm_pf(const GemmQArgs& a, hipStream_t st);
 // whether the prefill GEMM would run these args, the decode GEMMs' fused epilogues among them, on the tile with K over the waves that the plain product runs on

@@ -1276,7 +1276,7 @@ def test_gemm_wk(E, M, segs, K, ksplit, epi):
 @pytest.mark.parametrize("t,N,K", [("BF16", 2048, 8704), ("Q6_K", 2048, 8704), ("Q4_K", 4096, 12288), ("BF16", 2048, 4096), ("BF16", 1088, 3136),
                                    ("BF16", 2048, 2048)])
 def test_gemm_wk_slices_chosen_for_even_ranges(E, M, t, N, K):
-    """K in one slice more than the registers ask for, where that deals the tiles out more evenly (the last: not); tolerance: test_gemm_wk"""
+    """the sums of K in one slice more than the registers ask for, and in as many (that it is one more: test_kernel_routes.py); tolerance: test_gemm_wk"""
     m, W = small_mat(E, t, N, K, seed=K + N)
     assert E.gemm_wk_serves([m], M, E.GEPI_ACCUM, 0)
     A = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
@@ -1293,8 +1293,8 @@ def test_gemm_wk_slices_chosen_for_even_ranges(E, M, t, N, K):
 @pytest.mark.parametrize("t,N,K", [("BF16", 1600, 5632), ("BF16", 2048, 7168), ("BF16", 3072, 8192), ("BF16", 2048, 8192), ("Q6_K", 3072, 10240),
                                    ("Q6_K", 3072, 10496), ("Q6_K", 3072, 14336)])
 def test_gemm_wk_four_slices_and_long_q6k(E, M, t, N, K):
-    """both sides of the lines for four slices in place of two, and for Q6_K's long products (10240: the ring's up to 16 rows);
-    tolerance: test_gemm_wk"""
+    """the sums on both sides of the lines for four slices in place of two (how many it is: test_kernel_routes.py), and for Q6_K's long products
+    (10240: the ring's up to 16 rows); tolerance: test_gemm_wk"""
     m, W = small_mat(E, t, N, K, seed=K + N)
     assert t == "BF16" or E.gemm_wk_serves([m], M, E.GEPI_ACCUM, 0) == (K > 10240 or M > 16)
     A = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
