@@ -921,8 +921,9 @@ void Engine::gemm(GemmQArgs& g) {
 //   Mistral-7B bf16 (436 MB)         2 rows 2969 / 3058   3 rows 3271 / 3089   4 rows 3813 / 3096
 // The GEMV's dot work grows with the rows, the GEMM's does not.  Quantised weights: it wins from 4, and from 2 where the layers are
 // so small that launches bound a step (TinyLlama's d_ff has no GEMV plan at 2 rows either, so its GEMVs above are the
-// row-pair ones); where the GEMV would take int8 activations.  bf16: from 3.  Only where K-shared waves serve every projection (all
-// Q4_K / Q6_K, or all bf16); across ranks as before.
+// row-pair ones); where the GEMV would take int8 activations.  bf16: from 3.  Only where every projection is of a format that K-shared waves
+// serve (all Q4_K / Q6_K, or all bf16): shapes that they leave to others (gemm_wk.hip, wk_route) run those, as Mistral-7B's down of bf16
+// weights, 4096 x 14336, does the skinny GEMM in the times above.  Across ranks as for other formats.
 int Engine::default_gemm_min_b() const {
   if (cfg_.tp_size > 1 || !gemm_wk_on()) return dec_gemm_min_b_;
   size_t bytes = 0, n = 0, bf = 0, kq = 0;

@@ -31,15 +31,6 @@ __device__ __forceinline__ float ld_wt(const float* p) {
   return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// sum over aligned groups of N lanes (N = 8 or 16), result in every lane of the group
-template <int N>
-__device__ __forceinline__ float group_sum(float v) {
-  v += lane_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += lane_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += lane_dpp<0x141>(v);  // row_half_mirror: lane i <-> 7-i within 8
-  if constexpr (N == 16) v += lane_dpp<0x140>(v);  // row_mirror: lane i <-> 15-i within 16
-  return v;
-}
 // op(v[lane], v[lane ^ OFF]) for OFF = 8, 16, 32
 template <int OFF, typename Op>
 __device__ __forceinline__ float xlane_op(float v, Op op) {
@@ -674,7 +665,7 @@ __device__ __forceinline__ void attn_lanes(const AttnDecodeArgs& a, int kvh, int
       float d = dot2_bf16(kb[0], q2[0], 0.f);
 #pragma unroll
       for (int i = 1; i < NP; ++i) d = dot2_bf16(kb[i], q2[i], d);
-      d = group_sum<LPK>(d);
+      d = lanes_sum<LPK>(d);
       sc[s] = valid ? d : kNeg;
     }
     float mx = sc[0];
