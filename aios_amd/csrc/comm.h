@@ -12,7 +12,7 @@
 //    lm_head: each rank computes V/world logits, every rank needs all of them for the identical
 //    on-device sampler and the JSON-grammar mask).
 // All three are fused with their consumer where it is an elementwise op (residual add).
-//  * C1 / C2 of the batch-1 TP decode step fused into the PRODUCER instead (round 4): the O / down row
+//  * C1 / C2 of the batch-1 TP decode step fused into the PRODUCER instead: the O / down row
 //    GEMV's workgroups publish their rows' partials to per-workgroup stage slots behind the one-shot
 //    region and exchange per-slot flags (EPI_TP_RESID, gemv_q8.h) -- no all-reduce launch.  Stage and
 //    flags are uncached, so a retired store is visible to every peer without a system-scope fence.
@@ -125,7 +125,7 @@ class XgmiComm {
   uint32_t* myflags_ = nullptr;
   // the give-up flag lives in pinned, device-mapped host memory: the kernels set it with
   // system-scope stores and error() is a plain host load -- no per-call hipMemcpy (which
-  // serialised every leader call behind the device, verdict r2)
+  // serialised every leader call behind the device)
   volatile uint32_t* host_error_ = nullptr;
   std::vector<void*> opened_;
   int device_ = 0;

@@ -1199,6 +1199,7 @@ __device__ __forceinline__ void pf8_body(const GemmQArgs& a, int m0, int n0, int
   // us, weights from memory, so -> now: 1500 x 8704 x 2048 rows x columns x k 61.5 -> 54.8, 2048 x 11264 x 2048 120 -> 105, 2048 x 8192 x 8192 221 -> 212.)
   // Requests go B(0) B(1) A(0) B(2) A(1) .., B(t + NS + 1) in the middle of step t, when the wave has read B(t + 1), A(t + NS) at its end,
   // when all waves have read A(t).  Waits: B(t + 1) at its read, A(t + 1) at the barrier in front of its first read.
+  static_assert(NS * NA + (NS - 1) * NB <= 63, "vmcnt immediate");
   get_b(0, 0);
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p) {

@@ -141,7 +141,7 @@ def fused_self_test(comm, rank: int, world: int, device: int, allgather) -> bool
     from rank-keyed seeds, so each rank computes residual + sum over ranks of q8(x_r) . W_r^T itself.
     The fused protocol publishes partials with relaxed flag stores to uncached peer memory; a
     cross-device visibility problem would give wrong tokens, not an error -- this turns it into a
-    fallback (verdict r5 weak #8).  Every rank first reports whether the launch fits (dry run): a
+    fallback.  Every rank first reports whether the launch fits (dry run): a
     rank that would not launch would leave its peers waiting on flags."""
     import numpy as np
     import torch
@@ -210,7 +210,7 @@ def check_fused_comm(comm, rank: int, world: int, device: int, allgather) -> boo
 
 
 def share_prefill_plans(allgather):
-    """Every TP rank runs the leader's prefill-GEMM plans (ADVICE r5: each rank's own timing could
+    """Every TP rank runs the leader's prefill-GEMM plans (each rank's own timing could
     pick a different tile / split, i.e. a different summation order per rank)."""
     from ..runtime import native
 
@@ -222,7 +222,7 @@ def share_prefill_plans(allgather):
 def reconcile_tp_fuse(eng, allgather) -> bool:
     """After set_comm: every rank's per-layer fit of the fused O / down launch (Engine.tp_fuse_fits,
     which depends on the device's CU count and the co-residency cap) must be identical, or fusion goes
-    off on every rank (ADVICE r5: a rank falling back alone leaves its peers waiting on flags)."""
+    off on every rank (a rank falling back alone leaves its peers waiting on flags)."""
     if not getattr(eng, "tp_fused", False):
         allgather(None)  # (the other ranks' gather still needs this rank's turn)
         return False
