@@ -442,6 +442,10 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       .def_property_readonly("norm_fused_parts", &Engine::norm_fused_parts)
       .def_property_readonly("prefill_fused", &Engine::prefill_fused)
       .def_property_readonly("decode_gemm_min_batch", &Engine::decode_gemm_min_batch)
+      .def_property_readonly("decode_resident", &Engine::decode_resident)
+      .def_property_readonly("decode_resident_failed", &Engine::decode_resident_failed)
+      .def("set_decode_resident", &Engine::set_decode_resident, py::arg("on"))
+      .def("set_decode_resident_wait", &Engine::set_decode_resident_wait, py::arg("ticks"))
       .def("capture_graphs", &Engine::capture_graphs, py::arg("max_b"), py::call_guard<py::gil_scoped_release>())
       .def_property_readonly("stream", &Engine::stream_handle)
       .def_property_readonly("k_cache_ptr", &Engine::kv_cache_k)

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "common.h"
+#include "kernels/decode_stream.h"
 #include "layered.h"
 #include "ops.h"
 
@@ -189,6 +190,13 @@ class Engine {
   void release_slot(int slot);         // drop every block reference of the slot
   int kv_blocks_free() const { return (int)free_blocks_.size(); }
   int kv_blocks_total() const { return kv_nblocks_; }
+  // one row's decode step as one resident launch (decode_stream.h): whether this engine's steps take it; off for tests
+  // and comparisons; steps that its launch gave up on (another resident launch held part of the GPU) and that were done
+  // without it; the time, in 10 ns, after which it gives up
+  bool decode_resident() const;
+  void set_decode_resident(bool on) { ds_use_ = on; }
+  unsigned decode_resident_failed() const { return ds_failed_ ? *(volatile unsigned*)ds_failed_ : 0; }
+  void set_decode_resident_wait(unsigned long long ticks);
   int decode_gemm_min_batch() const { return dec_gemm_min_b_; }  // rows from which decode takes the GEMMs
   int norm_fused_parts() const { return nrm_parts_; }  // 0: batched-decode RMSNorm not split into the GEMMs
   // of the last prompt's portions above 32 rows: norms split over two products, QKV products that wrote q and the cache themselves
@@ -423,6 +431,21 @@ class Engine {
   void kv_sync(int B);                                 // upload dirty tables (rows 0..B-1)
 
   std::map<int, hipGraphExec_t> graphs_;
+  // resident decode step
+  void ds_setup();
+  static void ds_shares(const LayerW& L, int parts, int& wg_k, int& wg_v);
+  void ds_upload();                // the cache's scales (again, when they change)
+  bool ds_next();                  // whether the next step of one row runs resident (a while after a failure: no)
+  int graph_key(int B, int kind);  // kind: 0 step, 1 masked step, 2 forward
+  hipGraphExec_t captured(int key, bool forward, int B);
+  void launch_step(hipGraphExec_t g);
+  DsArgs ds_{};
+  bool ds_ok_ = false, ds_use_ = true;
+  bool ds_now_ = false;            // the step being enqueued runs resident
+  float* ds_scale_ = nullptr;
+  unsigned* ds_failed_ = nullptr;  // pinned
+  unsigned ds_seen_ = 0;
+  int ds_rest_ = 0;
   AllReduceFn allreduce_ = nullptr;
   void* allreduce_ctx_ = nullptr;
   AllGatherFn allgather_ = nullptr;

@@ -6,6 +6,7 @@
 #include "comm.h"
 #include <cstdlib>
 #include <map>
+#include <mutex>
 
 #include <algorithm>
 #include <cstring>
@@ -93,9 +94,36 @@ Engine::Engine(const EngineConfig& cfg) : cfg_(cfg) {
   }
 }
 
+// Resident launches of a process take turns on a GPU: two of them at once would each hold some of the CUs and wait for the
+// others.  An engine that follows another one waits, on the device, for what that one has queued; the steps of one engine
+// follow each other in its stream anyway.  (Of other processes' launches nothing is known: what the gate is for.)  The lock
+// also keeps a stream from being captured while another engine records its event there.
+namespace {
+struct DsTurn {
+  std::mutex mu;
+  const void* last = nullptr;
+  hipStream_t stream = nullptr;
+  hipEvent_t ev = nullptr;
+};
+DsTurn& ds_turn(int device) {
+  static std::mutex mu;
+  static auto* turns = new std::map<int, DsTurn>;  // (engines may go after static objects)
+  std::lock_guard<std::mutex> g(mu);
+  return (*turns)[device];
+}
+}  // namespace
+
 Engine::~Engine() {
   if (lm_) (void)hipStreamSynchronize(stream_);
   lm_.reset();
+  if (ds_ok_) {
+    DsTurn& t = ds_turn(cfg_.device);
+    std::lock_guard<std::mutex> lock(t.mu);
+    if (t.last == this) {
+      (void)hipStreamSynchronize(stream_);
+      t.last = nullptr;
+    }
+  }
   try {
     stage_release();
   } catch (...) {
@@ -105,6 +133,7 @@ Engine::~Engine() {
   if (h_par_) hipHostFree(h_par_);
   if (h_tok_out_) hipHostFree(h_tok_out_);
   if (h_mask_) hipHostFree(h_mask_);
+  if (ds_failed_) hipHostFree(ds_failed_);
   if (pipe_ev_) hipEventDestroy(pipe_ev_);
   if (stream_) hipStreamDestroy(stream_);
 }
@@ -743,9 +772,164 @@ void Engine::finalize() {
     }
   }
   ws_bytes_ = ws;
+  ds_setup();
   HIP_CHECK(hipDeviceSynchronize());
   tune_prefill_gemm();
   finalized_ = true;
+}
+
+// One row's step as one resident launch (decode_stream.h): a GPU to itself, every matrix Q4_K or Q6_K with int8 activations.
+// (A rank of several, or a tier on some of the CUs, would wait for others inside the launch; bf16 and the other formats have
+// their own GEMVs.  AIOS_DECODE_GEMM_MIN_B=0 asks for the GEMVs alone.)
+void Engine::ds_setup() {
+  if (dec_gemm_min_b_ <= 0) return;
+  if (lm_ || cfg_.tp_size > 1 || cfg_.vocab_parallel || !cfg_.act_q8 || !cfg_.cu_mask.empty() || !rope_cs_ || cfg_.n_layers < 1) return;
+  auto served = [](const QMat& m) { return m.valid() && (m.w.qtype == QT_Q4_K || m.w.qtype == QT_Q6_K); };
+  if (!served(output_) || cfg_.vocab_size % 2) return;
+  for (const LayerW& L : layers_)
+    for (const QMat* m : {&L.wq, &L.wk, &L.wv, &L.wo, &L.wgu, &L.wdown})
+      if (!served(*m)) return;
+  for (const LayerW& L : layers_)
+    if (!L.bqkv != !layers_[0].bqkv || (L.bqkv && (cfg_.qk_norm || cfg_.rope_neox)) || (cfg_.qk_norm && (!L.q_norm || !L.k_norm))) return;
+  const int hd = cfg_.head_dim, d = cfg_.d_model, H = cfg_.n_heads, Hkv = cfg_.n_kv_heads;
+  DsArgs& a = ds_;
+  a.parts = device_cu_count();
+  a.n_layers = cfg_.n_layers; a.d = d; a.n_heads = H; a.n_kv_heads = Hkv; a.ff = cfg_.d_ff; a.vocab = cfg_.vocab_size;
+  a.max_ctx = cfg_.max_ctx; a.rope_neox = cfg_.rope_neox; a.kv_fp8 = cfg_.kv_fp8;
+  a.eps = cfg_.norm_eps; a.scale = 1.f / std::sqrt((float)hd);
+  if (a.parts < 4) return;
+  auto share = [](int rows, int n) { return (rows + n - 1) / n; };  // rows of one workgroup of n, at most
+  int most = std::max({share(d, a.parts), 4 * share(cfg_.d_ff / 2, a.parts), share(cfg_.vocab_size, a.parts)});
+  for (const LayerW& L : layers_) {
+    int wk, wv;
+    ds_shares(L, a.parts, wk, wv);
+    most = std::max({most, share(L.wq.w.rows, wk), share(L.wk.w.rows, wv - wk), share(L.wv.w.rows, a.parts - wv)});
+  }
+  if (!ds_plan(a, hd, most)) return;
+  a.x = x_; a.logits = logits_; a.rope_cs = rope_cs_; a.pos = d_pos_; a.blocks = d_row_bt_;
+  auto words = [&](size_t n) {
+    auto* p = (uint64_t*)dmalloc(n * 8);
+    HIP_CHECK(hipMemset(p, 0, n * 8));
+    ws_bytes_ += n * 8;
+    return p;
+  };
+  const size_t nl = cfg_.n_layers;
+  a.nqkv = (H + 2 * Hkv) * hd;
+  a.xn = words(2 * nl * d);
+  a.sq = words(2 * nl * a.parts);
+  a.resid = (float*)words((d + 1) / 2);
+  a.qkv = words(nl * a.nqkv);
+  a.attn = words(nl * H * hd);
+  a.h = words(nl * cfg_.d_ff / 2);
+  a.part = words(ds_part_words(H, hd));
+  a.ctl = (DsCtl*)words((sizeof(DsCtl) + 7) / 8);
+  HIP_CHECK(hipHostMalloc((void**)&ds_failed_, 4, hipHostMallocDefault));
+  *ds_failed_ = 0;
+  a.host_failed = ds_failed_;
+  a.gate_ticks = 2000000;     // 20 ms: longer than a kernel of another queue holds the CUs
+  a.wait_ticks = 100000000;   // 1 s
+  // norms' gains, heads' gains and biases of all layers beside each other
+  auto table = [&](size_t n) {
+    ws_bytes_ += n * 4;
+    return (float*)dmalloc(n * 4);
+  };
+  auto keep = [&](float* to, const float* from, size_t n) { HIP_CHECK(hipMemcpy(to, from, n * 4, hipMemcpyDeviceToDevice)); };
+  const size_t nr = a.nqkv;
+  float* gains = table((size_t)(2 * cfg_.n_layers + 1) * d);
+  float* qk = cfg_.qk_norm ? table((size_t)2 * cfg_.n_layers * hd) : nullptr;
+  float* bias = layers_[0].bqkv ? table(cfg_.n_layers * nr) : nullptr;
+  for (int l = 0; l < cfg_.n_layers; ++l) {
+    const LayerW& L = layers_[l];
+    keep(gains + (size_t)2 * l * d, L.attn_norm, d);
+    keep(gains + (size_t)(2 * l + 1) * d, L.ffn_norm, d);
+    if (qk) keep(qk + (size_t)2 * l * hd, L.q_norm, hd), keep(qk + (size_t)(2 * l + 1) * hd, L.k_norm, hd);
+    if (bias) keep(bias + l * nr, L.bqkv, nr);
+  }
+  keep(gains + (size_t)2 * cfg_.n_layers * d, out_norm_, d);
+  a.gains = gains;
+  a.qk_gains = qk;
+  a.bias = bias;
+  a.kv_scale = ds_scale_ = table(2 * cfg_.n_layers);
+  a.kc = (uint8_t*)k_cache_;
+  a.vc = (uint8_t*)v_cache_;
+  a.kv_layer = layer_kv_elems_ * kv_es_;
+  ds_upload();
+  std::vector<DsCopy> jobs;
+  // rows of m, in whole units, over workgroups [w0, w1)
+  auto deal = [&](const QMat& m, int w0, int w1, int unit, int row0) {
+    const long units = m.w.rows / unit, n = w1 - w0;
+    for (long i = 0; i < n; ++i) {
+      const int r = unit * (int)(i * units / n), e = unit * (int)((i + 1) * units / n);
+      jobs.push_back(ds_job(m.w, r, e - r, row0));
+    }
+  };
+  for (const LayerW& L : layers_) {
+    int wk, wv;
+    ds_shares(L, a.parts, wk, wv);
+    deal(L.wq, 0, wk, 1, 0);
+    deal(L.wk, wk, wv, 1, H * hd);
+    deal(L.wv, wv, a.parts, 1, (H + Hkv) * hd);
+    deal(L.wo, 0, a.parts, 1, 0);
+    deal(L.wgu, 0, a.parts, 4, 0);  // (two gate/up pairs: a word of the exchange)
+    deal(L.wdown, 0, a.parts, 1, 0);
+  }
+  deal(output_, 0, a.parts, 1, 0);
+  auto* dj = (DsCopy*)dmalloc(sizeof(DsCopy) * jobs.size());
+  HIP_CHECK(hipMemcpy(dj, jobs.data(), sizeof(DsCopy) * jobs.size(), hipMemcpyHostToDevice));
+  ws_bytes_ += sizeof(DsCopy) * jobs.size();
+  a.jobs = dj;
+  ds_ok_ = true;
+}
+
+// Q, K and V of a layer have workgroups of their own, as many as their bytes are of all
+void Engine::ds_shares(const LayerW& L, int parts, int& wg_k, int& wg_v) {
+  auto cost = [](const QMat& m) { return (double)m.w.rows * (m.w.qtype == QT_Q4_K ? 144 : 210); };
+  const double q = cost(L.wq), k = cost(L.wk), all = q + k + cost(L.wv);
+  wg_k = std::min(std::max(1, (int)std::lround(parts * q / all)), parts - 2);
+  wg_v = std::min(std::max(wg_k + 1, (int)std::lround(parts * (q + k) / all)), parts - 1);
+}
+
+void Engine::ds_upload() {
+  HIP_CHECK(hipMemcpy(ds_scale_, kv_scale_.data(), kv_scale_.size() * 4, hipMemcpyHostToDevice));
+}
+
+bool Engine::decode_resident() const { return ds_ok_ && ds_use_; }
+
+void Engine::set_decode_resident_wait(unsigned long long ticks) {
+  if (finalized_) HIP_CHECK(hipStreamSynchronize(stream_));
+  ds_.gate_ticks = ticks;
+  reset_graphs();
+}
+
+bool Engine::ds_next() {
+  if (!decode_resident()) return false;
+  const unsigned n = decode_resident_failed();
+  if (n != ds_seen_) {  // another resident launch holds CUs: leave it the GPU for a while
+    ds_seen_ = n;
+    ds_rest_ = 4096;
+  }
+  if (ds_rest_ > 0) {
+    --ds_rest_;
+    return false;
+  }
+  return true;
+}
+
+void Engine::launch_step(hipGraphExec_t g) {
+  if (!ds_now_) {
+    HIP_CHECK(hipGraphLaunch(g, stream_));
+    return;
+  }
+  DsTurn& t = ds_turn(cfg_.device);
+  std::lock_guard<std::mutex> lock(t.mu);
+  if (t.last && t.last != this) {
+    if (!t.ev) HIP_CHECK(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
+    HIP_CHECK(hipEventRecord(t.ev, t.stream));
+    HIP_CHECK(hipStreamWaitEvent(stream_, t.ev, 0));
+  }
+  HIP_CHECK(hipGraphLaunch(g, stream_));
+  t.last = this;
+  t.stream = stream_;
 }
 
 // Measured prefill-GEMM plans (kernels/gemm_pf.hip): every distinct projection launch of this model
@@ -1249,8 +1433,12 @@ void Engine::enqueue_decode_forward(int B) {
     launch_get_rows_step(tok_embd_.w, d_tokens_, B, x_, d, 1.f, sp, stream_);
   }
   static const bool step_prep = !(std::getenv("AIOS_STEP_PREP") && std::atoi(std::getenv("AIOS_STEP_PREP")) == 0);
-  step_prep_on_ = step_prep && rope_cs_ != nullptr;
   nrm_lm_ = false;
+  if (B == 1 && ds_now_) {
+    launch_decode_stream(ds_, cfg_.head_dim, stream_);
+    return;
+  }
+  step_prep_on_ = step_prep && rope_cs_ != nullptr;
   for (int l = 0; l < cfg_.n_layers; ++l) layer_decode(l, B);
   step_prep_on_ = false;
   lm_head(B, x_, d);
@@ -1924,45 +2112,33 @@ void Engine::decode_loop_run(int B, int n_steps, bool use_graph) {
   }
   kv_sync(B);
   if (!use_graph) {
+    ds_now_ = false;
     for (int i = 0; i < n_steps; ++i) enqueue_decode_step(B);
     return;
   }
+  ds_now_ = B == 1 && ds_next();
   hipGraphExec_t ge = step_graph(B);
-  for (int i = 0; i < n_steps; ++i) HIP_CHECK(hipGraphLaunch(ge, stream_));
+  for (int i = 0; i < n_steps; ++i) launch_step(ge);
 }
+
+int Engine::graph_key(int B, int kind) { return B * 4 + kind + (B == 1 && ds_now_ ? 1 << 24 : 0); }
 
 // the captured decode step for (B, sample_mask_): captured once, replayed for every request --
 // the kernels read tokens / positions / slots / sampling parameters from device arrays
-hipGraphExec_t Engine::step_graph(int B) {
-  const int key = B * 4 + (sample_mask_ ? 1 : 0);
-  auto it = graphs_.find(key);
-  if (it == graphs_.end()) {
-    hipGraph_t g;
-    HIP_CHECK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-    try {
-      enqueue_decode_step(B);
-    } catch (...) {
-      hipStreamEndCapture(stream_, &g);
-      throw;
-    }
-    HIP_CHECK(hipStreamEndCapture(stream_, &g));
-    hipGraphExec_t ge;
-    HIP_CHECK(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
-    HIP_CHECK(hipGraphDestroy(g));
-    it = graphs_.emplace(key, ge).first;
-  }
-  return it->second;
-}
-
+hipGraphExec_t Engine::step_graph(int B) { return captured(graph_key(B, sample_mask_ ? 1 : 0), false, B); }
 // the forward of a decode step without its sampler (the pipelined decode's graph)
-hipGraphExec_t Engine::forward_graph(int B) {
-  const int key = B * 4 + 2;
+hipGraphExec_t Engine::forward_graph(int B) { return captured(graph_key(B, 2), true, B); }
+
+hipGraphExec_t Engine::captured(int key, bool forward, int B) {
   auto it = graphs_.find(key);
   if (it == graphs_.end()) {
+    std::unique_lock<std::mutex> turn;
+    if (ds_ok_) turn = std::unique_lock<std::mutex>(ds_turn(cfg_.device).mu);
     hipGraph_t g;
     HIP_CHECK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
     try {
-      enqueue_decode_forward(B);
+      if (forward) enqueue_decode_forward(B);
+      else enqueue_decode_step(B);
     } catch (...) {
       hipStreamEndCapture(stream_, &g);
       throw;
@@ -2026,7 +2202,8 @@ void Engine::decode_submit(const std::vector<int>& slots, const std::vector<int>
     row_pos_[b] = pos[b] + 1;
   }
   kv_sync(B);
-  HIP_CHECK(hipGraphLaunch(forward_graph(B), stream_));
+  ds_now_ = B == 1 && ds_next();
+  launch_step(forward_graph(B));
   pipe_B_ = B;
 }
 
@@ -2067,6 +2244,7 @@ int Engine::capture_graphs(int max_b) {
   const bool saved = sample_mask_;
   for (int B = 1; B <= std::min(max_b, cfg_.max_batch); ++B)
     for (int m = 0; m < 2; ++m) {
+      ds_now_ = B == 1 && decode_resident();
       sample_mask_ = m != 0;
       step_graph(B);
       if (m == 0) forward_graph(B);  // (the pipelined decode's forward)
@@ -2094,6 +2272,7 @@ void Engine::set_kv_scales(const std::vector<float>& s) {
     if (!(v > 0.f) || !std::isfinite(v)) throw std::runtime_error("set_kv_scales: scales must be positive");
   if (finalized_) HIP_CHECK(hipStreamSynchronize(stream_));  // (no replay of the old graphs in flight)
   kv_scale_ = s;
+  if (ds_ok_) ds_upload();
   reset_graphs();
 }
 

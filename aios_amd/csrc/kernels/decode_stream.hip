@@ -1,0 +1,997 @@
+// One row's decode step as ONE resident launch: a workgroup per CU runs the layers' products and the attention, and the
+// vectors between them go from workgroup to workgroup through memory.
+//
+// What bounds a step of one row is not its bytes: a chain of five launches a layer pays for each of them the launch, the
+// operand's round trip, the first weights' and the drain, 3.5 to 4 us in which the weight stream stands (gemv_lds.h).  Here the
+// stream does not stand: two waves of every workgroup copy the whole step's weights HBM -> LDS through one ring of 128 KB,
+// four slots ahead of the fourteen that multiply, across products and layers, so what the next product needs lies in LDS while
+// its operand is on its way.
+//
+// Exchanges.  A product's result is written as 64-bit words of (value, number of the exchange) with agent-scope stores, and
+// read the same way until every word carries the number: one trip through memory, no fence, no flag behind the data, no
+// barrier over the chip.  4096 values from and to 256 workgroups take 1.8 us (with a flag per workgroup written behind the
+// data 6.3).  Numbers run on from launch to launch (DsCtl::epoch), so nothing is cleared.  A buffer is used once a layer;
+// its words are overwritten only after an exchange that every reader of the old ones has contributed to (each workgroup owns
+// rows of O, gate/up and down).
+//
+// Waiting.  Workgroups wait for each other, so all of them have to be on the chip.  The first thing a workgroup does is to
+// sign in; the last one to do so opens the gate, and a workgroup that waited gate_ticks for it closes it for good: then all
+// of them leave, also those that come later, and the launch behind (one workgroup that takes every part in turn and so waits
+// for nobody) does the step.  Behind the open gate every wait is for a workgroup that runs; it is bounded all the same
+// (wait_ticks), with the same way out.
+//
+// A step, us, chain -> resident (MI355X, Q4_K_M): TinyLlama 128 keys 600 -> 464, 1000 keys 682 -> 578; Mistral-7B 128 keys 1424 -> 1190,
+// 3900 keys 1621 -> 1446; with the fp8 cache 2000 keys 1527 -> 1325, 16000 keys 1666 -> 1632; Qwen3-8B 128 keys 1755 -> 1325.
+#include "decode_stream.h"
+
+#include <algorithm>
+#include <numeric>
+
+#include "attn_decode.h"
+#include "gemv_impl.h"
+
+namespace aios {
+
+namespace {
+
+constexpr int DS_NG = 14, DS_NL = 2, DS_CT = DS_NG * 64, DS_THREADS = (DS_NG + DS_NL) * 64;
+constexpr int DS_SLOT = 32768, DS_R = 4;
+constexpr int DS_AW = 8;  // waves that attend
+
+// a slot: chunks (32 weights) and their planes, each a run of its own (1 KB an LDS-DMA; the last plane of Q6_K 256 B)
+template <int QT>
+struct DsFmt;
+template <>
+struct DsFmt<QT_Q4_K> {
+  static constexpr int CH = 1792, PAIRS = 1;  // a lane takes two chunks of a slot
+  static constexpr int off[4] = {0, 28672, 0, 0};
+  static constexpr int per_loader = 16;
+};
+template <>
+struct DsFmt<QT_Q6_K> {
+  static constexpr int CH = 896, PAIRS = 0;
+  static constexpr int off[4] = {0, 14336, 21504, 23552};
+  static constexpr int per_loader = 12;
+};
+
+// tables of the step through the scalar cache (uniform addresses, written before the launch): a vector load would be waited for
+// behind every weight request of a loader
+template <typename T>
+using ds_const = const __attribute__((address_space(4))) T*;
+template <typename T>
+__device__ __forceinline__ T ds_table(const T* p, int i) {
+  ds_const<uint32_t> q = (ds_const<uint32_t>)(uint64_t)(p + __builtin_amdgcn_readfirstlane(i));
+  uint32_t w[sizeof(T) / 4];
+#pragma unroll
+  for (int k = 0; k < (int)(sizeof(T) / 4); ++k) w[k] = q[k];
+  T v;
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
+
+enum { DS_QKV = 0, DS_O = 1, DS_GU = 2, DS_DOWN = 3 };
+
+// a loader's half of slot s, every other KB of each plane: every slot of a format is as many requests, what lies behind the
+// workgroup's rows reads as zeros without a memory access.  (No branch a request: with one each, a slot took 1 us to ask for.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ds_rsrc(const uint8_t* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)sgpr_ptr(p), (short)0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+template <int S>
+__device__ __forceinline__ void ds_request(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int voff, int at) {
+  // (non-temporal: each byte is read once a step)
+  auto* to = (__attribute__((address_space(3))) void*)(dst + at);
+  if constexpr (S == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 16, voff + at, 0, 0, 2);
+  else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 4, voff + at, 0, 0, 2);
+}
+template <int QT>
+__device__ __forceinline__ void ds_copy(const DsCopy& j, int s, uint8_t* dst, int lw) {
+  using F = DsFmt<QT>;
+  const int lane = threadIdx.x & 63;
+  const int c = s * F::CH, left = (j.job.chunks & ~DS_Q6) - c;
+  dst += lw * 1024;
+  const int v = lane * 16 + lw * 1024;
+  const auto r0 = ds_rsrc(j.p[0] + (size_t)c * 16, left * 16);
+  if constexpr (QT == QT_Q4_K) {
+    const auto r1 = ds_rsrc(j.p[1] + (size_t)c * 2, left * 2);
+    static_for<14>([&](auto i) { ds_request<16>(r0, dst, v, 2048 * i); });
+    static_for<2>([&](auto i) { ds_request<16>(r1, dst + F::off[1], v, 2048 * i); });
+  } else {
+    const auto r1 = ds_rsrc(j.p[1] + (size_t)c * 8, left * 8);
+    const auto r2 = ds_rsrc(j.p[2] + (size_t)c * 2, left * 2);
+    const auto r3 = ds_rsrc(j.p[3] + (c >> 2), left >> 2);
+    static_for<7>([&](auto i) { ds_request<16>(r0, dst, v, 2048 * i); });
+    static_for<3>([&](auto i) { ds_request<16>(r1, dst + F::off[1], v, 2048 * i); });
+    ds_request<16>(r2, dst + F::off[2], v, 0);
+    if (lw == 0) ds_request<16>(r1, dst + F::off[1], v, 6144);
+    else ds_request<4>(r3, dst - 1024 + F::off[3], lane * 4, 0);
+  }
+}
+
+// at most n of this wave's requests outstanding (n: a sum of up to three slots' counts)
+__device__ __forceinline__ void ds_wait(int n) {
+  switch (n) {
+    case 12: lg_vmcnt<12>(); break;
+    case 16: lg_vmcnt<16>(); break;
+    case 24: lg_vmcnt<24>(); break;
+    case 28: lg_vmcnt<28>(); break;
+    case 32: lg_vmcnt<32>(); break;
+    case 36: lg_vmcnt<36>(); break;
+    case 40: lg_vmcnt<40>(); break;
+    case 44: lg_vmcnt<44>(); break;
+    case 48: lg_vmcnt<48>(); break;
+    default: lg_vmcnt<0>(); break;
+  }
+}
+
+// the thread's number, opaque: what is worked out of it in one part of the step is not kept in registers through the others
+__device__ __forceinline__ int ds_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// ---- exchanges ---------------------------------------------------------------------------------------------------------
+// place of element e among a vector's words: the octets of a wave's lanes are a word apart, so that the loads that gather them are
+// whole lines (K a multiple of 512); two bf16 to a word: of word w of an octet of four
+__device__ __forceinline__ int ds_at(int e) { return (e & ~511) | ((e & 7) << 6) | ((e >> 3) & 63); }
+__device__ __forceinline__ int ds_at16(int w) { return (w & ~255) | ((w & 3) << 6) | ((w >> 2) & 63); }
+
+__device__ __forceinline__ void ds_put(uint64_t* p, uint32_t v, uint32_t no) {
+  __hip_atomic_store(p, (uint64_t)no << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t ds_get(const uint64_t* p) {
+  return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct DsClock {
+  unsigned long long t0, limit;
+  unsigned* late;
+};
+__device__ __forceinline__ bool ds_late(const DsClock& c) {
+  if (__builtin_amdgcn_s_memrealtime() - c.t0 <= c.limit) return false;
+  __hip_atomic_store(c.late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+// N words of each lane, stride apart, until all carry the number (or the time is up).  What waits must not keep the memory from
+// those it waits for (with all words asked for again and again an exchange beside a full stream took 5 us, and left it 4.5 TB/s):
+// a lane asks memory for its first word only, and for the others, which come with it, once that is there and through the XCD's L2,
+// where 32 workgroups share them.  An exchange has words of its own in each layer, so L2 holds none of an older number; one that
+// it took in too early is asked for from memory.
+template <int N>
+__device__ __forceinline__ void ds_poll(const uint64_t* p, int stride, uint32_t no, uint32_t (&v)[N], const DsClock& c) {
+  uint64_t w[N];
+  for (int it = 1;; ++it) {
+    w[0] = ds_get(p);
+    if ((uint32_t)(w[0] >> 32) == no || ((it & 63) == 0 && ds_late(c))) break;
+  }
+#pragma unroll
+  for (int i = 1; i < N; ++i) w[i] = __hip_atomic_load(const_cast<uint64_t*>(p + i * stride), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  bool ok = true;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    v[i] = (uint32_t)w[i];
+    ok = ok && (uint32_t)(w[i] >> 32) == no;
+  }
+  for (int it = 1; !ok; ++it) {
+    ok = true;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      w[i] = ds_get(p + i * stride);
+      v[i] = (uint32_t)w[i];
+      ok = ok && (uint32_t)(w[i] >> 32) == no;
+    }
+    if ((it & 63) == 0 && ds_late(c)) break;
+  }
+}
+
+struct DsLds {
+  uint8_t* ring;
+  float *rowacc, *red;  // two buffers each
+  DsJob* jobs;          // of this workgroup (the launch with all workgroups)
+  float* scale;         // of the caches, per layer
+  float* gains;         // of this workgroup's rows, per norm behind a residual
+  uint8_t* area;
+};
+
+// ---- a product's operand: gathered, multiplied by the norm's gains, quantised to int8 (gemv_q8.h) ------------------------
+// one octet to int8 codes in chunk order and {dx, dx * sum of codes} per 16 (q8_octet of gemv_q8.h; the codes rounded by
+// the addition of a number whose last place is 1, and their low bytes put together: a fifth of its instructions)
+__device__ __forceinline__ void ds_octet(int o, float (&v)[8], int8_t* xq, float2* ms) {
+  float am = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(v[i]));
+  am = fmaxf(am, dpp_xor1(am));
+  am = fmaxf(am, dpp_xor2(am));
+  const float dx = am * (1.f / 127.f), inv = am > 0.f ? 127.f / am : 0.f;
+  uint32_t w[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    uint32_t t[4];  // 1.5 * 2^23 + the code
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = __float_as_uint(fmaf(v[4 * j + e], inv, 12582912.f));
+    w[j] = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0400u) | __builtin_amdgcn_perm(t[3], t[2], 0x04000c0cu);
+  }
+  int sum = __builtin_amdgcn_sdot4((int)w[0], 0x01010101, __builtin_amdgcn_sdot4((int)w[1], 0x01010101, 0, false), false);
+  sum += dpp_xor1_i(sum);  // the other octet of this 16-run
+  const int quarter = o & 3;
+  int c, s0;
+  QFmt<QT_Q4_K>::run_pos(2 * (o >> 2) + (quarter >> 1), c, s0);
+  const int piece = ((s0 >> 4) + (c >> 3)) & 1;
+  *(uint2*)(xq + c * 32 + 16 * piece + 8 * (quarter & 1)) = make_uint2(w[0], w[1]);
+  if (!(quarter & 1)) ms[c * 2 + (s0 >> 4)] = make_float2(dx, dx * (float)sum);
+}
+
+// IN_X: plain values x and gains, the sum of squares to red; IN_F32: the exchange's values (multiplied by the gains where a norm is in
+// front); IN_BF16: pairs
+enum { IN_X, IN_F32, IN_BF16 };
+template <int IN>
+__device__ __forceinline__ void ds_stage(const float* x, const uint64_t* ex, uint32_t no, int K, const float* gain, int8_t* xq, float2* ms,
+                                         float* red, const DsClock& clk) {
+  const int tid = ds_tid(), noct = K >> 3;
+  constexpr int NW = IN == IN_BF16 ? 4 : 8;
+  float ssq = 0.f;
+  // (whole waves: K is a multiple of 512, a wave takes 512 elements)
+#pragma clang loop unroll(disable)
+  for (int o = tid; o < noct; o += DS_CT) {
+    float v[8];
+    if constexpr (IN == IN_X) {
+      const float4 f0 = *(const float4*)(x + 8 * o), f1 = *(const float4*)(x + 8 * o + 4);
+      const float4 g0 = *(const float4*)(gain + 8 * o), g1 = *(const float4*)(gain + 8 * o + 4);
+      const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w}, g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        ssq = fmaf(f[i], f[i], ssq);
+        v[i] = f[i] * g[i];
+      }
+    } else {
+      uint32_t w[NW];
+      ds_poll<NW>(ex + (size_t)(o >> 6) * (NW * 64) + (o & 63), 64, no, w, clk);
+      if constexpr (IN == IN_BF16) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v[2 * i] = __uint_as_float(w[i] << 16);
+          v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(w[i]);
+      }
+    }
+    ds_octet(o, v, xq, ms);
+  }
+  if constexpr (IN == IN_X) {
+    const float t = wave_sum(ssq);
+    if ((tid & 63) == 0) red[tid >> 6] = t;
+  }
+}
+
+// the sum of squares of the residual: a word of each workgroup, gathered by the last waves
+__device__ __forceinline__ void ds_squares(const DsArgs& a, const uint64_t* ex, uint32_t no, float* red, const DsClock& clk) {
+  const int tid = ds_tid();
+  float v = 0.f;
+#pragma clang loop unroll(disable)
+  for (int i = DS_CT - 1 - tid; i < a.parts; i += DS_CT) {
+    uint32_t w[1];
+    ds_poll<1>(ex + i, 0, no, w, clk);
+    v += __uint_as_float(w[0]);
+  }
+  const float t = wave_sum(v);
+  if ((tid & 63) == 0) red[tid >> 6] = t;
+}
+
+// sum over the first n = 8, 16, 32 or 64 lanes of every n
+__device__ __forceinline__ float ds_lanes(float v, int n) {
+  v = lanes_sum<8>(v);
+  if (n > 8) v += lane_dpp<0x140>(v);
+  if (n > 16) v = lane_xor16(v, LaneAdd{});
+  if (n > 32) v = lane_xor32(v, LaneAdd{});
+  return v;
+}
+
+__device__ __forceinline__ void ds_add(float* p, float v) {
+  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// one slot after the other against the staged operand; row sums in LDS.  A barrier behind each slot (or one)
+template <int QT>
+__device__ __forceinline__ void ds_dot(const DsJob& j, int nch, int run, int& slot, const DsLds& s, const int8_t* xq, const float2* ms,
+                                       float* acc, float* acc_next, int row_sums) {
+  using F = DsFmt<QT>;
+  const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // this lane's (pair of) chunk(s): place within the slot, and its row and column, which advance by a slot's chunks
+  const int at = F::PAIRS ? 2 * tid : tid;
+  int row = at / nch, c = at - row * nch;
+  const int drow = F::CH / nch, dc = F::CH - drow * nch;
+  const int wfirst = F::PAIRS ? 128 * wave : 64 * wave;
+  const bool same = dc == 0;  // the same columns in every slot: the operand stays in registers
+  Q4PairX X;
+  int xv[8];
+  float4 m;
+  auto load = [&]() __attribute__((always_inline)) {
+    if constexpr (F::PAIRS) {
+      q4p_load_x(xq, ms, c, X);
+    } else {
+      const int8_t* xc = xq + (size_t)c * 32;
+      const int rot = (c >> 3) & 1;
+      const uint4 p0 = *(const uint4*)(xc + 16 * rot), p1 = *(const uint4*)(xc + 16 * (rot ^ 1));
+      xv[0] = p0.x; xv[1] = p0.y; xv[2] = p0.z; xv[3] = p0.w;
+      xv[4] = p1.x; xv[5] = p1.y; xv[6] = p1.z; xv[7] = p1.w;
+      m = *(const float4*)(ms + (size_t)c * 2);
+    }
+  };
+  auto one = [&](const uint8_t* sl) __attribute__((always_inline)) {
+    float v;
+    if constexpr (F::PAIRS) {
+      const uint4 a0 = *(const uint4*)(sl + F::off[0] + at * 16), a1 = *(const uint4*)(sl + F::off[0] + at * 16 + 16);
+      const uint4 mt = *(const uint4*)(sl + F::off[1] + (at >> 3) * 16);
+      v = q4p_dot(a0, a1, mt, (c >> 1) & 3, X);
+    } else {
+      RawChunk r;
+      r.a = *(const uint4*)(sl + F::off[0] + at * 16);
+      const uint2 h = *(const uint2*)(sl + F::off[1] + at * 8);
+      r.b.x = h.x;
+      r.b.y = h.y;
+      r.c.x = *(const uint16_t*)(sl + F::off[2] + at * 2);
+      r.d = *(const uint16_t*)(sl + F::off[3] + (at >> 3) * 2);
+      float sc[2], of[2];
+      q8_scales_bf<QT>(r, c, sc, of);
+      int is[2];
+      QDot<QT>::isums(r, c, xv, is);
+      v = sc[0] * m.x * (float)is[0] - of[0] * m.y + sc[1] * m.z * (float)is[1] - of[1] * m.w;
+    }
+    v = ds_lanes(row < j.nrows ? v : 0.f, run);
+    if ((lane & (run - 1)) == 0 && row < j.nrows) ds_add(acc + row, v);
+  };
+  for (int i = tid; i < row_sums; i += DS_CT) acc_next[i] = 0.f;
+  if (same && j.slots) load();
+#pragma clang loop unroll(disable)
+  for (int t = 0; t < j.slots; ++t) {
+    if (t * F::CH + wfirst < j.chunks) {
+      if (!same) load();
+      one(s.ring + (size_t)((slot + t) % DS_R) * DS_SLOT);
+    }
+    row += drow;
+    c += dc;
+    if (c >= nch) {
+      c -= nch;
+      ++row;
+    }
+    if (t + 1 < j.slots) lg_barrier();
+  }
+  slot += j.slots;
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();
+}
+
+// tiles of keys that a wave has in flight (a request is 1 KB, of fp8 512 B), keys of a workgroup's pass
+template <int HD, bool F8>
+constexpr int ds_tiles() { return 1; }
+template <int HD, bool F8>
+constexpr int ds_pass() { return ds_tiles<HD, F8>() * DS_AW * 4 * (512 / HD); }
+
+// ---- attention -----------------------------------------------------------------------------------------------------------
+// G query heads of one KV head over the passes sp, sp + P, .. of its keys (attn_lanes of attn_decode.h, with the heads sharing what is
+// read); the row's own key is taken from the exchange, as the cache will hold it.
+// Four barriers.  LDS: queries in bf16, the own key and value as cached, the raw vectors and then the waves' results.
+template <int HD, int G, bool F8>
+struct DsAttnLds {
+  uint16_t q[G][HD];
+  uint16_t own[2][HD];  // (fp8: bytes)
+  float m[DS_AW][G], l[DS_AW][G];
+  union {
+    float vec[G + 2][HD];
+    float o[DS_AW][G][HD];
+  };
+};
+
+template <int HD, int G, bool F8>
+__device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P, int pos, uint32_t no, float2 cs, const DsLds& s,
+                                          const DsClock& clk) {
+  using S = DsAttnLds<HD, G, F8>;
+  S& L = *(S*)s.area;
+  constexpr int LPK = HD / 8, KPS = 64 / LPK;  // lanes of a key (8 elements each), keys of a request
+  constexpr int STEPS = 4, KPW = STEPS * KPS;  // requests of a tile, its keys
+  constexpr int NT = ds_tiles<HD, F8>(), PASS = ds_pass<HD, F8>(), ES = F8 ? 1 : 2;
+  using KVT = typename std::conditional<F8, uint2, uint4>::type;
+  const int units = a.n_heads / G;
+  const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (wg >= units * P) {
+    lg_barrier();
+    lg_barrier();
+    lg_barrier();
+    lg_barrier();
+    return;
+  }
+  // one head a workgroup: the heads of a KV head on one XCD (workgroups go round the eight in turn)
+  const int unit = P > 1 ? wg / P : ((units & 7) == 0 ? (wg & 7) * (units >> 3) + (wg >> 3) : wg), sp = P > 1 ? wg - unit * P : 0;
+  const int h0 = unit * G, gq = a.n_heads / a.n_kv_heads, kvh = h0 / gq;
+  const int ksub = lane / LPK, dsl = lane % LPK;
+  uint8_t *kc = a.kc + (size_t)l * a.kv_layer, *vc = a.vc + (size_t)l * a.kv_layer;
+  KVT kr[NT][STEPS], vr[NT][STEPS];
+  auto first_key = [&](int pass, int t) { return pass * PASS + t * (DS_AW * KPW) + wave * KPW; };
+  // a tile is a buffer of its live keys' bytes: what lies behind them reads as zeros without a memory access
+  const int voff = (ksub * HD + dsl * 8) * ES;
+  auto request = [&](KVT (&r)[STEPS], const uint8_t* pool, int k0) __attribute__((always_inline)) {
+    const int blk = ds_table(a.blocks, min(k0 / KV_BLOCK, a.max_ctx / KV_BLOCK - 1));
+    const int live = __builtin_amdgcn_readfirstlane(min(max(pos - k0, 0), KPW));
+    const auto rs = uniform_rsrc(pool + (((size_t)blk * a.n_kv_heads + kvh) * KV_BLOCK + (k0 % KV_BLOCK)) * HD * ES, live * HD * ES);
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      if constexpr (F8) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, voff + i * KPS * HD * ES, 0, 0);
+        r[i] = make_uint2(v[0], v[1]);
+      } else {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff + i * KPS * HD * ES, 0, 0);
+        r[i] = make_uint4(v[0], v[1], v[2], v[3]);
+      }
+    }
+  };
+  const int npass = pos / PASS + 1;
+  if (wave < DS_AW) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      request(kr[t], kc, first_key(sp, t));
+      request(vr[t], vc, first_key(sp, t));
+    }
+  }
+  // ---- the heads' raw vectors
+  if (tid < (G + 2) * HD) {
+    const int v = tid / HD, i = tid - v * HD;
+    const int row = v < G ? (h0 + v) * HD + i : (a.n_heads + (v == G ? kvh : a.n_kv_heads + kvh)) * HD + i;
+    const float b = a.bias ? a.bias[(size_t)l * a.nqkv + row] : 0.f;
+    uint32_t w[1];
+    ds_poll<1>(a.qkv + (size_t)l * a.nqkv + row, 0, no, w, clk);
+    L.vec[v][i] = __uint_as_float(w[0]) + b;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();
+  if (wave < G + 2) {
+    constexpr int HALF = HD / 2;
+    const int p = lane & (HALF - 1);  // (heads of 64: lanes 32 up repeat the lower ones)
+    const bool isq = wave < G, isv = wave == G + 1;
+    const bool neox = a.rope_neox && !isv;
+    const int ia = neox ? p : 2 * p, ib = neox ? p + HALF : 2 * p + 1;
+    float v0 = L.vec[wave][ia], v1 = L.vec[wave][ib];
+    if (!isv) {
+      if (a.qk_gains) {
+        const float* g = a.qk_gains + (size_t)(2 * l + !isq) * HD;
+        const float inv = rsqrtf(lanes_sum<HALF>(v0 * v0 + v1 * v1) / (float)HD + a.eps);
+        v0 *= inv * g[ia];
+        v1 *= inv * g[ib];
+      }
+      const float o0 = v0 * cs.x - v1 * cs.y, o1 = v0 * cs.y + v1 * cs.x;
+      v0 = o0;
+      v1 = o1;
+    }
+    if (lane < HALF) {
+      if (isq) {
+        const float qs = a.scale * kLog2e * (F8 ? s.scale[2 * l] : 1.f);  // scores in the log2 domain
+        const uint32_t u = pk_bf16(v0 * qs, v1 * qs);
+        L.q[wave][ia] = (uint16_t)u;
+        L.q[wave][ib] = (uint16_t)(u >> 16);
+      } else {
+        const float inv = F8 ? 1.f / (isv ? s.scale[2 * l + 1] : s.scale[2 * l]) : 1.f;
+        kv_store_pair((bf16_t*)L.own[isv], ia, ib, v0, v1, F8, inv);
+        if (sp == 0 && h0 % gq == 0) {  // one workgroup a KV head keeps it
+          const size_t i0 = (((size_t)ds_table(a.blocks, pos / KV_BLOCK) * a.n_kv_heads + kvh) * KV_BLOCK + pos % KV_BLOCK) * HD;
+          kv_store_pair((bf16_t*)(isv ? vc : kc), i0 + ia, i0 + ib, v0, v1, F8, inv);
+        }
+      }
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();
+  if (wave < DS_AW) {
+    uint4 q[G];  // (read for each tile: kept through the loop they spill)
+    auto read_q = [&]() __attribute__((always_inline)) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int g = 0; g < G; ++g) q[g] = *(const uint4*)&L.q[g][dsl * 8];
+    };
+    float m[G], sum[G], o[G][8];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      m[g] = kNeg;
+      sum[g] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[g][i] = 0.f;
+    }
+    auto score = [&](const KVT& r, float (&sc)[G], bool live) __attribute__((always_inline)) {
+      uint32_t kb[4];
+      if constexpr (F8) {
+        kb[0] = fp8x2_bf16x2<false>(r.x); kb[1] = fp8x2_bf16x2<true>(r.x);
+        kb[2] = fp8x2_bf16x2<false>(r.y); kb[3] = fp8x2_bf16x2<true>(r.y);
+      } else {
+        kb[0] = r.x; kb[1] = r.y; kb[2] = r.z; kb[3] = r.w;
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        float d = dot2_bf16(kb[0], q[g].x, 0.f);
+        d = dot2_bf16(kb[1], q[g].y, d);
+        d = dot2_bf16(kb[2], q[g].z, d);
+        d = dot2_bf16(kb[3], q[g].w, d);
+        d = lanes_sum<LPK>(d);
+        sc[g] = live ? d : kNeg;
+      }
+    };
+    auto weigh = [&](float mx, int g) __attribute__((always_inline)) {  // a head's running max, at least mx
+      const float mn = fmaxf(m[g], mx);
+      if (__builtin_amdgcn_ballot_w64(mn > m[g])) {
+        const float alpha = fast_exp2(m[g] - mn);
+        sum[g] *= alpha;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[g][i] *= alpha;
+        m[g] = mn;
+      }
+    };
+    auto add = [&](const KVT& r, const float (&p)[G]) __attribute__((always_inline)) {
+      float vf[8];
+      if constexpr (F8) {
+        const gf32x2 f0 = fp8x2_f32x2<false>(r.x), f1 = fp8x2_f32x2<true>(r.x), f2 = fp8x2_f32x2<false>(r.y), f3 = fp8x2_f32x2<true>(r.y);
+        vf[0] = f0.x; vf[1] = f0.y; vf[2] = f1.x; vf[3] = f1.y;
+        vf[4] = f2.x; vf[5] = f2.y; vf[6] = f3.x; vf[7] = f3.y;
+      } else {
+        const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          vf[2 * e] = __uint_as_float(w[e] << 16);
+          vf[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[g][e] = fmaf(p[g], vf[e], o[g][e]);
+    };
+    for (int pass = sp; pass < npass; pass += P) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int k0 = first_key(pass, t), kn = first_key(pass + P, t);
+        float sc[STEPS][G];
+        read_q();
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+          score(kr[t][i], sc[i], k0 + ksub + i * KPS < pos);
+          __builtin_amdgcn_sched_barrier(0);  // (steps interleaved spill)
+        }
+        if (pass + P < npass) request(kr[t], kc, kn);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          float mx = sc[0][g];
+#pragma unroll
+          for (int i = 1; i < STEPS; ++i) mx = fmaxf(mx, sc[i][g]);
+          weigh(mx, g);
+#pragma unroll
+          for (int i = 0; i < STEPS; ++i) {
+            sc[i][g] = fast_exp2(sc[i][g] - m[g]);
+            sum[g] += sc[i][g];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+          add(vr[t][i], sc[i]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (pass + P < npass) request(vr[t], vc, kn);
+      }
+    }
+    if (wave == 0 && sp == 0) {  // the row's own key, by the first key group
+      float sc[G];
+      read_q();
+      score(*(const KVT*)((const uint8_t*)L.own[0] + dsl * 8 * ES), sc, ksub == 0);
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        weigh(sc[g], g);
+        sc[g] = fast_exp2(sc[g] - m[g]);
+        sum[g] += sc[g];
+      }
+      if (ksub) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) sc[g] = 0.f;
+      }
+      add(*(const KVT*)((const uint8_t*)L.own[1] + dsl * 8 * ES), sc);
+    }
+    // the key groups of a wave, then (below) the waves
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const float M = keys_max<LPK>(m[g]), w = fast_exp2(m[g] - M);
+      const float S1 = keys_sum<LPK>(sum[g] * w);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[g][e] = keys_sum<LPK>(o[g][e] * w);
+      if (ksub == 0) {
+        float4* dst = (float4*)&L.o[wave][g][dsl * 8];
+        dst[0] = make_float4(o[g][0], o[g][1], o[g][2], o[g][3]);
+        dst[1] = make_float4(o[g][4], o[g][5], o[g][6], o[g][7]);
+      }
+      if (lane == 0) {
+        L.m[wave][g] = M;
+        L.l[wave][g] = S1;
+      }
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();
+  if (tid < G * HD) {
+    const int g = tid / HD, d = tid - g * HD;
+    float W = L.m[0][g];
+#pragma unroll
+    for (int w = 1; w < DS_AW; ++w) W = fmaxf(W, L.m[w][g]);
+    float S1 = 0.f, acc = 0.f;
+#pragma unroll
+    for (int w = 0; w < DS_AW; ++w) {
+      const float f = fast_exp2(L.m[w][g] - W);
+      S1 += f * L.l[w][g];
+      acc += f * L.o[w][g][d];
+    }
+    if (F8) acc *= s.scale[2 * l + 1];
+    if (P == 1) {
+      ds_put(a.attn + (size_t)l * a.n_heads * HD + ds_at((h0 + g) * HD + d), __float_as_uint(acc / S1), no);
+    } else {
+      uint64_t* p = a.part + ((size_t)(h0 + g) * DS_PMAX + sp) * (HD + 2);
+      ds_put(p + d, __float_as_uint(acc), no);
+      if (d < 2) ds_put(p + HD + d, __float_as_uint(d ? S1 : W), no);
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();  // (the area is the next operand's)
+}
+
+// the runs of a head's keys together: 16 elements of a head at a time.  Two barriers.
+template <int HD>
+__device__ __forceinline__ void ds_combine(const DsArgs& a, int l, int unit, int P, uint32_t no, const DsLds& s, const DsClock& clk) {
+  const int tid = ds_tid(), h = unit / (HD / 16), d0 = unit % (HD / 16) * 16;
+  float* v = (float*)s.area;  // [P][18]
+  const bool on = unit < a.n_heads * (HD / 16);
+  if (on && tid < P * 18) {
+    const int sp = tid / 18, j = tid - sp * 18;
+    uint32_t w[1];
+    ds_poll<1>(a.part + ((size_t)h * DS_PMAX + sp) * (HD + 2) + (j < 16 ? d0 + j : HD + j - 16), 0, no, w, clk);
+    v[tid] = __uint_as_float(w[0]);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();
+  if (on && tid < 16) {
+    float W = v[16];
+    for (int p = 1; p < P; ++p) W = fmaxf(W, v[p * 18 + 16]);
+    float S1 = 0.f, acc = 0.f;
+    for (int p = 0; p < P; ++p) {
+      const float f = fast_exp2(v[p * 18 + 16] - W);
+      S1 += f * v[p * 18 + 17];
+      acc += f * v[p * 18 + tid];
+    }
+    ds_put(a.attn + (size_t)l * a.n_heads * HD + ds_at(h * HD + d0 + tid), __float_as_uint(acc / S1), no);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();
+}
+
+// ---- the step ---------------------------------------------------------------------------------------------------------------
+// keys up to which a head has one workgroup (as attn_lanes), and how many workgroups share the others
+template <int HD, bool F8>
+__device__ __forceinline__ int ds_runs(const DsArgs& a, int G, int pos) {
+  if (pos < ATTN_SPLIT_LEN) return 1;
+  return min(min(pos / ds_pass<HD, F8>() + 1, a.parts / (a.n_heads / G)), DS_PMAX);
+}
+
+template <int HD, int G, bool F8>
+__global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  if (a.alone && !a.ctl->failed) return;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int first = blockIdx.x, step = gridDim.x;  // (parts of this workgroup: one, or all of them in turn)
+  DsLds s;
+  s.ring = smem;
+  s.area = smem + DS_R * DS_SLOT;
+  s.rowacc = (float*)(s.area + a.area_bytes);
+  s.red = s.rowacc + 2 * a.row_sums;
+  unsigned* gate = (unsigned*)(s.red + 32);
+  s.scale = s.red + 36;
+  s.jobs = (DsJob*)(s.scale + (2 * a.n_layers + 3) / 4 * 4);
+  s.gains = (float*)(s.jobs + 4 * a.n_layers + 1);
+  const int qd = a.n_heads * HD, pos = min(ds_table(a.pos, 0), a.max_ctx - 1);
+  const bool brief = pos < ATTN_SPLIT_LEN;
+  const int P = ds_runs<HD, F8>(a, G, pos);
+  const int nattend = brief ? a.n_heads : a.n_heads / G * P;  // parts that attend
+  const int ncomb = (a.n_heads * (HD / 16) + a.parts - 1) / a.parts;
+
+  if (wave >= DS_NG) {
+    // ---- loaders: the step's slots in order, as many ahead as the ring holds; they pass every barrier of the others
+    const int lw = wave - DS_NG;
+    const int last = 4 * a.n_layers;
+    int iq = 0, iw = first, is = 0, at = 0;  // next slot: product, part, slot of it; ring place
+    int h0 = 0, h1 = 0, h2 = 0;              // requests of the last three slots
+    DsCopy J = ds_table(a.jobs, first), N;              // the job being requested, the one after it
+    auto after = [&]() {
+      if ((iw += step) >= a.parts) {
+        iw = first;
+        ++iq;
+      }
+      N = ds_table(a.jobs, min(iq, last) * a.parts + iw);
+    };
+    after();
+    bool more = true;
+    auto issue = [&]() {
+      h2 = h1;
+      h1 = h0;
+      h0 = 0;
+      while (more && is >= J.job.slots) {
+        is = 0;
+        more = iq <= last;
+        J = N;
+        after();
+      }
+      if (!more) return;
+      uint8_t* dst = s.ring + (size_t)(at % DS_R) * DS_SLOT;
+      if (J.job.chunks & DS_Q6) {
+        ds_copy<QT_Q6_K>(J, is, dst, lw);
+        h0 = DsFmt<QT_Q6_K>::per_loader;
+      } else {
+        ds_copy<QT_Q4_K>(J, is, dst, lw);
+        h0 = DsFmt<QT_Q4_K>::per_loader;
+      }
+      ++is;
+      ++at;
+    };
+    for (int i = 0; i < DS_R; ++i) issue();
+    lg_barrier();  // the gate's answer
+    unsigned go;
+    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                 : "=v"(go)
+                 : "v"((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) unsigned*)gate)
+                 : "memory");
+    if (__builtin_amdgcn_readfirstlane(go) != 1) {
+      lg_vmcnt<0>();
+      return;
+    }
+    int slots = ds_table(&a.jobs->job.slots, first * 16);  // of the product that the others are at
+    // The slot that a product's end leaves free is asked for when the next operand is staged: a CU's loads return in order, and those
+    // that gather the operand would wait for it.  Workgroups that don't attend ask for it right away.
+    bool owed = false;
+    auto pass = [&](int q) {
+      for (int wg = first; wg < a.parts; wg += step) {
+        const int n = slots;
+        const bool wrap = wg + step >= a.parts;
+        slots = ds_table(&a.jobs->job.slots, (min(q + wrap, last) * a.parts + (wrap ? first : wg + step)) * 16);
+        if (!n) lg_barrier();
+        for (int t = 0; t < n; ++t) {
+          ds_wait(t || owed ? h0 + h1 : h0 + h1 + h2);
+          lg_barrier();
+          if (t || owed) issue();
+          owed = false;
+        }
+        lg_barrier();
+        if (n) owed = true;
+      }
+    };
+#pragma clang loop unroll(disable)
+    for (int q = 0; q <= last; ++q) {
+      if ((q & 3) == DS_O) {
+        int n = 4;
+        if (P > 1) n += 2 * ncomb;
+        if (owed && first >= nattend) {
+          issue();
+          owed = false;
+        }
+        for (int wg = first; wg < a.parts; wg += step)
+          for (int i = 0; i < n; ++i) lg_barrier();
+      }
+      pass(q);
+    }
+    return;
+  }
+
+  // ---- sign in, wait for the others
+  DsCtl* ctl = a.ctl;
+  DsClock clk{__builtin_amdgcn_s_memrealtime(), a.wait_ticks, &ctl->late};
+  if (tid == 0) {
+    unsigned go = 1;
+    const unsigned no = __hip_atomic_load(&ctl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!a.alone) {
+      if (__hip_atomic_fetch_add(&ctl->arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x) {
+        unsigned want = 0;
+        __hip_atomic_compare_exchange_strong(&ctl->state, &want, 1u, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      while ((go = __hip_atomic_load(&ctl->state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0) {
+        if (__builtin_amdgcn_s_memrealtime() - clk.t0 > a.gate_ticks) {
+          unsigned want = 0;
+          __hip_atomic_compare_exchange_strong(&ctl->state, &want, 2u, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+    }
+    gate[0] = go;
+    gate[1] = no;
+  }
+  for (int i = tid; i < 2 * a.row_sums + 32; i += DS_CT) s.rowacc[i] = 0.f;
+  for (int i = tid; i < 2 * a.n_layers; i += DS_CT) s.scale[i] = a.kv_scale[i];
+  for (int i = tid; i <= 4 * a.n_layers; i += DS_CT) s.jobs[i] = a.jobs[(size_t)i * a.parts + first].job;
+  {
+    const int r0 = a.jobs[(size_t)DS_O * a.parts + first].job.r0;
+    for (int i = tid; i < 2 * a.n_layers * a.own_rows; i += DS_CT) {
+      const int n = i / a.own_rows, r = i - n * a.own_rows;
+      s.gains[i] = a.gains[(size_t)(n + 1) * a.d + min(r0 + r, a.d - 1)];
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();
+  const bool go = __builtin_amdgcn_readfirstlane(gate[0]) == 1;
+  const uint32_t no0 = __builtin_amdgcn_readfirstlane(gate[1]) + 1;
+
+  if (go) {
+    int8_t* xq = (int8_t*)s.area;
+    int slot = 0, par = 0;
+    const float2 rope = a.rope_cs[(size_t)pos * (HD / 2) + (tid & (HD / 2 - 1))];  // of the lane's pair, in every layer
+    const int last = 4 * a.n_layers;
+    // the residual at this thread's row (of O and of down alike, in reverse order of the threads)
+    float own = 0.f;
+    if (!a.alone && DS_CT - 1 - tid < s.jobs[DS_O].nrows) own = a.x[s.jobs[DS_O].r0 + DS_CT - 1 - tid];
+    // one product after the other, with the attention in front of O's; the code of all of them is one (what a layer runs
+    // through stays in the instruction cache)
+#pragma clang loop unroll(disable)
+    for (int q = 0; q <= last; ++q) {
+      const int l = q >> 2, kind = q & 3;
+      const uint32_t no = no0 + l;
+      if (kind == DS_O) {
+        for (int wg = first; wg < a.parts; wg += step) {
+          if (brief) ds_attend<HD, 1, F8>(a, l, wg, 1, pos, no, rope, s, clk);
+          else ds_attend<HD, G, F8>(a, l, wg, P, pos, no, rope, s, clk);
+        }
+        if (P > 1)
+          for (int wg = first; wg < a.parts; wg += step)
+            for (int i = 0; i < ncomb; ++i) ds_combine<HD>(a, l, wg + i * a.parts, P, no, s, clk);
+      }
+#pragma clang loop unroll(disable)
+      for (int wg = first; wg < a.parts; wg += step) {
+        // (results are written, and the residual they are added to read, by the last waves: a wave's loads are counted behind
+        // its stores, and the first ones have the next operand to wait for)
+        const int tid = ds_tid(), rt = DS_CT - 1 - tid;
+        const DsJob job = a.alone ? ds_table(a.jobs, q * a.parts + wg).job : s.jobs[q];
+        DsJob j;
+        j.r0 = __builtin_amdgcn_readfirstlane(job.r0);
+        j.nrows = __builtin_amdgcn_readfirstlane(job.nrows);
+        j.chunks = __builtin_amdgcn_readfirstlane(job.chunks);
+        j.slots = __builtin_amdgcn_readfirstlane(job.slots);
+        const bool q6 = j.chunks & DS_Q6;
+        j.chunks &= ~DS_Q6;
+        const int K = kind == DS_O ? qd : (kind == DS_DOWN ? a.ff : a.d), nch = K >> 5;
+        float2* ms = (float2*)(xq + K);
+        float* acc = s.rowacc + par * a.row_sums;
+        float* red = s.red + par * 16;
+        par ^= 1;
+        const bool resid = kind == DS_O || kind == DS_DOWN;
+        const int nr = kind == DS_O ? 2 * l : kind == DS_GU ? 2 * l : kind == DS_DOWN ? 2 * l + 1 : 2 * l - 1;  // the residual it makes or reads
+        if (a.alone && resid && rt < j.nrows) {
+          own = nr ? __hip_atomic_load(a.resid + j.r0 + rt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.x[j.r0 + rt];
+          asm volatile("" : "+v"(own));  // (waited for here)
+        }
+        if (kind == DS_DOWN) {
+          ds_stage<IN_BF16>(nullptr, a.h + (size_t)l * (a.ff / 2), no, K, nullptr, xq, ms, red, clk);
+        } else if (q == 0) {
+          ds_stage<IN_X>(a.x, nullptr, 0, K, a.gains, xq, ms, red, clk);
+        } else {
+          const uint32_t nx = kind == DS_QKV ? no - 1 : no;
+          ds_stage<IN_F32>(nullptr, kind == DS_O ? a.attn + (size_t)l * qd : a.xn + (size_t)nr * a.d, nx, K, nullptr, xq, ms, red, clk);
+          if (kind != DS_O) ds_squares(a, a.sq + (size_t)nr * a.parts, nx, red, clk);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        lg_barrier();  // the operand is staged, slot 0 there
+        float inv = 1.f;
+        if (!resid) {
+          float t = 0.f;
+#pragma unroll
+          for (int w = 0; w < DS_NG; ++w) t += red[w];
+          inv = rsqrtf(t / (float)K + a.eps);
+        }
+        const int low = nch & -nch;  // (the largest power of two in it: lanes that share a row)
+        if (q6) ds_dot<QT_Q6_K>(j, nch, min(low, 64), slot, s, xq, ms, acc, s.rowacc + par * a.row_sums, a.row_sums);
+        else ds_dot<QT_Q4_K>(j, nch, min(low >> 1, 64), slot, s, xq, ms, acc, s.rowacc + par * a.row_sums, a.row_sums);
+        if (resid) {
+          // (rows by the last wave's lanes, further ones by those before; the squares go with the first word)
+          const bool on = rt < j.nrows;
+          const float x = on ? own + acc[rt] : 0.f;
+          float gain = s.gains[nr * a.own_rows + min(rt, a.own_rows - 1)];
+          if (a.alone) {
+            gain = a.gains[(size_t)(nr + 1) * a.d + j.r0 + (on ? rt : 0)];
+            asm volatile("" : "+v"(gain));
+          }
+          own = x;
+          if (on) {
+            ds_put(a.xn + (size_t)nr * a.d + ds_at(j.r0 + rt), __float_as_uint(x * gain), no);
+            if (a.alone) __hip_atomic_store(a.resid + j.r0 + rt, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+          const float sq = wave_sum(x * x);
+          if (tid == DS_CT - 1) ds_put(a.sq + (size_t)nr * a.parts + wg, __float_as_uint(sq), no);
+        } else {
+          if (q == last) {
+            for (int r = rt; r < j.nrows; r += DS_CT) a.logits[j.r0 + r] = acc[r] * inv;
+          } else if (kind == DS_QKV) {
+            for (int r = rt; r < j.nrows; r += DS_CT) ds_put(a.qkv + (size_t)l * a.nqkv + j.r0 + r, __float_as_uint(acc[r] * inv), no);
+          } else {
+            for (int u = rt; u < j.nrows >> 2; u += DS_CT) {
+              const float4 v = *(const float4*)(acc + 4 * u);
+              const float f0 = glu_act(v.x * inv, ACT_SILU) * (v.y * inv), f1 = glu_act(v.z * inv, ACT_SILU) * (v.w * inv);
+              ds_put(a.h + (size_t)l * (a.ff / 2) + ds_at16((j.r0 >> 2) + u), (uint32_t)f32_to_bf16(f0) | (uint32_t)f32_to_bf16(f1) << 16, no);
+            }
+          }
+        }
+      }
+    }
+  }
+  // ---- sign out; the last one clears the gate and says whether the step is done
+  if (tid == 0) {
+    if (__hip_atomic_fetch_add(&ctl->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x) {
+      const unsigned late = __hip_atomic_load(&ctl->late, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      ctl->arrive = 0;
+      ctl->state = 0;
+      ctl->done = 0;
+      ctl->late = 0;
+      ctl->epoch = no0 - 1 + a.n_layers;
+      ctl->failed = !a.alone && (!go || late);
+      if (a.alone) __hip_atomic_store(a.host_failed, ++ctl->alone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+}
+
+int ds_lds(const DsArgs& a) {
+  return DS_R * DS_SLOT + a.area_bytes + (2 * a.row_sums + 32 + 4 + (2 * a.n_layers + 3) / 4 * 4) * 4 + (4 * a.n_layers + 1) * (int)sizeof(DsJob) +
+         2 * a.n_layers * a.own_rows * 4;
+}
+
+template <int HD, int G, bool F8>
+void ds_launch(DsArgs a, hipStream_t st) {
+  const int lds = ds_lds(a);
+  auto* k = decode_stream_kernel<HD, G, F8>;
+  static const hipError_t set = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  HIP_CHECK(set);
+  a.alone = 0;
+  hipLaunchKernelGGL(k, dim3(a.parts), dim3(DS_THREADS), lds, st, a);
+  a.alone = 1;
+  a.wait_ticks = ~0ull;
+  hipLaunchKernelGGL(k, dim3(1), dim3(DS_THREADS), lds, st, a);
+  HIP_CHECK(hipGetLastError());
+}
+
+template <int HD, bool F8>
+void ds_heads(const DsArgs& a, hipStream_t st) {
+  const int g = a.n_heads / a.n_kv_heads;
+  if (g % 4 == 0) ds_launch<HD, 4, F8>(a, st);
+  else if (g == 2) ds_launch<HD, 2, F8>(a, st);
+  else ds_launch<HD, 1, F8>(a, st);
+}
+
+}  // namespace
+
+DsCopy ds_job(const QWeight& w, int r0, int nrows, int row0) {
+  const size_t nch = w.cols / 32, c = (size_t)r0 * nch;
+  const bool q6 = w.qtype == QT_Q6_K;
+  const int chunks = (int)(nrows * nch), ch = q6 ? DsFmt<QT_Q6_K>::CH : DsFmt<QT_Q4_K>::CH;
+  DsCopy j{};
+  j.p[0] = w.p0 + c * 16;
+  j.p[1] = w.p1 + (q6 ? c * 8 : c * 2);
+  j.p[2] = q6 ? w.p2 + c * 2 : w.p0;
+  j.p[3] = q6 ? w.p3 + c / 4 : w.p0;
+  j.job = {row0 + r0, nrows, chunks | (q6 ? DS_Q6 : 0), (chunks + ch - 1) / ch};
+  return j;
+}
+
+bool ds_plan(DsArgs& a, int hd, int max_rows) {
+  const int qd = a.n_heads * hd, g = a.n_heads / a.n_kv_heads;
+  if ((hd != 64 && hd != 128) || a.n_heads % a.n_kv_heads || !(g == 1 || g == 2 || g == 4 || g == 8)) return false;
+  // whole waves of octets, rows that 16 chunks divide; every workgroup with rows of O, gate/up and down (see the exchanges above)
+  if (a.d % 512 || qd % 512 || a.ff % 512 || a.d < 2 * a.parts || a.ff / 2 < 2 * a.parts || a.n_heads > a.parts) return false;
+  a.own_rows = (a.d + a.parts - 1) / a.parts;
+  if (a.own_rows > 64) return false;  // (a wave holds a workgroup's rows of the residual)
+  const int K = std::max({a.d, qd, a.ff});
+  const int gl = g % 4 == 0 ? 4 : g;
+  const int attn = gl * hd * 2 + 2 * hd * 2 + DS_AW * gl * 2 * 4 + DS_AW * gl * hd * 4;
+  a.area_bytes = (std::max({K + K / 2, attn, DS_PMAX * 18 * 4}) + 255) / 256 * 256;
+  a.row_sums = (max_rows + 63) / 64 * 64;
+  return ds_lds(a) <= 160 * 1024;
+}
+
+void launch_decode_stream(const DsArgs& a, int hd, hipStream_t st) {
+  if (hd == 64) a.kv_fp8 ? ds_heads<64, true>(a, st) : ds_heads<64, false>(a, st);
+  else a.kv_fp8 ? ds_heads<128, true>(a, st) : ds_heads<128, false>(a, st);
+}
+
+}  // namespace aios

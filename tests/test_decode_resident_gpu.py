@@ -1,0 +1,179 @@
+"""One row's decode step as one resident launch (kernels/decode_stream.hip) against the chain of launches it stands in for."""
+import dataclasses
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+from aios_amd.models.config import get_preset
+from aios_amd.models.reference import ReferenceModel
+from aios_amd.models.synthetic import write_synthetic_gguf
+from aios_amd.runtime.loader import load_engine
+
+pytestmark = pytest.mark.gpu
+
+BASE = get_preset("test-mistral-shape")  # 1024 wide, 8 / 2 heads of 128, 2048 hidden, 1024 tokens
+SHAPES = {
+    "gqa4-128": {},
+    "gqa2-128": dict(n_kv_heads=4, vocab_size=1002),              # a head of a vocabulary that no workgroup count divides
+    "gqa8-64": dict(d_model=1536, n_heads=16, n_kv_heads=2, head_dim=64, d_ff=1536),  # rows of 48 chunks: eight lanes share one
+    "gqa4-64": dict(n_heads=16, n_kv_heads=4, head_dim=64, d_ff=2560),
+    "mha-64": dict(d_model=512, n_heads=8, n_kv_heads=8, head_dim=64, d_ff=1024, vocab_size=4098),
+    "qwen": dict(n_kv_heads=4, qk_norm=True, rope_mode=2, d_ff=3072),
+}
+# both int8-activation paths are 0.013 from 64 bits (perf/cases.py); they differ in the order of fp32 sums and in codes that this rounds
+# the other way, so by no more than the two distances together
+TOL = 0.026
+
+
+@pytest.fixture(scope="module")
+def models(tmp_path_factory):
+    d, held = tmp_path_factory.mktemp("resident"), {}
+
+    def get(name):
+        if name not in held:
+            cfg = dataclasses.replace(BASE, max_ctx=2048, **SHAPES[name])
+            held[name] = write_synthetic_gguf(str(d / f"{name}.gguf"), cfg, "Q4_K_M", seed=11)
+        return held[name]
+
+    return get
+
+
+def _engine(path, **kw):
+    eng, cfg, _ = load_engine(path, max_ctx=kw.pop("max_ctx", 2048), max_batch=2, **kw)
+    assert eng.decode_resident
+    return eng, cfg
+
+
+def _steps(eng, slot, tokens, pos):
+    out = []
+    for i, t in enumerate(tokens):
+        eng.decode([slot], [t], [pos + i])
+        out.append(np.asarray(eng.last_logits(1), np.float64).reshape(-1))
+    return np.array(out)
+
+
+def _rel(a, b):
+    return np.linalg.norm(a - b, axis=-1) / np.linalg.norm(b, axis=-1)
+
+
+# the first token, one cached key, a block's border, the border of one workgroup a head, passes of 128 and 256 keys, a last pass that
+# holds the row's own key alone
+POSITIONS = [0, 1, 127, 128, 510, 511, 512, 767, 1023, 1024, 1500]
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp8_e4m3"])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_resident_step_is_the_chains(models, shape, kv):
+    eng, cfg = _engine(models(shape), kv_dtype=kv)
+    if kv != "bf16":
+        eng.set_kv_scales([1 / 64] * (2 * cfg.n_layers))
+    rng = np.random.default_rng(3)
+    for pos in POSITIONS:
+        prompt = [int(t) for t in rng.integers(3, cfg.vocab_size, pos)]
+        tokens = [int(t) for t in rng.integers(3, cfg.vocab_size, 3)]
+        got = []
+        for slot, on in ((0, False), (1, True)):
+            eng.set_decode_resident(on)
+            eng.release_slot(slot)
+            if pos:
+                eng.prefill(slot, prompt, 0, False)
+            got.append(_steps(eng, slot, tokens, pos))
+        assert np.isfinite(got[1]).all()
+        assert _rel(got[1], got[0]).max() < TOL, (pos, _rel(got[1], got[0]))
+    assert eng.decode_resident_failed == 0
+
+
+@pytest.mark.parametrize("shape", ["gqa4-128", "gqa8-64", "qwen"])
+def test_resident_step_matches_the_reference(models, shape):
+    path = models(shape)
+    eng, cfg = _engine(path)
+    ref = ReferenceModel.from_gguf(path, kv_bf16=True, act_q8=True)
+    toks = [1] + [int(t) for t in np.random.default_rng(5).integers(3, cfg.vocab_size, 43)]
+    eng.prefill(0, toks[:40], 0, False)
+    got = torch.from_numpy(_steps(eng, 0, toks[40:], 40))
+    want = ref.forward(toks)[40:].double()
+    assert (got - want).abs().max().item() < 2e-2 * max(want.abs().max().item(), 1.0)
+
+
+def test_pipelined_and_looped_steps_are_resident_too(models):
+    eng, cfg = _engine(models("gqa4-128"))
+    prompt = [int(t) for t in np.random.default_rng(7).integers(3, cfg.vocab_size, 120)]
+    made = []
+    for on in (False, True, True):
+        eng.set_decode_resident(on)
+        eng.release_slot(0)
+        eng.prefill(0, prompt, 0, False)
+        eng.decode_submit([0], [17], [120])
+        eng.decode_sample()
+        toks = []
+        for i in range(1, 12):
+            eng.decode_submit([0], [], [120 + i])
+            toks += eng.decode_collect()
+            eng.decode_sample()
+        toks += eng.decode_collect()
+        eng.release_slot(0)
+        eng.prefill(0, prompt, 0, False)
+        eng.decode_loop_prepare([0], [17], [120])
+        eng.decode_loop_run(1, 12, True)
+        eng.synchronize()
+        assert eng.decode_loop_history(1, 121, 12) == toks
+        made.append(toks)
+    assert made[0] == made[1] == made[2]
+
+
+@pytest.mark.parametrize("shape,pos", [("gqa8-64", 0), ("gqa8-64", 600), ("qwen", 5), ("gqa4-128", 1023)])
+def test_a_launch_that_cannot_be_resident_is_done_by_the_one_behind(models, shape, pos):
+    """No time to wait for the other workgroups: the resident launch gives up, and the launch behind it does the step; the next steps
+    take the chain"""
+    eng, cfg = _engine(models(shape))
+    prompt = [int(t) for t in np.random.default_rng(9).integers(3, cfg.vocab_size, pos)]
+    got = []
+    for on in (False, True):
+        eng.set_decode_resident(on)
+        eng.set_decode_resident_wait(0)
+        eng.release_slot(0)
+        if pos:
+            eng.prefill(0, prompt, 0, False)
+        got.append(_steps(eng, 0, [21, 22, 23], pos))
+    assert eng.decode_resident_failed == 1
+    assert _rel(got[1], got[0]).max() < TOL
+
+
+def test_engines_take_turns(models):
+    """Two engines of a process stepping in two threads: neither holds CUs that the other waits for"""
+    engs = [_engine(models(n))[0] for n in ("gqa4-128", "gqa8-64")]
+    want, got = [None, None], [None, None]
+
+    def run(i, out):
+        eng = engs[i]
+        eng.release_slot(0)
+        eng.prefill(0, [5, 6, 7, 8], 0, False)
+        eng.decode_loop_prepare([0], [17], [4])
+        for _ in range(20):
+            eng.decode_loop_run(1, 10, True)
+        eng.synchronize()
+        out[i] = eng.decode_loop_history(1, 5, 200)
+
+    for i in range(2):
+        run(i, want)
+    threads = [threading.Thread(target=run, args=(i, got)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert [e.decode_resident_failed for e in engs] == [0, 0]
+    for g, w in zip(got, want):
+        assert g[:50] == w[:50]
+
+
+def test_what_the_resident_step_leaves_to_the_chain(tmp_path):
+    """Formats, widths and engines that it is not built for take the chain"""
+    small = write_synthetic_gguf(str(tmp_path / "small.gguf"), dataclasses.replace(BASE, d_model=768), "Q4_K_M", seed=7)
+    plain = write_synthetic_gguf(str(tmp_path / "plain.gguf"), BASE, "BF16", seed=7)
+    quant = write_synthetic_gguf(str(tmp_path / "quant.gguf"), BASE, "Q4_K_M", seed=7)
+    for path, kw in ((small, {}), (plain, {}), (quant, dict(act_q8=False)), (quant, dict(cu_mask=[0xFFFFFFFF] * 4))):
+        eng, cfg, _ = load_engine(path, max_ctx=128, max_batch=1, **kw)
+        assert not eng.decode_resident
+        assert 0 <= eng.decode([0], [1], [0])[0] < cfg.vocab_size
