@@ -190,10 +190,10 @@ class Engine {
   void release_slot(int slot);         // drop every block reference of the slot
   int kv_blocks_free() const { return (int)free_blocks_.size(); }
   int kv_blocks_total() const { return kv_nblocks_; }
-  // one row's decode step as one resident launch (decode_stream.h): whether this engine's steps take it; off for tests
+  // decode steps of few rows as one resident launch (decode_stream.h): rows up to which this engine's steps take it; off for tests
   // and comparisons; steps that its launch gave up on (another resident launch held part of the GPU) and that were done
   // without it; the time, in 10 ns, after which it gives up
-  bool decode_resident() const;
+  int decode_resident() const;
   void set_decode_resident(bool on) { ds_use_ = on; }
   unsigned decode_resident_failed() const { return ds_failed_ ? *(volatile unsigned*)ds_failed_ : 0; }
   void set_decode_resident_wait(unsigned long long ticks);
@@ -435,12 +435,13 @@ class Engine {
   void ds_setup();
   static void ds_shares(const LayerW& L, int parts, int& wg_k, int& wg_v);
   void ds_upload();                // the cache's scales (again, when they change)
-  bool ds_next();                  // whether the next step of one row runs resident (a while after a failure: no)
+  bool ds_next(int B);             // whether the next step of B rows runs resident (a while after a failure: no)
   int graph_key(int B, int kind);  // kind: 0 step, 1 masked step, 2 forward
   hipGraphExec_t captured(int key, bool forward, int B);
   void launch_step(hipGraphExec_t g);
   DsArgs ds_{};
-  bool ds_ok_ = false, ds_use_ = true;
+  int ds_rows_ = 0, ds_most_ = 0;  // rows of a resident step, at most (0: none); rows of a product that a workgroup has, at most
+  bool ds_use_ = true;
   bool ds_now_ = false;            // the step being enqueued runs resident
   float* ds_scale_ = nullptr;
   unsigned* ds_failed_ = nullptr;  // pinned

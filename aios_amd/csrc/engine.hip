@@ -116,7 +116,7 @@ DsTurn& ds_turn(int device) {
 Engine::~Engine() {
   if (lm_) (void)hipStreamSynchronize(stream_);
   lm_.reset();
-  if (ds_ok_) {
+  if (ds_rows_) {
     DsTurn& t = ds_turn(cfg_.device);
     std::lock_guard<std::mutex> lock(t.mu);
     if (t.last == this) {
@@ -778,13 +778,15 @@ void Engine::finalize() {
   finalized_ = true;
 }
 
-// One row's step as one resident launch (decode_stream.h): a GPU to itself, every matrix Q4_K or Q6_K with int8 activations.
-// (A rank of several, or a tier on some of the CUs, would wait for others inside the launch; bf16 and the other formats have
-// their own GEMVs.  AIOS_DECODE_GEMM_MIN_B=0 asks for the GEMVs alone.)
+// The step of few rows as one resident launch (decode_stream.h): a GPU to itself, every matrix Q4_K or Q6_K with int8 activations
+// (one row) or every one bf16 (up to four).  (A rank of several, or a tier on some of the CUs, would wait for others inside the launch; the other
+// formats have their own GEMVs.  AIOS_DECODE_GEMM_MIN_B=0 asks for the GEMVs alone.)
 void Engine::ds_setup() {
   if (dec_gemm_min_b_ <= 0) return;
-  if (lm_ || cfg_.tp_size > 1 || cfg_.vocab_parallel || !cfg_.act_q8 || !cfg_.cu_mask.empty() || !rope_cs_ || cfg_.n_layers < 1) return;
-  auto served = [](const QMat& m) { return m.valid() && (m.w.qtype == QT_Q4_K || m.w.qtype == QT_Q6_K); };
+  if (lm_ || cfg_.tp_size > 1 || cfg_.vocab_parallel || !cfg_.cu_mask.empty() || !rope_cs_ || cfg_.n_layers < 1) return;
+  const bool bf16 = output_.valid() && output_.w.qtype == QT_BF16;
+  if (!bf16 && !cfg_.act_q8) return;
+  auto served = [&](const QMat& m) { return m.valid() && (bf16 ? m.w.qtype == QT_BF16 : m.w.qtype == QT_Q4_K || m.w.qtype == QT_Q6_K); };
   if (!served(output_) || cfg_.vocab_size % 2) return;
   for (const LayerW& L : layers_)
     for (const QMat* m : {&L.wq, &L.wk, &L.wv, &L.wo, &L.wgu, &L.wdown})
@@ -797,6 +799,7 @@ void Engine::ds_setup() {
   a.n_layers = cfg_.n_layers; a.d = d; a.n_heads = H; a.n_kv_heads = Hkv; a.ff = cfg_.d_ff; a.vocab = cfg_.vocab_size;
   a.max_ctx = cfg_.max_ctx; a.rope_neox = cfg_.rope_neox; a.kv_fp8 = cfg_.kv_fp8;
   a.eps = cfg_.norm_eps; a.scale = 1.f / std::sqrt((float)hd);
+  a.bf16 = bf16; a.bt_stride = kv_maxb_; a.ldl = ldl_;
   if (a.parts < 4) return;
   auto share = [](int rows, int n) { return (rows + n - 1) / n; };  // rows of one workgroup of n, at most
   int most = std::max({share(d, a.parts), 4 * share(cfg_.d_ff / 2, a.parts), share(cfg_.vocab_size, a.parts)});
@@ -805,7 +808,10 @@ void Engine::ds_setup() {
     ds_shares(L, a.parts, wk, wv);
     most = std::max({most, share(L.wq.w.rows, wk), share(L.wk.w.rows, wv - wk), share(L.wv.w.rows, a.parts - wv)});
   }
-  if (!ds_plan(a, hd, most)) return;
+  ds_most_ = most;
+  int rows = 0;
+  while (rows < cfg_.max_batch && ds_plan(a, hd, most, rows + 1)) ++rows;
+  if (!rows) return;
   a.x = x_; a.logits = logits_; a.rope_cs = rope_cs_; a.pos = d_pos_; a.blocks = d_row_bt_;
   auto words = [&](size_t n) {
     auto* p = (uint64_t*)dmalloc(n * 8);
@@ -815,13 +821,13 @@ void Engine::ds_setup() {
   };
   const size_t nl = cfg_.n_layers;
   a.nqkv = (H + 2 * Hkv) * hd;
-  a.xn = words(2 * nl * d);
-  a.sq = words(2 * nl * a.parts);
-  a.resid = (float*)words((d + 1) / 2);
-  a.qkv = words(nl * a.nqkv);
-  a.attn = words(nl * H * hd);
-  a.h = words(nl * cfg_.d_ff / 2);
-  a.part = words(ds_part_words(H, hd));
+  a.xn = words(2 * nl * rows * d);
+  a.sq = words(2 * nl * rows * a.parts);
+  a.resid = (float*)words(((size_t)rows * d + 1) / 2);
+  a.qkv = words(nl * rows * a.nqkv);
+  a.attn = words(nl * rows * H * hd);
+  a.h = words(nl * rows * cfg_.d_ff / 2);
+  a.part = words(rows * ds_part_words(H, hd));
   a.ctl = (DsCtl*)words((sizeof(DsCtl) + 7) / 8);
   HIP_CHECK(hipHostMalloc((void**)&ds_failed_, 4, hipHostMallocDefault));
   *ds_failed_ = 0;
@@ -878,12 +884,12 @@ void Engine::ds_setup() {
   HIP_CHECK(hipMemcpy(dj, jobs.data(), sizeof(DsCopy) * jobs.size(), hipMemcpyHostToDevice));
   ws_bytes_ += sizeof(DsCopy) * jobs.size();
   a.jobs = dj;
-  ds_ok_ = true;
+  ds_rows_ = rows;
 }
 
 // Q, K and V of a layer have workgroups of their own, as many as their bytes are of all
 void Engine::ds_shares(const LayerW& L, int parts, int& wg_k, int& wg_v) {
-  auto cost = [](const QMat& m) { return (double)m.w.rows * (m.w.qtype == QT_Q4_K ? 144 : 210); };
+  auto cost = [](const QMat& m) { return (double)m.w.rows * (m.w.qtype == QT_Q4_K ? 144 : m.w.qtype == QT_Q6_K ? 210 : 512); };
   const double q = cost(L.wq), k = cost(L.wk), all = q + k + cost(L.wv);
   wg_k = std::min(std::max(1, (int)std::lround(parts * q / all)), parts - 2);
   wg_v = std::min(std::max(wg_k + 1, (int)std::lround(parts * (q + k) / all)), parts - 1);
@@ -893,7 +899,7 @@ void Engine::ds_upload() {
   HIP_CHECK(hipMemcpy(ds_scale_, kv_scale_.data(), kv_scale_.size() * 4, hipMemcpyHostToDevice));
 }
 
-bool Engine::decode_resident() const { return ds_ok_ && ds_use_; }
+int Engine::decode_resident() const { return ds_use_ ? ds_rows_ : 0; }
 
 void Engine::set_decode_resident_wait(unsigned long long ticks) {
   if (finalized_) HIP_CHECK(hipStreamSynchronize(stream_));
@@ -901,8 +907,8 @@ void Engine::set_decode_resident_wait(unsigned long long ticks) {
   reset_graphs();
 }
 
-bool Engine::ds_next() {
-  if (!decode_resident()) return false;
+bool Engine::ds_next(int B) {
+  if (B > decode_resident()) return false;
   const unsigned n = decode_resident_failed();
   if (n != ds_seen_) {  // another resident launch holds CUs: leave it the GPU for a while
     ds_seen_ = n;
@@ -1434,8 +1440,10 @@ void Engine::enqueue_decode_forward(int B) {
   }
   static const bool step_prep = !(std::getenv("AIOS_STEP_PREP") && std::atoi(std::getenv("AIOS_STEP_PREP")) == 0);
   nrm_lm_ = false;
-  if (B == 1 && ds_now_) {
-    launch_decode_stream(ds_, cfg_.head_dim, stream_);
+  if (ds_now_ && B <= ds_rows_) {
+    DsArgs a = ds_;
+    if (!ds_plan(a, cfg_.head_dim, ds_most_, B)) throw std::runtime_error("decode: no resident step of " + std::to_string(B) + " rows");
+    launch_decode_stream(a, cfg_.head_dim, stream_);
     return;
   }
   step_prep_on_ = step_prep && rope_cs_ != nullptr;
@@ -2116,12 +2124,12 @@ void Engine::decode_loop_run(int B, int n_steps, bool use_graph) {
     for (int i = 0; i < n_steps; ++i) enqueue_decode_step(B);
     return;
   }
-  ds_now_ = B == 1 && ds_next();
+  ds_now_ = ds_next(B);
   hipGraphExec_t ge = step_graph(B);
   for (int i = 0; i < n_steps; ++i) launch_step(ge);
 }
 
-int Engine::graph_key(int B, int kind) { return B * 4 + kind + (B == 1 && ds_now_ ? 1 << 24 : 0); }
+int Engine::graph_key(int B, int kind) { return B * 4 + kind + (ds_now_ ? 1 << 24 : 0); }
 
 // the captured decode step for (B, sample_mask_): captured once, replayed for every request --
 // the kernels read tokens / positions / slots / sampling parameters from device arrays
@@ -2133,7 +2141,7 @@ hipGraphExec_t Engine::captured(int key, bool forward, int B) {
   auto it = graphs_.find(key);
   if (it == graphs_.end()) {
     std::unique_lock<std::mutex> turn;
-    if (ds_ok_) turn = std::unique_lock<std::mutex>(ds_turn(cfg_.device).mu);
+    if (ds_rows_) turn = std::unique_lock<std::mutex>(ds_turn(cfg_.device).mu);
     hipGraph_t g;
     HIP_CHECK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
     try {
@@ -2202,7 +2210,7 @@ void Engine::decode_submit(const std::vector<int>& slots, const std::vector<int>
     row_pos_[b] = pos[b] + 1;
   }
   kv_sync(B);
-  ds_now_ = B == 1 && ds_next();
+  ds_now_ = ds_next(B);
   launch_step(forward_graph(B));
   pipe_B_ = B;
 }
@@ -2244,7 +2252,7 @@ int Engine::capture_graphs(int max_b) {
   const bool saved = sample_mask_;
   for (int B = 1; B <= std::min(max_b, cfg_.max_batch); ++B)
     for (int m = 0; m < 2; ++m) {
-      ds_now_ = B == 1 && decode_resident();
+      ds_now_ = B <= decode_resident();
       sample_mask_ = m != 0;
       step_graph(B);
       if (m == 0) forward_graph(B);  // (the pipelined decode's forward)
@@ -2272,7 +2280,7 @@ void Engine::set_kv_scales(const std::vector<float>& s) {
     if (!(v > 0.f) || !std::isfinite(v)) throw std::runtime_error("set_kv_scales: scales must be positive");
   if (finalized_) HIP_CHECK(hipStreamSynchronize(stream_));  // (no replay of the old graphs in flight)
   kv_scale_ = s;
-  if (ds_ok_) ds_upload();
+  if (ds_rows_) ds_upload();
   reset_graphs();
 }
 

@@ -1,4 +1,4 @@
-// One row's decode step as ONE resident launch: a workgroup per CU runs the layers' products and the attention, and the
+// A decode step of one row, or of up to four against bf16 weights, as ONE resident launch: a workgroup per CU runs the layers' products and the attention, and the
 // vectors between them go from workgroup to workgroup through memory.
 //
 // What bounds a step of one row is not its bytes: a chain of five launches a layer pays for each of them the launch, the
@@ -22,6 +22,8 @@
 //
 // A step, us, chain -> resident (MI355X, Q4_K_M): TinyLlama 128 keys 600 -> 464, 1000 keys 682 -> 578; Mistral-7B 128 keys 1424 -> 1190,
 // 3900 keys 1621 -> 1446; with the fp8 cache 2000 keys 1527 -> 1325, 16000 keys 1666 -> 1632; Qwen3-8B 128 keys 1755 -> 1325.
+// TinyLlama bf16, 128 / 1000 keys: one row 742 -> 644 / 818 -> 756, two 815 -> 667 / 887 -> 769, three 839 -> 694 / 899 -> 825, four 854 -> 750 / 904 -> 881
+// (five and more stay with the GEMMs: a fifth row is a second matrix instruction for the same weights, and its operand leaves the ring three slots).
 #include "decode_stream.h"
 
 #include <algorithm>
@@ -37,6 +39,12 @@ namespace {
 constexpr int DS_NG = 14, DS_NL = 2, DS_CT = DS_NG * 64, DS_THREADS = (DS_NG + DS_NL) * 64;
 constexpr int DS_SLOT = 32768, DS_R = 4;
 constexpr int DS_AW = 8;  // waves that attend
+
+// bf16 weights, up to four rows: a slot is four groups of four rows by 512 columns, a KB a row; 8 waves take half a group each
+constexpr int DS_BROWS = 4, DS_BSLOT = 16384, DS_BGROUPS = 4, DS_BPAD = 64;
+constexpr int DS_BRING = 8;  // slots, at most (the requests of seven are 56 of a wave's 63)
+template <bool BF>
+constexpr int ds_red() { return BF ? 64 : 16; }  // floats of one buffer of squares
 
 // a slot: chunks (32 weights) and their planes, each a run of its own (1 KB an LDS-DMA; the last plane of Q6_K 256 B)
 template <int QT>
@@ -107,9 +115,27 @@ __device__ __forceinline__ void ds_copy(const DsCopy& j, int s, uint8_t* dst, in
   }
 }
 
-// at most n of this wave's requests outstanding (n: a sum of up to three slots' counts)
+// bf16: a request is a KB of one row, lane l's sixteen bytes 4 x row places further on (mod 64), so that the lanes of the products below
+// read their four rows from different banks.  base, kq: of the next group, from the workgroup's first row on, from its row's first column on
+__device__ __forceinline__ void ds_copy16(const DsCopy& j, int& base, int& kq, uint8_t* dst, int lw) {
+  const int lane = threadIdx.x & 63, rb = __builtin_amdgcn_readfirstlane((int)(uint64_t)j.p[1]);
+  const auto r = ds_rsrc(j.p[0], j.job.nrows * rb);
+  const int v0 = lw * rb + ((lane - 4 * lw) & 63) * 16, v1 = (lw + 2) * rb + ((lane - 4 * lw - 8) & 63) * 16;
+  dst += lw * 1024;
+  static_for<DS_BGROUPS>([&](auto g) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst + 4096 * g), 16, v0 + base, 0, 0, 2);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst + 4096 * g + 2048), 16, v1 + base, 0, 0, 2);
+    base += 1024;
+    const bool wrap = ++kq * 1024 == rb;
+    base += wrap ? 3 * rb : 0;
+    kq = wrap ? 0 : kq;
+  });
+}
+
+// at most n of this wave's requests outstanding (n: a sum of slots' counts)
 __device__ __forceinline__ void ds_wait(int n) {
   switch (n) {
+    case 8: lg_vmcnt<8>(); break;
     case 12: lg_vmcnt<12>(); break;
     case 16: lg_vmcnt<16>(); break;
     case 24: lg_vmcnt<24>(); break;
@@ -119,6 +145,7 @@ __device__ __forceinline__ void ds_wait(int n) {
     case 40: lg_vmcnt<40>(); break;
     case 44: lg_vmcnt<44>(); break;
     case 48: lg_vmcnt<48>(); break;
+    case 56: lg_vmcnt<56>(); break;
     default: lg_vmcnt<0>(); break;
   }
 }
@@ -158,31 +185,48 @@ __device__ __forceinline__ bool ds_late(const DsClock& c) {
 // a lane asks memory for its first word only, and for the others, which come with it, once that is there and through the XCD's L2,
 // where 32 workgroups share them.  An exchange has words of its own in each layer, so L2 holds none of an older number; one that
 // it took in too early is asked for from memory.
-template <int N>
-__device__ __forceinline__ void ds_poll(const uint64_t* p, int stride, uint32_t no, uint32_t (&v)[N], const DsClock& c) {
-  uint64_t w[N];
+template <int N, int U>
+__device__ __forceinline__ void ds_poll(const uint64_t* const (&p)[U], int stride, uint32_t no, uint32_t (&v)[U][N], const DsClock& c) {
+  uint64_t w[U][N];
   for (int it = 1;; ++it) {
-    w[0] = ds_get(p);
-    if ((uint32_t)(w[0] >> 32) == no || ((it & 63) == 0 && ds_late(c))) break;
+    bool ok = true;
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u][0] = ds_get(p[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) ok = ok && (uint32_t)(w[u][0] >> 32) == no;
+    if (ok || ((it & 63) == 0 && ds_late(c))) break;
   }
 #pragma unroll
-  for (int i = 1; i < N; ++i) w[i] = __hip_atomic_load(const_cast<uint64_t*>(p + i * stride), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int i = 1; i < N; ++i)
+      w[u][i] = __hip_atomic_load(const_cast<uint64_t*>(p[u] + i * stride), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   bool ok = true;
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    v[i] = (uint32_t)w[i];
-    ok = ok && (uint32_t)(w[i] >> 32) == no;
-  }
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      v[u][i] = (uint32_t)w[u][i];
+      ok = ok && (uint32_t)(w[u][i] >> 32) == no;
+    }
   for (int it = 1; !ok; ++it) {
     ok = true;
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      w[i] = ds_get(p + i * stride);
-      v[i] = (uint32_t)w[i];
-      ok = ok && (uint32_t)(w[i] >> 32) == no;
-    }
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        w[u][i] = ds_get(p[u] + i * stride);
+        v[u][i] = (uint32_t)w[u][i];
+        ok = ok && (uint32_t)(w[u][i] >> 32) == no;
+      }
     if ((it & 63) == 0 && ds_late(c)) break;
   }
+}
+__device__ __forceinline__ float ds_word(const uint64_t* p, uint32_t no, const DsClock& c) {
+  const uint64_t* const q[1] = {p};
+  uint32_t w[1][1];
+  ds_poll<1, 1>(q, 0, no, w, c);
+  return __uint_as_float(w[0][0]);
 }
 
 struct DsLds {
@@ -225,59 +269,94 @@ __device__ __forceinline__ void ds_octet(int o, float (&v)[8], int8_t* xq, float
 // IN_X: plain values x and gains, the sum of squares to red; IN_F32: the exchange's values (multiplied by the gains where a norm is in
 // front); IN_BF16: pairs
 enum { IN_X, IN_F32, IN_BF16 };
-template <int IN>
-__device__ __forceinline__ void ds_stage(const float* x, const uint64_t* ex, uint32_t no, int K, const float* gain, int8_t* xq, float2* ms,
-                                         float* red, const DsClock& clk) {
-  const int tid = ds_tid(), noct = K >> 3;
+template <int IN, bool BF>
+__device__ __forceinline__ void ds_stage(const float* x, const uint64_t* ex, uint32_t no, int rows, int K, const float* gain, uint8_t* xq,
+                                         float2* ms, float* red, const DsClock& clk) {
+  const int tid = ds_tid(), noct = K >> 3, all = BF ? rows * noct : noct;
   constexpr int NW = IN == IN_BF16 ? 4 : 8;
+  constexpr int U = IN == IN_BF16 ? (BF ? 3 : 2) : 1;  // octets of a lane that are waited for together
   float ssq = 0.f;
-  // (whole waves: K is a multiple of 512, a wave takes 512 elements)
+  auto row_of = [&](int o) { return BF ? (o >= noct) + (o >= 2 * noct) + (o >= 3 * noct) : 0; };
+  auto keep = [&](int o, float (&v)[8]) __attribute__((always_inline)) {
+    if constexpr (BF) {
+      const int b = row_of(o);
+      *(uint4*)(xq + (size_t)b * (2 * K + DS_BPAD) + (o - b * noct) * 16) =
+          make_uint4(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]), pk_bf16(v[4], v[5]), pk_bf16(v[6], v[7]));
+    } else {
+      ds_octet(o, v, (int8_t*)xq, ms);
+    }
+  };
+  // (whole waves: K is a multiple of 512, a wave takes 512 elements of one row)
 #pragma clang loop unroll(disable)
-  for (int o = tid; o < noct; o += DS_CT) {
-    float v[8];
+  for (int o = tid; o < all; o += U * DS_CT) {
     if constexpr (IN == IN_X) {
+      const int b = row_of(o), oc = o - b * noct;
       const float4 f0 = *(const float4*)(x + 8 * o), f1 = *(const float4*)(x + 8 * o + 4);
-      const float4 g0 = *(const float4*)(gain + 8 * o), g1 = *(const float4*)(gain + 8 * o + 4);
+      const float4 g0 = *(const float4*)(gain + 8 * oc), g1 = *(const float4*)(gain + 8 * oc + 4);
       const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w}, g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+      float v[8];
+      if constexpr (BF) ssq = 0.f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         ssq = fmaf(f[i], f[i], ssq);
         v[i] = f[i] * g[i];
       }
+      if constexpr (BF) {
+        const float t = wave_sum(ssq);
+        if ((tid & 63) == 0) red[o >> 6] = t;
+      }
+      keep(o, v);
     } else {
-      uint32_t w[NW];
-      ds_poll<NW>(ex + (size_t)(o >> 6) * (NW * 64) + (o & 63), 64, no, w, clk);
-      if constexpr (IN == IN_BF16) {
+      const uint64_t* p[U];
+      uint32_t w[U][NW];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          v[2 * i] = __uint_as_float(w[i] << 16);
-          v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+      for (int u = 0; u < U; ++u) {  // (rows of words follow each other as those of octets do)
+        const int ou = o + u * DS_CT < all ? o + u * DS_CT : o;
+        p[u] = ex + (size_t)(ou >> 6) * (NW * 64) + (ou & 63);
+      }
+      ds_poll<NW, U>(p, 64, no, w, clk);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (u && o + u * DS_CT >= all) continue;
+        float v[8];
+        if constexpr (IN == IN_BF16) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[2 * i] = __uint_as_float(w[u][i] << 16);
+            v[2 * i + 1] = __uint_as_float(w[u][i] & 0xffff0000u);
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(w[u][i]);
         }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(w[i]);
+        keep(o + u * DS_CT, v);
       }
     }
-    ds_octet(o, v, xq, ms);
   }
-  if constexpr (IN == IN_X) {
+  if constexpr (IN == IN_X && !BF) {
     const float t = wave_sum(ssq);
     if ((tid & 63) == 0) red[tid >> 6] = t;
   }
 }
 
-// the sum of squares of the residual: a word of each workgroup, gathered by the last waves
-__device__ __forceinline__ void ds_squares(const DsArgs& a, const uint64_t* ex, uint32_t no, float* red, const DsClock& clk) {
+// the sums of squares of the residual's rows: a word of each workgroup, gathered by the last waves
+template <bool BF>
+__device__ __forceinline__ void ds_squares(const DsArgs& a, const uint64_t* ex, uint32_t no, int rows, float* red, const DsClock& clk) {
   const int tid = ds_tid();
-  float v = 0.f;
+  if constexpr (BF) {  // (64 workgroups, of one row, to a wave)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = rows * (a.parts >> 6);
 #pragma clang loop unroll(disable)
-  for (int i = DS_CT - 1 - tid; i < a.parts; i += DS_CT) {
-    uint32_t w[1];
-    ds_poll<1>(ex + i, 0, no, w, clk);
-    v += __uint_as_float(w[0]);
+    for (int i = DS_NG - 1 - wave; i < n; i += DS_NG) {
+      const float t = wave_sum(ds_word(ex + i * 64 + lane, no, clk));
+      if (lane == 0) red[i] = t;
+    }
+  } else {
+    float v = 0.f;
+#pragma clang loop unroll(disable)
+    for (int i = DS_CT - 1 - tid; i < a.parts; i += DS_CT) v += ds_word(ex + i, no, clk);
+    const float t = wave_sum(v);
+    if ((tid & 63) == 0) red[tid >> 6] = t;
   }
-  const float t = wave_sum(v);
-  if ((tid & 63) == 0) red[tid >> 6] = t;
 }
 
 // sum over the first n = 8, 16, 32 or 64 lanes of every n
@@ -364,6 +443,58 @@ __device__ __forceinline__ void ds_dot(const DsJob& j, int nch, int run, int& sl
   lg_barrier();
 }
 
+// ... of bf16 weights against up to four rows: sixteen 4 x 4 products of four columns a matrix instruction (lane 4 b + i: weight row i or
+// operand row i, columns 8 b ..), so each byte of weights is read from LDS once whatever the rows, beside as much of the operand
+typedef short ds_s16x4 __attribute__((ext_vector_type(4)));
+typedef float ds_f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void ds_dot16(const DsJob& j, int K, int rows, int ring, int& cur, const DsLds& s, const uint8_t* xb, float* acc,
+                                         float* acc_next, int row_sums) {
+  const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 3, b = lane >> 2, g = wave >> 1, half = wave & 1;
+  const int KQ = K >> 9, drow = DS_BGROUPS / KQ, dk = DS_BGROUPS - drow * KQ;
+  int rg = g / KQ, kq = g - rg * KQ;
+  const uint8_t* x = xb + (size_t)min(i, rows - 1) * (2 * K + DS_BPAD) + (half * 32 + b) * 16;
+  const int w0 = g * 4096 + i * 1024 + ((half * 32 + b + 4 * i) & 63) * 16, w1 = g * 4096 + i * 1024 + ((half * 32 + 16 + b + 4 * i) & 63) * 16;
+  for (int n = tid; n < row_sums; n += DS_CT) acc_next[n] = 0.f;
+#pragma clang loop unroll(disable)
+  for (int t = 0; t < j.slots; ++t) {
+    if (wave < 2 * DS_BGROUPS && t * DS_BGROUPS + g < j.chunks) {
+      const uint8_t* sl = s.ring + (size_t)cur * DS_BSLOT;
+      const uint4 wa = *(const uint4*)(sl + w0), wb = *(const uint4*)(sl + w1);
+      const uint4 xa = *(const uint4*)(x + kq * 1024), xc = *(const uint4*)(x + kq * 1024 + 256);
+      auto mul = [](uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, ds_f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ds_s16x4, make_uint2(a0, a1)), __builtin_bit_cast(ds_s16x4, make_uint2(b0, b1)), c, 0, 0, 0);
+      };
+      ds_f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0;
+      c0 = mul(wa.x, wa.y, xa.x, xa.y, c0);
+      c1 = mul(wa.z, wa.w, xa.z, xa.w, c1);
+      c0 = mul(wb.x, wb.y, xc.x, xc.y, c0);
+      c1 = mul(wb.z, wb.w, xc.z, xc.w, c1);
+      c0 += c1;
+      // the sixteen blocks together: weight row r's sum goes to the lanes of row r of the wave
+      const auto r0 = __builtin_amdgcn_permlane16_swap(__float_as_uint(c0[0]), __float_as_uint(c0[1]), false, false);
+      const auto r1 = __builtin_amdgcn_permlane16_swap(__float_as_uint(c0[2]), __float_as_uint(c0[3]), false, false);
+      const float p0 = __uint_as_float(r0[0]) + __uint_as_float(r0[1]), p1 = __uint_as_float(r1[0]) + __uint_as_float(r1[1]);
+      const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(p0), __float_as_uint(p1), false, false);
+      float v = __uint_as_float(r2[0]) + __uint_as_float(r2[1]);
+      v += lane_dpp<0x124>(v);  // row_ror:4
+      v += lane_dpp<0x128>(v);  // row_ror:8
+      const int row = rg * 4 + (lane >> 4);
+      if ((lane & 15) < rows && row < j.nrows) ds_add(acc + row * DS_BROWS + i, v);
+    }
+    rg += drow;
+    kq += dk;
+    if (kq >= KQ) {
+      kq -= KQ;
+      ++rg;
+    }
+    if (++cur == ring) cur = 0;
+    if (t + 1 < j.slots) lg_barrier();
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lg_barrier();
+}
+
 // tiles of keys that a wave has in flight (a request is 1 KB, of fp8 512 B), keys of a workgroup's pass
 template <int HD, bool F8>
 constexpr int ds_tiles() { return 1; }
@@ -385,7 +516,19 @@ struct DsAttnLds {
   };
 };
 
-template <int HD, int G, bool F8>
+// a part that attends: row, unit of heads, run of its keys.  (One workgroup a unit: the heads of a KV head on one XCD; workgroups go
+// round the eight in turn)
+struct DsPlace {
+  int b, unit, sp;
+};
+__device__ __forceinline__ DsPlace ds_place(int wg, int units, int rows, int P) {
+  const int all = units * rows;
+  const int u = P > 1 ? wg / P : ((all & 7) == 0 ? (wg & 7) * (all >> 3) + (wg >> 3) : wg);
+  const int b = rows > 1 ? min(u / units, rows - 1) : 0;
+  return {b, u - b * units, P > 1 ? wg - u * P : 0};
+}
+
+template <int HD, int G, bool F8, bool BF>
 __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P, int pos, uint32_t no, float2 cs, const DsLds& s,
                                           const DsClock& clk) {
   using S = DsAttnLds<HD, G, F8>;
@@ -396,16 +539,18 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
   using KVT = typename std::conditional<F8, uint2, uint4>::type;
   const int units = a.n_heads / G;
   const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (wg >= units * P) {
+  const int rows = BF ? a.rows : 1;
+  if (wg >= rows * units * P) {
     lg_barrier();
     lg_barrier();
     lg_barrier();
     lg_barrier();
     return;
   }
-  // one head a workgroup: the heads of a KV head on one XCD (workgroups go round the eight in turn)
-  const int unit = P > 1 ? wg / P : ((units & 7) == 0 ? (wg & 7) * (units >> 3) + (wg >> 3) : wg), sp = P > 1 ? wg - unit * P : 0;
-  const int h0 = unit * G, gq = a.n_heads / a.n_kv_heads, kvh = h0 / gq;
+  const DsPlace at = ds_place(wg, units, rows, P);
+  const int sp = at.sp, lb = l * rows + at.b;
+  const int* blocks = a.blocks + (BF ? at.b * a.bt_stride : 0);
+  const int h0 = at.unit * G, gq = a.n_heads / a.n_kv_heads, kvh = h0 / gq;
   const int ksub = lane / LPK, dsl = lane % LPK;
   uint8_t *kc = a.kc + (size_t)l * a.kv_layer, *vc = a.vc + (size_t)l * a.kv_layer;
   KVT kr[NT][STEPS], vr[NT][STEPS];
@@ -413,7 +558,7 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
   // a tile is a buffer of its live keys' bytes: what lies behind them reads as zeros without a memory access
   const int voff = (ksub * HD + dsl * 8) * ES;
   auto request = [&](KVT (&r)[STEPS], const uint8_t* pool, int k0) __attribute__((always_inline)) {
-    const int blk = ds_table(a.blocks, min(k0 / KV_BLOCK, a.max_ctx / KV_BLOCK - 1));
+    const int blk = ds_table(blocks, min(k0 / KV_BLOCK, a.max_ctx / KV_BLOCK - 1));
     const int live = __builtin_amdgcn_readfirstlane(min(max(pos - k0, 0), KPW));
     const auto rs = uniform_rsrc(pool + (((size_t)blk * a.n_kv_heads + kvh) * KV_BLOCK + (k0 % KV_BLOCK)) * HD * ES, live * HD * ES);
 #pragma unroll
@@ -440,9 +585,7 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
     const int v = tid / HD, i = tid - v * HD;
     const int row = v < G ? (h0 + v) * HD + i : (a.n_heads + (v == G ? kvh : a.n_kv_heads + kvh)) * HD + i;
     const float b = a.bias ? a.bias[(size_t)l * a.nqkv + row] : 0.f;
-    uint32_t w[1];
-    ds_poll<1>(a.qkv + (size_t)l * a.nqkv + row, 0, no, w, clk);
-    L.vec[v][i] = __uint_as_float(w[0]) + b;
+    L.vec[v][i] = ds_word(a.qkv + (size_t)lb * a.nqkv + row, no, clk) + b;
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   lg_barrier();
@@ -474,7 +617,7 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
         const float inv = F8 ? 1.f / (isv ? s.scale[2 * l + 1] : s.scale[2 * l]) : 1.f;
         kv_store_pair((bf16_t*)L.own[isv], ia, ib, v0, v1, F8, inv);
         if (sp == 0 && h0 % gq == 0) {  // one workgroup a KV head keeps it
-          const size_t i0 = (((size_t)ds_table(a.blocks, pos / KV_BLOCK) * a.n_kv_heads + kvh) * KV_BLOCK + pos % KV_BLOCK) * HD;
+          const size_t i0 = (((size_t)ds_table(blocks, pos / KV_BLOCK) * a.n_kv_heads + kvh) * KV_BLOCK + pos % KV_BLOCK) * HD;
           kv_store_pair((bf16_t*)(isv ? vc : kc), i0 + ia, i0 + ib, v0, v1, F8, inv);
         }
       }
@@ -626,9 +769,9 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
     }
     if (F8) acc *= s.scale[2 * l + 1];
     if (P == 1) {
-      ds_put(a.attn + (size_t)l * a.n_heads * HD + ds_at((h0 + g) * HD + d), __float_as_uint(acc / S1), no);
+      ds_put(a.attn + (size_t)lb * a.n_heads * HD + ds_at((h0 + g) * HD + d), __float_as_uint(acc / S1), no);
     } else {
-      uint64_t* p = a.part + ((size_t)(h0 + g) * DS_PMAX + sp) * (HD + 2);
+      uint64_t* p = a.part + ((size_t)(at.b * a.n_heads + h0 + g) * DS_PMAX + sp) * (HD + 2);
       ds_put(p + d, __float_as_uint(acc), no);
       if (d < 2) ds_put(p + HD + d, __float_as_uint(d ? S1 : W), no);
     }
@@ -638,16 +781,15 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
 }
 
 // the runs of a head's keys together: 16 elements of a head at a time.  Two barriers.
-template <int HD>
+template <int HD, bool BF>
 __device__ __forceinline__ void ds_combine(const DsArgs& a, int l, int unit, int P, uint32_t no, const DsLds& s, const DsClock& clk) {
   const int tid = ds_tid(), h = unit / (HD / 16), d0 = unit % (HD / 16) * 16;
   float* v = (float*)s.area;  // [P][18]
-  const bool on = unit < a.n_heads * (HD / 16);
+  const int rows = BF ? a.rows : 1;
+  const bool on = unit < rows * a.n_heads * (HD / 16);
   if (on && tid < P * 18) {
     const int sp = tid / 18, j = tid - sp * 18;
-    uint32_t w[1];
-    ds_poll<1>(a.part + ((size_t)h * DS_PMAX + sp) * (HD + 2) + (j < 16 ? d0 + j : HD + j - 16), 0, no, w, clk);
-    v[tid] = __uint_as_float(w[0]);
+    v[tid] = ds_word(a.part + ((size_t)h * DS_PMAX + sp) * (HD + 2) + (j < 16 ? d0 + j : HD + j - 16), no, clk);
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   lg_barrier();
@@ -660,7 +802,8 @@ __device__ __forceinline__ void ds_combine(const DsArgs& a, int l, int unit, int
       S1 += f * v[p * 18 + 17];
       acc += f * v[p * 18 + tid];
     }
-    ds_put(a.attn + (size_t)l * a.n_heads * HD + ds_at(h * HD + d0 + tid), __float_as_uint(acc / S1), no);
+    const int b = BF ? h / a.n_heads : 0;
+    ds_put(a.attn + (size_t)(l * rows + b) * a.n_heads * HD + ds_at((h - b * a.n_heads) * HD + d0 + tid), __float_as_uint(acc / S1), no);
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   lg_barrier();
@@ -671,10 +814,10 @@ __device__ __forceinline__ void ds_combine(const DsArgs& a, int l, int unit, int
 template <int HD, bool F8>
 __device__ __forceinline__ int ds_runs(const DsArgs& a, int G, int pos) {
   if (pos < ATTN_SPLIT_LEN) return 1;
-  return min(min(pos / ds_pass<HD, F8>() + 1, a.parts / (a.n_heads / G)), DS_PMAX);
+  return min(min(pos / ds_pass<HD, F8>() + 1, a.parts / (a.rows * (a.n_heads / G))), DS_PMAX);
 }
 
-template <int HD, int G, bool F8>
+template <int HD, int G, bool F8, bool BF>
 __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   if (a.alone && !a.ctl->failed) return;
@@ -682,18 +825,25 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
   const int first = blockIdx.x, step = gridDim.x;  // (parts of this workgroup: one, or all of them in turn)
   DsLds s;
   s.ring = smem;
-  s.area = smem + DS_R * DS_SLOT;
+  s.area = smem + (BF ? a.ring * DS_BSLOT : DS_R * DS_SLOT);
   s.rowacc = (float*)(s.area + a.area_bytes);
   s.red = s.rowacc + 2 * a.row_sums;
-  unsigned* gate = (unsigned*)(s.red + 32);
-  s.scale = s.red + 36;
+  constexpr int RED = ds_red<BF>();
+  unsigned* gate = (unsigned*)(s.red + 2 * RED);
+  s.scale = s.red + 2 * RED + 4;
   s.jobs = (DsJob*)(s.scale + (2 * a.n_layers + 3) / 4 * 4);
   s.gains = (float*)(s.jobs + 4 * a.n_layers + 1);
-  const int qd = a.n_heads * HD, pos = min(ds_table(a.pos, 0), a.max_ctx - 1);
+  constexpr int SH = BF ? 2 : 0;  // a product's row has sums of four operand rows in LDS, or one
+  const int rows = BF ? a.rows : 1;
+  auto pos_of = [&](int b) { return min(ds_table(a.pos, b), a.max_ctx - 1); };
+  const int qd = a.n_heads * HD;
+  int pos = pos_of(0);  // the farthest
+  if constexpr (BF)
+    for (int b = 1; b < rows; ++b) pos = max(pos, pos_of(b));
   const bool brief = pos < ATTN_SPLIT_LEN;
   const int P = ds_runs<HD, F8>(a, G, pos);
-  const int nattend = brief ? a.n_heads : a.n_heads / G * P;  // parts that attend
-  const int ncomb = (a.n_heads * (HD / 16) + a.parts - 1) / a.parts;
+  const int nattend = rows * (brief ? a.n_heads : a.n_heads / G * P);  // parts that attend
+  const int ncomb = (rows * a.n_heads * (HD / 16) + a.parts - 1) / a.parts;
 
   if (wave >= DS_NG) {
     // ---- loaders: the step's slots in order, as many ahead as the ring holds; they pass every barrier of the others
@@ -701,6 +851,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
     const int last = 4 * a.n_layers;
     int iq = 0, iw = first, is = 0, at = 0;  // next slot: product, part, slot of it; ring place
     int h0 = 0, h1 = 0, h2 = 0;              // requests of the last three slots
+    int base = 0, kq = 0, ahead = 0;         // (bf16) next group; slots asked for, less those the others have had
     DsCopy J = ds_table(a.jobs, first), N;              // the job being requested, the one after it
     auto after = [&]() {
       if ((iw += step) >= a.parts) {
@@ -716,12 +867,19 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
       h1 = h0;
       h0 = 0;
       while (more && is >= J.job.slots) {
-        is = 0;
+        is = base = kq = 0;
         more = iq <= last;
         J = N;
         after();
       }
       if (!more) return;
+      if constexpr (BF) {
+        ds_copy16(J, base, kq, s.ring + (size_t)at * DS_BSLOT, lw);
+        if (++at == a.ring) at = 0;
+        ++is;
+        ++ahead;
+        return;
+      }
       uint8_t* dst = s.ring + (size_t)(at % DS_R) * DS_SLOT;
       if (J.job.chunks & DS_Q6) {
         ds_copy<QT_Q6_K>(J, is, dst, lw);
@@ -733,7 +891,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
       ++is;
       ++at;
     };
-    for (int i = 0; i < DS_R; ++i) issue();
+    for (int i = 0; i < (BF ? a.ring : DS_R); ++i) issue();
     lg_barrier();  // the gate's answer
     unsigned go;
     asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
@@ -755,7 +913,8 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
         slots = ds_table(&a.jobs->job.slots, (min(q + wrap, last) * a.parts + (wrap ? first : wg + step)) * 16);
         if (!n) lg_barrier();
         for (int t = 0; t < n; ++t) {
-          ds_wait(t || owed ? h0 + h1 : h0 + h1 + h2);
+          if constexpr (BF) ds_wait(2 * DS_BGROUPS * --ahead);
+          else ds_wait(t || owed ? h0 + h1 : h0 + h1 + h2);
           lg_barrier();
           if (t || owed) issue();
           owed = false;
@@ -802,7 +961,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
     gate[0] = go;
     gate[1] = no;
   }
-  for (int i = tid; i < 2 * a.row_sums + 32; i += DS_CT) s.rowacc[i] = 0.f;
+  for (int i = tid; i < 2 * a.row_sums + 2 * RED; i += DS_CT) s.rowacc[i] = 0.f;
   for (int i = tid; i < 2 * a.n_layers; i += DS_CT) s.scale[i] = a.kv_scale[i];
   for (int i = tid; i <= 4 * a.n_layers; i += DS_CT) s.jobs[i] = a.jobs[(size_t)i * a.parts + first].job;
   {
@@ -818,13 +977,18 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
   const uint32_t no0 = __builtin_amdgcn_readfirstlane(gate[1]) + 1;
 
   if (go) {
-    int8_t* xq = (int8_t*)s.area;
+    uint8_t* xq = s.area;
     int slot = 0, par = 0;
-    const float2 rope = a.rope_cs[(size_t)pos * (HD / 2) + (tid & (HD / 2 - 1))];  // of the lane's pair, in every layer
+    // of this workgroup's row (the launch with all workgroups): its position, and RoPE of the lane's pair, in every layer
+    auto row_of = [&](int wg) { return BF && wg < nattend ? ds_place(wg, brief ? a.n_heads : a.n_heads / G, rows, P).b : 0; };
+    auto rope_at = [&](int p) { return a.rope_cs[(size_t)p * (HD / 2) + (ds_tid() & (HD / 2 - 1))]; };
+    const int mine = BF ? pos_of(row_of(first)) : pos;
+    const float2 rope = rope_at(mine);
     const int last = 4 * a.n_layers;
     // the residual at this thread's row (of O and of down alike, in reverse order of the threads)
     float own = 0.f;
-    if (!a.alone && DS_CT - 1 - tid < s.jobs[DS_O].nrows) own = a.x[s.jobs[DS_O].r0 + DS_CT - 1 - tid];
+    const int rt0 = DS_CT - 1 - tid, b0 = BF ? rt0 & 3 : 0;
+    if (!a.alone && rt0 < s.jobs[DS_O].nrows << SH && b0 < rows) own = a.x[(size_t)b0 * a.d + s.jobs[DS_O].r0 + (rt0 >> SH)];
     // one product after the other, with the attention in front of O's; the code of all of them is one (what a layer runs
     // through stays in the instruction cache)
 #pragma clang loop unroll(disable)
@@ -833,18 +997,20 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
       const uint32_t no = no0 + l;
       if (kind == DS_O) {
         for (int wg = first; wg < a.parts; wg += step) {
-          if (brief) ds_attend<HD, 1, F8>(a, l, wg, 1, pos, no, rope, s, clk);
-          else ds_attend<HD, G, F8>(a, l, wg, P, pos, no, rope, s, clk);
+          const int p = BF && a.alone ? pos_of(row_of(wg)) : mine;
+          const float2 cs = BF && a.alone ? rope_at(p) : rope;
+          if (brief) ds_attend<HD, 1, F8, BF>(a, l, wg, 1, p, no, cs, s, clk);
+          else ds_attend<HD, G, F8, BF>(a, l, wg, P, p, no, cs, s, clk);
         }
         if (P > 1)
           for (int wg = first; wg < a.parts; wg += step)
-            for (int i = 0; i < ncomb; ++i) ds_combine<HD>(a, l, wg + i * a.parts, P, no, s, clk);
+            for (int i = 0; i < ncomb; ++i) ds_combine<HD, BF>(a, l, wg + i * a.parts, P, no, s, clk);
       }
 #pragma clang loop unroll(disable)
       for (int wg = first; wg < a.parts; wg += step) {
         // (results are written, and the residual they are added to read, by the last waves: a wave's loads are counted behind
         // its stores, and the first ones have the next operand to wait for)
-        const int tid = ds_tid(), rt = DS_CT - 1 - tid;
+        const int tid = ds_tid(), rt = DS_CT - 1 - tid, b = BF ? rt & 3 : 0;  // (and of operand row b)
         const DsJob job = a.alone ? ds_table(a.jobs, q * a.parts + wg).job : s.jobs[q];
         DsJob j;
         j.r0 = __builtin_amdgcn_readfirstlane(job.r0);
@@ -856,61 +1022,85 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
         const int K = kind == DS_O ? qd : (kind == DS_DOWN ? a.ff : a.d), nch = K >> 5;
         float2* ms = (float2*)(xq + K);
         float* acc = s.rowacc + par * a.row_sums;
-        float* red = s.red + par * 16;
+        float* red = s.red + par * RED;
         par ^= 1;
         const bool resid = kind == DS_O || kind == DS_DOWN;
         const int nr = kind == DS_O ? 2 * l : kind == DS_GU ? 2 * l : kind == DS_DOWN ? 2 * l + 1 : 2 * l - 1;  // the residual it makes or reads
-        if (a.alone && resid && rt < j.nrows) {
-          own = nr ? __hip_atomic_load(a.resid + j.r0 + rt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.x[j.r0 + rt];
+        const int n = j.nrows << SH;
+        if (a.alone && resid && rt < n && b < rows) {
+          const size_t at = (size_t)b * a.d + j.r0 + (rt >> SH);
+          own = nr ? __hip_atomic_load(a.resid + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.x[at];
           asm volatile("" : "+v"(own));  // (waited for here)
         }
         if (kind == DS_DOWN) {
-          ds_stage<IN_BF16>(nullptr, a.h + (size_t)l * (a.ff / 2), no, K, nullptr, xq, ms, red, clk);
+          ds_stage<IN_BF16, BF>(nullptr, a.h + (size_t)l * rows * (a.ff / 2), no, rows, K, nullptr, xq, ms, red, clk);
         } else if (q == 0) {
-          ds_stage<IN_X>(a.x, nullptr, 0, K, a.gains, xq, ms, red, clk);
+          ds_stage<IN_X, BF>(a.x, nullptr, 0, rows, K, a.gains, xq, ms, red, clk);
         } else {
           const uint32_t nx = kind == DS_QKV ? no - 1 : no;
-          ds_stage<IN_F32>(nullptr, kind == DS_O ? a.attn + (size_t)l * qd : a.xn + (size_t)nr * a.d, nx, K, nullptr, xq, ms, red, clk);
-          if (kind != DS_O) ds_squares(a, a.sq + (size_t)nr * a.parts, nx, red, clk);
+          ds_stage<IN_F32, BF>(nullptr, kind == DS_O ? a.attn + (size_t)l * rows * qd : a.xn + (size_t)nr * rows * a.d, nx, rows, K, nullptr, xq,
+                               ms, red, clk);
+          if (kind != DS_O) ds_squares<BF>(a, a.sq + (size_t)nr * rows * a.parts, nx, rows, red, clk);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         lg_barrier();  // the operand is staged, slot 0 there
         float inv = 1.f;
         if (!resid) {
           float t = 0.f;
+          if constexpr (BF) {
+            const int m = q ? a.parts >> 6 : K >> 9;  // sums of a row
+            for (int w = 0; w < m; ++w) t += red[min(b, rows - 1) * m + w];
+          } else {
 #pragma unroll
-          for (int w = 0; w < DS_NG; ++w) t += red[w];
+            for (int w = 0; w < DS_NG; ++w) t += red[w];
+          }
           inv = rsqrtf(t / (float)K + a.eps);
         }
-        const int low = nch & -nch;  // (the largest power of two in it: lanes that share a row)
-        if (q6) ds_dot<QT_Q6_K>(j, nch, min(low, 64), slot, s, xq, ms, acc, s.rowacc + par * a.row_sums, a.row_sums);
-        else ds_dot<QT_Q4_K>(j, nch, min(low >> 1, 64), slot, s, xq, ms, acc, s.rowacc + par * a.row_sums, a.row_sums);
+        float* acc_next = s.rowacc + par * a.row_sums;
+        if constexpr (BF) {
+          ds_dot16(j, K, rows, a.ring, slot, s, xq, acc, acc_next, a.row_sums);
+        } else {
+          const int low = nch & -nch;  // (the largest power of two in it: lanes that share a row)
+          if (q6) ds_dot<QT_Q6_K>(j, nch, min(low, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
+          else ds_dot<QT_Q4_K>(j, nch, min(low >> 1, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
+        }
         if (resid) {
           // (rows by the last wave's lanes, further ones by those before; the squares go with the first word)
-          const bool on = rt < j.nrows;
+          const int r = rt >> SH;
+          const bool on = rt < n && b < rows;
           const float x = on ? own + acc[rt] : 0.f;
-          float gain = s.gains[nr * a.own_rows + min(rt, a.own_rows - 1)];
+          float gain = s.gains[nr * a.own_rows + min(r, a.own_rows - 1)];
           if (a.alone) {
-            gain = a.gains[(size_t)(nr + 1) * a.d + j.r0 + (on ? rt : 0)];
+            gain = a.gains[(size_t)(nr + 1) * a.d + j.r0 + (on ? r : 0)];
             asm volatile("" : "+v"(gain));
           }
           own = x;
           if (on) {
-            ds_put(a.xn + (size_t)nr * a.d + ds_at(j.r0 + rt), __float_as_uint(x * gain), no);
-            if (a.alone) __hip_atomic_store(a.resid + j.r0 + rt, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ds_put(a.xn + ((size_t)nr * rows + b) * a.d + ds_at(j.r0 + r), __float_as_uint(x * gain), no);
+            if (a.alone) __hip_atomic_store(a.resid + (size_t)b * a.d + j.r0 + r, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
-          const float sq = wave_sum(x * x);
-          if (tid == DS_CT - 1) ds_put(a.sq + (size_t)nr * a.parts + wg, __float_as_uint(sq), no);
-        } else {
-          if (q == last) {
-            for (int r = rt; r < j.nrows; r += DS_CT) a.logits[j.r0 + r] = acc[r] * inv;
-          } else if (kind == DS_QKV) {
-            for (int r = rt; r < j.nrows; r += DS_CT) ds_put(a.qkv + (size_t)l * a.nqkv + j.r0 + r, __float_as_uint(acc[r] * inv), no);
+          float sq = x * x;
+          if constexpr (BF) {  // over the lanes of an operand row
+            sq += lane_dpp<0x124>(sq);
+            sq += lane_dpp<0x128>(sq);
+            sq = lane_xor32(lane_xor16(sq, LaneAdd{}), LaneAdd{});
           } else {
-            for (int u = rt; u < j.nrows >> 2; u += DS_CT) {
-              const float4 v = *(const float4*)(acc + 4 * u);
-              const float f0 = glu_act(v.x * inv, ACT_SILU) * (v.y * inv), f1 = glu_act(v.z * inv, ACT_SILU) * (v.w * inv);
-              ds_put(a.h + (size_t)l * (a.ff / 2) + ds_at16((j.r0 >> 2) + u), (uint32_t)f32_to_bf16(f0) | (uint32_t)f32_to_bf16(f1) << 16, no);
+            sq = wave_sum(sq);
+          }
+          if (rt < rows) ds_put(a.sq + ((size_t)nr * rows + rt) * a.parts + wg, __float_as_uint(sq), no);
+        } else if (b < rows) {
+          if (q == last) {
+            for (int i = rt; i < n; i += DS_CT) a.logits[(size_t)b * a.ldl + j.r0 + (i >> SH)] = acc[i] * inv;
+          } else if (kind == DS_QKV) {
+            for (int i = rt; i < n; i += DS_CT) ds_put(a.qkv + ((size_t)l * rows + b) * a.nqkv + j.r0 + (i >> SH), __float_as_uint(acc[i] * inv), no);
+          } else {
+            for (int i = rt; i < n >> 2; i += DS_CT) {
+              const int u = i >> SH;
+              float v[4];
+#pragma unroll
+              for (int k = 0; k < 4; ++k) v[k] = acc[((4 * u + k) << SH) + b];
+              const float f0 = glu_act(v[0] * inv, ACT_SILU) * (v[1] * inv), f1 = glu_act(v[2] * inv, ACT_SILU) * (v[3] * inv);
+              ds_put(a.h + ((size_t)l * rows + b) * (a.ff / 2) + ds_at16((j.r0 >> 2) + u), (uint32_t)f32_to_bf16(f0) | (uint32_t)f32_to_bf16(f1) << 16, no);
             }
           }
         }
@@ -932,15 +1122,17 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
   }
 }
 
-int ds_lds(const DsArgs& a) {
-  return DS_R * DS_SLOT + a.area_bytes + (2 * a.row_sums + 32 + 4 + (2 * a.n_layers + 3) / 4 * 4) * 4 + (4 * a.n_layers + 1) * (int)sizeof(DsJob) +
-         2 * a.n_layers * a.own_rows * 4;
+// LDS behind the ring and the operand
+int ds_rest(const DsArgs& a) {
+  const int red = a.bf16 ? ds_red<true>() : ds_red<false>();
+  return (2 * a.row_sums + 2 * red + 4 + (2 * a.n_layers + 3) / 4 * 4) * 4 + (4 * a.n_layers + 1) * (int)sizeof(DsJob) + 2 * a.n_layers * a.own_rows * 4;
 }
+int ds_lds(const DsArgs& a) { return (a.bf16 ? a.ring * DS_BSLOT : DS_R * DS_SLOT) + a.area_bytes + ds_rest(a); }
 
-template <int HD, int G, bool F8>
+template <int HD, int G, bool F8, bool BF>
 void ds_launch(DsArgs a, hipStream_t st) {
   const int lds = ds_lds(a);
-  auto* k = decode_stream_kernel<HD, G, F8>;
+  auto* k = decode_stream_kernel<HD, G, F8, BF>;
   static const hipError_t set = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   HIP_CHECK(set);
   a.alone = 0;
@@ -951,17 +1143,31 @@ void ds_launch(DsArgs a, hipStream_t st) {
   HIP_CHECK(hipGetLastError());
 }
 
-template <int HD, bool F8>
+template <int HD, bool F8, bool BF>
 void ds_heads(const DsArgs& a, hipStream_t st) {
   const int g = a.n_heads / a.n_kv_heads;
-  if (g % 4 == 0) ds_launch<HD, 4, F8>(a, st);
-  else if (g == 2) ds_launch<HD, 2, F8>(a, st);
-  else ds_launch<HD, 1, F8>(a, st);
+  if (g % 4 == 0) ds_launch<HD, 4, F8, BF>(a, st);
+  else if (g == 2) ds_launch<HD, 2, F8, BF>(a, st);
+  else ds_launch<HD, 1, F8, BF>(a, st);
+}
+template <int HD, bool F8>
+void ds_format(const DsArgs& a, hipStream_t st) {
+  if (a.bf16) ds_heads<HD, F8, true>(a, st);
+  else ds_heads<HD, F8, false>(a, st);
 }
 
 }  // namespace
 
 DsCopy ds_job(const QWeight& w, int r0, int nrows, int row0) {
+  if (w.qtype == QT_BF16) {
+    DsCopy j{};
+    const uint64_t rb = (uint64_t)w.cols * 2;  // (p[1] .. unused otherwise)
+    const int groups = (nrows + 3) / 4 * (w.cols / 512);
+    j.p[0] = j.p[2] = j.p[3] = w.p0 + (size_t)r0 * rb;
+    j.p[1] = (const uint8_t*)rb;
+    j.job = {row0 + r0, nrows, groups, (groups + DS_BGROUPS - 1) / DS_BGROUPS};
+    return j;
+  }
   const size_t nch = w.cols / 32, c = (size_t)r0 * nch;
   const bool q6 = w.qtype == QT_Q6_K;
   const int chunks = (int)(nrows * nch), ch = q6 ? DsFmt<QT_Q6_K>::CH : DsFmt<QT_Q4_K>::CH;
@@ -974,24 +1180,34 @@ DsCopy ds_job(const QWeight& w, int r0, int nrows, int row0) {
   return j;
 }
 
-bool ds_plan(DsArgs& a, int hd, int max_rows) {
+bool ds_plan(DsArgs& a, int hd, int max_rows, int rows) {
   const int qd = a.n_heads * hd, g = a.n_heads / a.n_kv_heads;
   if ((hd != 64 && hd != 128) || a.n_heads % a.n_kv_heads || !(g == 1 || g == 2 || g == 4 || g == 8)) return false;
   // whole waves of octets, rows that 16 chunks divide; every workgroup with rows of O, gate/up and down (see the exchanges above)
-  if (a.d % 512 || qd % 512 || a.ff % 512 || a.d < 2 * a.parts || a.ff / 2 < 2 * a.parts || a.n_heads > a.parts) return false;
+  if (a.d % 512 || qd % 512 || a.ff % 512 || a.d < 2 * a.parts || a.ff / 2 < 2 * a.parts) return false;
+  if (rows < 1 || rows > (a.bf16 ? DS_BROWS : 1) || rows * a.n_heads > a.parts) return false;
+  const int width = a.bf16 ? DS_BROWS : 1;  // sums of a product's row
+  a.rows = rows;
   a.own_rows = (a.d + a.parts - 1) / a.parts;
-  if (a.own_rows > 64) return false;  // (a wave holds a workgroup's rows of the residual)
+  if (a.own_rows * width > 64) return false;  // (a wave holds a workgroup's rows of the residual)
   const int K = std::max({a.d, qd, a.ff});
   const int gl = g % 4 == 0 ? 4 : g;
   const int attn = gl * hd * 2 + 2 * hd * 2 + DS_AW * gl * 2 * 4 + DS_AW * gl * hd * 4;
-  a.area_bytes = (std::max({K + K / 2, attn, DS_PMAX * 18 * 4}) + 255) / 256 * 256;
-  a.row_sums = (max_rows + 63) / 64 * 64;
+  const int operand = a.bf16 ? rows * (2 * K + DS_BPAD) : K + K / 2;
+  a.area_bytes = (std::max({operand, attn, DS_PMAX * 18 * 4}) + 255) / 256 * 256;
+  a.row_sums = (max_rows * width + 63) / 64 * 64;
+  if (a.bf16) {
+    // sums of squares: 64 workgroups a word of LDS, or 512 columns
+    if (a.parts % 64 || rows * std::max(a.parts / 64, a.d / 512) > ds_red<true>()) return false;
+    a.ring = std::min(DS_BRING, (160 * 1024 - a.area_bytes - ds_rest(a)) / DS_BSLOT);
+    if (a.ring < 4) return false;  // (what is in flight to a CU: 64 KB)
+  }
   return ds_lds(a) <= 160 * 1024;
 }
 
 void launch_decode_stream(const DsArgs& a, int hd, hipStream_t st) {
-  if (hd == 64) a.kv_fp8 ? ds_heads<64, true>(a, st) : ds_heads<64, false>(a, st);
-  else a.kv_fp8 ? ds_heads<128, true>(a, st) : ds_heads<128, false>(a, st);
+  if (hd == 64) a.kv_fp8 ? ds_format<64, true>(a, st) : ds_format<64, false>(a, st);
+  else a.kv_fp8 ? ds_format<128, true>(a, st) : ds_format<128, false>(a, st);
 }
 
 }  // namespace aios

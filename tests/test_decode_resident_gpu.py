@@ -1,4 +1,4 @@
-"""One row's decode step as one resident launch (kernels/decode_stream.hip) against the chain of launches it stands in for."""
+"""Decode steps of few rows as one resident launch (kernels/decode_stream.hip) against the chain of launches it stands in for."""
 import dataclasses
 import threading
 
@@ -25,23 +25,25 @@ SHAPES = {
 # both int8-activation paths are 0.013 from 64 bits (perf/cases.py); they differ in the order of fp32 sums and in codes that this rounds
 # the other way, so by no more than the two distances together
 TOL = 0.026
+# bf16 weights and operands: 0.0036 from 64 bits each (perf/cases.py), and further apart in the largest of a few hundred rows
+TOL16 = 0.015
 
 
 @pytest.fixture(scope="module")
 def models(tmp_path_factory):
     d, held = tmp_path_factory.mktemp("resident"), {}
 
-    def get(name):
-        if name not in held:
+    def get(name, recipe="Q4_K_M"):
+        if (name, recipe) not in held:
             cfg = dataclasses.replace(BASE, max_ctx=2048, **SHAPES[name])
-            held[name] = write_synthetic_gguf(str(d / f"{name}.gguf"), cfg, "Q4_K_M", seed=11)
-        return held[name]
+            held[name, recipe] = write_synthetic_gguf(str(d / f"{name}-{recipe}.gguf"), cfg, recipe, seed=11)
+        return held[name, recipe]
 
     return get
 
 
 def _engine(path, **kw):
-    eng, cfg, _ = load_engine(path, max_ctx=kw.pop("max_ctx", 2048), max_batch=2, **kw)
+    eng, cfg, _ = load_engine(path, max_ctx=kw.pop("max_ctx", 2048), max_batch=kw.pop("max_batch", 2), **kw)
     assert eng.decode_resident
     return eng, cfg
 
@@ -82,6 +84,41 @@ def test_resident_step_is_the_chains(models, shape, kv):
             got.append(_steps(eng, slot, tokens, pos))
         assert np.isfinite(got[1]).all()
         assert _rel(got[1], got[0]).max() < TOL, (pos, _rel(got[1], got[0]))
+    assert eng.decode_resident_failed == 0
+
+
+def _rows(eng, cfg, contexts, slots, seed):
+    """Logits of two steps of a batch behind contexts of these lengths"""
+    rng = np.random.default_rng(seed)
+    for s, n in zip(slots, contexts):
+        eng.release_slot(s)
+        if n:
+            eng.prefill(s, [int(t) for t in rng.integers(3, cfg.vocab_size, n)], 0, False)
+    out = []
+    for i in range(2):
+        eng.decode(slots, [int(t) for t in rng.integers(3, cfg.vocab_size, len(slots))], [n + i for n in contexts])
+        out.append(np.asarray(eng.last_logits(len(slots)), np.float64).reshape(len(slots), -1))
+    return np.concatenate(out)
+
+
+# one to four rows; short ones beside one that has its keys split, and beside one in its last pass
+BATCHES = [[0], [300], [700], [0, 1], [128, 511], [40, 512], [1, 0, 500], [1500, 3, 700], [7, 130, 256, 33], [1023, 1, 512, 1300]]
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp8_e4m3"])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_resident_step_of_bf16_rows_is_the_chains(models, shape, kv):
+    eng, cfg = _engine(models(shape, "BF16"), kv_dtype=kv, max_batch=4, max_slots=8)
+    assert eng.decode_resident == 4
+    if kv != "bf16":
+        eng.set_kv_scales([1 / 64] * (2 * cfg.n_layers))
+    for n, contexts in enumerate(BATCHES):
+        got = []
+        for at, on in ((0, False), (4, True)):
+            eng.set_decode_resident(on)
+            got.append(_rows(eng, cfg, contexts, list(range(at, at + len(contexts))), n))
+        assert np.isfinite(got[1]).all()
+        assert _rel(got[1], got[0]).max() < TOL16, (contexts, _rel(got[1], got[0]))
     assert eng.decode_resident_failed == 0
 
 
@@ -141,6 +178,18 @@ def test_a_launch_that_cannot_be_resident_is_done_by_the_one_behind(models, shap
     assert _rel(got[1], got[0]).max() < TOL
 
 
+@pytest.mark.parametrize("contexts", [[5], [3, 600, 40], [0, 10, 20, 30]])
+def test_bf16_rows_are_done_by_the_launch_behind(models, contexts):
+    eng, cfg = _engine(models("gqa8-64", "BF16"), max_batch=4, max_slots=4)
+    got = []
+    for on in (False, True):
+        eng.set_decode_resident(on)
+        eng.set_decode_resident_wait(0)
+        got.append(_rows(eng, cfg, contexts, list(range(len(contexts))), 3))
+    assert eng.decode_resident_failed == 1
+    assert _rel(got[1], got[0]).max() < TOL16
+
+
 def test_engines_take_turns(models):
     """Two engines of a process stepping in two threads: neither holds CUs that the other waits for"""
     engs = [_engine(models(n))[0] for n in ("gqa4-128", "gqa8-64")]
@@ -171,7 +220,7 @@ def test_engines_take_turns(models):
 def test_what_the_resident_step_leaves_to_the_chain(tmp_path):
     """Formats, widths and engines that it is not built for take the chain"""
     small = write_synthetic_gguf(str(tmp_path / "small.gguf"), dataclasses.replace(BASE, d_model=768), "Q4_K_M", seed=7)
-    plain = write_synthetic_gguf(str(tmp_path / "plain.gguf"), BASE, "BF16", seed=7)
+    plain = write_synthetic_gguf(str(tmp_path / "plain.gguf"), dataclasses.replace(BASE, d_ff=1280), "BF16", seed=7)
     quant = write_synthetic_gguf(str(tmp_path / "quant.gguf"), BASE, "Q4_K_M", seed=7)
     for path, kw in ((small, {}), (plain, {}), (quant, dict(act_q8=False)), (quant, dict(cu_mask=[0xFFFFFFFF] * 4))):
         eng, cfg, _ = load_engine(path, max_ctx=128, max_batch=1, **kw)
