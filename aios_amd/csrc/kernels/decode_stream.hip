@@ -339,21 +339,22 @@ __device__ __forceinline__ void ds_stage(const float* x, const uint64_t* ex, uin
   }
 }
 
-// the sums of squares of the residual's rows: a word of each workgroup, gathered by the last waves
+// the sums of squares of the residual's rows: a word of each workgroup, gathered by the waves in front of the last one (which writes this
+// workgroup's results, and came to these 0.3 to 0.5 us after the others to the operand)
 template <bool BF>
 __device__ __forceinline__ void ds_squares(const DsArgs& a, const uint64_t* ex, uint32_t no, int rows, float* red, const DsClock& clk) {
   const int tid = ds_tid();
   if constexpr (BF) {  // (64 workgroups, of one row, to a wave)
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = rows * (a.parts >> 6);
 #pragma clang loop unroll(disable)
-    for (int i = DS_NG - 1 - wave; i < n; i += DS_NG) {
+    for (int i = DS_NG - 2 - wave + (wave == DS_NG - 1 ? DS_NG : 0); i < n; i += DS_NG) {
       const float t = wave_sum(ds_word(ex + i * 64 + lane, no, clk));
       if (lane == 0) red[i] = t;
     }
   } else {
     float v = 0.f;
 #pragma clang loop unroll(disable)
-    for (int i = DS_CT - 1 - tid; i < a.parts; i += DS_CT) v += ds_word(ex + i, no, clk);
+    for (int i = DS_CT - 65 - tid + (tid >= DS_CT - 64 ? DS_CT : 0); i < a.parts; i += DS_CT) v += ds_word(ex + i, no, clk);
     const float t = wave_sum(v);
     if ((tid & 63) == 0) red[tid >> 6] = t;
   }
@@ -372,16 +373,31 @@ __device__ __forceinline__ void ds_add(float* p, float v) {
   __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// where a thread stands in a product: row and column of its (pair of) chunk(s), or group, in the first slot; what a slot advances them by.  (Worked
+// out before the operand is waited for.)
+struct DsAt {
+  int row, c, drow, dc;
+};
+__device__ __forceinline__ DsAt ds_at_first(int first, int slot, int n) {
+  DsAt p;
+  p.row = first / n;
+  p.c = first - p.row * n;
+  p.drow = slot / n;
+  p.dc = slot - p.drow * n;
+  asm volatile("" : "+v"(p.row), "+v"(p.c), "+s"(p.drow), "+s"(p.dc));
+  return p;
+}
+
 // one slot after the other against the staged operand; row sums in LDS.  A barrier behind each slot (or one)
 template <int QT>
-__device__ __forceinline__ void ds_dot(const DsJob& j, int nch, int run, int& slot, const DsLds& s, const int8_t* xq, const float2* ms,
+__device__ __forceinline__ void ds_dot(const DsJob& j, const DsAt& p, int nch, int run, int& slot, const DsLds& s, const int8_t* xq, const float2* ms,
                                        float* acc, float* acc_next, int row_sums) {
   using F = DsFmt<QT>;
   const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // this lane's (pair of) chunk(s): place within the slot, and its row and column, which advance by a slot's chunks
   const int at = F::PAIRS ? 2 * tid : tid;
-  int row = at / nch, c = at - row * nch;
-  const int drow = F::CH / nch, dc = F::CH - drow * nch;
+  int row = p.row, c = p.c;
+  const int drow = p.drow, dc = p.dc;
   const int wfirst = F::PAIRS ? 128 * wave : 64 * wave;
   const bool same = dc == 0;  // the same columns in every slot: the operand stays in registers
   Q4PairX X;
@@ -447,12 +463,12 @@ __device__ __forceinline__ void ds_dot(const DsJob& j, int nch, int run, int& sl
 // operand row i, columns 8 b ..), so each byte of weights is read from LDS once whatever the rows, beside as much of the operand
 typedef short ds_s16x4 __attribute__((ext_vector_type(4)));
 typedef float ds_f32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void ds_dot16(const DsJob& j, int K, int rows, int ring, int& cur, const DsLds& s, const uint8_t* xb, float* acc,
+__device__ __forceinline__ void ds_dot16(const DsJob& j, const DsAt& p, int K, int rows, int ring, int& cur, const DsLds& s, const uint8_t* xb, float* acc,
                                          float* acc_next, int row_sums) {
   const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 3, b = lane >> 2, g = wave >> 1, half = wave & 1;
-  const int KQ = K >> 9, drow = DS_BGROUPS / KQ, dk = DS_BGROUPS - drow * KQ;
-  int rg = g / KQ, kq = g - rg * KQ;
+  const int KQ = K >> 9;
+  int rg = p.row, kq = p.c;
   const uint8_t* x = xb + (size_t)min(i, rows - 1) * (2 * K + DS_BPAD) + (half * 32 + b) * 16;
   const int w0 = g * 4096 + i * 1024 + ((half * 32 + b + 4 * i) & 63) * 16, w1 = g * 4096 + i * 1024 + ((half * 32 + 16 + b + 4 * i) & 63) * 16;
   for (int n = tid; n < row_sums; n += DS_CT) acc_next[n] = 0.f;
@@ -482,8 +498,8 @@ __device__ __forceinline__ void ds_dot16(const DsJob& j, int K, int rows, int ri
       const int row = rg * 4 + (lane >> 4);
       if ((lane & 15) < rows && row < j.nrows) ds_add(acc + row * DS_BROWS + i, v);
     }
-    rg += drow;
-    kq += dk;
+    rg += p.drow;
+    kq += p.dc;
     if (kq >= KQ) {
       kq -= KQ;
       ++rg;
@@ -810,10 +826,15 @@ __device__ __forceinline__ void ds_combine(const DsArgs& a, int l, int unit, int
 }
 
 // ---- the step ---------------------------------------------------------------------------------------------------------------
-// keys up to which a head has one workgroup (as attn_lanes), and how many workgroups share the others
+// Keys below which a head has one workgroup, that needs no exchange of partial results (3.8 us a layer with the combination), and how many
+// workgroups share the others.  A step, us, one workgroup / several: heads of 64 (TinyLlama bf16) 750 keys 674 / 750, 1500 728 / 764, 1900 763 / 765
+// (four rows: 1500 871 / 891, 1900 922 / 902; Q4_K 1500 602 / 608, 1900 645 / 611); of 128 (Mistral-7B) 500 keys 1278 / 1306, 750 1350 / 1319
+// (fp8 500 1250 / 1287, 1000 1381 / 1301; Qwen3-8B 500 1429 / 1465, 750 1506 / 1477)
+template <int HD>
+constexpr int ds_brief() { return 81920 / HD; }
 template <int HD, bool F8>
 __device__ __forceinline__ int ds_runs(const DsArgs& a, int G, int pos) {
-  if (pos < ATTN_SPLIT_LEN) return 1;
+  if (pos < ds_brief<HD>()) return 1;
   return min(min(pos / ds_pass<HD, F8>() + 1, a.parts / (a.rows * (a.n_heads / G))), DS_PMAX);
 }
 
@@ -840,7 +861,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
   int pos = pos_of(0);  // the farthest
   if constexpr (BF)
     for (int b = 1; b < rows; ++b) pos = max(pos, pos_of(b));
-  const bool brief = pos < ATTN_SPLIT_LEN;
+  const bool brief = pos < ds_brief<HD>();
   const int P = ds_runs<HD, F8>(a, G, pos);
   const int nattend = rows * (brief ? a.n_heads : a.n_heads / G * P);  // parts that attend
   const int ncomb = (rows * a.n_heads * (HD / 16) + a.parts - 1) / a.parts;
@@ -1032,6 +1053,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
           own = nr ? __hip_atomic_load(a.resid + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.x[at];
           asm volatile("" : "+v"(own));  // (waited for here)
         }
+        const DsAt place = BF ? ds_at_first(tid >> 7, DS_BGROUPS, K >> 9) : q6 ? ds_at_first(tid, DsFmt<QT_Q6_K>::CH, nch) : ds_at_first(2 * tid, DsFmt<QT_Q4_K>::CH, nch);
         if (kind == DS_DOWN) {
           ds_stage<IN_BF16, BF>(nullptr, a.h + (size_t)l * rows * (a.ff / 2), no, rows, K, nullptr, xq, ms, red, clk);
         } else if (q == 0) {
@@ -1045,24 +1067,23 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         lg_barrier();  // the operand is staged, slot 0 there
         float inv = 1.f;
-        if (!resid) {
+        if (!resid && DS_CT - 64 - (tid & ~63) < n) {  // (waves that have results to write; behind the product it took 0.7 us)
           float t = 0.f;
           if constexpr (BF) {
             const int m = q ? a.parts >> 6 : K >> 9;  // sums of a row
             for (int w = 0; w < m; ++w) t += red[min(b, rows - 1) * m + w];
           } else {
-#pragma unroll
-            for (int w = 0; w < DS_NG; ++w) t += red[w];
+            t = lanes_sum<16>((tid & 15) < DS_NG ? red[tid & 15] : 0.f);
           }
           inv = rsqrtf(t / (float)K + a.eps);
         }
         float* acc_next = s.rowacc + par * a.row_sums;
         if constexpr (BF) {
-          ds_dot16(j, K, rows, a.ring, slot, s, xq, acc, acc_next, a.row_sums);
+          ds_dot16(j, place, K, rows, a.ring, slot, s, xq, acc, acc_next, a.row_sums);
         } else {
           const int low = nch & -nch;  // (the largest power of two in it: lanes that share a row)
-          if (q6) ds_dot<QT_Q6_K>(j, nch, min(low, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
-          else ds_dot<QT_Q4_K>(j, nch, min(low >> 1, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
+          if (q6) ds_dot<QT_Q6_K>(j, place, nch, min(low, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
+          else ds_dot<QT_Q4_K>(j, place, nch, min(low >> 1, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
         }
         if (resid) {
           // (rows by the last wave's lanes, further ones by those before; the squares go with the first word)
