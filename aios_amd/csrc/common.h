@@ -126,11 +126,12 @@ __device__ __forceinline__ void kv_store_pair(bf16_t* cache, size_t i0, size_t i
 
 // ---- reductions over the lanes of a wave, on the vector unit: a __shfl_xor is a trip through LDS that the next step waits for, six of
 // them ~0.3 us of a launch that has nothing else to do (a norm's sum in front of the first product, a row's in front of its store).
-// All lanes that take part are active.  ms, shuffles -> so: 8 steps of TinyLlama Q4_K_M 5.08 -> 4.97, a prompt of 23 tokens
+// All lanes that take part are active.  (bound_ctrl, though no pattern here reads outside: only with it is the move part of the addition that
+// follows; without it every step was a move, two wait states and an addition.)  ms, shuffles -> so: 8 steps of TinyLlama Q4_K_M 5.08 -> 4.97, a prompt of 23 tokens
 // (TinyLlama) 1.015 -> 0.977; 8 steps of Mistral-7B the same.
 template <int CTRL>
 __device__ __forceinline__ float lane_dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 struct LaneAdd { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
 struct LaneMax { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
