@@ -869,6 +869,8 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
   if (wave >= DS_NG) {
     // ---- loaders: the step's slots in order, as many ahead as the ring holds; they pass every barrier of the others
     const int lw = wave - DS_NG;
+    // (Q4_K / Q6_K: their requests in front of fourteen waves of vector work, 0.5 to 1 % of a step; bf16, which has little, lost 0.7 %)
+    if constexpr (!BF) __builtin_amdgcn_s_setprio(2);
     const int last = 4 * a.n_layers;
     int iq = 0, iw = first, is = 0, at = 0;  // next slot: product, part, slot of it; ring place
     int h0 = 0, h1 = 0, h2 = 0;              // requests of the last three slots
@@ -1048,6 +1050,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
         const bool resid = kind == DS_O || kind == DS_DOWN;
         const int nr = kind == DS_O ? 2 * l : kind == DS_GU ? 2 * l : kind == DS_DOWN ? 2 * l + 1 : 2 * l - 1;  // the residual it makes or reads
         const int n = j.nrows << SH;
+        const bool writes = (DS_NG - 1 - __builtin_amdgcn_readfirstlane(tid >> 6)) * 64 < n;  // waves that have results to write
         if (a.alone && resid && rt < n && b < rows) {
           const size_t at = (size_t)b * a.d + j.r0 + (rt >> SH);
           own = nr ? __hip_atomic_load(a.resid + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.x[at];
@@ -1067,7 +1070,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         lg_barrier();  // the operand is staged, slot 0 there
         float inv = 1.f;
-        if (!resid && DS_CT - 64 - (tid & ~63) < n) {  // (waves that have results to write; behind the product it took 0.7 us)
+        if (!resid && writes) {  // (behind the product it took 0.7 us)
           float t = 0.f;
           if constexpr (BF) {
             const int m = q ? a.parts >> 6 : K >> 9;  // sums of a row
@@ -1085,6 +1088,9 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
           if (q6) ds_dot<QT_Q6_K>(j, place, nch, min(low, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
           else ds_dot<QT_Q4_K>(j, place, nch, min(low >> 1, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
         }
+        // (what all other workgroups wait for: in front of the waves that go on to the next operand.  Those may not skip this part, though they
+        // have nothing to write: waiting earlier they take more from the writing wave than the priority gives back)
+        if (writes) __builtin_amdgcn_s_setprio(3);
         if (resid) {
           // (rows by the last wave's lanes, further ones by those before; the squares go with the first word)
           const int r = rt >> SH;
@@ -1125,6 +1131,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
             }
           }
         }
+        __builtin_amdgcn_s_setprio(0);
       }
     }
   }
