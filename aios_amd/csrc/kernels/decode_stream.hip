@@ -521,6 +521,19 @@ constexpr int ds_pass() { return ds_tiles<HD, F8>() * DS_AW * 4 * (512 / HD); }
 // G query heads of one KV head over the passes sp, sp + P, .. of its keys (attn_lanes of attn_decode.h, with the heads sharing what is
 // read); the row's own key is taken from the exchange, as the cache will hold it.
 // Four barriers.  LDS: queries in bf16, the own key and value as cached, the raw vectors and then the waves' results.
+// Four heads: a lane has one head's scores (its number mod 4's) and not all four, an exp2 instead of four and 18 registers less.
+// sum over a key's LPK lanes of four heads' terms, of head lane & 3
+template <int LPK>
+__device__ __forceinline__ float ds_quad_sum(const float (&d)[4]) {
+  const bool b0 = threadIdx.x & 1, b1 = threadIdx.x & 2;
+  const float r0 = (b0 ? d[1] : d[0]) + lane_dpp<0xB1>(b0 ? d[0] : d[1]);
+  const float r1 = (b0 ? d[3] : d[2]) + lane_dpp<0xB1>(b0 ? d[2] : d[3]);
+  float r = (b1 ? r1 : r0) + lane_dpp<0x4E>(b1 ? r0 : r1);
+  if constexpr (LPK == 8) return r + lane_dpp<0x141>(lane_dpp<0x1B>(r));  // the other quad of eight, in its order
+  r += lane_dpp<0x124>(r);
+  return r + lane_dpp<0x128>(r);
+}
+
 template <int HD, int G, bool F8>
 struct DsAttnLds {
   uint16_t q[G][HD];
@@ -648,15 +661,23 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
 #pragma unroll
       for (int g = 0; g < G; ++g) q[g] = *(const uint4*)&L.q[g][dsl * 8];
     };
-    float m[G], sum[G], o[G][8];
+    constexpr bool QUAD = G == 4;
+    constexpr int NS = QUAD ? 1 : G;  // heads whose scores a lane has
+    float m[NS], sum[NS], o[G][8];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      m[g] = kNeg;
-      sum[g] = 0.f;
+    for (int n = 0; n < NS; ++n) {
+      m[n] = kNeg;
+      sum[n] = 0.f;
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int i = 0; i < 8; ++i) o[g][i] = 0.f;
-    }
-    auto score = [&](const KVT& r, float (&sc)[G], bool live) __attribute__((always_inline)) {
+    auto of_head = [&](const float (&v)[NS], auto g) __attribute__((always_inline)) {
+      if constexpr (QUAD) return lane_dpp<0x55 * g.value>(v[0]);
+      else return v[g.value];
+    };
+    auto score = [&](const KVT& r, float (&sc)[NS], bool live) __attribute__((always_inline)) {
       uint32_t kb[4];
       if constexpr (F8) {
         kb[0] = fp8x2_bf16x2<false>(r.x); kb[1] = fp8x2_bf16x2<true>(r.x);
@@ -664,27 +685,49 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
       } else {
         kb[0] = r.x; kb[1] = r.y; kb[2] = r.z; kb[3] = r.w;
       }
+      float d[G];
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        float d = dot2_bf16(kb[0], q[g].x, 0.f);
-        d = dot2_bf16(kb[1], q[g].y, d);
-        d = dot2_bf16(kb[2], q[g].z, d);
-        d = dot2_bf16(kb[3], q[g].w, d);
-        d = lanes_sum<LPK>(d);
-        sc[g] = live ? d : kNeg;
+        d[g] = dot2_bf16(kb[0], q[g].x, 0.f);
+        d[g] = dot2_bf16(kb[1], q[g].y, d[g]);
+        d[g] = dot2_bf16(kb[2], q[g].z, d[g]);
+        d[g] = dot2_bf16(kb[3], q[g].w, d[g]);
       }
-    };
-    auto weigh = [&](float mx, int g) __attribute__((always_inline)) {  // a head's running max, at least mx
-      const float mn = fmaxf(m[g], mx);
-      if (__builtin_amdgcn_ballot_w64(mn > m[g])) {
-        const float alpha = fast_exp2(m[g] - mn);
-        sum[g] *= alpha;
+      if constexpr (QUAD) {
+        const float t = ds_quad_sum<LPK>(d);
+        sc[0] = live ? t : kNeg;
+      } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[g][i] *= alpha;
-        m[g] = mn;
+        for (int g = 0; g < G; ++g) {
+          const float t = lanes_sum<LPK>(d[g]);
+          sc[g] = live ? t : kNeg;
+        }
       }
     };
-    auto add = [&](const KVT& r, const float (&p)[G]) __attribute__((always_inline)) {
+    auto weigh = [&](const float (&mx)[NS]) __attribute__((always_inline)) {  // the heads' running max, at least mx
+      bool more = false;
+      float mn[NS];
+#pragma unroll
+      for (int n = 0; n < NS; ++n) {
+        mn[n] = fmaxf(m[n], mx[n]);
+        more = more || mn[n] > m[n];
+      }
+      if (__builtin_amdgcn_ballot_w64(more)) {
+        float alpha[NS];
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+          alpha[n] = fast_exp2(m[n] - mn[n]);
+          sum[n] *= alpha[n];
+          m[n] = mn[n];
+        }
+        static_for<G>([&](auto g) {
+          const float f = of_head(alpha, g);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) o[g][i] *= f;
+        });
+      }
+    };
+    auto add = [&](const KVT& r, const float (&p)[NS]) __attribute__((always_inline)) {
       float vf[8];
       if constexpr (F8) {
         const gf32x2 f0 = fp8x2_f32x2<false>(r.x), f1 = fp8x2_f32x2<true>(r.x), f2 = fp8x2_f32x2<false>(r.y), f3 = fp8x2_f32x2<true>(r.y);
@@ -698,16 +741,17 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
           vf[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
         }
       }
+      static_for<G>([&](auto g) {
+        const float f = of_head(p, g);
 #pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[g][e] = fmaf(p[g], vf[e], o[g][e]);
+        for (int e = 0; e < 8; ++e) o[g][e] = fmaf(f, vf[e], o[g][e]);
+      });
     };
     for (int pass = sp; pass < npass; pass += P) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const int k0 = first_key(pass, t), kn = first_key(pass + P, t);
-        float sc[STEPS][G];
+        float sc[STEPS][NS], mx[NS];
         read_q();
 #pragma unroll
         for (int i = 0; i < STEPS; ++i) {
@@ -716,17 +760,19 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
         }
         if (pass + P < npass) request(kr[t], kc, kn);
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-          float mx = sc[0][g];
+        for (int n = 0; n < NS; ++n) {
+          mx[n] = sc[0][n];
 #pragma unroll
-          for (int i = 1; i < STEPS; ++i) mx = fmaxf(mx, sc[i][g]);
-          weigh(mx, g);
+          for (int i = 1; i < STEPS; ++i) mx[n] = fmaxf(mx[n], sc[i][n]);
+        }
+        weigh(mx);
+#pragma unroll
+        for (int n = 0; n < NS; ++n)
 #pragma unroll
           for (int i = 0; i < STEPS; ++i) {
-            sc[i][g] = fast_exp2(sc[i][g] - m[g]);
-            sum[g] += sc[i][g];
+            sc[i][n] = fast_exp2(sc[i][n] - m[n]);
+            sum[n] += sc[i][n];
           }
-        }
 #pragma unroll
         for (int i = 0; i < STEPS; ++i) {
           add(vr[t][i], sc[i]);
@@ -736,38 +782,40 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
       }
     }
     if (wave == 0 && sp == 0) {  // the row's own key, by the first key group
-      float sc[G];
+      float sc[NS];
       read_q();
       score(*(const KVT*)((const uint8_t*)L.own[0] + dsl * 8 * ES), sc, ksub == 0);
+      weigh(sc);
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        weigh(sc[g], g);
-        sc[g] = fast_exp2(sc[g] - m[g]);
-        sum[g] += sc[g];
-      }
-      if (ksub) {
-#pragma unroll
-        for (int g = 0; g < G; ++g) sc[g] = 0.f;
+      for (int n = 0; n < NS; ++n) {
+        sc[n] = fast_exp2(sc[n] - m[n]);
+        sum[n] += sc[n];
+        if (ksub) sc[n] = 0.f;
       }
       add(*(const KVT*)((const uint8_t*)L.own[1] + dsl * 8 * ES), sc);
     }
     // the key groups of a wave, then (below) the waves
+    float w[NS];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const float M = keys_max<LPK>(m[g]), w = fast_exp2(m[g] - M);
-      const float S1 = keys_sum<LPK>(sum[g] * w);
+    for (int n = 0; n < NS; ++n) {
+      const float M = keys_max<LPK>(m[n]);
+      w[n] = fast_exp2(m[n] - M);
+      const float S1 = keys_sum<LPK>(sum[n] * w[n]);
+      if (lane < (QUAD ? 4 : 1)) {
+        L.m[wave][QUAD ? lane : n] = M;
+        L.l[wave][QUAD ? lane : n] = S1;
+      }
+    }
+    static_for<G>([&](auto g) {
+      const float f = of_head(w, g);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[g][e] = keys_sum<LPK>(o[g][e] * w);
+      for (int e = 0; e < 8; ++e) o[g][e] = keys_sum<LPK>(o[g][e] * f);
       if (ksub == 0) {
         float4* dst = (float4*)&L.o[wave][g][dsl * 8];
         dst[0] = make_float4(o[g][0], o[g][1], o[g][2], o[g][3]);
         dst[1] = make_float4(o[g][4], o[g][5], o[g][6], o[g][7]);
       }
-      if (lane == 0) {
-        L.m[wave][g] = M;
-        L.l[wave][g] = S1;
-      }
-    }
+    });
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   lg_barrier();
