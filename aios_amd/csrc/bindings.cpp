@@ -443,6 +443,7 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       .def_property_readonly("prefill_fused", &Engine::prefill_fused)
       .def_property_readonly("decode_gemm_min_batch", &Engine::decode_gemm_min_batch)
       .def_property_readonly("decode_resident", &Engine::decode_resident)
+      .def_property_readonly("decode_resident_last", &Engine::decode_resident_last)
       .def_property_readonly("decode_resident_failed", &Engine::decode_resident_failed)
       .def("set_decode_resident", &Engine::set_decode_resident, py::arg("on"))
       .def("set_decode_resident_wait", &Engine::set_decode_resident_wait, py::arg("ticks"))

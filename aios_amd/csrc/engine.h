@@ -194,6 +194,7 @@ class Engine {
   // and comparisons; steps that its launch gave up on (another resident launch held part of the GPU) and that were done
   // without it; the time, in 10 ns, after which it gives up
   int decode_resident() const;
+  bool decode_resident_last() const { return ds_now_; }  // whether the last step queued was one
   void set_decode_resident(bool on) { ds_use_ = on; }
   unsigned decode_resident_failed() const { return ds_failed_ ? *(volatile unsigned*)ds_failed_ : 0; }
   void set_decode_resident_wait(unsigned long long ticks);
@@ -435,7 +436,8 @@ class Engine {
   void ds_setup();
   static void ds_shares(const LayerW& L, int parts, int& wg_k, int& wg_v);
   void ds_upload();                // the cache's scales (again, when they change)
-  bool ds_next(int B);             // whether the next step of B rows runs resident (a while after a failure: no)
+  bool ds_beside();
+  bool ds_next(int B);             // whether the next step of B rows runs resident (not for a while after a failure, nor beside another engine's)
   int graph_key(int B, int kind);  // kind: 0 step, 1 masked step, 2 forward
   hipGraphExec_t captured(int key, bool forward, int B);
   void launch_step(hipGraphExec_t g);

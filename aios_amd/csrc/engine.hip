@@ -9,6 +9,7 @@
 #include <mutex>
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <cmath>
 #include <regex>
@@ -96,11 +97,17 @@ Engine::Engine(const EngineConfig& cfg) : cfg_(cfg) {
 
 // Resident launches of a process take turns on a GPU: two of them at once would each hold some of the CUs and wait for the
 // others.  An engine that follows another one waits, on the device, for what that one has queued; the steps of one engine
-// follow each other in its stream anyway.  (Of other processes' launches nothing is known: what the gate is for.)  The lock
-// also keeps a stream from being captured while another engine records its event there.
+// follow each other in its stream anyway.  (Of other processes' launches nothing is known: what the gate is for.)  Nor does a resident
+// launch leave room for the launches of an engine beside it: while another one decodes on the GPU, all take the chain, whose launches share
+// it.  The lock also keeps a stream from being captured while another engine records its event there or asks for its state.
 namespace {
+struct DsUse {
+  hipStream_t stream;
+  std::chrono::steady_clock::time_point at;  // of the last step
+};
 struct DsTurn {
   std::mutex mu;
+  std::map<const void*, DsUse> users;
   const void* last = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev = nullptr;
@@ -116,9 +123,10 @@ DsTurn& ds_turn(int device) {
 Engine::~Engine() {
   if (lm_) (void)hipStreamSynchronize(stream_);
   lm_.reset();
-  if (ds_rows_) {
+  {
     DsTurn& t = ds_turn(cfg_.device);
     std::lock_guard<std::mutex> lock(t.mu);
+    t.users.erase(this);
     if (t.last == this) {
       (void)hipStreamSynchronize(stream_);
       t.last = nullptr;
@@ -918,16 +926,35 @@ bool Engine::ds_next(int B) {
     --ds_rest_;
     return false;
   }
-  return true;
+  return !ds_beside();
+}
+
+// whether another engine decodes on this GPU: its last step was queued within the time of one, or is still on its way
+bool Engine::ds_beside() {
+  DsTurn& t = ds_turn(cfg_.device);
+  std::lock_guard<std::mutex> lock(t.mu);
+  const auto now = std::chrono::steady_clock::now();
+  for (const auto& [who, use] : t.users) {
+    if (who == this) continue;
+    const auto ago = now - use.at;
+    if (ago < std::chrono::milliseconds(2)) return true;
+    if (ago < std::chrono::seconds(10) && hipStreamQuery(use.stream) == hipErrorNotReady) {
+      if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();  // (no error of a launch that is checked next)
+      return true;
+    }
+  }
+  return false;
 }
 
 void Engine::launch_step(hipGraphExec_t g) {
+  DsTurn& t = ds_turn(cfg_.device);
+  std::unique_lock<std::mutex> lock(t.mu);
+  t.users[this] = {stream_, std::chrono::steady_clock::now()};
   if (!ds_now_) {
+    lock.unlock();
     HIP_CHECK(hipGraphLaunch(g, stream_));
     return;
   }
-  DsTurn& t = ds_turn(cfg_.device);
-  std::lock_guard<std::mutex> lock(t.mu);
   if (t.last && t.last != this) {
     if (!t.ev) HIP_CHECK(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
     HIP_CHECK(hipEventRecord(t.ev, t.stream));
@@ -2140,8 +2167,7 @@ hipGraphExec_t Engine::forward_graph(int B) { return captured(graph_key(B, 2), t
 hipGraphExec_t Engine::captured(int key, bool forward, int B) {
   auto it = graphs_.find(key);
   if (it == graphs_.end()) {
-    std::unique_lock<std::mutex> turn;
-    if (ds_rows_) turn = std::unique_lock<std::mutex>(ds_turn(cfg_.device).mu);
+    std::unique_lock<std::mutex> turn(ds_turn(cfg_.device).mu);
     hipGraph_t g;
     HIP_CHECK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
     try {

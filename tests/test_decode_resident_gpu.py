@@ -1,6 +1,7 @@
 """Decode steps of few rows as one resident launch (kernels/decode_stream.hip) against the chain of launches it stands in for."""
 import dataclasses
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -190,20 +191,16 @@ def test_bf16_rows_are_done_by_the_launch_behind(models, contexts):
     assert _rel(got[1], got[0]).max() < TOL16
 
 
-def test_engines_take_turns(models):
+def test_engines_beside_each_other(models):
     """Two engines of a process stepping in two threads: neither holds CUs that the other waits for"""
     engs = [_engine(models(n))[0] for n in ("gqa4-128", "gqa8-64")]
+    tokens = [int(t) for t in np.random.default_rng(13).integers(3, 1000, 100)]
     want, got = [None, None], [None, None]
 
     def run(i, out):
-        eng = engs[i]
-        eng.release_slot(0)
-        eng.prefill(0, [5, 6, 7, 8], 0, False)
-        eng.decode_loop_prepare([0], [17], [4])
-        for _ in range(20):
-            eng.decode_loop_run(1, 10, True)
-        eng.synchronize()
-        out[i] = eng.decode_loop_history(1, 5, 200)
+        engs[i].release_slot(0)
+        engs[i].prefill(0, [5, 6, 7, 8], 0, False)
+        out[i] = _steps(engs[i], 0, tokens, 4)
 
     for i in range(2):
         run(i, want)
@@ -214,7 +211,31 @@ def test_engines_take_turns(models):
         t.join()
     assert [e.decode_resident_failed for e in engs] == [0, 0]
     for g, w in zip(got, want):
-        assert g[:50] == w[:50]
+        assert _rel(g, w).max() < TOL
+
+
+def test_a_step_beside_another_engines_takes_the_chain(models):
+    """A resident launch leaves no room for another engine's launches: both take the chain until one of them rests"""
+    a, b = (_engine(models(n))[0] for n in ("gqa4-128", "gqa8-64"))
+    for e in (a, b):
+        e.prefill(0, [5, 6, 7, 8], 0, False)
+
+    def alone(e):
+        time.sleep(0.05)
+        e.decode([0], [9], [4])
+        return e.decode_resident_last
+
+    assert alone(a) and alone(b)
+    time.sleep(0.05)
+    b.decode_loop_prepare([0], [9], [5])
+    b.decode_loop_run(1, 1500, True)  # some hundred milliseconds
+    a.decode([0], [9], [5])
+    assert not a.decode_resident_last
+    b.synchronize()
+    assert alone(a)
+    del b
+    a.decode([0], [9], [6])
+    assert a.decode_resident_last
 
 
 def test_what_the_resident_step_leaves_to_the_chain(tmp_path):
