@@ -2151,9 +2151,10 @@ void Engine::decode_loop_run(int B, int n_steps, bool use_graph) {
     for (int i = 0; i < n_steps; ++i) enqueue_decode_step(B);
     return;
   }
-  ds_now_ = ds_next(B);
-  hipGraphExec_t ge = step_graph(B);
-  for (int i = 0; i < n_steps; ++i) launch_step(ge);
+  for (int i = 0; i < n_steps; ++i) {  // (another engine may start beside this one)
+    ds_now_ = ds_next(B);
+    launch_step(step_graph(B));
+  }
 }
 
 int Engine::graph_key(int B, int kind) { return B * 4 + kind + (ds_now_ ? 1 << 24 : 0); }

@@ -20,10 +20,11 @@
 // for nobody) does the step.  Behind the open gate every wait is for a workgroup that runs; it is bounded all the same
 // (wait_ticks), with the same way out.
 //
-// A step, us, chain -> resident (MI355X, Q4_K_M): TinyLlama 128 keys 600 -> 464, 1000 keys 682 -> 578; Mistral-7B 128 keys 1424 -> 1190,
-// 3900 keys 1621 -> 1446; with the fp8 cache 2000 keys 1527 -> 1325, 16000 keys 1666 -> 1632; Qwen3-8B 128 keys 1755 -> 1325.
-// TinyLlama bf16, 128 / 1000 keys: one row 742 -> 644 / 818 -> 756, two 815 -> 667 / 887 -> 769, three 839 -> 694 / 899 -> 825, four 854 -> 750 / 904 -> 881
-// (five and more stay with the GEMMs: a fifth row is a second matrix instruction for the same weights, and its operand leaves the ring three slots).
+// A step with its sampler, us, chain -> resident (MI355X).  Q4_K_M: TinyLlama 128 keys 614 -> 465, 1000 keys 695 -> 538; Mistral-7B 128 keys
+// 1434 -> 1149, 2000 keys 1569 -> 1294, 3900 keys 1631 -> 1376; with the fp8 cache 2000 keys 1536 -> 1279, 16000 keys 1675 -> 1548; Qwen3-8B 128
+// keys 1747 -> 1286.  TinyLlama bf16, 128 / 1000 keys: one row 740 -> 592 / 820 -> 646, two 809 -> 611 / 884 -> 663, three 833 -> 640 / 905 -> 696,
+// four 843 -> 691 / 905 -> 738 (five and more stay with the GEMMs: a fifth row is a second matrix instruction for the same weights, and its operand
+// leaves the ring three slots).
 #include "decode_stream.h"
 
 #include <algorithm>
@@ -875,11 +876,11 @@ __device__ __forceinline__ void ds_combine(const DsArgs& a, int l, int unit, int
 
 // ---- the step ---------------------------------------------------------------------------------------------------------------
 // Keys below which a head has one workgroup, that needs no exchange of partial results (3.8 us a layer with the combination), and how many
-// workgroups share the others.  A step, us, one workgroup / several: heads of 64 (TinyLlama bf16) 750 keys 674 / 750, 1500 728 / 764, 1900 763 / 765
-// (four rows: 1500 871 / 891, 1900 922 / 902; Q4_K 1500 602 / 608, 1900 645 / 611); of 128 (Mistral-7B) 500 keys 1278 / 1306, 750 1350 / 1319
-// (fp8 500 1250 / 1287, 1000 1381 / 1301; Qwen3-8B 500 1429 / 1465, 750 1506 / 1477)
+// workgroups share the others.  A step, us, one workgroup / several: heads of 64 (TinyLlama bf16) 750 keys 625 / 689, 1250 660 / 687, 1500 688 / 692
+// (four rows: 1250 767 / 801, 1500 798 / 811; Q4_K 1250 559 / 569, 1500 581 / 572); of 128 (Mistral-7B) 400 keys 1228 / 1241, 500 1231 / 1243, 600
+// 1261 / 1248 (Qwen3-8B 500 1375 / 1385, 600 1412 / 1389)
 template <int HD>
-constexpr int ds_brief() { return 81920 / HD; }
+constexpr int ds_brief() { return HD == 64 ? 1280 : 512; }
 template <int HD, bool F8>
 __device__ __forceinline__ int ds_runs(const DsArgs& a, int G, int pos) {
   if (pos < ds_brief<HD>()) return 1;

@@ -61,9 +61,9 @@ def _rel(a, b):
     return np.linalg.norm(a - b, axis=-1) / np.linalg.norm(b, axis=-1)
 
 
-# the first token, one cached key, a block's border, the borders of one workgroup a head (640 keys of 128, 1280 of 64), passes of 128 and 256
+# the first token, one cached key, a block's border, the borders of one workgroup a head (512 keys of 128, 1280 of 64), passes of 128 and 256
 # keys, a last pass that holds the row's own key alone
-POSITIONS = [0, 1, 127, 128, 511, 512, 638, 639, 640, 767, 1024, 1278, 1280, 1500]
+POSITIONS = [0, 1, 127, 128, 510, 511, 512, 767, 1023, 1024, 1278, 1279, 1280, 1500]
 
 
 @pytest.mark.parametrize("kv", ["bf16", "fp8_e4m3"])
