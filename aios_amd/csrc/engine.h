@@ -442,7 +442,8 @@ class Engine {
   hipGraphExec_t captured(int key, bool forward, int B);
   void launch_step(hipGraphExec_t g);
   DsArgs ds_{};
-  int ds_rows_ = 0, ds_most_ = 0;  // rows of a resident step, at most (0: none); rows of a product that a workgroup has, at most
+  int ds_rows_ = 0;                     // rows of a resident step, at most (0: none)
+  int ds_sums_ = 0, ds_head_sums_ = 0;  // words of the sums of a workgroup's rows (decode_stream.h)
   bool ds_use_ = true;
   bool ds_now_ = false;            // the step being enqueued runs resident
   float* ds_scale_ = nullptr;

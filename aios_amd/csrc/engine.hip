@@ -809,16 +809,18 @@ void Engine::ds_setup() {
   a.eps = cfg_.norm_eps; a.scale = 1.f / std::sqrt((float)hd);
   a.bf16 = bf16; a.bt_stride = kv_maxb_; a.ldl = ldl_;
   if (a.parts < 4) return;
-  auto share = [](int rows, int n) { return (rows + n - 1) / n; };  // rows of one workgroup of n, at most
-  int most = std::max({share(d, a.parts), 4 * share(cfg_.d_ff / 2, a.parts), share(cfg_.vocab_size, a.parts)});
+  // of the rows of one workgroup of n, at most (in units of `unit`)
+  auto sums = [](const QMat& m, int n, int unit = 1) { return ds_sums(m.w, (m.w.rows / unit + n - 1) / n * unit); };
+  ds_sums_ = 0;
   for (const LayerW& L : layers_) {
     int wk, wv;
     ds_shares(L, a.parts, wk, wv);
-    most = std::max({most, share(L.wq.w.rows, wk), share(L.wk.w.rows, wv - wk), share(L.wv.w.rows, a.parts - wv)});
+    ds_sums_ = std::max({ds_sums_, sums(L.wq, wk), sums(L.wk, wv - wk), sums(L.wv, a.parts - wv), sums(L.wo, a.parts),
+                         sums(L.wgu, a.parts, 4), sums(L.wdown, a.parts)});
   }
-  ds_most_ = most;
+  ds_head_sums_ = sums(output_, a.parts);
   int rows = 0;
-  while (rows < cfg_.max_batch && ds_plan(a, hd, most, rows + 1)) ++rows;
+  while (rows < cfg_.max_batch && ds_plan(a, hd, ds_sums_, ds_head_sums_, rows + 1)) ++rows;
   if (!rows) return;
   a.x = x_; a.logits = logits_; a.rope_cs = rope_cs_; a.pos = d_pos_; a.blocks = d_row_bt_;
   auto words = [&](size_t n) {
@@ -1469,7 +1471,7 @@ void Engine::enqueue_decode_forward(int B) {
   nrm_lm_ = false;
   if (ds_now_ && B <= ds_rows_) {
     DsArgs a = ds_;
-    if (!ds_plan(a, cfg_.head_dim, ds_most_, B)) throw std::runtime_error("decode: no resident step of " + std::to_string(B) + " rows");
+    if (!ds_plan(a, cfg_.head_dim, ds_sums_, ds_head_sums_, B)) throw std::runtime_error("decode: no resident step of " + std::to_string(B) + " rows");
     launch_decode_stream(a, cfg_.head_dim, stream_);
     return;
   }

@@ -41,9 +41,9 @@ struct DsArgs {
   int rows;            // of the batch: 1, bf16 up to 4
   int ring;            // (bf16) slots of the ring
   int bt_stride, ldl;  // of the block tables and the logits of a row
-  int row_sums;        // floats of one buffer of row sums in LDS
+  int row_sums;        // words of the sums of a layer product's rows in LDS, of one buffer
   int own_rows;        // rows of the residual that a workgroup has, at most
-  int area_bytes;      // LDS of the staged operand or of the attention's rows
+  int area_bytes;      // LDS of the staged operand (behind the head's its sums) or of the attention's rows
   float eps, scale;
   const float* x;      // the embedding
   float* logits;
@@ -69,8 +69,11 @@ inline size_t ds_part_words(int n_heads, int hd) { return (size_t)n_heads * DS_P
 // rows [r0, r0 + nrows) of matrix w, whose first row is row row0 of the output
 DsCopy ds_job(const QWeight& w, int r0, int nrows, int row0);
 // Whether the step of `rows` rows of such a model can run resident: the shapes that the kernel is built for, its LDS (fills rows,
-// row_sums, own_rows, area_bytes and ring).  max_rows: of a product, a workgroup's.  Formats, ranks and activations are the caller's to check.
-bool ds_plan(DsArgs& a, int head_dim, int max_rows, int rows);
+// row_sums, own_rows, area_bytes and ring).  max_sums, head_sums: words of the sums of a workgroup's rows, of a layer's product at most and of
+// the head.  Formats, ranks and activations are the caller's to check.
+bool ds_plan(DsArgs& a, int head_dim, int max_sums, int head_sums, int rows);
+// words of the sums of this many rows of w
+int ds_sums(const QWeight& w, int rows);
 // the resident launch and the one behind it (which returns at once unless the first gave up)
 void launch_decode_stream(const DsArgs& a, int head_dim, hipStream_t st);
 

@@ -232,7 +232,7 @@ __device__ __forceinline__ float ds_word(const uint64_t* p, uint32_t no, const D
 
 struct DsLds {
   uint8_t* ring;
-  float *rowacc, *red;  // two buffers each
+  float *sums, *red;    // of the rows (ds_sum); squares, two buffers
   DsJob* jobs;          // of this workgroup (the launch with all workgroups)
   float* scale;         // of the caches, per layer
   float* gains;         // of this workgroup's rows, per norm behind a residual
@@ -370,8 +370,31 @@ __device__ __forceinline__ float ds_lanes(float v, int n) {
   return v;
 }
 
-__device__ __forceinline__ void ds_add(float* p, float v) {
-  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+// A row's sum has a term from each group of lanes that holds a run of its columns, and a step done again gives the same logits whatever the order
+// in which the waves come (added to a word of 32 bits in that order, logits of three bf16 rows were 3e-3 apart: an operand on the border between
+// two bf16 values is enough).  Int8 products: each term has a word of LDS, [term][row], and who writes the result adds them up in their order; the
+// words of one product are read before a wave can be past the barrier behind the next operand, so one buffer serves all.  Bf16 products, of more
+// terms for up to four operand rows: sums of 64 bits, in which terms of 24 bits add up without rounding while their exponents lie within 2^24 of
+// each other; two buffers, one of zeros.  us, added in any order / so / the other way: 8 steps of TinyLlama Q4_K_M 3735 / 3755 / 3855, of three rows
+// of TinyLlama bf16 5395 / 5410 / 5620
+// lanes that share a term, of a row of n chunks (or pairs); words of a row's sum
+__host__ __device__ constexpr int ds_run(int n) { return (n & -n) < 64 ? n & -n : 64; }
+__host__ __device__ constexpr int ds_terms(int K, bool q6) {
+  const int n = q6 ? K / 32 : K / 64;
+  return n / ds_run(n);
+}
+// a row's sum of n terms, `stride` apart
+__device__ __forceinline__ float ds_sum(const float* p, int stride, int n) {
+  float v = p[0];
+  int t = 1;
+#pragma clang loop unroll(disable)
+  for (; t + 3 < n; t += 4) {
+    const float a = p[t * stride], b = p[(t + 1) * stride], c = p[(t + 2) * stride], d = p[(t + 3) * stride];
+    v = v + a + b + c + d;
+  }
+#pragma clang loop unroll(disable)
+  for (; t < n; ++t) v += p[t * stride];
+  return v;
 }
 
 // where a thread stands in a product: row and column of its (pair of) chunk(s), or group, in the first slot; what a slot advances them by.  (Worked
@@ -389,10 +412,10 @@ __device__ __forceinline__ DsAt ds_at_first(int first, int slot, int n) {
   return p;
 }
 
-// one slot after the other against the staged operand; row sums in LDS.  A barrier behind each slot (or one)
+// one slot after the other against the staged operand; the terms of the rows' sums to acc.  A barrier behind each slot (or one)
 template <int QT>
 __device__ __forceinline__ void ds_dot(const DsJob& j, const DsAt& p, int nch, int run, int& slot, const DsLds& s, const int8_t* xq, const float2* ms,
-                                       float* acc, float* acc_next, int row_sums) {
+                                       float* acc) {
   using F = DsFmt<QT>;
   const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // this lane's (pair of) chunk(s): place within the slot, and its row and column, which advance by a slot's chunks
@@ -400,6 +423,7 @@ __device__ __forceinline__ void ds_dot(const DsJob& j, const DsAt& p, int nch, i
   int row = p.row, c = p.c;
   const int drow = p.drow, dc = p.dc;
   const int wfirst = F::PAIRS ? 128 * wave : 64 * wave;
+  const int tsh = __builtin_ctz(run) + F::PAIRS;  // chunks of a term
   const bool same = dc == 0;  // the same columns in every slot: the operand stays in registers
   Q4PairX X;
   int xv[8];
@@ -437,9 +461,8 @@ __device__ __forceinline__ void ds_dot(const DsJob& j, const DsAt& p, int nch, i
       v = sc[0] * m.x * (float)is[0] - of[0] * m.y + sc[1] * m.z * (float)is[1] - of[1] * m.w;
     }
     v = ds_lanes(row < j.nrows ? v : 0.f, run);
-    if ((lane & (run - 1)) == 0 && row < j.nrows) ds_add(acc + row, v);
+    if ((lane & (run - 1)) == 0 && row < j.nrows) acc[(c >> tsh) * j.nrows + row] = v;
   };
-  for (int i = tid; i < row_sums; i += DS_CT) acc_next[i] = 0.f;
   if (same && j.slots) load();
 #pragma clang loop unroll(disable)
   for (int t = 0; t < j.slots; ++t) {
@@ -464,15 +487,14 @@ __device__ __forceinline__ void ds_dot(const DsJob& j, const DsAt& p, int nch, i
 // operand row i, columns 8 b ..), so each byte of weights is read from LDS once whatever the rows, beside as much of the operand
 typedef short ds_s16x4 __attribute__((ext_vector_type(4)));
 typedef float ds_f32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void ds_dot16(const DsJob& j, const DsAt& p, int K, int rows, int ring, int& cur, const DsLds& s, const uint8_t* xb, float* acc,
-                                         float* acc_next, int row_sums) {
+__device__ __forceinline__ void ds_dot16(const DsJob& j, const DsAt& p, int K, int rows, int ring, int& cur, const DsLds& s, const uint8_t* xb,
+                                         double* acc) {
   const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 3, b = lane >> 2, g = wave >> 1, half = wave & 1;
   const int KQ = K >> 9;
   int rg = p.row, kq = p.c;
   const uint8_t* x = xb + (size_t)min(i, rows - 1) * (2 * K + DS_BPAD) + (half * 32 + b) * 16;
   const int w0 = g * 4096 + i * 1024 + ((half * 32 + b + 4 * i) & 63) * 16, w1 = g * 4096 + i * 1024 + ((half * 32 + 16 + b + 4 * i) & 63) * 16;
-  for (int n = tid; n < row_sums; n += DS_CT) acc_next[n] = 0.f;
 #pragma clang loop unroll(disable)
   for (int t = 0; t < j.slots; ++t) {
     if (wave < 2 * DS_BGROUPS && t * DS_BGROUPS + g < j.chunks) {
@@ -497,7 +519,7 @@ __device__ __forceinline__ void ds_dot16(const DsJob& j, const DsAt& p, int K, i
       v += lane_dpp<0x124>(v);  // row_ror:4
       v += lane_dpp<0x128>(v);  // row_ror:8
       const int row = rg * 4 + (lane >> 4);
-      if ((lane & 15) < rows && row < j.nrows) ds_add(acc + row * DS_BROWS + i, v);
+      if ((lane & 15) < rows && row < j.nrows) __hip_atomic_fetch_add(acc + row * DS_BROWS + i, (double)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     rg += p.drow;
     kq += p.dc;
@@ -896,14 +918,14 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
   DsLds s;
   s.ring = smem;
   s.area = smem + (BF ? a.ring * DS_BSLOT : DS_R * DS_SLOT);
-  s.rowacc = (float*)(s.area + a.area_bytes);
-  s.red = s.rowacc + 2 * a.row_sums;
+  s.sums = (float*)(s.area + a.area_bytes);
+  s.red = s.sums + (BF ? 2 : 1) * a.row_sums;
   constexpr int RED = ds_red<BF>();
   unsigned* gate = (unsigned*)(s.red + 2 * RED);
   s.scale = s.red + 2 * RED + 4;
   s.jobs = (DsJob*)(s.scale + (2 * a.n_layers + 3) / 4 * 4);
   s.gains = (float*)(s.jobs + 4 * a.n_layers + 1);
-  constexpr int SH = BF ? 2 : 0;  // a product's row has sums of four operand rows in LDS, or one
+  constexpr int SH = BF ? 2 : 0;  // a product's row is four threads' that write it, of the operand's rows, or one's
   const int rows = BF ? a.rows : 1;
   auto pos_of = [&](int b) { return min(ds_table(a.pos, b), a.max_ctx - 1); };
   const int qd = a.n_heads * HD;
@@ -984,6 +1006,8 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
         const bool wrap = wg + step >= a.parts;
         slots = ds_table(&a.jobs->job.slots, (min(q + wrap, last) * a.parts + (wrap ? first : wg + step)) * 16);
         if (!n) lg_barrier();
+        if constexpr (BF)
+          if (a.alone && q == last) lg_barrier();
         for (int t = 0; t < n; ++t) {
           if constexpr (BF) ds_wait(2 * DS_BGROUPS * --ahead);
           else ds_wait(t || owed ? h0 + h1 : h0 + h1 + h2);
@@ -1033,7 +1057,9 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
     gate[0] = go;
     gate[1] = no;
   }
-  for (int i = tid; i < 2 * a.row_sums + 2 * RED; i += DS_CT) s.rowacc[i] = 0.f;
+  for (int i = tid; i < 2 * RED; i += DS_CT) s.red[i] = 0.f;
+  if constexpr (BF)
+    for (int i = tid; i < 2 * a.row_sums; i += DS_CT) s.sums[i] = 0.f;
   for (int i = tid; i < 2 * a.n_layers; i += DS_CT) s.scale[i] = a.kv_scale[i];
   for (int i = tid; i <= 4 * a.n_layers; i += DS_CT) s.jobs[i] = a.jobs[(size_t)i * a.parts + first].job;
   {
@@ -1093,7 +1119,8 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
         j.chunks &= ~DS_Q6;
         const int K = kind == DS_O ? qd : (kind == DS_DOWN ? a.ff : a.d), nch = K >> 5;
         float2* ms = (float2*)(xq + K);
-        float* acc = s.rowacc + par * a.row_sums;
+        // (of the head's rows, which are more, from behind its operand on)
+        float* acc = q == last ? (float*)(xq + (BF ? rows * (2 * K + DS_BPAD) : K + K / 2)) : s.sums + (BF ? par * a.row_sums : 0);
         float* red = s.red + par * RED;
         par ^= 1;
         const bool resid = kind == DS_O || kind == DS_DOWN;
@@ -1116,6 +1143,11 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
                                ms, red, clk);
           if (kind != DS_O) ds_squares<BF>(a, a.sq + (size_t)nr * rows * a.parts, nx, rows, red, clk);
         }
+        if constexpr (BF)
+          if (q == last) {
+            if (a.alone) lg_barrier();  // (the part before may still be read)
+            for (int i = tid; i < 2 * DS_BROWS * j.nrows; i += DS_CT) acc[i] = 0.f;
+          }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         lg_barrier();  // the operand is staged, slot 0 there
         float inv = 1.f;
@@ -1129,14 +1161,18 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
           }
           inv = rsqrtf(t / (float)K + a.eps);
         }
-        float* acc_next = s.rowacc + par * a.row_sums;
         if constexpr (BF) {
-          ds_dot16(j, place, K, rows, a.ring, slot, s, xq, acc, acc_next, a.row_sums);
+          for (int i = tid; i < a.row_sums; i += DS_CT) s.sums[par * a.row_sums + i] = 0.f;  // the next product's
+          ds_dot16(j, place, K, rows, a.ring, slot, s, xq, (double*)acc);
         } else {
-          const int low = nch & -nch;  // (the largest power of two in it: lanes that share a row)
-          if (q6) ds_dot<QT_Q6_K>(j, place, nch, min(low, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
-          else ds_dot<QT_Q4_K>(j, place, nch, min(low >> 1, 64), slot, s, (int8_t*)xq, ms, acc, acc_next, a.row_sums);
+          if (q6) ds_dot<QT_Q6_K>(j, place, nch, ds_run(nch), slot, s, (int8_t*)xq, ms, acc);
+          else ds_dot<QT_Q4_K>(j, place, nch, ds_run(nch >> 1), slot, s, (int8_t*)xq, ms, acc);
         }
+        const int n1 = q6 ? nch : nch >> 1, terms = n1 >> __builtin_ctz(ds_run(n1));
+        auto sum = [&](int i) __attribute__((always_inline)) {
+          if constexpr (BF) return (float)((const double*)acc)[i];
+          else return ds_sum(acc + i, j.nrows, terms);
+        };
         // (what all other workgroups wait for: in front of the waves that go on to the next operand.  Those may not skip this part, though they
         // have nothing to write: waiting earlier they take more from the writing wave than the priority gives back)
         if (writes) __builtin_amdgcn_s_setprio(3);
@@ -1144,7 +1180,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
           // (rows by the last wave's lanes, further ones by those before; the squares go with the first word)
           const int r = rt >> SH;
           const bool on = rt < n && b < rows;
-          const float x = on ? own + acc[rt] : 0.f;
+          const float x = on ? own + sum(rt) : 0.f;
           float gain = s.gains[nr * a.own_rows + min(r, a.own_rows - 1)];
           if (a.alone) {
             gain = a.gains[(size_t)(nr + 1) * a.d + j.r0 + (on ? r : 0)];
@@ -1166,15 +1202,15 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
           if (rt < rows) ds_put(a.sq + ((size_t)nr * rows + rt) * a.parts + wg, __float_as_uint(sq), no);
         } else if (b < rows) {
           if (q == last) {
-            for (int i = rt; i < n; i += DS_CT) a.logits[(size_t)b * a.ldl + j.r0 + (i >> SH)] = acc[i] * inv;
+            for (int i = rt; i < n; i += DS_CT) a.logits[(size_t)b * a.ldl + j.r0 + (i >> SH)] = sum(i) * inv;
           } else if (kind == DS_QKV) {
-            for (int i = rt; i < n; i += DS_CT) ds_put(a.qkv + ((size_t)l * rows + b) * a.nqkv + j.r0 + (i >> SH), __float_as_uint(acc[i] * inv), no);
+            for (int i = rt; i < n; i += DS_CT) ds_put(a.qkv + ((size_t)l * rows + b) * a.nqkv + j.r0 + (i >> SH), __float_as_uint(sum(i) * inv), no);
           } else {
             for (int i = rt; i < n >> 2; i += DS_CT) {
               const int u = i >> SH;
               float v[4];
 #pragma unroll
-              for (int k = 0; k < 4; ++k) v[k] = acc[((4 * u + k) << SH) + b];
+              for (int k = 0; k < 4; ++k) v[k] = sum(((4 * u + k) << SH) + b);
               const float f0 = glu_act(v[0] * inv, ACT_SILU) * (v[1] * inv), f1 = glu_act(v[2] * inv, ACT_SILU) * (v[3] * inv);
               ds_put(a.h + ((size_t)l * rows + b) * (a.ff / 2) + ds_at16((j.r0 >> 2) + u), (uint32_t)f32_to_bf16(f0) | (uint32_t)f32_to_bf16(f1) << 16, no);
             }
@@ -1202,7 +1238,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
 // LDS behind the ring and the operand
 int ds_rest(const DsArgs& a) {
   const int red = a.bf16 ? ds_red<true>() : ds_red<false>();
-  return (2 * a.row_sums + 2 * red + 4 + (2 * a.n_layers + 3) / 4 * 4) * 4 + (4 * a.n_layers + 1) * (int)sizeof(DsJob) + 2 * a.n_layers * a.own_rows * 4;
+  return ((a.bf16 ? 2 : 1) * a.row_sums + 2 * red + 4 + (2 * a.n_layers + 3) / 4 * 4) * 4 + (4 * a.n_layers + 1) * (int)sizeof(DsJob) + 2 * a.n_layers * a.own_rows * 4;
 }
 int ds_lds(const DsArgs& a) { return (a.bf16 ? a.ring * DS_BSLOT : DS_R * DS_SLOT) + a.area_bytes + ds_rest(a); }
 
@@ -1257,22 +1293,26 @@ DsCopy ds_job(const QWeight& w, int r0, int nrows, int row0) {
   return j;
 }
 
-bool ds_plan(DsArgs& a, int hd, int max_rows, int rows) {
+int ds_sums(const QWeight& w, int rows) { return w.qtype == QT_BF16 ? rows * 2 * DS_BROWS : rows * ds_terms(w.cols, w.qtype == QT_Q6_K); }
+
+bool ds_plan(DsArgs& a, int hd, int max_sums, int head_sums, int rows) {
   const int qd = a.n_heads * hd, g = a.n_heads / a.n_kv_heads;
   if ((hd != 64 && hd != 128) || a.n_heads % a.n_kv_heads || !(g == 1 || g == 2 || g == 4 || g == 8)) return false;
   // whole waves of octets, rows that 16 chunks divide; every workgroup with rows of O, gate/up and down (see the exchanges above)
   if (a.d % 512 || qd % 512 || a.ff % 512 || a.d < 2 * a.parts || a.ff / 2 < 2 * a.parts) return false;
   if (rows < 1 || rows > (a.bf16 ? DS_BROWS : 1) || rows * a.n_heads > a.parts) return false;
-  const int width = a.bf16 ? DS_BROWS : 1;  // sums of a product's row
+  const int width = a.bf16 ? DS_BROWS : 1;  // threads of a row that is written
   a.rows = rows;
   a.own_rows = (a.d + a.parts - 1) / a.parts;
   if (a.own_rows * width > 64) return false;  // (a wave holds a workgroup's rows of the residual)
   const int K = std::max({a.d, qd, a.ff});
   const int gl = g % 4 == 0 ? 4 : g;
   const int attn = gl * hd * 2 + 2 * hd * 2 + DS_AW * gl * 2 * 4 + DS_AW * gl * hd * 4;
-  const int operand = a.bf16 ? rows * (2 * K + DS_BPAD) : K + K / 2;
-  a.area_bytes = (std::max({operand, attn, DS_PMAX * 18 * 4}) + 255) / 256 * 256;
-  a.row_sums = (max_rows * width + 63) / 64 * 64;
+  auto operand = [&](int k) { return a.bf16 ? rows * (2 * k + DS_BPAD) : k + k / 2; };
+  a.row_sums = (max_sums + 63) / 64 * 64;
+  // (int8: the head's sums run on into the layers')
+  const int head = operand(a.d) + head_sums * 4 - (a.bf16 ? 0 : a.row_sums * 4);
+  a.area_bytes = (std::max({operand(K), head, attn, DS_PMAX * 18 * 4}) + 255) / 256 * 256;
   if (a.bf16) {
     // sums of squares: 64 workgroups a word of LDS, or 512 columns
     if (a.parts % 64 || rows * std::max(a.parts / 64, a.d / 512) > ds_red<true>()) return false;

@@ -135,6 +135,22 @@ def test_resident_step_matches_the_reference(models, shape):
     assert (got - want).abs().max().item() < 2e-2 * max(want.abs().max().item(), 1.0)
 
 
+@pytest.mark.parametrize("shape,recipe,batch", [("gqa8-64", "Q4_K_M", 1), ("qwen", "BF16", 1), ("gqa4-64", "BF16", 3), ("mha-64", "BF16", 4)])
+def test_a_step_done_again_gives_the_same_logits(models, shape, recipe, batch):
+    """Rows whose sums have more terms than two, added in the order in which the waves come"""
+    eng, cfg = _engine(models(shape, recipe), max_batch=4, max_slots=4)
+    slots = list(range(batch))
+    for s in slots:
+        eng.prefill(s, [int(t) for t in np.random.default_rng(s).integers(3, cfg.vocab_size, 40 + s)], 0, False)
+    first = None
+    for _ in range(30):
+        eng.decode(slots, [11 + s for s in slots], [40 + s for s in slots])
+        assert eng.decode_resident_last
+        got = np.asarray(eng.last_logits(batch)).copy()
+        first = got if first is None else first
+        assert np.array_equal(got, first)
+
+
 def test_pipelined_and_looped_steps_are_resident_too(models):
     eng, cfg = _engine(models("gqa4-128"))
     prompt = [int(t) for t in np.random.default_rng(7).integers(3, cfg.vocab_size, 120)]
