@@ -446,7 +446,7 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       .def_property_readonly("decode_resident_last", &Engine::decode_resident_last)
       .def_property_readonly("decode_resident_failed", &Engine::decode_resident_failed)
       .def("set_decode_resident", &Engine::set_decode_resident, py::arg("on"))
-      .def("set_decode_resident_wait", &Engine::set_decode_resident_wait, py::arg("ticks"))
+      .def("set_decode_resident_wait", &Engine::set_decode_resident_wait, py::arg("ticks"), py::arg("behind") = -1)
       .def("capture_graphs", &Engine::capture_graphs, py::arg("max_b"), py::call_guard<py::gil_scoped_release>())
       .def_property_readonly("stream", &Engine::stream_handle)
       .def_property_readonly("k_cache_ptr", &Engine::kv_cache_k)

@@ -192,12 +192,12 @@ class Engine {
   int kv_blocks_total() const { return kv_nblocks_; }
   // decode steps of few rows as one resident launch (decode_stream.h): rows up to which this engine's steps take it; off for tests
   // and comparisons; steps that its launch gave up on (another resident launch held part of the GPU) and that were done
-  // without it; the time, in 10 ns, after which it gives up
+  // without it; the time, in 10 ns, after which it gives up at its gate, and in a wait behind it (negative: as it was)
   int decode_resident() const;
   bool decode_resident_last() const { return ds_now_; }  // whether the last step queued was one
   void set_decode_resident(bool on) { ds_use_ = on; }
   unsigned decode_resident_failed() const { return ds_failed_ ? *(volatile unsigned*)ds_failed_ : 0; }
-  void set_decode_resident_wait(unsigned long long ticks);
+  void set_decode_resident_wait(unsigned long long ticks, long long behind = -1);
   int decode_gemm_min_batch() const { return dec_gemm_min_b_; }  // rows from which decode takes the GEMMs
   int norm_fused_parts() const { return nrm_parts_; }  // 0: batched-decode RMSNorm not split into the GEMMs
   // of the last prompt's portions above 32 rows: norms split over two products, QKV products that wrote q and the cache themselves

@@ -911,9 +911,10 @@ void Engine::ds_upload() {
 
 int Engine::decode_resident() const { return ds_use_ ? ds_rows_ : 0; }
 
-void Engine::set_decode_resident_wait(unsigned long long ticks) {
+void Engine::set_decode_resident_wait(unsigned long long ticks, long long behind) {
   if (finalized_) HIP_CHECK(hipStreamSynchronize(stream_));
   ds_.gate_ticks = ticks;
+  if (behind >= 0) ds_.wait_ticks = behind;
   reset_graphs();
 }
 

@@ -20,10 +20,9 @@ struct alignas(64) DsCopy {
 
 // what launches leave each other; all zero before the first one
 struct DsCtl {
-  unsigned arrive, state, done;  // of the running launch: workgroups there, 1 go / 2 given up, workgroups gone
+  unsigned arrive, state, done;  // of the running launch: workgroups there, 1 go / 2 given up, workgroups gone (above 16 bits: that waited too long)
   unsigned epoch;                // numbers of the exchanges used so far
   unsigned failed;               // the last resident launch gave up: the launch behind it does the step
-  unsigned late;                 // ... because a workgroup waited too long for others that were there
   unsigned alone;                // steps that the launch behind did
 };
 

@@ -40,6 +40,7 @@ namespace {
 constexpr int DS_NG = 14, DS_NL = 2, DS_CT = DS_NG * 64, DS_THREADS = (DS_NG + DS_NL) * 64;
 constexpr int DS_SLOT = 32768, DS_R = 4;
 constexpr int DS_AW = 8;  // waves that attend
+constexpr unsigned DS_LATE = 1 << 16;  // of DsCtl::done: a workgroup that gave up waiting
 
 // bf16 weights, up to four rows: a slot is four groups of four rows by 512 columns, a KB a row; 8 waves take half a group each
 constexpr int DS_BROWS = 4, DS_BSLOT = 16384, DS_BGROUPS = 4, DS_BPAD = 64;
@@ -173,11 +174,11 @@ __device__ __forceinline__ uint64_t ds_get(const uint64_t* p) {
 
 struct DsClock {
   unsigned long long t0, limit;
-  unsigned* late;
+  unsigned* late;  // (LDS: signed out with)
 };
 __device__ __forceinline__ bool ds_late(const DsClock& c) {
-  if (__builtin_amdgcn_s_memrealtime() - c.t0 <= c.limit) return false;
-  __hip_atomic_store(c.late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_expect(__builtin_amdgcn_s_memrealtime() - c.t0 <= c.limit, 1)) return false;
+  *c.late = 1;
   return true;
 }
 
@@ -189,13 +190,13 @@ __device__ __forceinline__ bool ds_late(const DsClock& c) {
 template <int N, int U>
 __device__ __forceinline__ void ds_poll(const uint64_t* const (&p)[U], int stride, uint32_t no, uint32_t (&v)[U][N], const DsClock& c) {
   uint64_t w[U][N];
-  for (int it = 1;; ++it) {
+  for (int it = c.limit ? 1 : 64;; ++it) {  // (the time is looked at every 64 rounds; with none to wait, in the first)
     bool ok = true;
 #pragma unroll
     for (int u = 0; u < U; ++u) w[u][0] = ds_get(p[u]);
 #pragma unroll
     for (int u = 0; u < U; ++u) ok = ok && (uint32_t)(w[u][0] >> 32) == no;
-    if (ok || ((it & 63) == 0 && ds_late(c))) break;
+    if (ok || (__builtin_expect((it & 63) == 0, 0) && ds_late(c))) break;
   }
 #pragma unroll
   for (int u = 0; u < U; ++u)
@@ -210,7 +211,7 @@ __device__ __forceinline__ void ds_poll(const uint64_t* const (&p)[U], int strid
       v[u][i] = (uint32_t)w[u][i];
       ok = ok && (uint32_t)(w[u][i] >> 32) == no;
     }
-  for (int it = 1; !ok; ++it) {
+  for (int it = c.limit ? 1 : 64; !ok; ++it) {
     ok = true;
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -220,7 +221,7 @@ __device__ __forceinline__ void ds_poll(const uint64_t* const (&p)[U], int strid
         v[u][i] = (uint32_t)w[u][i];
         ok = ok && (uint32_t)(w[u][i] >> 32) == no;
       }
-    if ((it & 63) == 0 && ds_late(c)) break;
+    if (__builtin_expect((it & 63) == 0, 0) && ds_late(c)) break;
   }
 }
 __device__ __forceinline__ float ds_word(const uint64_t* p, uint32_t no, const DsClock& c) {
@@ -1038,7 +1039,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
 
   // ---- sign in, wait for the others
   DsCtl* ctl = a.ctl;
-  DsClock clk{__builtin_amdgcn_s_memrealtime(), a.wait_ticks, &ctl->late};
+  DsClock clk{__builtin_amdgcn_s_memrealtime(), a.wait_ticks, gate + 2};
   if (tid == 0) {
     unsigned go = 1;
     const unsigned no = __hip_atomic_load(&ctl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1056,6 +1057,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
     }
     gate[0] = go;
     gate[1] = no;
+    gate[2] = 0;
   }
   for (int i = tid; i < 2 * RED; i += DS_CT) s.red[i] = 0.f;
   if constexpr (BF)
@@ -1220,16 +1222,17 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
       }
     }
   }
-  // ---- sign out; the last one clears the gate and says whether the step is done
+  // ---- sign out, late workgroups with a count of their own in the same word, so that the last one has seen them all; it clears the gate and says
+  // whether the step is done
   if (tid == 0) {
-    if (__hip_atomic_fetch_add(&ctl->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x) {
-      const unsigned late = __hip_atomic_load(&ctl->late, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned mine = go && gate[2] ? DS_LATE + 1 : 1;
+    const unsigned gone = __hip_atomic_fetch_add(&ctl->done, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine;
+    if (gone % DS_LATE == gridDim.x) {
       ctl->arrive = 0;
       ctl->state = 0;
       ctl->done = 0;
-      ctl->late = 0;
       ctl->epoch = no0 - 1 + a.n_layers;
-      ctl->failed = !a.alone && (!go || late);
+      ctl->failed = !a.alone && (!go || gone > DS_LATE);
       if (a.alone) __hip_atomic_store(a.host_failed, ++ctl->alone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }

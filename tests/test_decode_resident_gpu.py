@@ -195,6 +195,20 @@ def test_a_launch_that_cannot_be_resident_is_done_by_the_one_behind(models, shap
     assert _rel(got[1], got[0]).max() < TOL
 
 
+@pytest.mark.parametrize("shape,recipe,batch", [("gqa8-64", "Q4_K_M", 1), ("qwen", "BF16", 3)])
+def test_a_launch_that_loses_a_wait_is_done_by_the_one_behind(models, shape, recipe, batch):
+    """No time to wait behind the open gate: waits end with words of no number, the last workgroup to sign out sees the flag of the
+    first that gave up, and the launch behind does the step over"""
+    eng, cfg = _engine(models(shape, recipe), max_batch=4, max_slots=4)
+    contexts = [600, 30, 5][:batch]
+    want = _rows(eng, cfg, contexts, list(range(batch)), 3)
+    assert eng.decode_resident_last and eng.decode_resident_failed == 0
+    eng.set_decode_resident_wait(2000000, 0)
+    got = _rows(eng, cfg, contexts, list(range(batch)), 3)
+    assert eng.decode_resident_failed == 1
+    assert _rel(got, want).max() < (TOL if recipe == "Q4_K_M" else TOL16)
+
+
 @pytest.mark.parametrize("contexts", [[5], [3, 600, 40], [0, 10, 20, 30]])
 def test_bf16_rows_are_done_by_the_launch_behind(models, contexts):
     eng, cfg = _engine(models("gqa8-64", "BF16"), max_batch=4, max_slots=4)
