@@ -5,6 +5,7 @@
 #include <set>
 #include "comm.h"
 #include <cstdlib>
+#include <unistd.h>
 #include <map>
 #include <mutex>
 
@@ -786,11 +787,26 @@ void Engine::finalize() {
   finalized_ = true;
 }
 
+// Whether the environment asks for the chain of launches: AIOS_DECODE_RESIDENT=0, or a setting of its launches that is not the default (32 bits
+// between gate/up and down, the GEMVs or GEMMs of some rows, their tuning, the attention's)
+static bool ds_chain_asked() {
+  for (const char* on : {"AIOS_DECODE_RESIDENT", "AIOS_FF16", "AIOS_GEMV_LDS", "AIOS_GEMV_BF16_LDS", "AIOS_GEMM_WK", "AIOS_STEP_PREP", "AIOS_Q8_BALANCE"}) {
+    const char* e = std::getenv(on);
+    if (e && std::atoi(e) != 1) return true;
+  }
+  for (char** e = environ; e && *e; ++e)
+    for (const char* set : {"AIOS_DECODE_GEMM_MIN_B=", "AIOS_GEMV_LDS_", "AIOS_GEMV_CU=", "AIOS_GEMV_U_", "AIOS_GEMV_GRID_", "AIOS_GEMV_KSPLIT_", "AIOS_LDS_B1_",
+                            "AIOS_LB_CFG=", "AIOS_QKV_DBG=", "AIOS_ATTN_", "AIOS_SKINNY_", "AIOS_GEMM_RING=", "AIOS_GEMM_NORM_FUSE=",
+                            "AIOS_GEMM_QKV_EPI_MAX_B="})
+      if (std::strncmp(*e, set, std::strlen(set)) == 0) return true;
+  return false;
+}
+
 // The step of few rows as one resident launch (decode_stream.h): a GPU to itself, every matrix Q4_K or Q6_K with int8 activations
 // (one row) or every one bf16 (up to four).  (A rank of several, or a tier on some of the CUs, would wait for others inside the launch; the other
-// formats have their own GEMVs.  AIOS_DECODE_GEMM_MIN_B=0 asks for the GEMVs alone.)
+// formats have their own GEMVs.)
 void Engine::ds_setup() {
-  if (dec_gemm_min_b_ <= 0) return;
+  if (ds_chain_asked()) return;
   if (lm_ || cfg_.tp_size > 1 || cfg_.vocab_parallel || !cfg_.cu_mask.empty() || !rope_cs_ || cfg_.n_layers < 1) return;
   const bool bf16 = output_.valid() && output_.w.qtype == QT_BF16;
   if (!bf16 && !cfg_.act_q8) return;

@@ -277,3 +277,16 @@ def test_what_the_resident_step_leaves_to_the_chain(tmp_path):
         eng, cfg, _ = load_engine(path, max_ctx=128, max_batch=1, **kw)
         assert not eng.decode_resident
         assert 0 <= eng.decode([0], [1], [0])[0] < cfg.vocab_size
+
+
+@pytest.mark.parametrize("recipe,name,value", [
+    ("Q4_K_M", "AIOS_DECODE_RESIDENT", "0"), ("Q4_K_M", "AIOS_FF16", "0"), ("BF16", "AIOS_FF16", "0"), ("BF16", "AIOS_GEMV_BF16_LDS", "0"),
+    ("Q4_K_M", "AIOS_GEMV_LDS", "0"), ("Q4_K_M", "AIOS_GEMV_GRID_O", "128"), ("Q4_K_M", "AIOS_DECODE_GEMM_MIN_B", "1"),
+    ("BF16", "AIOS_DECODE_GEMM_MIN_B", "5"), ("Q4_K_M", "AIOS_FF16", "1"), ("BF16", "AIOS_DECODE_RESIDENT", "1")])
+def test_what_the_environment_asks_of_the_chain_is_done_by_it(models, monkeypatch, recipe, name, value):
+    monkeypatch.setenv(name, value)
+    eng, _, _ = load_engine(models("gqa4-64", recipe), max_ctx=256, max_batch=2)
+    default = value == "1" and name != "AIOS_DECODE_GEMM_MIN_B"
+    assert bool(eng.decode_resident) == default
+    eng.decode([0], [5], [0])
+    assert eng.decode_resident_last == default
