@@ -535,11 +535,9 @@ __device__ __forceinline__ void ds_dot16(const DsJob& j, const DsAt& p, int K, i
   lg_barrier();
 }
 
-// tiles of keys that a wave has in flight (a request is 1 KB, of fp8 512 B), keys of a workgroup's pass
-template <int HD, bool F8>
-constexpr int ds_tiles() { return 1; }
-template <int HD, bool F8>
-constexpr int ds_pass() { return ds_tiles<HD, F8>() * DS_AW * 4 * (512 / HD); }
+// keys of a workgroup's pass: a tile of four requests (of 1 KB, of fp8 512 B) a wave
+template <int HD>
+constexpr int ds_pass() { return DS_AW * 4 * (512 / HD); }
 
 // ---- attention -----------------------------------------------------------------------------------------------------------
 // G query heads of one KV head over the passes sp, sp + P, .. of its keys (attn_lanes of attn_decode.h, with the heads sharing what is
@@ -588,7 +586,7 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
   S& L = *(S*)s.area;
   constexpr int LPK = HD / 8, KPS = 64 / LPK;  // lanes of a key (8 elements each), keys of a request
   constexpr int STEPS = 4, KPW = STEPS * KPS;  // requests of a tile, its keys
-  constexpr int NT = ds_tiles<HD, F8>(), PASS = ds_pass<HD, F8>(), ES = F8 ? 1 : 2;
+  constexpr int PASS = ds_pass<HD>(), ES = F8 ? 1 : 2;
   using KVT = typename std::conditional<F8, uint2, uint4>::type;
   const int units = a.n_heads / G;
   const int tid = ds_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -606,8 +604,8 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
   const int h0 = at.unit * G, gq = a.n_heads / a.n_kv_heads, kvh = h0 / gq;
   const int ksub = lane / LPK, dsl = lane % LPK;
   uint8_t *kc = a.kc + (size_t)l * a.kv_layer, *vc = a.vc + (size_t)l * a.kv_layer;
-  KVT kr[NT][STEPS], vr[NT][STEPS];
-  auto first_key = [&](int pass, int t) { return pass * PASS + t * (DS_AW * KPW) + wave * KPW; };
+  KVT kr[STEPS], vr[STEPS];
+  auto first_key = [&](int pass) { return pass * PASS + wave * KPW; };
   // a tile is a buffer of its live keys' bytes: what lies behind them reads as zeros without a memory access
   const int voff = (ksub * HD + dsl * 8) * ES;
   auto request = [&](KVT (&r)[STEPS], const uint8_t* pool, int k0) __attribute__((always_inline)) {
@@ -627,11 +625,8 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
   };
   const int npass = pos / PASS + 1;
   if (wave < DS_AW) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      request(kr[t], kc, first_key(sp, t));
-      request(vr[t], vc, first_key(sp, t));
-    }
+    request(kr, kc, first_key(sp));
+    request(vr, vc, first_key(sp));
   }
   // ---- the heads' raw vectors
   if (tid < (G + 2) * HD) {
@@ -772,38 +767,35 @@ __device__ __forceinline__ void ds_attend(const DsArgs& a, int l, int wg, int P,
       });
     };
     for (int pass = sp; pass < npass; pass += P) {
+      const int k0 = first_key(pass), kn = first_key(pass + P);
+      float sc[STEPS][NS], mx[NS];
+      read_q();
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int k0 = first_key(pass, t), kn = first_key(pass + P, t);
-        float sc[STEPS][NS], mx[NS];
-        read_q();
-#pragma unroll
-        for (int i = 0; i < STEPS; ++i) {
-          score(kr[t][i], sc[i], k0 + ksub + i * KPS < pos);
-          __builtin_amdgcn_sched_barrier(0);  // (steps interleaved spill)
-        }
-        if (pass + P < npass) request(kr[t], kc, kn);
-#pragma unroll
-        for (int n = 0; n < NS; ++n) {
-          mx[n] = sc[0][n];
-#pragma unroll
-          for (int i = 1; i < STEPS; ++i) mx[n] = fmaxf(mx[n], sc[i][n]);
-        }
-        weigh(mx);
-#pragma unroll
-        for (int n = 0; n < NS; ++n)
-#pragma unroll
-          for (int i = 0; i < STEPS; ++i) {
-            sc[i][n] = fast_exp2(sc[i][n] - m[n]);
-            sum[n] += sc[i][n];
-          }
-#pragma unroll
-        for (int i = 0; i < STEPS; ++i) {
-          add(vr[t][i], sc[i]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (pass + P < npass) request(vr[t], vc, kn);
+      for (int i = 0; i < STEPS; ++i) {
+        score(kr[i], sc[i], k0 + ksub + i * KPS < pos);
+        __builtin_amdgcn_sched_barrier(0);  // (steps interleaved spill)
       }
+      if (pass + P < npass) request(kr, kc, kn);
+#pragma unroll
+      for (int n = 0; n < NS; ++n) {
+        mx[n] = sc[0][n];
+#pragma unroll
+        for (int i = 1; i < STEPS; ++i) mx[n] = fmaxf(mx[n], sc[i][n]);
+      }
+      weigh(mx);
+#pragma unroll
+      for (int n = 0; n < NS; ++n)
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+          sc[i][n] = fast_exp2(sc[i][n] - m[n]);
+          sum[n] += sc[i][n];
+        }
+#pragma unroll
+      for (int i = 0; i < STEPS; ++i) {
+        add(vr[i], sc[i]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (pass + P < npass) request(vr, vc, kn);
     }
     if (wave == 0 && sp == 0) {  // the row's own key, by the first key group
       float sc[NS];
@@ -904,10 +896,10 @@ __device__ __forceinline__ void ds_combine(const DsArgs& a, int l, int unit, int
 // 1261 / 1248 (Qwen3-8B 500 1375 / 1385, 600 1412 / 1389)
 template <int HD>
 constexpr int ds_brief() { return HD == 64 ? 1280 : 512; }
-template <int HD, bool F8>
+template <int HD>
 __device__ __forceinline__ int ds_runs(const DsArgs& a, int G, int pos) {
   if (pos < ds_brief<HD>()) return 1;
-  return min(min(pos / ds_pass<HD, F8>() + 1, a.parts / (a.rows * (a.n_heads / G))), DS_PMAX);
+  return min(min(pos / ds_pass<HD>() + 1, a.parts / (a.rows * (a.n_heads / G))), DS_PMAX);
 }
 
 template <int HD, int G, bool F8, bool BF>
@@ -934,7 +926,7 @@ __global__ void __launch_bounds__(DS_THREADS) decode_stream_kernel(DsArgs a) {
   if constexpr (BF)
     for (int b = 1; b < rows; ++b) pos = max(pos, pos_of(b));
   const bool brief = pos < ds_brief<HD>();
-  const int P = ds_runs<HD, F8>(a, G, pos);
+  const int P = ds_runs<HD>(a, G, pos);
   const int nattend = rows * (brief ? a.n_heads : a.n_heads / G * P);  // parts that attend
   const int ncomb = (rows * a.n_heads * (HD / 16) + a.parts - 1) / a.parts;
 
