@@ -445,6 +445,7 @@ PYBIND11_MODULE(AIOS_MODULE, m) {
       .def_property_readonly("decode_resident", &Engine::decode_resident)
       .def_property_readonly("decode_resident_last", &Engine::decode_resident_last)
       .def_property_readonly("decode_resident_failed", &Engine::decode_resident_failed)
+      .def_property_readonly("decode_graphs", &Engine::decode_graphs)
       .def("set_decode_resident", &Engine::set_decode_resident, py::arg("on"))
       .def("set_decode_resident_wait", &Engine::set_decode_resident_wait, py::arg("ticks"), py::arg("behind") = -1)
       .def("capture_graphs", &Engine::capture_graphs, py::arg("max_b"), py::call_guard<py::gil_scoped_release>())

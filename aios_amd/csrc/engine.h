@@ -195,6 +195,7 @@ class Engine {
   // without it; the time, in 10 ns, after which it gives up at its gate, and in a wait behind it (negative: as it was)
   int decode_resident() const;
   bool decode_resident_last() const { return ds_now_; }  // whether the last step queued was one
+  int decode_graphs() const { return (int)graphs_.size(); }  // captured so far, of either route
   void set_decode_resident(bool on) { ds_use_ = on; }
   unsigned decode_resident_failed() const { return ds_failed_ ? *(volatile unsigned*)ds_failed_ : 0; }
   void set_decode_resident_wait(unsigned long long ticks, long long behind = -1);

@@ -99,19 +99,27 @@ Engine::Engine(const EngineConfig& cfg) : cfg_(cfg) {
 // Resident launches of a process take turns on a GPU: two of them at once would each hold some of the CUs and wait for the
 // others.  An engine that follows another one waits, on the device, for what that one has queued; the steps of one engine
 // follow each other in its stream anyway.  (Of other processes' launches nothing is known: what the gate is for.)  Nor does a resident
-// launch leave room for the launches of an engine beside it: while another one decodes on the GPU, all take the chain, whose launches share
-// it.  The lock also keeps a stream from being captured while another engine records its event there or asks for its state.
+// launch leave room for the launches of an engine beside it: while another one decodes on the GPU, all take the chain, whose
+// launches share it.  While an engine captures, its stream may be neither asked for its state nor get an event: it says so and leaves the event of its last resident launch; the lock is not held meanwhile.
 namespace {
 struct DsUse {
-  hipStream_t stream;
-  std::chrono::steady_clock::time_point at;  // of the last step
+  hipStream_t stream = nullptr;
+  std::chrono::steady_clock::time_point at;  // when it last went about a step (never: long ago)
+  bool capturing = false;
 };
 struct DsTurn {
   std::mutex mu;
   std::map<const void*, DsUse> users;
-  const void* last = nullptr;
+  const void* last = nullptr;  // whose resident launch was the last, its stream, and whether the event stands behind it
   hipStream_t stream = nullptr;
   hipEvent_t ev = nullptr;
+  bool recorded = false;
+  void record() {
+    if (recorded) return;
+    if (!ev) HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    HIP_CHECK(hipEventRecord(ev, stream));
+    recorded = true;
+  }
 };
 DsTurn& ds_turn(int device) {
   static std::mutex mu;
@@ -119,6 +127,23 @@ DsTurn& ds_turn(int device) {
   std::lock_guard<std::mutex> g(mu);
   return (*turns)[device];
 }
+struct DsCapture {
+  DsTurn& t;
+  const void* who;
+  DsCapture(DsTurn& turn, const void* engine, hipStream_t stream) : t(turn), who(engine) {
+    std::lock_guard<std::mutex> lock(t.mu);
+    if (t.last == who) t.record();
+    DsUse& u = t.users[who];
+    u.stream = stream;
+    u.capturing = true;
+  }
+  ~DsCapture() {
+    std::lock_guard<std::mutex> lock(t.mu);
+    DsUse& u = t.users[who];
+    u.capturing = false;
+    if (u.at != decltype(u.at)()) u.at = std::chrono::steady_clock::now();  // (captured within a step, whose launch is next)
+  }
+};
 }  // namespace
 
 Engine::~Engine() {
@@ -948,7 +973,8 @@ bool Engine::ds_next(int B) {
   return !ds_beside();
 }
 
-// whether another engine decodes on this GPU: its last step was queued within the time of one, or is still on its way
+// whether another engine uses this GPU: it went about its last step within the time of one, is capturing one, or what it queued is still
+// on its way
 bool Engine::ds_beside() {
   DsTurn& t = ds_turn(cfg_.device);
   std::lock_guard<std::mutex> lock(t.mu);
@@ -957,7 +983,9 @@ bool Engine::ds_beside() {
     if (who == this) continue;
     const auto ago = now - use.at;
     if (ago < std::chrono::milliseconds(2)) return true;
-    if (ago < std::chrono::seconds(10) && hipStreamQuery(use.stream) == hipErrorNotReady) {
+    if (ago >= std::chrono::seconds(10)) continue;
+    if (use.capturing) return true;
+    if (hipStreamQuery(use.stream) == hipErrorNotReady) {
       if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();  // (no error of a launch that is checked next)
       return true;
     }
@@ -967,21 +995,23 @@ bool Engine::ds_beside() {
 
 void Engine::launch_step(hipGraphExec_t g) {
   DsTurn& t = ds_turn(cfg_.device);
-  std::unique_lock<std::mutex> lock(t.mu);
-  t.users[this] = {stream_, std::chrono::steady_clock::now()};
+  std::unique_lock<std::mutex> lock(t.mu);  // (the launch and what the next engine waits for)
+  DsUse& u = t.users[this];
+  u.stream = stream_;
+  u.at = std::chrono::steady_clock::now();
   if (!ds_now_) {
     lock.unlock();
     HIP_CHECK(hipGraphLaunch(g, stream_));
     return;
   }
   if (t.last && t.last != this) {
-    if (!t.ev) HIP_CHECK(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
-    HIP_CHECK(hipEventRecord(t.ev, t.stream));
+    t.record();
     HIP_CHECK(hipStreamWaitEvent(stream_, t.ev, 0));
   }
   HIP_CHECK(hipGraphLaunch(g, stream_));
   t.last = this;
   t.stream = stream_;
+  t.recorded = false;
 }
 
 // Measured prefill-GEMM plans (kernels/gemm_pf.hip): every distinct projection launch of this model
@@ -2176,7 +2206,8 @@ void Engine::decode_loop_run(int B, int n_steps, bool use_graph) {
   }
 }
 
-int Engine::graph_key(int B, int kind) { return B * 4 + kind + (ds_now_ ? 1 << 24 : 0); }
+static constexpr int DS_KEY = 1 << 24;  // graphs of resident steps
+int Engine::graph_key(int B, int kind) { return B * 4 + kind + (ds_now_ ? DS_KEY : 0); }
 
 // the captured decode step for (B, sample_mask_): captured once, replayed for every request --
 // the kernels read tokens / positions / slots / sampling parameters from device arrays
@@ -2187,7 +2218,7 @@ hipGraphExec_t Engine::forward_graph(int B) { return captured(graph_key(B, 2), t
 hipGraphExec_t Engine::captured(int key, bool forward, int B) {
   auto it = graphs_.find(key);
   if (it == graphs_.end()) {
-    std::unique_lock<std::mutex> turn(ds_turn(cfg_.device).mu);
+    DsCapture mark(ds_turn(cfg_.device), this, stream_);
     hipGraph_t g;
     HIP_CHECK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
     try {
@@ -2290,21 +2321,23 @@ std::vector<int> Engine::decode_collect() {
 
 // capture (without running) the decode-step graphs of every batch size up to max_b, masked and
 // unmasked, so a serving scheduler whose batch grows and shrinks never stalls a step on a capture
-// (a 160-launch capture + instantiate costs milliseconds); returns the graphs held
+// (a 160-launch capture + instantiate costs milliseconds); returns the graphs held (of the chain of launches: resident steps' come on top)
 int Engine::capture_graphs(int max_b) {
   const CuScope cu_scope(cus_);  // (grids sized to this engine's CU mask)
   if (!finalized_) throw std::runtime_error("engine not finalized");
   HIP_CHECK(hipSetDevice(cfg_.device));
-  const bool saved = sample_mask_;
+  const bool saved = sample_mask_, route = ds_now_;
   for (int B = 1; B <= std::min(max_b, cfg_.max_batch); ++B)
-    for (int m = 0; m < 2; ++m) {
-      ds_now_ = B <= decode_resident();
-      sample_mask_ = m != 0;
+    for (int m = 0; m < 4; ++m) {
+      ds_now_ = m > 1;  // (rows that may run resident: both routes, each step asks for its own)
+      if (ds_now_ && B > decode_resident()) break;
+      sample_mask_ = m & 1;
       step_graph(B);
-      if (m == 0) forward_graph(B);  // (the pipelined decode's forward)
+      if (!sample_mask_) forward_graph(B);  // (the pipelined decode's forward)
     }
   sample_mask_ = saved;
-  return (int)graphs_.size();
+  ds_now_ = route;
+  return (int)std::count_if(graphs_.begin(), graphs_.end(), [](const auto& g) { return g.first < DS_KEY; });
 }
 
 std::vector<int> Engine::decode_loop_history(int B, int from_pos, int n) {

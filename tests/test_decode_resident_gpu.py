@@ -268,6 +268,29 @@ def test_a_step_beside_another_engines_takes_the_chain(models):
     assert a.decode_resident_last
 
 
+def test_a_warmed_engine_has_the_graphs_of_both_routes(models):
+    """What capture_graphs is for: no step captures, whichever route it takes"""
+    eng, cfg = _engine(models("gqa4-128"))
+    eng.prefill(0, [5, 6, 7, 8], 0, False)
+    eng.decode([0], [9], [4])
+    assert eng.decode_resident_last and eng.decode_resident == 1
+    assert eng.capture_graphs(2) == 6  # two batch sizes: the step, masked and not, and the forward alone
+    assert eng.decode_resident_last    # (of the last step still)
+    held = eng.decode_graphs
+    assert held == 9
+    mask = b"\xff" * ((cfg.vocab_size + 7) // 8)
+    for on in (True, False):
+        eng.set_decode_resident(on)
+        eng.decode([0], [9], [4])
+        assert eng.decode_resident_last == on
+        eng.decode([0], [9], [4], mask=mask)
+        eng.decode_submit([0], [9], [4])
+        eng.decode_sample()
+        eng.decode_collect()
+        eng.decode([0, 1], [9, 9], [4, 0])
+    assert eng.decode_graphs == held
+
+
 def test_what_the_resident_step_leaves_to_the_chain(tmp_path):
     """Formats, widths and engines that it is not built for take the chain"""
     small = write_synthetic_gguf(str(tmp_path / "small.gguf"), dataclasses.replace(BASE, d_model=768), "Q4_K_M", seed=7)
