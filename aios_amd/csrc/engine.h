@@ -437,6 +437,8 @@ class Engine {
   void ds_setup();
   static void ds_shares(const LayerW& L, int parts, int& wg_k, int& wg_v);
   void ds_upload();                // the cache's scales (again, when they change)
+  void ds_bound();                 // waits while many resident steps are queued
+  void ds_busy();                  // this engine is about to queue work
   bool ds_beside();
   bool ds_next(int B);             // whether the next step of B rows runs resident (not for a while after a failure, nor beside another engine's)
   int graph_key(int B, int kind);  // kind: 0 step, 1 masked step, 2 forward
@@ -449,6 +451,9 @@ class Engine {
   bool ds_now_ = false;            // the step being enqueued runs resident
   float* ds_scale_ = nullptr;
   unsigned* ds_failed_ = nullptr;  // pinned
+  hipEvent_t ds_ev_ = nullptr;     // among the resident steps that a loop queued
+  bool ds_marked_ = false;         // (recorded)
+  int ds_queued_ = 0;              // steps behind it
   unsigned ds_seen_ = 0;
   int ds_rest_ = 0;
   AllReduceFn allreduce_ = nullptr;

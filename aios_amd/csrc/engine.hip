@@ -100,7 +100,8 @@ Engine::Engine(const EngineConfig& cfg) : cfg_(cfg) {
 // others.  An engine that follows another one waits, on the device, for what that one has queued; the steps of one engine
 // follow each other in its stream anyway.  (Of other processes' launches nothing is known: what the gate is for.)  Nor does a resident
 // launch leave room for the launches of an engine beside it: while another one decodes on the GPU, all take the chain, whose
-// launches share it.  While an engine captures, its stream may be neither asked for its state nor get an event: it says so and leaves the event of its last resident launch; the lock is not held meanwhile.
+// launches share it.  An engine says so before it queues anything, a capture included.  While it captures, its stream may be neither asked for its
+// state nor get an event: it says that too, and leaves the event of its last resident launch; the lock is not held meanwhile.
 namespace {
 struct DsUse {
   hipStream_t stream = nullptr;
@@ -168,6 +169,7 @@ Engine::~Engine() {
   if (h_tok_out_) hipHostFree(h_tok_out_);
   if (h_mask_) hipHostFree(h_mask_);
   if (ds_failed_) hipHostFree(ds_failed_);
+  if (ds_ev_) hipEventDestroy(ds_ev_);
   if (pipe_ev_) hipEventDestroy(pipe_ev_);
   if (stream_) hipStreamDestroy(stream_);
 }
@@ -883,6 +885,7 @@ void Engine::ds_setup() {
   HIP_CHECK(hipHostMalloc((void**)&ds_failed_, 4, hipHostMallocDefault));
   *ds_failed_ = 0;
   a.host_failed = ds_failed_;
+  HIP_CHECK(hipEventCreateWithFlags(&ds_ev_, hipEventDisableTiming));
   a.gate_ticks = 2000000;     // 20 ms: longer than a kernel of another queue holds the CUs
   a.wait_ticks = 100000000;   // 1 s
   // norms' gains, heads' gains and biases of all layers beside each other
@@ -959,7 +962,16 @@ void Engine::set_decode_resident_wait(unsigned long long ticks, long long behind
   reset_graphs();
 }
 
+void Engine::ds_busy() {
+  DsTurn& t = ds_turn(cfg_.device);
+  std::lock_guard<std::mutex> lock(t.mu);
+  DsUse& u = t.users[this];
+  u.stream = stream_;
+  u.at = std::chrono::steady_clock::now();
+}
+
 bool Engine::ds_next(int B) {
+  ds_busy();
   if (B > decode_resident()) return false;
   const unsigned n = decode_resident_failed();
   if (n != ds_seen_) {  // another resident launch holds CUs: leave it the GPU for a while
@@ -971,6 +983,23 @@ bool Engine::ds_next(int B) {
     return false;
   }
   return !ds_beside();
+}
+
+// A step's route is chosen when it is queued: a loop's resident steps are queued a few ahead of the GPU and no further, so that the route is left soon
+// after another engine starts beside this one, or after a launch gave up (each one queued behind it may do the same).  An event a few steps, and
+// the one before it waited for: up to four steps where the process has other engines, up to sixteen where it has not.  (An event takes 2 to 4 us of a stream.)
+void Engine::ds_bound() {
+  DsTurn& t = ds_turn(cfg_.device);
+  bool others;
+  {
+    std::lock_guard<std::mutex> lock(t.mu);
+    others = t.users.size() > 1;
+  }
+  if (++ds_queued_ < (others ? 2 : 8)) return;
+  if (ds_marked_) HIP_CHECK(hipEventSynchronize(ds_ev_));
+  HIP_CHECK(hipEventRecord(ds_ev_, stream_));
+  ds_marked_ = true;
+  ds_queued_ = 0;
 }
 
 // whether another engine uses this GPU: it went about its last step within the time of one, is capturing one, or what it queued is still
@@ -994,16 +1023,12 @@ bool Engine::ds_beside() {
 }
 
 void Engine::launch_step(hipGraphExec_t g) {
-  DsTurn& t = ds_turn(cfg_.device);
-  std::unique_lock<std::mutex> lock(t.mu);  // (the launch and what the next engine waits for)
-  DsUse& u = t.users[this];
-  u.stream = stream_;
-  u.at = std::chrono::steady_clock::now();
   if (!ds_now_) {
-    lock.unlock();
     HIP_CHECK(hipGraphLaunch(g, stream_));
     return;
   }
+  DsTurn& t = ds_turn(cfg_.device);
+  std::lock_guard<std::mutex> lock(t.mu);  // (the launch and what the next engine waits for)
   if (t.last && t.last != this) {
     t.record();
     HIP_CHECK(hipStreamWaitEvent(stream_, t.ev, 0));
@@ -2197,12 +2222,14 @@ void Engine::decode_loop_run(int B, int n_steps, bool use_graph) {
   kv_sync(B);
   if (!use_graph) {
     ds_now_ = false;
+    ds_busy();
     for (int i = 0; i < n_steps; ++i) enqueue_decode_step(B);
     return;
   }
-  for (int i = 0; i < n_steps; ++i) {  // (another engine may start beside this one)
+  for (int i = 0; i < n_steps; ++i) {
     ds_now_ = ds_next(B);
     launch_step(step_graph(B));
+    if (ds_now_) ds_bound();
   }
 }
 

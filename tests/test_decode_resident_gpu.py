@@ -291,6 +291,59 @@ def test_a_warmed_engine_has_the_graphs_of_both_routes(models):
     assert eng.decode_graphs == held
 
 
+def test_a_loop_queues_few_resident_steps_ahead(models):
+    """A route is chosen when a step is queued: what is queued must not be hundreds of steps old when it runs, in one call or in many"""
+    eng, cfg = _engine(models("gqa4-128"))
+    for n, calls in ((1000, 1), (10, 100)):
+        eng.release_slot(0)
+        eng.prefill(0, [5, 6, 7, 8], 0, False)
+        eng.decode_loop_prepare([0], [9], [4])
+        eng.decode_loop_run(1, 8, True)
+        eng.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(calls):
+            eng.decode_loop_run(1, n, True)
+        t1 = time.perf_counter()
+        assert eng.decode_resident_last
+        eng.synchronize()
+        t2 = time.perf_counter()
+        assert t2 - t1 < 0.1 * (t2 - t0), (t1 - t0, t2 - t1)  # (four steps of a thousand, and what waiting takes)
+
+
+def test_an_engine_that_captures_is_seen(models):
+    """An engine that has only run alone has no graph of the chain.  Its first step beside another captures one, and the other engine's steps,
+    resident until then, leave it the GPU meanwhile"""
+    a, b = (_engine(models(n))[0] for n in ("gqa4-128", "gqa8-64"))
+    for e in (a, b):
+        e.prefill(0, [5, 6, 7, 8], 0, False)
+        time.sleep(0.05)
+        e.decode([0], [9], [4])
+        assert e.decode_resident_last
+    b.decode_loop_prepare([0], [9], [5])
+    b.decode_loop_run(1, 1, True)
+    time.sleep(0.05)
+    routes, done = [], threading.Event()
+
+    def loop():
+        for _ in range(1500):
+            b.decode_loop_run(1, 1, True)
+            routes.append(b.decode_resident_last)
+            if done.is_set():
+                return
+
+    t = threading.Thread(target=loop)
+    t.start()
+    time.sleep(0.02)
+    for i in range(20):
+        a.decode([0], [9], [5 + i])
+        assert not a.decode_resident_last
+    done.set()
+    t.join()
+    b.synchronize()
+    assert routes[0] and not routes[-1]  # alone at first; not beside the other
+    assert a.decode_resident_failed == b.decode_resident_failed == 0
+
+
 def test_what_the_resident_step_leaves_to_the_chain(tmp_path):
     """Formats, widths and engines that it is not built for take the chain"""
     small = write_synthetic_gguf(str(tmp_path / "small.gguf"), dataclasses.replace(BASE, d_model=768), "Q4_K_M", seed=7)
