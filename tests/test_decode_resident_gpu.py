@@ -49,10 +49,11 @@ def _engine(path, **kw):
     return eng, cfg
 
 
-def _steps(eng, slot, tokens, pos):
+def _steps(eng, slot, tokens, pos, on=None):
     out = []
     for i, t in enumerate(tokens):
         eng.decode([slot], [t], [pos + i])
+        assert on is None or eng.decode_resident_last == on
         out.append(np.asarray(eng.last_logits(1), np.float64).reshape(-1))
     return np.array(out)
 
@@ -82,13 +83,13 @@ def test_resident_step_is_the_chains(models, shape, kv):
             eng.release_slot(slot)
             if pos:
                 eng.prefill(slot, prompt, 0, False)
-            got.append(_steps(eng, slot, tokens, pos))
+            got.append(_steps(eng, slot, tokens, pos, on))
         assert np.isfinite(got[1]).all()
         assert _rel(got[1], got[0]).max() < TOL, (pos, _rel(got[1], got[0]))
     assert eng.decode_resident_failed == 0
 
 
-def _rows(eng, cfg, contexts, slots, seed):
+def _rows(eng, cfg, contexts, slots, seed, on=None):
     """Logits of two steps of a batch behind contexts of these lengths"""
     rng = np.random.default_rng(seed)
     for s, n in zip(slots, contexts):
@@ -98,6 +99,7 @@ def _rows(eng, cfg, contexts, slots, seed):
     out = []
     for i in range(2):
         eng.decode(slots, [int(t) for t in rng.integers(3, cfg.vocab_size, len(slots))], [n + i for n in contexts])
+        assert on is None or eng.decode_resident_last == on
         out.append(np.asarray(eng.last_logits(len(slots)), np.float64).reshape(len(slots), -1))
     return np.concatenate(out)
 
@@ -117,7 +119,7 @@ def test_resident_step_of_bf16_rows_is_the_chains(models, shape, kv):
         got = []
         for at, on in ((0, False), (4, True)):
             eng.set_decode_resident(on)
-            got.append(_rows(eng, cfg, contexts, list(range(at, at + len(contexts))), n))
+            got.append(_rows(eng, cfg, contexts, list(range(at, at + len(contexts))), n, on))
         assert np.isfinite(got[1]).all()
         assert _rel(got[1], got[0]).max() < TOL16, (contexts, _rel(got[1], got[0]))
     assert eng.decode_resident_failed == 0
@@ -130,7 +132,7 @@ def test_resident_step_matches_the_reference(models, shape):
     ref = ReferenceModel.from_gguf(path, kv_bf16=True, act_q8=True)
     toks = [1] + [int(t) for t in np.random.default_rng(5).integers(3, cfg.vocab_size, 43)]
     eng.prefill(0, toks[:40], 0, False)
-    got = torch.from_numpy(_steps(eng, 0, toks[40:], 40))
+    got = torch.from_numpy(_steps(eng, 0, toks[40:], 40, True))
     want = ref.forward(toks)[40:].double()
     assert (got - want).abs().max().item() < 2e-2 * max(want.abs().max().item(), 1.0)
 
@@ -160,10 +162,12 @@ def test_pipelined_and_looped_steps_are_resident_too(models):
         eng.release_slot(0)
         eng.prefill(0, prompt, 0, False)
         eng.decode_submit([0], [17], [120])
+        assert eng.decode_resident_last == on
         eng.decode_sample()
         toks = []
         for i in range(1, 12):
             eng.decode_submit([0], [], [120 + i])
+            assert eng.decode_resident_last == on
             toks += eng.decode_collect()
             eng.decode_sample()
         toks += eng.decode_collect()
@@ -171,6 +175,7 @@ def test_pipelined_and_looped_steps_are_resident_too(models):
         eng.prefill(0, prompt, 0, False)
         eng.decode_loop_prepare([0], [17], [120])
         eng.decode_loop_run(1, 12, True)
+        assert eng.decode_resident_last == on
         eng.synchronize()
         assert eng.decode_loop_history(1, 121, 12) == toks
         made.append(toks)
