@@ -99,13 +99,13 @@ Engine::Engine(const EngineConfig& cfg) : cfg_(cfg) {
 // Resident launches of a process take turns on a GPU: two of them at once would each hold some of the CUs and wait for the
 // others.  An engine that follows another one waits, on the device, for what that one has queued; the steps of one engine
 // follow each other in its stream anyway.  (Of other processes' launches nothing is known: what the gate is for.)  Nor does a resident
-// launch leave room for the launches of an engine beside it: while another one decodes on the GPU, all take the chain, whose
+// launch leave room for the launches of an engine beside it: while another one decodes or takes a prompt on the GPU, all take the chain, whose
 // launches share it.  An engine says so before it queues anything, a capture included.  While it captures, its stream may be neither asked for its
 // state nor get an event: it says that too, and leaves the event of its last resident launch; the lock is not held meanwhile.
 namespace {
 struct DsUse {
   hipStream_t stream = nullptr;
-  std::chrono::steady_clock::time_point at;  // when it last went about a step (never: long ago)
+  std::chrono::steady_clock::time_point at;  // when it last went about a step or a prompt (never: long ago)
   bool capturing = false;
 };
 struct DsTurn {
@@ -886,8 +886,8 @@ void Engine::ds_setup() {
   *ds_failed_ = 0;
   a.host_failed = ds_failed_;
   HIP_CHECK(hipEventCreateWithFlags(&ds_ev_, hipEventDisableTiming));
-  a.gate_ticks = 2000000;     // 20 ms: longer than a kernel of another queue holds the CUs
-  a.wait_ticks = 100000000;   // 1 s
+  a.gate_ticks = 2000000;     // 20 ms: CUs come free as another queue's kernels end, the longest of which (gate/up of a prompt's portion) is 0.75 ms
+  a.wait_ticks = 100000000;   // 1 s: behind the gate a wait is over in microseconds unless something is wrong
   // norms' gains, heads' gains and biases of all layers beside each other
   auto table = [&](size_t n) {
     ws_bytes_ += n * 4;
@@ -974,7 +974,9 @@ bool Engine::ds_next(int B) {
   ds_busy();
   if (B > decode_resident()) return false;
   const unsigned n = decode_resident_failed();
-  if (n != ds_seen_) {  // another resident launch holds CUs: leave it the GPU for a while
+  // Another resident launch (of another process) holds CUs: leave it the GPU for a while.  A step that the launch behind does takes 67 ms (TinyLlama
+  // Q4_K_M) to 212 (Mistral-7B), and the gate 20; tried again after 4096 steps, 2.5 to 5.9 s on the chain, that is 4 % at most
+  if (n != ds_seen_) {
     ds_seen_ = n;
     ds_rest_ = 4096;
   }
@@ -1002,7 +1004,7 @@ void Engine::ds_bound() {
   ds_queued_ = 0;
 }
 
-// whether another engine uses this GPU: it went about its last step within the time of one, is capturing one, or what it queued is still
+// whether another engine uses this GPU: it went about its last step or prompt within the time of a step, is capturing one, or what it queued is still
 // on its way
 bool Engine::ds_beside() {
   DsTurn& t = ds_turn(cfg_.device);
@@ -1011,8 +1013,8 @@ bool Engine::ds_beside() {
   for (const auto& [who, use] : t.users) {
     if (who == this) continue;
     const auto ago = now - use.at;
-    if (ago < std::chrono::milliseconds(2)) return true;
-    if (ago >= std::chrono::seconds(10)) continue;
+    if (ago < std::chrono::milliseconds(2)) return true;  // (between two steps: one takes 0.6 to 2.3 ms)
+    if (ago >= std::chrono::seconds(10)) continue;        // (idle: not asked at each step.  A loop of 4096 steps is queued for 6 s at most)
     if (use.capturing) return true;
     if (hipStreamQuery(use.stream) == hipErrorNotReady) {
       if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();  // (no error of a launch that is checked next)
@@ -1592,6 +1594,7 @@ void Engine::prefill_gemm(int slot, const std::vector<int>& tokens, int start_po
   // bf16(x * g_next) + per-tile sums, the next GEMM scales its rows) -- 3 launches per layer fewer
   static const bool short_fuse = !(std::getenv("AIOS_PREFILL_SHORT_FUSE") && std::atoi(std::getenv("AIOS_PREFILL_SHORT_FUSE")) == 0);
   for (int r0 = 0; r0 < T; r0 += gm_rows_) {
+    ds_busy();
     const int n = std::min(gm_rows_, T - r0);
     // chunks of <= 32 rows: the batched-decode GEMMs and their fused epilogues
     const bool sh = short_fuse && !tp && n <= 32;
@@ -1755,6 +1758,7 @@ std::vector<float> Engine::prefill(int slot, const std::vector<int>& tokens, int
   std::vector<int> hp(R), hs(R), hsl(R);
   try {
     for (int r0 = 0; r0 < T; r0 += R) {
+      ds_busy();
       const int n = std::min(R, T - r0);
       for (int i = 0; i < n; ++i) { hp[i] = start_pos + r0 + i; hsl[i] = hp[i] + 1; hs[i] = slot; }
       HIP_CHECK(hipMemcpyAsync(pf_tokens_, tokens.data() + r0, n * 4, hipMemcpyHostToDevice, stream_));
@@ -1941,6 +1945,7 @@ void Engine::run_step(const std::vector<int>& slots, const std::vector<int>& sta
       }
     }
     std::vector<int> first;
+    ds_busy();
     lm_->forward(pieces, first);
     std::vector<int> xrows;
     size_t p = 0, at = base;

@@ -349,6 +349,47 @@ def test_an_engine_that_captures_is_seen(models):
     assert a.decode_resident_failed == b.decode_resident_failed == 0
 
 
+@pytest.mark.parametrize("kind", ["short", "long", "layered"])
+def test_a_step_beside_a_prompt_takes_the_chain(models, kind, tmp_models):
+    """A prompt's launches need CUs too: those of another engine's prompt are seen as its decode steps are"""
+    a, cfg = _engine(models("gqa4-128"))
+    if kind == "layered":
+        import test_seledra_gpu
+
+        p = test_seledra_gpu.engine(test_seledra_gpu.model("aligned", tmp_models)[0])
+        prompt = [3 + i % 80 for i in range(400)]
+    else:
+        p = _engine(models("gqa8-64"))[0]
+        prompt = [int(t) for t in np.random.default_rng(17).integers(3, 1000, 6 if kind == "short" else 2000)]
+    a.prefill(0, [5, 6, 7, 8], 0, False)
+    p.prefill(0, prompt, 0, False)
+    time.sleep(0.05)
+    tokens = [int(t) for t in np.random.default_rng(19).integers(3, 1000, 60)]
+    want = _steps(a, 0, tokens, 4, True)
+    done = threading.Event()
+
+    def prompts():
+        while not done.is_set():
+            p.prefill(0, prompt, 0, False)
+
+    t = threading.Thread(target=prompts)
+    t.start()
+    time.sleep(0.02)
+    got, chain = [], 0
+    for i, tok in enumerate(tokens):
+        a.decode([0], [tok], [4 + i])
+        chain += not a.decode_resident_last
+        got.append(np.asarray(a.last_logits(1), np.float64).reshape(-1))
+    done.set()
+    t.join()
+    assert chain > len(tokens) // 2  # (between two prompts a step may run resident)
+    assert a.decode_resident_failed == 0
+    assert _rel(np.array(got), want).max() < TOL
+    time.sleep(0.05)
+    a.decode([0], [9], [4])
+    assert a.decode_resident_last
+
+
 def test_what_the_resident_step_leaves_to_the_chain(tmp_path):
     """Formats, widths and engines that it is not built for take the chain"""
     small = write_synthetic_gguf(str(tmp_path / "small.gguf"), dataclasses.replace(BASE, d_model=768), "Q4_K_M", seed=7)
