@@ -20,10 +20,10 @@
 // for nobody) does the step.  Behind the open gate every wait is for a workgroup that runs; it is bounded all the same
 // (wait_ticks), with the same way out.
 //
-// A step with its sampler, us, chain -> resident (MI355X).  Q4_K_M: TinyLlama 128 keys 614 -> 465, 1000 keys 695 -> 538; Mistral-7B 128 keys
-// 1434 -> 1149, 2000 keys 1569 -> 1294, 3900 keys 1631 -> 1376; with the fp8 cache 2000 keys 1536 -> 1279, 16000 keys 1675 -> 1548; Qwen3-8B 128
-// keys 1747 -> 1286.  TinyLlama bf16, 128 / 1000 keys: one row 740 -> 592 / 820 -> 646, two 809 -> 611 / 884 -> 663, three 833 -> 640 / 905 -> 696,
-// four 843 -> 691 / 905 -> 738 (five and more stay with the GEMMs: a fifth row is a second matrix instruction for the same weights, and its operand
+// A step with its sampler, us, chain -> resident (MI355X).  Q4_K_M: TinyLlama 128 keys 596 -> 453, 1000 keys 674 -> 534; Mistral-7B 128 keys
+// 1412 -> 1138, 2000 keys 1551 -> 1280, 3900 keys 1610 -> 1365; with the fp8 cache 2000 keys 1512 -> 1238, 16000 keys 1657 -> 1508; Qwen3-8B 128
+// keys 1733 -> 1269.  TinyLlama bf16, 128 / 1000 keys: one row 722 -> 584 / 799 -> 648, two 794 -> 603 / 862 -> 665, three 822 -> 625 / 873 -> 689,
+// four 822 -> 672 / 887 -> 733 (five and more stay with the GEMMs: a fifth row is a second matrix instruction for the same weights, and its operand
 // leaves the ring three slots).
 #include "decode_stream.h"
 
